@@ -2,12 +2,12 @@
 // Conv2dWinogradAlgorithm<float>::winograd_f63 / winograd_f23
 // (src/kernels/cpu/winograd_algorithm.cpp:504-947 / :57-459) with the padding rule of
 // KernelCommonFunc::in_out_pad_and_fix_size (src/kernels/common/function.cpp:14-78).
-// F(6,3) is described below; F(2,3) is its twin with 4x4 patches (stride 2), 16 GEMMs and
+// F(6,3) is described below; F(2,3) is its twin with 4x4 patches (stride 2), 16 frequencies and
 // transforms made of sums and differences only.
 //
-//   U = G g G^T      kernel transform, once per weight tensor          -> u[64][Cout][Cin]
-//   V = B^T d B      input transform of every 8x8 patch (stride 6)      -> v[N][64][Cin][tiles]
-//   M_t = U_t V_t    64 independent GEMMs (Cout x Cin x tiles) per image -> m[N][64][Cout][tiles]
+//   U = G g G^T      kernel transform, once per weight tensor
+//   V = B^T d B      input transform of every 8x8 patch (stride 6)
+//   M_f = U_f V_f    64 independent GEMMs (Cout x Cin x tiles)
 //   Y = A^T M A      output transform, cut to the true output size       -> out NCHW
 //
 // F(6,3) in fp32 amplifies single roundings to ~1e-5 of an O(1) output, the same size as the
@@ -17,18 +17,32 @@
 //     is built with gcc -O3 -mfma, whose default contraction fuses a*b+c patterns (in
 //     a*c1 - b*c2 it fuses the first product and rounds the second); those FMAs are written
 //     out explicitly here and the file is compiled with -ffp-contract=off;
-//   * the 64 small GEMMs accumulate like the reference's pack8/kernel_8x8 micro-kernel
+//   * the GEMMs accumulate like the reference's pack8/kernel_8x8 micro-kernel
 //     (src/kernels/cpu/math_cpu.cpp:386-700): one k-ascending FMA chain per output, and for
-//     columns beyond the last full block of 8 four interleaved chains combined as
-//     (s0+s1), (s2+s3), 0+s01, +s23.  They run on the vector ALUs -- the work is 4.4x smaller
-//     than the direct convolution and the fp32 MFMA would change the summation order.
-// All kernels here are memory/latency-bound elementwise or small-GEMM kernels.
+//     columns beyond an image's last full block of 8 four interleaved chains combined as
+//     (s0+s1), (s2+s3), 0+s01, +s23.  v_mfma_f32_32x32x2_f32 IS such a chain: every output is
+//     fma(a1, b1, fma(a0, b0, c)) with one rounding per step and denormals kept (compared with
+//     fmaf on the host, bit for bit, over normal, widely scaled and denormal operands), so the
+//     matrix cores give the reference's bits as long as a step carries k and k + 1 in order.
+//
+// Layouts.  A "column" is one tile of one image.  The columns an image computes as plain chains (its
+// first tiles/8*8) come first, image after image, padded to whole fragments of 32; then the rest
+// ("tail" columns), padded likewise.  U and V are stored as MFMA operands: [frequency][fragment of 32
+// rows or columns][group t of 8 channels][lane][4], lane l's element j being channel 8t + 2j + l/32 of row or
+// column l%32 -- one contiguous KiB per four MFMA steps, loaded straight into registers (no LDS: with 64 cycles
+// per MFMA the operands of a 32 x 64 tile need a quarter of the CU's load path).  M is [frequency][cout][columns].
+// Channels beyond Cin are -0 in U and +0 in V: their product -0 leaves every accumulator as it is, signed zeros
+// included.
 #include "tsx_common.hpp"
 
-#include <atomic>
+#include <algorithm>
 
 namespace tsx {
 namespace {
+
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 
 // ---------------------------------------------------------------- transforms (explicit FMAs)
 
@@ -85,407 +99,369 @@ __device__ __forceinline__ void at_pass(const float *t, float *o) {
     o[5] = re1 + re3 * 32 + re5 + t[7];
 }
 
-// U[t = i*8+j][cout][cin] = (G g G^T)[i][j]  (winograd_algorithm.cpp:504-566, before its pack8_A)
-__global__ __launch_bounds__(256) void wino_kernel_transform_kernel(const float *__restrict__ w, int cout, int cin,
-                                                                   float *__restrict__ u) {
-    const int id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= cout * cin) return;
-    const float G[8][3] = {{1.0f, 0.0f, 0.0f},
-                           {-2.f / 9, -2.f / 9, -2.f / 9},
-                           {-2.f / 9, 2.f / 9, -2.f / 9},
-                           {1.f / 90, 1.f / 45, 2.f / 45},
-                           {1.f / 90, -1.f / 45, 2.f / 45},
-                           {1.f / 45, 1.f / 90, 1.f / 180},
-                           {1.f / 45, -1.f / 90, 1.f / 180},
-                           {0.0f, 0.0f, 1.0f}};
-    float g[9];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) g[i] = w[int64_t(id) * 9 + i];
-    float tmp[3][8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-            tmp[r][i] = fmaf(g[r * 3 + 2], G[i][2], fmaf(g[r * 3 + 0], G[i][0], g[r * 3 + 1] * G[i][1]));
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            u[int64_t(i * 8 + j) * cout * cin + id] =
-                fmaf(tmp[2][j], G[i][2], fmaf(tmp[0][j], G[i][0], tmp[1][j] * G[i][1]));
-}
 
 struct WinoGeom {
     int n, c, h, w, cout, ho, wo, pad_top, pad_left, th, tw, tiles;
     float padding_value;
+    int rfrags, kgroups;       // 32-row fragments of U, groups of 8 channels
+    int n8, mfrags, nfrags;    // chain columns per image, their fragments, all fragments
+    int cols;                  // 32 * nfrags: the row pitch of M
 };
 
-// One thread per (image, channel, tile); adjacent lanes take adjacent tiles, so the 64 stores of a
-// lane (stride Cin*tiles) are coalesced across the wavefront.
-__global__ __launch_bounds__(256) void wino_input_transform_kernel(const float *__restrict__ x, WinoGeom g,
-                                                                  float *__restrict__ v) {
-    const int64_t total = int64_t(g.n) * g.c * g.tiles;
+// The image and tile of a column; false for the columns that pad a fragment.
+__device__ __forceinline__ bool column_tile(const WinoGeom &g, int col, int &img, int &tile) {
+    const bool tail = col >= g.mfrags * 32;
+    const int c = tail ? col - g.mfrags * 32 : col, per = tail ? g.tiles - g.n8 : g.n8;
+    img = per > 0 ? c / per : 0;
+    tile = c - img * per + (tail ? g.n8 : 0);
+    return per > 0 && img < g.n;
+}
+
+// Element (channel, row or column) -> float index inside one frequency of U or V
+__device__ __forceinline__ int64_t operand_index(int frag, int kgroups, int t, int lane, int j) {
+    return ((int64_t(frag) * kgroups + t) * 64 + lane) * 4 + j;
+}
+
+// U = G g G^T, one thread per (cout, cin) of the padded operand (TILE 6: winograd_algorithm.cpp:504-566, TILE 2:
+// :57-105, before their pack8_A).
+template <int TILE>
+__global__ __launch_bounds__(256) void wino_kernel_transform_kernel(const float *__restrict__ w, int cout, int cin, int rfrags,
+                                                                   int kgroups, float *__restrict__ u) {
+    constexpr int P = TILE + 2;
+    const int64_t per_f = int64_t(rfrags) * kgroups * 256;
     const int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (id >= total) return;
-    const int tile = int(id % g.tiles);
-    const int ch = int((id / g.tiles) % g.c);
-    const int img = int(id / g.tiles / g.c);
+    if (id >= per_f) return;
+    const int j = int(id % 4), lane = int(id / 4 % 64), t = int(id / 256 % kgroups), rf = int(id / 256 / kgroups);
+    const int co = rf * 32 + lane % 32, ci = 8 * t + 2 * j + lane / 32;
+    if (co >= cout || ci >= cin) {
+        for (int f = 0; f < P * P; ++f) u[f * per_f + id] = -0.f;
+        return;
+    }
+    const float G6[8][3] = {{1.0f, 0.0f, 0.0f},
+                            {-2.f / 9, -2.f / 9, -2.f / 9},
+                            {-2.f / 9, 2.f / 9, -2.f / 9},
+                            {1.f / 90, 1.f / 45, 2.f / 45},
+                            {1.f / 90, -1.f / 45, 2.f / 45},
+                            {1.f / 45, 1.f / 90, 1.f / 180},
+                            {1.f / 45, -1.f / 90, 1.f / 180},
+                            {0.0f, 0.0f, 1.0f}};
+    const float G2[4][3] = {{1.f, 0.f, 0.f}, {0.5f, 0.5f, 0.5f}, {0.5f, -0.5f, 0.5f}, {0.f, 0.f, 1.f}};
+    float g[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) g[i] = w[(int64_t(co) * cin + ci) * 9 + i];
+    float tmp[3][P];
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const float *G = TILE == 6 ? G6[i] : G2[i % 4];
+            tmp[r][i] = fmaf(g[r * 3 + 2], G[2], fmaf(g[r * 3 + 0], G[0], g[r * 3 + 1] * G[1]));
+        }
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+#pragma unroll
+        for (int q = 0; q < P; ++q) {
+            const float *G = TILE == 6 ? G6[i] : G2[i % 4];
+            u[(i * P + q) * per_f + id] = fmaf(tmp[2][q], G[2], fmaf(tmp[0][q], G[0], tmp[1][q] * G[1]));
+        }
+}
+
+// V of F(6,3).  One workgroup = the 32 columns of a fragment x four channels of one parity of a channel group (a
+// lane then owns whole 16-byte operand elements); thread (i, column) transforms row i of the column's four patches,
+// the rows cross to columns through LDS, and it transforms column i and stores its eight frequencies.  One thread
+// per patch, as before, is under one wavefront per SIMD on 8 images of 28x28x256 and waits for its 64 loads alone:
+// 9.2 us there.
+constexpr int WT_CH = 4;      // channels per workgroup
+
+__global__ __launch_bounds__(256) void wino_input_transform_kernel(const float *__restrict__ x, WinoGeom g, float *__restrict__ v) {
+    __shared__ float rows[WT_CH][8][8][32];
+    const int i = threadIdx.x / 32, lc = threadIdx.x % 32;
+    const int frag = blockIdx.x, t = blockIdx.y / 2, hf = blockIdx.y % 2;
+    int img, tile;
+    const bool valid = column_tile(g, frag * 32 + lc, img, tile);
+    if (!valid) img = tile = 0;                              // a padding column: loads tile 0, result never used
     const int ty = tile / g.tw, tx = tile - ty * g.tw;
-    const float *src = x + (int64_t(img) * g.c + ch) * g.h * g.w;
-    float db[8][8];
+    const int hh = ty * 6 + i - g.pad_top, w0 = tx * 6 - g.pad_left;
+    const bool row_in = hh >= 0 && hh < g.h;
+    const float *src = x + int64_t(img) * g.c * g.h * g.w + min(max(hh, 0), g.h - 1) * g.w;
+    float d[WT_CH][8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        float row[8];
-        const int hh = ty * 6 + i - g.pad_top;
+    for (int q = 0; q < WT_CH; ++q) {
+        const float *plane = src + int64_t(min(8 * t + 2 * q + hf, g.c - 1)) * g.h * g.w;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int ww = tx * 6 + j - g.pad_left;
-            // outside the tensor: the conv padding and the bottom/right fill both use padding_value
-            row[j] = (hh >= 0 && hh < g.h && ww >= 0 && ww < g.w) ? src[hh * g.w + ww] : g.padding_value;
+        for (int jj = 0; jj < 8; ++jj) d[q][jj] = plane[min(max(w0 + jj, 0), g.w - 1)];
+    }
+#pragma unroll
+    for (int q = 0; q < WT_CH; ++q) {
+        // outside the tensor: the conv padding and the bottom/right fill both use padding_value
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) d[q][jj] = (row_in && w0 + jj >= 0 && w0 + jj < g.w) ? d[q][jj] : g.padding_value;
+        float o[8];
+        bt_row(d[q], o);
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) rows[q][i][jj][lc] = o[jj];
+    }
+    __syncthreads();
+    float o[WT_CH][8];
+#pragma unroll
+    for (int q = 0; q < WT_CH; ++q) {
+        float col[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) col[r] = rows[q][r][i][lc];
+        bt_col(col, o[q]);
+        if (8 * t + 2 * q + hf >= g.c) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) o[q][r] = 0.f;       // channel padding
         }
-        bt_row(row, db[i]);
     }
-    float *dst = v + (int64_t(img) * 64 * g.c + ch) * g.tiles + tile;
-    const int64_t stride = int64_t(g.c) * g.tiles;
+    const int64_t per_f = int64_t(g.nfrags) * g.kgroups * 256;
+    float *dst = v + operand_index(frag, g.kgroups, t, lc + 32 * hf, 0);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        float col[8], o[8];
-#pragma unroll
-        for (int r = 0; r < 8; ++r) col[r] = db[r][i];
-        bt_col(col, o);
-#pragma unroll
-        for (int r = 0; r < 8; ++r) dst[(r * 8 + i) * stride] = o[r];
-    }
+    for (int r = 0; r < 8; ++r) *reinterpret_cast<v4f *>(dst + (r * 8 + i) * per_f) = v4f{o[0][r], o[1][r], o[2][r], o[3][r]};
 }
 
-// C[b][m][n] = A[b % a_batches][m][k] * B[b][k][n] in the reference's accumulation order
-// (math_cpu.cpp:386-700 as restated by the CPU oracle): m8/n8 = extents rounded down to 8.
-// Columns below n8 are one fused-multiply-add chain in ascending k per output; the columns from n8 on sum four
-// interleaved partial chains first.  Two kernels: the tiled one for the columns below n8, this one (one lane per
-// output, columns j0..n) for the rest.
-__global__ __launch_bounds__(256) void gemm_f32_seq_kernel(const float *__restrict__ a, const float *__restrict__ b,
-                                                          float *__restrict__ c, int m, int n, int k, int batches,
-                                                          int a_batches, int j0) {
-    const int cols = n - j0;
-    const int64_t total = int64_t(batches) * m * cols;
-    const int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (id >= total) return;
-    const int j = j0 + int(id % cols);
-    const int i = int((id / cols) % m);
-    const int bt = int(id / cols / m);
-    const float *ar = a + (int64_t(bt % a_batches) * m + i) * k;
-    const float *bc = b + int64_t(bt) * k * n + j;
-    const int m8 = m / 8 * 8, n8 = n / 8 * 8, k4 = k / 4 * 4;
-    float r;
-    if (j < n8) {
-        float acc = 0.f;
-        for (int kk = 0; kk < k; ++kk) acc = fmaf(bc[int64_t(kk) * n], ar[kk], acc);
-        r = acc;
-    } else {
-        float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-        for (int kk = 0; kk < k4; kk += 4) {
-            s0 = fmaf(ar[kk + 0], bc[int64_t(kk + 0) * n], s0);
-            s1 = fmaf(ar[kk + 1], bc[int64_t(kk + 1) * n], s1);
-            s2 = fmaf(ar[kk + 2], bc[int64_t(kk + 2) * n], s2);
-            s3 = fmaf(ar[kk + 3], bc[int64_t(kk + 3) * n], s3);
-        }
-        float acc;
-        if (i < m8) {
-            const float s01 = s0 + s1, s23 = s2 + s3;
-            acc = 0.f + s01;
-            acc = acc + s23;
-        } else {
-            acc = ((s0 + s1) + s2) + s3;
-        }
-        for (int kk = k4; kk < k; ++kk) acc = fmaf(ar[kk], bc[int64_t(kk) * n], acc);
-        r = acc;
+// V of F(2,3): B^T d B (winograd_algorithm.cpp:181-243), row combinations (i0-i2, i1+i2, i2-i1, i1-i3) first, then the
+// same combination across columns, in the reference's grouping.  Thread = one column x four channels of one parity.
+__global__ __launch_bounds__(256) void wino23_input_transform_kernel(const float *__restrict__ x, WinoGeom g, float *__restrict__ v) {
+    const int lc = threadIdx.x % 32, part = blockIdx.y * 8 + threadIdx.x / 32;     // part = (channel group, parity)
+    const int frag = blockIdx.x, t = part / 2, hf = part % 2;
+    if (t >= g.kgroups) return;
+    int img, tile;
+    const bool valid = column_tile(g, frag * 32 + lc, img, tile);
+    if (!valid) img = tile = 0;
+    const int ty = tile / g.tw, tx = tile - ty * g.tw;
+    const int h0 = ty * 2 - g.pad_top, w0 = tx * 2 - g.pad_left;
+    const float *src = x + int64_t(img) * g.c * g.h * g.w;
+    float d[4][4][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float *plane = src + int64_t(min(8 * t + 2 * q + hf, g.c - 1)) * g.h * g.w;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) d[q][i][j] = plane[min(max(h0 + i, 0), g.h - 1) * g.w + min(max(w0 + j, 0), g.w - 1)];
     }
-    c[(int64_t(bt) * m + i) * n + j] = r;
-}
-
-// The columns below n8: every output is the same chain acc = fma(B[k][j], A[i][k], acc) over ascending k, so a
-// lane can hold a 4 x 4 block of outputs and feed 16 chains from 4 values of A and 4 of B per k -- an eighth of
-// the loads of one lane per output, the same bits.  VEC: k and n multiples of 4 and 16-byte aligned operands, so
-// A is read four k at a time and B four columns at a time as 16-byte loads.  Lanes run along the column blocks.
-template <bool VEC>
-__global__ __launch_bounds__(256) void gemm_f32_seq_tiled_kernel(const float *__restrict__ a, const float *__restrict__ b,
-                                                                float *__restrict__ c, int m, int n, int k, int batches,
-                                                                int a_batches, int n8) {
-    const int jb = n8 / 4, ib = (m + 3) / 4;
-    const int64_t total = int64_t(batches) * ib * jb;
-    const int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (id >= total) return;
-    const int j = int(id % jb) * 4;
-    const int i = int((id / jb) % ib) * 4;
-    const int bt = int(id / jb / ib);
-    const float *ab = a + int64_t(bt % a_batches) * m * k;
-    const float *bc = b + int64_t(bt) * k * n + j;
-    const float *ar[4];
+    v4f o[16];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ar[r] = ab + int64_t(min(i + r, m - 1)) * k;   // rows past m: computed, not stored
-    float acc[4][4];
+    for (int q = 0; q < 4; ++q) {
+        const bool real = 8 * t + 2 * q + hf < g.c;
+        float r[4][4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[r][q] = 0.f;
-    int kk = 0;
-    if (VEC) {
-        for (; kk + 4 <= k; kk += 4) {
-            float4 av[4], bv[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) av[r] = *reinterpret_cast<const float4 *>(ar[r] + kk);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) bv[t] = *reinterpret_cast<const float4 *>(bc + int64_t(kk + t) * n);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float av_t = t == 0 ? av[r].x : t == 1 ? av[r].y : t == 2 ? av[r].z : av[r].w;
-                    acc[r][0] = fmaf(bv[t].x, av_t, acc[r][0]);
-                    acc[r][1] = fmaf(bv[t].y, av_t, acc[r][1]);
-                    acc[r][2] = fmaf(bv[t].z, av_t, acc[r][2]);
-                    acc[r][3] = fmaf(bv[t].w, av_t, acc[r][3]);
-                }
+            for (int j = 0; j < 4; ++j) {
+                const bool in = h0 + i >= 0 && h0 + i < g.h && w0 + j >= 0 && w0 + j < g.w;
+                d[q][i][j] = in ? d[q][i][j] : g.padding_value;
             }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            r[0][j] = d[q][0][j] - d[q][2][j];
+            r[1][j] = d[q][1][j] + d[q][2][j];
+            r[2][j] = d[q][2][j] - d[q][1][j];
+            r[3][j] = d[q][1][j] - d[q][3][j];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            o[k * 4 + 0][q] = real ? r[k][0] - r[k][2] : 0.f;
+            o[k * 4 + 1][q] = real ? r[k][1] + r[k][2] : 0.f;
+            o[k * 4 + 2][q] = real ? r[k][2] - r[k][1] : 0.f;
+            o[k * 4 + 3][q] = real ? r[k][1] - r[k][3] : 0.f;
         }
     }
-    for (; kk < k; ++kk) {
-        float bv[4], av[4];
+    const int64_t per_f = int64_t(g.nfrags) * g.kgroups * 256;
+    float *dst = v + operand_index(frag, g.kgroups, t, lc + 32 * hf, 0);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) bv[q] = bc[int64_t(kk) * n + q];
+    for (int f = 0; f < 16; ++f) *reinterpret_cast<v4f *>(dst + f * per_f) = o[f];
+}
+
+// M_f = U_f V_f for every frequency, in the reference's accumulation order.  A wavefront computes 32 output channels x
+// FN fragments of columns; the four wavefronts of a workgroup take consecutive row fragments of the same columns (their V
+// loads meet in L1).  Workgroups b, b + 8, ... run on one XCD: each XCD gets whole frequencies, whose U and V then
+// stay in its L2 (8 x 456 KB at 8 images of 28x28x256).  RING groups of 8 channels are in flight per wavefront.
+// Bound by the fp32 MFMA: 1.68 GFLOP at that shape = 11 us at 157 TFLOP/s.
+// Chains on the vector ALUs, one lane per 4 x 4 outputs, took 276 + 31 us there.
+constexpr int WG_RING = 4;
+
+template <int FN>
+__device__ __forceinline__ void wino_gemm_chain(const v4f *__restrict__ u, const v4f *__restrict__ v, float *__restrict__ m, const WinoGeom &g,
+                                                int f, int rf, int cf0, int lane) {
+    const int T = g.kgroups;
+    const v4f *ua = u + (int64_t(f) * g.rfrags + rf) * T * 64 + lane;
+    const v4f *vb[FN];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) av[r] = ar[r][kk];
+    for (int n = 0; n < FN; ++n) vb[n] = v + (int64_t(f) * g.nfrags + min(cf0 + n, g.mfrags - 1)) * T * 64 + lane;
+    v4f a[WG_RING], b[FN][WG_RING];
+    v16f acc[FN];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+    for (int n = 0; n < FN; ++n)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[r][q] = fmaf(bv[q], av[r], acc[r][q]);
-    }
+        for (int r = 0; r < 16; ++r) acc[n][r] = 0.f;
+    auto load = [&](auto slot, int t) __attribute__((always_inline)) {
+        constexpr int s = decltype(slot)::value;
+        const int tt = min(t, T - 1);                        // beyond the last group: its lines again, never used
+        a[s] = ua[tt * 64];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        if (i + r >= m) break;
-        float *dst = c + (int64_t(bt) * m + i + r) * n + j;
-        if (VEC) *reinterpret_cast<float4 *>(dst) = make_float4(acc[r][0], acc[r][1], acc[r][2], acc[r][3]);
-        else {
+        for (int n = 0; n < FN; ++n) b[n][s] = vb[n][tt * 64];
+    };
+    auto multiply = [&](auto slot) __attribute__((always_inline)) {
+        constexpr int s = decltype(slot)::value;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) dst[q] = acc[r][q];
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int n = 0; n < FN; ++n) acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s][j], b[n][s][j], acc[n], 0, 0, 0);
+    };
+    static_for<0, WG_RING - 1>([&](auto sc) { load(sc, decltype(sc)::value); });
+    int t = 0;
+    for (; t + WG_RING <= T; t += WG_RING)
+        static_for<0, WG_RING>([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            load(std::integral_constant<int, (s + WG_RING - 1) % WG_RING>{}, t + s + WG_RING - 1);
+            multiply(sc);
+        });
+    static_for<0, WG_RING - 1>([&](auto sc) {                // the groups left over are in the ring already
+        if (t + decltype(sc)::value < T) multiply(sc);
+    });
+#pragma unroll
+    for (int n = 0; n < FN; ++n) {
+        if (cf0 + n >= g.mfrags) break;
+        float *dst = m + (int64_t(f) * g.cout + rf * 32) * g.cols + (cf0 + n) * 32 + lane % 32;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = 8 * (r / 4) + 4 * (lane / 32) + r % 4;
+            if (rf * 32 + row < g.cout) dst[int64_t(row) * g.cols] = acc[n][r];
         }
     }
 }
 
-// Both parts of the sequential-order GEMM on `stream`.
-int launch_gemm_f32_seq(const float *a, const float *b, float *c, int m, int n, int k, int batches, int a_batches,
-                        hipStream_t stream) {
-    const int n8 = n / 8 * 8;
-    if (n8 > 0) {
-        const int64_t threads = int64_t(batches) * ((m + 3) / 4) * (n8 / 4);
-        const bool vec = k % 4 == 0 && n % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
-                         reinterpret_cast<uintptr_t>(b) % 16 == 0 && reinterpret_cast<uintptr_t>(c) % 16 == 0;
-        const dim3 grid(unsigned(ceil_div(threads, 256)));
-        if (vec) hipLaunchKernelGGL(gemm_f32_seq_tiled_kernel<true>, grid, dim3(256), 0, stream, a, b, c, m, n, k, batches, a_batches, n8);
-        else hipLaunchKernelGGL(gemm_f32_seq_tiled_kernel<false>, grid, dim3(256), 0, stream, a, b, c, m, n, k, batches, a_batches, n8);
-        TSX_LAUNCH_CHECK("gemm_f32_seq_tiled_kernel");
+// The tail columns: chains over k = q, q + 4, q + 8, ... (q = 0..3) up to k4 = k/4*4, their combination, then the up to
+// three channels left as a chain behind it.  An MFMA step takes channels 8t + q and 8t + 4 + q: lanes of half H need
+// elements 2H, 2H + 1 of both half-lanes' operands, two 8-byte loads.
+__device__ __forceinline__ void wino_gemm_tail(const float *__restrict__ u, const float *__restrict__ v, float *__restrict__ m, const WinoGeom &g,
+                                               int f, int rf, int cf, int lane) {
+    const int T = g.kgroups, H = lane / 32;
+    const float *ua = u + operand_index(0, 1, 0, lane % 32, 2 * H) + (int64_t(f) * g.rfrags + rf) * T * 256;
+    const float *vb = v + operand_index(0, 1, 0, lane % 32, 2 * H) + (int64_t(f) * g.nfrags + cf) * T * 256;
+    v16f s[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[q][r] = 0.f;
+    const int k4 = g.c / 4 * 4, full = k4 / 8;
+    v2f a[2][2], b[2][2];                                    // [slot][parity]
+    auto load = [&](auto slot, int t) __attribute__((always_inline)) {
+        constexpr int sl = decltype(slot)::value;
+        const int64_t off = int64_t(min(t, T - 1)) * 256;
+#pragma unroll
+        for (int par = 0; par < 2; ++par) {
+            a[sl][par] = *reinterpret_cast<const v2f *>(ua + off + par * 128);
+            b[sl][par] = *reinterpret_cast<const v2f *>(vb + off + par * 128);
+        }
+    };
+    auto multiply = [&](auto slot, bool live) __attribute__((always_inline)) {
+        constexpr int sl = decltype(slot)::value;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            s[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(live ? a[sl][q % 2][q / 2] : -0.f, live ? b[sl][q % 2][q / 2] : 0.f, s[q], 0, 0, 0);
+    };
+    load(std::integral_constant<int, 0>{}, 0);
+    int t = 0;
+    for (; t + 2 <= full; t += 2) {
+        load(std::integral_constant<int, 1>{}, t + 1);
+        multiply(std::integral_constant<int, 0>{}, true);
+        load(std::integral_constant<int, 0>{}, t + 2);
+        multiply(std::integral_constant<int, 1>{}, true);
     }
-    if (n8 < n) {
-        const int64_t threads = int64_t(batches) * m * (n - n8);
-        hipLaunchKernelGGL(gemm_f32_seq_kernel, dim3(unsigned(ceil_div(threads, 256))), dim3(256), 0, stream, a, b, c, m, n, k,
-                           batches, a_batches, n8);
-        TSX_LAUNCH_CHECK("gemm_f32_seq_kernel");
+    if (t < full) {
+        load(std::integral_constant<int, 1>{}, t + 1);
+        multiply(std::integral_constant<int, 0>{}, true);
+        a[0][0] = a[1][0]; a[0][1] = a[1][1]; b[0][0] = b[1][0]; b[0][1] = b[1][1];
     }
-    return 0;
+    if (k4 % 8) multiply(std::integral_constant<int, 0>{}, H == 0);      // a group whose upper four channels are not chained
+    v16f acc;
+    const int m8 = g.cout / 8 * 8;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int row = rf * 32 + 8 * (r / 4) + 4 * H + r % 4;
+        const float s01 = s[0][r] + s[1][r], s23 = s[2][r] + s[3][r];
+        acc[r] = row < m8 ? (0.f + s01) + s23 : (s01 + s[2][r]) + s[3][r];
+    }
+    for (int k = k4; k < g.c; k += 2) {                      // channels k and k + 1, one per half
+        const int kk = k + H, at = kk / 8 * 256 + (kk % 2) * 128 + (kk % 8) / 2 - 2 * H;
+        const bool live = kk < g.c;
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(live ? ua[live ? at : 0] : -0.f, live ? vb[live ? at : 0] : 0.f, acc, 0, 0, 0);
+    }
+    float *dst = m + (int64_t(f) * g.cout + rf * 32) * g.cols + cf * 32 + lane % 32;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int row = 8 * (r / 4) + 4 * H + r % 4;
+        if (rf * 32 + row < g.cout) dst[int64_t(row) * g.cols] = acc[r];
+    }
 }
 
-// One thread per (image, cout, tile): Y = A^T M A, cut to the true output, then the optional
-// add_bias / activation that follow the convolution in the graph.
+template <int FN>
+__global__ __launch_bounds__(256) void wino_gemm_kernel(const float *__restrict__ u, const float *__restrict__ v, float *__restrict__ m, WinoGeom g,
+                                                       int row_blocks, int col_blocks) {
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int per_f = row_blocks * (col_blocks + g.nfrags - g.mfrags);
+    const int slot = blockIdx.x >> 3;
+    const int f = (blockIdx.x & 7) + 8 * (slot / per_f);     // frequencies are a multiple of 8, so is the grid
+    const int item = slot % per_f, cb = item / row_blocks;
+    const int rf = (item % row_blocks) * 4 + wave;
+    if (rf >= g.rfrags) return;
+    if (cb < col_blocks)
+        wino_gemm_chain<FN>(reinterpret_cast<const v4f *>(u), reinterpret_cast<const v4f *>(v), m, g, f, rf, cb * FN, lane);
+    else
+        wino_gemm_tail(u, v, m, g, f, rf, g.mfrags + cb - col_blocks, lane);
+}
+
+// Y = A^T M A of F(6,3), cut to the true output, then the optional add_bias / activation that follow the convolution in
+// the graph.  Workgroup = 32 columns x WT_CH output channels, thread (i, column): row i of M's 8x8 first, the 8x6
+// intermediate crosses through LDS, then column i (i < 6).
 // MISH: whether the activation may be Mish (see apply_act_basic for why that is a compile-time matter here)
 template <bool MISH>
 __global__ __launch_bounds__(256) void wino_output_transform_kernel(const float *__restrict__ mm, WinoGeom g,
                                                                    const float *__restrict__ bias, int act,
                                                                    float slope, int64_t act_body,
                                                                    float *__restrict__ out) {
-    const int64_t total = int64_t(g.n) * g.cout * g.tiles;
-    const int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (id >= total) return;
-    const int tile = int(id % g.tiles);
-    const int co = int((id / g.tiles) % g.cout);
-    const int img = int(id / g.tiles / g.cout);
-    const int ty = tile / g.tw, tx = tile - ty * g.tw;
-    const float *src = mm + (int64_t(img) * 64 * g.cout + co) * g.tiles + tile;
-    const int64_t stride = int64_t(g.cout) * g.tiles;
-    float tmpa[8][6];
+    __shared__ float half[WT_CH][8][6][32];
+    const int i = threadIdx.x / 32, lc = threadIdx.x % 32;
+    const int col = blockIdx.x * 32 + lc, co0 = blockIdx.y * WT_CH;
+    const int64_t stride = int64_t(g.cout) * g.cols;
+    float t8[WT_CH][8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        float t8[8];
+    for (int q = 0; q < WT_CH; ++q) {
+        const float *src = mm + int64_t(min(co0 + q, g.cout - 1)) * g.cols + col;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) t8[j] = src[(i * 8 + j) * stride];
-        at_pass(t8, tmpa[i]);
+        for (int j = 0; j < 8; ++j) t8[q][j] = src[(i * 8 + j) * stride];
     }
-    const float bv = bias ? bias[co] : 0.f;
-    float *dst = out + (int64_t(img) * g.cout + co) * g.ho * g.wo;
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        float t8[8], o[6];
+    for (int q = 0; q < WT_CH; ++q) {
+        float o[6];
+        at_pass(t8[q], o);
 #pragma unroll
-        for (int r = 0; r < 8; ++r) t8[r] = tmpa[r][i];
-        at_pass(t8, o);
-        const int ww = tx * 6 + i;
+        for (int j = 0; j < 6; ++j) half[q][i][j][lc] = o[j];
+    }
+    __syncthreads();
+    int img, tile;
+    if (i >= 6 || !column_tile(g, col, img, tile)) return;
+    const int ty = tile / g.tw, tx = tile - ty * g.tw;
+    const int ww = tx * 6 + i;
+#pragma unroll
+    for (int q = 0; q < WT_CH; ++q) {
+        const int co = co0 + q;
+        if (co >= g.cout) return;
+        float tt[8], o[6];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) tt[r] = half[q][r][i][lc];
+        at_pass(tt, o);
+        const float bv = bias ? bias[co] : 0.f;
+        const int64_t plane = (int64_t(img) * g.cout + co) * g.ho * g.wo;
 #pragma unroll
         for (int r = 0; r < 6; ++r) {
             const int hh = ty * 6 + r;
             if (hh < g.ho && ww < g.wo) {
                 float val = o[r];
                 if (bias) val = __fadd_rn(val, bv);
-                const int64_t idx = (int64_t(img) * g.cout + co) * g.ho * g.wo + hh * g.wo + ww;
-                dst[hh * g.wo + ww] = MISH ? apply_act(val, act, slope, idx < act_body) : apply_act_basic(val, act, slope, idx < act_body);
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------- F(6,3), fast path
-// The same algorithm on the fp32 MFMA, for callers that hold the path to its floating-point tolerance rather than
-// to its bits (the MFMA sums the channel products in another order than the reference's FMA chains): the input
-// transform kernel above, then ONE kernel for the 64 frequency GEMMs and the output transform -- M never exists in
-// memory.  A workgroup owns 16 tiles x 16 output channels and all 64 frequencies; wavefront w multiplies
-// frequencies 16w .. 16w+15 on v_mfma_f32_16x16x4_f32 with both operands loaded from global memory (L2: U and V
-// are a few MB) straight into the MFMA operand registers, four 16-channel blocks in flight: lane l holds
-// U_f[cout l%16][4 consecutive channels of group l/16] as one 16-byte load and V_f[those channels][tile l%16]; the
-// four MFMAs of a block take the channels group by group (a sum does not care which k a step carries).
-// Accumulator register r of lane l is output channel 4*(l/16) + r, tile l%16.  The 64 products of every (output
-// channel, tile) then go through LDS to one thread, which applies A^T M A, bias and activation and stores the 6x6
-// outputs.
-constexpr int WF_TILES = 16, WF_COUT = 16;
-constexpr int WF_DEPTH = 4;   // ring of 16-channel blocks per wavefront: WF_DEPTH - 1 in flight
-
-typedef float wf_v4f __attribute__((ext_vector_type(4)));
-
-// BLOCKS = C / 16 when C is 64, 128 or 256 (then the whole walk over frequencies and channel blocks is unrolled
-// around a 16-slot ring, 15 blocks in flight: with one wavefront per SIMD nothing else hides an L2 round trip),
-// 0 for any other channel count (rounds of WF_DEPTH blocks per frequency).
-template <int BLOCKS, bool MISH>
-__global__ __launch_bounds__(256) void wino_f63_gemm_output_kernel(const float *__restrict__ v, const float *__restrict__ u,
-                                                                  WinoGeom g, const float *__restrict__ bias, int act, float slope,
-                                                                  int64_t act_body, float *__restrict__ out) {
-    __shared__ float ms[64 * WF_COUT * WF_TILES];           // M[f][cout][tile]
-    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-    const int total_tiles = g.n * g.tiles;
-    const int t0 = blockIdx.x * WF_TILES, co0 = blockIdx.y * WF_COUT;
-    // operand rows / columns of this lane (beyond the edge: the last one again; computed, never stored)
-    const int a_co = min(co0 + lane % 16, g.cout - 1);
-    const int b_t = min(t0 + lane % 16, total_tiles - 1);
-    const int b_img = b_t / g.tiles, b_tile = b_t - b_img * g.tiles;
-    const int kgrp = (lane / 16) * 4;
-    const bool a_vec = g.c % 4 == 0 && reinterpret_cast<uintptr_t>(u) % 16 == 0;
-    wf_v4f acc[16];
-#pragma unroll
-    for (int f = 0; f < 16; ++f) acc[f] = wf_v4f{0.f, 0.f, 0.f, 0.f};
-    if constexpr (BLOCKS > 0) {
-        constexpr int RING = 16, STEPS = 16 * BLOCKS;
-        float av[RING][4], bv[RING][4];
-        auto load = [&](auto stepc) __attribute__((always_inline)) {
-            constexpr int step = decltype(stepc)::value;
-            constexpr int s = step % RING;
-            const int f = wave * 16 + step / BLOCKS, k0 = (step % BLOCKS) * 16 + kgrp;
-            const wf_v4f t = *reinterpret_cast<const wf_v4f *>(u + (int64_t(f) * g.cout + a_co) * g.c + k0);
-            static_for<0, 4>([&](auto ic) { av[s][decltype(ic)::value] = t[decltype(ic)::value]; });
-            const float *bp = v + ((int64_t(b_img) * 64 + f) * g.c + k0) * g.tiles + b_tile;
-            static_for<0, 4>([&](auto ic) {
-                constexpr int i = decltype(ic)::value;
-                bv[s][i] = bp[int64_t(i) * g.tiles];
-            });
-        };
-        static_for<0, RING - 1>([&](auto sc) { load(sc); });
-        static_for<0, STEPS>([&](auto stepc) {
-            constexpr int step = decltype(stepc)::value;
-            if constexpr (step + RING - 1 < STEPS) load(std::integral_constant<int, step + RING - 1>{});
-            static_for<0, 4>([&](auto ic) {
-                constexpr int i = decltype(ic)::value;
-                acc[step / BLOCKS] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[step % RING][i], bv[step % RING][i], acc[step / BLOCKS], 0, 0, 0);
-            });
-        });
-    } else {
-    // 16-channel blocks per frequency, rounded up to whole rounds of the ring (blocks beyond C multiply zeros)
-    const int blocks = (g.c + 16 * WF_DEPTH - 1) / (16 * WF_DEPTH) * WF_DEPTH;
-    const int steps = 16 * blocks;            // (frequency, block) pairs of this wavefront, frequency-major
-
-    float av[WF_DEPTH][4], bv[WF_DEPTH][4];
-    // unconditional loads from clamped addresses; what lies beyond C is zeroed where the block is used
-    auto load = [&](auto slot, int step) __attribute__((always_inline)) {
-        constexpr int s = decltype(slot)::value;
-        if (step >= steps) step = steps - 1;
-        const int f = wave * 16 + step / blocks, k0 = (step % blocks) * 16 + kgrp;
-        const float *ap = u + (int64_t(f) * g.cout + a_co) * g.c;
-        const float *bp = v + ((int64_t(b_img) * 64 + f) * g.c) * g.tiles + b_tile;
-        if (a_vec) {
-            const wf_v4f t = *reinterpret_cast<const wf_v4f *>(ap + max(0, min(k0, g.c - 4)));
-            static_for<0, 4>([&](auto ic) { av[s][decltype(ic)::value] = t[decltype(ic)::value]; });
-        } else {
-            static_for<0, 4>([&](auto ic) {
-                constexpr int i = decltype(ic)::value;
-                av[s][i] = ap[min(k0 + i, g.c - 1)];
-            });
-        }
-        static_for<0, 4>([&](auto ic) {
-            constexpr int i = decltype(ic)::value;
-            bv[s][i] = bp[int64_t(min(k0 + i, g.c - 1)) * g.tiles];
-        });
-    };
-
-    static_for<0, WF_DEPTH - 1>([&](auto sc) { load(sc, decltype(sc)::value); });
-    int step = 0;
-    static_for<0, 16>([&](auto fc) {
-        constexpr int fl = decltype(fc)::value;
-        for (int blk = 0; blk < blocks; blk += WF_DEPTH) {
-            static_for<0, WF_DEPTH>([&](auto uc) {
-                constexpr int uu = decltype(uc)::value;       // = step % WF_DEPTH: every frequency starts a round
-                load(std::integral_constant<int, (uu + WF_DEPTH - 1) % WF_DEPTH>{}, step + WF_DEPTH - 1);
-                const int k0 = (blk + uu) * 16 + kgrp;
-                static_for<0, 4>([&](auto ic) {
-                    constexpr int i = decltype(ic)::value;
-                    const bool ok = k0 + i < g.c;
-                    acc[fl] = __builtin_amdgcn_mfma_f32_16x16x4f32(ok ? av[uu][i] : 0.f, ok ? bv[uu][i] : 0.f, acc[fl], 0, 0, 0);
-                });
-                ++step;
-            });
-        }
-    });
-    }
-
-    // ---- M[f][cout][tile] into LDS, then one thread per (cout, tile)
-#pragma unroll
-    for (int fl = 0; fl < 16; ++fl) {
-        const int f = wave * 16 + fl;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) ms[(f * WF_COUT + 4 * (lane / 16) + r) * WF_TILES + lane % 16] = acc[fl][r];
-    }
-    __syncthreads();
-    const int co = co0 + tid / WF_TILES;
-    const int my_t = t0 + tid % WF_TILES;
-    if (my_t >= total_tiles || co >= g.cout) return;
-    const int my_img = my_t / g.tiles, my_tile = my_t - my_img * g.tiles;
-    const int my_ty = my_tile / g.tw, my_tx = my_tile - my_ty * g.tw;
-    float tmpa[8][6];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        float t8[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) t8[j] = ms[((i * 8 + j) * WF_COUT + tid / WF_TILES) * WF_TILES + tid % WF_TILES];
-        at_pass(t8, tmpa[i]);
-    }
-    const float bvv = bias ? bias[co] : 0.f;
-    const int64_t plane = (int64_t(my_img) * g.cout + co) * g.ho * g.wo;
-#pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        float t8[8], o[6];
-#pragma unroll
-        for (int r = 0; r < 8; ++r) t8[r] = tmpa[r][i];
-        at_pass(t8, o);
-        const int ww = my_tx * 6 + i;
-#pragma unroll
-        for (int r = 0; r < 6; ++r) {
-            const int hh = my_ty * 6 + r;
-            if (hh < g.ho && ww < g.wo) {
-                float val = o[r];
-                if (bias) val = __fadd_rn(val, bvv);
                 const int64_t idx = plane + hh * g.wo + ww;
                 out[idx] = MISH ? apply_act(val, act, slope, idx < act_body) : apply_act_basic(val, act, slope, idx < act_body);
             }
@@ -493,88 +469,19 @@ __global__ __launch_bounds__(256) void wino_f63_gemm_output_kernel(const float *
     }
 }
 
-// ---------------------------------------------------------------- F(2,3)
-
-// U[t = i*4+j][cout][cin] = (G g G^T)[i][j], G = {1,0,0; 1/2,1/2,1/2; 1/2,-1/2,1/2; 0,0,1}
-// (winograd_algorithm.cpp:57-105, before its pack8_A); same contraction as the F(6,3) transform.
-__global__ __launch_bounds__(256) void wino23_kernel_transform_kernel(const float *__restrict__ w, int cout, int cin,
-                                                                     float *__restrict__ u) {
-    const int id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= cout * cin) return;
-    const float G[4][3] = {{1.f, 0.f, 0.f}, {0.5f, 0.5f, 0.5f}, {0.5f, -0.5f, 0.5f}, {0.f, 0.f, 1.f}};
-    float g[9];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) g[i] = w[int64_t(id) * 9 + i];
-    float tmp[3][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-            tmp[r][i] = fmaf(g[r * 3 + 2], G[i][2], fmaf(g[r * 3 + 0], G[i][0], g[r * 3 + 1] * G[i][1]));
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            u[int64_t(i * 4 + j) * cout * cin + id] =
-                fmaf(tmp[2][j], G[i][2], fmaf(tmp[0][j], G[i][0], tmp[1][j] * G[i][1]));
-}
-
-// V = B^T d B (winograd_algorithm.cpp:181-243): row combinations (i0-i2, i1+i2, i2-i1, i1-i3) first,
-// then the same combination across columns, in the reference's grouping.
-__global__ __launch_bounds__(256) void wino23_input_transform_kernel(const float *__restrict__ x, WinoGeom g,
-                                                                    float *__restrict__ v) {
-    const int64_t total = int64_t(g.n) * g.c * g.tiles;
-    const int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (id >= total) return;
-    const int tile = int(id % g.tiles);
-    const int ch = int((id / g.tiles) % g.c);
-    const int img = int(id / g.tiles / g.c);
-    const int ty = tile / g.tw, tx = tile - ty * g.tw;
-    const float *src = x + (int64_t(img) * g.c + ch) * g.h * g.w;
-    float d[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int hh = ty * 2 + i - g.pad_top;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int ww = tx * 2 + j - g.pad_left;
-            d[i][j] = (hh >= 0 && hh < g.h && ww >= 0 && ww < g.w) ? src[hh * g.w + ww] : g.padding_value;
-        }
-    }
-    float *dst = v + (int64_t(img) * 16 * g.c + ch) * g.tiles + tile;
-    const int64_t stride = int64_t(g.c) * g.tiles;
-    float r[4][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        r[0][j] = d[0][j] - d[2][j];
-        r[1][j] = d[1][j] + d[2][j];
-        r[2][j] = d[2][j] - d[1][j];
-        r[3][j] = d[1][j] - d[3][j];
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        dst[(k * 4 + 0) * stride] = r[k][0] - r[k][2];
-        dst[(k * 4 + 1) * stride] = r[k][1] + r[k][2];
-        dst[(k * 4 + 2) * stride] = r[k][2] - r[k][1];
-        dst[(k * 4 + 3) * stride] = r[k][1] - r[k][3];
-    }
-}
-
-// Y = A^T M A (winograd_algorithm.cpp:262-330), cut to the true output, + optional bias / activation.
+// Y of F(2,3) (winograd_algorithm.cpp:262-330), cut to the true output, + optional bias / activation.  Thread = one
+// column of one output channel.
 template <bool MISH>
 __global__ __launch_bounds__(256) void wino23_output_transform_kernel(const float *__restrict__ mm, WinoGeom g,
                                                                      const float *__restrict__ bias, int act,
                                                                      float slope, int64_t act_body,
                                                                      float *__restrict__ out) {
-    const int64_t total = int64_t(g.n) * g.cout * g.tiles;
-    const int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (id >= total) return;
-    const int tile = int(id % g.tiles);
-    const int co = int((id / g.tiles) % g.cout);
-    const int img = int(id / g.tiles / g.cout);
+    const int col = blockIdx.x * 256 + threadIdx.x, co = blockIdx.y;
+    int img, tile;
+    if (col >= g.cols || !column_tile(g, col, img, tile)) return;
     const int ty = tile / g.tw, tx = tile - ty * g.tw;
-    const float *src = mm + (int64_t(img) * 16 * g.cout + co) * g.tiles + tile;
-    const int64_t stride = int64_t(g.cout) * g.tiles;
+    const float *src = mm + int64_t(co) * g.cols + col;
+    const int64_t stride = int64_t(g.cout) * g.cols;
     float m[16], a[8], o[4];
 #pragma unroll
     for (int t = 0; t < 16; ++t) m[t] = src[t * stride];
@@ -603,7 +510,7 @@ __global__ __launch_bounds__(256) void wino23_output_transform_kernel(const floa
         }
 }
 
-int make_geom(const tsx_conv2d_geom *q, float padding_value, WinoGeom *g, int tile = 6) {
+int make_geom(const tsx_conv2d_geom *q, float padding_value, WinoGeom *g, int tile) {
     TSX_REQUIRE(q, "winograd: null geometry");
     TSX_REQUIRE(q->kh == 3 && q->kw == 3 && q->stride_h == 1 && q->stride_w == 1 && q->dilation_h == 1 &&
                     q->dilation_w == 1,
@@ -623,8 +530,89 @@ int make_geom(const tsx_conv2d_geom *q, float padding_value, WinoGeom *g, int ti
     g->pad_left = q->pad_left;
     g->th = (g->ho + tile - 1) / tile;
     g->tw = (g->wo + tile - 1) / tile;
+    TSX_REQUIRE(int64_t(g->n) * g->th * g->tw < (int64_t(1) << 30), "winograd: too many tiles");
     g->tiles = g->th * g->tw;
     g->padding_value = padding_value;
+    g->rfrags = (q->cout + 31) / 32;
+    g->kgroups = (q->c + 7) / 8;
+    g->n8 = g->tiles / 8 * 8;
+    g->mfrags = int(ceil_div(int64_t(g->n) * g->n8, 32));
+    g->nfrags = g->mfrags + int(ceil_div(int64_t(g->n) * (g->tiles - g->n8), 32));
+    g->cols = 32 * g->nfrags;
+    return 0;
+}
+
+size_t kernel_bytes(int cout, int cin, int freqs) {
+    if (cout <= 0 || cin <= 0) return 0;
+    return size_t(freqs) * size_t(round_up(cout, 32)) * size_t(round_up(cin, 8)) * sizeof(float);
+}
+
+size_t operand_floats(const WinoGeom &g, int freqs) { return size_t(freqs) * g.nfrags * g.kgroups * 256; }     // V
+
+size_t workspace_bytes(const tsx_conv2d_geom *q, int tile) {
+    WinoGeom g;
+    if (make_geom(q, 0.f, &g, tile)) return 0;
+    const int freqs = (tile + 2) * (tile + 2);
+    return (operand_floats(g, freqs) + size_t(freqs) * g.cout * g.cols) * sizeof(float);
+}
+
+template <int TILE>
+int transform_kernel(int cout, int cin, const float *w, float *u, hipStream_t stream) {
+    TSX_REQUIRE(cout > 0 && cin > 0 && w && u, "winograd transform_kernel: bad argument");
+    const int rfrags = (cout + 31) / 32, kgroups = (cin + 7) / 8;
+    hipLaunchKernelGGL(wino_kernel_transform_kernel<TILE>, dim3(unsigned(rfrags) * unsigned(kgroups)), dim3(256), 0, stream, w, cout, cin, rfrags,
+                       kgroups, u);
+    TSX_LAUNCH_CHECK("wino_kernel_transform_kernel");
+    return 0;
+}
+
+template <int TILE>
+int conv2d(const tsx_conv2d_geom *q, const float *x, const float *u, float padding_value, const float *bias, int act, float slope,
+           float *out, void *workspace, size_t bytes, hipStream_t stream) {
+    WinoGeom g;
+    if (int rc = make_geom(q, padding_value, &g, TILE)) return rc;
+    TSX_REQUIRE(x && u && out, "winograd: null argument");
+    TSX_REQUIRE(act >= TSX_ACT_NONE && act <= TSX_ACT_MISH_FAST, "winograd: unknown activation %d", act);
+    constexpr int FREQS = (TILE + 2) * (TILE + 2);
+    const size_t need = workspace_bytes(q, TILE);
+    if (!workspace || bytes < need) return fail(TSX_E_WORKSPACE, "winograd: workspace %zu < %zu bytes", bytes, need);
+    TSX_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && reinterpret_cast<uintptr_t>(u) % 16 == 0,
+                "winograd: workspace and transformed kernel must be 16-byte aligned");
+    TSX_REQUIRE(g.cout <= 65535 * WT_CH && g.kgroups <= 32767, "winograd: too many channels");
+    float *v = static_cast<float *>(workspace), *m = v + operand_floats(g, FREQS);
+    if (TILE == 6)
+        hipLaunchKernelGGL(wino_input_transform_kernel, dim3(unsigned(g.nfrags), unsigned(2 * g.kgroups)), dim3(256), 0, stream, x, g, v);
+    else
+        hipLaunchKernelGGL(wino23_input_transform_kernel, dim3(unsigned(g.nfrags), unsigned(ceil_div(2 * g.kgroups, 8))), dim3(256), 0, stream, x,
+                           g, v);
+    TSX_LAUNCH_CHECK("wino_input_transform_kernel");
+
+    // two column fragments per wavefront halve the loads of U; with fewer than two wavefronts per SIMD (a small layer) one
+    // fragment each spreads the chains over twice the wavefronts
+    const int row_blocks = (g.rfrags + 3) / 4, tails = g.nfrags - g.mfrags;
+    const bool two = int64_t(FREQS) * g.rfrags * ((g.mfrags + 1) / 2) >= 2048;
+    const int col_blocks = two ? (g.mfrags + 1) / 2 : g.mfrags;
+    const int64_t blocks = int64_t(FREQS) * row_blocks * (col_blocks + tails);
+    TSX_REQUIRE(blocks < (int64_t(1) << 31), "winograd: tensor too large");
+    if (two)
+        hipLaunchKernelGGL(wino_gemm_kernel<2>, dim3(unsigned(blocks)), dim3(256), 0, stream, u, v, m, g, row_blocks, col_blocks);
+    else
+        hipLaunchKernelGGL(wino_gemm_kernel<1>, dim3(unsigned(blocks)), dim3(256), 0, stream, u, v, m, g, row_blocks, col_blocks);
+    TSX_LAUNCH_CHECK("wino_gemm_kernel");
+
+    const int64_t body = int64_t(g.n) * g.cout * g.ho * g.wo / 4 * 4;
+    const bool mish = act >= TSX_ACT_MISH;
+    if (TILE == 6) {
+        const dim3 grid(unsigned(g.nfrags), unsigned(ceil_div(g.cout, WT_CH)));
+        if (mish) hipLaunchKernelGGL(wino_output_transform_kernel<true>, grid, dim3(256), 0, stream, m, g, bias, act, slope, body, out);
+        else hipLaunchKernelGGL(wino_output_transform_kernel<false>, grid, dim3(256), 0, stream, m, g, bias, act, slope, body, out);
+    } else {
+        TSX_REQUIRE(g.cout <= 65535, "winograd: too many output channels");
+        const dim3 grid(unsigned(ceil_div(g.cols, 256)), unsigned(g.cout));
+        if (mish) hipLaunchKernelGGL(wino23_output_transform_kernel<true>, grid, dim3(256), 0, stream, m, g, bias, act, slope, body, out);
+        else hipLaunchKernelGGL(wino23_output_transform_kernel<false>, grid, dim3(256), 0, stream, m, g, bias, act, slope, body, out);
+    }
+    TSX_LAUNCH_CHECK("wino_output_transform_kernel");
     return 0;
 }
 
@@ -633,156 +621,41 @@ int make_geom(const tsx_conv2d_geom *q, float padding_value, WinoGeom *g, int ti
 
 extern "C" {
 
-size_t tsx_winograd_f63_kernel_bytes(int32_t cout, int32_t cin) {
-    if (cout <= 0 || cin <= 0) return 0;
-    return size_t(64) * size_t(cout) * size_t(cin) * sizeof(float);
-}
+size_t tsx_winograd_f63_kernel_bytes(int32_t cout, int32_t cin) { return tsx::kernel_bytes(cout, cin, 64); }
 
 int tsx_winograd_f63_transform_kernel(int32_t cout, int32_t cin, const float *w_oihw_dev, float *u_dev, void *stream) {
-    TSX_REQUIRE(cout > 0 && cin > 0 && w_oihw_dev && u_dev, "winograd_f63_transform_kernel: bad argument");
-    const int total = cout * cin;
-    hipLaunchKernelGGL(tsx::wino_kernel_transform_kernel, dim3(unsigned(tsx::ceil_div(total, 256))), dim3(256), 0,
-                       tsx::as_stream(stream), w_oihw_dev, cout, cin, u_dev);
-    TSX_LAUNCH_CHECK("wino_kernel_transform_kernel");
-    return 0;
+    return tsx::transform_kernel<6>(cout, cin, w_oihw_dev, u_dev, tsx::as_stream(stream));
 }
 
-size_t tsx_winograd_f63_workspace_bytes(const tsx_conv2d_geom *q) {
-    tsx::WinoGeom g;
-    if (tsx::make_geom(q, 0.f, &g)) return 0;
-    return size_t(g.n) * 64 * g.tiles * (size_t(g.c) + size_t(g.cout)) * sizeof(float);
-}
+size_t tsx_winograd_f63_workspace_bytes(const tsx_conv2d_geom *q) { return tsx::workspace_bytes(q, 6); }
 
 int tsx_conv2d_winograd_f63_nchw(const tsx_conv2d_geom *q, const float *x_dev, const float *u_dev, float padding_value,
                                  const float *bias_dev, int32_t act, float slope, float *out_dev, void *workspace_dev,
                                  size_t workspace_bytes, void *stream_) {
-    tsx::WinoGeom g;
-    int rc = tsx::make_geom(q, padding_value, &g);
-    if (rc) return rc;
-    TSX_REQUIRE(x_dev && u_dev && out_dev, "winograd: null argument");
-    TSX_REQUIRE(act >= TSX_ACT_NONE && act <= TSX_ACT_MISH_FAST, "winograd: unknown activation %d", act);
-    const size_t need = tsx_winograd_f63_workspace_bytes(q);
-    if (!workspace_dev || workspace_bytes < need)
-        return tsx::fail(TSX_E_WORKSPACE, "winograd: workspace %zu < %zu bytes", workspace_bytes, need);
-    hipStream_t stream = tsx::as_stream(stream_);
-    float *v = static_cast<float *>(workspace_dev);
-    float *mm = v + size_t(g.n) * 64 * g.c * g.tiles;
-
-    const int64_t in_threads = int64_t(g.n) * g.c * g.tiles;
-    hipLaunchKernelGGL(tsx::wino_input_transform_kernel, dim3(unsigned(tsx::ceil_div(in_threads, 256))), dim3(256), 0,
-                       stream, x_dev, g, v);
-    TSX_LAUNCH_CHECK("wino_input_transform_kernel");
-
-    const int batches = g.n * 64;
-    if (int rc = tsx::launch_gemm_f32_seq(u_dev, v, mm, g.cout, g.tiles, g.c, batches, 64, stream)) return rc;
-
-    const int64_t out_threads = int64_t(g.n) * g.cout * g.tiles;
-    const int64_t count = int64_t(g.n) * g.cout * g.ho * g.wo;
-    if (act >= TSX_ACT_MISH)
-        hipLaunchKernelGGL(tsx::wino_output_transform_kernel<true>, dim3(unsigned(tsx::ceil_div(out_threads, 256))), dim3(256), 0,
-                           stream, mm, g, bias_dev, act, slope, count / 4 * 4, out_dev);
-    else
-        hipLaunchKernelGGL(tsx::wino_output_transform_kernel<false>, dim3(unsigned(tsx::ceil_div(out_threads, 256))), dim3(256), 0,
-                           stream, mm, g, bias_dev, act, slope, count / 4 * 4, out_dev);
-    TSX_LAUNCH_CHECK("wino_output_transform_kernel");
-    return 0;
+    return tsx::conv2d<6>(q, x_dev, u_dev, padding_value, bias_dev, act, slope, out_dev, workspace_dev, workspace_bytes, tsx::as_stream(stream_));
 }
 
-size_t tsx_winograd_f63_fast_workspace_bytes(const tsx_conv2d_geom *q) {
-    tsx::WinoGeom g;
-    if (tsx::make_geom(q, 0.f, &g)) return 0;
-    return size_t(g.n) * 64 * g.tiles * size_t(g.c) * sizeof(float);
-}
+// The tolerance-based entry: the exact form is the fastest there is.
+size_t tsx_winograd_f63_fast_workspace_bytes(const tsx_conv2d_geom *q) { return tsx::workspace_bytes(q, 6); }
 
 int tsx_conv2d_winograd_f63_fast_nchw(const tsx_conv2d_geom *q, const float *x_dev, const float *u_dev, float padding_value,
                                       const float *bias_dev, int32_t act, float slope, float *out_dev, void *workspace_dev,
                                       size_t workspace_bytes, void *stream_) {
-    tsx::WinoGeom g;
-    int rc = tsx::make_geom(q, padding_value, &g);
-    if (rc) return rc;
-    TSX_REQUIRE(x_dev && u_dev && out_dev, "winograd: null argument");
-    TSX_REQUIRE(act >= TSX_ACT_NONE && act <= TSX_ACT_MISH_FAST, "winograd: unknown activation %d", act);
-    const size_t need = tsx_winograd_f63_fast_workspace_bytes(q);
-    if (!workspace_dev || workspace_bytes < need)
-        return tsx::fail(TSX_E_WORKSPACE, "winograd: workspace %zu < %zu bytes", workspace_bytes, need);
-    const int64_t total_tiles = int64_t(g.n) * g.tiles;
-    TSX_REQUIRE(total_tiles < (int64_t(1) << 31) - tsx::WF_TILES, "winograd: too many tiles");
-    hipStream_t stream = tsx::as_stream(stream_);
-    float *v = static_cast<float *>(workspace_dev);
-    const int64_t in_threads = int64_t(g.n) * g.c * g.tiles;
-    hipLaunchKernelGGL(tsx::wino_input_transform_kernel, dim3(unsigned(tsx::ceil_div(in_threads, 256))), dim3(256), 0,
-                       stream, x_dev, g, v);
-    TSX_LAUNCH_CHECK("wino_input_transform_kernel");
-    const int64_t count = int64_t(g.n) * g.cout * g.ho * g.wo;
-    const dim3 grid(unsigned(tsx::ceil_div(total_tiles, int64_t(tsx::WF_TILES))), unsigned(tsx::ceil_div(g.cout, tsx::WF_COUT)));
-    const bool aligned = reinterpret_cast<uintptr_t>(u_dev) % 16 == 0;
-    const int blocks = aligned && (g.c == 64 || g.c == 128 || g.c == 256) ? g.c / 16 : 0;
-    const bool mish = act >= TSX_ACT_MISH;
-#define TSX_WF_LAUNCH(B, M)                                                                                         \
-    hipLaunchKernelGGL((tsx::wino_f63_gemm_output_kernel<B, M>), grid, dim3(256), 0, stream, v, u_dev, g, bias_dev, act, \
-                       slope, count / 4 * 4, out_dev)
-    if (blocks == 4) { if (mish) TSX_WF_LAUNCH(4, true); else TSX_WF_LAUNCH(4, false); }
-    else if (blocks == 8) { if (mish) TSX_WF_LAUNCH(8, true); else TSX_WF_LAUNCH(8, false); }
-    else if (blocks == 16) { if (mish) TSX_WF_LAUNCH(16, true); else TSX_WF_LAUNCH(16, false); }
-    else { if (mish) TSX_WF_LAUNCH(0, true); else TSX_WF_LAUNCH(0, false); }
-#undef TSX_WF_LAUNCH
-    TSX_LAUNCH_CHECK("wino_f63_gemm_output_kernel");
-    return 0;
+    return tsx::conv2d<6>(q, x_dev, u_dev, padding_value, bias_dev, act, slope, out_dev, workspace_dev, workspace_bytes, tsx::as_stream(stream_));
 }
 
-size_t tsx_winograd_f23_kernel_bytes(int32_t cout, int32_t cin) {
-    if (cout <= 0 || cin <= 0) return 0;
-    return size_t(16) * size_t(cout) * size_t(cin) * sizeof(float);
-}
+size_t tsx_winograd_f23_kernel_bytes(int32_t cout, int32_t cin) { return tsx::kernel_bytes(cout, cin, 16); }
 
 int tsx_winograd_f23_transform_kernel(int32_t cout, int32_t cin, const float *w_oihw_dev, float *u_dev, void *stream) {
-    TSX_REQUIRE(cout > 0 && cin > 0 && w_oihw_dev && u_dev, "winograd_f23_transform_kernel: bad argument");
-    const int total = cout * cin;
-    hipLaunchKernelGGL(tsx::wino23_kernel_transform_kernel, dim3(unsigned(tsx::ceil_div(total, 256))), dim3(256), 0,
-                       tsx::as_stream(stream), w_oihw_dev, cout, cin, u_dev);
-    TSX_LAUNCH_CHECK("wino23_kernel_transform_kernel");
-    return 0;
+    return tsx::transform_kernel<2>(cout, cin, w_oihw_dev, u_dev, tsx::as_stream(stream));
 }
 
-size_t tsx_winograd_f23_workspace_bytes(const tsx_conv2d_geom *q) {
-    tsx::WinoGeom g;
-    if (tsx::make_geom(q, 0.f, &g, 2)) return 0;
-    return size_t(g.n) * 16 * g.tiles * (size_t(g.c) + size_t(g.cout)) * sizeof(float);
-}
+size_t tsx_winograd_f23_workspace_bytes(const tsx_conv2d_geom *q) { return tsx::workspace_bytes(q, 2); }
 
 int tsx_conv2d_winograd_f23_nchw(const tsx_conv2d_geom *q, const float *x_dev, const float *u_dev, float padding_value,
                                  const float *bias_dev, int32_t act, float slope, float *out_dev, void *workspace_dev,
                                  size_t workspace_bytes, void *stream_) {
-    tsx::WinoGeom g;
-    int rc = tsx::make_geom(q, padding_value, &g, 2);
-    if (rc) return rc;
-    TSX_REQUIRE(x_dev && u_dev && out_dev, "winograd_f23: null argument");
-    TSX_REQUIRE(act >= TSX_ACT_NONE && act <= TSX_ACT_MISH_FAST, "winograd_f23: unknown activation %d", act);
-    const size_t need = tsx_winograd_f23_workspace_bytes(q);
-    if (!workspace_dev || workspace_bytes < need)
-        return tsx::fail(TSX_E_WORKSPACE, "winograd_f23: workspace %zu < %zu bytes", workspace_bytes, need);
-    hipStream_t stream = tsx::as_stream(stream_);
-    float *v = static_cast<float *>(workspace_dev);
-    float *mm = v + size_t(g.n) * 16 * g.c * g.tiles;
-
-    const int64_t in_threads = int64_t(g.n) * g.c * g.tiles;
-    hipLaunchKernelGGL(tsx::wino23_input_transform_kernel, dim3(unsigned(tsx::ceil_div(in_threads, 256))), dim3(256), 0,
-                       stream, x_dev, g, v);
-    TSX_LAUNCH_CHECK("wino23_input_transform_kernel");
-
-    const int batches = g.n * 16;
-    if (int rc = tsx::launch_gemm_f32_seq(u_dev, v, mm, g.cout, g.tiles, g.c, batches, 16, stream)) return rc;
-
-    const int64_t out_threads = int64_t(g.n) * g.cout * g.tiles;
-    const int64_t count = int64_t(g.n) * g.cout * g.ho * g.wo;
-    if (act >= TSX_ACT_MISH)
-        hipLaunchKernelGGL(tsx::wino23_output_transform_kernel<true>, dim3(unsigned(tsx::ceil_div(out_threads, 256))), dim3(256), 0,
-                           stream, mm, g, bias_dev, act, slope, count / 4 * 4, out_dev);
-    else
-        hipLaunchKernelGGL(tsx::wino23_output_transform_kernel<false>, dim3(unsigned(tsx::ceil_div(out_threads, 256))), dim3(256), 0,
-                           stream, mm, g, bias_dev, act, slope, count / 4 * 4, out_dev);
-    TSX_LAUNCH_CHECK("wino23_output_transform_kernel");
-    return 0;
+    return tsx::conv2d<2>(q, x_dev, u_dev, padding_value, bias_dev, act, slope, out_dev, workspace_dev, workspace_bytes, tsx::as_stream(stream_));
 }
 
 }  // extern "C"
