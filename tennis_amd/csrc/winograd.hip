@@ -279,8 +279,11 @@ __global__ __launch_bounds__(256) void wino23_input_transform_kernel(const float
 // loads meet in L1).  Workgroups b, b + 8, ... run on one XCD: each XCD gets whole frequencies, whose U and V then
 // stay in its L2 (8 x 456 KB at 8 images of 28x28x256).  RING groups of 8 channels are in flight per wavefront.
 // Bound by the fp32 MFMA: 1.68 GFLOP at that shape = 11 us at 157 TFLOP/s.
-// Chains on the vector ALUs, one lane per 4 x 4 outputs, took 276 + 31 us there.
+// It takes 26 us there (the tail's
+// fragments hold 8 real columns of 32, and a wavefront's chain of 128 dependent MFMAs fills its SIMD 3.5 times over);
+// chains on the vector ALUs, one lane per 4 x 4 outputs, took 276 + 31 us.
 constexpr int WG_RING = 4;
+constexpr int TAIL_RING = 4;
 
 template <int FN>
 __device__ __forceinline__ void wino_gemm_chain(const v4f *__restrict__ u, const v4f *__restrict__ v, float *__restrict__ m, const WinoGeom &g,
@@ -316,7 +319,9 @@ __device__ __forceinline__ void wino_gemm_chain(const v4f *__restrict__ u, const
         static_for<0, WG_RING>([&](auto sc) {
             constexpr int s = decltype(sc)::value;
             load(std::integral_constant<int, (s + WG_RING - 1) % WG_RING>{}, t + s + WG_RING - 1);
+            __builtin_amdgcn_sched_barrier(0);               // left alone the scheduler sinks the loads to where they are waited for
             multiply(sc);
+            __builtin_amdgcn_sched_barrier(0);
         });
     static_for<0, WG_RING - 1>([&](auto sc) {                // the groups left over are in the ring already
         if (t + decltype(sc)::value < T) multiply(sc);
@@ -347,7 +352,7 @@ __device__ __forceinline__ void wino_gemm_tail(const float *__restrict__ u, cons
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[q][r] = 0.f;
     const int k4 = g.c / 4 * 4, full = k4 / 8;
-    v2f a[2][2], b[2][2];                                    // [slot][parity]
+    v2f a[TAIL_RING][2], b[TAIL_RING][2];                    // [slot][parity]
     auto load = [&](auto slot, int t) __attribute__((always_inline)) {
         constexpr int sl = decltype(slot)::value;
         const int64_t off = int64_t(min(t, T - 1)) * 256;
@@ -363,20 +368,23 @@ __device__ __forceinline__ void wino_gemm_tail(const float *__restrict__ u, cons
         for (int q = 0; q < 4; ++q)
             s[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(live ? a[sl][q % 2][q / 2] : -0.f, live ? b[sl][q % 2][q / 2] : 0.f, s[q], 0, 0, 0);
     };
-    load(std::integral_constant<int, 0>{}, 0);
+    static_for<0, TAIL_RING - 1>([&](auto sc) { load(sc, decltype(sc)::value); });
     int t = 0;
-    for (; t + 2 <= full; t += 2) {
-        load(std::integral_constant<int, 1>{}, t + 1);
-        multiply(std::integral_constant<int, 0>{}, true);
-        load(std::integral_constant<int, 0>{}, t + 2);
-        multiply(std::integral_constant<int, 1>{}, true);
-    }
-    if (t < full) {
-        load(std::integral_constant<int, 1>{}, t + 1);
-        multiply(std::integral_constant<int, 0>{}, true);
-        a[0][0] = a[1][0]; a[0][1] = a[1][1]; b[0][0] = b[1][0]; b[0][1] = b[1][1];
-    }
-    if (k4 % 8) multiply(std::integral_constant<int, 0>{}, H == 0);      // a group whose upper four channels are not chained
+    for (; t + TAIL_RING <= full; t += TAIL_RING)
+        static_for<0, TAIL_RING>([&](auto sc) {
+            constexpr int sl = decltype(sc)::value;
+            load(std::integral_constant<int, (sl + TAIL_RING - 1) % TAIL_RING>{}, t + sl + TAIL_RING - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(sc, true);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    // the groups left over, and behind them one whose upper four channels are not chained
+    static_for<0, TAIL_RING>([&](auto sc) {
+        constexpr int sl = decltype(sc)::value;
+        if constexpr (sl == TAIL_RING - 1) load(sc, t + sl);
+        if (t + sl < full) multiply(sc, true);
+        else if (t + sl == full && k4 % 8) multiply(sc, H == 0);
+    });
     v16f acc;
     const int m8 = g.cout / 8 * 8;
 #pragma unroll
@@ -587,8 +595,8 @@ int conv2d(const tsx_conv2d_geom *q, const float *x, const float *u, float paddi
                            g, v);
     TSX_LAUNCH_CHECK("wino_input_transform_kernel");
 
-    // two column fragments per wavefront halve the loads of U; with fewer than two wavefronts per SIMD (a small layer) one
-    // fragment each spreads the chains over twice the wavefronts
+    // two column fragments per wavefront halve the loads of U; a layer that fills the SIMDs less than twice that way takes one
+    // fragment each (8 images of 28x28x256: 41.9 us against 43.8)
     const int row_blocks = (g.rfrags + 3) / 4, tails = g.nfrags - g.mfrags;
     const bool two = int64_t(FREQS) * g.rfrags * ((g.mfrags + 1) / 2) >= 2048;
     const int col_blocks = two ? (g.mfrags + 1) / 2 : g.mfrags;
