@@ -1,10 +1,10 @@
-// fp32 GEMM-shaped kernels on the gfx950 fp32 MFMA (v_mfma_f32_32x32x2_f32):
+// fp32 GEMM-shaped kernels on the gfx950 fp32 MFMA (v_mfma_f32_32x32x2_f32), for the smallest layers and what the window
+// kernel (conv2d_f32_window.hip: every larger convolution) does not take:
 //   * conv2d as implicit im2col-GEMM straight from NCHW (no col buffer), standing in for
 //     cpu::Conv2DCore::conv2d (src/kernels/cpu/conv2d_core.cpp:17-119: im2col_cpu + pack8 +
 //     kernel_8x8 of src/kernels/cpu/math_cpu.cpp:386-743);
-//   * inner_prod, standing in for cpu::InnerProd (src/kernels/cpu/inner_prod.cpp:19-74);
-//   * the strided-batch GEMM used by the Winograd path.
-// One kernel, three ways of fetching the B operand.  C[m][n] = sum_k A[m][k] * B[k][n] with
+//   * inner_prod, standing in for cpu::InnerProd (src/kernels/cpu/inner_prod.cpp:19-74).
+// One kernel, two ways of fetching the B operand.  C[m][n] = sum_k A[m][k] * B[k][n] with
 // A row-major [M][K] (OIHW weights are exactly that with K = Cin*KH*KW), accumulated in the
 // MFMA's fp32 accumulators; the summation order differs from the reference's sequential FMA
 // chain, which the parity tolerance (1e-4 relative / 1e-5 absolute) covers.
@@ -695,27 +695,24 @@ int launch(const GemmArgs &g, const Loader &ld, int batches, hipStream_t stream)
     return 0;
 }
 
-}  // namespace
-
-int gemm_f32_batched(const float *a, int64_t a_batch, const float *b, int64_t ld_k, int64_t ld_n, int64_t b_batch,
-                     float *c, int64_t c_batch, int m, int n, int k, int batches, hipStream_t stream) {
-    GemmArgs g{};
-    g.a = a;
-    g.c = c;
-    g.m = m;
-    g.n = n;
-    g.k = k;
-    g.a_batch = a_batch;
-    g.b_batch = b_batch;
-    g.c_batch = c_batch;
-    g.howo = 0;
-    g.act = TSX_ACT_NONE;
-    MatLoader ld{};
-    ld.b = b;
-    ld.ld_k = ld_k;
-    ld.ld_n = ld_n;
-    return launch(g, ld, batches, stream);
+ConvF32Layer window_layer(const tsx_conv2d_geom *geo, const GemmArgs &g, const ConvLoader &ld) {
+    return ConvF32Layer{geo->n, geo->c, geo->h, geo->w, geo->cout, geo->kh, geo->kw, geo->pad_top, geo->pad_left, geo->stride_h, geo->stride_w,
+                        geo->dilation_h, geo->dilation_w, g.howo / ld.wo, ld.wo, ld.x, g.a};
 }
+
+// The window kernel's tile for the layer, -1 where the kernels of this file take it: tensors of 2 GiB and more, and the
+// problems of up to a quarter of a GFLOP that the register-fed kernel admits.  Up to a K of some 500 the two take the same
+// few microseconds; with more K the window kernel wins (256 channels at 28x28, 256 3x3 filters: 25 us against 41; 512 at
+// 7x7: 44 against 76), by 7 of 22 us at the far end of what stays with the register-fed one.
+int window_tile(const ConvF32Layer &layer, const GemmArgs &g) {
+    if (choose_gemm(g, 1) == GEMM_REGISTER_FED) {
+        const char *e = std::getenv("TSX_GEMM_F32_REGFED");
+        if ((e && e[0] == 'f') || ceil_div(g.m, 32) * ceil_div(g.n, 32) * g.k * 2048 < 250000000) return -1;
+    }
+    return conv_f32_window_tile(layer);
+}
+
+}  // namespace
 
 }  // namespace tsx
 
@@ -775,6 +772,10 @@ int tsx_conv2d_f32_nchw(const tsx_conv2d_geom *geo, const float *x_dev, const fl
     if (tsx::conv3x3_small_takes(g, ld))
         return geo->c <= 32 ? tsx::launch_conv3x3_small<2>(g, ld, tsx::as_stream(stream))
                             : tsx::launch_conv3x3_small<4>(g, ld, tsx::as_stream(stream));
+    const tsx::ConvF32Layer layer = tsx::window_layer(geo, g, ld);
+    const int tile = tsx::window_tile(layer, g);
+    if (tile >= 0)
+        return tsx::conv_f32_window(layer, tile, bias_dev, act, slope, padding_value, out_dev, tsx::as_stream(stream));
     return tsx::launch(g, ld, 1, tsx::as_stream(stream));
 }
 
@@ -790,6 +791,14 @@ int tsx_conv2d_f32_plan_info(const tsx_conv2d_geom *geo, const float *w_oihw_dev
         const tsx::GemmKernel k = tsx::choose_gemm(g, 1);
         name = k == tsx::GEMM_REGISTER_FED ? "register_fed" : k == tsx::GEMM_STAGED_64 ? "staged_64x64" : "staged_32x32_ksplit";
         if (k == tsx::GEMM_STAGED_64) tile = 64;
+        const int win = tsx::window_tile(tsx::window_layer(geo, g, ld), g);
+        if (win >= 0) {        // a K-split 32-row tile or a larger one without, by its input patches
+            int rows, positions;
+            tsx::conv_f32_window_tile_size(win, &rows, &positions);
+            std::snprintf(text, text_bytes, "kernel=%s tiles=%lld tile=%dx%d window=%s", rows * positions == 1024 ? "staged_32x32_ksplit" : "staged_64x64",
+                          (long long)(tsx::ceil_div(g.m, rows) * tsx::ceil_div(g.n, positions)), rows, positions, win % 2 ? "flat" : "segments");
+            return 0;
+        }
     }
     std::snprintf(text, text_bytes, "kernel=%s tiles=%lld", name,
                   (long long)(tsx::ceil_div(g.m, tile) * tsx::ceil_div(g.n, tile)));
@@ -817,6 +826,11 @@ int tsx_inner_prod_f32(int32_t m, int32_t n, int32_t k, const float *lhs_dev, co
     g.howo = 0;
     g.bias = nullptr;
     g.act = TSX_ACT_NONE;
+    if (!transpose) {      // a 1x1 layer over one image of one row
+        const tsx::ConvF32Layer layer{1, k, 1, n, m, 1, 1, 0, 0, 1, 1, 1, 1, 1, n, rhs_dev, lhs_dev};
+        const int tile = tsx::window_tile(layer, g);
+        if (tile >= 0) return tsx::conv_f32_window(layer, tile, nullptr, TSX_ACT_NONE, 0.f, 0.f, out_dev, tsx::as_stream(stream));
+    }
     tsx::MatLoader ld{};
     ld.b = rhs_dev;
     ld.ld_k = transpose ? 1 : n;   // rhs [k][n], or [n][k] when transposed

@@ -1,12 +1,19 @@
-// Internal interface of the fp32 MFMA GEMM (gemm_f32.hip), shared with the Winograd path.
+// Internal interface of the fp32 convolution kernel of large layers (conv2d_f32_window.hip), used by gemm_f32.hip.
 #pragma once
 #include "tsx_common.hpp"
 
 namespace tsx {
 
-// Strided-batch C[b] = A[b] * B[b]: A [m][k] row-major, B element (k, n) at b[k*ld_k + n*ld_n],
-// C [m][n] row-major; batch b adds a_batch / b_batch / c_batch elements to the bases.
-int gemm_f32_batched(const float *a, int64_t a_batch, const float *b, int64_t ld_k, int64_t ld_n, int64_t b_batch,
-                     float *c, int64_t c_batch, int m, int n, int k, int batches, hipStream_t stream);
+// One layer's geometry and operands; a matrix product [cout][c] x [c][wo] is the 1x1 layer n = ho = h = 1.
+struct ConvF32Layer {
+    int n, c, h, w, cout, kh, kw, pad_top, pad_left, stride_h, stride_w, dil_h, dil_w, ho, wo;
+    const float *x_dev, *w_dev;
+};
+
+// The tile (and patch form) the kernel would take for the layer, -1 where it cannot; its extents; the launch.
+int conv_f32_window_tile(const ConvF32Layer &l);
+void conv_f32_window_tile_size(int tile, int *rows, int *positions);
+int conv_f32_window(const ConvF32Layer &l, int tile, const float *bias, int act, float slope, float padding_value, float *out,
+                    hipStream_t stream);
 
 }  // namespace tsx
