@@ -106,6 +106,7 @@ def build(verbose=True, jobs=8, incremental=False):
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
     build_backend(verbose)
+    build_native(verbose)
     return LIB_PATH
 
 
@@ -168,6 +169,26 @@ def build_backend(verbose=True):
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
     return BACKEND_LIB
+
+
+NATIVE_LIB = os.path.join(LIB_DIR, "_tsx_native.so")
+
+
+def build_native(verbose=True):
+    """The extension module behind tennis_amd.capi's hot calls (host code; against torch's headers and libraries)."""
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-I" + os.path.join(ROOT, "include")]
+    cmd += ["-isystem" + p for p in (os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                                     "/opt/rocm/include", sysconfig.get_paths()["include"])]
+    cmd += [os.path.join(HERE, "native", "capi_native.cpp"), "-o", NATIVE_LIB, "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip",
+            "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-Wl,-rpath," + os.path.join(root, "lib")]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
+    return NATIVE_LIB
 
 
 if __name__ == "__main__":

@@ -3,8 +3,14 @@
 PyTorch is used only for device memory and streams: every function takes CUDA (HIP)
 tensors, hands their raw pointers to libtsx_hip.so and returns tensors.  There is no CPU
 fallback -- if the library is missing or a launch fails this module raises.
+
+The calls that networks make layer by layer go through lib/_tsx_native.so (native/capi_native.cpp), which does their
+checks, output allocation and C ABI call in a few microseconds; it answers NotImplemented for operands that have to be
+converted or arguments that are wrong, and the Python code below each such call then does what it says.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
@@ -21,6 +27,9 @@ _sz = ctypes.c_size_t
 
 ACT_NONE, ACT_RELU, ACT_LEAKY_RELU = 0, 1, 2
 _ACT = {None: ACT_NONE, "none": ACT_NONE, "relu": ACT_RELU, "leaky_relu": ACT_LEAKY_RELU, "mish": 3, "mish_fast": 4}
+
+
+_POOL = {"max": 0, "avg": 1}
 
 
 class ConvGeom(ctypes.Structure):
@@ -125,8 +134,31 @@ def lib():
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args
+        _bind_native(L)
         _lib = L
     return _lib
+
+
+NATIVE_PATH = os.path.join(_HERE, "lib", "_tsx_native.so")
+_native_module = None
+
+
+def _bind_native(L):
+    """Load the extension behind the hot calls and hand it the entry points of the library just loaded."""
+    global _native_module
+    if not os.path.exists(NATIVE_PATH):
+        raise TsxError("%s is not built: run `python -m tennis_amd.build`" % NATIVE_PATH)
+    loader = importlib.machinery.ExtensionFileLoader("_tsx_native", NATIVE_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_tsx_native", loader))
+    loader.exec_module(module)
+    module.bind({name: ctypes.cast(getattr(L, name), _vp).value for name in SIGNATURES}, TsxError)
+    _native_module = module
+
+
+def _native():
+    if _native_module is None:
+        lib()
+    return _native_module
 
 
 AIDS_LIB_PATH = os.path.join(os.path.dirname(LIB_PATH), "libtsx_hip_aids.so")
@@ -195,6 +227,9 @@ def conv2d_i8_plan_info(geom):
 
 def quantize(x, scales):
     """tsx_quantize_f32_i8: x fp32 device tensor, scales fp32 device tensor [x.shape[0]] (or [1])."""
+    out = _native().quantize(x, scales)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     scales = _dev(scales, torch.float32)
     out = torch.empty(x.shape, dtype=torch.int8, device=x.device)
@@ -384,6 +419,7 @@ class Conv2dI8:
         self.padding_value = float(padding_value)
         self._packed = {}
         self._workspace = None
+        self._state = _native().ConvState(self.w, self.pads, self.strides, self.dilations, self.padding_value)
 
     def _plan(self, x_shape):
         geom = make_geom(x_shape, self.w.shape, self.pads, self.strides, self.dilations)
@@ -414,6 +450,10 @@ class Conv2dI8:
                    staged_out=None, residual_after_act=False):
         """The convolution on a StagedInput (its own, or another consumer's of the same tensor).  Returns
         (out_f32 or None, out_i8 or None); with staged_out the int8 output goes to that StagedInput instead."""
+        out = _native_module.conv_i8_staged(self._state, self, staged, dq, bias, _ACT[act], slope, q_scales, want_f32, residual,
+                                            staged_out, residual_after_act)
+        if out is not NotImplemented:
+            return out
         geom, packed, _ = self._plan(staged.x_shape)
         ho, wo = conv_out_size(geom)
         shape = (staged.x_shape[0], self.w.shape[0], ho, wo)
@@ -434,6 +474,10 @@ class Conv2dI8:
         the output's shape added before the activation.
 
         Returns (out_f32 or None, out_i8 or None, acc_i32 or None)."""
+        out = _native_module.conv_i8(self._state, self, x, dq, bias, _ACT[act], slope, q_scales, x_scales, want_f32, want_acc, residual,
+                                     staged_out, residual_after_act)
+        if out is not NotImplemented:
+            return out
         fused_quant = x_scales is not None
         x = _dev(x, torch.float32 if fused_quant else torch.int8)
         geom, packed, ws_bytes = self._plan(tuple(x.shape))
@@ -475,6 +519,10 @@ class GemmI8:
 
     def __call__(self, a, dq=None, row_scale=None, bias=None, act=None, slope=0.0, q_scales=None, want_f32=True,
                  want_acc=False):
+        out = _native_module.gemm_i8(self.packed, self.k, self.n, self._workspace, a, dq, row_scale, bias, _ACT[act], slope, q_scales,
+                                     want_f32, want_acc)
+        if out is not NotImplemented:
+            return out
         a = _dev(a, torch.int8)
         m, k = a.shape
         if k != self.k:
@@ -497,6 +545,9 @@ class GemmI8:
 def conv2d_f32(x, w, pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1), padding_value=0.0, bias=None, act=None,
                slope=0.0):
     """tsx_conv2d_f32_nchw: fp32 implicit-GEMM conv2d (optionally + add_bias + activation)."""
+    out = _native().conv2d_f32(x, w, pads, strides, dilations, padding_value, bias, _ACT[act], slope)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     w = _dev(w, torch.float32)
     bias = _dev(bias, torch.float32)
@@ -541,6 +592,9 @@ def conv2d_f32_prepared(x, w, pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1
 
 def inner_prod_f32(lhs, rhs, transpose=False):
     """tsx_inner_prod_f32: out[m][n] = lhs[m][k] * rhs ([k][n], or [n][k] when transpose)."""
+    out = _native().inner_prod_f32(lhs, rhs, transpose)
+    if out is not NotImplemented:
+        return out
     lhs = _dev(lhs, torch.float32)
     rhs = _dev(rhs, torch.float32)
     m, k = lhs.shape
@@ -574,6 +628,11 @@ class Winograd:
 
     def __call__(self, x, bias=None, act=None, slope=0.0, fast=False):
         """fast (f63 only): the MFMA form, held to the fp32 tolerance instead of the reference's bits."""
+        if self.mode == "f63" or not fast:
+            out = _native_module.winograd((2 if fast else 1) if self.mode == "f63" else 0, x, self.w, self.u, self._workspace, self.pads,
+                                          self.padding_value, bias, _ACT[act], slope)
+            if out is not NotImplemented:
+                return out
         x = _dev(x, torch.float32)
         bias = _dev(bias, torch.float32)
         geom = make_geom(tuple(x.shape), tuple(self.w.shape), self.pads)
@@ -603,6 +662,9 @@ class WinogradF23(Winograd):
 
 
 def add_bias(x, bias, dim=1):
+    out = _native().add_bias(x, bias, dim)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     bias = _dev(bias, torch.float32)
     pre = 1
@@ -627,6 +689,9 @@ def _channel_layout(x, dim):
 
 
 def batch_norm(x, mean, variance, epsilon=1e-5, dim=1):
+    out = _native().batch_norm(x, mean, variance, None, None, epsilon, dim)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     pre, ch, inner = _channel_layout(x, dim)
     out = torch.empty_like(x)
@@ -636,6 +701,9 @@ def batch_norm(x, mean, variance, epsilon=1e-5, dim=1):
 
 
 def batch_scale(x, scale, bias, dim=1):
+    out = _native().batch_norm(x, None, None, scale, bias, 0.0, dim)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     pre, ch, inner = _channel_layout(x, dim)
     out = torch.empty_like(x)
@@ -645,6 +713,9 @@ def batch_scale(x, scale, bias, dim=1):
 
 
 def fused_batch_norm(x, mean, variance, scale, bias, epsilon=1e-5, dim=1):
+    out = _native().batch_norm(x, mean, variance, scale, bias, epsilon, dim)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     pre, ch, inner = _channel_layout(x, dim)
     out = torch.empty_like(x)
@@ -655,6 +726,9 @@ def fused_batch_norm(x, mean, variance, scale, bias, epsilon=1e-5, dim=1):
 
 
 def relu(x):
+    out = _native().unary(0, x, 0.0)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     out = torch.empty_like(x)
     check(lib().tsx_relu_f32(_ptr(x), x.numel(), _ptr(out), _stream()))
@@ -662,6 +736,9 @@ def relu(x):
 
 
 def leaky_relu(x, scale):
+    out = _native().unary(1, x, scale)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     out = torch.empty_like(x)
     check(lib().tsx_leaky_relu_f32(_ptr(x), x.numel(), float(scale), _ptr(out), _stream()))
@@ -670,6 +747,9 @@ def leaky_relu(x, scale):
 
 def add(a, b, act=None, slope=0.0, out=None):
     """tsx_add_f32: act(a + b) on equal shapes."""
+    done = _native().add(a, b, _ACT[act], slope, out)
+    if done is not NotImplemented:
+        return done
     a = _dev(a, torch.float32)
     b = _dev(b, torch.float32)
     assert a.shape == b.shape
@@ -688,11 +768,14 @@ def pool_out_size(h, w, ksize, pads, strides):
 
 def pooling2d(x, kind, ksize, strides, pads=(0, 0, 0, 0), white=False):
     """tsx_pooling2d_f32: kind "max" | "avg", pads = (top, bottom, left, right)."""
+    out = _native().pooling2d(x, _POOL[kind], ksize, strides, pads, white)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     n, c, h, w = x.shape
     ho, wo = pool_out_size(h, w, ksize, pads, strides)
     out = torch.empty((n, c, ho, wo), dtype=torch.float32, device=x.device)
-    check(lib().tsx_pooling2d_f32(_ptr(x), n * c, h, w, {"max": 0, "avg": 1}[kind], pads[0], pads[2], ksize[0], ksize[1],
+    check(lib().tsx_pooling2d_f32(_ptr(x), n * c, h, w, _POOL[kind], pads[0], pads[2], ksize[0], ksize[1],
                                   strides[0], strides[1], int(white), _ptr(out), ho, wo, _stream()))
     return out
 
@@ -710,6 +793,9 @@ def _staged_map(st):
 
 def max_pooling2d_staged(src, dst, ksize, strides, pads=(0, 0, 0, 0)):
     """tsx_max_pooling2d_i8_staged between two StagedInput buffers (int8, pixel-major)."""
+    out = _native().max_pooling2d_staged(src, dst, ksize, strides, pads)
+    if out is not NotImplemented:
+        return out
     ho, wo = pool_out_size(src.x_shape[2], src.x_shape[3], ksize, pads, strides)
     assert (ho, wo) == tuple(dst.x_shape[2:]), "destination map is not the pooled size"
     a, b = _staged_map(src), _staged_map(dst)
@@ -723,6 +809,9 @@ def global_pooling2d(x, kind):
 
 
 def mish(x):
+    out = _native().unary(2, x, 0.0)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     out = torch.empty_like(x)
     check(lib().tsx_mish_f32(_ptr(x), x.numel(), _ptr(out), _stream()))
@@ -730,6 +819,9 @@ def mish(x):
 
 
 def softplus(x):
+    out = _native().unary(3, x, 0.0)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     out = torch.empty_like(x)
     check(lib().tsx_softplus_f32(_ptr(x), x.numel(), _ptr(out), _stream()))
@@ -737,6 +829,9 @@ def softplus(x):
 
 
 def tanh(x):
+    out = _native().unary(4, x, 0.0)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     out = torch.empty_like(x)
     check(lib().tsx_tanh_f32(_ptr(x), x.numel(), _ptr(out), _stream()))
@@ -745,6 +840,9 @@ def tanh(x):
 
 def mul(a, b):
     """tsx_mul_f32: a * b on equal shapes."""
+    out = _native().mul(a, b)
+    if out is not NotImplemented:
+        return out
     a, b = _dev(a, torch.float32), _dev(b, torch.float32)
     if a.shape != b.shape:
         raise TsxError("mul: shapes %s and %s differ" % (tuple(a.shape), tuple(b.shape)))
@@ -781,6 +879,9 @@ def resize_nearest(x, ho, wo):
 def depthwise_conv2d(x, w, pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1), padding_value=0.0, bias=None, act=None,
                      slope=0.0):
     """tsx_depthwise_conv2d_f32: w is [1, C, KH, KW]."""
+    out = _native().depthwise_conv2d(x, w, pads, strides, dilations, padding_value, bias, _ACT[act], slope)
+    if out is not NotImplemented:
+        return out
     x = _dev(x, torch.float32)
     w = _dev(w, torch.float32)
     bias = _dev(bias, torch.float32)

@@ -34,6 +34,8 @@
 #include "conv2d_i8_ws_kernel.hpp"
 
 #include <algorithm>
+#include <cstdlib>
+#include <cstring>
 
 namespace tsx {
 namespace {
@@ -69,7 +71,48 @@ __global__ __launch_bounds__(256) void ws_pack_kernel(const int8_t *__restrict__
 
 }  // namespace
 
-WsPlan ws_plan(const WsGeom &g_in) {
+static WsPlan make_ws_plan(const WsGeom &g_in);
+
+// Planning walks hundreds of tile shapes (9 us for a 28x28 layer on the host, as long as the kernel it plans for), and a
+// program plans the same few layers again and again: each host thread keeps its last plans, one per slot of a small
+// table.  The switches the planners read are part of the key.
+WsPlan ws_plan(const WsGeom &g) {
+    struct Key {
+        WsGeom g;
+        char flat[12], rs[12];
+    };
+    struct Slot {
+        Key key;
+        bool used;
+        WsPlan plan;
+    };
+    constexpr int SLOTS = 256;
+    static thread_local Slot *slots = nullptr;
+    Key key;
+    std::memset(&key, 0, sizeof(key));
+    key.g = g;
+    const char *flat = std::getenv("TSX_CONV_I8_FLAT"), *rs = std::getenv("TSX_CONV_I8_RS");
+    if ((flat && std::strlen(flat) >= sizeof(key.flat)) || (rs && std::strlen(rs) >= sizeof(key.rs))) return make_ws_plan(g);
+    if (flat) std::strcpy(key.flat, flat);
+    if (rs) std::strcpy(key.rs, rs);
+    static thread_local struct Owner {
+        ~Owner() { delete[] slots; slots = nullptr; }
+    } owner;
+    (void)owner;
+    if (!slots) slots = new Slot[SLOTS]();
+    static_assert(sizeof(WsGeom) % sizeof(int) == 0, "the key is hashed as ints");
+    uint32_t h = 0;
+    for (size_t i = 0; i < sizeof(WsGeom) / sizeof(int); ++i) h = (h ^ uint32_t(reinterpret_cast<const int *>(&key.g)[i])) * 0x9e3779b1u;
+    Slot &slot = slots[h >> 24];
+    if (!slot.used || std::memcmp(&slot.key, &key, sizeof(key)) != 0) {
+        slot.plan = make_ws_plan(g);
+        slot.key = key;
+        slot.used = true;
+    }
+    return slot.plan;
+}
+
+static WsPlan make_ws_plan(const WsGeom &g_in) {
     WsPlan pl{};
     pl.ok = false;
     // A 1x1 layer reading a buffer without halo is a plain [positions][channels] matrix: rows mean nothing,
