@@ -149,6 +149,39 @@ __global__ __launch_bounds__(256) void channel_affine_kernel(const float *__rest
     }
 }
 
+// The same with one wavefront per plane, for planes of a multiple of 4 elements: the channel's parameters, and with them
+// the reciprocal root in double (as many issue slots as fifteen elements), are worked out once per plane instead of once
+// per 4 elements (32x256x56x56: 38.8 -> 36.3 us).
+template <int NORM>
+__global__ __launch_bounds__(256) void plane_affine_kernel(const float *__restrict__ x, int64_t planes, int channels, int inner4,
+                                                          const float *__restrict__ mean, const float *__restrict__ variance,
+                                                          const float *__restrict__ scale, const float *__restrict__ bias, float epsilon,
+                                                          float *__restrict__ out) {
+    const int lane = threadIdx.x % 64;
+    const int64_t plane = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    if (plane >= planes) return;
+    const v4f *in = reinterpret_cast<const v4f *>(x) + plane * inner4;
+    v4f *o = reinterpret_cast<v4f *>(out) + plane * inner4;
+    const int c = int(plane % channels);
+    const float m = NORM != 0 ? mean[c] : 0.f, var = NORM != 0 ? variance[c] : 0.f;
+    const float sc = NORM != 1 ? scale[c] : 0.f, bi = NORM != 1 ? bias[c] : 0.f;
+    const float inv = NORM != 0 ? float(1.0 / sqrt(double(__fadd_rn(var, epsilon)))) : 0.f;
+    for (int i = lane; i < inner4; i += 64 * 4) {
+        v4f v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = in[min(i + 64 * u, inner4 - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (NORM != 0) v[u][j] = __fmul_rn(__fsub_rn(v[u][j], m), inv);
+                if (NORM != 1) v[u][j] = __builtin_fmaf(v[u][j], sc, bi);
+            }
+            if (i + 64 * u < inner4) o[i + 64 * u] = v[u];
+        }
+    }
+}
+
 template <int NORM>
 int launch_affine(const char *who, const float *x, int64_t pre, int channels, int64_t inner, const float *mean,
                   const float *variance, const float *scale, const float *bias, float epsilon, float *out, void *stream) {
@@ -158,6 +191,14 @@ int launch_affine(const char *who, const float *x, int64_t pre, int channels, in
     if (count == 0) return 0;
     TSX_REQUIRE(x && out, "%s: null pointer", who);
     const bool vec = reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+    const int64_t planes = pre * channels;
+    if (vec && inner % 4 == 0 && inner >= 256 && inner < (int64_t(1) << 31) && planes >= 1024 && planes < (int64_t(1) << 32)) {
+        // enough planes to fill the chip, large enough to fill a wavefront
+        hipLaunchKernelGGL(plane_affine_kernel<NORM>, dim3(unsigned(tsx::ceil_div(planes, 4))), dim3(256), 0, tsx::as_stream(stream), x, planes, channels,
+                           int(inner / 4), mean, variance, scale, bias, epsilon, out);
+        TSX_LAUNCH_CHECK("plane_affine_kernel");
+        return 0;
+    }
     int64_t blocks = tsx::ceil_div(tsx::ceil_div(count, 4), 256);
     if (blocks > 256 * 8) blocks = 256 * 8;
     hipLaunchKernelGGL(channel_affine_kernel<NORM>, dim3(unsigned(blocks)), dim3(256), 0, tsx::as_stream(stream), x, count,

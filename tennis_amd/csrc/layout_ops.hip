@@ -63,12 +63,9 @@ struct DwGeom {
 // value = fma(w, x, value) over (kh, kw) in the reference's order, padding taps contributing
 // w * padding_value.  K3 = a 3x3 kernel at stride 1, dilation 1 (the usual depthwise layer): the taps are
 // unrolled, the nine weights sit in registers and a lane loads each input row's DW_RUN + 2 columns once for
-// its DW_RUN outputs instead of three per output.  K3V = the same with padding 1 on both sides of a row whose
-// length is a multiple of 4: a lane's four centre columns are one aligned 16-byte load (a wavefront reads whole
-// cache lines; scalar loads at a 16-byte lane stride fetch every line four times over) and the two columns
-// beside them come from the neighbouring lanes' registers.
+// its DW_RUN outputs instead of three per output.
 constexpr int DW_RUN = 4;
-enum { DW_GENERIC = 0, DW_K3 = 1, DW_K3V = 2 };
+enum { DW_GENERIC = 0, DW_K3 = 1 };
 
 template <int MODE>
 __global__ __launch_bounds__(256) void depthwise_kernel(const float *__restrict__ x, const float *__restrict__ wt, DwGeom g,
@@ -86,36 +83,7 @@ __global__ __launch_bounds__(256) void depthwise_kernel(const float *__restrict_
     float value[DW_RUN];
 #pragma unroll
     for (int t = 0; t < DW_RUN; ++t) value[t] = 0.f;
-    if (MODE == DW_K3V) {
-        float kk[9];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) kk[i] = k[i];
-        const int lane = threadIdx.x % 64;
-        const bool first = ow0 == 0, last = ow0 + DW_RUN == g.w;   // the row's first / last run (w == wo here)
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            const int hi = oh - g.pt + i;
-            const bool row_in = hi >= 0 && hi < g.h;
-            const float *row = in + min(max(hi, 0), g.h - 1) * g.w;
-            const float4 c4 = *reinterpret_cast<const float4 *>(row + ow0);
-            // column ow0 - 1 is the previous lane's last value, column ow0 + 4 the next lane's first one (same row
-            // unless this is the row's first / last run); the wavefront's edge lanes load theirs
-            float left = __shfl_up(c4.w, 1), right = __shfl_down(c4.x, 1);
-            if (lane == 0 && !first) left = row[ow0 - 1];
-            if (lane == 63 && !last) right = row[ow0 + DW_RUN];
-            float v[DW_RUN + 2] = {left, c4.x, c4.y, c4.z, c4.w, right};
-            if (first) v[0] = g.padding_value;
-            if (last) v[DW_RUN + 1] = g.padding_value;
-            if (!row_in) {
-#pragma unroll
-                for (int c = 0; c < DW_RUN + 2; ++c) v[c] = g.padding_value;
-            }
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-#pragma unroll
-                for (int t = 0; t < DW_RUN; ++t) value[t] = __builtin_fmaf(kk[i * 3 + j], v[t + j], value[t]);
-        }
-    } else if (MODE == DW_K3) {
+    if (MODE == DW_K3) {
         float kk[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) kk[i] = k[i];
@@ -172,6 +140,74 @@ __global__ __launch_bounds__(256) void depthwise_kernel(const float *__restrict_
     }
 }
 
+// 3x3, stride 1, dilation 1, padding 1 on both sides of a row whose length is a multiple of 4: a lane's four centre
+// columns are one aligned 16-byte load (a wavefront reads whole cache lines) and the two columns beside them come from the
+// neighbouring lanes' registers.  A lane walks DW_ROWS output rows down, all its input rows requested up front: an input
+// row is loaded DW_ROWS + 2 times in DW_ROWS instead of three times, and four times the bytes are in flight per wavefront
+// (a row per lane: 58 us on 32x256x56x56; here 38.5).  Lanes run over (plane, row group, run) of the whole tensor: no workgroup is
+// left half empty at a plane's end.  BASIC: the activation is none / relu / leaky_relu.
+constexpr int DW_ROWS = 4;
+
+template <bool BASIC>
+__global__ __launch_bounds__(256) void depthwise3x3_kernel(const float *__restrict__ x, const float *__restrict__ wt, DwGeom g, int64_t items,
+                                                          const float *__restrict__ bias, int act, float slope, int64_t act_body,
+                                                          float *__restrict__ out) {
+    const int64_t id = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    const bool live = id < items;
+    const unsigned u = unsigned(live ? id : items - 1);           // items below 2^32
+    const unsigned runs = unsigned(g.w) / 4, groups = unsigned(g.ho + DW_ROWS - 1) / DW_ROWS;
+    const unsigned r1 = u / runs, run = u - r1 * runs, plane = r1 / groups, group = r1 - plane * groups;
+    const int ci = int(plane % unsigned(g.c)), oh0 = int(group) * DW_ROWS, lane = threadIdx.x % 64;
+    const float *in = x + int64_t(plane) * g.h * g.w + 4 * run;
+    const bool first = run == 0, last = run == runs - 1;
+    v4f row[DW_ROWS + 2];
+    float left[DW_ROWS + 2], right[DW_ROWS + 2];
+#pragma unroll
+    for (int i = 0; i < DW_ROWS + 2; ++i) {
+        const float *at = in + min(max(oh0 - g.pt + i, 0), g.h - 1) * g.w;
+        row[i] = *reinterpret_cast<const v4f *>(at);
+        left[i] = lane == 0 && !first ? at[-1] : g.padding_value;
+        right[i] = lane == 63 && !last ? at[4] : g.padding_value;
+    }
+    float kk[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) kk[i] = wt[ci * 9 + i];
+    const float b = bias ? bias[ci] : 0.f;
+#pragma unroll
+    for (int i = 0; i < DW_ROWS + 2; ++i) {
+        const float l = __shfl_up(row[i][3], 1), r = __shfl_down(row[i][0], 1);
+        if (lane > 0 && !first) left[i] = l;
+        if (lane < 63 && !last) right[i] = r;
+        const int hi = oh0 - g.pt + i;
+        if (hi < 0 || hi >= g.h) {
+            row[i] = v4f{g.padding_value, g.padding_value, g.padding_value, g.padding_value};
+            left[i] = right[i] = g.padding_value;
+        }
+    }
+    if (!live) return;
+#pragma unroll
+    for (int o = 0; o < DW_ROWS; ++o) {
+        if (oh0 + o >= g.ho) return;
+        v4f value = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const v4f q = row[o + i];
+            const float v[6] = {left[o + i], q[0], q[1], q[2], q[3], right[o + i]};
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) value[t] = __builtin_fmaf(kk[i * 3 + j], v[t + j], value[t]);
+        }
+        const int64_t at = (int64_t(plane) * g.ho + oh0 + o) * g.wo + 4 * run;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float v = bias ? __fadd_rn(value[t], b) : value[t];
+            value[t] = BASIC ? tsx::apply_act_basic(v, act, slope, at + t < act_body) : tsx::apply_act(v, act, slope, at + t < act_body);
+        }
+        *reinterpret_cast<v4f *>(out + at) = value;
+    }
+}
+
 }  // namespace
 
 extern "C" {
@@ -225,11 +261,17 @@ int tsx_depthwise_conv2d_f32(const tsx_conv2d_geom *g, const float *x_dev, const
                 "depthwise_conv2d: tensor too large");
     const dim3 grid(unsigned(planes), unsigned(tsx::ceil_div(lanes_per_plane, 256)));
     const bool k3 = g->kh == 3 && g->kw == 3 && g->stride_h == 1 && g->stride_w == 1 && g->dilation_h == 1 && g->dilation_w == 1;
-    const bool k3v = k3 && g->pad_left == 1 && wo == g->w && g->w % 4 == 0 && reinterpret_cast<uintptr_t>(x_dev) % 16 == 0;
-    if (k3v)
-        hipLaunchKernelGGL(depthwise_kernel<DW_K3V>, grid, dim3(256), 0, tsx::as_stream(stream), x_dev, w_dev, d, bias_dev, act,
-                           slope, total / 4 * 4, out_dev);
-    else if (k3)
+    const int64_t items = planes * tsx::ceil_div(ho, DW_ROWS) * (g->w / 4);
+    if (k3 && g->pad_left == 1 && wo == g->w && g->w % 4 == 0 && items < (int64_t(1) << 32) - 256 &&
+        reinterpret_cast<uintptr_t>(x_dev) % 16 == 0 && reinterpret_cast<uintptr_t>(out_dev) % 16 == 0) {
+        const dim3 flat(unsigned(tsx::ceil_div(items, 256)));
+        if (act >= TSX_ACT_MISH)
+            hipLaunchKernelGGL(depthwise3x3_kernel<false>, flat, dim3(256), 0, tsx::as_stream(stream), x_dev, w_dev, d, items, bias_dev, act, slope,
+                               total / 4 * 4, out_dev);
+        else
+            hipLaunchKernelGGL(depthwise3x3_kernel<true>, flat, dim3(256), 0, tsx::as_stream(stream), x_dev, w_dev, d, items, bias_dev, act, slope,
+                               total / 4 * 4, out_dev);
+    } else if (k3)
         hipLaunchKernelGGL(depthwise_kernel<DW_K3>, grid, dim3(256), 0, tsx::as_stream(stream), x_dev, w_dev, d, bias_dev, act,
                            slope, total / 4 * 4, out_dev);
     else

@@ -94,9 +94,117 @@ __global__ __launch_bounds__(256) void pooling2d_kernel(const float *__restrict_
     out[id] = r;
 }
 
-// Global pooling of large maps: one wavefront per plane would change the summation order, so the
-// sequential order is kept and parallelism comes from the N*C planes (32 x 2048 at the end of a
-// ResNet-50-shaped network).
+// Global pooling (one window over the whole map): every plane is one sequential chain in the reference, 784 dependent steps
+// of a memory round trip for a lane that walks its plane by itself (247 us for 32x256 planes of 29x29; 13 us here).  Here a workgroup
+// takes 16 planes, its wavefronts copy them to LDS in chunks with whole cache lines and all of a chunk's loads in flight,
+// and 16 lanes walk one plane each from there, the next chunk's loads on their way.  LDS pitch odd: the walking lanes
+// meet no bank twice.
+constexpr int GP_PLANES = 16, GP_CHUNK = 512, GP_PER = GP_CHUNK / 64, GP_ROWS = GP_PLANES / 4;
+
+__global__ __launch_bounds__(256) void global_pooling2d_kernel(const float *__restrict__ x, int64_t planes, int count, int type, float divisor,
+                                                               float *__restrict__ out) {
+    __shared__ float buf[GP_PLANES][GP_CHUNK + 1];
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int64_t first = int64_t(blockIdx.x) * GP_PLANES;
+    float v[GP_ROWS][GP_PER];
+    auto load = [&](int at) {
+#pragma unroll
+        for (int r = 0; r < GP_ROWS; ++r) {
+            const float *plane = x + min(first + wave + 4 * r, planes - 1) * count;
+#pragma unroll
+            for (int i = 0; i < GP_PER; ++i) v[r][i] = plane[min(at + i * 64 + lane, count - 1)];
+        }
+    };
+    load(0);
+    float acc = 0.f;
+    for (int at = 0; at < count; at += GP_CHUNK) {
+#pragma unroll
+        for (int r = 0; r < GP_ROWS; ++r)
+#pragma unroll
+            for (int i = 0; i < GP_PER; ++i) buf[wave + 4 * r][i * 64 + lane] = v[r][i];
+        __syncthreads();
+        if (at + GP_CHUNK < count) load(at + GP_CHUNK);
+        if (threadIdx.x < GP_PLANES) {
+            const float *row = buf[threadIdx.x];
+            const int n = min(GP_CHUNK, count - at);
+            if (type == 0) {
+                if (at == 0) acc = row[0];
+#pragma unroll 8
+                for (int i = 0; i < n; ++i) acc = row[i] > acc ? row[i] : acc;
+            } else {
+#pragma unroll 8
+                for (int i = 0; i < n; ++i) acc = __fadd_rn(acc, row[i]);
+            }
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x < GP_PLANES && first + threadIdx.x < planes) out[first + threadIdx.x] = type == 0 ? acc : __fdiv_rn(acc, divisor);
+}
+
+// 3x3 max pooling at stride 2 with one row and column of padding in front, on rows of a multiple of 4 (28x28 and up of
+// the usual networks): a lane takes two neighbouring outputs of MP_ROWS output rows, so that its input is one aligned
+// 16-byte load per row plus the column to the left from the neighbouring lane, each row loaded once for both output rows
+// that read it.  The windows are walked in the reference's order (the first valid element, then `>`).  One output per
+// lane and nine 4-byte loads each took 37 us on 32x256x56x56 (129 MB).
+constexpr int MP_ROWS = 2;
+
+__global__ __launch_bounds__(256) void max_pooling2d_3x3s2_kernel(const float *__restrict__ x, int64_t items, int h, int w, int ho, int wo,
+                                                                  float *__restrict__ out) {
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    const int64_t id = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    const bool live = id < items;
+    const unsigned u = unsigned(live ? id : items - 1);           // items below 2^32
+    const unsigned runs = unsigned(wo + 1) / 2, groups = unsigned(ho + MP_ROWS - 1) / MP_ROWS;
+    const unsigned r1 = u / runs, run = u - r1 * runs, plane = r1 / groups, group = r1 - plane * groups;
+    const float *in = x + int64_t(plane) * h * w;
+    const int col = 4 * int(run);                                 // w: only the window at the right border's last column
+    const bool inside = col < w;
+    const int oh0 = int(group) * MP_ROWS, lane = threadIdx.x % 64;
+    v4f row[2 * MP_ROWS + 1];
+    float left[2 * MP_ROWS + 1];
+#pragma unroll
+    for (int i = 0; i < 2 * MP_ROWS + 1; ++i) {
+        const float *at = in + min(max(2 * oh0 - 1 + i, 0), h - 1) * w;
+        row[i] = *reinterpret_cast<const v4f *>(at + (inside ? col : 0));
+        left[i] = lane == 0 && run > 0 ? at[col - 1] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * MP_ROWS + 1; ++i) {
+        const float next = __shfl_up(row[i][3], 1);
+        if (lane > 0) left[i] = next;
+    }
+    if (!live) return;
+#pragma unroll
+    for (int o = 0; o < MP_ROWS; ++o) {
+        const int oh = oh0 + o;
+        if (oh >= ho) return;
+        float m0 = 0.f, m1 = 0.f;
+        bool any0 = false, any1 = false;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const int hh = 2 * oh - 1 + i;
+            const v4f q = row[2 * o + i];
+            if (hh >= 0 && hh < h) {
+                if (run > 0) {
+                    m0 = !any0 || left[2 * o + i] > m0 ? left[2 * o + i] : m0;
+                    any0 = true;
+                }
+                if (inside) {
+                    m0 = !any0 || q[0] > m0 ? q[0] : m0;
+                    m0 = q[1] > m0 ? q[1] : m0;
+                    any0 = true;
+                    m1 = !any1 || q[1] > m1 ? q[1] : m1;
+                    m1 = q[2] > m1 ? q[2] : m1;
+                    m1 = q[3] > m1 ? q[3] : m1;
+                    any1 = true;
+                }
+            }
+        }
+        float *dst = out + (int64_t(plane) * ho + oh) * wo + 2 * run;
+        dst[0] = m0;
+        if (2 * int(run) + 1 < wo) dst[1] = m1;
+    }
+}
 
 // MAX pooling between two quantized convolutions, on int8 in the pixel-major staged layout
 // [n][hs][ws][cp] on both sides.  quantize is monotone non-decreasing for a positive scale, so
@@ -211,6 +319,24 @@ int tsx_pooling2d_f32(const float *x_dev, int64_t planes, int32_t h, int32_t w, 
     const int64_t total = planes * out_h * out_w;
     TSX_REQUIRE(tsx::ceil_div(total, 256) < (int64_t(1) << 31), "pooling2d: tensor too large");
     const dim3 grid(unsigned(tsx::ceil_div(total, 256)));
+    // one window over the whole map and planes enough of elements that a lane's walk is what takes the time
+    if (out_h == 1 && out_w == 1 && pad_top == 0 && pad_left == 0 && kh >= h && kw >= w && h * int64_t(w) >= 16 && int64_t(h) * w < (1 << 30)) {
+        const float divisor = white_padding ? float(kh * kw) : float(h * w);
+        hipLaunchKernelGGL(global_pooling2d_kernel, dim3(unsigned(tsx::ceil_div(planes, GP_PLANES))), dim3(256), 0, tsx::as_stream(stream), x_dev,
+                           planes, h * w, type, divisor, out_dev);
+        TSX_LAUNCH_CHECK("global_pooling2d_kernel");
+        return 0;
+    }
+    if (type == 0 && kh == 3 && kw == 3 && stride_h == 2 && stride_w == 2 && pad_top == 1 && pad_left == 1 && w % 4 == 0 && out_w <= w / 2 + 1 &&
+        reinterpret_cast<uintptr_t>(x_dev) % 16 == 0) {
+        const int64_t items = planes * ((out_w + 1) / 2) * tsx::ceil_div(out_h, MP_ROWS);
+        if (items < (int64_t(1) << 32) - 256) {
+            hipLaunchKernelGGL(max_pooling2d_3x3s2_kernel, dim3(unsigned(tsx::ceil_div(items, 256))), dim3(256), 0, tsx::as_stream(stream), x_dev, items,
+                               h, w, out_h, out_w, out_dev);
+            TSX_LAUNCH_CHECK("max_pooling2d_3x3s2_kernel");
+            return 0;
+        }
+    }
     if (kh == 3 && kw == 3)
         hipLaunchKernelGGL((pooling2d_kernel<3, 3>), grid, dim3(256), 0, tsx::as_stream(stream), x_dev, g, out_dev);
     else if (kh == 2 && kw == 2)
