@@ -21,6 +21,7 @@
 // so any consistent K permutation gives the same exact integer result.  Accumulator register
 // r of lane l holds row 8*(r/4) + 4*(l/32) + (r%4), column l % 32.
 #include "igemm_i8.hpp"
+#include "stage_i8.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -32,17 +33,11 @@ namespace {
 
 using tsx::v4i;
 using tsx::v16i;
+using tsx::StageGeom;
 
 constexpr int KSTEP = 64;  // bytes of K per pipeline step (two MFMAs of K=32)
 
 // ------------------------------------------------------------------ staging kernels
-
-struct StageGeom {
-    int n, c, h, w;        // source NCHW
-    int hs, ws, cp;        // staged extent
-    int pad_top, pad_left;
-    int pad_value;         // int8 halo value
-};
 
 // One lane produces one 16-byte channel chunk of one staged pixel.  Adjacent lanes take
 // adjacent ws, so each of the 16 byte loads is coalesced along W of the NCHW source.
@@ -105,251 +100,6 @@ __global__ __launch_bounds__(256) void stage_nchw_kernel(const void *__restrict_
     }
     const int64_t o = ((int64_t(ni) * g.hs + hsi) * g.ws + wsi) * g.cp + chunk * 16;
     *reinterpret_cast<uint4 *>(xs + o) = make_uint4(words[0], words[1], words[2], words[3]);
-}
-
-// Row-at-a-time staging through LDS: one workgroup builds one staged row xs[n][hs][0..ws)[c0..c0+CG)
-// for a group of CG <= 256 channels.  Phase 1 reads the NCHW source coalesced along W (runs of
-// W elements per channel), quantizes (QUANT) and scatters bytes into an LDS tile [ws][CG+16]
-// pre-filled with the halo value; phase 2 writes the tile out as whole 16-byte chunks, a pixel's
-// channel group contiguous.  HBM traffic is exactly the algorithmic 4 B (or 1 B) read + 1 B
-// written per element; the older one-lane-per-chunk kernel remains for very wide rows.
-constexpr int STAGE_CG = 256;                 // channels per pass
-constexpr int STAGE_LROW = STAGE_CG + 16;     // LDS bytes per pixel: 16-byte aligned, bank-shifted
-constexpr int STAGE_MAX_WS = 232;             // ws * LROW <= 63 KiB
-
-struct StageRow {
-    const void *src;
-    const float *scales;
-    int n_scales;
-    int64_t group_len, bulk8;
-    bool uniform_scale;
-    float row_scale;
-    int ni, hi, c0, creal;
-};
-
-// Phase 1 of stage_rows_kernel for one source row and one channel group.  Lane = (run of VW pixels
-// along W, channel quad): a lane loads the same VW pixels of 4 consecutive channels (one VW-wide load
-// per channel, coalesced along W across lanes), packs the 4 quantized bytes of each pixel into one
-// dword and writes VW dwords to the tile -- no byte-granular LDS traffic.  WL = power of two >= W/VW
-// keeps the mapping division-free; loads are issued in batches of NB quads before any is consumed.
-// RMODE says how the row's elements round: 0 = all half away from zero (the reference's scalar loop),
-// 1 = all half to even (its AVX body), 2 = per element (the one row that holds the body/tail border).
-template <bool QUANT, int VW, int RMODE, bool UNIFORM = false>
-__device__ __forceinline__ void stage_quads(const StageGeom &g, const StageRow &r, int8_t *tile, int tid) {
-    typedef float vf __attribute__((ext_vector_type(VW == 1 ? 2 : VW)));   // VW == 1 uses scalars
-    constexpr int NB = VW == 4 ? 2 : 4;
-    const int pw = g.w / VW;
-    int wl = 1, wl_shift = 0;
-    while (wl < pw) {
-        wl <<= 1;
-        ++wl_shift;
-    }
-    const int lane = tid & 63, wave = tid >> 6;
-    const int qpw = 64 >> wl_shift;                 // channel quads per wavefront per step
-    const int pi = lane & (wl - 1);
-    const int wi = pi * VW;
-    const int q_lane = wave * qpw + (lane >> wl_shift);
-    const int qstep = 4 * qpw;                      // quads per workgroup step
-    const bool lane_ok = pi < pw;
-    const int64_t plane = int64_t(g.h) * g.w;
-    const int64_t row_base = (int64_t(r.ni) * g.c + r.c0) * plane + int64_t(r.hi) * g.w + wi;
-    const int quads = (r.creal + 3) / 4;
-    for (int qb = 0; qb < quads; qb += NB * qstep) {
-        float fv[NB][4][VW];
-        int bv[NB][4][VW];
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-            const int c = (qb + u * qstep + q_lane) * 4;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const bool ok = lane_ok && c + j < r.creal;
-                const int64_t e = row_base + int64_t(c + j) * plane;
-                if (QUANT) {
-                    const float *p = static_cast<const float *>(r.src) + e;
-                    if (VW == 1) {
-                        fv[u][j][0] = ok ? *p : 0.f;
-                    } else {
-                        vf t;
-#pragma unroll
-                        for (int v = 0; v < VW; ++v) t[v] = 0.f;
-                        if (ok) t = *reinterpret_cast<const vf *>(p);
-#pragma unroll
-                        for (int v = 0; v < VW; ++v) fv[u][j][v] = t[v];
-                    }
-                } else {
-                    const int8_t *p = static_cast<const int8_t *>(r.src) + e;
-                    uint32_t t = 0;
-                    if (ok) {
-                        if (VW == 4) t = *reinterpret_cast<const uint32_t *>(p);
-                        else if (VW == 2) t = *reinterpret_cast<const uint16_t *>(p);
-                        else t = uint8_t(*p);
-                    }
-#pragma unroll
-                    for (int v = 0; v < VW; ++v) bv[u][j][v] = int8_t(t >> (8 * v));
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-            const int c = (qb + u * qstep + q_lane) * 4;
-            if (!(lane_ok && c < r.creal)) continue;
-            // bytes of the quad that are real channels (the last quad of a ragged channel count keeps zeros above)
-            const uint32_t keep = c + 3 < r.creal ? 0xffffffffu : 0xffffffffu >> (8 * (c + 4 - r.creal));
-#pragma unroll
-            for (int v = 0; v < VW; ++v) {
-                int q[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (QUANT) {
-                        float sc = r.row_scale;
-                        bool half_even = RMODE == 1;
-                        if (RMODE == 2 || (!UNIFORM && !r.uniform_scale)) {   // the element's linear index is only needed here
-                            const int64_t e = row_base + int64_t(c + j) * plane + v;
-                            if (!UNIFORM && !r.uniform_scale) sc = c + j < r.creal ? r.scales[e / r.group_len] : 0.f;
-                            if (RMODE == 2) half_even = e < r.bulk8;
-                        }
-                        q[j] = tsx::quantize_value(__fmul_rn(fv[u][j][v], sc), half_even);
-                    } else {
-                        q[j] = bv[u][j][v];
-                    }
-                }
-                // low bytes of q[0..3] into one dword: three byte permutes (selector 0-3 = bytes of the second
-                // operand, 4-7 = bytes of the first, 0x0c = zero)
-                const uint32_t lo = __builtin_amdgcn_perm(uint32_t(q[1]), uint32_t(q[0]), 0x0c0c0400u);
-                const uint32_t hi = __builtin_amdgcn_perm(uint32_t(q[3]), uint32_t(q[2]), 0x0c0c0400u);
-                const uint32_t word = __builtin_amdgcn_perm(hi, lo, 0x05040100u) & keep;
-                *reinterpret_cast<uint32_t *>(&tile[(wi + v + g.pad_left) * STAGE_LROW + c]) = word;
-            }
-        }
-    }
-}
-
-// FAST: what the launcher has checked for the whole launch -- rows of a multiple of 4 elements from a 16-byte
-// aligned tensor (4-byte aligned for int8), at most 256 of them, one scale per image and more than one image (so
-// every element rounds half away from zero, base_quantize / quantize.cpp's scalar path).  The general kernel
-// carries the per-element 64-bit divisions and the three rounding variants of every load width inline, ~47 000
-// instructions of which a row executes a few hundred scattered over 40 KiB of code; this one is the row's own code.
-template <bool QUANT, bool FAST = false>
-__global__ __launch_bounds__(256) void stage_rows_kernel(const void *__restrict__ src, StageGeom g,
-                                                        const float *__restrict__ scales, int n_scales,
-                                                        int64_t group_len, int64_t bulk8,
-                                                        int8_t *__restrict__ xs) {
-    extern __shared__ __attribute__((aligned(16))) int8_t tile[];   // [ws][STAGE_LROW]
-    const int tid = threadIdx.x;
-    // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Neighbouring rows of a
-    // channel plane share cache lines (a W-float run is rarely line-aligned), so give each XCD a
-    // contiguous run of rows: the shared lines are then fetched from HBM once, not once per XCD.
-    const unsigned total_rows = unsigned(g.n) * g.hs, per_xcd = (total_rows + 7) / 8;
-    const unsigned row_id = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (row_id >= total_rows) return;
-    const int hsi = row_id % g.hs, ni = row_id / g.hs;
-    const int hi = hsi - g.pad_top;
-    const bool row_inside = hi >= 0 && hi < g.h;
-    const uint32_t pad4 = uint32_t(g.pad_value & 0xff) * 0x01010101u;
-    // The scale group of element e is e / group_len (a 64-bit division).  With one scale, or one
-    // group per image (the usual case: the count divides evenly), it is uniform for this row.
-    const bool uniform_scale = QUANT && (n_scales == 1 || group_len == int64_t(g.c) * g.h * g.w);
-    const float row_scale = uniform_scale ? scales[n_scales == 1 ? 0 : ni] : 0.f;
-    for (int c0 = 0; c0 < g.cp; c0 += STAGE_CG) {
-        const int cg = min(STAGE_CG, g.cp - c0);        // multiple of 64
-        const int creal = max(0, min(cg, g.c - c0));    // channels that exist in the source
-        // Lane = (run of VW pixels along W, channel quad): see stage_quads.  The widest run the row
-        // length and the source alignment allow keeps the number of load instructions down.
-        const uintptr_t addr = reinterpret_cast<uintptr_t>(src);
-        const int esz = QUANT ? 4 : 1;
-        int vw = 1;
-        if (FAST || (g.w % 4 == 0 && addr % (4 * esz) == 0)) vw = 4;
-        else if (g.w % 2 == 0 && addr % (2 * esz) == 0) vw = 2;
-        int wl = 1;
-        while (wl * vw < g.w) wl <<= 1;
-        // stage_quads writes every dword of the interior pixels up to the last real channel quad, so
-        // on that path the pre-fill only has to cover the halo pixels and the channel padding: the
-        // two write disjoint dwords and need no barrier between them.
-        const bool quad_path = row_inside && (FAST || wl <= 64);
-        const int real_words = (creal + 3) / 4;
-        // pre-fill: halo value for real channels, zero for channel padding
-        const int wpr = cg / 4;   // dwords per pixel
-        auto fill_word = [&](int pix, int cw) {
-            uint32_t v = pad4;
-            if (cw * 4 + 4 > creal) {
-                v = 0;
-                for (int j = 0; j < 4; ++j)
-                    if (cw * 4 + j < creal) v |= uint32_t(g.pad_value & 0xff) << (8 * j);
-            }
-            *reinterpret_cast<uint32_t *>(&tile[pix * STAGE_LROW + cw * 4]) = v;
-        };
-        if (quad_path) {
-            // only the halo pixels (left and right of the row) and the channel padding of the interior pixels:
-            // a loop over the whole tile costs a division per dword, as much arithmetic as the row itself
-            const int halo_px = g.ws - g.w;
-            for (int idx = tid; idx < halo_px * wpr; idx += 256) {
-                const int hp = idx / wpr, cw = idx - hp * wpr;
-                fill_word(hp < g.pad_left ? hp : hp + g.w, cw);
-            }
-            const int pad_words = wpr - real_words;
-            if (pad_words > 0)
-                for (int idx = tid; idx < g.w * pad_words; idx += 256) {
-                    const int ip = idx / pad_words;
-                    fill_word(g.pad_left + ip, real_words + idx - ip * pad_words);
-                }
-        } else {
-            for (int idx = tid; idx < g.ws * wpr; idx += 256) {
-                const int pix = idx / wpr;
-                fill_word(pix, idx - pix * wpr);
-            }
-            __syncthreads();
-        }
-        if (row_inside) {
-            if constexpr (FAST) {
-                const StageRow r{src, scales, n_scales, group_len, bulk8, true, row_scale, ni, hi, c0, creal};
-                stage_quads<QUANT, 4, 0, true>(g, r, tile, tid);
-            } else if (quad_path) {
-                const StageRow r{src, scales, n_scales, group_len, bulk8, uniform_scale, row_scale, ni, hi, c0, creal};
-                // how this row's elements round: linear indices run from lo to hi_e, the AVX body ends at bulk8
-                int rmode = 0;
-                if (QUANT && n_scales == 1) {
-                    const int64_t lo = ((int64_t(ni) * g.c + c0) * g.h + hi) * g.w;
-                    const int64_t hi_e = lo + int64_t(creal - 1) * g.h * g.w + g.w - 1;
-                    rmode = hi_e < bulk8 ? 1 : lo >= bulk8 ? 0 : 2;
-                }
-                if (vw == 4) {
-                    if (rmode == 0) stage_quads<QUANT, 4, 0>(g, r, tile, tid);
-                    else if (rmode == 1) stage_quads<QUANT, 4, 1>(g, r, tile, tid);
-                    else stage_quads<QUANT, 4, 2>(g, r, tile, tid);
-                } else if (vw == 2) {
-                    if (rmode == 0) stage_quads<QUANT, 2, 0>(g, r, tile, tid);
-                    else if (rmode == 1) stage_quads<QUANT, 2, 1>(g, r, tile, tid);
-                    else stage_quads<QUANT, 2, 2>(g, r, tile, tid);
-                } else {
-                    if (rmode == 0) stage_quads<QUANT, 1, 0>(g, r, tile, tid);
-                    else if (rmode == 1) stage_quads<QUANT, 1, 1>(g, r, tile, tid);
-                    else stage_quads<QUANT, 1, 2>(g, r, tile, tid);
-                }
-            } else {
-                for (int idx = tid; idx < creal * g.w; idx += 256) {
-                    const int c = idx / g.w, wi = idx - c * g.w;
-                    const int64_t e = ((int64_t(ni) * g.c + c0 + c) * g.h + hi) * g.w + wi;
-                    int q;
-                    if (QUANT) {
-                        const float sc = uniform_scale ? row_scale : scales[e / group_len];
-                        q = tsx::quantize_value(__fmul_rn(static_cast<const float *>(src)[e], sc), n_scales == 1 && e < bulk8);
-                    } else {
-                        q = static_cast<const int8_t *>(src)[e];
-                    }
-                    tile[(wi + g.pad_left) * STAGE_LROW + c] = int8_t(q);
-                }
-            }
-        }
-        __syncthreads();
-        const int chunks = cg / 16;
-        int8_t *dst = xs + ((int64_t(ni) * g.hs + hsi) * g.ws) * g.cp + c0;
-        for (int idx = tid; idx < g.ws * chunks; idx += 256) {
-            const int pix = idx / chunks, ch = idx - pix * chunks;
-            *reinterpret_cast<v4i *>(dst + int64_t(pix) * g.cp + ch * 16) =
-                *reinterpret_cast<const v4i *>(&tile[pix * STAGE_LROW + ch * 16]);
-        }
-        if (c0 + STAGE_CG < g.cp) __syncthreads();     // the next pass refills the tile
-    }
 }
 
 // Explicit im2col staging for layers with very few input channels and a large kernel (a 7x7 stem on
@@ -1373,42 +1123,29 @@ int run_stage(const tsx_conv2d_geom *g, const Plan &pl, const void *x, bool x_is
     }
     StageGeom sg{g->n, g->c, g->h, g->w, pl.hs, pl.ws, pl.cp, g->pad_top, g->pad_left,
                  int(int8_t(padding_value))};  // T(padding_value), conv2d_quantized_core.cpp:72
-    const int64_t stage_threads = int64_t(g->n) * pl.hs * pl.ws * (pl.cp / 16);
-    const unsigned stage_blocks = unsigned(tsx::ceil_div(stage_threads, 256));
-    const bool by_rows = pl.ws <= STAGE_MAX_WS;
-    const unsigned row_blocks = (unsigned(g->n) * unsigned(pl.hs) + 7) / 8 * 8;   // whole runs per XCD
-    const size_t row_lds = size_t(pl.ws) * STAGE_LROW;
+    int64_t group_len = 1, bulk8 = 0;
     if (x_is_f32) {
         TSX_REQUIRE(x_scales && n_x_scales >= 1, "quantize_conv2d_i8: missing quantize scales");
         // base_quantize.cpp:26
         TSX_REQUIRE(n_x_scales == g->n, "quantize_conv2d_i8: n_x_scales (%d) must equal the batch (%d)", n_x_scales, g->n);
         const int64_t count = int64_t(g->n) * g->c * g->h * g->w;
-        const int64_t group_len = int64_t(std::ceil(static_cast<float>(count) / static_cast<float>(n_x_scales)));
-        const bool fast = by_rows && n_x_scales > 1 && g->w % 4 == 0 && g->w <= 256 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
-        if (fast)
-            hipLaunchKernelGGL((stage_rows_kernel<true, true>), dim3(row_blocks), dim3(256), row_lds, stream, x, sg, x_scales,
-                               n_x_scales, group_len, (count >> 3) << 3, static_cast<int8_t *>(staged));
-        else if (by_rows)
-            hipLaunchKernelGGL((stage_rows_kernel<true, false>), dim3(row_blocks), dim3(256), row_lds, stream, x, sg, x_scales,
-                               n_x_scales, group_len, (count >> 3) << 3, static_cast<int8_t *>(staged));
-        else
-            hipLaunchKernelGGL(stage_nchw_kernel<true>, dim3(stage_blocks), dim3(256), 0, stream, x, sg, x_scales,
-                               n_x_scales, group_len, (count >> 3) << 3, static_cast<int8_t *>(staged));
+        group_len = int64_t(std::ceil(static_cast<float>(count) / static_cast<float>(n_x_scales)));
+        bulk8 = (count >> 3) << 3;
     } else {
-        const bool fast = by_rows && g->w % 4 == 0 && g->w <= 256 && reinterpret_cast<uintptr_t>(x) % 4 == 0;
-        if (fast)
-            hipLaunchKernelGGL((stage_rows_kernel<false, true>), dim3(row_blocks), dim3(256), row_lds, stream, x, sg,
-                               static_cast<const float *>(nullptr), 1, int64_t(1), int64_t(0),
-                               static_cast<int8_t *>(staged));
-        else if (by_rows)
-            hipLaunchKernelGGL((stage_rows_kernel<false, false>), dim3(row_blocks), dim3(256), row_lds, stream, x, sg,
-                               static_cast<const float *>(nullptr), 1, int64_t(1), int64_t(0),
-                               static_cast<int8_t *>(staged));
-        else
-            hipLaunchKernelGGL(stage_nchw_kernel<false>, dim3(stage_blocks), dim3(256), 0, stream, x, sg,
-                               static_cast<const float *>(nullptr), 1, int64_t(1), int64_t(0),
-                               static_cast<int8_t *>(staged));
+        x_scales = nullptr;
+        n_x_scales = 1;
     }
+    // by runs of a channel plane; a lane per 16-byte chunk for planes shorter than a lane's run (1x1 maps: fully
+    // connected layers as convolutions)
+    if (tsx::stage_planes_takes(sg))
+        return tsx::stage_planes(sg, x, x_scales, n_x_scales, group_len, bulk8, static_cast<int8_t *>(staged), stream);
+    const dim3 grid(unsigned(tsx::ceil_div(int64_t(g->n) * pl.hs * pl.ws * (pl.cp / 16), 256)));
+    if (x_is_f32)
+        hipLaunchKernelGGL(stage_nchw_kernel<true>, grid, dim3(256), 0, stream, x, sg, x_scales, n_x_scales, group_len, bulk8,
+                           static_cast<int8_t *>(staged));
+    else
+        hipLaunchKernelGGL(stage_nchw_kernel<false>, grid, dim3(256), 0, stream, x, sg, static_cast<const float *>(nullptr), 1,
+                           group_len, bulk8, static_cast<int8_t *>(staged));
     TSX_LAUNCH_CHECK("stage_nchw_kernel");
     return 0;
 }
