@@ -20,6 +20,7 @@
 // (l % 32) and 16 consecutive K bytes of K-group (l / 32); A and B use the same K mapping,
 // so any consistent K permutation gives the same exact integer result.  Accumulator register
 // r of lane l holds row 8*(r/4) + 4*(l/32) + (r%4), column l % 32.
+#include "gemm_i8_tile.hpp"
 #include "igemm_i8.hpp"
 #include "stage_i8.hpp"
 
@@ -1529,6 +1530,24 @@ int tsx_gemm_i8(int32_t m, int32_t n, int32_t k, const int8_t *a_dev, const void
             hipLaunchKernelGGL((gemm_i8_ksplit_kernel<2, 2, 4>), grid, dim3(KS_WAVES * 64), 0, stream, p);
             TSX_LAUNCH_CHECK("gemm_i8_ksplit_kernel");
             return 0;
+        }
+    }
+    // the tile kernel's quantize groups are rows; beyond 2^24 elements the reference's group length can round away from that
+    if (!p.residual && !p.st_out && p.act != TSX_ACT_MISH && (!p.out_i8 || p.q_group_len == n) && n < (1 << 23) && kp < (1 << 23)) {
+        // TSX_GEMM_I8_TILE: "0" never, "1" .. "3" every GEMM that comes this far on that tile (tests)
+        const char *e = std::getenv("TSX_GEMM_I8_TILE");
+        const int tile = e && e[0] >= '0' && e[0] <= '3' ? e[0] - '0' : tsx::gemm_i8_tile_choose(m, n, kp, p.out_i8 != nullptr);
+        if (tile) {
+            tsx::GemmTileParams tp{};
+            static_cast<tsx::EpiParams &>(tp) = p;
+            tp.xs = p.xs;
+            tp.wp = p.wp;
+            tp.m = m;
+            tp.cout = n;
+            tp.coutp = p.coutp;
+            tp.cp = kp;
+            tp.cblocks = kp / KSTEP;
+            return tsx::gemm_i8_tile_launch(tp, tile, stream);
         }
     }
     // Enough rows to fill MFMA fragments: the window-stationary kernel in its GEMM form (a 1x1 layer over m

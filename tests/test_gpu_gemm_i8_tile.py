@@ -1,0 +1,44 @@
+"""The tile kernel of the int8 GEMM by itself (TSX_GEMM_I8_TILE=1..3 gives it every GEMM of more than 32 rows that no
+K-split kernel takes), bit for bit against the oracle: rows and columns that end inside a tile, an odd number of K-steps (half
+a last chunk), one K-step, columns that are no multiple of 4 or 16 (elements behind the activation's SIMD body, single-byte
+stores), packed int8 output, and more tiles than one group of four rows of tiles."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(x):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(x)).cuda()
+
+
+def bits(x):
+    return np.ascontiguousarray(x).view(np.int32)
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 64, 128), (129, 100, 131), (257, 192, 400), (300, 321, 30), (1300, 128, 272), (128, 640, 513)])
+@pytest.mark.parametrize("tile", ["1", "2", "3"])
+def test_gemm_i8_tile_kernel(port, monkeypatch, m, k, n, tile):
+    from tennis_amd import capi
+    monkeypatch.setenv("TSX_GEMM_I8_TILE", tile)
+    monkeypatch.setenv("TSX_GEMM_I8_KSPLIT", "0")
+    rng = np.random.default_rng(340 + m + n)
+    a = rng.integers(-128, 128, (m, k)).astype(np.int8)
+    b = rng.integers(-128, 128, (k, n)).astype(np.int8)
+    dqw = rng.uniform(1e-4, 1e-3, n).astype(np.float32)
+    dqa = rng.uniform(0.5, 2.0, m).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    qs = rng.uniform(5, 20, m).astype(np.float32)
+    g = capi.GemmI8(_dev(b))
+    for row_scale, with_bias, act in ((dqa, True, "relu"), (None, False, None), (dqa, True, "leaky_relu")):
+        kw = dict(dq=_dev(dqw), row_scale=None if row_scale is None else _dev(row_scale), bias=_dev(bias) if with_bias else None, act=act, slope=0.1)
+        exp, exp_acc = port.gemm_i8_dequant(a, b, dqw, row_scale, bias if with_bias else None, return_acc=True)
+        exp = port.relu(exp) if act == "relu" else port.leaky_relu(exp, 0.1) if act else exp
+        out, _, _ = g(_dev(a), **kw)
+        assert np.array_equal(bits(out.cpu().numpy()), bits(exp)), act
+        _, q, _ = g(_dev(a), q_scales=_dev(qs), want_f32=False, **kw)
+        assert np.array_equal(q.cpu().numpy(), port.quantize(exp, qs)), act
+        out, q, acc = g(_dev(a), q_scales=_dev(qs), want_acc=True, **kw)
+        assert np.array_equal(acc.cpu().numpy(), exp_acc)
+        assert np.array_equal(bits(out.cpu().numpy()), bits(exp)) and np.array_equal(q.cpu().numpy(), port.quantize(exp, qs)), act
