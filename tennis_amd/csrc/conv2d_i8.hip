@@ -398,6 +398,9 @@ struct GemmParams : tsx::EpiParams {
     int stride_h, stride_w, dil_h, dil_w, kw;
     int taps, cblocks;
     int cout, coutp;
+    // GEMMs on kernels that read their rows where they are: bytes from row to row, and of the whole matrix
+    int pitch;
+    int64_t x_bytes;
 };
 
 using tsx::emit;
@@ -634,7 +637,8 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_i8_skinny_kernel(GemmParam
     const int row = lane % 32;
     const bool row_ok = row < p.positions;
     // B operand: activation row `row`, the 16 K bytes of group lane/32 of each half K-step
-    const int8_t *b_ptr = p.xs + int64_t(row_ok ? row : 0) * p.cp + (lane / 32) * 16;
+    const int64_t b_off = int64_t(row_ok ? row : 0) * p.pitch + (lane / 32) * 16;
+    const int64_t b_limit = p.x_bytes - 16;     // the last piece of the matrix
     // A operand: packed[ks][frag][half][lane][16]
     const int8_t *a_ptr = p.wp + (int64_t(frag) * 128 + lane) * 16;
     const int64_t a_kstride = int64_t(frags) * 2048;
@@ -652,11 +656,17 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_i8_skinny_kernel(GemmParam
             tsx::static_for<0, 2>([&](auto hc) {
                 constexpr int h = decltype(hc)::value;
                 a[u][h] = on ? *reinterpret_cast<const v4i *>(a_ptr + kk * a_kstride + h * 1024) : zero;
-                b[u][h] = (on && row_ok) ? *reinterpret_cast<const v4i *>(b_ptr + kk * 64 + h * 32) : zero;
+                b[u][h] = (on && row_ok) ? tsx::load_piece(p.xs + min(b_off + kk * 64 + h * 32, b_limit)) : zero;
             });
         });
         tsx::static_for<0, SK_BATCH>([&](auto uc) {
             constexpr int u = decltype(uc)::value;
+            if (ks0 + u * SK_WAVES == ksteps - 1 && p.pitch != p.cp) {      // uniform
+                tsx::static_for<0, 2>([&](auto hc) {
+                    constexpr int h = decltype(hc)::value;
+                    b[u][h] = tsx::shift_piece(b[u][h], int(max(b_off + (ksteps - 1) * 64 + h * 32 - b_limit, int64_t(0))));
+                });
+            }
             acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u][0], b[u][0], acc, 0, 0, 0);
             acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u][1], b[u][1], acc, 0, 0, 0);
         });
@@ -672,7 +682,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_i8_skinny_kernel(GemmParam
         const int co = frag * 32 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4);
         if (row_ok && co < p.cout) {
             const float rs = p.row_scale ? p.row_scale[row] : 0.f;
-            emit(p, sum, int64_t(row) * p.cout + co, p.dq ? p.dq[co] : 0.f, p.bias ? p.bias[co] : 0.f, rs);
+            tsx::emit_row(p, p.cout, sum, row, int64_t(row) * p.cout + co, p.dq ? p.dq[co] : 0.f, p.bias ? p.bias[co] : 0.f, rs);
         }
     });
 }
@@ -680,33 +690,31 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_i8_skinny_kernel(GemmParam
 // ------------------------------------------------------------------ K-split int8 GEMM (a few hundred rows)
 // A GEMM with a few hundred activation rows and a large weight matrix has too few output tiles to give every CU a
 // tile of a shape that reuses its operands: the tiled kernels would walk K serially on a fraction of the chip, or
-// read the weights once per 32 rows.  Here a workgroup owns FR x FC fragments (32 FR rows x
-// 32 FC output columns) and its 8 wavefronts SPLIT K (interleaved K-steps): each wavefront loads the operands of
-// BATCH K-steps straight from global memory into MFMA operand registers (no LDS on the way in: no two wavefronts
-// read the same bytes), multiplies them into its own FR x FC accumulators, and the eight partial tiles are added
+// read the weights once per 32 rows.  Here a workgroup owns 64 rows x 64 output columns and its 8 wavefronts SPLIT K
+// (interleaved K-steps): each multiplies its K-steps into accumulators of its own, and the eight partial tiles are added
 // through LDS -- int32, exact, so the order is free and results equal the tiled kernels' and the oracle's.  The
-// epilogue then runs on all eight wavefronts with lanes along 4 consecutive output columns (one 16-byte store per
-// lane for plain fp32 output).
+// epilogue then runs on all eight wavefronts with lanes along 4 consecutive output columns (one 16-byte store of fp32
+// values or one word of int8 values per lane).
 // acc register r of lane l: column (weight row) 8*(r/4) + 4*(l/32) + r%4 of the fragment, activation row l%32.
 constexpr int KS_WAVES = 8;
 
-// The end of a K-split tile: the eight wavefronts' partial accumulators go to LDS (SLOTS = 8: all eight and one
-// barrier; SLOTS = 4, for a kernel with 64 KiB of LDS: wavefronts 4..7 hand theirs to 0..3 first), where every
-// wavefront picks up its share of the sums and runs the epilogue on it: (fragment f, register group g) -- registers
-// 4g .. 4g+3 of a lane are 4 consecutive output columns of one row.  The scales and biases of a wavefront's share are
-// requested before the reduction and arrive under it.  red: SLOTS x FR FC x 16 x 64 ints.
-template <int FR, int FC, int SLOTS>
+// The end of a K-split tile: the eight wavefronts' partial accumulators go to LDS, where every wavefront picks up its
+// share of the sums and runs the epilogue on it: (fragment f, register group g) -- registers 4g .. 4g+3 of a lane are 4
+// consecutive output columns of one row.  The scales and biases of a wavefront's share are requested before the reduction
+// and arrive under it.  red: 8 x FR FC x 16 x 64 ints.
+template <int FR, int FC>
 __device__ __forceinline__ void ksplit_finish(const GemmParams &p, v16i (&acc)[FR][FC], int (*red)[FR * FC][16][64], int frag0,
                                               int row0, int lane, int wave) {
     typedef float v4f __attribute__((ext_vector_type(4)));
     constexpr int FRAGS = FR * FC;
     constexpr int ITEMS = (FRAGS * 4 + KS_WAVES - 1) / KS_WAVES;
-    const bool plain = p.out_f32 && !p.out_i8 && !p.st_out && !p.out_acc && !p.residual && p.act <= TSX_ACT_LEAKY_RELU &&
-                       p.cout % 4 == 0 && reinterpret_cast<uintptr_t>(p.out_f32) % 16 == 0 &&
+    const bool plain = !p.out_acc && !p.residual && p.act <= TSX_ACT_LEAKY_RELU && p.cout % 4 == 0 &&
+                       reinterpret_cast<uintptr_t>(p.out_f32) % 16 == 0 &&
+                       (!p.out_i8 || (reinterpret_cast<uintptr_t>(p.out_i8) % 4 == 0 && p.n_qscales > 1 && p.q_group_len == p.cout)) &&
                        reinterpret_cast<uintptr_t>(p.dq) % 16 == 0 && reinterpret_cast<uintptr_t>(p.bias) % 16 == 0;
     int row[ITEMS], co[ITEMS];
     bool ok[ITEMS];
-    float rs[ITEMS];
+    float rs[ITEMS], qs[ITEMS];
     v4f dq[ITEMS], bias[ITEMS];
     tsx::static_for<0, ITEMS>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
@@ -716,46 +724,23 @@ __device__ __forceinline__ void ksplit_finish(const GemmParams &p, v16i (&acc)[F
         co[i] = (frag0 + f % FC) * 32 + 8 * g4 + 4 * (lane / 32);
         ok[i] = item < FRAGS * 4 && row[i] < p.positions && co[i] < p.cout;
         rs[i] = (ok[i] && p.row_scale) ? p.row_scale[row[i]] : 0.f;
+        qs[i] = (plain && ok[i] && p.out_i8) ? p.q_scales[row[i]] : 0.f;
         const v4f z = {0.f, 0.f, 0.f, 0.f};
         dq[i] = (plain && ok[i]) ? *reinterpret_cast<const v4f *>(p.dq + co[i]) : z;      // co % 4 == 0
         bias[i] = (plain && ok[i] && p.bias) ? *reinterpret_cast<const v4f *>(p.bias + co[i]) : z;
     });
-    if (SLOTS == 8) {
-        tsx::static_for<0, FRAGS>([&](auto fc_) {
-            constexpr int f = decltype(fc_)::value;
-            tsx::static_for<0, 16>([&](auto rc) { red[wave][f][decltype(rc)::value][lane] = acc[f / FC][f % FC][decltype(rc)::value]; });
-        });
-        __syncthreads();
-    } else {
-        if (wave >= 4) {
-            tsx::static_for<0, FRAGS>([&](auto fc_) {
-                constexpr int f = decltype(fc_)::value;
-                tsx::static_for<0, 16>([&](auto rc) { red[wave - 4][f][decltype(rc)::value][lane] = acc[f / FC][f % FC][decltype(rc)::value]; });
-            });
-        }
-        __syncthreads();
-        if (wave < 4) {
-            tsx::static_for<0, FRAGS>([&](auto fc_) {
-                constexpr int f = decltype(fc_)::value;
-                tsx::static_for<0, 16>([&](auto rc) { acc[f / FC][f % FC][decltype(rc)::value] += red[wave][f][decltype(rc)::value][lane]; });
-            });
-        }
-        __syncthreads();
-        if (wave < 4) {
-            tsx::static_for<0, FRAGS>([&](auto fc_) {
-                constexpr int f = decltype(fc_)::value;
-                tsx::static_for<0, 16>([&](auto rc) { red[wave][f][decltype(rc)::value][lane] = acc[f / FC][f % FC][decltype(rc)::value]; });
-            });
-        }
-        __syncthreads();
-    }
+    tsx::static_for<0, FRAGS>([&](auto fc_) {
+        constexpr int f = decltype(fc_)::value;
+        tsx::static_for<0, 16>([&](auto rc) { red[wave][f][decltype(rc)::value][lane] = acc[f / FC][f % FC][decltype(rc)::value]; });
+    });
+    __syncthreads();
     tsx::static_for<0, ITEMS>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         const int item = wave + KS_WAVES * i;
         if (item < FRAGS * 4) {         // uniform
             const int f = item / 4, g4 = item % 4;
             int sum[4] = {0, 0, 0, 0};
-            tsx::static_for<0, SLOTS>([&](auto sc) {
+            tsx::static_for<0, KS_WAVES>([&](auto sc) {
                 constexpr int sl = decltype(sc)::value;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) sum[j] += red[sl][f][4 * g4 + j][lane];
@@ -766,93 +751,38 @@ __device__ __forceinline__ void ksplit_finish(const GemmParams &p, v16i (&acc)[F
                     v4f v;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) v[j] = tsx::epi_value<false>(p, sum[j], idx + j, dq[i][j], bias[i][j], rs[i]);
-                    *reinterpret_cast<v4f *>(p.out_f32 + idx) = v;
+                    if (p.out_f32) *reinterpret_cast<v4f *>(p.out_f32 + idx) = v;
+                    if (p.out_i8) {
+                        uint32_t word = 0;
+                        tsx::static_for<0, 4>([&](auto jc) {
+                            constexpr int j = decltype(jc)::value;
+                            word = tsx::quantize_pack<j>(__fmul_rn(v[j], qs[i]), false, word);
+                        });
+                        *reinterpret_cast<uint32_t *>(p.out_i8 + idx) = word ^ 0x80808080u;
+                    }
                 } else {
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                         if (co[i] + j < p.cout)
-                            emit(p, sum[j], idx + j, p.dq ? p.dq[co[i] + j] : 0.f, p.bias ? p.bias[co[i] + j] : 0.f, rs[i]);
+                            tsx::emit_row(p, p.cout, sum[j], row[i], idx + j, p.dq ? p.dq[co[i] + j] : 0.f, p.bias ? p.bias[co[i] + j] : 0.f, rs[i]);
                 }
             }
         }
     });
 }
 
-template <int FR, int FC, int BATCH>
-__global__ __launch_bounds__(KS_WAVES * 64) void gemm_i8_ksplit_kernel(GemmParams p) {
-    constexpr int FRAGS = FR * FC;
-    __shared__ int red[4][FRAGS][16][64];
-    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
-    const int frag0 = blockIdx.x * FC, row0 = blockIdx.y * FR * 32;
-    const int frags = p.coutp / 32;
-    const int ksteps = p.cblocks;
-    // B operands: activation rows row0 + 32 fr + lane % 32 (beyond m: the last row, never stored), the 16 K bytes
-    // of group lane / 32 of each half K-step.  Lanes of rows beyond m load nothing (a masked lane costs the
-    // memory pipeline nothing; with a single row the B loads all but vanish).
-    const int8_t *b_ptr[FR];
-    bool row_ok[FR];
-    tsx::static_for<0, FR>([&](auto fc_) {
-        constexpr int fr = decltype(fc_)::value;
-        b_ptr[fr] = p.xs + int64_t(min(row0 + fr * 32 + lane % 32, p.positions - 1)) * p.cp + (lane / 32) * 16;
-        row_ok[fr] = row0 + fr * 32 + lane % 32 < p.positions;
-    });
-    // A operands: packed[ks][frag][half][lane][16]; fragments beyond the packed columns: the last one, never stored
-    const int8_t *a_ptr[FC];
-    tsx::static_for<0, FC>([&](auto fc_) {
-        constexpr int fc = decltype(fc_)::value;
-        a_ptr[fc] = p.wp + (int64_t(min(frag0 + fc, frags - 1)) * 128 + lane) * 16;
-    });
-    const int64_t a_kstride = int64_t(frags) * 2048;
-    v16i acc[FR][FC];
-    tsx::static_for<0, FRAGS>([&](auto fc_) {
-        constexpr int f = decltype(fc_)::value;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[f / FC][f % FC][r] = 0;
-    });
-    const v4i zero = {0, 0, 0, 0};
-    for (int ks0 = wave; ks0 < ksteps; ks0 += KS_WAVES * BATCH) {
-        v4i a[BATCH][FC][2], b[BATCH][FR][2];
-        tsx::static_for<0, BATCH>([&](auto uc) {
-            constexpr int u = decltype(uc)::value;
-            const int ks = ks0 + u * KS_WAVES;
-            const bool on = ks < ksteps;        // uniform
-            const int kk = on ? ks : 0;
-            tsx::static_for<0, 2>([&](auto hc) {
-                constexpr int h = decltype(hc)::value;
-                tsx::static_for<0, FC>([&](auto fc_) {
-                    constexpr int fc = decltype(fc_)::value;
-                    a[u][fc][h] = on ? *reinterpret_cast<const v4i *>(a_ptr[fc] + kk * a_kstride + h * 1024) : zero;
-                });
-                tsx::static_for<0, FR>([&](auto fr_) {
-                    constexpr int fr = decltype(fr_)::value;
-                    b[u][fr][h] = (on && row_ok[fr]) ? *reinterpret_cast<const v4i *>(b_ptr[fr] + kk * 64 + h * 32) : zero;
-                });
-            });
-        });
-        tsx::static_for<0, BATCH>([&](auto uc) {
-            constexpr int u = decltype(uc)::value;
-            tsx::static_for<0, 2>([&](auto hc) {
-                constexpr int h = decltype(hc)::value;
-                tsx::static_for<0, FRAGS>([&](auto fc_) {
-                    constexpr int fr = decltype(fc_)::value / FC, fc = decltype(fc_)::value % FC;
-                    acc[fr][fc] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u][fc][h], b[u][fr][h], acc[fr][fc], 0, 0, 0);
-                });
-            });
-        });
-    }
-    ksplit_finish<FR, FC, 4>(p, acc, red, frag0, row0, lane, wave);
-}
-
-// The same tile with the activations through LDS.  Read straight into MFMA operand registers, the activation
-// operand of a K-step is 32 rows x 32 bytes per load instruction, which the CU's vector memory path serves at half
-// the rate of whole cache lines.  Here the workgroup copies its 64 rows in chunks of 16 K-steps (1 KiB per row, one
-// row per load instruction, double-buffered: chunk c + 1 is on its way while chunk c is multiplied, one barrier per
-// chunk) and every wavefront reads the operands of its own two K-steps of the chunk from LDS; the weights still go
-// from global memory straight into registers (1 KiB contiguous per operand).  For K of 2048 and more.
+// The activations go through LDS: read straight into MFMA operand registers, the activation operand of a K-step is 32
+// rows x 32 bytes per load instruction, which the CU's vector memory path serves at half the rate of whole cache lines.
+// The workgroup copies its 64 rows in chunks of 16 K-steps (1 KiB per row, one row per load instruction,
+// double-buffered: chunk c + 1 is on its way while chunk c is multiplied, one barrier per chunk) and every wavefront reads
+// the operands of its own two K-steps of the chunk from LDS; the weights go from global memory straight into registers
+// (1 KiB contiguous per operand).
 constexpr int KL_CHUNK = 16;                      // K-steps per chunk
 constexpr int KL_PITCH = KL_CHUNK * KSTEP + 16;   // bytes per row and chunk in LDS (the 16: rows 8 apart share banks, not all)
 constexpr int KL_LDS = 2 * 64 * KL_PITCH;         // two chunk buffers; the partial tiles reuse them (131 072 bytes)
 
+// ANY: rows of any length and alignment (apart, because aligned rows lost 3 to 4 % to the last row's handling).
+template <bool ANY>
 __global__ __launch_bounds__(KS_WAVES * 64) void gemm_i8_ksplit_lds_kernel(GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) int8_t kl_lds[];
     static_assert(KL_LDS >= 8 * 4 * 16 * 64 * 4, "the chunk buffers hold the eight partial tiles");
@@ -866,18 +796,32 @@ __global__ __launch_bounds__(KS_WAVES * 64) void gemm_i8_ksplit_lds_kernel(GemmP
     const int8_t *src[8];
     tsx::static_for<0, 8>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        src[i] = p.xs + int64_t(min(row0 + wave + 8 * i, p.positions - 1)) * p.cp + lane * 16;
+        src[i] = p.xs + int64_t(min(row0 + wave + 8 * i, p.positions - 1)) * p.pitch + lane * 16;
     });
+    // the tile of the last row, or the one before where rows are shorter than a K-step, in the last chunk: pieces must end
+    // with the matrix
+    const bool last_rows = ANY && int64_t(p.positions - row0 - 64) * p.pitch < 64;
+    const int8_t *const limit = p.xs + p.x_bytes - 16;
     v4i stage[8];
     auto load_chunk = [&](int c) __attribute__((always_inline)) {
         const int koff = c * (KL_CHUNK * KSTEP);
         const bool inside = koff + lane * 16 < p.cp;             // K-steps beyond K: zeros
         tsx::static_for<0, 8>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
-            stage[i] = inside ? *reinterpret_cast<const v4i *>(src[i] + koff) : zero;
+            const int8_t *at = src[i] + koff;
+            if (ANY && last_rows) at = at < limit ? at : limit;
+            if constexpr (ANY) stage[i] = inside ? tsx::load_piece(at) : zero;
+            else stage[i] = inside ? *reinterpret_cast<const v4i *>(at) : zero;
         });
     };
-    auto store_chunk = [&](int buf) __attribute__((always_inline)) {
+    auto store_chunk = [&](int buf, int c) __attribute__((always_inline)) {
+        if (ANY && last_rows && c == chunks - 1) {
+            tsx::static_for<0, 8>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const int64_t over = src[i] + c * (KL_CHUNK * KSTEP) - limit;
+                stage[i] = tsx::shift_piece(stage[i], int(over > 0 ? over : 0));
+            });
+        }
         tsx::static_for<0, 8>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
             *reinterpret_cast<v4i *>(kl_lds + (buf * 64 + wave + 8 * i) * KL_PITCH + lane * 16) = stage[i];
@@ -914,7 +858,7 @@ __global__ __launch_bounds__(KS_WAVES * 64) void gemm_i8_ksplit_lds_kernel(GemmP
     };
     load_chunk(0);
     load_weights(0);
-    store_chunk(0);
+    store_chunk(0, 0);
     __syncthreads();
     for (int c = 0; c < chunks; ++c) {
         v4i a[2][2][2], b[2][2][2];
@@ -947,10 +891,10 @@ __global__ __launch_bounds__(KS_WAVES * 64) void gemm_i8_ksplit_lds_kernel(GemmP
                 });
             });
         });
-        if (c + 1 < chunks) store_chunk((c + 1) & 1);
+        if (c + 1 < chunks) store_chunk((c + 1) & 1, c + 1);
         __syncthreads();
     }
-    ksplit_finish<2, 2, 8>(p, acc, reinterpret_cast<int (*)[4][16][64]>(kl_lds), frag0, row0, lane, wave);
+    ksplit_finish<2, 2>(p, acc, reinterpret_cast<int (*)[4][16][64]>(kl_lds), frag0, row0, lane, wave);
 }
 
 // ------------------------------------------------------------------ host side
@@ -1464,22 +1408,17 @@ int tsx_gemm_i8(int32_t m, int32_t n, int32_t k, const int8_t *a_dev, const void
     if (rc) return rc;
     hipStream_t stream = tsx::as_stream(stream_);
     const int kp = int(tsx::round_up(k, KSTEP));
-    const int8_t *xs = a_dev;
-    if (kp != k || reinterpret_cast<uintptr_t>(a_dev) % 16 != 0) {
+    const bool padded = kp != k || reinterpret_cast<uintptr_t>(a_dev) % 16 != 0;     // kernels that want whole K-steps need a copy
+    if (padded) {
         const size_t need = size_t(m) * kp;
         if (!workspace_dev || workspace_bytes < need)
             return tsx::fail(TSX_E_WORKSPACE, "gemm_i8: workspace %zu < %zu bytes", workspace_bytes, need);
         TSX_REQUIRE(reinterpret_cast<uintptr_t>(workspace_dev) % 16 == 0, "gemm_i8: workspace must be 16-byte aligned");
-        StageGeom sg{m, k, 1, 1, 1, 1, kp, 0, 0, 0};
-        const int64_t threads = int64_t(m) * (kp / 16);
-        hipLaunchKernelGGL(stage_nchw_kernel<false>, dim3(unsigned(tsx::ceil_div(threads, 256))), dim3(256), 0, stream,
-                           static_cast<const void *>(a_dev), sg, static_cast<const float *>(nullptr), 1, int64_t(1),
-                           int64_t(0), static_cast<int8_t *>(workspace_dev));
-        TSX_LAUNCH_CHECK("stage_nchw_kernel");
-        xs = static_cast<const int8_t *>(workspace_dev);
     }
     GemmParams p{};
-    p.xs = xs;
+    p.xs = a_dev;
+    p.pitch = k;
+    p.x_bytes = int64_t(m) * k;
     p.wp = static_cast<const int8_t *>(packed_w_dev);
     p.positions = m;
     p.howo = 1;
@@ -1493,42 +1432,58 @@ int tsx_gemm_i8(int32_t m, int32_t n, int32_t k, const int8_t *a_dev, const void
     p.cout = n;
     p.coutp = int(tsx::round_up(n, BM));
     fill_epilogue(p, ep, int64_t(m) * n, out_f32_dev, out_i8_dev, out_acc_dev);
+    // a copy with rows of whole K-steps, for the kernels that want one
+    auto pad_rows = [&]() -> int {
+        if (!padded) return 0;
+        const StageGeom sg{m, k, 1, 1, 1, 1, kp, 0, 0, 0};
+        const int64_t threads = int64_t(m) * (kp / 16);
+        hipLaunchKernelGGL(stage_nchw_kernel<false>, dim3(unsigned(tsx::ceil_div(threads, 256))), dim3(256), 0, stream,
+                           static_cast<const void *>(a_dev), sg, static_cast<const float *>(nullptr), 1, int64_t(1),
+                           int64_t(0), static_cast<int8_t *>(workspace_dev));
+        TSX_LAUNCH_CHECK("stage_nchw_kernel");
+        p.xs = static_cast<const int8_t *>(workspace_dev);
+        p.pitch = kp;
+        p.x_bytes = int64_t(m) * kp;
+        return 0;
+    };
     if (m <= 32) {
+        if (p.x_bytes < 16 && (rc = pad_rows())) return rc;      // less than a piece
         hipLaunchKernelGGL(gemm_i8_skinny_kernel, dim3(unsigned(tsx::ceil_div(n, 32))), dim3(SK_WAVES * 64), 0, stream, p);
         TSX_LAUNCH_CHECK("gemm_i8_skinny_kernel");
         return 0;
     }
-    // TSX_GEMM_I8_KSPLIT: "0" never, "force" every GEMM of more than 32 rows (tests); otherwise GEMMs with a K long
-    // enough to split (2048 and more: the LDS form) whose 64 x 64 tiles run in one round (at most 256: that form holds
-    // one workgroup per CU).  Measured against the window-stationary kernel: K = N = 4096 with 48 / 256 rows 10.9 /
-    // 12.4 us against 14.1 / 23.0; K = N = 2048 with 64 / 256 / 512 rows 7.5 / 7.9 / 8.6 us against 8.0 / 9.5 / 10.3;
-    // K = 4096, N = 1024 with 256 / 1024 rows 10.9 / 14.2 us against 14.2 / 15.4; K = 8192, N = 2048 with 512 rows
-    // 20.7 us against 26.8.  Beyond one round it wins or loses by the shape (N = 4096, K = 4096, 512 rows: 23.6 us
-    // against 24.0; N = 2048, K = 8192, 768 rows: 37.4 against 29.8), and with K = 1024 (the register form) it loses:
-    // 7.9 us against 6.2 at 256 rows.  (Chunks of 8 K-steps kept four deep in flight through rotating register sets
-    // measured slower by 0.9 us.)
+    // TSX_GEMM_I8_KSPLIT: "0" never, "force" every GEMM of more than 32 rows (tests); otherwise GEMMs whose 64 x 64 tiles
+    // run in one round (at most 256: one workgroup per CU) with a K long enough to split.  Measured, fp32 output, against
+    // the window-stationary kernel: K = N = 4096 with 48 / 256 rows 10.9 / 12.4 us against 14.1 / 23.0; K = N = 2048 with 64 /
+    // 256 / 512 rows 7.5 / 7.9 / 8.6 against 8.0 / 9.5 / 10.3; 777 x 1112, K = 1536 8.6 against 10.2; even at K = 1024 (256
+    // rows, N = 1024: 6.3 and 6.2), behind it below (K = 512: 6.3 and 5.2).  Rows that kernel would have copied first are
+    // this one's at any K (64 x 1000, K = 250: 6.5 against 8.1; 197 x 777, K = 1500: 10.2 against 13.7).  int8 output goes
+    // out as words of four columns here: against the tile kernel's 16-byte stores from K = 768 on (300 x 1536, K = 1920: 8.3
+    // against 10.8; K = 640: 6.8 and 6.7), against its single bytes always (197 x 777, K = 1500: 11.5 and 13.4).
+    // Beyond one round it wins or loses by the shape (N = 4096, K = 4096, 512 rows: 23.6 us against 24.0; N = 2048, K = 8192,
+    // 768 rows: 37.4 against 29.8).  (Chunks of 8 K-steps kept four deep in flight through rotating register sets measured
+    // slower by 0.9 us.)
     {
         const char *e = std::getenv("TSX_GEMM_I8_KSPLIT");
         const int64_t tiles = tsx::ceil_div(m, 64) * tsx::ceil_div(n, 64);
-        const bool pays = tiles <= 256 && kp >= 2048;
+        const bool pays = tiles <= 256 && (p.out_i8 ? kp >= 768 || n % 16 != 0 : kp > 1024 || padded);
         if (!(e && e[0] == '0') && ((e && e[0] == 'f') || pays)) {
             const dim3 grid(unsigned(tsx::ceil_div(n, 64)), unsigned(tsx::ceil_div(m, 64)));
-            // activations through LDS where K gives the double buffer something to overlap ("forcereg": never)
-            if (kp >= 2048 && !(e && e[0] == 'f' && e[5] == 'r')) {
-                static std::atomic<bool> granted[64];
-                int dev = 0;
-                TSX_HIP(hipGetDevice(&dev));
-                if (dev < 64 && !granted[dev].load()) {     // dynamic LDS beyond 64 KiB: granted per kernel and device
-                    TSX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_i8_ksplit_lds_kernel),
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-                    granted[dev].store(true);
-                }
-                hipLaunchKernelGGL(gemm_i8_ksplit_lds_kernel, grid, dim3(KS_WAVES * 64), KL_LDS, stream, p);
-                TSX_LAUNCH_CHECK("gemm_i8_ksplit_lds_kernel");
-                return 0;
+            // pieces at odd addresses take longer than aligned ones; from K of 3072 on the copy is the cheaper way
+            // (51 x 3280, K = 3917: 14.4 us with it, 15.4 without; 44 x 531, K = 3051: 14.8 and 14.9; 197 x 777, K = 1500:
+            // 13 and 10.2)
+            if (padded && kp >= 3072 && (k % 4 != 0 || reinterpret_cast<uintptr_t>(a_dev) % 4 != 0) && (rc = pad_rows())) return rc;
+            const auto kernel = p.pitch == kp && reinterpret_cast<uintptr_t>(p.xs) % 16 == 0 ? gemm_i8_ksplit_lds_kernel<false> : gemm_i8_ksplit_lds_kernel<true>;
+            static std::atomic<bool> granted[2][64];
+            const int form = kernel == gemm_i8_ksplit_lds_kernel<true>;
+            int dev = 0;
+            TSX_HIP(hipGetDevice(&dev));
+            if (dev < 64 && !granted[form][dev].load()) {     // dynamic LDS beyond 64 KiB: granted per kernel and device
+                TSX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+                granted[form][dev].store(true);
             }
-            hipLaunchKernelGGL((gemm_i8_ksplit_kernel<2, 2, 4>), grid, dim3(KS_WAVES * 64), 0, stream, p);
-            TSX_LAUNCH_CHECK("gemm_i8_ksplit_kernel");
+            hipLaunchKernelGGL(kernel, grid, dim3(KS_WAVES * 64), KL_LDS, stream, p);
+            TSX_LAUNCH_CHECK("gemm_i8_ksplit_lds_kernel");
             return 0;
         }
     }
@@ -1536,7 +1491,7 @@ int tsx_gemm_i8(int32_t m, int32_t n, int32_t k, const int8_t *a_dev, const void
     if (!p.residual && !p.st_out && p.act != TSX_ACT_MISH && (!p.out_i8 || p.q_group_len == n) && n < (1 << 23) && kp < (1 << 23)) {
         // TSX_GEMM_I8_TILE: "0" never, "1" .. "3" every GEMM that comes this far on that tile (tests)
         const char *e = std::getenv("TSX_GEMM_I8_TILE");
-        const int tile = e && e[0] >= '0' && e[0] <= '3' ? e[0] - '0' : tsx::gemm_i8_tile_choose(m, n, kp, p.out_i8 != nullptr);
+        const int tile = e && e[0] >= '0' && e[0] <= '3' ? e[0] - '0' : tsx::gemm_i8_tile_choose(m, n, kp, p.out_i8 != nullptr, padded);
         if (tile) {
             tsx::GemmTileParams tp{};
             static_cast<tsx::EpiParams &>(tp) = p;
@@ -1547,9 +1502,11 @@ int tsx_gemm_i8(int32_t m, int32_t n, int32_t k, const int8_t *a_dev, const void
             tp.coutp = p.coutp;
             tp.cp = kp;
             tp.cblocks = kp / KSTEP;
+            tp.pitch = p.pitch;
             return tsx::gemm_i8_tile_launch(tp, tile, stream);
         }
     }
+    if ((rc = pad_rows())) return rc;
     // Enough rows to fill MFMA fragments: the window-stationary kernel in its GEMM form (a 1x1 layer over m
     // one-pixel rows, row-major output).  Residual terms stay on the tiled kernel.
     if (!p.residual && !p.st_out && p.act != TSX_ACT_MISH) {   // (... and so does the exact Mish)

@@ -61,27 +61,41 @@ __global__ __launch_bounds__(THREADS) void gemm_i8_tile_kernel(GemmTileParams p)
     // chunk copy: thread -> piece tid % 8 of rows tid / 8 + 64 i (rows beyond m: the last one, never stored).  Scalar base
     // and 32-bit lane offsets: no address arithmetic between the MFMAs.
     const int piece = tid % 8;
-    const int8_t *const x_base = p.xs + int64_t(row0) * p.cp;
+    const int8_t *const x_base = p.xs + int64_t(row0) * p.pitch;
     unsigned src[FR];
     int dst[FR];
     static_for<0, FR>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         const int r = tid / 8 + 64 * i;
-        src[i] = unsigned(min(r, p.m - 1 - row0)) * unsigned(p.cp) + piece * 16;
+        src[i] = unsigned(min(r, p.m - 1 - row0)) * unsigned(p.pitch) + piece * 16 + 16;
         dst[i] = r * CHUNK + ((piece ^ ((r >> 1) & 7)) * 16);
     });
+    // the tile of the last row, or the one before where rows are shorter than a K-step, in the last chunk: pieces must end
+    // with the matrix.  Offsets carry 16 so that the limit, 15 bytes ahead of the chunk at most, is no negative one.
+    const bool last_rows = int64_t(p.m - row0 - ROWS) * p.pitch < 64 && p.pitch != p.cp;
+    const int limit = last_rows ? int(int64_t(p.m - row0) * p.pitch) - (chunks - 1) * CHUNK : 0;
     v4i stage[FR];
     auto stage_load = [&](int c) __attribute__((always_inline)) {
         // an odd number of K-steps ends in half a chunk: the last half again, against weights that are zero
         const int back = c * CHUNK + piece * 16 < p.cp ? 0 : 64;
+        const bool clamp = last_rows && c == chunks - 1;
         static_for<0, FR>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
-            unsigned off = src[i] - back;
-            asm volatile("" : "+v"(off));       // keeps the widening at the load, which then takes the scalar base
-            stage[i] = *reinterpret_cast<const v4i *>(x_base + c * CHUNK + off);
+            int off = int(src[i]) - back;
+            if (clamp) off = min(off, limit);
+            unsigned uoff = unsigned(off);
+            asm volatile("" : "+v"(uoff));       // keeps the widening at the load, which then takes the scalar base
+            stage[i] = load_piece(x_base + (c * CHUNK - 16) + uoff);
         });
     };
-    auto stage_store = [&](int buf) __attribute__((always_inline)) {
+    auto stage_store = [&](int buf, int c) __attribute__((always_inline)) {
+        if (last_rows && c == chunks - 1) {
+            const int back = c * CHUNK + piece * 16 < p.cp ? 0 : 64;
+            static_for<0, FR>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                stage[i] = shift_piece(stage[i], max(int(src[i]) - back - limit, 0));
+            });
+        }
         static_for<0, FR>([&](auto ic) { *reinterpret_cast<v4i *>(&lds[buf][dst[decltype(ic)::value]]) = stage[decltype(ic)::value]; });
     };
 
@@ -121,7 +135,7 @@ __global__ __launch_bounds__(THREADS) void gemm_i8_tile_kernel(GemmTileParams p)
 
     stage_load(0);
     static_for<0, HALVES>([&](auto hc) { w_load(hc, 0); });
-    stage_store(0);
+    stage_store(0, 0);
     __syncthreads();
     b_read(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, 0);
     for (int c = 0; c < chunks; ++c) {
@@ -135,7 +149,7 @@ __global__ __launch_bounds__(THREADS) void gemm_i8_tile_kernel(GemmTileParams p)
             } else {
                 // every wavefront has its reads of this buffer's last half behind it, and those of the other buffer since
                 // the barrier before: the other buffer is free, and full behind this barrier
-                stage_store(buf ^ 1);
+                stage_store(buf ^ 1, next);
                 __syncthreads();
                 b_read(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, buf ^ 1);
             }
@@ -272,7 +286,7 @@ int launch(GemmTileParams p, hipStream_t stream) {
 
 }  // namespace
 
-int gemm_i8_tile_choose(int m, int n, int k, bool int8_out) {
+int gemm_i8_tile_choose(int m, int n, int k, bool int8_out, bool unpadded) {
     // One workgroup of any tile fills a CU's issue slots, so a launch takes rounds of 256 tiles; a round takes the tile's
     // fixed part (first loads, epilogue) and a time per 128 of K, in us as fitted to the sweeps quoted below.
     static const float fixed_f32[3] = {7.f, 10.f, 16.f}, fixed_i8[3] = {5.f, 8.5f, 12.f}, per_chunk[3] = {0.57f, 0.9f, 1.75f};
@@ -296,6 +310,8 @@ int gemm_i8_tile_choose(int m, int n, int k, bool int8_out) {
     // int8 output: that kernel divides by the row length for each element, so packed stores win everywhere (512^3: 11.6
     // and 5.8; 256 x 1024 x 1024: 12.9 and 7.4; 4096^3: 155 and 69); single bytes, where the columns are no multiple of
     // 16, only from half a round on (777 x 1111, K = 1500, 63 tiles: 19.1 and 19.9; 3000^3: 92 and 65).
+    // Rows that the other kernel would need copied first: always (732 x 226, K = 177, with the copy 17, here 8 us).
+    if (unpadded) return best;
     if (int8_out) return n % 16 == 0 || best_tiles >= 128 ? best : 0;
     return best_tiles >= (best == 1 ? 192 : 144) ? best : 0;
 }

@@ -42,3 +42,30 @@ def test_gemm_i8_tile_kernel(port, monkeypatch, m, k, n, tile):
         out, q, acc = g(_dev(a), q_scales=_dev(qs), want_acc=True, **kw)
         assert np.array_equal(acc.cpu().numpy(), exp_acc)
         assert np.array_equal(bits(out.cpu().numpy()), bits(exp)) and np.array_equal(q.cpu().numpy(), port.quantize(exp, qs)), act
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 7, 5), (1, 17, 64), (2, 8, 33), (32, 100, 33), (31, 1500, 96), (33, 1, 40), (129, 3, 33), (192, 5, 144), (130, 77, 64),
+                                   (197, 1500, 77), (65, 2049, 66), (64, 2500, 72), (130, 1985, 48), (70, 2048, 64)])
+def test_gemm_i8_rows_of_any_length(port, m, k, n):
+    """Rows that are no multiple of a K-step, from a pointer that is no multiple of anything, read where they are: the
+    last row's last pieces, rows shorter than a piece, a matrix shorter than one, on the skinny, the tile and the K-split kernel."""
+    import torch
+    from tennis_amd import capi
+    rng = np.random.default_rng(350 + m + n)
+    a = rng.integers(-128, 128, (m, k)).astype(np.int8)
+    b = rng.integers(-128, 128, (k, n)).astype(np.int8)
+    dqw = rng.uniform(1e-4, 1e-3, n).astype(np.float32)
+    dqa = rng.uniform(0.5, 2.0, m).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    qs = rng.uniform(5, 20, m).astype(np.float32)
+    exp, exp_acc = port.gemm_i8_dequant(a, b, dqw, dqa, bias, return_acc=True)
+    exp = port.relu(exp)
+    kw = dict(dq=_dev(dqw), row_scale=_dev(dqa), bias=_dev(bias), act="relu")
+    g = capi.GemmI8(_dev(b))
+    flat = torch.from_numpy(a).reshape(-1)
+    for x in (_dev(a), torch.cat([flat[:1], flat]).cuda()[1:].view(m, k)):
+        out, _, acc = g(x, want_acc=True, **kw)
+        assert np.array_equal(acc.cpu().numpy(), exp_acc)
+        assert np.array_equal(bits(out.cpu().numpy()), bits(exp))
+        _, q, _ = g(x, q_scales=_dev(qs), want_f32=False, **kw)
+        assert np.array_equal(q.cpu().numpy(), port.quantize(exp, qs))
