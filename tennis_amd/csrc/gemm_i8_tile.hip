@@ -11,7 +11,7 @@
 //   * weights: the packed operands are 1 KiB contiguous per fragment and half K-step and go straight into registers, a
 //     chunk ahead of their MFMAs;
 //   * one barrier per chunk, ahead of the chunk's last MFMAs, whose time covers the first LDS reads behind it.
-// 4096 x 4096 x 4096: 71 .. 76 us with fp32 output (86 .. 105 on the window-stationary kernel's GEMM form), 69 us with int8 output
+// 4096 x 4096 x 4096: 67 .. 74 us with fp32 output (86 .. 105 on the window-stationary kernel's GEMM form), 66 us with int8 output
 // (155); MFMAs are busy 60 % of a CU's time, the rest goes to operand waits around the barrier.  fp32 accumulators go out
 // as 4-byte stores with lanes along columns: two whole 128-byte lines per instruction.
 // int32 accumulation is exact, so the results are the other GEMM kernels' and the oracle's.
@@ -156,11 +156,15 @@ __global__ __launch_bounds__(THREADS) void gemm_i8_tile_kernel(GemmTileParams p)
             // left to itself the compiler gathers the weight loads at the end of the chunk and puts every LDS read right
             // in front of its MFMA
             __builtin_amdgcn_sched_barrier(0);
+            // the wavefront that has its operands goes ahead of the other one's loads (4096^3 with int8 output: 69 -> 66 us,
+            // 3000^3 64 -> 54)
+            __builtin_amdgcn_s_setprio(1);
             static_for<0, FR * FC>([&](auto fc) {
                 constexpr int i = decltype(fc)::value / FC, f = decltype(fc)::value % FC;
                 if constexpr (COLS) acc[i][f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b[h % 2][i], w[h][f], acc[i][f], 0, 0, 0);
                 else acc[i][f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[h][f], b[h % 2][i], acc[i][f], 0, 0, 0);
             });
+            __builtin_amdgcn_s_setprio(0);
             w_load(hc, next);
             __builtin_amdgcn_sched_barrier(0);
         });
