@@ -137,21 +137,26 @@ __device__ __forceinline__ float apply_act(float v, int act, float slope, bool i
     if (act == TSX_ACT_MISH_FAST) return mish_short(v);
     return apply_act_basic(v, act, slope, in_body);
 }
-// The 2^(i/32) table of the host's expf held by the wavefront itself: lane l keeps entry l % 32 in two registers, and
-// a lane's look-up is two cross-lane reads (ds_bpermute) instead of a gather from memory -- twice per Mish value, in
-// the middle of its dependent chain.  Every lane must be active where it is used.
+// The tables of the exact Mish held by the wavefront itself: lane l keeps entry l % 32 of the host's expf in two registers and
+// entry l of the logarithm's in three, and a look-up is two or three cross-lane reads (ds_bpermute) instead of a gather from
+// memory -- three times per Mish value, in the middle of its dependent chain.  Every lane must be active where it is used.
 struct Exp2fTableInLanes {
-    int lo, hi;
+    int lo, hi, inv, log_lo, log_hi;
     __device__ __forceinline__ explicit Exp2fTableInLanes(int lane) {
-        const uint64_t mine = exp2f_table[lane & 31];
+        const uint64_t mine = exp2f_table[lane & 31], log_mine = bits_of_f64(log_of_interval[lane & 63]);
         lo = int(uint32_t(mine));
         hi = int(uint32_t(mine >> 32));
+        inv = __float_as_int(log_inverse[lane & 63]);
+        log_lo = int(uint32_t(log_mine));
+        log_hi = int(uint32_t(log_mine >> 32));
     }
-    __device__ __forceinline__ uint64_t operator()(uint64_t i) const {
-        const int addr = int(i) * 4;
+    __device__ __forceinline__ static uint64_t read(int addr, int lo, int hi) {
         return uint64_t(uint32_t(__builtin_amdgcn_ds_bpermute(addr, lo))) |
                (uint64_t(uint32_t(__builtin_amdgcn_ds_bpermute(addr, hi))) << 32);
     }
+    __device__ __forceinline__ uint64_t operator()(uint64_t i) const { return read(int(i) * 4, lo, hi); }
+    __device__ __forceinline__ float inverse(int i) const { return __int_as_float(__builtin_amdgcn_ds_bpermute(i * 4, inv)); }
+    __device__ __forceinline__ double log_of(int i) const { return f64_of_bits(read(i * 4, log_lo, log_hi)); }
 };
 
 // The exact Mish of the 16 values of an accumulator fragment, two values per turn of a loop that stays a loop: each

@@ -36,15 +36,48 @@ TSX_MISH_TABLE uint64_t exp2f_table[32] = {
     0x3fef5818dcfba487ULL, 0x3fef7c97337b9b5fULL, 0x3fefa4afa2a490daULL, 0x3fefd0765b6e4540ULL,
 };
 
+// log(m) for m in [1, 2) by intervals of 1/64: an approximation of 1/m inside the interval that a float holds exactly, and
+// minus its logarithm.  The first interval has 1 and 0, so that log(1 + f) keeps its relative accuracy for small f.
+TSX_MISH_TABLE float log_inverse[64] = {
+    4096.f / 4096, 4002.f / 4096, 3942.f / 4096, 3884.f / 4096, 3827.f / 4096, 3772.f / 4096, 3718.f / 4096, 3666.f / 4096,
+    3616.f / 4096, 3567.f / 4096, 3519.f / 4096, 3472.f / 4096, 3427.f / 4096, 3383.f / 4096, 3339.f / 4096, 3297.f / 4096,
+    3256.f / 4096, 3216.f / 4096, 3178.f / 4096, 3139.f / 4096, 3102.f / 4096, 3066.f / 4096, 3031.f / 4096, 2996.f / 4096,
+    2962.f / 4096, 2929.f / 4096, 2897.f / 4096, 2865.f / 4096, 2834.f / 4096, 2804.f / 4096, 2774.f / 4096, 2745.f / 4096,
+    2717.f / 4096, 2689.f / 4096, 2661.f / 4096, 2635.f / 4096, 2608.f / 4096, 2583.f / 4096, 2558.f / 4096, 2533.f / 4096,
+    2509.f / 4096, 2485.f / 4096, 2461.f / 4096, 2439.f / 4096, 2416.f / 4096, 2394.f / 4096, 2372.f / 4096, 2351.f / 4096,
+    2330.f / 4096, 2310.f / 4096, 2289.f / 4096, 2270.f / 4096, 2250.f / 4096, 2231.f / 4096, 2212.f / 4096, 2194.f / 4096,
+    2175.f / 4096, 2158.f / 4096, 2140.f / 4096, 2123.f / 4096, 2106.f / 4096, 2089.f / 4096, 2072.f / 4096, 2056.f / 4096,
+};
+TSX_MISH_TABLE double log_of_interval[64] = {
+    0x0.0p+0, 0x1.7c61b1cf5dee0p-6, 0x1.39f07ba0ebd62p-5, 0x1.b35dd9b58baadp-5,
+    0x1.163d6ef957a03p-4, 0x1.518874226130ap-4, 0x1.8c985e9b9ec84p-4, 0x1.c6494a2e418a6p-4,
+    0x1.fe89139dbd566p-4, 0x1.1b35ae3b81dbfp-3, 0x1.36f4c27577593p-3, 0x1.527e5e4a1b58dp-3,
+    0x1.6d35fee52b83bp-3, 0x1.87ad07c493478p-3, 0x1.a27cc30640ecbp-3, 0x1.bc69684aee63ep-3,
+    0x1.d60a17f903515p-3, 0x1.ef5ade4dcffe6p-3, 0x1.03d95a1d67686p-2, 0x1.107e404ab0f81p-2,
+    0x1.1ca28c64bae54p-2, 0x1.2896a13e086a4p-2, 0x1.34585a594b8adp-2, 0x1.403d086cea79cp-2,
+    0x1.4becf95d97913p-2, 0x1.5765f1749da6bp-2, 0x1.62a5afc06121fp-2, 0x1.6e056aa4421d5p-2,
+    0x1.792955fdf47a2p-2, 0x1.840f1e12667f0p-2, 0x1.8f12e873862c8p-2, 0x1.99d5d8130607dp-2,
+    0x1.a4558a1c9b824p-2, 0x1.aef113b0bc778p-2, 0x1.b9a90a06bcb3ep-2, 0x1.c3b6fb361e301p-2,
+    0x1.ce42f18064743p-2, 0x1.d81ff2cce8a4ep-2, 0x1.e21582ecdbf74p-2, 0x1.ec241d5e2ffd0p-2,
+    0x1.f5e3c0b5425c6p-2, 0x1.ffbb60ca863b3p-2, 0x1.04d5ba679ac9bp-1, 0x1.096eb58872addp-1,
+    0x1.0e4898611cce1p-1, 0x1.12f799594efbcp-1, 0x1.17b1ac17cbd5bp-1, 0x1.1c3f41fa97c6bp-1,
+    0x1.20d74d2fbafe5p-1, 0x1.25413d529caeep-1, 0x1.29ee409f15440p-1, 0x1.2e32c3d74d58bp-1,
+    0x1.32bab3a7b21e8p-1, 0x1.37123b54987b6p-1, 0x1.3b7344be40311p-1, 0x1.3fa238ac248a5p-1,
+    0x1.44163ef7283d9p-1, 0x1.481abdce327f6p-1, 0x1.4c649aff0ee16p-1, 0x1.5079fd47366f8p-1,
+    0x1.5497c729233afp-1, 0x1.58be1b857aebep-1, 0x1.5ced1e17c35c5p-1, 0x1.60e52f45788e3p-1,
+};
+
 #ifdef __HIPCC__
 TSX_MISH_FN float div_rn(float a, float b) { return __fdiv_rn(a, b); }   // IEEE division whatever the build's default
 #else
 TSX_MISH_FN float div_rn(float a, float b) { return a / b; }
 #endif
-// where expf_host finds 2^(i/32): this table in memory, or whatever holds a copy of it (on the device, the lanes of
-// the wavefront)
+// where expf_host finds 2^(i/32), and log_precise its interval: these tables in memory, or whatever holds a copy of them (on
+// the device, the lanes of the wavefront)
 struct Exp2fTableInMemory {
     TSX_MISH_MEMBER uint64_t operator()(uint64_t i) const { return exp2f_table[i]; }
+    TSX_MISH_MEMBER float inverse(int i) const { return log_inverse[i]; }
+    TSX_MISH_MEMBER double log_of(int i) const { return log_of_interval[i]; }
 };
 
 TSX_MISH_FN double f64_of_bits(uint64_t u) { double d; __builtin_memcpy(&d, &u, 8); return d; }
@@ -72,38 +105,38 @@ TSX_MISH_FN float expf_host(float x, const Table &table = Table()) {
     return x != x ? x : e;
 }
 
-// log(s) for a finite double s >= 1, to well under 2^-50 relative: s = 2^k m with m in [sqrt(1/2), sqrt(2)),
-// log m = 2 atanh(z), z = (m - 1) / (m + 1), as a series in z^2.  Rounded to float it is what the host's log gives
-// rounded to float: both are far inside half a float ulp of the exact value.
-TSX_MISH_FN double log_precise(double s) {
+// log(s) for a finite double s >= 1, to under 2^-50 relative: s = 2^k m with m in [1, 2), m = (1 + r) / c with the c of m's
+// interval, |r| < 2^-6, log s = k ln2 - log c + log(1 + r), the last as its series up to r^9 / 9.  Rounded to float it is what
+// the host's log gives rounded to float: both are far inside half a float ulp of the exact value.  (Without the table, by
+// atanh((m - 1) / (m + 1)), it is a double division and eleven terms: 45 issue slots instead of 20 of the chain's 127.)
+template <class Table = Exp2fTableInMemory>
+TSX_MISH_FN double log_precise(double s, const Table &table = Table()) {
     const uint64_t ix = bits_of_f64(s);
-    const int64_t k = int64_t(ix - 0x3fe6a09e667f3bcdULL) >> 52;
-    const double m = f64_of_bits(ix - (uint64_t(k) << 52));
-    const double f = m - 1.0;
-    const double z = f / (2.0 + f);
-    const double w = z * z;
-    double p = 1.0 / 23;
-    p = __builtin_fma(p, w, 1.0 / 21);
-    p = __builtin_fma(p, w, 1.0 / 19);
-    p = __builtin_fma(p, w, 1.0 / 17);
-    p = __builtin_fma(p, w, 1.0 / 15);
-    p = __builtin_fma(p, w, 1.0 / 13);
-    p = __builtin_fma(p, w, 1.0 / 11);
-    p = __builtin_fma(p, w, 1.0 / 9);
-    p = __builtin_fma(p, w, 1.0 / 7);
-    p = __builtin_fma(p, w, 1.0 / 5);
-    p = __builtin_fma(p, w, 1.0 / 3);
-    const double zz = z + z;
-    const double lm = __builtin_fma(zz * w, p, zz);
-    const double kd = double(k);
-    return __builtin_fma(kd, 0x1.62e42fefa38p-1, __builtin_fma(kd, 0x1.ef35793c7673p-45, lm));   // k ln2, ln2 in two parts
+    const uint32_t hi = uint32_t(ix >> 32);
+    const int i = int(hi >> 14) & 63;
+    const double m = f64_of_bits((uint64_t((hi & 0xfffffu) | 0x3ff00000u) << 32) | uint32_t(ix));
+    const double r = __builtin_fma(m, double(table.inverse(i)), -1.0);
+    double p = 1.0 / 9;
+    p = __builtin_fma(p, r, -1.0 / 8);
+    p = __builtin_fma(p, r, 1.0 / 7);
+    p = __builtin_fma(p, r, -1.0 / 6);
+    p = __builtin_fma(p, r, 1.0 / 5);
+    p = __builtin_fma(p, r, -1.0 / 4);
+    p = __builtin_fma(p, r, 1.0 / 3);
+    p = __builtin_fma(p, r, -1.0 / 2);
+    const double lm = __builtin_fma(r * r, p, r);
+    const double kd = double(int(hi >> 20) - 1023);
+    // k ln2, ln2 in two parts
+    return __builtin_fma(kd, 0x1.62e42fefa38p-1, table.log_of(i)) + __builtin_fma(kd, 0x1.ef35793c7673p-45, lm);
 }
 
 // cpu::Softplus (src/kernels/cpu/softplus.cpp:30-39): float(log(double(expf(x)) + 1.0))
 template <class Table = Exp2fTableInMemory>
 TSX_MISH_FN float softplus_value(float x, const Table &table = Table()) {
     const double s = double(expf_host(x, table)) + 1.0;
-    return s < __builtin_inf() ? float(log_precise(s)) : float(s);   // +inf and NaN pass through
+    // outside the condition: a table held by a wavefront's lanes is read by all of them
+    const double l = log_precise(s, table);
+    return s < __builtin_inf() ? float(l) : float(s);   // +inf and NaN pass through
 }
 
 // cpu::Tanh (src/kernels/cpu/tanh.cpp:14-23): T(2) * (T(1) / (T(1) + exp(-(T(2) * x)))) - T(1) in float
