@@ -173,8 +173,10 @@ __global__ __launch_bounds__(THREADS) void gemm_i8_tile_kernel(GemmTileParams p)
     if constexpr (COLS) {
         // accumulator r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4 of the fragment, column l % 32: a store instruction
         // writes two runs of 32 consecutive columns
-        const int tail = int(int64_t(p.m) * p.cout - p.act_body);        // last elements of the last row
         const int64_t out0 = int64_t(row0) * p.cout;
+        // from this element of the tile on the activation's scalar tail: the tensor's last one to three elements, which are
+        // elements of several rows where there is one column
+        const unsigned body = unsigned(min(max(p.act_body - out0, int64_t(0)), int64_t(0xffffffff)));
         int co[FC];
         float dq[FC], bias[FC];
         static_for<0, FC>([&](auto fc) {
@@ -214,8 +216,7 @@ __global__ __launch_bounds__(THREADS) void gemm_i8_tile_kernel(GemmTileParams p)
                     static_for<0, 16>([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fmul_rn(float(acc[i][f][r]), dq[f]); });
                     if (p.row_scale) static_for<0, 16>([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fmul_rn(v[r], rs[r]); });
                     if (p.bias) static_for<0, 16>([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], bias[f]); });
-                    const bool lane_tail = co[f] >= p.cout - tail;
-                    activate(v, p, [&](auto rc) { constexpr int r = decltype(rc)::value; return !(lane_tail && first + 8 * (r / 4) + r % 4 == rows - 1); });
+                    activate(v, p, [&](auto rc) { constexpr int r = decltype(rc)::value; return off[r] < body; });
                     if (p.out_f32)
                         static_for<0, 16>([&](auto rc) { constexpr int r = decltype(rc)::value; if (stored(rc)) (p.out_f32 + out0)[off[r]] = v[r]; });
                     if (p.out_i8)

@@ -69,3 +69,34 @@ def test_gemm_i8_rows_of_any_length(port, m, k, n):
         assert np.array_equal(bits(out.cpu().numpy()), bits(exp))
         _, q, _ = g(x, q_scales=_dev(qs), want_f32=False, **kw)
         assert np.array_equal(q.cpu().numpy(), port.quantize(exp, qs))
+
+
+@pytest.mark.parametrize("m", [65, 130, 131, 259])
+@pytest.mark.parametrize("n", [1, 2, 3, 5])
+@pytest.mark.parametrize("tile", ["1", "2", "3", "0", "force"])
+def test_gemm_i8_tile_kernel_few_columns(port, monkeypatch, tile, n, m):
+    """The up to three elements behind the activation's SIMD body are the last of the tensor: with one output column they
+    are several rows.  Body and tail differ in what they make of NaN and of -0, which fill the last rows here.  The other
+    GEMM kernels besides: "0" the window-stationary kernel's GEMM form, "force" the K-split kernel."""
+    from tennis_amd import capi
+    monkeypatch.setenv("TSX_GEMM_I8_TILE", tile if tile != "force" else "0")
+    monkeypatch.setenv("TSX_GEMM_I8_KSPLIT", "force" if tile == "force" else "0")
+    rng = np.random.default_rng(345 + m + n)
+    k = 70
+    a = rng.integers(-128, 128, (m, k)).astype(np.int8)
+    b = rng.integers(-128, 128, (k, n)).astype(np.int8)
+    dqw = rng.uniform(1e-4, 1e-3, n).astype(np.float32)
+    qs = rng.uniform(5, 20, m).astype(np.float32)
+    g = capi.GemmI8(_dev(b))
+    for row_value in (np.nan, -0.0):
+        dqa = rng.uniform(0.5, 2.0, m).astype(np.float32)
+        dqa[m - 5:] = row_value
+        for act in ("relu", "leaky_relu"):
+            exp = port.gemm_i8_dequant(a, b, dqw, dqa, None)
+            exp = port.relu(exp) if act == "relu" else port.leaky_relu(exp, 0.1)
+            kw = dict(dq=_dev(dqw), row_scale=_dev(dqa), act=act, slope=0.1)
+            out = g(_dev(a), **kw)[0].cpu().numpy()
+            assert np.array_equal(np.isnan(out), np.isnan(exp))
+            assert np.array_equal(bits(np.nan_to_num(out)), bits(np.nan_to_num(exp))), (row_value, act)
+            q = g(_dev(a), q_scales=_dev(qs), want_f32=False, **kw)[1].cpu().numpy()
+            assert np.array_equal(q, port.quantize(exp, qs)), (row_value, act)
