@@ -12,6 +12,7 @@
 #include <ATen/core/TensorBase.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstring>
@@ -125,8 +126,9 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
         Py_RETURN_NOTIMPLEMENTED;
     } catch (const Raised &) {
         return nullptr;
-    } catch (const std::exception &e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
+    } catch (const std::exception &) {
+        // as torch raises it from Python: an output that does not fit is a torch.OutOfMemoryError, which programs catch
+        torch::translate_exception_to_python(std::current_exception());
         return nullptr;
     }
 }
