@@ -57,3 +57,61 @@ def test_out_of_memory_is_torch_out_of_memory(capi):
                 call()
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+# ---------------------------------------------------------------- copies and stored layers
+
+def _on_host(capi, monkeypatch):
+    monkeypatch.setattr(capi, "_dev", lambda t, dtype: t)
+
+
+@pytest.mark.parametrize("how", ["deepcopy", "copy", "pickle"])
+def test_a_layer_can_be_copied_and_stored(capi, monkeypatch, how):
+    import torch
+    _on_host(capi, monkeypatch)
+    conv = capi.Conv2dI8(torch.arange(2 * 3 * 9, dtype=torch.int8).view(2, 3, 3, 3), (1, 0, 1, 0), (2, 1), (1, 2), padding_value=-3)
+    other = {"deepcopy": copy.deepcopy, "copy": copy.copy, "pickle": lambda c: pickle.loads(pickle.dumps(c))}[how](conv)
+    assert torch.equal(other.w, conv.w) and (other.w is conv.w) == (how == "copy")
+    assert (other.pads, other.strides, other.dilations, other.padding_value) == ((1, 0, 1, 0), (2, 1), (1, 2), -3.0)
+    assert other._state is not conv._state and type(other._state) is type(conv._state)
+
+
+def test_a_layer_stored_without_its_native_state_loads(capi, monkeypatch):
+    """What a layer's pickle held before there was a native state."""
+    import torch
+    _on_host(capi, monkeypatch)
+    conv = object.__new__(capi.Conv2dI8)
+    conv.__setstate__(dict(w=torch.zeros((2, 3, 1, 1), dtype=torch.int8), pads=(0,) * 4, strides=(1, 1), dilations=(1, 1), padding_value=0.0,
+                           _packed={}, _workspace=None))
+    assert type(conv._state).__name__ == "ConvState"
+
+
+def test_a_stored_layer_is_called_in_a_process_that_made_none(capi, monkeypatch):
+    """The library is loaded by the first call that needs it, also where that is a call of a layer read from a file."""
+    import torch
+    gemm = object.__new__(capi.GemmI8)
+    gemm.__dict__.update(w=torch.zeros((64, 8), dtype=torch.int8), transpose=False, n=8, k=64, packed=torch.zeros(8192, dtype=torch.uint8), _workspace=None)
+    conv = object.__new__(capi.Conv2dI8)
+    conv.__setstate__(dict(w=torch.zeros((2, 3, 1, 1), dtype=torch.int8), pads=(0,) * 4, strides=(1, 1), dilations=(1, 1), padding_value=0.0,
+                           _packed={}, _workspace=None))
+    for call in (lambda: gemm(torch.zeros((2, 64), dtype=torch.int8)), lambda: conv(torch.zeros((1, 3, 4, 4), dtype=torch.int8))):
+        monkeypatch.setattr(capi, "_native_module", None)
+        monkeypatch.setattr(capi, "_lib", None)
+        with pytest.raises(capi.TsxError, match="device tensor"):
+            call()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", ["deepcopy", "pickle"])
+def test_copied_layers_and_networks_compute_the_same(capi, how):
+    import torch
+    from tennis_amd import resnet50
+    twin = copy.deepcopy if how == "deepcopy" else lambda c: pickle.loads(pickle.dumps(c))
+    conv, dq = _layer(capi)
+    x = _input(2, 40, 9, 11)
+    first = conv(x, dq=dq)[0]                         # a state that holds a plan
+    assert torch.equal(first, twin(conv)(x, dq=dq)[0])
+    net = resnet50.ResNet50Int8(*resnet50.make_parameters(width=0.25, blocks=[1, 1, 1, 1], classes=10))
+    image = torch.randn((1, 3, 64, 64), device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    net.calibrate(image)
+    assert torch.equal(net.forward(image), twin(net).forward(image))
