@@ -16,6 +16,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstring>
+#include <memory>
 #include <vector>
 
 #include "tsx_hip.h"
@@ -339,9 +340,13 @@ struct EpilogueArgs {
     PyObject *dq, *row_scale, *bias, *act, *slope, *q_scales, *residual, *staged_out, *residual_after_act;
 };
 
-tsx_epilogue epilogue(const EpilogueArgs &a) {
-    tsx_epilogue e;
-    std::memset(&e, 0, sizeof(e));
+struct HeldEpilogue : tsx_epilogue {
+    at::Tensor staged;                // what staged_out_dev points into, whatever the attribute holds by the launch
+    HeldEpilogue() : tsx_epilogue{} {}
+};
+
+HeldEpilogue epilogue(const EpilogueArgs &a) {
+    HeldEpilogue e;
     e.dq_dev = f32(a.dq).const_data_ptr<float>();
     e.row_scale_dev = f32_or_null(a.row_scale);
     e.bias_dev = f32_or_null(a.bias);
@@ -355,8 +360,8 @@ tsx_epilogue epilogue(const EpilogueArgs &a) {
     e.residual_dev = f32_or_null(a.residual);
     e.residual_after_act = truth(a.residual_after_act) ? 1 : 0;
     if (a.staged_out != Py_None) {
-        Attr buf(a.staged_out, n_buf);
-        e.staged_out_dev = i8(buf.o).mutable_data_ptr<int8_t>();
+        e.staged = i8(Attr(a.staged_out, n_buf).o);
+        e.staged_out_dev = e.staged.mutable_data_ptr<int8_t>();
         e.staged_hs = int_attr(a.staged_out, n_hs);
         e.staged_ws = int_attr(a.staged_out, n_ws);
         e.staged_cp = int_attr(a.staged_out, n_cp);
@@ -391,7 +396,7 @@ PyObject *gemm_i8(PyObject *const *a, Py_ssize_t) {
         ws = workspace.mutable_data_ptr();
     }
     const bool with = a[5] != Py_None;
-    tsx_epilogue e;
+    HeldEpilogue e;
     if (with) e = epilogue({a[5], a[6], a[7], a[8], a[9], a[10], Py_None, Py_None, Py_False});
     at::TensorBase out_f32, out_i8, acc;
     if (with && truth(a[11])) out_f32 = empty({m, n}, c10::kFloat, lhs);
@@ -403,6 +408,8 @@ PyObject *gemm_i8(PyObject *const *a, Py_ssize_t) {
 }
 
 // What one Conv2dI8 has in hand for the input shapes it has seen last: geometry, packed weights, workspace, output size.
+// A call holds the plan it uses: reading the attributes of its other arguments can run Python code, and with it other calls
+// of the layer that replace the plans kept.
 struct Plan {
     tsx_conv2d_geom geom;
     at::Tensor packed, workspace;
@@ -414,7 +421,7 @@ struct ConvState {
     int32_t consts[11];               // cout, kh, kw, pads, strides, dilations
     int32_t cin;
     float padding_value;
-    std::vector<Plan> *plans;
+    std::vector<std::shared_ptr<const Plan>> *plans;
     size_t turn;
 };
 
@@ -434,7 +441,7 @@ PyObject *conv_state_new(PyTypeObject *type, PyObject *args, PyObject *) {
     std::memcpy(self->consts, c, sizeof(c));
     self->cin = int32_t(t.size(1));
     self->padding_value = padding_value;
-    self->plans = new std::vector<Plan>();
+    self->plans = new std::vector<std::shared_ptr<const Plan>>();
     return reinterpret_cast<PyObject *>(self);
 }
 void conv_state_dealloc(PyObject *o) {
@@ -443,9 +450,9 @@ void conv_state_dealloc(PyObject *o) {
 }
 
 // The plan of `layer` (a capi.Conv2dI8) for an input shape; layer._plan makes it, packing the weights where that is due.
-Plan &conv_plan(ConvState *st, PyObject *layer, int32_t n, int32_t c, int32_t h, int32_t w) {
-    for (Plan &p : *st->plans)
-        if (p.geom.n == n && p.geom.h == h && p.geom.w == w && p.geom.c == c) return p;
+std::shared_ptr<const Plan> conv_plan(ConvState *st, PyObject *layer, int32_t n, int32_t c, int32_t h, int32_t w) {
+    for (const auto &p : *st->plans)
+        if (p->geom.n == n && p->geom.h == h && p->geom.w == w && p->geom.c == c) return p;
     if (c != st->cin) throw Decline{};
     PyObject *shape = Py_BuildValue("(iiii)", n, c, h, w);
     PyObject *got = shape ? PyObject_CallMethodObjArgs(layer, n_plan, shape, nullptr) : nullptr;
@@ -467,13 +474,10 @@ Plan &conv_plan(ConvState *st, PyObject *layer, int32_t n, int32_t c, int32_t h,
     p.workspace = tensor(ws.o, c10::kByte);
     check(L.tsx_conv2d_out_size(&p.geom, &p.ho, &p.wo));
     constexpr size_t MOST = 8;        // input shapes a layer keeps plans for
-    if (st->plans->size() < MOST) {
-        st->plans->push_back(std::move(p));
-        return st->plans->back();
-    }
-    Plan &slot = (*st->plans)[st->turn++ % MOST];
-    slot = std::move(p);
-    return slot;
+    auto made = std::make_shared<const Plan>(std::move(p));
+    if (st->plans->size() < MOST) st->plans->push_back(made);
+    else (*st->plans)[st->turn++ % MOST] = made;
+    return made;
 }
 
 void check_residual(PyObject *residual, const Plan &p) {
@@ -488,9 +492,10 @@ PyObject *conv_i8(PyObject *const *a, Py_ssize_t) {
     const bool fused = a[8] != Py_None;
     const at::Tensor &x = fused ? f32(a[2]) : i8(a[2]);
     if (x.dim() != 4) throw Decline{};
-    const Plan &p = conv_plan(st, a[1], int32_t(x.size(0)), int32_t(x.size(1)), int32_t(x.size(2)), int32_t(x.size(3)));
+    const auto plan = conv_plan(st, a[1], int32_t(x.size(0)), int32_t(x.size(1)), int32_t(x.size(2)), int32_t(x.size(3)));
+    const Plan &p = *plan;
     const bool with = a[3] != Py_None;
-    tsx_epilogue e;
+    HeldEpilogue e;
     if (with) {
         check_residual(a[11], p);
         e = epilogue({a[3], Py_None, a[4], a[5], a[6], a[7], a[11], a[12], a[13]});
@@ -519,11 +524,12 @@ PyObject *conv_i8_staged(PyObject *const *a, Py_ssize_t) {
     // state, layer, staged, dq, bias, act, slope, q_scales, want_f32, residual, staged_out, residual_after_act
     ConvState *st = reinterpret_cast<ConvState *>(a[0]);
     const Shape4 s(a[2]);
-    const Plan &p = conv_plan(st, a[1], s.n, s.c, s.h, s.w);
+    const auto plan = conv_plan(st, a[1], s.n, s.c, s.h, s.w);
+    const Plan &p = *plan;
     Attr buf(a[2], n_buf);
     const at::Tensor &in = i8(buf.o);
     check_residual(a[9], p);
-    const tsx_epilogue e = epilogue({a[3], Py_None, a[4], a[5], a[6], a[7], a[9], a[10], a[11]});
+    const HeldEpilogue e = epilogue({a[3], Py_None, a[4], a[5], a[6], a[7], a[9], a[10], a[11]});
     at::TensorBase out_f32, out_i8;
     const int64_t shape[4] = {p.geom.n, p.geom.cout, p.ho, p.wo};
     if (truth(a[8])) out_f32 = empty(shape, c10::kFloat, in);

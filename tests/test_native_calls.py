@@ -115,3 +115,33 @@ def test_copied_layers_and_networks_compute_the_same(capi, how):
     image = torch.randn((1, 3, 64, 64), device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
     net.calibrate(image)
     assert torch.equal(net.forward(image), twin(net).forward(image))
+
+
+# ---------------------------------------------------------------- threads and re-entry
+
+@pytest.mark.gpu
+def test_a_call_made_while_another_reads_its_arguments(capi):
+    """A staged output whose attribute runs the layer on other shapes: the outer call's plan stays what it is."""
+    import torch
+    conv, dq = _layer(capi)
+    x = _input(2, 40, 12, 13)
+    consumer = capi.Conv2dI8(_dev(np.ones((8, 48, 1, 1), np.int8)))
+    qs = torch.full((2,), 5.0, device="cuda")
+    plain = capi.StagedInput(consumer, (2, 48, 12, 13))
+    kw = dict(dq=dq, act="relu", q_scales=qs)
+    want = conv(x, staged_out=plain, **kw)[0]
+
+    class Busy(capi.StagedInput):
+        @property
+        def hs(self):
+            for i in range(20):
+                conv(_input(1, 40, 4 + i, 6), dq=dq)
+            return self._hs
+
+        @hs.setter
+        def hs(self, v):
+            self._hs = v
+
+    busy = Busy(consumer, (2, 48, 12, 13))
+    got = conv(x, staged_out=busy, **kw)[0]
+    assert torch.equal(got, want) and torch.equal(busy.buf, plain.buf)
