@@ -140,7 +140,16 @@ def lib():
 
 
 NATIVE_PATH = os.path.join(_HERE, "lib", "_tsx_native.so")
-_native_module = None
+
+
+class _NotLoaded:
+    """In the place of the extension until a call asks for one of its functions."""
+
+    def __getattr__(self, name):
+        return getattr(_native(), name)
+
+
+_native_module = _NotLoaded()
 
 
 def _bind_native(L):
@@ -156,7 +165,7 @@ def _bind_native(L):
 
 
 def _native():
-    if _native_module is None:
+    if type(_native_module) is _NotLoaded:
         lib()
     return _native_module
 
@@ -461,8 +470,8 @@ class Conv2dI8:
                    staged_out=None, residual_after_act=False):
         """The convolution on a StagedInput (its own, or another consumer's of the same tensor).  Returns
         (out_f32 or None, out_i8 or None); with staged_out the int8 output goes to that StagedInput instead."""
-        out = _native().conv_i8_staged(self._state, self, staged, dq, bias, _ACT[act], slope, q_scales, want_f32, residual,
-                                       staged_out, residual_after_act)
+        out = _native_module.conv_i8_staged(self._state, self, staged, dq, bias, _ACT[act], slope, q_scales, want_f32, residual,
+                                            staged_out, residual_after_act)
         if out is not NotImplemented:
             return out
         geom, packed, _ = self._plan(staged.x_shape)
@@ -485,8 +494,8 @@ class Conv2dI8:
         the output's shape added before the activation.
 
         Returns (out_f32 or None, out_i8 or None, acc_i32 or None)."""
-        out = _native().conv_i8(self._state, self, x, dq, bias, _ACT[act], slope, q_scales, x_scales, want_f32, want_acc, residual,
-                                staged_out, residual_after_act)
+        out = _native_module.conv_i8(self._state, self, x, dq, bias, _ACT[act], slope, q_scales, x_scales, want_f32, want_acc, residual,
+                                     staged_out, residual_after_act)
         if out is not NotImplemented:
             return out
         fused_quant = x_scales is not None
@@ -530,8 +539,8 @@ class GemmI8:
 
     def __call__(self, a, dq=None, row_scale=None, bias=None, act=None, slope=0.0, q_scales=None, want_f32=True,
                  want_acc=False):
-        out = _native().gemm_i8(self.packed, self.k, self.n, self._workspace, a, dq, row_scale, bias, _ACT[act], slope, q_scales,
-                                want_f32, want_acc)
+        out = _native_module.gemm_i8(self.packed, self.k, self.n, self._workspace, a, dq, row_scale, bias, _ACT[act], slope, q_scales,
+                                     want_f32, want_acc)
         if out is not NotImplemented:
             return out
         a = _dev(a, torch.int8)
@@ -640,8 +649,8 @@ class Winograd:
     def __call__(self, x, bias=None, act=None, slope=0.0, fast=False):
         """fast (f63 only): the MFMA form, held to the fp32 tolerance instead of the reference's bits."""
         if self.mode == "f63" or not fast:
-            out = _native().winograd((2 if fast else 1) if self.mode == "f63" else 0, x, self.w, self.u, self._workspace, self.pads,
-                                     self.padding_value, bias, _ACT[act], slope)
+            out = _native_module.winograd((2 if fast else 1) if self.mode == "f63" else 0, x, self.w, self.u, self._workspace, self.pads,
+                                          self.padding_value, bias, _ACT[act], slope)
             if out is not NotImplemented:
                 return out
         x = _dev(x, torch.float32)

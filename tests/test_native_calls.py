@@ -95,7 +95,7 @@ def test_a_stored_layer_is_called_in_a_process_that_made_none(capi, monkeypatch)
     conv.__setstate__(dict(w=torch.zeros((2, 3, 1, 1), dtype=torch.int8), pads=(0,) * 4, strides=(1, 1), dilations=(1, 1), padding_value=0.0,
                            _packed={}, _workspace=None))
     for call in (lambda: gemm(torch.zeros((2, 64), dtype=torch.int8)), lambda: conv(torch.zeros((1, 3, 4, 4), dtype=torch.int8))):
-        monkeypatch.setattr(capi, "_native_module", None)
+        monkeypatch.setattr(capi, "_native_module", capi._NotLoaded())
         monkeypatch.setattr(capi, "_lib", None)
         with pytest.raises(capi.TsxError, match="device tensor"):
             call()
