@@ -17,6 +17,7 @@
 
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "tsx_hip.h"
@@ -115,6 +116,37 @@ void *stream() { return c10::hip::getCurrentHIPStream().stream(); }
 template <class T>
 T *data(at::TensorBase &t) { return t.defined() ? static_cast<T *>(t.mutable_data_ptr()) : nullptr; }
 
+// ---- launches
+
+// Outputs are allocated and kernels launched with the interpreter released: a launch waits where the stream's queue is full, an
+// allocation may wait for the device, and other Python threads run meanwhile.  Everything that reads Python objects comes
+// before; what a launch needs of them is held by the caller's arguments or by the function's own references.
+struct WithoutGil {
+    PyThreadState *state = PyEval_SaveThread();
+    ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+template <class F>
+void launch(F &&enqueue) {
+    int rc;
+    {
+        WithoutGil released;
+        rc = enqueue();
+    }
+    check(rc);
+}
+
+// The kernels of one call write its workspace and read it back: two threads that share a layer and a stream must not enqueue
+// theirs in between.  One of a fixed set of locks by address, held while a call's kernels are enqueued, never while the
+// interpreter is waited for.
+struct WorkspaceLock {
+    std::lock_guard<std::mutex> held;
+    explicit WorkspaceLock(const void *workspace) : held(of(workspace)) {}
+    static std::mutex &of(const void *workspace) {
+        static std::mutex locks[64];
+        return locks[(reinterpret_cast<uintptr_t>(workspace) >> 9) % 64];       // allocations lie 512 bytes apart at least
+    }
+};
+
 template <PyObject *(*F)(PyObject *const *, Py_ssize_t), int N>
 PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (n != N) {
@@ -138,48 +170,58 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
 
 PyObject *unary(PyObject *const *a, Py_ssize_t) {      // what, x, slope
     const at::Tensor &x = f32(a[1]);
-    at::TensorBase out = empty(x.sizes(), c10::kFloat, x);
-    const float *in = x.const_data_ptr<float>();
-    float *o = data<float>(out);
-    const int64_t n = x.numel();
-    switch (integer(a[0])) {
-        case 0: check(L.tsx_relu_f32(in, n, o, stream())); break;
-        case 1: check(L.tsx_leaky_relu_f32(in, n, float(number(a[2])), o, stream())); break;
-        case 2: check(L.tsx_mish_f32(in, n, o, stream())); break;
-        case 3: check(L.tsx_softplus_f32(in, n, o, stream())); break;
-        case 4: check(L.tsx_tanh_f32(in, n, o, stream())); break;
-        default: throw Decline{};
-    }
+    const long what = integer(a[0]);
+    const float slope = what == 1 ? float(number(a[2])) : 0.f;
+    if (what < 0 || what > 4) throw Decline{};
+    at::TensorBase out;
+    launch([&] {
+        out = empty(x.sizes(), c10::kFloat, x);
+        const float *in = x.const_data_ptr<float>();
+        float *o = data<float>(out);
+        const int64_t n = x.numel();
+        switch (what) {
+            case 0: return L.tsx_relu_f32(in, n, o, stream());
+            case 1: return L.tsx_leaky_relu_f32(in, n, slope, o, stream());
+            case 2: return L.tsx_mish_f32(in, n, o, stream());
+            case 3: return L.tsx_softplus_f32(in, n, o, stream());
+            default: return L.tsx_tanh_f32(in, n, o, stream());
+        }
+    });
     return wrap(out);
 }
 
 PyObject *add(PyObject *const *a, Py_ssize_t) {        // a, b, act, slope, out
     const at::Tensor &x = f32(a[0]), &y = f32(a[1]);
     if (x.sizes() != y.sizes()) throw Decline{};
-    if (a[4] != Py_None) {
-        const at::Tensor &out = f32(a[4]);
-        check(L.tsx_add_f32(x.const_data_ptr<float>(), y.const_data_ptr<float>(), x.numel(), int32_t(integer(a[2])), float(number(a[3])),
-                            out.mutable_data_ptr<float>(), stream()));
-        return Py_NewRef(a[4]);
-    }
-    at::TensorBase out = empty(x.sizes(), c10::kFloat, x);
-    check(L.tsx_add_f32(x.const_data_ptr<float>(), y.const_data_ptr<float>(), x.numel(), int32_t(integer(a[2])), float(number(a[3])),
-                        data<float>(out), stream()));
-    return wrap(out);
+    const int32_t act = int32_t(integer(a[2]));
+    const float slope = float(number(a[3]));
+    at::TensorBase out;
+    if (a[4] != Py_None) out = f32(a[4]);
+    launch([&] {
+        if (!out.defined()) out = empty(x.sizes(), c10::kFloat, x);
+        return L.tsx_add_f32(x.const_data_ptr<float>(), y.const_data_ptr<float>(), x.numel(), act, slope, data<float>(out), stream());
+    });
+    return a[4] != Py_None ? Py_NewRef(a[4]) : wrap(out);
 }
 
 PyObject *mul(PyObject *const *a, Py_ssize_t) {
     const at::Tensor &x = f32(a[0]), &y = f32(a[1]);
     if (x.sizes() != y.sizes()) throw Decline{};
-    at::TensorBase out = empty(x.sizes(), c10::kFloat, x);
-    check(L.tsx_mul_f32(x.const_data_ptr<float>(), y.const_data_ptr<float>(), x.numel(), data<float>(out), stream()));
+    at::TensorBase out;
+    launch([&] {
+        out = empty(x.sizes(), c10::kFloat, x);
+        return L.tsx_mul_f32(x.const_data_ptr<float>(), y.const_data_ptr<float>(), x.numel(), data<float>(out), stream());
+    });
     return wrap(out);
 }
 
 PyObject *quantize(PyObject *const *a, Py_ssize_t) {
     const at::Tensor &x = f32(a[0]), &s = f32(a[1]);
-    at::TensorBase out = empty(x.sizes(), c10::kChar, x);
-    check(L.tsx_quantize_f32_i8(x.const_data_ptr<float>(), x.numel(), s.const_data_ptr<float>(), int32_t(s.numel()), data<int8_t>(out), stream()));
+    at::TensorBase out;
+    launch([&] {
+        out = empty(x.sizes(), c10::kChar, x);
+        return L.tsx_quantize_f32_i8(x.const_data_ptr<float>(), x.numel(), s.const_data_ptr<float>(), int32_t(s.numel()), data<int8_t>(out), stream());
+    });
     return wrap(out);
 }
 
@@ -198,8 +240,11 @@ PyObject *add_bias(PyObject *const *a, Py_ssize_t) {   // x, bias, dim
     const at::Tensor &x = f32(a[0]);
     const Channels c(x, integer(a[2]));
     const float *bias = f32(a[1]).const_data_ptr<float>();
-    at::TensorBase out = empty(x.sizes(), c10::kFloat, x);
-    check(L.tsx_add_bias_f32(x.const_data_ptr<float>(), c.pre, c.channels, c.inner, bias, data<float>(out), stream()));
+    at::TensorBase out;
+    launch([&] {
+        out = empty(x.sizes(), c10::kFloat, x);
+        return L.tsx_add_bias_f32(x.const_data_ptr<float>(), c.pre, c.channels, c.inner, bias, data<float>(out), stream());
+    });
     return wrap(out);
 }
 
@@ -208,12 +253,15 @@ PyObject *batch_norm(PyObject *const *a, Py_ssize_t) { // x, mean, variance, sca
     const float *mean = f32_or_null(a[1]), *variance = f32_or_null(a[2]), *scale = f32_or_null(a[3]), *bias = f32_or_null(a[4]);
     const float epsilon = float(number(a[5]));
     const Channels c(x, integer(a[6]));
-    at::TensorBase out = empty(x.sizes(), c10::kFloat, x);
-    const float *in = x.const_data_ptr<float>();
-    float *o = data<float>(out);
-    if (mean && scale) check(L.tsx_fused_batch_norm_f32(in, c.pre, c.channels, c.inner, mean, variance, scale, bias, epsilon, o, stream()));
-    else if (mean) check(L.tsx_batch_norm_f32(in, c.pre, c.channels, c.inner, mean, variance, epsilon, o, stream()));
-    else check(L.tsx_batch_scale_f32(in, c.pre, c.channels, c.inner, scale, bias, o, stream()));
+    at::TensorBase out;
+    launch([&] {
+        out = empty(x.sizes(), c10::kFloat, x);
+        const float *in = x.const_data_ptr<float>();
+        float *o = data<float>(out);
+        if (mean && scale) return L.tsx_fused_batch_norm_f32(in, c.pre, c.channels, c.inner, mean, variance, scale, bias, epsilon, o, stream());
+        if (mean) return L.tsx_batch_norm_f32(in, c.pre, c.channels, c.inner, mean, variance, epsilon, o, stream());
+        return L.tsx_batch_scale_f32(in, c.pre, c.channels, c.inner, scale, bias, o, stream());
+    });
     return wrap(out);
 }
 
@@ -229,9 +277,13 @@ PyObject *pooling2d(PyObject *const *a, Py_ssize_t) {  // x, type, ksize, stride
     const int32_t h = int32_t(x.size(2)), w = int32_t(x.size(3));
     check(L.tsx_pooling2d_out_size(h, w, k[0], k[1], p[0], p[1], p[2], p[3], s[0], s[1], &ho, &wo));
     if (ho <= 0 || wo <= 0) throw Decline{};
-    at::TensorBase out = empty({x.size(0), x.size(1), ho, wo}, c10::kFloat, x);
-    check(L.tsx_pooling2d_f32(x.const_data_ptr<float>(), x.size(0) * x.size(1), h, w, int32_t(integer(a[1])), p[0], p[2], k[0], k[1], s[0], s[1],
-                              truth(a[5]) ? 1 : 0, data<float>(out), ho, wo, stream()));
+    const int32_t type = int32_t(integer(a[1])), white = truth(a[5]) ? 1 : 0;
+    at::TensorBase out;
+    launch([&] {
+        out = empty({x.size(0), x.size(1), ho, wo}, c10::kFloat, x);
+        return L.tsx_pooling2d_f32(x.const_data_ptr<float>(), x.size(0) * x.size(1), h, w, type, p[0], p[2], k[0], k[1], s[0], s[1], white,
+                                   data<float>(out), ho, wo, stream());
+    });
     return wrap(out);
 }
 
@@ -260,7 +312,7 @@ PyObject *max_pooling2d_staged(PyObject *const *a, Py_ssize_t) {      // src, ds
     const tsx_staged_map src = staged_map(a[0], i8(from.o)), dst = staged_map(a[1], i8(to.o));
     check(L.tsx_pooling2d_out_size(src.h, src.w, k[0], k[1], p[0], p[1], p[2], p[3], s[0], s[1], &ho, &wo));
     if (ho != dst.h || wo != dst.w) throw Decline{};
-    check(L.tsx_max_pooling2d_i8_staged(&src, &dst, k[0], k[1], p[0], p[2], s[0], s[1], stream()));
+    launch([&] { return L.tsx_max_pooling2d_i8_staged(&src, &dst, k[0], k[1], p[0], p[2], s[0], s[1], stream()); });
     return Py_NewRef(a[1]);
 }
 
@@ -276,20 +328,27 @@ tsx_conv2d_geom geometry(const at::Tensor &x, const at::Tensor &w, PyObject *pad
             int32_t(w.size(3)), p[0], p[1], p[2], p[3], s[0], s[1], d[0], d[1]};
 }
 
-at::TensorBase conv_out(const tsx_conv2d_geom &g, const at::TensorBase &like) {
-    int32_t ho, wo;
-    check(L.tsx_conv2d_out_size(&g, &ho, &wo));
-    if (ho <= 0 || wo <= 0) throw Decline{};
-    return empty({g.n, g.cout, ho, wo}, c10::kFloat, like);
-}
+struct OutSize {
+    int32_t h, w;
+    explicit OutSize(const tsx_conv2d_geom &g) {
+        check(L.tsx_conv2d_out_size(&g, &h, &w));
+        if (h <= 0 || w <= 0) throw Decline{};
+    }
+};
 
 PyObject *conv2d_f32(PyObject *const *a, Py_ssize_t) {  // x, w, pads, strides, dilations, padding_value, bias, act, slope
     const at::Tensor &x = f32(a[0]), &w = f32(a[1]);
     const tsx_conv2d_geom g = geometry(x, w, a[2], a[3], a[4]);
     const float *bias = f32_or_null(a[6]);
-    at::TensorBase out = conv_out(g, x);
-    check(L.tsx_conv2d_f32_nchw(&g, x.const_data_ptr<float>(), w.const_data_ptr<float>(), float(number(a[5])), bias, int32_t(integer(a[7])),
-                                float(number(a[8])), data<float>(out), stream()));
+    const float padding_value = float(number(a[5])), slope = float(number(a[8]));
+    const int32_t act = int32_t(integer(a[7]));
+    const OutSize o(g);
+    at::TensorBase out;
+    launch([&] {
+        out = empty({g.n, g.cout, o.h, o.w}, c10::kFloat, x);
+        return L.tsx_conv2d_f32_nchw(&g, x.const_data_ptr<float>(), w.const_data_ptr<float>(), padding_value, bias, act, slope, data<float>(out),
+                                     stream());
+    });
     return wrap(out);
 }
 
@@ -298,9 +357,15 @@ PyObject *depthwise_conv2d(PyObject *const *a, Py_ssize_t) {          // the sam
     tsx_conv2d_geom g = geometry(x, w, a[2], a[3], a[4]);
     g.cout = g.c;
     const float *bias = f32_or_null(a[6]);
-    at::TensorBase out = conv_out(g, x);
-    check(L.tsx_depthwise_conv2d_f32(&g, x.const_data_ptr<float>(), w.const_data_ptr<float>(), float(number(a[5])), bias, int32_t(integer(a[7])),
-                                     float(number(a[8])), data<float>(out), stream()));
+    const float padding_value = float(number(a[5])), slope = float(number(a[8]));
+    const int32_t act = int32_t(integer(a[7]));
+    const OutSize o(g);
+    at::TensorBase out;
+    launch([&] {
+        out = empty({g.n, g.cout, o.h, o.w}, c10::kFloat, x);
+        return L.tsx_depthwise_conv2d_f32(&g, x.const_data_ptr<float>(), w.const_data_ptr<float>(), padding_value, bias, act, slope, data<float>(out),
+                                          stream());
+    });
     return wrap(out);
 }
 
@@ -310,9 +375,12 @@ PyObject *inner_prod_f32(PyObject *const *a, Py_ssize_t) {            // lhs, rh
     const bool t = truth(a[2]);
     const int64_t k = l.size(1), n = r.size(t ? 0 : 1);
     if (r.size(t ? 1 : 0) != k) throw Decline{};
-    at::TensorBase out = empty({l.size(0), n}, c10::kFloat, l);
-    check(L.tsx_inner_prod_f32(int32_t(l.size(0)), int32_t(n), int32_t(k), l.const_data_ptr<float>(), r.const_data_ptr<float>(), t ? 1 : 0,
-                               data<float>(out), stream()));
+    at::TensorBase out;
+    launch([&] {
+        out = empty({l.size(0), n}, c10::kFloat, l);
+        return L.tsx_inner_prod_f32(int32_t(l.size(0)), int32_t(n), int32_t(k), l.const_data_ptr<float>(), r.const_data_ptr<float>(), t ? 1 : 0,
+                                    data<float>(out), stream());
+    });
     return wrap(out);
 }
 
@@ -326,10 +394,17 @@ PyObject *winograd(PyObject *const *a, Py_ssize_t) {   // mode (0 f23, 1 f63, 2 
                                                                                         : L.tsx_winograd_f63_fast_workspace_bytes(&g);
     if (bytes == 0 || size_t(workspace.numel()) < bytes) throw Decline{};
     const float *bias = f32_or_null(a[7]);
-    at::TensorBase out = conv_out(g, x);
+    const float padding_value = float(number(a[6])), slope = float(number(a[9]));
+    const int32_t act = int32_t(integer(a[8]));
+    const OutSize o(g);
     const auto conv = mode == 0 ? L.tsx_conv2d_winograd_f23_nchw : mode == 1 ? L.tsx_conv2d_winograd_f63_nchw : L.tsx_conv2d_winograd_f63_fast_nchw;
-    check(conv(&g, x.const_data_ptr<float>(), u.const_data_ptr<float>(), float(number(a[6])), bias, int32_t(integer(a[8])), float(number(a[9])),
-               data<float>(out), workspace.mutable_data_ptr(), bytes, stream()));
+    at::TensorBase out;
+    launch([&] {
+        out = empty({g.n, g.cout, o.h, o.w}, c10::kFloat, x);
+        void *ws = workspace.mutable_data_ptr();
+        const WorkspaceLock lock(ws);
+        return conv(&g, x.const_data_ptr<float>(), u.const_data_ptr<float>(), padding_value, bias, act, slope, data<float>(out), ws, bytes, stream());
+    });
     return wrap(out);
 }
 
@@ -398,12 +473,20 @@ PyObject *gemm_i8(PyObject *const *a, Py_ssize_t) {
     const bool with = a[5] != Py_None;
     HeldEpilogue e;
     if (with) e = epilogue({a[5], a[6], a[7], a[8], a[9], a[10], Py_None, Py_None, Py_False});
+    const bool want_f32 = with && truth(a[11]), want_i8 = with && a[10] != Py_None, want_acc = truth(a[12]);
     at::TensorBase out_f32, out_i8, acc;
-    if (with && truth(a[11])) out_f32 = empty({m, n}, c10::kFloat, lhs);
-    if (with && a[10] != Py_None) out_i8 = empty({m, n}, c10::kChar, lhs);
-    if (truth(a[12])) acc = empty({m, n}, c10::kInt, lhs);
-    check(L.tsx_gemm_i8(m, n, k, lhs.const_data_ptr<int8_t>(), packed.const_data_ptr(), with ? &e : nullptr, data<float>(out_f32), data<int8_t>(out_i8),
-                        data<int32_t>(acc), ws, ws_bytes, stream()));
+    launch([&] {
+        if (want_f32) out_f32 = empty({m, n}, c10::kFloat, lhs);
+        if (want_i8) out_i8 = empty({m, n}, c10::kChar, lhs);
+        if (want_acc) acc = empty({m, n}, c10::kInt, lhs);
+        const auto enqueue = [&] {
+            return L.tsx_gemm_i8(m, n, k, lhs.const_data_ptr<int8_t>(), packed.const_data_ptr(), with ? &e : nullptr, data<float>(out_f32),
+                                 data<int8_t>(out_i8), data<int32_t>(acc), ws, ws_bytes, stream());
+        };
+        if (!ws) return enqueue();
+        const WorkspaceLock lock(ws);
+        return enqueue();
+    });
     return Py_BuildValue("(NNN)", wrap(out_f32), wrap(out_i8), wrap(acc));
 }
 
@@ -502,21 +585,24 @@ PyObject *conv_i8(PyObject *const *a, Py_ssize_t) {
     } else if (a[11] != Py_None) {
         throw Decline{};
     }
+    const bool want_f32 = with && truth(a[9]), want_i8 = with && a[7] != Py_None && a[12] == Py_None, want_acc = truth(a[10]);
+    const at::Tensor *xs = fused ? &f32(a[8]) : nullptr;
     at::TensorBase out_f32, out_i8, acc;
-    const int64_t shape[4] = {p.geom.n, p.geom.cout, p.ho, p.wo};
-    if (with && truth(a[9])) out_f32 = empty(shape, c10::kFloat, x);
-    if (with && a[7] != Py_None && a[12] == Py_None) out_i8 = empty(shape, c10::kChar, x);
-    if (truth(a[10])) acc = empty(shape, c10::kInt, x);
-    const tsx_epilogue *ep = with ? &e : nullptr;
-    if (fused) {
-        const at::Tensor &xs = f32(a[8]);
-        check(L.tsx_quantize_conv2d_i8_nchw(&p.geom, x.const_data_ptr<float>(), xs.const_data_ptr<float>(), int32_t(xs.numel()), p.packed.const_data_ptr(),
-                                            st->padding_value, ep, data<float>(out_f32), data<int8_t>(out_i8), data<int32_t>(acc),
-                                            p.workspace.mutable_data_ptr(), p.ws_bytes, stream()));
-    } else {
-        check(L.tsx_conv2d_i8_nchw(&p.geom, x.const_data_ptr<int8_t>(), p.packed.const_data_ptr(), st->padding_value, ep, data<float>(out_f32),
-                                   data<int8_t>(out_i8), data<int32_t>(acc), p.workspace.mutable_data_ptr(), p.ws_bytes, stream()));
-    }
+    launch([&] {
+        const int64_t shape[4] = {p.geom.n, p.geom.cout, p.ho, p.wo};
+        if (want_f32) out_f32 = empty(shape, c10::kFloat, x);
+        if (want_i8) out_i8 = empty(shape, c10::kChar, x);
+        if (want_acc) acc = empty(shape, c10::kInt, x);
+        const tsx_epilogue *ep = with ? &e : nullptr;
+        void *ws = p.workspace.mutable_data_ptr();
+        const WorkspaceLock lock(ws);
+        if (fused)
+            return L.tsx_quantize_conv2d_i8_nchw(&p.geom, x.const_data_ptr<float>(), xs->const_data_ptr<float>(), int32_t(xs->numel()),
+                                                 p.packed.const_data_ptr(), st->padding_value, ep, data<float>(out_f32), data<int8_t>(out_i8),
+                                                 data<int32_t>(acc), ws, p.ws_bytes, stream());
+        return L.tsx_conv2d_i8_nchw(&p.geom, x.const_data_ptr<int8_t>(), p.packed.const_data_ptr(), st->padding_value, ep, data<float>(out_f32),
+                                    data<int8_t>(out_i8), data<int32_t>(acc), ws, p.ws_bytes, stream());
+    });
     return Py_BuildValue("(NNN)", wrap(out_f32), wrap(out_i8), wrap(acc));
 }
 
@@ -530,12 +616,16 @@ PyObject *conv_i8_staged(PyObject *const *a, Py_ssize_t) {
     const at::Tensor &in = i8(buf.o);
     check_residual(a[9], p);
     const HeldEpilogue e = epilogue({a[3], Py_None, a[4], a[5], a[6], a[7], a[9], a[10], a[11]});
+    const int hs = int_attr(a[2], n_hs), ws = int_attr(a[2], n_ws);
+    const bool want_f32 = truth(a[8]), want_i8 = a[7] != Py_None && a[10] == Py_None;
     at::TensorBase out_f32, out_i8;
-    const int64_t shape[4] = {p.geom.n, p.geom.cout, p.ho, p.wo};
-    if (truth(a[8])) out_f32 = empty(shape, c10::kFloat, in);
-    if (a[7] != Py_None && a[10] == Py_None) out_i8 = empty(shape, c10::kChar, in);
-    check(L.tsx_conv2d_i8_staged_at(&p.geom, in.const_data_ptr(), int_attr(a[2], n_hs), int_attr(a[2], n_ws), p.packed.const_data_ptr(), &e,
-                                    data<float>(out_f32), data<int8_t>(out_i8), nullptr, stream()));
+    launch([&] {
+        const int64_t shape[4] = {p.geom.n, p.geom.cout, p.ho, p.wo};
+        if (want_f32) out_f32 = empty(shape, c10::kFloat, in);
+        if (want_i8) out_i8 = empty(shape, c10::kChar, in);
+        return L.tsx_conv2d_i8_staged_at(&p.geom, in.const_data_ptr(), hs, ws, p.packed.const_data_ptr(), &e, data<float>(out_f32), data<int8_t>(out_i8),
+                                         nullptr, stream());
+    });
     return Py_BuildValue("(NN)", wrap(out_f32), wrap(out_i8));
 }
 

@@ -119,6 +119,68 @@ def test_copied_layers_and_networks_compute_the_same(capi, how):
 
 # ---------------------------------------------------------------- threads and re-entry
 
+SLOW = "#include <unistd.h>\nint slow(const void *x, long long n, void *out, void *stream) { usleep(400000); return 0; }\n"
+
+
+@pytest.mark.gpu
+def test_other_threads_run_while_a_launch_waits(capi, tmp_path):
+    """An entry point that blocks, as a launch into a full queue does, stands in for tsx_relu_f32."""
+    import torch
+    source, so = tmp_path / "slow.c", tmp_path / "libslow.so"
+    source.write_text(SLOW)
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(so), str(source)])
+    slow = ctypes.CDLL(str(so)).slow
+    real = {name: ctypes.cast(getattr(capi.lib(), name), ctypes.c_void_p).value for name in capi.SIGNATURES}
+    x = torch.zeros(16, device="cuda")
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            ticks.append(time.perf_counter())
+            time.sleep(0.005)
+
+    thread = threading.Thread(target=tick)
+    capi._native().bind(dict(real, tsx_relu_f32=ctypes.cast(slow, ctypes.c_void_p).value), capi.TsxError)
+    try:
+        thread.start()
+        began = time.perf_counter()
+        capi.relu(x)
+        ended = time.perf_counter()
+    finally:
+        stop.set()
+        thread.join()
+        capi._native().bind(real, capi.TsxError)
+    assert ended - began > 0.39
+    assert sum(began < t < ended for t in ticks) >= 10
+    assert torch.equal(capi.relu(x), x)
+
+
+@pytest.mark.gpu
+def test_threads_share_a_layer(capi):
+    """Four threads call one layer with more shapes than it keeps plans for, on one stream: staging and convolution of a
+    call are enqueued together although the calls share a workspace, and a plan outlives its place among the kept ones."""
+    import torch
+    conv, dq = _layer(capi)
+    inputs = [_input(1 + i % 3, 40, 5 + i, 7 + 2 * i, seed=i) for i in range(12)]
+    want = [conv(x, dq=dq)[0] for x in inputs]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(k):
+        for turn in range(40):
+            i = (5 * turn + 3 * k) % len(inputs)
+            got = conv(inputs[i], dq=dq)[0]
+            if not torch.equal(got, want[i]):
+                wrong.append((k, turn, i))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+
 @pytest.mark.gpu
 def test_a_call_made_while_another_reads_its_arguments(capi):
     """A staged output whose attribute runs the layer on other shapes: the outer call's plan stays what it is."""
