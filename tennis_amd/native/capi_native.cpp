@@ -11,6 +11,7 @@
 
 #include <ATen/core/TensorBase.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -490,12 +491,12 @@ PyObject *gemm_i8(PyObject *const *a, Py_ssize_t) {
     return Py_BuildValue("(NNN)", wrap(out_f32), wrap(out_i8), wrap(acc));
 }
 
-// What one Conv2dI8 has in hand for the input shapes it has seen last: geometry, packed weights, workspace, output size.
+// What one Conv2dI8 has in hand for the input shapes it has seen last: geometry, packed weights, workspace and output size.
 // A call holds the plan it uses: reading the attributes of its other arguments can run Python code, and with it other calls
 // of the layer that replace the plans kept.
 struct Plan {
     tsx_conv2d_geom geom;
-    at::Tensor packed, workspace;
+    at::Tensor packed;
     size_t ws_bytes;
     int32_t ho, wo;
 };
@@ -532,15 +533,21 @@ void conv_state_dealloc(PyObject *o) {
     Py_TYPE(o)->tp_free(o);
 }
 
-// The plan of `layer` (a capi.Conv2dI8) for an input shape; layer._plan makes it, packing the weights where that is due.
-std::shared_ptr<const Plan> conv_plan(ConvState *st, PyObject *layer, int32_t n, int32_t c, int32_t h, int32_t w) {
-    for (const auto &p : *st->plans)
-        if (p->geom.n == n && p->geom.h == h && p->geom.w == w && p->geom.c == c) return p;
-    if (c != st->cin) throw Decline{};
+// layer._plan: packs the weights where that is due and grows layer._workspace to what the shape needs
+PyObject *call_plan(PyObject *layer, int32_t n, int32_t c, int32_t h, int32_t w) {
     PyObject *shape = Py_BuildValue("(iiii)", n, c, h, w);
     PyObject *got = shape ? PyObject_CallMethodObjArgs(layer, n_plan, shape, nullptr) : nullptr;
     Py_XDECREF(shape);
     if (!got) throw Raised{};
+    return got;
+}
+
+// The plan of `layer` (a capi.Conv2dI8) for an input shape
+std::shared_ptr<const Plan> conv_plan(ConvState *st, PyObject *layer, int32_t n, int32_t c, int32_t h, int32_t w) {
+    for (const auto &p : *st->plans)
+        if (p->geom.n == n && p->geom.h == h && p->geom.w == w && p->geom.c == c) return p;
+    if (c != st->cin) throw Decline{};
+    PyObject *got = call_plan(layer, n, c, h, w);
     Plan p;
     const int32_t *k = st->consts;
     p.geom = {n, c, h, w, k[0], k[1], k[2], k[3], k[4], k[5], k[6], k[7], k[8], k[9], k[10]};
@@ -553,14 +560,25 @@ std::shared_ptr<const Plan> conv_plan(ConvState *st, PyObject *layer, int32_t n,
     p.packed = THPVariable_Unpack(packed);
     p.ws_bytes = PyLong_AsSize_t(bytes);
     Py_DECREF(got);
-    Attr ws(layer, n_workspace);
-    p.workspace = tensor(ws.o, c10::kByte);
     check(L.tsx_conv2d_out_size(&p.geom, &p.ho, &p.wo));
     constexpr size_t MOST = 8;        // input shapes a layer keeps plans for
     auto made = std::make_shared<const Plan>(std::move(p));
     if (st->plans->size() < MOST) st->plans->push_back(made);
     else (*st->plans)[st->turn++ % MOST] = made;
     return made;
+}
+
+// The layer's one workspace, as large as the largest shape it has been called with; the call holds it while it enqueues
+at::Tensor conv_workspace(PyObject *layer, const Plan &p) {
+    for (int turn = 0; turn < 2; ++turn) {
+        Attr held(layer, n_workspace);
+        if (held.o != Py_None) {
+            const at::Tensor &t = tensor(held.o, c10::kByte);
+            if (size_t(t.numel()) >= p.ws_bytes) return t;
+        }
+        if (turn == 0) Py_DECREF(call_plan(layer, p.geom.n, p.geom.c, p.geom.h, p.geom.w));
+    }
+    throw Decline{};
 }
 
 void check_residual(PyObject *residual, const Plan &p) {
@@ -587,6 +605,7 @@ PyObject *conv_i8(PyObject *const *a, Py_ssize_t) {
     }
     const bool want_f32 = with && truth(a[9]), want_i8 = with && a[7] != Py_None && a[12] == Py_None, want_acc = truth(a[10]);
     const at::Tensor *xs = fused ? &f32(a[8]) : nullptr;
+    at::TensorBase workspace = conv_workspace(a[1], p);
     at::TensorBase out_f32, out_i8, acc;
     launch([&] {
         const int64_t shape[4] = {p.geom.n, p.geom.cout, p.ho, p.wo};
@@ -594,7 +613,10 @@ PyObject *conv_i8(PyObject *const *a, Py_ssize_t) {
         if (want_i8) out_i8 = empty(shape, c10::kChar, x);
         if (want_acc) acc = empty(shape, c10::kInt, x);
         const tsx_epilogue *ep = with ? &e : nullptr;
-        void *ws = p.workspace.mutable_data_ptr();
+        // a captured graph outlives the layer's workspace, which a larger shape replaces: it gets one of its own pool
+        if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None)
+            workspace = empty({int64_t(p.ws_bytes)}, c10::kByte, x);
+        void *ws = workspace.mutable_data_ptr();
         const WorkspaceLock lock(ws);
         if (fused)
             return L.tsx_quantize_conv2d_i8_nchw(&p.geom, x.const_data_ptr<float>(), xs->const_data_ptr<float>(), int32_t(xs->numel()),

@@ -207,3 +207,46 @@ def test_a_call_made_while_another_reads_its_arguments(capi):
     busy = Busy(consumer, (2, 48, 12, 13))
     got = conv(x, staged_out=busy, **kw)[0]
     assert torch.equal(got, want) and torch.equal(busy.buf, plain.buf)
+
+
+# ---------------------------------------------------------------- workspaces
+
+@pytest.mark.gpu
+def test_a_larger_shape_gives_the_smaller_workspace_back(capi):
+    import torch
+    conv, dq = _layer(capi, c=64)
+    shapes = [(1, 64, 180 + 40 * i, 256) for i in range(6)]
+    small = _input(*shapes[0])
+    conv(small, dq=dq)                                # weights packed
+    del small
+    conv._workspace = None
+    before = torch.cuda.memory_allocated()
+    first = None
+    for shape in shapes:
+        out = conv(_input(*shape), dq=dq)[0]
+        first = out.cpu() if first is None else first
+        del out
+    kept = torch.cuda.memory_allocated() - before
+    assert kept <= conv._workspace.numel() + 4096, (kept, conv._workspace.numel())
+    assert torch.equal(conv(_input(*shapes[0]), dq=dq)[0].cpu(), first)
+
+
+@pytest.mark.gpu
+def test_a_captured_layer_outlives_its_workspace(capi):
+    """A larger shape replaces the layer's workspace; a graph captured before goes on with memory of its own."""
+    import torch
+    conv, dq = _layer(capi)
+    x = _input(2, 40, 14, 15)
+    want = conv(x, dq=dq)[0]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = conv(x, dq=dq)[0]
+    large = _input(4, 40, 60, 62)
+    for turn in range(3):
+        conv(large, dq=dq)
+        small = torch.full((conv._workspace.numel(),), 77, dtype=torch.int8, device="cuda")    # where a freed workspace would lie
+        out.zero_()
+        graph.replay()
+        assert torch.equal(out, want) and (small == 77).all(), turn
+        large = torch.cat([large, large])
