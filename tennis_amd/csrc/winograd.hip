@@ -40,8 +40,9 @@
 namespace tsx {
 namespace {
 
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef float v4f __attribute__((ext_vector_type(4)));
+// U and V are float arrays to the caller: 16- and 8-byte accesses at any float's address (the instructions are the same)
+typedef float v2f __attribute__((ext_vector_type(2), aligned(4)));
+typedef float v4f __attribute__((ext_vector_type(4), aligned(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 // ---------------------------------------------------------------- transforms (explicit FMAs)
@@ -584,8 +585,6 @@ int conv2d(const tsx_conv2d_geom *q, const float *x, const float *u, float paddi
     constexpr int FREQS = (TILE + 2) * (TILE + 2);
     const size_t need = workspace_bytes(q, TILE);
     if (!workspace || bytes < need) return fail(TSX_E_WORKSPACE, "winograd: workspace %zu < %zu bytes", bytes, need);
-    TSX_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && reinterpret_cast<uintptr_t>(u) % 16 == 0,
-                "winograd: workspace and transformed kernel must be 16-byte aligned");
     TSX_REQUIRE(g.cout <= 65535 * WT_CH && g.kgroups <= 32767, "winograd: too many channels");
     float *v = static_cast<float *>(workspace), *m = v + operand_floats(g, FREQS);
     if (TILE == 6)

@@ -34,3 +34,32 @@ def test_winograd_gemm_edges(port, case, mode):
     got = op(torch.from_numpy(x).cuda()).cpu().numpy()
     exp = getattr(port, "winograd_" + mode)(x, wt, (1, 1, 1, 1), padding_value=0.25)
     assert np.array_equal(bits(got), bits(exp)), (bits(got) != bits(exp)).mean()
+
+
+@pytest.mark.parametrize("entry", ["f63", "f63_fast", "f23"])
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_winograd_operands_at_any_float_address(port, entry, offset):
+    """Workspace and transformed kernel one to three floats behind a 16-byte boundary: both are float arrays, no more."""
+    import ctypes
+    import torch
+    from tennis_amd import capi
+    n, c, h, w, cout = 2, 13, 28, 30, 40
+    rng = np.random.default_rng(offset)
+    x = rng.uniform(-1, 1, (n, c, h, w)).astype(np.float32)
+    wt = rng.standard_normal((cout, c, 3, 3)).astype(np.float32)
+    L, mode = capi.lib(), entry[:3]
+    xd, wd = torch.from_numpy(x).cuda(), torch.from_numpy(wt).cuda()
+    geom = capi.make_geom(x.shape, wt.shape, (1, 1, 1, 1))
+    need = getattr(L, "tsx_winograd_%s_workspace_bytes" % entry)(ctypes.byref(geom))
+    u = torch.zeros(getattr(L, "tsx_winograd_%s_kernel_bytes" % mode)(cout, c) // 4 + 8, device="cuda")
+    workspace = torch.full((need // 4 + 8,), float("nan"), device="cuda")
+    out = torch.empty((n, cout, h, w), device="cuda")
+    at = ctypes.c_void_p(u.data_ptr() + 4 * offset)
+    capi.check(getattr(L, "tsx_winograd_%s_transform_kernel" % mode)(cout, c, capi._ptr(wd), at, capi._stream()))
+    capi.check(getattr(L, "tsx_conv2d_winograd_%s_nchw" % entry)(ctypes.byref(geom), capi._ptr(xd), at, 0.0, None, 0, 0.0, capi._ptr(out),
+                                                                 ctypes.c_void_p(workspace.data_ptr() + 4 * offset), need, capi._stream()))
+    exp = getattr(port, "winograd_" + mode)(x, wt, (1, 1, 1, 1))
+    assert np.array_equal(bits(out.cpu().numpy()), bits(exp))
+    # and nothing beside the two ranges was written
+    assert torch.isnan(workspace[:offset]).all() and torch.isnan(workspace[need // 4 + offset:]).all()
+    assert (u[:offset] == 0).all() and (u[u.numel() - 8 + offset:] == 0).all()
