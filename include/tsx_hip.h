@@ -328,8 +328,9 @@ int tsx_max_pooling2d_i8_staged(const tsx_staged_map *src, const tsx_staged_map 
  * (include/backend/base/base_conv2d_winograd.h:24-27):
  *   conv2d_tranform_kernel(mode, kernel, kernel_transformed)  -> tsx_winograd_f63_transform_kernel
  *   conv2d_winograd(x, mode, padding, padding_value, w, ...)   -> tsx_conv2d_winograd_f63_nchw
- * 3x3 kernels, stride 1, dilation 1 only.  The transformed kernel u_dev ([64][cout][cin] floats,
- * tsx_winograd_f63_kernel_bytes) is this backend's own layout, produced and consumed only here.
+ * 3x3 kernels, stride 1, dilation 1 only.  The transformed kernel u_dev (tsx_winograd_f63_kernel_bytes) and the
+ * workspace (tsx_winograd_f63_workspace_bytes: the transformed input and the 64 products) are float arrays at any
+ * address a float may have; their layouts are this backend's own, produced and consumed only here.
  * Transforms and accumulation order restate the reference's arithmetic exactly (including the
  * fused multiply-adds of its AVX2/FMA build), so results match its F(6,3) to the bit; optional
  * bias/activation are the add_bias / relu operators fused behind the output transform. */
@@ -339,13 +340,9 @@ size_t tsx_winograd_f63_workspace_bytes(const tsx_conv2d_geom *g);
 int tsx_conv2d_winograd_f63_nchw(const tsx_conv2d_geom *g, const float *x_dev, const float *u_dev, float padding_value,
                                  const float *bias_dev, int32_t act, float slope, float *out_dev, void *workspace_dev,
                                  size_t workspace_bytes, void *stream);
-/* The same operator (same u_dev, same arguments) with the 64 frequency GEMMs on the fp32 MFMA and the output
- * transform fused behind them: two launches instead of three, the products M never reach memory, workspace = the
- * transformed input only (tsx_winograd_f63_fast_workspace_bytes).  The MFMA sums the channel products in another
- * order than the reference's FMA chains, so this entry is held to a floating-point bar -- the one TenniS's own
- * backend test applies between devices, max 1e-4 / mean 1e-5 (tools/run_test/test_case.hpp:491-503) -- against
- * winograd_f63 (src/kernels/cpu/winograd_algorithm.cpp:846-947), not to its bits; tsx_conv2d_winograd_f63_nchw is
- * the bit-exact one. */
+/* The same operator (same u_dev, same arguments) for callers content with a floating-point bar -- the one TenniS's
+ * own backend test applies between devices, max 1e-4 / mean 1e-5 (tools/run_test/test_case.hpp:491-503).  It promises
+ * no more; today the exact form is also the fastest one and this entry runs it, with the workspace of the exact form. */
 size_t tsx_winograd_f63_fast_workspace_bytes(const tsx_conv2d_geom *g);
 int tsx_conv2d_winograd_f63_fast_nchw(const tsx_conv2d_geom *g, const float *x_dev, const float *u_dev, float padding_value,
                                       const float *bias_dev, int32_t act, float slope, float *out_dev, void *workspace_dev,
@@ -355,8 +352,7 @@ int tsx_conv2d_winograd_f63_fast_nchw(const tsx_conv2d_geom *g, const float *x_d
  * Conv2dWinogradAlgorithm<float>::winograd_f23 (src/kernels/cpu/winograd_algorithm.cpp:347-459), the
  * mode base::Conv2DWinograd picks unless Cin*Cout >= 256*256 on maps larger than 16x16
  * (KernelCommonFunc::winograd_mode_select_on_arm, src/kernels/common/function.cpp:154-173).  Same
- * contract as the F(6,3) calls above with 16 instead of 64 tile positions (u_dev is [16][cout][cin]);
- * results match the reference's F(2,3) to the bit. */
+ * contract as the F(6,3) calls above with 16 instead of 64 tile positions; results match the reference's F(2,3) to the bit. */
 size_t tsx_winograd_f23_kernel_bytes(int32_t cout, int32_t cin);
 int tsx_winograd_f23_transform_kernel(int32_t cout, int32_t cin, const float *w_oihw_dev, float *u_dev, void *stream);
 size_t tsx_winograd_f23_workspace_bytes(const tsx_conv2d_geom *g);

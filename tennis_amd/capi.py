@@ -647,7 +647,7 @@ class Winograd:
         self._workspace = None
 
     def __call__(self, x, bias=None, act=None, slope=0.0, fast=False):
-        """fast (f63 only): the MFMA form, held to the fp32 tolerance instead of the reference's bits."""
+        """fast (f63 only): the entry that promises the fp32 tolerance only (the exact form serves it as well)."""
         if self.mode == "f63" or not fast:
             out = _native_module.winograd((2 if fast else 1) if self.mode == "f63" else 0, x, self.w, self.u, self._workspace, self.pads,
                                           self.padding_value, bias, _ACT[act], slope)
