@@ -192,9 +192,10 @@ int launch_affine(const char *who, const float *x, int64_t pre, int channels, in
     TSX_REQUIRE(x && out, "%s: null pointer", who);
     const bool vec = reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
     const int64_t planes = pre * channels;
-    if (vec && inner % 4 == 0 && inner >= 256 && inner < (int64_t(1) << 31) && planes >= 1024 && planes < (int64_t(1) << 32)) {
-        // enough planes to fill the chip, large enough to fill a wavefront
-        hipLaunchKernelGGL(plane_affine_kernel<NORM>, dim3(unsigned(tsx::ceil_div(planes, 4))), dim3(256), 0, tsx::as_stream(stream), x, planes, channels,
+    const int64_t plane_blocks = tsx::ceil_div(planes, 4);
+    if (vec && inner % 4 == 0 && inner >= 256 && inner < (int64_t(1) << 31) && planes >= 1024 && plane_blocks * 256 < (int64_t(1) << 32)) {
+        // enough planes to fill the chip, large enough to fill a wavefront, and no more than a launch holds
+        hipLaunchKernelGGL(plane_affine_kernel<NORM>, dim3(unsigned(plane_blocks)), dim3(256), 0, tsx::as_stream(stream), x, planes, channels,
                            int(inner / 4), mean, variance, scale, bias, epsilon, out);
         TSX_LAUNCH_CHECK("plane_affine_kernel");
         return 0;

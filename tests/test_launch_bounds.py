@@ -1,0 +1,77 @@
+"""The grids of kernels that take a plane or more per workgroup, at extents no test allocates: a launch holds fewer than
+2^32 work items along an axis, so beyond that a kernel with capped or smaller grids has to run.  The library is loaded in a
+process where the runtime's launch calls are recorded and not carried out: no device and no memory are needed."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+RECORDER = r"""
+#include <stddef.h>
+#include <stdint.h>
+typedef struct { uint32_t x, y, z; } dims;
+static dims grid, block;
+uint32_t last[6];
+int launches;
+unsigned __hipPushCallConfiguration(dims g, dims b, size_t shared, void *stream) { grid = g; block = b; return 0; }
+unsigned __hipPopCallConfiguration(dims *g, dims *b, size_t *shared, void **stream) { *g = grid; *b = block; *shared = 0; *stream = 0; return 0; }
+int hipLaunchKernel(const void *f, dims g, dims b, void **args, size_t shared, void *stream) {
+    last[0] = g.x, last[1] = g.y, last[2] = g.z, last[3] = b.x, last[4] = b.y, last[5] = b.z;
+    ++launches;
+    return 0;
+}
+int hipGetLastError(void) { return 0; }
+"""
+
+CALLS = r"""
+import ctypes, json, sys
+recorder = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+L = ctypes.CDLL(sys.argv[2])
+i32, i64, f32, p = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
+L.tsx_batch_norm_f32.argtypes = [p, i64, i32, i64, p, p, f32, p, p]
+L.tsx_batch_scale_f32.argtypes = [p, i64, i32, i64, p, p, p, p]
+L.tsx_fused_batch_norm_f32.argtypes = [p, i64, i32, i64, p, p, p, p, f32, p, p]
+L.tsx_pooling2d_f32.argtypes = [p, i64] + [i32] * 10 + [p, i32, i32, p]
+last = (ctypes.c_uint32 * 6).in_dll(recorder, "last")
+launches = ctypes.c_int.in_dll(recorder, "launches")
+at = 1 << 20                      # an address that nothing reads
+out = []
+for what, planes, extent in json.loads(sys.argv[3]):
+    launches.value = 0
+    if what == "batch_norm":
+        rc = L.tsx_batch_norm_f32(at, planes, 1, extent, at, at, 1e-5, at, None)
+    elif what == "batch_scale":
+        rc = L.tsx_batch_scale_f32(at, planes, 1, extent, at, at, at, None)
+    elif what == "fused_batch_norm":
+        rc = L.tsx_fused_batch_norm_f32(at, planes, 1, extent, at, at, at, at, 1e-5, at, None)
+    else:
+        rc = L.tsx_pooling2d_f32(at, planes, extent, 4, what == "avg", 0, 0, extent, 4, 1, 1, 0, at, 1, 1, None)
+    out.append([rc, launches.value, list(last)])
+print(json.dumps(out))
+"""
+
+CASES = [[what, planes, extent] for what in ("batch_norm", "batch_scale", "fused_batch_norm") for extent in (256, 1024)
+         for planes in (1024, (1 << 26) - 4, (1 << 26) - 3, 1 << 26, (1 << 26) + 1, (1 << 28) + 5, (1 << 31) + 7)]
+
+
+@pytest.fixture(scope="module")
+def recorded(tmp_path_factory):
+    from tennis_amd.build import LIB_PATH
+    where = tmp_path_factory.mktemp("recorder")
+    source, so = where / "recorder.c", where / "librecorder.so"
+    source.write_text(RECORDER)
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(so), str(source)])
+    run = subprocess.run([sys.executable, "-c", CALLS, str(so), LIB_PATH, json.dumps(CASES)], capture_output=True, text=True, cwd=ROOT)
+    assert run.returncode == 0, run.stderr
+    return json.loads(run.stdout)
+
+
+@pytest.mark.parametrize("i", range(len(CASES)), ids=lambda i: "%s-%d-%d" % tuple(CASES[i]))
+def test_planes_fit_a_launch(recorded, i):
+    rc, launches, (gx, gy, gz, bx, by, bz) = recorded[i]
+    assert rc == 0 and launches == 1
+    assert gx * bx < 1 << 32 and gy * by < 1 << 32 and gz * bz < 1 << 32, (gx, bx)
