@@ -319,10 +319,13 @@ int tsx_pooling2d_f32(const float *x_dev, int64_t planes, int32_t h, int32_t w, 
     const int64_t total = planes * out_h * out_w;
     TSX_REQUIRE(tsx::ceil_div(total, 256) < (int64_t(1) << 31), "pooling2d: tensor too large");
     const dim3 grid(unsigned(tsx::ceil_div(total, 256)));
-    // one window over the whole map and planes enough of elements that a lane's walk is what takes the time
-    if (out_h == 1 && out_w == 1 && pad_top == 0 && pad_left == 0 && kh >= h && kw >= w && h * int64_t(w) >= 16 && int64_t(h) * w < (1 << 30)) {
+    // one window over the whole map and planes enough of elements that a lane's walk is what takes the time (and no more planes
+    // than a launch holds: from 2^28 on a lane each has to do)
+    const int64_t plane_blocks = tsx::ceil_div(planes, GP_PLANES);
+    if (out_h == 1 && out_w == 1 && pad_top == 0 && pad_left == 0 && kh >= h && kw >= w && h * int64_t(w) >= 16 && int64_t(h) * w < (1 << 30) &&
+        plane_blocks * 256 < (int64_t(1) << 32)) {
         const float divisor = white_padding ? float(kh * kw) : float(h * w);
-        hipLaunchKernelGGL(global_pooling2d_kernel, dim3(unsigned(tsx::ceil_div(planes, GP_PLANES))), dim3(256), 0, tsx::as_stream(stream), x_dev,
+        hipLaunchKernelGGL(global_pooling2d_kernel, dim3(unsigned(plane_blocks)), dim3(256), 0, tsx::as_stream(stream), x_dev,
                            planes, h * w, type, divisor, out_dev);
         TSX_LAUNCH_CHECK("global_pooling2d_kernel");
         return 0;

@@ -54,8 +54,10 @@ for what, planes, extent in json.loads(sys.argv[3]):
 print(json.dumps(out))
 """
 
-CASES = [[what, planes, extent] for what in ("batch_norm", "batch_scale", "fused_batch_norm") for extent in (256, 1024)
-         for planes in (1024, (1 << 26) - 4, (1 << 26) - 3, 1 << 26, (1 << 26) + 1, (1 << 28) + 5, (1 << 31) + 7)]
+CASES = ([[what, planes, extent] for what in ("batch_norm", "batch_scale", "fused_batch_norm") for extent in (256, 1024)
+          for planes in (1024, (1 << 26) - 4, (1 << 26) - 3, 1 << 26, (1 << 26) + 1, (1 << 28) + 5, (1 << 31) + 7)] +
+         [[what, planes, extent] for what in ("max", "avg") for extent in (4, 56)
+          for planes in (1, (1 << 28) - 16, (1 << 28) - 15, 1 << 28, (1 << 28) + 1, (1 << 32) - 256)])
 
 
 @pytest.fixture(scope="module")
