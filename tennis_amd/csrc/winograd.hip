@@ -407,14 +407,13 @@ __device__ __forceinline__ void wino_gemm_tail(const float *__restrict__ u, cons
     }
 }
 
+// A launch takes the column blocks from `first` on, of col_blocks blocks of FN fragments and, behind them, the tail's fragments.
 template <int FN>
 __global__ __launch_bounds__(256) void wino_gemm_kernel(const float *__restrict__ u, const float *__restrict__ v, float *__restrict__ m, WinoGeom g,
-                                                       int row_blocks, int col_blocks) {
+                                                       int row_blocks, int col_blocks, int first) {
     const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const int per_f = row_blocks * (col_blocks + g.nfrags - g.mfrags);
-    const int slot = blockIdx.x >> 3;
-    const int f = (blockIdx.x & 7) + 8 * (slot / per_f);     // frequencies are a multiple of 8, so is the grid
-    const int item = slot % per_f, cb = item / row_blocks;
+    const int f = (blockIdx.x & 7) + 8 * blockIdx.y;         // frequencies are a multiple of 8, so is a row of the grid
+    const int item = blockIdx.x >> 3, cb = first + item / row_blocks;
     const int rf = (item % row_blocks) * 4 + wave;
     if (rf >= g.rfrags) return;
     if (cb < col_blocks)
@@ -599,13 +598,14 @@ int conv2d(const tsx_conv2d_geom *q, const float *x, const float *u, float paddi
     const int row_blocks = (g.rfrags + 3) / 4, tails = g.nfrags - g.mfrags;
     const bool two = int64_t(FREQS) * g.rfrags * ((g.mfrags + 1) / 2) >= 2048;
     const int col_blocks = two ? (g.mfrags + 1) / 2 : g.mfrags;
-    const int64_t blocks = int64_t(FREQS) * row_blocks * (col_blocks + tails);
-    TSX_REQUIRE(blocks < (int64_t(1) << 31), "winograd: tensor too large");
-    if (two)
-        hipLaunchKernelGGL(wino_gemm_kernel<2>, dim3(unsigned(blocks)), dim3(256), 0, stream, u, v, m, g, row_blocks, col_blocks);
-    else
-        hipLaunchKernelGGL(wino_gemm_kernel<1>, dim3(unsigned(blocks)), dim3(256), 0, stream, u, v, m, g, row_blocks, col_blocks);
-    TSX_LAUNCH_CHECK("wino_gemm_kernel");
+    // one launch, except where its work items would be 2^32 or more
+    const int all = col_blocks + tails, most = int(((int64_t(1) << 24) - 1) / (8 * row_blocks));
+    for (int first = 0; first < all; first += most) {
+        const dim3 grid(8u * unsigned(row_blocks) * unsigned(std::min(most, all - first)), FREQS / 8);
+        if (two) hipLaunchKernelGGL(wino_gemm_kernel<2>, grid, dim3(256), 0, stream, u, v, m, g, row_blocks, col_blocks, first);
+        else hipLaunchKernelGGL(wino_gemm_kernel<1>, grid, dim3(256), 0, stream, u, v, m, g, row_blocks, col_blocks, first);
+        TSX_LAUNCH_CHECK("wino_gemm_kernel");
+    }
 
     const int64_t body = int64_t(g.n) * g.cout * g.ho * g.wo / 4 * 4;
     const bool mish = act >= TSX_ACT_MISH;

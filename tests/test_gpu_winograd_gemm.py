@@ -63,3 +63,22 @@ def test_winograd_operands_at_any_float_address(port, entry, offset):
     # and nothing beside the two ranges was written
     assert torch.isnan(workspace[:offset]).all() and torch.isnan(workspace[need // 4 + offset:]).all()
     assert (u[:offset] == 0).all() and (u[u.numel() - 8 + offset:] == 0).all()
+
+
+def test_winograd_products_in_several_launches(port):
+    """More blocks of columns than one launch holds (8.4 million images of 12 tiles, 8 of them chains and 4 tail columns):
+    the same bits as the images in parts that take one launch each."""
+    import torch
+    from tennis_amd import capi
+    n, h, w = (1 << 23) + 4097, 6, 8
+    if torch.cuda.mem_get_info()[0] < 96 << 30:
+        pytest.skip("needs 64 GiB of device memory")
+    wt = torch.randn((1, 1, 3, 3), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    x = torch.randn((n, 1, h, w), device="cuda", generator=torch.Generator(device="cuda").manual_seed(2))
+    op = capi.Winograd(wt, (1, 1, 1, 1), mode="f23")
+    whole = op(x)
+    part = (1 << 20) + 33
+    for first in range(0, n, part):
+        assert torch.equal(whole[first:first + part], op(x[first:first + part])), first
+    some = x[-5:].cpu().numpy()
+    assert np.array_equal(bits(whole[-5:].cpu().numpy()), bits(port.winograd_f23(some, wt.cpu().numpy(), (1, 1, 1, 1))))
