@@ -50,3 +50,42 @@ def test_conv_f32_window_tiles(port, monkeypatch, tile):
         assert got.shape == exp.shape and np.array_equal(bits(got), bits(exp)), case
         ran += 1
     assert ran >= 3
+
+
+@pytest.mark.parametrize("padding_value", [np.nan, np.inf, 3.0])
+@pytest.mark.parametrize("tile", range(10))
+def test_conv_f32_window_tiles_not_finite(port, monkeypatch, tile, padding_value):
+    """NaN and infinities stay where the windows that hold them are: in the padding, in the last channels (a chunk that is not
+    full reads other data behind them), and all over the last image, whose elements lie next to those of the one before.
+    Sums of them do not depend on the order; all else is small integers."""
+    import torch
+    from tennis_amd import capi
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    for env in ("TSX_CONV_F32_SMALL", "TSX_GEMM_F32_REGFED"):
+        monkeypatch.setenv(env, "0")
+    monkeypatch.setenv("TSX_CONV_F32_TILE", str(tile))
+    rng = np.random.default_rng(78)
+    ran = 0
+    for case in LAYERS:
+        n, c, h, w, cout, kh, kw, pads, st, dl = case
+        if kh * kw == 1 and tile % 2 == 0:
+            continue
+        x = rng.integers(-8, 9, (n, c, h, w)).astype(np.float32)
+        x[0, c - 1, h // 2, w // 3] = np.inf
+        x[0, 0, 0, w - 1] = -np.inf
+        x[0, c // 2, h - 1, 0] = np.nan
+        if n > 1:
+            x[n - 1] = np.nan
+        wt = rng.integers(-4, 5, (cout, c, kh, kw)).astype(np.float32)
+        wt[cout - 1, c - 1, 0, 0] = np.inf
+        try:
+            got = capi.conv2d_f32(dev(x), dev(wt), pads, st, dl, padding_value=padding_value).cpu().numpy()
+        except capi.TsxError as e:
+            assert "does not suit" in str(e), case
+            continue
+        exp = port.conv2d_f32(x, wt, pads, st, dl, padding_value=padding_value)
+        nan = np.isnan(exp)
+        assert np.array_equal(np.isnan(got), nan) and np.array_equal(bits(got[~nan]), bits(exp[~nan])), case
+        assert not nan.all(), case
+        ran += 1
+    assert ran >= 3
