@@ -431,15 +431,20 @@ class Conv2dI8:
         self._make_state()
 
     def _make_state(self):
-        # what the native calls keep for this object alone: neither copied nor stored, a copy has its own
+        # what belongs to this object alone, neither copied nor stored: the native calls' state, and workspaces in graphs
+        self._graph_workspaces = []
         self._state = _native().ConvState(self.w, self.pads, self.strides, self.dilations, self.padding_value)
 
     def __getstate__(self):
-        return {k: v for k, v in self.__dict__.items() if k != "_state"}
+        return {k: v for k, v in self.__dict__.items() if k not in ("_state", "_graph_workspaces")}
 
     def __setstate__(self, state):
         self.__dict__.update(state)
         self._make_state()
+
+    def _keep_for_graph(self, workspace):
+        if not any(t is workspace for t in self._graph_workspaces):
+            self._graph_workspaces.append(workspace)
 
     def _plan(self, x_shape):
         geom = make_geom(x_shape, self.w.shape, self.pads, self.strides, self.dilations)

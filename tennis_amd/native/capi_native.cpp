@@ -104,7 +104,7 @@ struct Attr {                         // a new reference, released
     Attr(const Attr &) = delete;
     Attr &operator=(const Attr &) = delete;
 };
-PyObject *n_buf, *n_hs, *n_ws, *n_cp, *n_pad_top, *n_pad_left, *n_upsample, *n_x_shape, *n_plan, *n_workspace;
+PyObject *n_buf, *n_hs, *n_ws, *n_cp, *n_pad_top, *n_pad_left, *n_upsample, *n_x_shape, *n_plan, *n_workspace, *n_keep;
 int int_attr(PyObject *of, PyObject *name) { return int(integer(Attr(of, name).o)); }
 
 // ---- results
@@ -574,7 +574,15 @@ at::Tensor conv_workspace(PyObject *layer, const Plan &p) {
         Attr held(layer, n_workspace);
         if (held.o != Py_None) {
             const at::Tensor &t = tensor(held.o, c10::kByte);
-            if (size_t(t.numel()) >= p.ws_bytes) return t;
+            if (size_t(t.numel()) >= p.ws_bytes) {
+                // a graph that is being captured goes on writing it when a larger shape has replaced it
+                if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) {
+                    PyObject *none = PyObject_CallMethodObjArgs(layer, n_keep, held.o, nullptr);
+                    if (!none) throw Raised{};
+                    Py_DECREF(none);
+                }
+                return t;
+            }
         }
         if (turn == 0) Py_DECREF(call_plan(layer, p.geom.n, p.geom.c, p.geom.h, p.geom.w));
     }
@@ -605,7 +613,7 @@ PyObject *conv_i8(PyObject *const *a, Py_ssize_t) {
     }
     const bool want_f32 = with && truth(a[9]), want_i8 = with && a[7] != Py_None && a[12] == Py_None, want_acc = truth(a[10]);
     const at::Tensor *xs = fused ? &f32(a[8]) : nullptr;
-    at::TensorBase workspace = conv_workspace(a[1], p);
+    const at::Tensor workspace = conv_workspace(a[1], p);
     at::TensorBase out_f32, out_i8, acc;
     launch([&] {
         const int64_t shape[4] = {p.geom.n, p.geom.cout, p.ho, p.wo};
@@ -613,9 +621,6 @@ PyObject *conv_i8(PyObject *const *a, Py_ssize_t) {
         if (want_i8) out_i8 = empty(shape, c10::kChar, x);
         if (want_acc) acc = empty(shape, c10::kInt, x);
         const tsx_epilogue *ep = with ? &e : nullptr;
-        // a captured graph outlives the layer's workspace, which a larger shape replaces: it gets one of its own pool
-        if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None)
-            workspace = empty({int64_t(p.ws_bytes)}, c10::kByte, x);
         void *ws = workspace.mutable_data_ptr();
         const WorkspaceLock lock(ws);
         if (fused)
@@ -690,7 +695,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_tsx_native", "The host work of te
 PyMODINIT_FUNC PyInit__tsx_native() {
     struct { PyObject **at; const char *name; } names[] = {
         {&n_buf, "buf"}, {&n_hs, "hs"}, {&n_ws, "ws"}, {&n_cp, "cp"}, {&n_pad_top, "pad_top"}, {&n_pad_left, "pad_left"},
-        {&n_upsample, "upsample"}, {&n_x_shape, "x_shape"}, {&n_plan, "_plan"}, {&n_workspace, "_workspace"}};
+        {&n_upsample, "upsample"}, {&n_x_shape, "x_shape"}, {&n_plan, "_plan"}, {&n_workspace, "_workspace"}, {&n_keep, "_keep_for_graph"}};
     for (auto &n : names)
         if (!(*n.at = PyUnicode_InternFromString(n.name))) return nullptr;
     conv_state_type.tp_name = "_tsx_native.ConvState";

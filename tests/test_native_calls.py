@@ -233,7 +233,7 @@ def test_a_larger_shape_gives_the_smaller_workspace_back(capi):
 
 @pytest.mark.gpu
 def test_a_captured_layer_outlives_its_workspace(capi):
-    """A larger shape replaces the layer's workspace; a graph captured before goes on with memory of its own."""
+    """A larger shape replaces the layer's workspace; a graph captured before goes on with the one it was captured with."""
     import torch
     conv, dq = _layer(capi)
     x = _input(2, 40, 14, 15)
@@ -250,3 +250,4 @@ def test_a_captured_layer_outlives_its_workspace(capi):
         graph.replay()
         assert torch.equal(out, want) and (small == 77).all(), turn
         large = torch.cat([large, large])
+    assert len(conv._graph_workspaces) == 1 and copy.deepcopy(conv)._graph_workspaces == []
