@@ -35,7 +35,7 @@ CFG = dict(n=32, c=256, h=28, w=28, cout=256, k=3, pad=1)
 # HBM bytes per launch of the two kernels on this workload, from rocprofv3 FETCH_SIZE / WRITE_SIZE scaled by a
 # known-size copy (profiles/conv2d_i8_config2_hbm_traffic.txt); a profiler figure, not measured by this script.
 TRAFFIC_CONV_BYTES = 43.02e6
-TRAFFIC_STAGE_BYTES = 32.54e6
+TRAFFIC_STAGE_BYTES = 32.62e6
 
 
 def make_inputs(cfg, seed=1234):
@@ -109,8 +109,8 @@ def cpu_baseline_all_cores(x, x_scales, wq, dq, bias, pad):
 
 
 def _fp32_conv_rows(shape_x, shape_w, reps, seed):
-    """conv2d_f32 (implicit im2col GEMM on the fp32 MFMA), both Winograd modes in their bit-exact form and F(6,3) as
-    one MFMA launch on one 3x3 / stride 1 / pad 1 layer with bias + ReLU, all credited the direct convolution's
+    """conv2d_f32 (the direct convolution; its row keeps the name im2col_gemm), both Winograd modes and F(6,3) through
+    its tolerance-based entry on one 3x3 / stride 1 / pad 1 layer with bias + ReLU, all credited the direct convolution's
     flops; seconds per launch = median of 5 batches of `reps` back-to-back launches between events."""
     import torch
     from tennis_amd import capi
@@ -156,7 +156,7 @@ def config1_leg(reps=50):
 def winograd_shape_leg(reps=20):
     """A layer the reference's own selector gives to Winograd F(6,3) (winograd_mode_select_on_arm,
     src/kernels/common/function.cpp:154-173: Cin * Cout >= 65536 and a map larger than 16 x 16): 8x256x28x28 *
-    256x256x3x3, stride 1, pad 1, bias + ReLU -- the same four kernels as on config 1."""
+    256x256x3x3, stride 1, pad 1, bias + ReLU -- the same four calls as on config 1."""
     flops, rows = _fp32_conv_rows((8, 256, 28, 28), (256, 256, 3, 3), reps, 6)
     return {"workload": "fp32 conv2d 8x256x28x28 * 256x256x3x3 s1 p1 + bias + ReLU (a shape the reference routes to Winograd "
                         "F(6,3)); %.2f GFLOP per launch by the direct convolution's count" % (flops / 1e9),
@@ -417,11 +417,12 @@ def kernels_leg(reps=20):
     # fp32 on a shape the reference's selector routes to Winograd F(6,3): 8x256x28x28 * 256x256x3x3
     x8, w8, b8 = torch.rand((8, 256, 28, 28), device=dev) * 2 - 1, rnd(256, 256, 3, 3) * 0.03, rnd(256) * 0.01
     flops8 = 2.0 * 8 * 256 * 28 * 28 * 256 * 9
-    timed("conv2d_f32 8x256x28x28 (gemm_f32_kernel)", "mfma_f32", flops8, lambda: capi.conv2d_f32(x8, w8, (1, 1, 1, 1), bias=b8, act="relu"))
+    timed("conv2d_f32 8x256x28x28 (conv_f32_window_kernel)", "mfma_f32", flops8, lambda: capi.conv2d_f32(x8, w8, (1, 1, 1, 1), bias=b8, act="relu"))
     w63b = capi.WinogradF63(w8, (1, 1, 1, 1))
-    timed("winograd F(6,3) 8x256x28x28, bit-exact form (direct-conv flops)", "mfma_f32", flops8, lambda: w63b(x8, bias=b8, act="relu"))
-    timed("winograd F(6,3) 8x256x28x28, one MFMA launch (direct-conv flops)", "mfma_f32", flops8,
-          lambda: w63b(x8, bias=b8, act="relu", fast=True))
+    timed("winograd F(6,3) 8x256x28x28 (direct-conv flops)", "mfma_f32", flops8, lambda: w63b(x8, bias=b8, act="relu"))
+    x11, w11 = rnd(32, 256, 56, 56), rnd(256, 256, 1, 1) * 0.06
+    timed("conv2d_f32 1x1 256->256 @56x56 bs32 (conv_f32_window_kernel)", "mfma_f32", 2.0 * 32 * 256 * 56 * 56 * 256, lambda: capi.conv2d_f32(x11, w11))
+    del x11
     # int8 GEMM: largest and a mid shape of BASELINE config 3, and the weight-streaming single row
     k = n = 4096
     gemm = capi.GemmI8(ri8(k, n))
@@ -429,12 +430,16 @@ def kernels_leg(reps=20):
     for m in (4096, 256, 1):
         a, rs = ri8(m, k), torch.rand(m, device=dev) * 1e-2
         if m > 32:
-            timed("gemm_i8 M=%d K=N=4096 (%s)" % (m, "gemm_i8_ksplit_lds_kernel" if m <= 512 else "conv_i8_ws_kernel, row-major"),
+            timed("gemm_i8 M=%d K=N=4096 (%s)" % (m, "gemm_i8_ksplit_lds_kernel" if m <= 256 else "gemm_i8_tile_kernel"),
                   "mfma_i8", 2.0 * m * n * k,
                   lambda a=a, rs=rs: gemm(a, dq=dq, row_scale=rs, bias=bias))
         else:
             timed("gemm_i8 M=%d K=N=4096 (gemm_i8_skinny_kernel)" % m, "hbm", m * k + k * n + 4.0 * m * n + 4.0 * n,
                   lambda a=a, rs=rs: gemm(a, dq=dq, row_scale=rs, bias=bias))
+    ragged = capi.GemmI8(ri8(1500, 777))
+    a, rdq, rqs = ri8(197, 1500), torch.rand(777, device=dev) * 1e-2, torch.full((197,), 32.0, device=dev)
+    timed("gemm_i8 197x777 K=1500, int8 out (gemm_i8_ksplit_lds_kernel)", "mfma_i8", 2.0 * 197 * 777 * 1500,
+          lambda: ragged(a, dq=rdq, q_scales=rqs, act="relu", want_f32=False))
     # memory-bound 1x1 int8 layer (ResNet stage 1 expansion, 64 -> 256 channels at 56x56, batch 32), staged int8 in, fp32 out
     xq = ri8(32, 64, 56, 56)
     c11 = capi.Conv2dI8(ri8(256, 64, 1, 1))
@@ -444,6 +449,11 @@ def kernels_leg(reps=20):
     ws_bytes = c11._plan(tuple(xq.shape))[2]
     timed("conv2d_i8 1x1 64->256 @56x56 bs32, fp32 out (conv_i8_ws_kernel)", "hbm", float(ws_bytes) + 4.0 * 32 * 256 * 56 * 56,
           lambda: c11.run_staged(st, dq11, b11, "relu"))
+    # the staging of config 2's input: quantize and NCHW -> padded pixel-major
+    c2, xs = capi.Conv2dI8(ri8(256, 256, 3, 3), (1, 1, 1, 1)), torch.full((32,), 30.0, device=dev)
+    x28 = rnd(32, 256, 28, 28)
+    st2 = capi.StagedInput(c2, x28.shape)
+    timed("stage 32x256x28x28 fp32 (stage_planes_kernel)", "hbm", 4.0 * x28.numel() + 32 * 30 * 30 * 256, lambda: c2.stage(x28, st2, xs))
     # HBM-bound glue on a 32x256x56x56 fp32 tensor (103 MB)
     x = rnd(32, 256, 56, 56)
     nb = 4.0 * x.numel()
@@ -457,6 +467,9 @@ def kernels_leg(reps=20):
     qs = torch.full((32,), 20.0, device=dev)
     timed("quantize", "hbm", 1.25 * nb, lambda: capi.quantize(x, qs))
     timed("pooling2d max 3x3 s2 p1", "hbm", 1.25 * nb, lambda: capi.pooling2d(x, "max", (3, 3), (2, 2), (1, 1, 1, 1)))
+    timed("global_pooling2d avg", "hbm", nb, lambda: capi.global_pooling2d(x, "avg"))
+    mean, var, sc = rnd(256), torch.rand(256, device=dev) + 0.5, rnd(256)
+    timed("fused_batch_norm", "hbm", 2 * nb, lambda: capi.fused_batch_norm(x, mean, var, sc, bb))
     return {"workload": "kernels of the path one by one; time per launch includes the wrapper's output allocation from "
                         "torch's caching allocator (no device allocation in steady state)", "reps": reps, "kernels": rows}
 
@@ -683,7 +696,7 @@ def main():
         "int8_output_variant": None if args.profile else {
             "achieved": ops / t_mfma_q / 1e12, "unit": "TOPS", "us": t_mfma_q * 1e6,
             "note": "same kernel, epilogue requantizes to int8 for a following quantized layer"},
-        "stage_kernel": {"bound": "hbm", "kernel": "stage_rows_kernel<quantize>", "achieved": stage_bytes / t_stage / 1e9,
+        "stage_kernel": {"bound": "hbm", "kernel": "stage_planes_kernel<quantize>", "achieved": stage_bytes / t_stage / 1e9,
                          "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": stage_bytes / t_stage / 1e9 / PEAK_HBM_GBS,
                          "us": t_stage * 1e6, "bytes": stage_bytes, "traffic": TRAFFIC_STAGE_BYTES,
                          "device_copy_of_the_same_bytes": {"us": t_copy * 1e6, "GB_per_s": 2.0 * half / t_copy / 1e9,

@@ -205,7 +205,7 @@ int tsx_gemm_i8(int32_t m, int32_t n, int32_t k, const int8_t *a_dev, const void
  * include/backend/base/base_conv2d_core.h:14-32): im2col + GEMM, here one implicit-GEMM kernel on
  * the fp32 MFMA reading NCHW directly (weights are used as they are: no packing, no workspace).
  * bias_dev (optional, [cout]) and act fuse the add_bias / relu operators that follow the conv in
- * BASELINE config 1; pass NULL / TSX_ACT_NONE for the bare operator.  Parity bar for this
+ * config 1; pass NULL / TSX_ACT_NONE for the bare operator.  Parity bar for this
  * floating-point path: 1e-4 relative / 1e-5 absolute against the reference CPU kernels. */
 int tsx_conv2d_f32_nchw(const tsx_conv2d_geom *g, const float *x_dev, const float *w_oihw_dev, float padding_value,
                         const float *bias_dev, int32_t act, float slope, float *out_dev, void *stream);

@@ -700,8 +700,9 @@ constexpr int KS_WAVES = 8;
 
 // The end of a K-split tile: the eight wavefronts' partial accumulators go to LDS, where every wavefront picks up its
 // share of the sums and runs the epilogue on it: (fragment f, register group g) -- registers 4g .. 4g+3 of a lane are 4
-// consecutive output columns of one row.  The scales and biases of a wavefront's share are requested before the reduction
-// and arrive under it.  red: 8 x FR FC x 16 x 64 ints.
+// consecutive output columns of one row.  Where rows are a multiple of 4 columns and all pointers aligned (`plain`) the
+// scales and biases of a wavefront's share are requested before the reduction and arrive under it; otherwise they are
+// loaded element by element behind it, where nothing hides a miss of the caches.  red: 8 x FR FC x 16 x 64 ints.
 template <int FR, int FC>
 __device__ __forceinline__ void ksplit_finish(const GemmParams &p, v16i (&acc)[FR][FC], int (*red)[FR * FC][16][64], int frag0,
                                               int row0, int lane, int wave) {

@@ -1,5 +1,5 @@
 // Flat-tile int8 convolution for layers with more than one tap whose whole-row window fits LDS (the 3x3
-// body of ResNet-like networks and BASELINE config 2).  Same arithmetic, staged input, packed weights,
+// body of ResNet-like networks and config 2).  Same arithmetic, staged input, packed weights,
 // window-in-LDS data movement and epilogue as the window-stationary kernel in conv2d_i8_ws.hip (exact int32
 // sums of cpu::Conv2DQuantizedCore, src/kernels/cpu/quantized/conv2d_quantized_core.cpp:18-147); what
 // differs is how output positions are dealt to workgroups:
@@ -41,7 +41,7 @@ void fl_plan(const WsGeom &g, WsPlan *pl) {
     const int wc = (g.wo - 1) * g.sw + (g.kw - 1) * g.dil_w + 1;
     if (wc > g.ws) return;
     // Measured against the window-stationary kernel, the flat tiles pay on large layers that fill most of the
-    // chip with tiles of 6 to 8 fragments in one round (24.9 -> 23.4 us; the large 3x3
+    // chip with tiles of 6 to 8 fragments in one round (config 2: 24.9 -> 23.4 us; the large 3x3
     // layers of the YOLOv4-shaped network); small maps (ResNet's 14x14 and 7x7 layers, under 200 workgroups of
     // short tiles) run 1-20 % slower on it and stay where they were.  The smaller splits remain instantiated
     // for the planner to use once that changes.

@@ -1,4 +1,4 @@
-// Weight-stationary int8 convolution for large 3x3 layers on 256 input channels (
+// Weight-stationary int8 convolution for large 3x3 layers on 256 input channels (config 2:
 // 32x256x28x28 * 256x256x3x3).  Same arithmetic, staged input and packed weights as the window-stationary and
 // flat-tile kernels (exact int32 sums of cpu::Conv2DQuantizedCore,
 // src/kernels/cpu/quantized/conv2d_quantized_core.cpp:18-147, dequantized as its lines 81-106 do); what differs

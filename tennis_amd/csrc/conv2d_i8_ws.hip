@@ -1,4 +1,4 @@
-// Window-stationary int8 convolution (the 3x3 body of ResNet-like nets and BASELINE config 2; any
+// Window-stationary int8 convolution (the 3x3 body of ResNet-like nets and config 2; any
 // stride, maps of any width through column tiles) on v_mfma_i32_32x32x32_i8
 // (the 16x16x64 form runs at half the rate on this part).
 //

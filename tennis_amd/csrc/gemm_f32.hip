@@ -400,7 +400,7 @@ __global__ __launch_bounds__(64 * KS_WAVES) void gemm_f32_regfed_kernel(GemmArgs
     tile_store(g, g.c + batch * g.c_batch, acc, bias, m0, lane, col_base, row_stride);
 }
 
-// A single small 3x3 layer (1 x 64 x 56 x 56, 64 output channels: 196 tiles of 32 x 32, under one
+// A single small 3x3 layer (config 1: 1 x 64 x 56 x 56, 64 output channels: 196 tiles of 32 x 32, under one
 // per CU) is bound by what the kernels above do per element of B: the im2col gather computes an address, two
 // bounds and a padding select per element per K chunk, and walks K in dependent round trips.  This kernel orders K
 // as the layer is laid out -- (input channel, tap) -- and gives every lane ONE input channel per MFMA step: lane l of

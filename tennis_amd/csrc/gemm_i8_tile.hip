@@ -11,9 +11,11 @@
 //   * weights: the packed operands are 1 KiB contiguous per fragment and half K-step and go straight into registers, a
 //     chunk ahead of their MFMAs;
 //   * one barrier per chunk, ahead of the chunk's last MFMAs, whose time covers the first LDS reads behind it.
-// 4096 x 4096 x 4096: 67 .. 74 us with fp32 output (86 .. 105 on the window-stationary kernel's GEMM form), 66 us with int8 output
-// (155); MFMAs are busy 60 % of a CU's time, the rest goes to operand waits around the barrier.  fp32 accumulators go out
-// as 4-byte stores with lanes along columns: two whole 128-byte lines per instruction.
+// 4096 x 4096 x 4096: 67 .. 74 us with fp32 output on rounded normal operands (86 .. 105 on the window-stationary kernel's
+// GEMM form; uniformly random bytes, which toggle most and get the lowest clocks: 82 us), 66 us with int8 output (155).
+// Counted at this size MFMAs are busy half of a CU's time; the rest goes to operand waits around the barrier and to the
+// stores, which begin everywhere when the last MFMA is done.  fp32 accumulators go out as 4-byte stores with lanes along
+// columns: two whole 128-byte lines per instruction.
 // int32 accumulation is exact, so the results are the other GEMM kernels' and the oracle's.
 #include "gemm_i8_tile.hpp"
 

@@ -280,9 +280,9 @@ __global__ __launch_bounds__(256) void wino23_input_transform_kernel(const float
 // loads meet in L1).  Workgroups b, b + 8, ... run on one XCD: each XCD gets whole frequencies, whose U and V then
 // stay in its L2 (8 x 456 KB at 8 images of 28x28x256).  RING groups of 8 channels are in flight per wavefront.
 // Bound by the fp32 MFMA: 1.68 GFLOP at that shape = 11 us at 157 TFLOP/s.
-// It takes 26 us there (the tail's
-// fragments hold 8 real columns of 32, and a wavefront's chain of 128 dependent MFMAs fills its SIMD 3.5 times over);
-// chains on the vector ALUs, one lane per 4 x 4 outputs, took 276 + 31 us.
+// It takes 26 .. 28 us there (the tail's
+// fragments hold 8 real columns of 32, and a wavefront's chain of 128 dependent MFMAs fills its SIMD 3.5 times over; MFMAs
+// are busy 58 % of the CUs' time); chains on the vector ALUs, one lane per 4 x 4 outputs, took 276 + 31 us.
 constexpr int WG_RING = 4;
 constexpr int TAIL_RING = 4;
 

@@ -12,7 +12,7 @@ def quantize_weights_per_channel(w):
 
 
 def c2_like(rng, n, c, h, w, cout, k=3):
-    """BASELINE config 2 shaped inputs: x ~ N(0,1), w ~ N(0,0.05), per-tensor activation scale."""
+    """config 2 shaped inputs: x ~ N(0,1), w ~ N(0,0.05), per-tensor activation scale."""
     x = rng.standard_normal((n, c, h, w)).astype(np.float32)
     wt = (rng.standard_normal((cout, c, k, k)) * 0.05).astype(np.float32)
     bias = (rng.standard_normal(cout) * 0.1).astype(np.float32)

@@ -35,7 +35,7 @@ def test_argument_errors_need_no_device():
     g = capi.ConvGeom(1, 8, 9, 9, 4, 5, 5, 1, 1, 1, 1, 1, 1, 1, 1)          # Winograd needs 3x3
     assert L.tsx_winograd_f63_workspace_bytes(ctypes.byref(g)) == 0
     assert L.tsx_quantize_f32_i8(None, -1, None, 1, None, None) == -1
-    # geometry bookkeeping of BASELINE config 2
+    # geometry bookkeeping of config 2
     g = capi.ConvGeom(32, 256, 28, 28, 256, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1)
     assert L.tsx_conv2d_i8_workspace_bytes(ctypes.byref(g)) == 32 * 30 * 30 * 256
     assert L.tsx_conv2d_i8_packed_weight_bytes(ctypes.byref(g)) == 256 * 256 * 9

@@ -40,7 +40,7 @@ CONV_CASES = [
     (3, 2, 7, 7, 7, 7, 7, (3, 3, 3, 3), (2, 2), (1, 1)),
     (2, 70, 13, 9, 90, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),       # ragged in every GEMM dimension
     (4, 128, 28, 28, 128, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),    # large enough for the 64x64 tiles
-    (1, 64, 56, 56, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
+    (1, 64, 56, 56, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),      # config 1
 ]
 
 
@@ -57,7 +57,7 @@ def test_conv2d_f32(tsx, port, case):
 
 
 def test_conv2d_f32_config1_bias_relu(tsx, port):
-    """1x64x56x56, 64x64x3x3 Kaiming-normal, bias N(0,0.01), s1 p1, then ReLU."""
+    """config 1: 1x64x56x56, 64x64x3x3 Kaiming-normal, bias N(0,0.01), s1 p1, then ReLU."""
     rng = np.random.default_rng(1234)
     x = rng.uniform(-1, 1, (1, 64, 56, 56)).astype(np.float32)
     wt = (rng.standard_normal((64, 64, 3, 3)) * np.sqrt(2.0 / 576)).astype(np.float32)
@@ -87,7 +87,7 @@ def small_layer_cases(count, seed):
 
 
 SMALL_FIXED = [
-    (1, 64, 56, 56, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
+    (1, 64, 56, 56, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),      # config 1
     (2, 64, 28, 28, 128, 3, 3, (1, 0, 2, 1), (2, 1), (1, 1)),
     (1, 60, 30, 30, 70, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
     (3, 32, 5, 5, 48, 3, 3, (3, 3, 3, 3), (1, 1), (2, 2)),        # more padding than map
@@ -206,7 +206,7 @@ WINO_CASES = [
     (1, 8, 10, 10, 16, (0, 0, 0, 0)),
     (1, 5, 7, 7, 3, (2, 1, 1, 2)),
     (2, 70, 20, 17, 36, (1, 1, 1, 1)),
-    (1, 64, 56, 56, 64, (1, 1, 1, 1)),      # BASELINE config 1 through F(6,3)
+    (1, 64, 56, 56, 64, (1, 1, 1, 1)),      # config 1 through F(6,3)
 ]
 
 

@@ -108,7 +108,7 @@ CONV_CASES = [
     (2, 64, 14, 14, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
     (1, 130, 9, 9, 200, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),     # ragged channels / cout > one tile
     (5, 96, 7, 7, 129, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1)),
-    (2, 256, 28, 28, 256, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),   # two images of BASELINE config 2
+    (2, 256, 28, 28, 256, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),   # two images of config 2
     (1, 16, 5, 300, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),     # rows wider than a tile: column tiles
     (2, 16, 7, 301, 72, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1)),     # ... with stride 2
     (2, 16, 9, 50, 24, 3, 3, (1, 0, 2, 1), (1, 1), (1, 1)),      # at most 32 output channels: one wavefront along cout
@@ -536,7 +536,7 @@ def test_quantize_conv2d_fused_input(tsx, port):
 
 
 def test_conv2d_i8_baseline_config2_full(tsx, port):
-    """BASELINE config 2 at full size: 32x256x28x28, 256x256x3x3, s1 p1, dequant + bias + ReLU."""
+    """config 2 at full size: 32x256x28x28, 256x256x3x3, s1 p1, dequant + bias + ReLU."""
     rng = np.random.default_rng(1234)
     x, x_scales, wq, dq, bias = c2_like(rng, 32, 256, 28, 28, 256)
     conv = tsx.Conv2dI8(_dev(wq), (1, 1, 1, 1))

@@ -266,7 +266,7 @@ def rs_cases(count, seed):
 
 RS_FIXED = [
     # n, c, h, w, cout, pads, strides, dilations, fragments per tile ("": at most 5)
-    (2, 256, 28, 28, 256, (1, 1, 1, 1), (1, 1), (1, 1), ""),      # two images of BASELINE config 2
+    (2, 256, 28, 28, 256, (1, 1, 1, 1), (1, 1), (1, 1), ""),      # two images of config 2
     (2, 256, 28, 28, 256, (1, 1, 1, 1), (1, 1), (1, 1), "9"),     # ... in tiles of 9 fragments (odd: the loop's tail)
     (3, 256, 17, 20, 128, (1, 1, 1, 1), (1, 1), (1, 1), "4"),     # 10.6 fragments an image: tiles that span two images
     (1, 200, 9, 30, 65, (0, 0, 0, 0), (1, 1), (1, 1), "3"),       # no padding, a second 64-channel tile with one channel

@@ -71,7 +71,7 @@ def test_conv2d_quantized_operator(ops, port, case):
 
 
 def test_operator_chain_quantize_conv_bias_relu(ops, port):
-    """The graph fragment of BASELINE config 2 as four separate operators, small batch."""
+    """The graph fragment of config 2 as four separate operators, small batch."""
     rng = np.random.default_rng(502)
     x, x_scales, wq, dq, bias = c2_like(rng, 3, 64, 14, 14, 64)
     params = ops.conv_params((1, 1, 1, 1))

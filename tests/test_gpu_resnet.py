@@ -83,7 +83,7 @@ def test_resnet_shaped_network_bit_exact(port):
 
 
 def test_full_size_network_every_layer(port):
-    """BASELINE config 4 at its real size (batch 32, 3x224x224, full width and depth): the tile plans the
+    """config 4 at its real size (batch 32, 3x224x224, full width and depth): the tile plans the
     kernels pick here differ from the small network's.  Every convolution of the chained pass is checked by
     itself for the first and the last image of the batch: the oracle runs the operator chain on the very
     tensor the device kernel read (its staged int8 input), so one layer's result does not depend on another's.

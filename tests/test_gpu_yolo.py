@@ -74,7 +74,7 @@ def test_yolov4_shaped_network(port, mish):
 
 @pytest.mark.parametrize("mish", ["exact", "fast"])
 def test_full_size_network_every_layer(port, capsys, mish):
-    """BASELINE config 5 at its real size (batch 8, 3x608x608, full width): every convolution of the chained
+    """config 5 at its real size (batch 8, 3x608x608, full width): every convolution of the chained
     pass checked by itself for the first and the last image -- the oracle runs the operator chain on the very
     tensor the device kernel read, so one layer's result does not depend on another's.  Bar for LeakyReLU / linear
     layers: bit-exact fp32 outputs and int8 hand-overs.  Mish layers, exact form (the default): fp32 outputs bit for

@@ -63,7 +63,7 @@ CONV_CASES = [
     (2, 5, 9, 7, 6, 3, 3, (0, 0, 0, 0), (2, 2), (1, 1)),
     (2, 16, 8, 8, 8, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1)),
     (1, 3, 10, 11, 4, 3, 2, (2, 1, 0, 1), (1, 2), (2, 1)),
-    (1, 64, 56, 56, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),
+    (1, 64, 56, 56, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1)),      # config 1
 ]
 
 
@@ -110,7 +110,7 @@ WINO_CASES = [
     (2, 16, 9, 11, 8, (1, 1, 1, 1)),       # ragged: padded to 12x12 tiles and cut back
     (1, 8, 10, 10, 16, (0, 0, 0, 0)),      # no padding: output 8x8
     (1, 5, 7, 7, 3, (2, 1, 1, 2)),         # asymmetric padding, channel counts off the 8-blocks
-    (1, 64, 56, 56, 64, (1, 1, 1, 1)),     # BASELINE config 1 through F(6,3)
+    (1, 64, 56, 56, 64, (1, 1, 1, 1)),     # config 1 through F(6,3)
 ]
 
 
