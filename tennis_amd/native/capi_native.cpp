@@ -113,6 +113,21 @@ at::TensorBase empty(at::IntArrayRef shape, c10::ScalarType type, const at::Tens
     return at::detail::empty_cuda(shape, type, like.device(), std::nullopt);
 }
 PyObject *wrap(at::TensorBase t) { return t.defined() ? THPVariable_Wrap(std::move(t)) : Py_NewRef(Py_None); }
+template <class... T>
+PyObject *results(T &...out) {        // a tuple of them
+    PyObject *all = PyTuple_New(sizeof...(out));
+    bool whole = all != nullptr;
+    Py_ssize_t i = 0;
+    const auto put = [&](at::TensorBase t) {
+        PyObject *o = whole ? wrap(std::move(t)) : nullptr;
+        whole = o != nullptr;
+        if (o) PyTuple_SET_ITEM(all, i++, o);
+    };
+    (put(std::move(out)), ...);
+    if (whole) return all;
+    Py_XDECREF(all);
+    throw Raised{};
+}
 void *stream() { return c10::hip::getCurrentHIPStream().stream(); }
 template <class T>
 T *data(at::TensorBase &t) { return t.defined() ? static_cast<T *>(t.mutable_data_ptr()) : nullptr; }
@@ -488,7 +503,7 @@ PyObject *gemm_i8(PyObject *const *a, Py_ssize_t) {
         const WorkspaceLock lock(ws);
         return enqueue();
     });
-    return Py_BuildValue("(NNN)", wrap(out_f32), wrap(out_i8), wrap(acc));
+    return results(out_f32, out_i8, acc);
 }
 
 // What one Conv2dI8 has in hand for the input shapes it has seen last: geometry, packed weights, workspace and output size.
@@ -630,7 +645,7 @@ PyObject *conv_i8(PyObject *const *a, Py_ssize_t) {
         return L.tsx_conv2d_i8_nchw(&p.geom, x.const_data_ptr<int8_t>(), p.packed.const_data_ptr(), st->padding_value, ep, data<float>(out_f32),
                                     data<int8_t>(out_i8), data<int32_t>(acc), ws, p.ws_bytes, stream());
     });
-    return Py_BuildValue("(NNN)", wrap(out_f32), wrap(out_i8), wrap(acc));
+    return results(out_f32, out_i8, acc);
 }
 
 PyObject *conv_i8_staged(PyObject *const *a, Py_ssize_t) {
@@ -653,7 +668,7 @@ PyObject *conv_i8_staged(PyObject *const *a, Py_ssize_t) {
         return L.tsx_conv2d_i8_staged_at(&p.geom, in.const_data_ptr(), hs, ws, p.packed.const_data_ptr(), &e, data<float>(out_f32), data<int8_t>(out_i8),
                                          nullptr, stream());
     });
-    return Py_BuildValue("(NN)", wrap(out_f32), wrap(out_i8));
+    return results(out_f32, out_i8);
 }
 
 // ---- module
