@@ -428,18 +428,24 @@ class Conv2dI8:
         self.padding_value = float(padding_value)
         self._packed = {}
         self._workspace = None
+        self._graph_workspaces = []
         self._make_state()
 
     def _make_state(self):
-        # what belongs to this object alone, neither copied nor stored: the native calls' state, and workspaces in graphs
-        self._graph_workspaces = []
+        # what the native calls keep for this object: geometry and plans of the shapes seen last
         self._state = _native().ConvState(self.w, self.pads, self.strides, self.dilations, self.padding_value)
 
+    def __setattr__(self, name, value):
+        super().__setattr__(name, value)
+        if name in ("w", "pads", "strides", "dilations", "padding_value") and "_state" in self.__dict__:
+            self._make_state()
+
     def __getstate__(self):
+        # the state and the workspaces in graphs belong to this object alone
         return {k: v for k, v in self.__dict__.items() if k not in ("_state", "_graph_workspaces")}
 
     def __setstate__(self, state):
-        self.__dict__.update(state)
+        self.__dict__.update(state, _graph_workspaces=[])
         self._make_state()
 
     def _keep_for_graph(self, workspace):

@@ -117,6 +117,20 @@ def test_copied_layers_and_networks_compute_the_same(capi, how):
     assert torch.equal(net.forward(image), twin(net).forward(image))
 
 
+@pytest.mark.gpu
+def test_a_layer_follows_its_attributes(capi):
+    """Padding and its value set after calls: the layer computes what one made with them computes."""
+    import torch
+    conv, dq = _layer(capi)
+    x = _input(2, 40, 9, 11)
+    conv(x, dq=dq)
+    for change in ({"padding_value": -7.0}, {"pads": (0, 1, 2, 0)}, {"pads": (1, 1, 1, 1), "padding_value": 3.0}):
+        for name, value in change.items():
+            setattr(conv, name, value)
+        made = capi.Conv2dI8(conv.w, conv.pads, padding_value=conv.padding_value)
+        assert torch.equal(conv(x, dq=dq)[0], made(x, dq=dq)[0]), change
+
+
 # ---------------------------------------------------------------- threads and re-entry
 
 SLOW = "#include <unistd.h>\nint slow(const void *x, long long n, void *out, void *stream) { usleep(400000); return 0; }\n"
