@@ -209,6 +209,13 @@ int tsx_gemm_i8(int32_t m, int32_t n, int32_t k, const int8_t *a_dev, const void
  * floating-point path: 1e-4 relative / 1e-5 absolute against the reference CPU kernels. */
 int tsx_conv2d_f32_nchw(const tsx_conv2d_geom *g, const float *x_dev, const float *w_oihw_dev, float padding_value,
                         const float *bias_dev, int32_t act, float slope, float *out_dev, void *stream);
+/* The same with a workspace of tsx_conv2d_f32_workspace_bytes() (0: the layer has no use for one): there large layers run
+ * on the bf16 matrix cores, every float as the exact sum of three bf16 numbers, with smaller errors than the fp32 MFMA's.
+ * The workspace is 16-byte aligned device memory; its contents are written and read by each call. */
+size_t tsx_conv2d_f32_workspace_bytes(const tsx_conv2d_geom *g, const float *w_oihw_dev);
+int tsx_conv2d_f32_nchw_ws(const tsx_conv2d_geom *g, const float *x_dev, const float *w_oihw_dev, float padding_value,
+                           const float *bias_dev, int32_t act, float slope, float *out_dev, void *workspace_dev,
+                           size_t workspace_bytes, void *stream);
 /* Which kernel tsx_conv2d_f32_nchw launches for this layer and these weights (their alignment counts), as text:
  * "kernel=small_3x3 | register_fed | staged_64x64 | staged_32x32_ksplit tiles=<output tiles>".  No counterpart in
  * the reference; for tests that must know a given kernel ran, and for logs.  The environment variables

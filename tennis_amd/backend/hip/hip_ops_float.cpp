@@ -24,15 +24,20 @@ public:
         // receives them unpacked (src/compiler/option/pack_translator_option.cpp:14-27)
         if (kernel_packed) TS_LOG_ERROR << "[hip] conv2d expects OIHW weights (kernel_packed=false)" << eject;
         const tsx_conv2d_geom g = make_geom(x, w, padding, stride, dilation);
-        check(tsx_conv2d_f32_nchw(&g, x.data<float>(), w.data<float>(), padding_value, nullptr, TSX_ACT_NONE, 0.f,
-                                  out.data<float>(), current_stream()),
-              "tsx_conv2d_f32_nchw");
+        const size_t ws_bytes = tsx_conv2d_f32_workspace_bytes(&g, w.data<float>());
+        if (ws_bytes && (m_workspace.empty() || size_t(m_workspace.count()) < ws_bytes)) m_workspace = byte_tensor(out.device(), ws_bytes);
+        check(tsx_conv2d_f32_nchw_ws(&g, x.data<float>(), w.data<float>(), padding_value, nullptr, TSX_ACT_NONE, 0.f,
+                                     out.data<float>(), ws_bytes ? m_workspace.data() : nullptr, ws_bytes, current_stream()),
+              "tsx_conv2d_f32_nchw_ws");
     }
 
 protected:
-    // fp32 NCHW on the MFMA kernel; fp64 and NHWC graphs (the reference's device classes take both,
+    // fp32 NCHW on the MFMA kernels; fp64 and NHWC graphs (the reference's device classes take both,
     // src/kernels/gpu/conv2d_core.cu) run the host operator
     bool covers(Stack &stack) override { return format_is_nchw(*this) && inputs_are(stack, 2, FLOAT32); }
+
+private:
+    Tensor m_workspace;
 };
 
 // ---------------------------------------------------------------- conv2d_winograd (fp32, F(6,3) and F(2,3))

@@ -83,6 +83,8 @@ SIGNATURES = {
     "tsx_gemm_i8_workspace_bytes": (_sz, [_i32, _i32]),
     "tsx_gemm_i8": (ctypes.c_int, [_i32, _i32, _i32, _vp, _vp, ctypes.POINTER(Epilogue), _vp, _vp, _vp, _vp, _sz, _vp]),
     "tsx_conv2d_f32_nchw": (ctypes.c_int, [ctypes.POINTER(ConvGeom), _vp, _vp, _f32, _vp, _i32, _f32, _vp, _vp]),
+    "tsx_conv2d_f32_nchw_ws": (ctypes.c_int, [ctypes.POINTER(ConvGeom), _vp, _vp, _f32, _vp, _i32, _f32, _vp, _vp, _sz, _vp]),
+    "tsx_conv2d_f32_workspace_bytes": (_sz, [ctypes.POINTER(ConvGeom), _vp]),
     "tsx_conv2d_f32_plan_info": (ctypes.c_int, [ctypes.POINTER(ConvGeom), _vp, ctypes.c_char_p, _sz]),
     "tsx_inner_prod_f32": (ctypes.c_int, [_i32, _i32, _i32, _vp, _vp, _i32, _vp, _vp]),
     "tsx_add_bias_f32": (ctypes.c_int, [_vp, _i64, _i32, _i64, _vp, _vp, _vp]),
@@ -575,7 +577,7 @@ class GemmI8:
 
 def conv2d_f32(x, w, pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1), padding_value=0.0, bias=None, act=None,
                slope=0.0):
-    """tsx_conv2d_f32_nchw: fp32 implicit-GEMM conv2d (optionally + add_bias + activation)."""
+    """tsx_conv2d_f32_nchw_ws: fp32 implicit-GEMM conv2d (optionally + add_bias + activation)."""
     out = _native().conv2d_f32(x, w, pads, strides, dilations, padding_value, bias, _ACT[act], slope)
     if out is not NotImplemented:
         return out
@@ -585,9 +587,15 @@ def conv2d_f32(x, w, pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1), paddin
     geom = make_geom(tuple(x.shape), tuple(w.shape), pads, strides, dilations)
     ho, wo = conv_out_size(geom)
     out = torch.empty((x.shape[0], w.shape[0], ho, wo), dtype=torch.float32, device=x.device)
-    check(lib().tsx_conv2d_f32_nchw(ctypes.byref(geom), _ptr(x), _ptr(w), float(padding_value), _ptr(bias), _ACT[act],
-                                    float(slope), _ptr(out), _stream()))
+    workspace = _conv_f32_workspace(geom, x, w)
+    check(lib().tsx_conv2d_f32_nchw_ws(ctypes.byref(geom), _ptr(x), _ptr(w), float(padding_value), _ptr(bias), _ACT[act],
+                                       float(slope), _ptr(out), _ptr(workspace), workspace.numel() if workspace is not None else 0, _stream()))
     return out
+
+
+def _conv_f32_workspace(geom, x, w):
+    size = lib().tsx_conv2d_f32_workspace_bytes(ctypes.byref(geom), _ptr(w))
+    return torch.empty(size, dtype=torch.uint8, device=x.device) if size else None
 
 
 def conv2d_f32_plan_info(x_shape, w, pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1)):
@@ -601,7 +609,7 @@ def conv2d_f32_plan_info(x_shape, w, pads=(0, 0, 0, 0), strides=(1, 1), dilation
 
 def conv2d_f32_prepared(x, w, pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1), padding_value=0.0, bias=None,
                         act=None, slope=0.0):
-    """(launch, out): tsx_conv2d_f32_nchw on fixed tensors with every argument marshalled once, for callers that issue
+    """(launch, out): tsx_conv2d_f32_nchw_ws on fixed tensors with every argument marshalled once, for callers that issue
     the same layer again and again (a layer of a few microseconds is otherwise bound by this module's per-call work:
     geometry, output allocation, argument conversion).  `launch()` enqueues one convolution on the stream that was
     current here and raises TsxError like conv2d_f32; `out` is the tensor it writes."""
@@ -611,10 +619,11 @@ def conv2d_f32_prepared(x, w, pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1
     geom = make_geom(tuple(x.shape), tuple(w.shape), pads, strides, dilations)
     ho, wo = conv_out_size(geom)
     out = torch.empty((x.shape[0], w.shape[0], ho, wo), dtype=torch.float32, device=x.device)
-    fn = lib().tsx_conv2d_f32_nchw
+    fn = lib().tsx_conv2d_f32_nchw_ws
+    workspace = _conv_f32_workspace(geom, x, w)
     args = (ctypes.byref(geom), _ptr(x), _ptr(w), float(padding_value), _ptr(bias), _ACT[act], float(slope), _ptr(out),
-            _stream())
-    keep = (x, w, bias, geom)
+            _ptr(workspace), workspace.numel() if workspace is not None else 0, _stream())
+    keep = (x, w, bias, geom, workspace)
 
     def launch(_keep=keep):
         check(fn(*args))

@@ -1,0 +1,514 @@
+// fp32 convolution on the bf16 matrix cores, for layers of more than some ten million products whose fp32 MFMAs are
+// what bounds them (cpu::Conv2DCore, src/kernels/cpu/conv2d_core.cpp:17-119).
+//
+// v_mfma_f32_32x32x2_f32 gives 64 operations per cycle and SIMD, v_mfma_f32_32x32x16_bf16 1024.  A float of 24
+// significant bits is the sum of three bf16 numbers of 8, exactly: x = h + m + l, h the upper half of its bits, m the
+// remainder rounded, l what is left of that.  Of the nine products of two such sums six are formed,
+//     x w = h h' + (h m' + m h') + (m m' + h l' + l h'),
+// the other three lie below 2^-23 of the product, with either sign; each product of two bf16 is exact in the MFMA's
+// fp32 accumulator.  h h' goes to an accumulator of its own, the five small products to a second one, added once at the
+// end: a sum of K terms takes K / 16 roundings where the fp32 MFMA takes K, and the small terms are not lost beside the
+// large ones.  Measured against 64 bits (normally distributed operands, 2-norm): 4.5e-8 at K = 32, 9.1e-8 at 256,
+// 2.9e-7 at 2304; the fp32 MFMA's chain has 1.0e-7, 2.9e-7, 8.6e-7.  Numbers below 2^-110 lose bits to the bf16
+// denormals (steps of 2^-133).
+//
+// NaN and infinities: such a value goes into l, with h = +-1 and m = 0.  l meets h' only, so an infinity times w has the
+// sign of w, and NaN where w is 0; what h = +-1 adds to the sum is finite.  Infinity times infinity is l h' = infinity
+// too.
+#include "conv2d_f32_split.hpp"
+
+#include <algorithm>
+#include <atomic>
+#include <cstdlib>
+
+namespace tsx {
+namespace {
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2b __attribute__((ext_vector_type(2)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+struct Parts {
+    v4u h, m, l;
+};
+
+// The three parts of eight floats, element by element in the order of the MFMA operand.  `odd` stays finite unless a value
+// is infinite or NaN (or some 10^23): those need SPECIAL.
+template <bool SPECIAL>
+__device__ __forceinline__ Parts split8(float (&x)[8], float &odd) {
+    Parts p;
+    unsigned special[4] = {0, 0, 0, 0};
+    if constexpr (SPECIAL)
+        static_for<0, 8>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            const bool finite = __builtin_fabsf(x[j]) < __builtin_inff();
+            const unsigned bits = __float_as_uint(x[j]) >> 16 | (x[j] != x[j] ? 0x40u : 0u);      // a NaN stays one
+            special[j / 2] |= finite ? 0u : bits << (16 * (j % 2));
+            x[j] = finite ? x[j] : __builtin_copysignf(1.f, x[j]);
+        });
+    static_for<0, 4>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const unsigned a = __float_as_uint(x[2 * j]), b = __float_as_uint(x[2 * j + 1]);
+        p.h[j] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+        const float ra = __fsub_rn(x[2 * j], __uint_as_float(a & 0xffff0000u)), rb = __fsub_rn(x[2 * j + 1], __uint_as_float(b & 0xffff0000u));
+        const unsigned m = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{ra, rb}), v2b));
+        const float qa = __fsub_rn(ra, __uint_as_float(m << 16)), qb = __fsub_rn(rb, __uint_as_float(m & 0xffff0000u));
+        p.m[j] = m;
+        p.l[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{qa, qb}), v2b)) | special[j];
+        if constexpr (!SPECIAL) odd = __builtin_fmaf(qa, qb, odd);
+    });
+    return p;
+}
+
+// ---- weights [M][C][taps] to MFMA operands [16 channels][tap][32 rows][part][lane][8], zeros behind M and C.
+// A workgroup takes 16 channels of 32 rows, through LDS: read as they lie (a lane reading its own 8 channels x taps touches a
+// cache line per lane and load: 7.2 us for 256 x 256 x 3 x 3), written a KiB per store instruction.
+template <int TAPS>
+__global__ __launch_bounds__(256) void split_weights_kernel(const float *w, int M, int C, int mfrags, v4u *out) {
+    constexpr int RUN = 16 * TAPS, PITCH = RUN + 1, LOADS = 32 * RUN / 256;
+    __shared__ float rows[32 * PITCH];
+    const int tid = threadIdx.x, c0 = blockIdx.y * 16, live = min(16, C - c0) * TAPS;
+    float x[LOADS];
+    static_for<0, LOADS>([&](auto ic) {
+        const int e = tid + 256 * decltype(ic)::value, k = e % RUN, row = blockIdx.x * 32 + e / RUN;
+        x[decltype(ic)::value] = row < M && k < live ? w[(int64_t(row) * C + c0) * TAPS + k] : 0.f;
+    });
+    static_for<0, LOADS>([&](auto ic) {
+        const int e = tid + 256 * decltype(ic)::value;
+        rows[e / RUN * PITCH + e % RUN] = x[decltype(ic)::value];
+    });
+    __syncthreads();
+    v4u *to = out + (int64_t(blockIdx.y) * TAPS * mfrags + blockIdx.x) * 192;
+    for (int e = tid; e < 64 * TAPS; e += 256) {
+        const int lane = e % 64, tap = e / 64;
+        float v[8], unused = 0.f;
+        static_for<0, 8>([&](auto jc) { v[decltype(jc)::value] = rows[lane % 32 * PITCH + (8 * (lane / 32) + decltype(jc)::value) * TAPS + tap]; });
+        const Parts p = split8<true>(v, unused);
+        v4u *dst = to + int64_t(tap) * mfrags * 192 + lane;
+        dst[0] = p.h;
+        dst[64] = p.m;
+        dst[128] = p.l;
+    }
+}
+
+struct SplitParams {
+    const float *x, *bias;
+    const void *w;                 // split weights
+    float *out;
+    int M, N;                      // output channels, positions (n ho wo)
+    int n, C, H, W, dil_h, sh, sw, pad_top, pad_left;
+    int ho, wo, howo;
+    int hv, wv;                    // rows of one image with the padding its windows reach; patch columns
+    int seg, col_tiles;            // a fragment is 32 columns of one row; column tiles per row
+    int chunks, mfrags, tiles_m, tiles_n;
+    unsigned w_bytes;
+    float padding_value;
+    int act;
+    float slope;
+    int64_t act_body;
+};
+
+// A barrier for what has been exchanged through LDS: loads from memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// A workgroup of WM x WN x WK wavefronts (8, or two workgroups of 4 per CU) owns 32 WM output channels x 64 WN positions; a wavefront's 32 x 64 take 12
+// MFMAs (384 cycles) per 16 channels and tap for 3 KiB of weights, from L2 straight into registers AHEAD steps early, and
+// 6 KiB of activations from LDS.  As in the fp32 form (conv2d_f32_window.hip) a chunk of CC channels of the input patch
+// -- the rows and columns the tile's positions read through all taps, padding included -- goes to LDS once per element,
+// here in three parts, [part][8 channels][PITCH cells][8], and every tap is a shifted read; a thread converts eight
+// channels of a cell at a time while the other wavefront of its SIMD multiplies.  With WK > 1 the wavefronts split a
+// chunk's channels and add their sums through LDS in a fixed order.  TAPS: 9 (3x3), 25 (5x5), 1 (the patch is the tile's
+// positions themselves, at any stride).
+// What bounds it: the MFMAs, which at the clock the bf16 matrix cores leave (1.5 GHz and less) take two thirds of the time
+// (8 images of 28x28x256 with 256 3x3 filters: 36 of 52 us with everything but them left out), then the conversions, operand
+// reads and weights beside them.  Against the fp32 MFMAs (us, weights' split included): that layer 86 -> 52, 128 channels at
+// 56x56 86 -> 48, 256 to 256 channels 1x1 at 56x56, 32 images, 129 -> 94, 100 to 150 channels 5x5 at 33x41, 4 images, 128 -> 59.
+template <int WM, int WN, int WK, int TAPS, int PITCH, int CC>
+__global__ __launch_bounds__(64 * WM * WN * WK, 2) void conv_f32_split_kernel(SplitParams p) {
+    constexpr int THREADS = 64 * WM * WN * WK;
+    constexpr int BM = 32 * WM, BN = 64 * WN, KW = TAPS == 9 ? 3 : TAPS == 25 ? 5 : 1;
+    constexpr int SUBS = CC / 16 / WK, STEPS = SUBS * TAPS;
+    constexpr int AHEAD = STEPS <= 4 ? STEPS : 3;
+    constexpr int PART = CC / 8 * PITCH * 16, BUFFER = 3 * PART;           // bytes
+    constexpr int SLOTS = CC / 8 * PITCH / THREADS;
+    static_assert(SUBS >= 1 && CC % (16 * WK) == 0 && CC / 8 * PITCH % THREADS == 0 && (TAPS != 1 || PITCH == BN) &&
+                      2 * PART + ((SUBS - 1) * 2 * WK * PITCH + KW) * 16 < 65536 && SLOTS <= STEPS,
+                  "whole slots, one a step; every operand read within an instruction's offset");
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int hf = lane / 32;
+    const int wk = wave % WK, wn = (wave / WK) % WN, wm = wave / (WK * WN);
+
+    // Tiles that share their positions are consecutive, and each XCD takes a contiguous run of tiles: a patch is fetched
+    // into one L2.
+    const int total = p.tiles_m * p.tiles_n, per_xcd = (total + 7) / 8;
+    const int t = int(blockIdx.x & 7) * per_xcd + int(blockIdx.x >> 3);
+    if (int(blockIdx.x >> 3) >= per_xcd || t >= total) return;
+    const int tn = t / p.tiles_m, m0 = (t - tn * p.tiles_m) * BM;
+
+    // ---- positions: flat over the batch, or segments (image, first row inside it, first column)
+    const int seg_rows = (p.ho + BN / 32 - 1) / (BN / 32), seg_tile = p.seg ? tn / p.col_tiles : 0, seg_img = seg_tile / seg_rows;
+    const int seg_row = (seg_tile - seg_img * seg_rows) * (BN / 32);
+    const int col0 = p.seg ? (tn - seg_tile * p.col_tiles) * 32 : 0;
+    auto decode = [&](int q, int &row, int &col) -> bool {                 // tile position -> batch-wide output row, column
+        if (p.seg) {
+            row = seg_img * p.ho + seg_row + q / 32;
+            col = col0 + q % 32;
+            return seg_row + q / 32 < p.ho && col < p.wo;
+        }
+        const int pos = tn * BN + q;
+        row = pos / p.wo;
+        col = pos - row * p.wo;
+        return pos < p.N;
+    };
+    auto virtual_row = [&](int row) { const int img = row / p.ho; return img * p.hv + (row - img * p.ho) * p.sh; };
+    const int vr0 = virtual_row(p.seg ? seg_img * p.ho + seg_row : tn * BN / p.wo);
+
+    // ---- patch bookkeeping: slot i of a thread is cell (tid + 512 i) % PITCH of the chunk's eight channels (tid + 512 i) / PITCH
+    constexpr unsigned NOWHERE = 0x80000000u;                              // beyond any buffer: loads 0, stores nothing
+    const unsigned plane = unsigned(p.H) * unsigned(p.W);
+    unsigned x_off[SLOTS], x_pad = 0;                                      // bit: the cell is padding
+    static_for<0, SLOTS>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        const int e = tid + THREADS * i, octet = e / PITCH, cell = e % PITCH;
+        int img, h, w;
+        bool in = true;
+        if (TAPS == 1) {
+            const int pos = tn * BN + cell, r = pos % p.howo, oh = r / p.wo;
+            img = pos / p.howo;
+            in = pos < p.N;
+            h = oh * p.sh - p.pad_top;
+            w = (r - oh * p.wo) * p.sw - p.pad_left;
+        } else {
+            const int pr = cell / p.wv, v = vr0 + pr;
+            img = v / p.hv;
+            in = img < p.n;                                                // cells behind the tile's patch: loaded, never used
+            h = v - img * p.hv - p.pad_top;
+            w = cell - pr * p.wv + col0 * p.sw - p.pad_left;
+        }
+        in = in && h >= 0 && h < p.H && w >= 0 && w < p.W;
+        x_pad |= unsigned(!in) << i;
+        x_off[i] = in ? ((unsigned(img) * unsigned(p.C) + unsigned(8 * octet)) * plane + unsigned(h * p.W + w)) * 4u : NOWHERE;
+    });
+
+    auto x_octet = [&](int i) {                // computed where it is used, not kept over the whole loop
+        int e = tid + THREADS * i;
+        asm volatile("" : "+v"(e));
+        return e / PITCH;
+    };
+    float x_reg[SLOTS][8];
+    const int x_bytes = int(int64_t(p.n) * p.C * plane * 4);               // below 2 GiB
+    // Three forms of what follows, none with a branch between the MFMAs.  0: eight channels are there or not, padding is 0.
+    // 1: any channels and padding value.  2: NaN and infinities too -- form 0 or 1 notices them and the tile starts over.
+    const bool ragged = p.C % 8 != 0 || p.padding_value != 0.f;
+    float odd = 0.f;
+    // Channels FROM to TO of the chunk for slot i.  A chunk behind the last one reads nothing: its loads are out of bounds.
+    auto load_patch = [&](auto form, auto ic, auto from, auto to, int chunk) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        const bool live = chunk < p.chunks;
+        const int c0 = live ? chunk * CC : 0, at = c0 * int(plane) * 4;
+        const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(p.x) + at), 0, live ? x_bytes - at : 0, 0x00020000);
+        const int left = p.C - c0 - 8 * x_octet(i);
+        unsigned base = x_off[i];
+        if constexpr (decltype(form)::value != 0) asm volatile("" : "+v"(base));      // no sums of it kept either
+        static_for<decltype(from)::value, decltype(to)::value>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            if constexpr (decltype(form)::value == 0) {
+                x_reg[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, left > 0 ? int(base) : int(NOWHERE), j * int(plane) * 4, 0));
+            } else {                           // (the sum of an offset beyond the buffer and a channel's stays beyond it)
+                const unsigned off = base + unsigned(j) * plane * 4u;
+                x_reg[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, int(j < left ? off : NOWHERE), 0, 0));
+            }
+        });
+    };
+    auto store_patch = [&](auto form, auto ic, int chunk, int at) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (decltype(form)::value != 0) {
+            const int channels = p.C - chunk * CC - 8 * x_octet(i), left = (x_pad >> i) & 1u ? channels : 0;
+            static_for<0, 8>([&](auto jc) { x_reg[i][decltype(jc)::value] = decltype(jc)::value < left ? p.padding_value : x_reg[i][decltype(jc)::value]; });
+        }
+        const Parts s = split8<decltype(form)::value == 2>(x_reg[i], odd);
+        char *to = lds + at + (tid + THREADS * i) * 16;
+        *reinterpret_cast<v4u *>(to) = s.h;
+        *reinterpret_cast<v4u *>(to + PART) = s.m;
+        *reinterpret_cast<v4u *>(to + 2 * PART) = s.l;
+    };
+
+    // ---- operands.  Step (sub, tap) of a chunk takes channels 16 (wk + WK sub) ... of it.
+    const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.w), 0, int(p.w_bytes), 0x00020000);
+    const int w_off = min(m0 / 32 + wm, p.mfrags - 1) * 3072 + lane * 16, w_step = p.mfrags * 3072;
+    struct A { v4u part[3]; } a[AHEAD];
+    struct B { v4u part[2][3]; } b;
+    auto load_weights = [&](auto sc, int chunk) __attribute__((always_inline)) {      // step sc of the chunk, its steps beyond STEPS in the next
+        constexpr int s = decltype(sc)::value % STEPS, over = decltype(sc)::value / STEPS, sub = s / TAPS, tap = s % TAPS;
+        const int q = ((min(chunk + over, p.chunks - 1) * (CC / 16) + wk + WK * sub) * TAPS + tap) * w_step;
+        static_for<0, 3>([&](auto pc) {
+            constexpr int part = decltype(pc)::value;
+            a[s % AHEAD].part[part] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(wr, w_off + part * 1024, q, 0));
+        });
+    };
+    int b_at[2];                               // LDS address of this lane's positions in the patch
+    const int row_bytes = p.dil_h * p.wv * 16; // from one kernel row to the next
+    static_for<0, 2>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const int q = (wn * 2 + j) * 32 + lane % 32;
+        int row, col;
+        const bool ok = decode(q, row, col);
+        const int cell = TAPS == 1 ? q : ok ? (virtual_row(row) - vr0) * p.wv + (col - col0) * p.sw : 0;
+        b_at[j] = ((hf + 2 * wk) * PITCH + cell) * 16;
+    });
+    auto read = [&](auto sc, int at) __attribute__((always_inline)) {
+        constexpr int s = decltype(sc)::value, sub = s / TAPS, tap = s % TAPS;
+        B v;
+        static_for<0, 6>([&](auto ec) {
+            constexpr int j = decltype(ec)::value / 3, part = decltype(ec)::value % 3;
+            v.part[j][part] = *reinterpret_cast<const v4u *>(lds + (b_at[j] + (at + tap / KW * row_bytes)) + part * PART + (2 * WK * sub * PITCH + tap % KW) * 16);
+        });
+        return v;
+    };
+    v16f sum[2], large[2], small[2];
+    auto multiply = [&](const A &w, const B &v) __attribute__((always_inline)) {
+        const auto mfma = [&](auto wc, auto vc, v16f(&to)[2]) __attribute__((always_inline)) {
+            static_for<0, 2>([&](auto jc) {
+                constexpr int j = decltype(jc)::value;
+                to[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, w.part[decltype(wc)::value]),
+                                                                __builtin_bit_cast(v8b, v.part[j][decltype(vc)::value]), to[j], 0, 0, 0);
+            });
+        };
+        const std::integral_constant<int, 0> h;
+        const std::integral_constant<int, 1> m;
+        const std::integral_constant<int, 2> l;
+        mfma(l, h, small);
+        mfma(h, l, small);
+        mfma(m, m, small);
+        mfma(m, h, small);
+        mfma(h, m, small);
+        mfma(h, h, large);
+    };
+
+    // The steps of a chunk: the next step's activations are read under a step's MFMAs, the weights AHEAD steps early.  The next
+    // chunk's patch is stored slot by slot, spread over the steps, and the one behind it requested into the registers that
+    // become free, a few loads a step (all at once they would hold up the weights behind them).  The barrier in front of the
+    // last step: the other buffer is stored, and this one's last reads have returned.
+    auto run = [&](auto form) __attribute__((always_inline)) {
+        const std::integral_constant<int, 0> none;
+        const std::integral_constant<int, 8> all;
+        static_for<0, SLOTS>([&](auto ic) { load_patch(form, ic, none, all, 0); });
+        static_for<0, AHEAD>([&](auto sc) { load_weights(sc, 0); });
+        static_for<0, SLOTS>([&](auto ic) { store_patch(form, ic, 0, 0); });
+        static_for<0, SLOTS>([&](auto ic) { load_patch(form, ic, none, all, 1); });
+        sum[0] = sum[1] = small[0] = small[1] = v16f{};
+        lds_barrier();
+        b = read(none, 0);
+        int chunk = 0, now = 0;
+        do {
+            const int next = BUFFER - now;
+            large[0] = large[1] = v16f{};
+            static_for<0, STEPS>([&](auto sc) {
+                constexpr int s = decltype(sc)::value, slot = s * SLOTS / STEPS, first = (slot * STEPS + SLOTS - 1) / SLOTS;
+                constexpr int steps = ((slot + 1) * STEPS + SLOTS - 1) / SLOTS - first;      // from this slot's store to the next one's
+                const std::integral_constant<int, slot> ic;
+                if constexpr (s + 1 == STEPS) {
+                    if constexpr (s == first) store_patch(form, ic, chunk + 1, next);
+                    lds_barrier();
+                }
+                B after;
+                if constexpr (s + 1 < STEPS) after = read(std::integral_constant<int, s + 1>{}, now);
+                else after = read(none, next);
+                multiply(a[s % AHEAD], b);
+                load_weights(std::integral_constant<int, s + AHEAD < STEPS ? s + AHEAD : STEPS + s % AHEAD>{}, chunk);
+                if constexpr (s == first && s + 1 < STEPS) store_patch(form, ic, chunk + 1, next);
+                load_patch(form, ic, std::integral_constant<int, (s - first) * 8 / steps>{}, std::integral_constant<int, (s - first + 1) * 8 / steps>{}, chunk + 2);
+                b = after;
+                // vector instructions go between the MFMAs, which take 32 cycles each
+                static_for<0, 12>([&](auto) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, s == first ? 8 : 3, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+                });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            sum[0] += large[0];
+            sum[1] += large[1];
+            now = next;
+        } while (++chunk < p.chunks);
+    };
+    if (ragged) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 0>{});
+    if (__syncthreads_or(!(__builtin_fabsf(odd) < __builtin_inff()))) run(std::integral_constant<int, 2>{});
+
+    // ---- bias values of the tile's rows, requested together
+    float bias[16];
+    static_for<0, 16>([&](auto rc) {
+        constexpr int r = decltype(rc)::value;
+        bias[r] = p.bias && wk == 0 ? p.bias[min(m0 + wm * 32 + 8 * (r / 4) + 4 * hf + r % 4, p.M - 1)] : 0.f;
+    });
+    sum[0] += small[0];
+    sum[1] += small[1];
+    if constexpr (WK > 1) {
+        constexpr int SLOT = WM * WN * 32 * 64;
+        float *red = reinterpret_cast<float *>(lds) + (wm * WN + wn) * 32 * 64 + lane;      // the chunks' space takes the partial tiles
+        __syncthreads();                       // the reads ahead have returned
+        if (wk > 0)
+            static_for<0, 32>([&](auto rc) {
+                constexpr int r = decltype(rc)::value;
+                red[(wk - 1) * SLOT + r * 64] = sum[r / 16][r % 16];
+            });
+        __syncthreads();
+        if (wk > 0) return;
+        static_for<0, WK - 1>([&](auto sc) {
+            static_for<0, 32>([&](auto rc) {
+                constexpr int r = decltype(rc)::value;
+                sum[r / 16][r % 16] += red[decltype(sc)::value * SLOT + r * 64];
+            });
+        });
+    }
+    // A lane's element of a row is its own offset plus a uniform one; 32-bit offsets, the output is below 2 GiB.
+    const auto out = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, int(int64_t(p.M) * p.N * 4), 0x00020000);
+    const bool body = p.act_body == int64_t(p.M) * p.N;      // no element behind the activation's SIMD body
+    int in_row = lane % 32;
+    asm volatile("" : "+v"(in_row));           // positions decoded again, not kept over the loop
+    static_for<0, 2>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        int row, col;
+        const bool ok = decode((wn * 2 + j) * 32 + in_row, row, col);
+        const int img = row / p.ho;
+        const int base = img * p.M * p.howo + (row - img * p.ho) * p.wo + col + (m0 + wm * 32 + 4 * hf) * p.howo;
+        static_for<0, 16>([&](auto rc) {
+            constexpr int r = decltype(rc)::value, up = 8 * (r / 4) + r % 4;
+            float v = sum[j][r];
+            if (p.bias) v = __fadd_rn(v, bias[r]);
+            v = apply_act_basic(v, p.act, p.slope, body || base + up * p.howo < p.act_body);
+            const bool in = ok && m0 + wm * 32 + 4 * hf + up < p.M;
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), out, in ? base * 4 : int(NOWHERE), up * p.howo * 4, 0);
+        });
+    });
+}
+
+// ---- tiles.  Each with the patch pitches it is built for, smallest first.
+struct SplitTile {
+    int wm, wn, wk, taps, pitch, cc;
+    int (*launch)(const SplitParams &, hipStream_t);
+    int bm() const { return 32 * wm; }
+    int bn() const { return 64 * wn; }
+};
+
+template <int WM, int WN, int WK, int TAPS, int PITCH, int CC>
+int launch_split(const SplitParams &p, hipStream_t stream) {
+    auto kernel = conv_f32_split_kernel<WM, WN, WK, TAPS, PITCH, CC>;
+    constexpr size_t lds_bytes = std::max(2 * 3 * CC / 8 * PITCH * 16, (WK - 1) * WM * WN * 32 * 64 * 4);
+    static_assert(lds_bytes <= 159 * 1024, "LDS of a compute unit");
+    if (lds_bytes > 65536) {                   // dynamic LDS beyond 64 KiB is granted per kernel and device
+        static std::atomic<bool> granted[64];
+        int dev = 0;
+        TSX_HIP(hipGetDevice(&dev));
+        if (dev >= 64 || !granted[dev].load()) {
+            TSX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds_bytes)));
+            if (dev < 64) granted[dev].store(true);
+        }
+    }
+    const int total = p.tiles_m * p.tiles_n;
+    hipLaunchKernelGGL(kernel, dim3(unsigned((total + 7) / 8 * 8)), dim3(64 * WM * WN * WK), lds_bytes, stream, p);
+    TSX_LAUNCH_CHECK("conv_f32_split_kernel");
+    return 0;
+}
+
+template <int WM, int WN, int WK, int TAPS, int PITCH, int CC>
+constexpr SplitTile split_tile() { return {WM, WN, WK, TAPS, PITCH, CC, launch_split<WM, WN, WK, TAPS, PITCH, CC>}; }
+
+const SplitTile SPLIT_TILES[] = {
+    split_tile<2, 2, 1, 9, 256, 16>(), split_tile<2, 2, 1, 9, 384, 16>(), split_tile<4, 1, 1, 9, 256, 16>(), split_tile<4, 1, 1, 9, 384, 16>(),
+    split_tile<4, 2, 1, 9, 512, 16>(), split_tile<2, 2, 1, 25, 256, 16>(), split_tile<2, 2, 1, 25, 384, 16>(), split_tile<4, 1, 1, 25, 256, 16>(),
+    split_tile<4, 1, 1, 25, 384, 16>(), split_tile<2, 2, 2, 25, 384, 32>(), split_tile<4, 1, 1, 1, 64, 64>(), split_tile<2, 2, 1, 1, 128, 32>(),
+};
+constexpr int SPLIT_TILE_COUNT = int(sizeof(SPLIT_TILES) / sizeof(SPLIT_TILES[0]));
+
+// The launch of one layer with one tile; false if the tile is not the layer's or its patch does not fit.
+bool plan_tile(const ConvF32Layer &l, int tile, bool flat, SplitParams *p) {
+    const SplitTile &t = SPLIT_TILES[tile];
+    const int bn = t.bn(), k = t.taps == 9 ? 3 : t.taps == 25 ? 5 : 1;
+    if (l.kh != k || l.kw != k || l.dil_w != 1 || (k == 1 && !flat)) return false;
+    p->M = l.cout;
+    p->N = int(int64_t(l.n) * l.ho * l.wo);
+    p->n = l.n; p->C = l.c; p->H = l.h; p->W = l.w;
+    p->dil_h = l.dil_h; p->sh = l.stride_h; p->sw = l.stride_w;
+    p->pad_top = l.pad_top; p->pad_left = l.pad_left;
+    p->ho = l.ho; p->wo = l.wo; p->howo = l.ho * l.wo;
+    p->hv = (l.ho - 1) * l.stride_h + (k - 1) * l.dil_h + 1;
+    p->chunks = int(ceil_div(l.c, t.cc));
+    p->mfrags = int(ceil_div(l.cout, 32));
+    p->tiles_m = int(ceil_div(l.cout, t.bm()));
+    p->seg = !flat;
+    p->col_tiles = flat ? 1 : int(ceil_div(l.wo, 32));
+    p->wv = (flat ? l.wo - 1 : 31) * l.stride_w + k;
+    const int64_t tiles_n = flat ? ceil_div(p->N, bn) : int64_t(l.n) * ceil_div(l.ho, bn / 32) * p->col_tiles;
+    if (tiles_n * p->tiles_m >= (int64_t(1) << 22)) return false;
+    p->tiles_n = int(tiles_n);
+    if (k > 1) {
+        // rows of the largest patch: output rows a tile touches, and per image border it crosses the padding rows between
+        const int64_t rows = flat ? ceil_div(bn + l.wo - 1, l.wo) : bn / 32;
+        const int64_t borders = flat ? ceil_div(rows - 1, l.ho) : 0, wrap = std::max(0, p->hv - l.ho * l.stride_h);
+        if (((rows - 1) * l.stride_h + borders * wrap + (k - 1) * l.dil_h + 1) * p->wv > t.pitch) return false;
+    }
+    const int64_t w_bytes = int64_t(p->chunks) * (t.cc / 16) * t.taps * p->mfrags * 3072;
+    if (w_bytes > (int64_t(1) << 31) - 64) return false;
+    p->w_bytes = unsigned(w_bytes);
+    return true;
+}
+
+}  // namespace
+
+ConvF32Split conv_f32_split_choose(const ConvF32Layer &l) {
+    ConvF32Split best{-1, 0, 0.};
+    const char *e = std::getenv("TSX_CONV_F32_SPLIT");         // "0": never; a number: that tile wherever it suits (tests)
+    if (e && e[0] == '0' && !e[1]) return best;
+    const int only = e && e[0] ? std::atoi(e) - 1 : -1;
+    const int64_t most = (int64_t(1) << 31) - 64;              // 32-bit byte offsets into every tensor
+    const int64_t positions = int64_t(l.n) * l.ho * l.wo;
+    if (int64_t(l.n) * l.c * l.h * l.w * 4 > most || positions * l.cout * 4 > most || positions >= (int64_t(1) << 30) || l.pad_top < 0 || l.pad_left < 0)
+        return best;
+    for (int i = 0; i < SPLIT_TILE_COUNT; ++i)
+        for (int flat = 1; flat >= 0; --flat) {
+            SplitParams p{};
+            if ((only >= 0 && i * 2 + flat != only) || !plan_tile(l, i, flat != 0, &p)) continue;
+            const SplitTile &t = SPLIT_TILES[i];
+            // Time of the busiest CU in us, fitted to 45 layers of 0.01 to 17 GFLOP: 12 MFMAs per step at the 1.28 GHz that the
+            // bf16 matrix cores come to beside everything else, 2 for a tile's start and end, 7 for the launches and the weights.
+            const double tiles = double(ceil_div(int64_t(p.tiles_m) * p.tiles_n, 256)), waves = t.wm * t.wn * t.wk / 4;
+            const double us = tiles * (waves * p.chunks * (t.cc / 16 / t.wk) * t.taps * 384 / 1280. + 2) + 7;
+            if (best.tile < 0 || us < best.us) best = {i * 2 + flat, p.w_bytes, us};
+        }
+    if (only >= 0) best.us = 0;
+    return best;
+}
+
+int conv_f32_split(const ConvF32Layer &l, int tile, const float *bias, int act, float slope, float padding_value, float *out, void *workspace,
+                   hipStream_t stream) {
+    SplitParams p{};
+    if (tile < 0 || tile / 2 >= SPLIT_TILE_COUNT || !plan_tile(l, tile / 2, tile % 2 != 0, &p))
+        return fail(TSX_E_INVALID, "conv_f32_split: tile %d does not suit this layer", tile);
+    const SplitTile &t = SPLIT_TILES[tile / 2];
+    const dim3 grid(unsigned(p.mfrags), unsigned(p.chunks * (t.cc / 16)));
+    const auto pack = t.taps == 9 ? split_weights_kernel<9> : t.taps == 25 ? split_weights_kernel<25> : split_weights_kernel<1>;
+    hipLaunchKernelGGL(pack, grid, dim3(256), 0, stream, l.w_dev, l.cout, l.c, p.mfrags, static_cast<v4u *>(workspace));
+    TSX_LAUNCH_CHECK("split_weights_kernel");
+    p.x = l.x_dev;
+    p.w = workspace;
+    p.bias = bias;
+    p.out = out;
+    p.padding_value = padding_value;
+    p.act = act;
+    p.slope = slope;
+    p.act_body = int64_t(p.N) * p.M / 4 * 4;
+    return t.launch(p, stream);
+}
+
+}  // namespace tsx

@@ -1,0 +1,16 @@
+// Internal interface of the fp32 convolution on the bf16 matrix cores (conv2d_f32_split.hip), used by gemm_f32.hip.
+#pragma once
+#include "gemm_f32.hpp"
+
+namespace tsx {
+
+struct ConvF32Split {
+    int tile;                 // -1: no tile suits the layer
+    size_t workspace_bytes;
+    double us;                // expected; 0: the tile is forced
+};
+ConvF32Split conv_f32_split_choose(const ConvF32Layer &l);
+int conv_f32_split(const ConvF32Layer &l, int tile, const float *bias, int act, float slope, float padding_value, float *out, void *workspace,
+                   hipStream_t stream);
+
+}  // namespace tsx

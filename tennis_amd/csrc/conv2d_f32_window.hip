@@ -497,7 +497,7 @@ int launch_tile(int tile, const WinParams &p, size_t lds, hipStream_t s) {
 
 }  // namespace
 
-int conv_f32_window_tile(const ConvF32Layer &l) {
+int conv_f32_window_tile(const ConvF32Layer &l, double *cycles) {
     const int64_t positions = int64_t(l.n) * l.ho * l.wo;
     // 32-bit byte offsets into every tensor
     const int64_t most = (int64_t(1) << 31) - 64;
@@ -529,8 +529,13 @@ int conv_f32_window_tile(const ConvF32Layer &l) {
                 best_cost = cost;
             }
         }
+    // the best tile's fragments on four SIMDs: K / 2 MFMAs of 64 cycles each
+    if (cycles) *cycles = best_cost * l.c * l.kh * l.kw * 8;
     const char *e = std::getenv("TSX_CONV_F32_TILE");
-    if (e && e[0]) best = std::atoi(e);
+    if (e && e[0]) {
+        best = std::atoi(e);
+        if (cycles) *cycles = 0;
+    }
     return best;
 }
 

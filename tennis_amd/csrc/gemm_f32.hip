@@ -17,6 +17,7 @@
 //
 // MFMA layout (32x32x2 f32): lane l supplies A[row l%32][k l/32] and B[k l/32][col l%32];
 // accumulator register r of lane l is row 8*(r/4) + 4*(l/32) + r%4, column l%32.
+#include "conv2d_f32_split.hpp"
 #include "gemm_f32.hpp"
 
 #include <algorithm>
@@ -704,12 +705,26 @@ ConvF32Layer window_layer(const tsx_conv2d_geom *geo, const GemmArgs &g, const C
 // problems of up to a quarter of a GFLOP that the register-fed kernel admits.  Up to a K of some 500 the two take the same
 // few microseconds; with more K the window kernel wins (256 channels at 28x28, 256 3x3 filters: 25 us against 41; 512 at
 // 7x7: 44 against 76), by 7 of 22 us at the far end of what stays with the register-fed one.
-int window_tile(const ConvF32Layer &layer, const GemmArgs &g) {
+int window_tile(const ConvF32Layer &layer, const GemmArgs &g, double *cycles = nullptr) {
     if (choose_gemm(g, 1) == GEMM_REGISTER_FED) {
         const char *e = std::getenv("TSX_GEMM_F32_REGFED");
         if ((e && e[0] == 'f') || ceil_div(g.m, 32) * ceil_div(g.n, 32) * g.k * 2048 < 250000000) return -1;
     }
-    return conv_f32_window_tile(layer);
+    return conv_f32_window_tile(layer, cycles);
+}
+
+// The tile on the bf16 matrix cores for the layer, where that is expected to be at least a twentieth faster than the window
+// kernel; what the register-fed kernel takes stays there.  The window kernel's time is its cost model's at 2.2 GHz times
+// what 45 layers of 0.01 to 17 GFLOP took over it at least: 1.2 with its vector forms, 1.9 without (1.6 to 4.6 measured).  Kept
+// on the window kernel by that: 1x256x28x28, 256 3x3 filters (25 us against 43), 8x512x14x14 to 512 1x1 (14 against 20), all
+// layers of some 10 us.
+ConvF32Split split_choice(const ConvF32Layer &layer, const GemmArgs &g) {
+    double cycles = 0;
+    const ConvF32Split none{-1, 0, 0.}, split = conv_f32_split_choose(layer);
+    if (split.tile < 0 || window_tile(layer, g, &cycles) < 0) return none;
+    if (split.us == 0) return split;
+    const bool vector = layer.c * layer.kh * layer.kw % 4 == 0 && (layer.kh == 1 || layer.kh == 3) && reinterpret_cast<uintptr_t>(layer.w_dev) % 16 == 0;
+    return split.us * 1.05 < cycles / 2200 * (vector ? 1.2 : 1.9) + 4 ? split : none;
 }
 
 }  // namespace
@@ -762,8 +777,22 @@ static int conv_f32_problem(const tsx_conv2d_geom *geo, const float *x_dev, cons
     return 0;
 }
 
+size_t tsx_conv2d_f32_workspace_bytes(const tsx_conv2d_geom *geo, const float *w_oihw_dev) {
+    tsx::GemmArgs g;
+    tsx::ConvLoader ld;
+    if (!geo || conv_f32_problem(geo, nullptr, w_oihw_dev, 0.f, nullptr, TSX_ACT_NONE, 0.f, nullptr, g, ld)) return 0;
+    if (tsx::conv3x3_small_takes(g, ld)) return 0;
+    return tsx::split_choice(tsx::window_layer(geo, g, ld), g).workspace_bytes;
+}
+
 int tsx_conv2d_f32_nchw(const tsx_conv2d_geom *geo, const float *x_dev, const float *w_oihw_dev, float padding_value,
                         const float *bias_dev, int32_t act, float slope, float *out_dev, void *stream) {
+    return tsx_conv2d_f32_nchw_ws(geo, x_dev, w_oihw_dev, padding_value, bias_dev, act, slope, out_dev, nullptr, 0, stream);
+}
+
+int tsx_conv2d_f32_nchw_ws(const tsx_conv2d_geom *geo, const float *x_dev, const float *w_oihw_dev, float padding_value,
+                           const float *bias_dev, int32_t act, float slope, float *out_dev, void *workspace_dev,
+                           size_t workspace_bytes, void *stream) {
     TSX_REQUIRE(geo && x_dev && w_oihw_dev && out_dev, "conv2d_f32: null argument");
     tsx::GemmArgs g;
     tsx::ConvLoader ld;
@@ -773,6 +802,12 @@ int tsx_conv2d_f32_nchw(const tsx_conv2d_geom *geo, const float *x_dev, const fl
         return geo->c <= 32 ? tsx::launch_conv3x3_small<2>(g, ld, tsx::as_stream(stream))
                             : tsx::launch_conv3x3_small<4>(g, ld, tsx::as_stream(stream));
     const tsx::ConvF32Layer layer = tsx::window_layer(geo, g, ld);
+    if (workspace_dev) {
+        TSX_REQUIRE(reinterpret_cast<uintptr_t>(workspace_dev) % 16 == 0, "conv2d_f32: workspace not aligned to 16 bytes");
+        const tsx::ConvF32Split split = tsx::split_choice(layer, g);
+        if (split.tile >= 0 && split.workspace_bytes <= workspace_bytes)
+            return tsx::conv_f32_split(layer, split.tile, bias_dev, act, slope, padding_value, out_dev, workspace_dev, tsx::as_stream(stream));
+    }
     const int tile = tsx::window_tile(layer, g);
     if (tile >= 0)
         return tsx::conv_f32_window(layer, tile, bias_dev, act, slope, padding_value, out_dev, tsx::as_stream(stream));

@@ -10,8 +10,9 @@ struct ConvF32Layer {
     const float *x_dev, *w_dev;
 };
 
-// The tile (and patch form) the kernel would take for the layer, -1 where it cannot; its extents; the launch.
-int conv_f32_window_tile(const ConvF32Layer &l);
+// The tile (and patch form) the kernel would take for the layer, -1 where it cannot, and the cycles expected of the busiest
+// CU (0: the tile is forced); its extents; the launch.
+int conv_f32_window_tile(const ConvF32Layer &l, double *cycles = nullptr);
 void conv_f32_window_tile_size(int tile, int *rows, int *positions);
 int conv_f32_window(const ConvF32Layer &l, int tile, const float *bias, int act, float slope, float padding_value, float *out,
                     hipStream_t stream);

@@ -27,7 +27,7 @@ namespace {
 
 #define TSX_NATIVE_ENTRIES(X)                                                                                              \
     X(tsx_last_error) X(tsx_conv2d_out_size) X(tsx_quantize_f32_i8) X(tsx_conv2d_i8_nchw) X(tsx_quantize_conv2d_i8_nchw)     \
-    X(tsx_conv2d_i8_staged_at) X(tsx_gemm_i8) X(tsx_conv2d_f32_nchw) X(tsx_inner_prod_f32) X(tsx_add_bias_f32)              \
+    X(tsx_conv2d_i8_staged_at) X(tsx_gemm_i8) X(tsx_conv2d_f32_nchw_ws) X(tsx_conv2d_f32_workspace_bytes) X(tsx_inner_prod_f32) X(tsx_add_bias_f32)              \
     X(tsx_relu_f32) X(tsx_leaky_relu_f32) X(tsx_add_f32) X(tsx_mul_f32) X(tsx_mish_f32) X(tsx_softplus_f32) X(tsx_tanh_f32) \
     X(tsx_batch_norm_f32) X(tsx_batch_scale_f32) X(tsx_fused_batch_norm_f32) X(tsx_depthwise_conv2d_f32)                    \
     X(tsx_pooling2d_out_size) X(tsx_pooling2d_f32) X(tsx_max_pooling2d_i8_staged) X(tsx_winograd_f63_workspace_bytes)       \
@@ -362,8 +362,11 @@ PyObject *conv2d_f32(PyObject *const *a, Py_ssize_t) {  // x, w, pads, strides, 
     at::TensorBase out;
     launch([&] {
         out = empty({g.n, g.cout, o.h, o.w}, c10::kFloat, x);
-        return L.tsx_conv2d_f32_nchw(&g, x.const_data_ptr<float>(), w.const_data_ptr<float>(), padding_value, bias, act, slope, data<float>(out),
-                                     stream());
+        const size_t bytes = L.tsx_conv2d_f32_workspace_bytes(&g, w.const_data_ptr<float>());
+        at::TensorBase workspace;     // the allocator's again when the call is enqueued, for what follows on this stream
+        if (bytes) workspace = empty({int64_t(bytes)}, c10::kByte, x);
+        return L.tsx_conv2d_f32_nchw_ws(&g, x.const_data_ptr<float>(), w.const_data_ptr<float>(), padding_value, bias, act, slope, data<float>(out),
+                                        data<uint8_t>(workspace), bytes, stream());
     });
     return wrap(out);
 }
