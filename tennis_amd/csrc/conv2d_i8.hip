@@ -960,6 +960,8 @@ int make_plan(const tsx_conv2d_geom *g, Plan *pl) {
         if (pl->wsp.ok && !strided_1x1) {
             pl->use_ws = true;
             pl->packed_bytes = pl->wsp.packed_bytes;
+        } else if (strided_1x1) {
+            pl->wsp.coutp = pl->coutp;     // the K-split kernel, which small ones take, reads the generic kernel's weights
         }
     }
     return 0;
@@ -1126,7 +1128,7 @@ int run_staged(const tsx_conv2d_geom *g, const Plan &pl, const void *staged, con
     p.o_c = g->cout;
     p.o_h = pl.ho;
     p.o_w = pl.wo;
-    if (pl.use_ws)
+    if (pl.use_ws || pl.wsp.ks)
         return tsx::ws_launch(pl.wsg, pl.wsp, p.xs, p.wp, static_cast<const tsx::EpiParams &>(p), stream);
     return launch_igemm<false>(p, stream);
 }
@@ -1179,6 +1181,7 @@ int tsx_conv2d_i8_plan_info(const tsx_conv2d_geom *g, char *text, size_t text_by
                       base, base, pl.wsp.nt, pl.wsp.wm, (long long)(pl.wsp.tiles * ((g->cout + 32 * pl.wsp.wm - 1) / (32 * pl.wsp.wm))), pl.wsp.cbs);
     else
         std::snprintf(text, text_bytes, "kernel=%s fp32_kernel=%s", base, base);
+    if (pl.wsp.ks) std::snprintf(text, text_bytes, "kernel=k_split fp32_kernel=k_split tile=%d", pl.wsp.ks);
     return 0;
 }
 
@@ -1365,6 +1368,11 @@ int tsx_conv2d_i8_staged_at(const tsx_conv2d_geom *g, const void *staged_dev, in
             return tsx::fail(TSX_E_INVALID, "staged_at: a %dx%d staged buffer does not fit this layer's kernel", staged_hs,
                              staged_ws);
         }
+    } else if (pl.wsp.ks) {
+        pl.wsg.hs = staged_hs;
+        pl.wsg.ws = staged_ws;
+        const tsx::WsPlan wide = tsx::ws_plan(pl.wsg);
+        pl.wsp.ks = wide.ok ? wide.ks : 0;
     }
     return run_staged(g, pl, staged_dev, packed_w_dev, ep, out_f32_dev, out_i8_dev, out_acc_dev, tsx::as_stream(stream));
 }

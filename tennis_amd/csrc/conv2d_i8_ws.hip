@@ -32,6 +32,7 @@
 // K bytes of group l/32 (two MFMAs, "halves", cover a 64-byte K-step); accumulator register r
 // of lane l is row 8*(r/4) + 4*(l/32) + r%4, column l%32.  Rows = cout, columns = positions.
 #include "conv2d_i8_ws_kernel.hpp"
+#include "conv2d_i8_ks.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -79,7 +80,7 @@ static WsPlan make_ws_plan(const WsGeom &g_in);
 WsPlan ws_plan(const WsGeom &g) {
     struct Key {
         WsGeom g;
-        char flat[12], rs[12];
+        char flat[12], rs[12], ks[12];
     };
     struct Slot {
         Key key;
@@ -91,10 +92,14 @@ WsPlan ws_plan(const WsGeom &g) {
     Key key;
     std::memset(&key, 0, sizeof(key));
     key.g = g;
-    const char *flat = std::getenv("TSX_CONV_I8_FLAT"), *rs = std::getenv("TSX_CONV_I8_RS");
-    if ((flat && std::strlen(flat) >= sizeof(key.flat)) || (rs && std::strlen(rs) >= sizeof(key.rs))) return make_ws_plan(g);
-    if (flat) std::strcpy(key.flat, flat);
-    if (rs) std::strcpy(key.rs, rs);
+    const char *flat = std::getenv("TSX_CONV_I8_FLAT"), *rs = std::getenv("TSX_CONV_I8_RS"), *ks = std::getenv("TSX_CONV_I8_KS");
+    if ((flat && std::strlen(flat) + 1 >= sizeof(key.flat)) || (rs && std::strlen(rs) + 1 >= sizeof(key.rs)) || (ks && std::strlen(ks) + 1 >= sizeof(key.ks)))
+        return make_ws_plan(g);
+    // (set but empty is another choice than not set)
+    const auto note = [](char *to, const char *value) { if (value) { to[0] = '='; std::strcpy(to + 1, value); } };
+    note(key.flat, flat);
+    note(key.rs, rs);
+    note(key.ks, ks);
     static thread_local struct Owner {
         ~Owner() { delete[] slots; slots = nullptr; }
     } owner;
@@ -210,6 +215,7 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
     pl.ok = true;
     fl_plan(g_in, &pl);   // layers the flat-tile kernel suits better (same packed weights)
     rs_plan(g_in, &pl);   // ... and the weight-stationary one
+    ks_plan(g_in, &pl);   // ... and the one that splits K
     return pl;
 }
 
@@ -223,6 +229,7 @@ int ws_pack_weights(const WsGeom &g, const WsPlan &pl, const int8_t *w_oihw, int
 
 int ws_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t *packed, const EpiParams &ep,
               hipStream_t stream) {
+    if (pl.ks) return ks_launch(g, pl, xs, packed, ep, stream);
     if (rs_takes(pl, ep, int64_t(g.n) * g.cout * g.ho * g.wo)) return rs_launch(g, pl, xs, packed, ep, stream);
     if (pl.flat) return fl_launch(g, pl, xs, packed, ep, stream);
     WsParams p{};
