@@ -122,10 +122,11 @@ int tsx_conv2d_i8_pack_weights(const tsx_conv2d_geom *g, const int8_t *w_oihw_de
 /* Scratch the conv needs (channel-blocked padded copy of the activations). */
 size_t tsx_conv2d_i8_workspace_bytes(const tsx_conv2d_geom *g);
 /* Which kernel the plan of this layer launches, as text ("kernel=flat_tile fp32_kernel=weight_stationary ..."):
- * kernel = igemm | window_stationary | flat_tile, and fp32_kernel = the kernel that takes the layer when the
+ * kernel = igemm | window_stationary | flat_tile | k_split, and fp32_kernel = the kernel that takes the layer when the
  * epilogue is fp32 output with dequantize scales, bias and activation only.  No counterpart in the reference; for
  * tests that must know a given kernel ran, and for logs.  The environment variables TSX_CONV_I8_FLAT and
- * TSX_CONV_I8_RS ("0" = never, "force" = wherever the geometry allows) are read at every call that plans. */
+ * TSX_CONV_I8_RS ("0" = never, "force" = wherever the geometry allows) are read at every call that plans, and so is
+ * TSX_CONV_I8_KS ("0" = never, a number = that tile of the K-split kernel wherever the geometry allows). */
 int tsx_conv2d_i8_plan_info(const tsx_conv2d_geom *g, char *text, size_t text_bytes);
 /* padding_value is the reference's float parameter; it is cast to int8 as the reference
  * does (conv2d_quantized_core.cpp:72).  Any of out_f32_dev / out_i8_dev / out_acc_dev may be

@@ -280,7 +280,11 @@ int ws_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t 
     p.tw_magic = div_magic(p.tw, 4 * 7 * 32);
     p.ow_magic = div_magic(ep.o_w, int64_t(p.ho) * p.wo);
     const int bm = 32 * WS_FM * pl.wm;
-    const dim3 grid(unsigned(pl.tiles), unsigned((g.cout + bm - 1) / bm));
+    p.tiles = int(pl.tiles);
+    p.blocks_m = (g.cout + bm - 1) / bm;
+    const int64_t total = pl.tiles * p.blocks_m;
+    p.per_xcd = total < (1 << 23) ? int((total + 7) / 8) : 0;      // (a launch holds fewer than 2^32 work items along x)
+    const dim3 grid = p.per_xcd ? dim3(unsigned(p.per_xcd * 8)) : dim3(unsigned(pl.tiles), unsigned(p.blocks_m));
     // two window buffers (one channel block ahead); a layer whose channels fit one window never swaps and takes one:
     // more workgroups per CU where the window is large (stride-2 3x3 layers on 32 or 64 channels)
     const size_t lds_bytes = size_t(p.cblocks > 1 ? 2 : 1) * pl.wp * (64 * pl.cbs + 16);

@@ -28,6 +28,7 @@ struct WsParams : EpiParams {
     // a tap is tap_row/tap_col bytes further into the window per kernel row / column (for cbs > 1 the "taps"
     // are the window's channel blocks: kh = 1, kw = cbs, tap_col = 64)
     int pix, chunk_shift, stage_bytes, tap_row, tap_col;
+    int per_xcd, tiles, blocks_m;   // workgroups of each XCD's run (0: grid of tiles x channel blocks), position tiles, channel blocks
     int stream_out;   // fp32 output written with streaming stores
     int rowmajor;     // GEMM: output index position * cout + channel, row_scale[position] applied behind dq
     // per-lane divisions by uniform divisors as one multiply-high (div_magic / udiv)
@@ -82,8 +83,18 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
     // the wavefront's index as a scalar: what derives from it (first cout, tile bases, the choice of epilogue path)
     // then stays in scalar registers and branches uniformly
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
-    const int rtile = blockIdx.x / p.ctiles;
-    const int col0 = (blockIdx.x - rtile * p.ctiles) * p.tw;   // first output column of the tile
+    // Each XCD takes a contiguous run of position tiles with all their channel blocks: what neighbouring tiles share -- the
+    // cache line that a run of output positions ends in, halo rows, the window that all channel blocks read -- meets in one
+    // L2, and so does what the layer before left there for these positions.
+    int tile = blockIdx.x, block_m = blockIdx.y;
+    if (p.per_xcd) {
+        const int t = int(blockIdx.x & 7) * p.per_xcd + int(blockIdx.x >> 3);
+        tile = p.blocks_m == 1 ? t : t / p.blocks_m;
+        block_m = t - tile * p.blocks_m;
+        if (tile >= p.tiles) return;
+    }
+    const int rtile = p.ctiles == 1 ? tile : tile / p.ctiles;
+    const int col0 = (tile - rtile * p.ctiles) * p.tw;         // first output column of the tile
     const int row0 = rtile * p.th;           // first output row of the tile, counted over the whole batch
     const int img = row0 / p.ho;             // image of the tile's first row
     const int th0 = row0 - img * p.ho;       // ... and that row inside it
@@ -92,7 +103,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
     const int wrap = p.hs - p.ho * p.sh;
     const int wave_m = wave & (p.wm - 1);                            // position along cout
     const int pos0 = (p.wm == 4 ? 0 : p.wm == 2 ? wave >> 1 : wave) * (NT * 32);   // first tile position of this wavefront
-    const int m0 = (blockIdx.y * p.wm + wave_m) * (32 * FM);         // first cout of this wavefront
+    const int m0 = (block_m * p.wm + wave_m) * (32 * FM);         // first cout of this wavefront
     const int taps = p.kh * p.kw;
     const int win_bytes = p.wpix * p.pix;
 
@@ -554,7 +565,7 @@ int ws_launch_nt<TSX_WS_NT>(const WsParams &p, dim3 grid, size_t lds_bytes, hipS
     const bool small_fill = NT <= 2 && ((p.wpix << p.chunk_shift) + WS_THREADS - 1) / WS_THREADS <= SMALL_FILL;
     // one fragment per wavefront, a K of two rounds or more, and few enough workgroups that a SIMD holds one or
     // two wavefronts: the B ring (more registers: three workgroups per CU)
-    const bool look = NT == 1 && small_fill && p.ksteps >= 2 * RING && int64_t(grid.x) * grid.y <= 1024;
+    const bool look = NT == 1 && small_fill && p.ksteps >= 2 * RING && int64_t(p.tiles) * p.blocks_m <= 1024;
 #define TSX_WS_LAUNCH(EXTRA, STREAM, ROWM, MISHX)                                                                      \
     do {                                                                                                               \
         constexpr int F = NT <= 2 ? SMALL_FILL : MAX_FILL;                                                             \
