@@ -133,16 +133,11 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
     pl.wo = g.wo;
     pl.hs = g.hs;
     pl.ws = g.ws;
-    // A tile is TH output rows of the batch-wide row sequence x TW output columns (whole rows when they fit),
-    // at most MAX_NT fragments of 32 positions per wavefront.  Candidates are ranked by a model of the busiest
-    // CU's time in units of one fragment's work,
-    //     (rounds of resident workgroups) x (overlap factor) x (0.5 + fragments x slow),
-    // where 0.5 is the per-workgroup fixed cost and slow = 1.45 for tiles of more than 4 fragments
-    // (one workgroup per CU, so one wavefront per SIMD with nothing to hide its LDS/L2 waits).  The
-    // constants come from a sweep over 32x256x28x28 (1/2/4/8-row tiles: 35 / 30.5 / 23.0 / 23.4 us) and the
-    // layers of a ResNet-50-shaped network, whose small maps want many small workgroups: 196 workgroups of 4
-    // fragments per wavefront (60 CUs idle) take 11.7 us on 32x512x28x28 -> 128 channels, 392 of 2 take 9.4.
-    // Ties go to the fewest total fragments (least padding).
+    // A tile is TH output rows of the batch-wide row sequence x TW output columns, at most MAX_NT fragments of 32 positions
+    // per wavefront.  Candidates are ranked by a model of the busiest CU's time in units of one fragment's work,
+    //     (rounds of resident workgroups) x (overlap factor) x (fixed + fragments x slow),
+    // where slow = 1.45 for tiles of more than 4 fragments (one workgroup per CU, so one wavefront per SIMD with nothing to
+    // hide its LDS/L2 waits).  Ties go to the fewest total fragments (least padding), then to the longest rows.
     constexpr int MAX_NT = 7;
     // few output channels: fewer wavefronts along cout, the others take more positions of a larger tile
     const int wm = g.cout <= 32 ? 1 : g.cout <= 64 ? 2 : 4, wn = 4 / wm;
@@ -155,9 +150,7 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
     const int ksteps_p = (g.cblocks * g.kh * g.kw + RING - 1) / RING * RING;
     double best_cost = -1;
     int64_t best_frags = 0;
-    // tile widths: the whole row where it (and its window) fits, else multiples of 32 columns (a fragment is
-    // then one run of a row)
-    const bool tiny_k = g.cblocks * g.kh * g.kw <= 2;
+    const bool several_taps = g.kh * g.kw > 1;
     auto consider = [&](int tw) {
         const int ctiles = (g.wo + tw - 1) / tw;
         const int wc = (tw - 1) * g.sw + (g.kw - 1) * g.dil_w + 1;
@@ -170,18 +163,32 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
             if (wp > MAX_WP || size_t(2) * wp * PIX > 65536) continue;   // two windows must fit 64 KiB of LDS
             const int64_t wgs = tiles * (coutp / bm);
             const int64_t frags = tiles * nt * wn;
-            // workgroups of up to 2 fragments per wavefront fit three to a CU, up to 4 two, larger ones one; those
-            // resident together overlap (each further one adds about half of a lone workgroup's time), the rest
-            // run in rounds -- so a layer that leaves CUs idle with large tiles takes tiles of half the size
             const int64_t per_cu = (wgs + 255) / 256;
-            const int resident = nt <= 2 ? 3 : nt <= 4 ? 2 : 1;
-            const int64_t rounds = (per_cu + resident - 1) / resident;
-            const double together = 1.0 + 0.5 * double(std::min<int64_t>(per_cu, resident) - 1);
-            const double cost = double(rounds) * together * (0.5 + nt * (nt > 4 ? 1.45 : 1.0));
-            // One or two K-steps (a 1x1 layer on 64 or 128 channels): the workgroup is all epilogue, its time is the
-            // store traffic of its tile, and what pays is many small workgroups in flight per CU -- measured on
-            // 32x64x56x56 -> 256 channels: 63 us with 4 fragments per wavefront and a residual join, 55 us with 2.
-            if (tiny_k && nt > 2) continue;
+            double cost;
+            if (several_taps) {
+                // Small near-square tiles: their windows hold few pixels beyond their own, four (one fragment per wavefront)
+                // or three (two) of them share a CU, and beyond two rounds a CU takes its next one as soon as one ends.  A
+                // wavefront with one fragment still fetches a K-step's weights, 0.3 of a fragment's work at 1.6.  Fitted to
+                // some thousand tiles of 35 3x3 layers (us, whole rows before -> now, exact Mish: 8 images of 76x76, 128 to 128
+                // channels 25.9 -> 17.8, with a residual 52.8 -> 34.5, 38x38, 256 to 256, with a residual 37.0 -> 25.5, 152x152,
+                // 128 to 256 at stride 2, 41.5 -> 31.8; leaky, 76x76, 128 to 256: 26.2 -> 23.0).
+                const bool small = nt <= 2 && (wp * 4 + WS_THREADS - 1) / WS_THREADS <= SMALL_FILL;
+                const int resident = small ? (nt == 1 ? 4 : 3) : nt <= 4 ? 2 : 1;
+                const double rounds = per_cu <= 2 * resident ? double((per_cu + resident - 1) / resident) : double(wgs) / 256 / resident + 0.5;
+                const double work = nt * (nt > 4 ? 1.45 : 1.0);
+                cost = rounds * (1.0 + 0.55 * double(std::min<int64_t>(per_cu, resident) - 1)) * (0.2 + 0.7 * work + 0.3 * std::max(work, 1.6));
+            } else {
+                // Workgroups of up to 2 fragments per wavefront fit three to a CU, up to 4 two, larger ones one; those
+                // resident together overlap (each further one adds about half of a lone workgroup's time), the rest run in
+                // rounds -- so a layer that leaves CUs idle with large tiles takes tiles of half the size.
+                const int resident = nt <= 2 ? 3 : nt <= 4 ? 2 : 1;
+                const int64_t rounds = (per_cu + resident - 1) / resident;
+                cost = double(rounds) * (1.0 + 0.5 * double(std::min<int64_t>(per_cu, resident) - 1)) * (0.5 + nt * (nt > 4 ? 1.45 : 1.0));
+            }
+            // A 1x1 layer's workgroup is mostly epilogue, its time is the traffic of its tile, and what pays is many small
+            // workgroups in flight per CU (us, 32 images: 64 to 256 channels 56x56 with a residual join, 4 fragments per
+            // wavefront 63, 2 55; 256 to 128 56x56 20.9 -> 17.9; 256 to 1024 14x14 with a join 18.1 -> 15.8).
+            if (!several_taps && (!g.gemm || g.cblocks <= 2) && nt > 2) continue;
             if (best_cost < 0 || cost < best_cost || (cost == best_cost && frags < best_frags)) {
                 best_cost = cost;
                 best_frags = frags;
@@ -197,6 +204,13 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
         }
     };
     if (g.wo <= cap) consider(g.wo);
+    if (several_taps) {
+        // equal shares of a row, and widths that fill fragments with a few rows
+        for (int tw = 64; tw >= 8; tw /= 2)
+            if (tw < g.wo) consider(tw);
+        for (int parts = 2; parts <= 8; ++parts)
+            if ((g.wo + parts - 1) / parts >= 8) consider((g.wo + parts - 1) / parts);
+    }
     if (best_cost < 0)
         for (int tw = 32; tw <= cap && tw < g.wo; tw += 32) consider(tw);
     if (best_cost < 0 || pl.tiles >= (int64_t(1) << 31)) return pl;
@@ -227,8 +241,17 @@ int ws_pack_weights(const WsGeom &g, const WsPlan &pl, const int8_t *w_oihw, int
     return 0;
 }
 
-int ws_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t *packed, const EpiParams &ep,
+int ws_launch(const WsGeom &g, const WsPlan &plan, const int8_t *xs, const int8_t *packed, const EpiParams &ep,
               hipStream_t stream) {
+    WsPlan pl = plan;
+    // The exact Mish's arithmetic is most of a 1x1 layer: tiles of one fragment per wavefront, which hide it behind one another
+    // (us, 8 images: 64 to 64 channels 304x304, fp32 output, 146 -> 138; 128 to 64 152x152 45.8 -> 40.4).  A small grid keeps
+    // its tiles.
+    if (ep.act == TSX_ACT_MISH && g.kh * g.kw == 1 && pl.wo == 1 && pl.nt == 2 && pl.th == pl.wp && pl.th % 2 == 0 && pl.tiles * ceil_div(g.cout, 32 * pl.wm) >= 1024) {
+        pl.nt = 1;
+        pl.th = pl.wr = pl.wp = pl.th / 2;
+        pl.tiles = ceil_div(int64_t(g.n) * pl.ho, pl.th);
+    }
     if (pl.ks) return ks_launch(g, pl, xs, packed, ep, stream);
     if (rs_takes(pl, ep, int64_t(g.n) * g.cout * g.ho * g.wo)) return rs_launch(g, pl, xs, packed, ep, stream);
     if (pl.flat) return fl_launch(g, pl, xs, packed, ep, stream);

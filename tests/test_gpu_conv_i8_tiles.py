@@ -1,0 +1,51 @@
+"""The window-stationary int8 kernel on tiles narrower than the map: last column tiles that end outside it, tiles that span two
+images, strides, and runs of one image's end and the next one's start on different workgroups, against the CPU oracle bit for bit."""
+import numpy as np
+import pytest
+
+from _util import bits
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+@pytest.mark.parametrize("act", ["leaky_relu", "mish"])
+@pytest.mark.parametrize("case", [
+    # n, c, h, w, cout, k, stride
+    (8, 64, 38, 37, 96, 3, 1), (9, 70, 19, 19, 130, 3, 1), (4, 33, 77, 75, 64, 3, 2), (3, 64, 43, 100, 40, 3, 1), (2, 20, 61, 130, 20, 5, 1),
+    (16, 16, 11, 301, 64, 3, 1), (5, 40, 57, 113, 65, 1, 1),
+], ids=lambda c: "-".join(map(str, c)))
+def test_conv_i8_tiles(port, monkeypatch, case, act):
+    from tennis_amd import capi
+    monkeypatch.setenv("TSX_CONV_I8_KS", "0")
+    monkeypatch.setenv("TSX_CONV_I8_FLAT", "0")
+    n, c, h, w, cout, k, s = case
+    rng = np.random.default_rng(63)
+    x = rng.integers(-128, 128, (n, c, h, w)).astype(np.int8)
+    wt = rng.integers(-127, 128, (cout, c, k, k)).astype(np.int8)
+    dq = rng.uniform(1e-5, 3e-5, cout).astype(np.float32)
+    bias = rng.standard_normal(cout).astype(np.float32)
+    qs = rng.uniform(20, 30, n).astype(np.float32)
+    conv = capi.Conv2dI8(dev(wt), (k // 2,) * 4, (s, s))
+    info = capi.conv2d_i8_plan_info(conv._plan(x.shape)[0])
+    assert info["kernel"] == "window_stationary" and info["fragments_per_wavefront"] in "1234", info
+    plain = port.add_bias(port.conv2d_quantized(x, wt, dq, (k // 2,) * 4, (s, s)), bias)
+    exp = port.leaky_relu(plain, 0.1) if act == "leaky_relu" else port.mish(plain)
+    exp_q = port.quantize(exp, qs)
+    out, q, _ = conv(dev(x), dq=dev(dq), bias=dev(bias), act=act, slope=0.1, q_scales=dev(qs))
+    assert np.array_equal(bits(out.cpu().numpy()), bits(exp)) and np.array_equal(q.cpu().numpy(), exp_q)
+    # ... into the next layer's staged input, behind a residual join
+    second = capi.Conv2dI8(dev(rng.integers(-127, 128, (8, cout, 3, 3)).astype(np.int8)), (1, 1, 1, 1))
+    dq2 = rng.uniform(1e-4, 3e-4, 8).astype(np.float32)
+    staged, to = capi.StagedInput(conv, x.shape), capi.StagedInput(second, exp.shape)
+    conv.stage(dev(x), staged)
+    res = rng.standard_normal(exp.shape).astype(np.float32)
+    out = conv.run_staged(staged, dev(dq), dev(bias), act, 0.1, q_scales=dev(qs), residual=dev(res), residual_after_act=True, staged_out=to)[0]
+    joined = port.add(exp, res)
+    assert np.array_equal(bits(out.cpu().numpy()), bits(joined))
+    got = second.run_staged(to, dev(dq2))[0].cpu().numpy()
+    assert np.array_equal(bits(got), bits(port.conv2d_quantized(port.quantize(joined, qs), second.w.cpu().numpy(), dq2, (1, 1, 1, 1))))
