@@ -276,6 +276,112 @@ __global__ __launch_bounds__(256) void stage_im2col_rows_kernel(const void *__re
     }
 }
 
+// ... for kernels of three and more columns without column dilation, on images whose width is a multiple of 4, R output rows
+// per workgroup.  The patch holds a dword per byte, the byte and the three to its right: any 4 consecutive bytes of the K axis
+// are then one aligned read, or two (the end of one kernel row, the start of the next) and a byte permute, where the form above
+// reads byte by byte; and R rows share the patch rows that several of them read.  What bounds it: the conversions, each
+// (R SH + KH - SH) / (R SH) times, and the stores.  32 images 3x224x224, 7x9 at strides 2 and 4: 36.9 us by bytes, 19.5 here
+// (57 MB: 2.9 TB/s); 8 images 3x608x608, 3x4: 59.8, 28 (224 MB: 8 TB/s, most of it into the caches); one image 3x224x224: 9.8, 6.3.
+template <bool QUANT>
+__global__ __launch_bounds__(256) void stage_im2col_words_kernel(const void *__restrict__ src, Im2colGeom g, int wpatch, int R,
+                                                                const float *__restrict__ scales, int n_scales, int64_t bulk8,
+                                                                int8_t *__restrict__ xs) {
+    extern __shared__ __attribute__((aligned(16))) int8_t lds[];
+    uint32_t *patch = reinterpret_cast<uint32_t *>(lds);             // [c][patch rows][wpatch]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int groups = (g.ho + R - 1) / R, ni = blockIdx.x / groups, oh0 = (blockIdx.x - ni * groups) * R;
+    const float scale = QUANT ? scales[n_scales == 1 ? 0 : ni] : 0.f;
+    const int h0 = oh0 * g.sh - g.pad_top, prows = (R - 1) * g.sh + (g.kh - 1) * g.dh + 1;
+    // phase 1: a wavefront takes every fourth run of 252 columns of a patch row, a lane four columns (the last lane's serve the
+    // one before it).  Patch columns count from image column -4 on, and the image's width is a multiple of 4: a lane's
+    // columns are all in the image or all beside it, one load.
+    constexpr int RUN = 63, BATCH = 4;
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+    const int quads = wpatch / 4, runs = (quads + RUN - 1) / RUN;
+    const uint32_t pad = uint32_t(g.pad_value & 0xff) * 0x01010101u;
+    int run = wave, r = 0, ci = 0;
+    auto settle = [&]() {
+        while (run >= runs) {
+            run -= runs;
+            if (++r == prows) {
+                r = 0;
+                ++ci;
+            }
+        }
+    };
+    settle();
+    while (ci < g.c) {
+        v4f fv[BATCH];
+        uint32_t bv[BATCH];
+        int to[BATCH];
+        bool in[BATCH], even[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            const int hi = h0 + r, quad = run * RUN + lane, wi = 4 * quad - 4;
+            in[u] = ci < g.c && hi >= 0 && hi < g.h && wi >= 0 && wi < g.w;
+            to[u] = ci < g.c && lane < RUN && quad < quads ? (ci * prows + r) * quads + quad : -1;
+            // unconditional loads (the row's first elements where the cells are halo): a load behind a branch is waited for
+            // before the next one is issued
+            const int64_t row = ci < g.c && hi >= 0 && hi < g.h ? ((int64_t(ni) * g.c + ci) * g.h + hi) * g.w : 0;
+            const unsigned lane_at = in[u] ? unsigned(wi) : 0u;
+            even[u] = n_scales == 1 && row + lane_at < bulk8;        // (both multiples of 4, and bulk8 of 8)
+            typedef v4f v4f_at_4 __attribute__((aligned(4)));
+            if (QUANT) fv[u] = *reinterpret_cast<const v4f_at_4 *>(static_cast<const float *>(src) + row + lane_at);
+            else __builtin_memcpy(&bv[u], static_cast<const int8_t *>(src) + row + lane_at, 4);
+            run += 4;
+            settle();
+        }
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            uint32_t four = 0;
+            if (QUANT) {
+                tsx::static_for<0, 4>([&](auto jc) {
+                    constexpr int j = decltype(jc)::value;
+                    four = tsx::quantize_pack<j>(__fmul_rn(fv[u][j], scale), even[u], four);
+                });
+                four ^= 0x80808080u;
+            } else {
+                four = bv[u];
+            }
+            four = in[u] ? four : pad;
+            const uint32_t next = uint32_t(__builtin_amdgcn_update_dpp(0, int(four), 0x130, 0xf, 0xf, false));     // wave_shl:1
+            const v4u cells = {four, __builtin_amdgcn_alignbyte(next, four, 1), __builtin_amdgcn_alignbyte(next, four, 2),
+                               __builtin_amdgcn_alignbyte(next, four, 3)};
+            if (to[u] >= 0) reinterpret_cast<v4u *>(patch)[to[u]] = cells;
+        }
+    }
+    __syncthreads();
+    // phase 2: a lane keeps one K chunk; of each of its dwords, where the 4 bytes lie (A), and where the ones of the next
+    // kernel row lie (B), and which bytes of both to take (0x0c: zero, beyond K)
+    const int chunks = g.cp / 16, ppi = 256 / chunks, chunk = tid % chunks, p0 = tid / chunks;
+    if (p0 >= ppi) return;
+    int a[4], b[4];
+    uint32_t pick[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const int k = chunk * 16 + 4 * d, line = k / g.kw, kw = k - line * g.kw;        // line = ci * KH + kh
+        const int in_line = min(4, g.kw - kw);
+        auto at = [&](int l) { const int c = l / g.kh; return (c * prows + (l - c * g.kh) * g.dh) * wpatch; };
+        const int left = 4 - g.pad_left;
+        a[d] = left + (k < g.kk ? at(line) + kw : 0);
+        b[d] = in_line < 4 && k + in_line < g.kk ? left + at(line + 1) : a[d];
+        pick[d] = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) pick[d] |= (k + j >= g.kk ? 0x0cu : j < in_line ? uint32_t(j) : uint32_t(4 + j - in_line)) << (8 * j);
+    }
+    for (int ro = 0; ro < R && oh0 + ro < g.ho; ++ro) {
+        int8_t *dst = xs + (int64_t(ni) * g.ho + oh0 + ro) * g.wo * g.cp + chunk * 16;
+        for (int ow = p0; ow < g.wo; ow += ppi) {
+            const uint32_t *base = patch + ro * g.sh * wpatch + ow * g.sw;
+            uint32_t words[4];
+#pragma unroll
+            for (int d = 0; d < 4; ++d) words[d] = __builtin_amdgcn_perm(base[b[d]], base[a[d]], pick[d]);
+            *reinterpret_cast<uint4 *>(dst + int64_t(ow) * g.cp) = make_uint4(words[0], words[1], words[2], words[3]);
+        }
+    }
+}
+
 // Whole staged buffer = halo: T(padding_value) in the real channels, 0 in the channel padding.
 __global__ __launch_bounds__(256) void stage_fill_kernel(int8_t *__restrict__ xs, int64_t chunks, int cp, int c, int pad_value) {
     const int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1048,17 +1154,32 @@ int run_stage(const tsx_conv2d_geom *g, const Plan &pl, const void *x, bool x_is
         const size_t patch_bytes = size_t(g->c) * g->kh * wpatch;
         const bool by_rows = patch_bytes <= 48 * 1024 && int64_t(g->n) * pl.ho < (int64_t(1) << 31);
         const dim3 row_grid(unsigned(int64_t(g->n) * pl.ho));
+        // The form by words: as many rows per workgroup as leave most CUs a workgroup and fit 48 KiB.  (us for 1, 2, 4 rows: 32
+        // images 3x224x224, 7x9 at strides 2 and 4: 31.5, 20.2, 19.0; 4 images: 8.3, 7.2, 9.3; one: 6.3, 6.7, 8.8; 8 images
+        // 3x608x608, 3x4: 36.7, 29.5, 27.0.)
+        const int wwords = int(tsx::round_up(wpatch + 4 - std::min(g->pad_left, 4), 4));
+        auto words_bytes = [&](int R) { return size_t(g->c) * ((R - 1) * g->stride_h + (g->kh - 1) * g->dilation_h + 1) * wwords * 4; };
+        int R = 4;
+        while (R > 1 && (int64_t(g->n) * tsx::ceil_div(pl.ho, R) < 200 || words_bytes(R) > 48 * 1024)) R /= 2;
+        const bool by_words = by_rows && g->kw >= 3 && g->dilation_w == 1 && g->w % 4 == 0 && g->pad_left <= 4 && words_bytes(R) <= 64 * 1024;
+        const dim3 words_grid(unsigned(int64_t(g->n) * tsx::ceil_div(pl.ho, R)));
         if (x_is_f32) {
             TSX_REQUIRE(x_scales && n_x_scales >= 1, "quantize_conv2d_i8: missing quantize scales");
             TSX_REQUIRE(n_x_scales == g->n, "quantize_conv2d_i8: n_x_scales (%d) must equal the batch (%d)", n_x_scales, g->n);
             const int64_t count = int64_t(g->n) * g->c * g->h * g->w;
             const int64_t group_len = int64_t(std::ceil(static_cast<float>(count) / static_cast<float>(n_x_scales)));
-            if (by_rows)
+            if (by_words && (n_x_scales == 1 || group_len == int64_t(g->c) * g->h * g->w))
+                hipLaunchKernelGGL(stage_im2col_words_kernel<true>, words_grid, dim3(256), words_bytes(R), stream, x, ig, wwords, R, x_scales,
+                                   n_x_scales, (count >> 3) << 3, static_cast<int8_t *>(staged));
+            else if (by_rows)
                 hipLaunchKernelGGL(stage_im2col_rows_kernel<true>, row_grid, dim3(256), patch_bytes, stream, x, ig, wpatch, x_scales,
                                    n_x_scales, group_len, (count >> 3) << 3, static_cast<int8_t *>(staged));
             else
                 hipLaunchKernelGGL(stage_im2col_kernel<true>, grid, dim3(256), 0, stream, x, ig, x_scales, n_x_scales, group_len,
                                    (count >> 3) << 3, static_cast<int8_t *>(staged));
+        } else if (by_words) {
+            hipLaunchKernelGGL(stage_im2col_words_kernel<false>, words_grid, dim3(256), words_bytes(R), stream, x, ig, wwords, R,
+                               static_cast<const float *>(nullptr), 1, int64_t(0), static_cast<int8_t *>(staged));
         } else if (by_rows) {
             hipLaunchKernelGGL(stage_im2col_rows_kernel<false>, row_grid, dim3(256), patch_bytes, stream, x, ig, wpatch,
                                static_cast<const float *>(nullptr), 1, int64_t(1), int64_t(0), static_cast<int8_t *>(staged));
