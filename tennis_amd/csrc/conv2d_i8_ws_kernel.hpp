@@ -386,8 +386,12 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
             });
         }
         // One branch around the fragments, not one per fragment: inside it the compiler knows what is still in
-        // flight, and a fragment does not wait for the stores of the one before it.
-        if (fast_f) {
+        // flight, and a fragment does not wait for the stores of the one before it.  FULL: all 32 channels exist; otherwise
+        // only those that do are stored (without residual and staged output, whose partial form would cost every such kernel
+        // nineteen registers).
+        auto fragments = [&](auto fullc) __attribute__((always_inline)) {
+            constexpr bool FULL = decltype(fullc)::value;
+            const int left = p.cout - co_lane;                         // channels from the lane's first one on
             // the other branch of a residual join: the loads of every fragment are in flight before the first use
             float res[NT][16];
             if (EXTRA && p.residual) {
@@ -474,7 +478,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
                             constexpr int g4 = decltype(gc)::value;
                             typedef float v4f __attribute__((ext_vector_type(4)));
                             const v4f q4 = {v[4 * g4], v[4 * g4 + 1], v[4 * g4 + 2], v[4 * g4 + 3]};
-                            *reinterpret_cast<v4f *>(o + 8 * g4) = q4;
+                            if (FULL || 8 * g4 < left) *reinterpret_cast<v4f *>(o + 8 * g4) = q4;      // (whole: cout is a multiple of 4)
                         });
                     } else if (p.out_f32) static_for<0, 16>([&](auto rc) {
                         constexpr int r = decltype(rc)::value;
@@ -482,6 +486,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
                         // streaming store for large plain outputs: lines that never become dirty in L2 need no
                         // write-back burst when the kernel ends; outputs a following kernel reads stay cached
                         float *o = &(p.out_f32 + tile_base + int64_t(dco) * howo)[lane_off];
+                        if (!FULL && dco >= left) return;
                         if (STREAM) __builtin_nontemporal_store(v[r], o);
                         else *o = v[r];
                     });
@@ -501,7 +506,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
                         if (p.out_i8) static_for<0, 16>([&](auto rc) {
                             constexpr int r = decltype(rc)::value;
                             constexpr int dco = 8 * (r / 4) + (r % 4);
-                            (p.out_i8 + tile_base + int64_t(dco) * howo)[lane_off] = int8_t(word[r / 4] >> (8 * (r % 4)));
+                            if (FULL || dco < left) (p.out_i8 + tile_base + int64_t(dco) * howo)[lane_off] = int8_t(word[r / 4] >> (8 * (r % 4)));
                         });
                         if (EXTRA && p.st_out) {
                             // consumer's staged layout [pixel][channel].  Accumulator registers 4g..4g+3 of a lane are 4
@@ -530,6 +535,11 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
                     }
                 }
             });
+        };
+        if (fast_f) {
+            fragments(std::true_type{});
+        } else if (fast && !EXTRA && !MISHX) {
+            if constexpr (!EXTRA && !MISHX) fragments(std::false_type{});
         } else {
             static_for<0, NT>([&](auto jc) {
                 constexpr int j = decltype(jc)::value;
