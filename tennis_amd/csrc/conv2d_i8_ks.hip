@@ -273,8 +273,12 @@ void ks_plan(const WsGeom &g, WsPlan *pl) {
     // than their chain of K-steps.  (One image, us, those kernels -> this one: 3x3 512 to 512 channels 7x7 10.9 -> 5.4, 256
     // to 256 14x14 7.2 -> 4.1, 1x1 1024 to 256 14x14 6.1 -> 3.6, 3x3 100 to 150 13x13 at stride 2 17.8 -> 3.6; 8 images, 3x3
     // 256 to 256 14x14: 7.5, here 8.4.)
+    // 1x1 layers with a stride stand against the generic kernel's 128 x 128 tiles, whose epilogue goes element by element where
+    // a fragment's 32 channels do not all exist.  (25 images 380 channels 26x130 to 55 at stride 2 with LeakyReLU: 41.4 -> 7.1 us; 4 images 100 100x100 to 90: 15.3 -> 4.3.)
     const int ksteps = g.cblocks * g.kh * g.kw;
     double best = 4.4 + 0.09 * ksteps;
+    if (g.kh == 1 && g.kw == 1 && (g.sh > 1 || g.sw > 1))
+        best = 5.5 + 0.32 * ksteps + (g.cout % 32 ? 12. * double(ceil_div(ceil_div(positions, 128) * ceil_div(g.cout, 128), 512)) : 0.);
     for (int i = 0; i < TILE_COUNT; ++i) {
         const int64_t tiles = ceil_div(positions, TILES[i].columns) * ceil_div(g.cout, TILES[i].rows);
         if (tiles >= (int64_t(1) << 23)) continue;                         // a launch holds fewer than 2^32 work items
