@@ -1476,9 +1476,12 @@ int tsx_conv2d_i8_staged_at(const tsx_conv2d_geom *g, const void *staged_dev, in
     TSX_REQUIRE(staged_hs >= pl.hs && staged_ws >= pl.ws, "staged_at: buffer rows/columns %dx%d smaller than the %dx%d read",
                 staged_hs, staged_ws, pl.hs, pl.ws);
     // same kernels, with the buffer's own pitches; the window-stationary plan is re-derived for them
+    const bool wider = staged_hs != pl.hs || staged_ws != pl.ws;
     pl.hs = staged_hs;
     pl.ws = staged_ws;
-    if (pl.use_ws) {
+    if (!wider) {
+        // the plan is this buffer's
+    } else if (pl.use_ws) {
         pl.wsg.hs = staged_hs;
         pl.wsg.ws = staged_ws;
         const tsx::WsPlan wide = tsx::ws_plan(pl.wsg);
