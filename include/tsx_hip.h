@@ -218,10 +218,13 @@ int tsx_conv2d_f32_nchw_ws(const tsx_conv2d_geom *g, const float *x_dev, const f
                            const float *bias_dev, int32_t act, float slope, float *out_dev, void *workspace_dev,
                            size_t workspace_bytes, void *stream);
 /* Which kernel tsx_conv2d_f32_nchw launches for this layer and these weights (their alignment counts), as text:
- * "kernel=small_3x3 | register_fed | staged_64x64 | staged_32x32_ksplit tiles=<output tiles>".  No counterpart in
- * the reference; for tests that must know a given kernel ran, and for logs.  The environment variables
- * TSX_CONV_F32_SMALL and TSX_GEMM_F32_REGFED ("0" = never, "force" = wherever the operands allow) are read at every
- * call. */
+ * "kernel=small_3x3 | register_fed | staged_64x64 | staged_32x32_ksplit tiles=<output tiles>", and where
+ * tsx_conv2d_f32_nchw_ws with its workspace launches another one, that: "workspace_kernel=bf16_split
+ * workspace_tile=<output channels>x<positions> workspace_patch=<cells> workspace_window=flat | segments".  No counterpart
+ * in the reference; for tests that must know a given kernel ran, and for logs.  The environment variables
+ * TSX_CONV_F32_SMALL and TSX_GEMM_F32_REGFED ("0" = never, "force" = wherever the operands allow) and TSX_CONV_F32_SPLIT
+ * ("0" = the workspace is not used, a number = that tile and patch form of the kernel on the bf16 matrix cores wherever it
+ * suits the layer) are read at every call. */
 int tsx_conv2d_f32_plan_info(const tsx_conv2d_geom *g, const float *w_oihw_dev, char *text, size_t text_bytes);
 
 /* cpu::InnerProd::inner_prod (src/kernels/cpu/inner_prod.cpp:54-69, interface

@@ -599,7 +599,8 @@ def _conv_f32_workspace(geom, x, w):
 
 
 def conv2d_f32_plan_info(x_shape, w, pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1)):
-    """tsx_conv2d_f32_plan_info as a dict ({"kernel": ..., "tiles": ...}) for an input of x_shape and weights w."""
+    """tsx_conv2d_f32_plan_info as a dict for an input of x_shape and weights w: "workspace_kernel" is the kernel that
+    conv2d_f32 runs, which hands over a workspace; where there is none, "kernel"."""
     w = _dev(w, torch.float32)
     geom = make_geom(tuple(x_shape), tuple(w.shape), pads, strides, dilations)
     text = ctypes.create_string_buffer(256)

@@ -490,6 +490,12 @@ ConvF32Split conv_f32_split_choose(const ConvF32Layer &l) {
     return best;
 }
 
+void conv_f32_split_tile_size(int tile, int *rows, int *positions, int *patch) {
+    *rows = SPLIT_TILES[tile / 2].bm();
+    *positions = SPLIT_TILES[tile / 2].bn();
+    *patch = SPLIT_TILES[tile / 2].pitch;
+}
+
 int conv_f32_split(const ConvF32Layer &l, int tile, const float *bias, int act, float slope, float padding_value, float *out, void *workspace,
                    hipStream_t stream) {
     SplitParams p{};

@@ -10,6 +10,7 @@ struct ConvF32Split {
     double us;                // expected; 0: the tile is forced
 };
 ConvF32Split conv_f32_split_choose(const ConvF32Layer &l);
+void conv_f32_split_tile_size(int tile, int *rows, int *positions, int *patch);      // patch: cells it is built for
 int conv_f32_split(const ConvF32Layer &l, int tile, const float *bias, int act, float slope, float padding_value, float *out, void *workspace,
                    hipStream_t stream);
 

@@ -820,23 +820,32 @@ int tsx_conv2d_f32_plan_info(const tsx_conv2d_geom *geo, const float *w_oihw_dev
     tsx::ConvLoader ld;
     const int rc = conv_f32_problem(geo, nullptr, w_oihw_dev, 0.f, nullptr, TSX_ACT_NONE, 0.f, nullptr, g, ld);
     if (rc) return rc;
-    const char *name = "small_3x3";
-    int tile = 32;
-    if (!tsx::conv3x3_small_takes(g, ld)) {
-        const tsx::GemmKernel k = tsx::choose_gemm(g, 1);
-        name = k == tsx::GEMM_REGISTER_FED ? "register_fed" : k == tsx::GEMM_STAGED_64 ? "staged_64x64" : "staged_32x32_ksplit";
-        if (k == tsx::GEMM_STAGED_64) tile = 64;
-        const int win = tsx::window_tile(tsx::window_layer(geo, g, ld), g);
-        if (win >= 0) {        // a K-split 32-row tile or a larger one without, by its input patches
-            int rows, positions;
-            tsx::conv_f32_window_tile_size(win, &rows, &positions);
-            std::snprintf(text, text_bytes, "kernel=%s tiles=%lld tile=%dx%d window=%s", rows * positions == 1024 ? "staged_32x32_ksplit" : "staged_64x64",
-                          (long long)(tsx::ceil_div(g.m, rows) * tsx::ceil_div(g.n, positions)), rows, positions, win % 2 ? "flat" : "segments");
-            return 0;
-        }
+    if (tsx::conv3x3_small_takes(g, ld)) {
+        std::snprintf(text, text_bytes, "kernel=small_3x3 tiles=%lld", (long long)(tsx::ceil_div(g.m, 32) * tsx::ceil_div(g.n, 32)));
+        return 0;
     }
-    std::snprintf(text, text_bytes, "kernel=%s tiles=%lld", name,
-                  (long long)(tsx::ceil_div(g.m, tile) * tsx::ceil_div(g.n, tile)));
+    const tsx::ConvF32Layer layer = tsx::window_layer(geo, g, ld);
+    char with_workspace[128] = "";
+    const tsx::ConvF32Split split = tsx::split_choice(layer, g);
+    if (split.tile >= 0) {
+        int rows, positions, patch;
+        tsx::conv_f32_split_tile_size(split.tile, &rows, &positions, &patch);
+        std::snprintf(with_workspace, sizeof(with_workspace), " workspace_kernel=bf16_split workspace_tile=%dx%d workspace_patch=%d workspace_window=%s",
+                      rows, positions, patch, split.tile % 2 ? "flat" : "segments");
+    }
+    const int win = tsx::window_tile(layer, g);
+    if (win >= 0) {            // a K-split 32-row tile or a larger one without, by its input patches
+        int rows, positions;
+        tsx::conv_f32_window_tile_size(win, &rows, &positions);
+        std::snprintf(text, text_bytes, "kernel=%s tiles=%lld tile=%dx%d window=%s%s", rows * positions == 1024 ? "staged_32x32_ksplit" : "staged_64x64",
+                      (long long)(tsx::ceil_div(g.m, rows) * tsx::ceil_div(g.n, positions)), rows, positions, win % 2 ? "flat" : "segments",
+                      with_workspace);
+        return 0;
+    }
+    const tsx::GemmKernel k = tsx::choose_gemm(g, 1);
+    const int tile = k == tsx::GEMM_STAGED_64 ? 64 : 32;
+    std::snprintf(text, text_bytes, "kernel=%s tiles=%lld%s", k == tsx::GEMM_REGISTER_FED ? "register_fed" : tile == 64 ? "staged_64x64" : "staged_32x32_ksplit",
+                  (long long)(tsx::ceil_div(g.m, tile) * tsx::ceil_div(g.n, tile)), with_workspace);
     return 0;
 }
 

@@ -78,6 +78,32 @@ def test_kernel_choices_need_no_device(monkeypatch):
     assert L.tsx_conv2d_f32_plan_info(ctypes.byref(c1), None, None, 0) == -1
 
 
+def test_fp32_plan_info_names_the_kernel_of_a_call_with_workspace(monkeypatch):
+    """A layer has use for a workspace exactly where the plan names a kernel of its own for that call."""
+    from tennis_amd import capi
+    L = capi.lib()
+    for name in ("TSX_CONV_F32_SMALL", "TSX_GEMM_F32_REGFED", "TSX_CONV_F32_SPLIT"):
+        monkeypatch.delenv(name, raising=False)
+
+    def plan(geom):
+        buf = ctypes.create_string_buffer(256)
+        assert L.tsx_conv2d_f32_plan_info(ctypes.byref(geom), ctypes.c_void_p(4096), buf, len(buf)) == 0
+        info = dict(word.split("=", 1) for word in buf.value.decode().split())
+        assert ("workspace_kernel" in info) == (L.tsx_conv2d_f32_workspace_bytes(ctypes.byref(geom), ctypes.c_void_p(4096)) > 0)
+        return info
+
+    large = capi.ConvGeom(8, 256, 28, 28, 256, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1)
+    info = plan(large)
+    assert info["workspace_kernel"] == "bf16_split" and info["kernel"] == "staged_64x64"
+    rows, positions = map(int, info["workspace_tile"].split("x"))
+    assert rows % 32 == 0 and positions % 32 == 0 and info["workspace_window"] in ("flat", "segments")
+    monkeypatch.setenv("TSX_CONV_F32_SPLIT", "0")
+    assert "workspace_kernel" not in plan(large)
+    monkeypatch.delenv("TSX_CONV_F32_SPLIT")
+    assert "workspace_kernel" not in plan(capi.ConvGeom(1, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1))
+    assert "workspace_kernel" not in plan(capi.ConvGeom(1, 128, 28, 28, 128, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1))
+
+
 def test_hot_path_operators_are_registered_for_hip():
     from tennis_amd import operators as ops
     for name in ops.SYMBOLS:
