@@ -117,33 +117,32 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// A workgroup of WM x WN x WK wavefronts (8, or two workgroups of 4 per CU) owns 32 WM output channels x 64 WN positions; a wavefront's 32 x 64 take 12
-// MFMAs (384 cycles) per 16 channels and tap for 3 KiB of weights, from L2 straight into registers AHEAD steps early, and
-// 6 KiB of activations from LDS.  As in the fp32 form (conv2d_f32_window.hip) a chunk of CC channels of the input patch
-// -- the rows and columns the tile's positions read through all taps, padding included -- goes to LDS once per element,
-// here in three parts, [part][8 channels][PITCH cells][8], and every tap is a shifted read; a thread converts eight
-// channels of a cell at a time while the other wavefront of its SIMD multiplies.  With WK > 1 the wavefronts split a
-// chunk's channels and add their sums through LDS in a fixed order.  TAPS: 9 (3x3), 25 (5x5), 1 (the patch is the tile's
-// positions themselves, at any stride).
+// A workgroup of WM x WN wavefronts (8, or two workgroups of 4 per CU) owns 32 WM output channels x 64 WN positions; a
+// wavefront's 32 x 64 take 12 MFMAs (384 cycles) per 16 channels and tap for 3 KiB of weights, from L2 straight into
+// registers AHEAD steps early, and 6 KiB of activations from LDS.  As in the fp32 form (conv2d_f32_window.hip) a chunk of CC
+// channels of the input patch -- the rows and columns the tile's positions read through all taps, padding included -- goes
+// to LDS once per element, here in three parts, [part][8 channels][PITCH cells][8], and every tap is a shifted read; a
+// thread converts eight channels of a cell at a time while the other wavefront of its SIMD multiplies.  TAPS: 9 (3x3), 25
+// (5x5), 1 (the patch is the tile's positions themselves, at any stride).
 // What bounds it: the MFMAs, which at the clock the bf16 matrix cores leave (1.5 GHz and less) take two thirds of the time
 // (8 images of 28x28x256 with 256 3x3 filters: 36 of 52 us with everything but them left out), then the conversions, operand
 // reads and weights beside them.  Against the fp32 MFMAs (us, weights' split included): that layer 86 -> 52, 128 channels at
 // 56x56 86 -> 48, 256 to 256 channels 1x1 at 56x56, 32 images, 129 -> 94, 100 to 150 channels 5x5 at 33x41, 4 images, 128 -> 59.
-template <int WM, int WN, int WK, int TAPS, int PITCH, int CC>
-__global__ __launch_bounds__(64 * WM * WN * WK, 2) void conv_f32_split_kernel(SplitParams p) {
-    constexpr int THREADS = 64 * WM * WN * WK;
+template <int WM, int WN, int TAPS, int PITCH, int CC>
+__global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitParams p) {
+    constexpr int THREADS = 64 * WM * WN;
     constexpr int BM = 32 * WM, BN = 64 * WN, KW = TAPS == 9 ? 3 : TAPS == 25 ? 5 : 1;
-    constexpr int SUBS = CC / 16 / WK, STEPS = SUBS * TAPS;
+    constexpr int SUBS = CC / 16, STEPS = SUBS * TAPS;
     constexpr int AHEAD = STEPS <= 4 ? STEPS : 3;
     constexpr int PART = CC / 8 * PITCH * 16, BUFFER = 3 * PART;           // bytes
     constexpr int SLOTS = CC / 8 * PITCH / THREADS;
-    static_assert(SUBS >= 1 && CC % (16 * WK) == 0 && CC / 8 * PITCH % THREADS == 0 && (TAPS != 1 || PITCH == BN) &&
-                      2 * PART + ((SUBS - 1) * 2 * WK * PITCH + KW) * 16 < 65536 && SLOTS <= STEPS,
+    static_assert(SUBS >= 1 && CC % 16 == 0 && CC / 8 * PITCH % THREADS == 0 && (TAPS != 1 || PITCH == BN) &&
+                      2 * PART + ((SUBS - 1) * 2 * PITCH + KW) * 16 < 65536 && SLOTS <= STEPS,
                   "whole slots, one a step; every operand read within an instruction's offset");
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int hf = lane / 32;
-    const int wk = wave % WK, wn = (wave / WK) % WN, wm = wave / (WK * WN);
+    const int wn = wave % WN, wm = wave / WN;
 
     // Tiles that share their positions are consecutive, and each XCD takes a contiguous run of tiles: a patch is fetched
     // into one L2.
@@ -240,14 +239,14 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void conv_f32_split_kernel(Sp
         *reinterpret_cast<v4u *>(to + 2 * PART) = s.l;
     };
 
-    // ---- operands.  Step (sub, tap) of a chunk takes channels 16 (wk + WK sub) ... of it.
+    // ---- operands.  Step (sub, tap) of a chunk takes channels 16 sub ... of it.
     const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.w), 0, int(p.w_bytes), 0x00020000);
     const int w_off = min(m0 / 32 + wm, p.mfrags - 1) * 3072 + lane * 16, w_step = p.mfrags * 3072;
     struct A { v4u part[3]; } a[AHEAD];
     struct B { v4u part[2][3]; } b;
     auto load_weights = [&](auto sc, int chunk) __attribute__((always_inline)) {      // step sc of the chunk, its steps beyond STEPS in the next
         constexpr int s = decltype(sc)::value % STEPS, over = decltype(sc)::value / STEPS, sub = s / TAPS, tap = s % TAPS;
-        const int q = ((min(chunk + over, p.chunks - 1) * (CC / 16) + wk + WK * sub) * TAPS + tap) * w_step;
+        const int q = ((min(chunk + over, p.chunks - 1) * (CC / 16) + sub) * TAPS + tap) * w_step;
         static_for<0, 3>([&](auto pc) {
             constexpr int part = decltype(pc)::value;
             a[s % AHEAD].part[part] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(wr, w_off + part * 1024, q, 0));
@@ -261,14 +260,14 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void conv_f32_split_kernel(Sp
         int row, col;
         const bool ok = decode(q, row, col);
         const int cell = TAPS == 1 ? q : ok ? (virtual_row(row) - vr0) * p.wv + (col - col0) * p.sw : 0;
-        b_at[j] = ((hf + 2 * wk) * PITCH + cell) * 16;
+        b_at[j] = (hf * PITCH + cell) * 16;
     });
     auto read = [&](auto sc, int at) __attribute__((always_inline)) {
         constexpr int s = decltype(sc)::value, sub = s / TAPS, tap = s % TAPS;
         B v;
         static_for<0, 6>([&](auto ec) {
             constexpr int j = decltype(ec)::value / 3, part = decltype(ec)::value % 3;
-            v.part[j][part] = *reinterpret_cast<const v4u *>(lds + (b_at[j] + (at + tap / KW * row_bytes)) + part * PART + (2 * WK * sub * PITCH + tap % KW) * 16);
+            v.part[j][part] = *reinterpret_cast<const v4u *>(lds + (b_at[j] + (at + tap / KW * row_bytes)) + part * PART + (2 * sub * PITCH + tap % KW) * 16);
         });
         return v;
     };
@@ -349,28 +348,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void conv_f32_split_kernel(Sp
     float bias[16];
     static_for<0, 16>([&](auto rc) {
         constexpr int r = decltype(rc)::value;
-        bias[r] = p.bias && wk == 0 ? p.bias[min(m0 + wm * 32 + 8 * (r / 4) + 4 * hf + r % 4, p.M - 1)] : 0.f;
+        bias[r] = p.bias ? p.bias[min(m0 + wm * 32 + 8 * (r / 4) + 4 * hf + r % 4, p.M - 1)] : 0.f;
     });
     sum[0] += small[0];
     sum[1] += small[1];
-    if constexpr (WK > 1) {
-        constexpr int SLOT = WM * WN * 32 * 64;
-        float *red = reinterpret_cast<float *>(lds) + (wm * WN + wn) * 32 * 64 + lane;      // the chunks' space takes the partial tiles
-        __syncthreads();                       // the reads ahead have returned
-        if (wk > 0)
-            static_for<0, 32>([&](auto rc) {
-                constexpr int r = decltype(rc)::value;
-                red[(wk - 1) * SLOT + r * 64] = sum[r / 16][r % 16];
-            });
-        __syncthreads();
-        if (wk > 0) return;
-        static_for<0, WK - 1>([&](auto sc) {
-            static_for<0, 32>([&](auto rc) {
-                constexpr int r = decltype(rc)::value;
-                sum[r / 16][r % 16] += red[decltype(sc)::value * SLOT + r * 64];
-            });
-        });
-    }
     // A lane's element of a row is its own offset plus a uniform one; 32-bit offsets, the output is below 2 GiB.
     const auto out = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, int(int64_t(p.M) * p.N * 4), 0x00020000);
     const bool body = p.act_body == int64_t(p.M) * p.N;      // no element behind the activation's SIMD body
@@ -395,16 +376,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void conv_f32_split_kernel(Sp
 
 // ---- tiles.  Each with the patch pitches it is built for, smallest first.
 struct SplitTile {
-    int wm, wn, wk, taps, pitch, cc;
+    int wm, wn, taps, pitch, cc;
     int (*launch)(const SplitParams &, hipStream_t);
     int bm() const { return 32 * wm; }
     int bn() const { return 64 * wn; }
 };
 
-template <int WM, int WN, int WK, int TAPS, int PITCH, int CC>
+template <int WM, int WN, int TAPS, int PITCH, int CC>
 int launch_split(const SplitParams &p, hipStream_t stream) {
-    auto kernel = conv_f32_split_kernel<WM, WN, WK, TAPS, PITCH, CC>;
-    constexpr size_t lds_bytes = std::max(2 * 3 * CC / 8 * PITCH * 16, (WK - 1) * WM * WN * 32 * 64 * 4);
+    auto kernel = conv_f32_split_kernel<WM, WN, TAPS, PITCH, CC>;
+    constexpr size_t lds_bytes = 2 * 3 * CC / 8 * PITCH * 16;
     static_assert(lds_bytes <= 159 * 1024, "LDS of a compute unit");
     if (lds_bytes > 65536) {                   // dynamic LDS beyond 64 KiB is granted per kernel and device
         static std::atomic<bool> granted[64];
@@ -416,18 +397,18 @@ int launch_split(const SplitParams &p, hipStream_t stream) {
         }
     }
     const int total = p.tiles_m * p.tiles_n;
-    hipLaunchKernelGGL(kernel, dim3(unsigned((total + 7) / 8 * 8)), dim3(64 * WM * WN * WK), lds_bytes, stream, p);
+    hipLaunchKernelGGL(kernel, dim3(unsigned((total + 7) / 8 * 8)), dim3(64 * WM * WN), lds_bytes, stream, p);
     TSX_LAUNCH_CHECK("conv_f32_split_kernel");
     return 0;
 }
 
-template <int WM, int WN, int WK, int TAPS, int PITCH, int CC>
-constexpr SplitTile split_tile() { return {WM, WN, WK, TAPS, PITCH, CC, launch_split<WM, WN, WK, TAPS, PITCH, CC>}; }
+template <int WM, int WN, int TAPS, int PITCH, int CC>
+constexpr SplitTile split_tile() { return {WM, WN, TAPS, PITCH, CC, launch_split<WM, WN, TAPS, PITCH, CC>}; }
 
 const SplitTile SPLIT_TILES[] = {
-    split_tile<2, 2, 1, 9, 256, 16>(), split_tile<2, 2, 1, 9, 384, 16>(), split_tile<4, 1, 1, 9, 256, 16>(), split_tile<4, 1, 1, 9, 384, 16>(),
-    split_tile<4, 2, 1, 9, 512, 16>(), split_tile<2, 2, 1, 25, 256, 16>(), split_tile<2, 2, 1, 25, 384, 16>(), split_tile<4, 1, 1, 25, 256, 16>(),
-    split_tile<4, 1, 1, 25, 384, 16>(), split_tile<2, 2, 2, 25, 384, 32>(), split_tile<4, 1, 1, 1, 64, 64>(), split_tile<2, 2, 1, 1, 128, 32>(),
+    split_tile<2, 2, 9, 256, 16>(), split_tile<2, 2, 9, 384, 16>(), split_tile<4, 1, 9, 256, 16>(), split_tile<4, 1, 9, 384, 16>(), split_tile<4, 2, 9, 512, 16>(),
+    split_tile<2, 2, 25, 384, 16>(), split_tile<4, 1, 25, 256, 16>(), split_tile<4, 1, 25, 384, 16>(),
+    split_tile<4, 1, 1, 64, 64>(), split_tile<2, 2, 1, 128, 32>(),
 };
 constexpr int SPLIT_TILE_COUNT = int(sizeof(SPLIT_TILES) / sizeof(SPLIT_TILES[0]));
 
@@ -482,8 +463,8 @@ ConvF32Split conv_f32_split_choose(const ConvF32Layer &l) {
             const SplitTile &t = SPLIT_TILES[i];
             // Time of the busiest CU in us, fitted to 45 layers of 0.01 to 17 GFLOP: 12 MFMAs per step at the 1.28 GHz that the
             // bf16 matrix cores come to beside everything else, 2 for a tile's start and end, 7 for the launches and the weights.
-            const double tiles = double(ceil_div(int64_t(p.tiles_m) * p.tiles_n, 256)), waves = t.wm * t.wn * t.wk / 4;
-            const double us = tiles * (waves * p.chunks * (t.cc / 16 / t.wk) * t.taps * 384 / 1280. + 2) + 7;
+            const double tiles = double(ceil_div(int64_t(p.tiles_m) * p.tiles_n, 256)), waves = t.wm * t.wn / 4;
+            const double us = tiles * (waves * p.chunks * (t.cc / 16) * t.taps * 384 / 1280. + 2) + 7;
             if (best.tile < 0 || us < best.us) best = {i * 2 + flat, p.w_bytes, us};
         }
     if (only >= 0) best.us = 0;

@@ -104,6 +104,41 @@ def test_fp32_plan_info_names_the_kernel_of_a_call_with_workspace(monkeypatch):
     assert "workspace_kernel" not in plan(capi.ConvGeom(1, 128, 28, 28, 128, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1))
 
 
+def test_every_tile_of_the_bf16_split_kernel_is_reached(monkeypatch):
+    """Each tile that TSX_CONV_F32_SPLIT can name takes some layer, is no twin of another one, and is what the planner
+    chooses for some layer by itself."""
+    import random
+    from tennis_amd import capi
+    L = capi.lib()
+    for name in ("TSX_CONV_F32_SMALL", "TSX_GEMM_F32_REGFED", "TSX_CONV_F32_SPLIT"):
+        monkeypatch.delenv(name, raising=False)
+    rng = random.Random(1)
+    between = lambda lo, hi: int(round(lo * (hi / lo) ** rng.random()))
+    layers = []
+    for _ in range(12000):
+        k = rng.choice([1, 3, 5])
+        pad, stride = rng.choice([0, k // 2, k // 2]), rng.choice([1, 1, 2])
+        layers.append(capi.ConvGeom(between(1, 32), between(3, 1024), between(5, 304), between(5, 304), between(16, 1024), k, k, pad, pad, pad, pad,
+                                    stride, stride, 1, 1))
+
+    def tile(geom):
+        buf = ctypes.create_string_buffer(256)
+        assert L.tsx_conv2d_f32_plan_info(ctypes.byref(geom), ctypes.c_void_p(4096), buf, len(buf)) == 0
+        info = dict(word.split("=", 1) for word in buf.value.decode().split())
+        return (geom.kh, info["workspace_tile"], info["workspace_patch"]) if "workspace_kernel" in info else None
+
+    chosen = {tile(geom) for geom in layers} - {None}
+    named = {}
+    for number in range(1, 65):
+        monkeypatch.setenv("TSX_CONV_F32_SPLIT", str(number))
+        found = next((t for t in map(tile, layers[:3000]) if t is not None), None)
+        if found is not None:
+            named.setdefault((number - 1) // 2, set()).add(found)
+    assert sorted(named) == list(range(len(named))), "tiles that take no layer"
+    names = [t for tiles in named.values() for t in tiles]
+    assert len(names) == len(set(names)) == len(named) and set(names) == chosen, set(names) ^ chosen
+
+
 def test_hot_path_operators_are_registered_for_hip():
     from tennis_amd import operators as ops
     for name in ops.SYMBOLS:

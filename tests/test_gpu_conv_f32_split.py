@@ -23,7 +23,7 @@ LAYERS = [
     (3, 5, 12, 13, 31, 1, (1, 0, 0, 1), (2, 2), 1),
     (1, 131, 4, 4, 300, 1, (0, 0, 0, 0), (1, 1), 1),
 ]
-TILES = range(24)
+TILES = range(20)                # ten tiles, each with column segments and with flat positions
 
 
 def dev(a):
@@ -74,8 +74,8 @@ def test_conv_f32_split_tiles(port, monkeypatch, padding_value):
             ok = ~nan & ~(huge & np.isfinite(exp))
             assert np.array_equal(bits(got[ok]), bits(exp[ok])), (case, tile)
             runs[tile] += 1
-    # a pointwise patch is the tile's positions: one form; the smaller patches hold no segments
-    assert sum(r > 0 for r in runs) >= 18, runs
+    # a pointwise patch is the tile's positions: flat only
+    assert all(r > 0 for t, r in enumerate(runs) if t not in (16, 18)), runs
 
 
 @pytest.mark.parametrize("case", [(2, 48, 20, 20, 64, 3), (1, 256, 28, 28, 128, 3), (2, 64, 24, 24, 32, 5), (4, 512, 14, 14, 128, 1)])
