@@ -204,14 +204,16 @@ int tsx_gemm_i8(int32_t m, int32_t n, int32_t k, const int8_t *a_dev, const void
 /* ---------------------------------------------------------------- fp32 conv2d / inner_prod
  * cpu::Conv2DCore::conv2d (src/kernels/cpu/conv2d_core.cpp:101-119, interface
  * include/backend/base/base_conv2d_core.h:14-32): im2col + GEMM, here one implicit-GEMM kernel on
- * the fp32 MFMA reading NCHW directly (weights are used as they are: no packing, no workspace).
+ * the fp32 MFMA reading NCHW directly (weights are used as they are: no packing).
  * bias_dev (optional, [cout]) and act fuse the add_bias / relu operators that follow the conv in
  * config 1; pass NULL / TSX_ACT_NONE for the bare operator.  Parity bar for this
  * floating-point path: 1e-4 relative / 1e-5 absolute against the reference CPU kernels. */
 int tsx_conv2d_f32_nchw(const tsx_conv2d_geom *g, const float *x_dev, const float *w_oihw_dev, float padding_value,
                         const float *bias_dev, int32_t act, float slope, float *out_dev, void *stream);
 /* The same with a workspace of tsx_conv2d_f32_workspace_bytes() (0: the layer has no use for one): there large layers run
- * on the bf16 matrix cores, every float as the exact sum of three bf16 numbers, with smaller errors than the fp32 MFMA's.
+ * on the bf16 matrix cores, every float as the exact sum of three bf16 numbers.  Any floats: denormals count
+ * in full, and what meets numbers of 2^89 and more, infinities, NaN or sums above 2^50 is computed by the fp32 MFMA after all.
+ * A sum is off by less than the fp32 MFMA's chain of roundings leaves, a single product by at most 2^-24 + 2^-29 of it.
  * The workspace is 16-byte aligned device memory; its contents are written and read by each call. */
 size_t tsx_conv2d_f32_workspace_bytes(const tsx_conv2d_geom *g, const float *w_oihw_dev);
 int tsx_conv2d_f32_nchw_ws(const tsx_conv2d_geom *g, const float *x_dev, const float *w_oihw_dev, float padding_value,

@@ -3,18 +3,21 @@
 //
 // v_mfma_f32_32x32x2_f32 gives 64 operations per cycle and SIMD, v_mfma_f32_32x32x16_bf16 1024.  A float of 24
 // significant bits is the sum of three bf16 numbers of 8, exactly: x = h + m + l, h the upper half of its bits, m the
-// remainder rounded, l what is left of that.  Of the nine products of two such sums six are formed,
-//     x w = h h' + (h m' + m h') + (m m' + h l' + l h'),
-// the other three lie below 2^-23 of the product, with either sign; each product of two bf16 is exact in the MFMA's
-// fp32 accumulator.  h h' goes to an accumulator of its own, the five small products to a second one, added once at the
-// end: a sum of K terms takes K / 16 roundings where the fp32 MFMA takes K, and the small terms are not lost beside the
-// large ones.  Measured against 64 bits (normally distributed operands, 2-norm): 4.5e-8 at K = 32, 9.1e-8 at 256,
-// 2.9e-7 at 2304; the fp32 MFMA's chain has 1.0e-7, 2.9e-7, 8.6e-7.  Numbers below 2^-110 lose bits to the bf16
-// denormals (steps of 2^-133).
+// remainder rounded, l what is left of that (m <= 2^-7, l <= 2^-16 of the power of two at or below x).  Of the nine
+// products of two such sums eight are formed,
+//     x w = h h' + (h m' + m h') + (m m' + h l' + l h') + (m l' + l m'),
+// the ninth is below 2^-32 of the product (without m l' and l m', 2^-22, an output that is one product is rounded worse
+// than the fp32 MFMA rounds it); each product of two bf16 is exact in the MFMA's fp32 accumulator.  h h' goes to an
+// accumulator of its own, the seven small products to a second one, added once at the end: a sum of K terms takes K / 16
+// roundings where the fp32 MFMA takes K, and the small terms are not lost beside the large ones.  Measured
+// against 64 bits (2-norm; normally distributed and positive operands): 3.9e-8 and 4.0e-8 at K = 32, 6.5e-8 and 5.5e-8 at
+// 256, 1.0e-7 and 6.9e-8 at 2304, where the fp32 MFMA kernels have 1.0e-7 and 8.6e-8, 2.9e-7 and 2.5e-7, 4.2e-7 and
+// 1.8e-7; on 64 layers that come here by the planner's choice, K from 99 to 7475, 1.2 to 9.2 times less than theirs.
 //
-// NaN and infinities: such a value goes into l, with h = +-1 and m = 0.  l meets h' only, so an infinity times w has the
-// sign of w, and NaN where w is 0; what h = +-1 adds to the sum is finite.  Infinity times infinity is l h' = infinity
-// too.
+// Both operands are split times 2^39, and the result is scaled back: l is a multiple of 2^-23 of x, bf16 ends at 2^-133, and
+// times 2^39 the smallest denormal is 2^-110.  So the parts are exact for every number below 2^89, and no part of a product
+// that counts is lost.  A tile that meets larger numbers, infinities or NaN, or a sum of 2^50 on its way, is computed again by
+// the fp32 MFMA (exact() below): all of them leave an infinity or NaN in the sums they go into.
 #include "conv2d_f32_split.hpp"
 
 #include <algorithm>
@@ -34,20 +37,14 @@ struct Parts {
     v4u h, m, l;
 };
 
-// The three parts of eight floats, element by element in the order of the MFMA operand.  `odd` stays finite unless a value
-// is infinite or NaN (or some 10^23): those need SPECIAL.
-template <bool SPECIAL>
-__device__ __forceinline__ Parts split8(float (&x)[8], float &odd) {
+constexpr float UP = 0x1p39f, DOWN = 0x1p-78f;        // of an operand, of a product
+
+// The three parts of eight floats, times UP, element by element in the order of the MFMA operand; m is NaN where that is
+// infinite or NaN.
+__device__ __forceinline__ Parts split8(const float (&number)[8]) {
     Parts p;
-    unsigned special[4] = {0, 0, 0, 0};
-    if constexpr (SPECIAL)
-        static_for<0, 8>([&](auto jc) {
-            constexpr int j = decltype(jc)::value;
-            const bool finite = __builtin_fabsf(x[j]) < __builtin_inff();
-            const unsigned bits = __float_as_uint(x[j]) >> 16 | (x[j] != x[j] ? 0x40u : 0u);      // a NaN stays one
-            special[j / 2] |= finite ? 0u : bits << (16 * (j % 2));
-            x[j] = finite ? x[j] : __builtin_copysignf(1.f, x[j]);
-        });
+    float x[8];
+    static_for<0, 8>([&](auto jc) { x[decltype(jc)::value] = __fmul_rn(number[decltype(jc)::value], UP); });
     static_for<0, 4>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
         const unsigned a = __float_as_uint(x[2 * j]), b = __float_as_uint(x[2 * j + 1]);
@@ -56,8 +53,7 @@ __device__ __forceinline__ Parts split8(float (&x)[8], float &odd) {
         const unsigned m = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{ra, rb}), v2b));
         const float qa = __fsub_rn(ra, __uint_as_float(m << 16)), qb = __fsub_rn(rb, __uint_as_float(m & 0xffff0000u));
         p.m[j] = m;
-        p.l[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{qa, qb}), v2b)) | special[j];
-        if constexpr (!SPECIAL) odd = __builtin_fmaf(qa, qb, odd);
+        p.l[j] = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{qa, qb}), v2b));
     });
     return p;
 }
@@ -83,9 +79,9 @@ __global__ __launch_bounds__(256) void split_weights_kernel(const float *w, int 
     v4u *to = out + (int64_t(blockIdx.y) * TAPS * mfrags + blockIdx.x) * 192;
     for (int e = tid; e < 64 * TAPS; e += 256) {
         const int lane = e % 64, tap = e / 64;
-        float v[8], unused = 0.f;
+        float v[8];
         static_for<0, 8>([&](auto jc) { v[decltype(jc)::value] = rows[lane % 32 * PITCH + (8 * (lane / 32) + decltype(jc)::value) * TAPS + tap]; });
-        const Parts p = split8<true>(v, unused);
+        const Parts p = split8(v);
         v4u *dst = to + int64_t(tap) * mfrags * 192 + lane;
         dst[0] = p.h;
         dst[64] = p.m;
@@ -94,7 +90,7 @@ __global__ __launch_bounds__(256) void split_weights_kernel(const float *w, int 
 }
 
 struct SplitParams {
-    const float *x, *bias;
+    const float *x, *w32, *bias;
     const void *w;                 // split weights
     float *out;
     int M, N;                      // output channels, positions (n ho wo)
@@ -118,16 +114,16 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // A workgroup of WM x WN wavefronts (8, or two workgroups of 4 per CU) owns 32 WM output channels x 64 WN positions; a
-// wavefront's 32 x 64 take 12 MFMAs (384 cycles) per 16 channels and tap for 3 KiB of weights, from L2 straight into
+// wavefront's 32 x 64 take 16 MFMAs (512 cycles) per 16 channels and tap for 3 KiB of weights, from L2 straight into
 // registers AHEAD steps early, and 6 KiB of activations from LDS.  As in the fp32 form (conv2d_f32_window.hip) a chunk of CC
 // channels of the input patch -- the rows and columns the tile's positions read through all taps, padding included -- goes
 // to LDS once per element, here in three parts, [part][8 channels][PITCH cells][8], and every tap is a shifted read; a
 // thread converts eight channels of a cell at a time while the other wavefront of its SIMD multiplies.  TAPS: 9 (3x3), 25
 // (5x5), 1 (the patch is the tile's positions themselves, at any stride).
-// What bounds it: the MFMAs, which at the clock the bf16 matrix cores leave (1.5 GHz and less) take two thirds of the time
-// (8 images of 28x28x256 with 256 3x3 filters: 36 of 52 us with everything but them left out), then the conversions, operand
-// reads and weights beside them.  Against the fp32 MFMAs (us, weights' split included): that layer 86 -> 52, 128 channels at
-// 56x56 86 -> 48, 256 to 256 channels 1x1 at 56x56, 32 images, 129 -> 94, 100 to 150 channels 5x5 at 33x41, 4 images, 128 -> 59.
+// What bounds it: the MFMAs at the clock the bf16 matrix cores leave, with conversions, operand reads and weights beside them
+// (six products instead of eight, a quarter of the MFMAs less: 55 us instead of 64 on 8 images of 28x28x256 with 256 3x3
+// filters).  Against the fp32 MFMAs (us, weights' split included): that layer 84 -> 64, 128 channels at 56x56 77 -> 55, 256 to
+// 256 channels 1x1 at 56x56, 32 images, 132 -> 105, 100 to 150 channels 5x5 at 33x41, 4 images, 128 -> 67.
 template <int WM, int WN, int TAPS, int PITCH, int CC>
 __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitParams p) {
     constexpr int THREADS = 64 * WM * WN;
@@ -172,7 +168,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
     // ---- patch bookkeeping: slot i of a thread is cell (tid + 512 i) % PITCH of the chunk's eight channels (tid + 512 i) / PITCH
     constexpr unsigned NOWHERE = 0x80000000u;                              // beyond any buffer: loads 0, stores nothing
     const unsigned plane = unsigned(p.H) * unsigned(p.W);
-    unsigned x_off[SLOTS], x_pad = 0;                                      // bit: the cell is padding
+    unsigned x_off[SLOTS];                                                 // NOWHERE: the cell is padding
     static_for<0, SLOTS>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         const int e = tid + THREADS * i, octet = e / PITCH, cell = e % PITCH;
@@ -192,7 +188,6 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
             w = cell - pr * p.wv + col0 * p.sw - p.pad_left;
         }
         in = in && h >= 0 && h < p.H && w >= 0 && w < p.W;
-        x_pad |= unsigned(!in) << i;
         x_off[i] = in ? ((unsigned(img) * unsigned(p.C) + unsigned(8 * octet)) * plane + unsigned(h * p.W + w)) * 4u : NOWHERE;
     });
 
@@ -203,10 +198,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
     };
     float x_reg[SLOTS][8];
     const int x_bytes = int(int64_t(p.n) * p.C * plane * 4);               // below 2 GiB
-    // Three forms of what follows, none with a branch between the MFMAs.  0: eight channels are there or not, padding is 0.
-    // 1: any channels and padding value.  2: NaN and infinities too -- form 0 or 1 notices them and the tile starts over.
+    // Two forms of what follows, neither with a branch between the MFMAs.  0: eight channels are there or not, padding is 0.
+    // 1: any channels and padding value.
     const bool ragged = p.C % 8 != 0 || p.padding_value != 0.f;
-    float odd = 0.f;
     // Channels FROM to TO of the chunk for slot i.  A chunk behind the last one reads nothing: its loads are out of bounds.
     auto load_patch = [&](auto form, auto ic, auto from, auto to, int chunk) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
@@ -229,10 +223,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
     auto store_patch = [&](auto form, auto ic, int chunk, int at) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
         if constexpr (decltype(form)::value != 0) {
-            const int channels = p.C - chunk * CC - 8 * x_octet(i), left = (x_pad >> i) & 1u ? channels : 0;
+            const int channels = p.C - chunk * CC - 8 * x_octet(i), left = x_off[i] == NOWHERE ? channels : 0;
             static_for<0, 8>([&](auto jc) { x_reg[i][decltype(jc)::value] = decltype(jc)::value < left ? p.padding_value : x_reg[i][decltype(jc)::value]; });
         }
-        const Parts s = split8<decltype(form)::value == 2>(x_reg[i], odd);
+        const Parts s = split8(x_reg[i]);
         char *to = lds + at + (tid + THREADS * i) * 16;
         *reinterpret_cast<v4u *>(to) = s.h;
         *reinterpret_cast<v4u *>(to + PART) = s.m;
@@ -283,6 +277,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
         const std::integral_constant<int, 0> h;
         const std::integral_constant<int, 1> m;
         const std::integral_constant<int, 2> l;
+        mfma(m, l, small);
+        mfma(l, m, small);
         mfma(l, h, small);
         mfma(h, l, small);
         mfma(m, m, small);
@@ -326,10 +322,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
                 load_patch(form, ic, std::integral_constant<int, (s - first) * 8 / steps>{}, std::integral_constant<int, (s - first + 1) * 8 / steps>{}, chunk + 2);
                 b = after;
                 // vector instructions go between the MFMAs, which take 32 cycles each
-                static_for<0, 12>([&](auto) {
+                static_for<0, 16>([&](auto) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                     __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, s == first ? 8 : 3, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, s == first ? 6 : 3, 0);
                     __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                     __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
                 });
@@ -342,33 +338,91 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
     };
     if (ragged) run(std::integral_constant<int, 1>{});
     else run(std::integral_constant<int, 0>{});
-    if (__syncthreads_or(!(__builtin_fabsf(odd) < __builtin_inff()))) run(std::integral_constant<int, 2>{});
+    sum[0] += small[0];
+    sum[1] += small[1];
+    int late = __lane_id();
+    asm volatile("" : "+v"(late));             // nothing of what follows is kept over the loop: positions are decoded again
+    const int in_row = late % 32, half = late / 32;
+
+    // The tile on the fp32 MFMA, operands straight from the tensors: products in the order of the weights (channel, tap), one
+    // rounding each, every second one in the wavefront's upper half.
+    auto exact = [&]() __attribute__((always_inline)) {
+        constexpr int BLOCK = 8;               // MFMAs per fragment whose operands are requested together
+        const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.x), 0, x_bytes, 0x00020000);
+        const auto wr32 = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.w32), 0, p.M * p.C * TAPS * 4, 0x00020000);
+        const int products = p.C * TAPS, w_row = min(m0 + wm * 32 + in_row, p.M - 1) * products;
+        unsigned first[2], inside[2];          // element of the first tap in the first channel; a bit per tap
+        static_for<0, 2>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            int row, col;
+            const bool ok = decode((wn * 2 + j) * 32 + in_row, row, col);
+            const int img = row / p.ho, h = (row - img * p.ho) * p.sh - p.pad_top, w = col * p.sw - p.pad_left;
+            first[j] = unsigned(img) * unsigned(p.C) * plane + unsigned(h * p.W + w);
+            inside[j] = 0;
+            for (int tap = 0; tap < TAPS; ++tap) {
+                const int y = h + tap / KW * p.dil_h, x = w + tap % KW;
+                inside[j] |= unsigned(ok && y >= 0 && y < p.H && x >= 0 && x < p.W) << tap;
+            }
+        });
+        sum[0] = sum[1] = v16f{};
+        for (int k0 = 0; k0 < products; k0 += 2 * BLOCK) {
+            float w[BLOCK], x[2][BLOCK];
+            unsigned at[2][BLOCK];
+            static_for<0, BLOCK>([&](auto ec) {
+                constexpr int e = decltype(ec)::value;
+                const int k = k0 + 2 * e + half, ch = k / TAPS, tap = k % TAPS;
+                const bool there = k < products;
+                w[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wr32, there ? (w_row + k) * 4 : int(NOWHERE), 0, 0));
+                static_for<0, 2>([&](auto jc) {
+                    constexpr int j = decltype(jc)::value;
+                    const unsigned off = (first[j] + unsigned(ch) * plane + unsigned(tap / KW * p.dil_h * p.W + tap % KW)) * 4u;
+                    at[j][e] = !there ? NOWHERE + 4 : inside[j] >> tap & 1u ? off : NOWHERE;
+                    x[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, int(at[j][e]), 0, 0));
+                });
+                __builtin_amdgcn_sched_barrier(0);      // a few conditions at a time: scalar registers
+            });
+            static_for<0, 2 * BLOCK>([&](auto ec) {
+                constexpr int e = decltype(ec)::value / 2, j = decltype(ec)::value % 2;
+                sum[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[e], at[j][e] == NOWHERE ? p.padding_value : x[j][e], sum[j], 0, 0, 0);
+            });
+        }
+    };
+    bool odd = false;
+    static_for<0, 32>([&](auto rc) {
+        const float v = sum[decltype(rc)::value / 16][decltype(rc)::value % 16];
+        odd |= !(__builtin_fabsf(v) < __builtin_inff());
+        sum[decltype(rc)::value / 16][decltype(rc)::value % 16] = __fmul_rn(v, DOWN);
+    });
+    // (behind the last step's barrier no one uses what is read from LDS; __syncthreads_or would keep a register over the loop)
+    int *const odd_wave = reinterpret_cast<int *>(lds);
+    const int any = __any(odd);
+    if (late == 0) odd_wave[wave] = any;
+    lds_barrier();
+    int odd_tile = 0;
+    static_for<0, THREADS / 64>([&](auto wc) { odd_tile |= odd_wave[decltype(wc)::value]; });
+    if (__builtin_amdgcn_readfirstlane(odd_tile)) exact();
 
     // ---- bias values of the tile's rows, requested together
     float bias[16];
     static_for<0, 16>([&](auto rc) {
         constexpr int r = decltype(rc)::value;
-        bias[r] = p.bias ? p.bias[min(m0 + wm * 32 + 8 * (r / 4) + 4 * hf + r % 4, p.M - 1)] : 0.f;
+        bias[r] = p.bias ? p.bias[min(m0 + wm * 32 + 8 * (r / 4) + 4 * half + r % 4, p.M - 1)] : 0.f;
     });
-    sum[0] += small[0];
-    sum[1] += small[1];
     // A lane's element of a row is its own offset plus a uniform one; 32-bit offsets, the output is below 2 GiB.
     const auto out = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, int(int64_t(p.M) * p.N * 4), 0x00020000);
     const bool body = p.act_body == int64_t(p.M) * p.N;      // no element behind the activation's SIMD body
-    int in_row = lane % 32;
-    asm volatile("" : "+v"(in_row));           // positions decoded again, not kept over the loop
     static_for<0, 2>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
         int row, col;
         const bool ok = decode((wn * 2 + j) * 32 + in_row, row, col);
         const int img = row / p.ho;
-        const int base = img * p.M * p.howo + (row - img * p.ho) * p.wo + col + (m0 + wm * 32 + 4 * hf) * p.howo;
+        const int base = img * p.M * p.howo + (row - img * p.ho) * p.wo + col + (m0 + wm * 32 + 4 * half) * p.howo;
         static_for<0, 16>([&](auto rc) {
             constexpr int r = decltype(rc)::value, up = 8 * (r / 4) + r % 4;
             float v = sum[j][r];
             if (p.bias) v = __fadd_rn(v, bias[r]);
             v = apply_act_basic(v, p.act, p.slope, body || base + up * p.howo < p.act_body);
-            const bool in = ok && m0 + wm * 32 + 4 * hf + up < p.M;
+            const bool in = ok && m0 + wm * 32 + 4 * half + up < p.M;
             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), out, in ? base * 4 : int(NOWHERE), up * p.howo * 4, 0);
         });
     });
@@ -461,10 +515,11 @@ ConvF32Split conv_f32_split_choose(const ConvF32Layer &l) {
             SplitParams p{};
             if ((only >= 0 && i * 2 + flat != only) || !plan_tile(l, i, flat != 0, &p)) continue;
             const SplitTile &t = SPLIT_TILES[i];
-            // Time of the busiest CU in us, fitted to 45 layers of 0.01 to 17 GFLOP: 12 MFMAs per step at the 1.28 GHz that the
-            // bf16 matrix cores come to beside everything else, 2 for a tile's start and end, 7 for the launches and the weights.
+            // Time of the busiest CU in us: a step's 16 MFMAs at the 1.7 GHz that the bf16 matrix cores come to beside everything
+            // else, 2 for a tile's start and end, 8 for the launches and the weights.  Chosen together with the line in
+            // split_choice by the tiles of 156 layers of 0.05 to 13 GFLOP.
             const double tiles = double(ceil_div(int64_t(p.tiles_m) * p.tiles_n, 256)), waves = t.wm * t.wn / 4;
-            const double us = tiles * (waves * p.chunks * (t.cc / 16) * t.taps * 384 / 1280. + 2) + 7;
+            const double us = tiles * (waves * p.chunks * (t.cc / 16) * t.taps * 512 / 1700. + 2) + 8;
             if (best.tile < 0 || us < best.us) best = {i * 2 + flat, p.w_bytes, us};
         }
     if (only >= 0) best.us = 0;
@@ -488,6 +543,7 @@ int conv_f32_split(const ConvF32Layer &l, int tile, const float *bias, int act, 
     hipLaunchKernelGGL(pack, grid, dim3(256), 0, stream, l.w_dev, l.cout, l.c, p.mfrags, static_cast<v4u *>(workspace));
     TSX_LAUNCH_CHECK("split_weights_kernel");
     p.x = l.x_dev;
+    p.w32 = l.w_dev;
     p.w = workspace;
     p.bias = bias;
     p.out = out;

@@ -716,8 +716,8 @@ int window_tile(const ConvF32Layer &layer, const GemmArgs &g, double *cycles = n
 // The tile on the bf16 matrix cores for the layer, where that is expected to be at least a twentieth faster than the window
 // kernel; what the register-fed kernel takes stays there.  The window kernel's time is its cost model's at 2.2 GHz times
 // what 45 layers of 0.01 to 17 GFLOP took over it at least: 1.2 with its vector forms, 1.9 without (1.6 to 4.6 measured).  Kept
-// on the window kernel by that: 1x256x28x28, 256 3x3 filters (25 us against 43), 8x512x14x14 to 512 1x1 (14 against 20), all
-// layers of some 10 us.
+// on the window kernel by that: 1x256x28x28, 256 3x3 filters (25 us against 49), 8x512x14x14 to 512 1x1 (15 against 22), all
+// layers of some 10 us.  Of 156 layers two take longer this way by more than 2 % (33.2 -> 36.3 us, 74.4 -> 76.2).
 ConvF32Split split_choice(const ConvF32Layer &layer, const GemmArgs &g) {
     double cycles = 0;
     const ConvF32Split none{-1, 0, 0.}, split = conv_f32_split_choose(layer);

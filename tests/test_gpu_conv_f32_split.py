@@ -112,3 +112,122 @@ def test_conv_f32_split_choice(monkeypatch):
     assert not uses_split(capi, shape(1, 64, 56, 56), shape(64, 64, 3, 3), (1, 1, 1, 1), (1, 1), (1, 1))
     monkeypatch.setenv("TSX_CONV_F32_SPLIT", "0")
     assert not uses_split(capi, *big, (1, 1))
+
+
+def split_modes(monkeypatch, capi, x, wt, pads, strides=(1, 1)):
+    """The fp32 MFMA kernel ("0"), then every tile of the split kernel that takes the layer, set one after the other."""
+    for mode in ["0"] + [str(t + 1) for t in TILES]:
+        monkeypatch.setenv("TSX_CONV_F32_SPLIT", mode)
+        if mode == "0" or uses_split(capi, x, wt, pads, strides, (1, 1)):
+            yield mode
+
+
+def one_weight_per_output(rng, cout, c, k, values):
+    w = np.zeros((cout, c * k * k), np.float32)
+    w[np.arange(cout), rng.integers(0, c * k * k, cout)] = values
+    return w.reshape(cout, c, k, k)
+
+
+@pytest.fixture
+def large_kernels(monkeypatch):
+    for env in ("TSX_CONV_F32_SMALL", "TSX_GEMM_F32_REGFED"):
+        monkeypatch.setenv(env, "0")
+
+
+SPARSE = [(2, 40, 20, 21, 70, 3), (1, 33, 17, 30, 48, 5), (2, 72, 12, 13, 130, 1)]
+
+
+@pytest.mark.parametrize("case", SPARSE)
+def test_conv_f32_split_one_product_per_output(monkeypatch, large_kernels, case):
+    """Kernels with one weight that is not 0: an output is one product, which the fp32 MFMA rounds once.  The split kernel's
+    sum of parts is off by 2^-29 of the product at most before that rounding (what is left out is 2^-32, the sum of the small
+    parts reaches 2^-6 of the product and is rounded twice at that size)."""
+    import torch
+    from tennis_amd import capi
+    n, c, h, w, cout, k = case
+    rng = np.random.default_rng(9)
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    wt = one_weight_per_output(rng, cout, c, k, rng.standard_normal(cout))
+    wt[0][wt[0] != 0] = np.uint32(0x3f80ff80).view(np.float32)      # the largest middle and low parts there are
+    x[0, :, :3] = np.uint32(0x3f80ff80).view(np.float32)
+    pads = (k // 2,) * 4
+    exact = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(), padding=k // 2).numpy()
+    err, seen = {}, exact != 0
+    for mode in split_modes(monkeypatch, capi, x, wt, pads):
+        got = capi.conv2d_f32(dev(x), dev(wt), pads).cpu().numpy().astype(np.float64)
+        assert np.array_equal(got[~seen], exact[~seen])
+        rel = np.abs(got[seen] - exact[seen]) / np.abs(exact[seen])
+        assert rel.max() <= 2.0 ** -24 + 2.0 ** -29, (mode, rel.max())
+        err[mode] = np.sqrt(np.mean(rel ** 2))
+    assert len(err) > 2 and all(e <= err["0"] + 2.0 ** -29 for e in err.values()), err
+
+
+@pytest.mark.parametrize("case", SPARSE)
+@pytest.mark.parametrize("side", ["input", "weights"])
+@pytest.mark.parametrize("exponents", [(0, 40), (140, 190), (200, 255)])
+def test_conv_f32_split_numbers_of_any_size(monkeypatch, large_kernels, case, side, exponents):
+    """Numbers from the smallest denormal on, and up to the largest there are, each times one power of two: every product is a
+    float, and has to arrive as it is."""
+    import torch
+    from tennis_amd import capi
+    n, c, h, w, cout, k = case
+    rng = np.random.default_rng(10)
+
+    def numbers(*shape):
+        sign, exponent, mantissa = rng.integers(0, 2, shape), rng.integers(*exponents, shape), rng.integers(0, 1 << 23, shape)
+        return (sign << 31 | exponent << 23 | mantissa).astype(np.uint32).view(np.float32)
+
+    powers = lambda shape: (2.0 ** (rng.integers(0, 60, shape) * (1 if exponents[0] < 200 else -1))).astype(np.float32)
+    if side == "input":
+        x, wt = numbers(n, c, h, w), one_weight_per_output(rng, cout, c, k, powers(cout))
+    else:
+        wt, x = numbers(cout, c, k, k), np.zeros((n, c, h, w), np.float32)
+        x[:, c - 2, ::k, ::k] = powers(x[:, 0, ::k, ::k].shape)      # a window holds one of them
+    pads = (k // 2,) * 4
+    exact = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(), padding=k // 2).numpy().astype(np.float32)
+    runs = 0
+    for mode in split_modes(monkeypatch, capi, x, wt, pads):
+        got = capi.conv2d_f32(dev(x), dev(wt), pads).cpu().numpy()
+        assert np.array_equal(got, exact), (mode, np.abs(got - exact).max())
+        runs += 1
+    assert runs > 2
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -61, 2.0 ** -66])
+def test_conv_f32_split_tiny_products(monkeypatch, large_kernels, scale):
+    """Operands of an ordinary size whose products, or the parts of them, are denormal."""
+    import torch
+    from tennis_amd import capi
+    g = torch.Generator().manual_seed(6)
+    x, wt = torch.randn(2, 48, 20, 20, generator=g) * scale, torch.randn(64, 48, 3, 3, generator=g) * scale
+    exact = torch.nn.functional.conv2d(x.double(), wt.double(), padding=1)
+    err = {}
+    for mode in split_modes(monkeypatch, capi, x, wt, (1, 1, 1, 1)):
+        err[mode] = float((capi.conv2d_f32(x.cuda(), wt.cuda(), (1, 1, 1, 1)).cpu().double() - exact).norm() / exact.norm())
+    assert len(err) > 2 and all(e <= err["0"] for e in err.values()), err
+
+
+@pytest.mark.parametrize("infinite", ["input", "weights"])
+def test_conv_f32_split_infinity_against_tiny(monkeypatch, large_kernels, infinite):
+    """An infinity times a denormal is an infinity of the product's sign, times 0 it is NaN."""
+    from tennis_amd import capi
+    rng = np.random.default_rng(12)
+    x, wt = rng.standard_normal((1, 40, 14, 15)).astype(np.float32), rng.standard_normal((70, 40, 3, 3)).astype(np.float32)
+    small = np.array([1e-45, -1e-45, 3e-41, -1e-39, 0.0], np.float32)
+    if infinite == "input":
+        x[0, 7, 5, 6] = -np.inf
+        wt[:, 7] = small[np.arange(70) % 5][:, None, None]
+        one = wt[:, 7, 1, 1]
+    else:
+        x[0, 7] = small[rng.integers(0, 5, (14, 15))]
+        wt[33, 7] = 0
+        wt[33, 7, 1, 1] = -np.inf
+        one = x[0, 7]
+    expected = np.where(one == 0, np.nan, np.where(one > 0, -np.inf, np.inf))
+    runs = 0
+    for mode in split_modes(monkeypatch, capi, x, wt, (1, 1, 1, 1)):
+        got = capi.conv2d_f32(dev(x), dev(wt), (1, 1, 1, 1)).cpu().numpy()
+        got = got[0, :, 5, 6] if infinite == "input" else got[0, 33]
+        assert np.array_equal(got, expected, equal_nan=True), mode
+        runs += 1
+    assert runs > 2
