@@ -33,6 +33,7 @@
 // of lane l is row 8*(r/4) + 4*(l/32) + r%4, column l%32.  Rows = cout, columns = positions.
 #include "conv2d_i8_ws_kernel.hpp"
 #include "conv2d_i8_ks.hpp"
+#include "tsx_plans.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -74,47 +75,15 @@ __global__ __launch_bounds__(256) void ws_pack_kernel(const int8_t *__restrict__
 
 static WsPlan make_ws_plan(const WsGeom &g_in);
 
-// Planning walks hundreds of tile shapes (9 us for a 28x28 layer on the host, as long as the kernel it plans for), and a
-// program plans the same few layers again and again: each host thread keeps its last plans, one per slot of a small
-// table.  The switches the planners read are part of the key.
 WsPlan ws_plan(const WsGeom &g) {
     struct Key {
         WsGeom g;
-        char flat[12], rs[12], ks[12];
-    };
-    struct Slot {
-        Key key;
-        bool used;
-        WsPlan plan;
-    };
-    constexpr int SLOTS = 256;
-    static thread_local Slot *slots = nullptr;
-    Key key;
+        PlanSwitch flat, rs, ks;
+    } key;
     std::memset(&key, 0, sizeof(key));
     key.g = g;
-    const char *flat = std::getenv("TSX_CONV_I8_FLAT"), *rs = std::getenv("TSX_CONV_I8_RS"), *ks = std::getenv("TSX_CONV_I8_KS");
-    if ((flat && std::strlen(flat) + 1 >= sizeof(key.flat)) || (rs && std::strlen(rs) + 1 >= sizeof(key.rs)) || (ks && std::strlen(ks) + 1 >= sizeof(key.ks)))
-        return make_ws_plan(g);
-    // (set but empty is another choice than not set)
-    const auto note = [](char *to, const char *value) { if (value) { to[0] = '='; std::strcpy(to + 1, value); } };
-    note(key.flat, flat);
-    note(key.rs, rs);
-    note(key.ks, ks);
-    static thread_local struct Owner {
-        ~Owner() { delete[] slots; slots = nullptr; }
-    } owner;
-    (void)owner;
-    if (!slots) slots = new Slot[SLOTS]();
-    static_assert(sizeof(WsGeom) % sizeof(int) == 0, "the key is hashed as ints");
-    uint32_t h = 0;
-    for (size_t i = 0; i < sizeof(WsGeom) / sizeof(int); ++i) h = (h ^ uint32_t(reinterpret_cast<const int *>(&key.g)[i])) * 0x9e3779b1u;
-    Slot &slot = slots[h >> 24];
-    if (!slot.used || std::memcmp(&slot.key, &key, sizeof(key)) != 0) {
-        slot.plan = make_ws_plan(g);
-        slot.key = key;
-        slot.used = true;
-    }
-    return slot.plan;
+    if (!key.flat.read("TSX_CONV_I8_FLAT") || !key.rs.read("TSX_CONV_I8_RS") || !key.ks.read("TSX_CONV_I8_KS")) return make_ws_plan(g);
+    return kept_plan<WsPlan>(key, [&] { return make_ws_plan(g); });
 }
 
 static WsPlan make_ws_plan(const WsGeom &g_in) {

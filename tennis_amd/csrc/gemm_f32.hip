@@ -19,6 +19,7 @@
 // accumulator register r of lane l is row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 #include "conv2d_f32_split.hpp"
 #include "gemm_f32.hpp"
+#include "tsx_plans.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -718,13 +719,40 @@ int window_tile(const ConvF32Layer &layer, const GemmArgs &g, double *cycles = n
 // what 45 layers of 0.01 to 17 GFLOP took over it at least: 1.2 with its vector forms, 1.9 without (1.6 to 4.6 measured).  Kept
 // on the window kernel by that: 1x256x28x28, 256 3x3 filters (25 us against 49), 8x512x14x14 to 512 1x1 (15 against 22), all
 // layers of some 10 us.  Of 156 layers two take longer this way by more than 2 % (33.2 -> 36.3 us, 74.4 -> 76.2).
-ConvF32Split split_choice(const ConvF32Layer &layer, const GemmArgs &g) {
-    double cycles = 0;
+ConvF32Split split_choice(const ConvF32Layer &layer, int window, double cycles) {
     const ConvF32Split none{-1, 0, 0.}, split = conv_f32_split_choose(layer);
-    if (split.tile < 0 || window_tile(layer, g, &cycles) < 0) return none;
+    if (split.tile < 0 || window < 0) return none;
     if (split.us == 0) return split;
     const bool vector = layer.c * layer.kh * layer.kw % 4 == 0 && (layer.kh == 1 || layer.kh == 3) && reinterpret_cast<uintptr_t>(layer.w_dev) % 16 == 0;
     return split.us * 1.05 < cycles / 2200 * (vector ? 1.2 : 1.9) + 4 ? split : none;
+}
+
+// What a layer beyond the small-layer kernel runs on: with its workspace, and without (-1: a kernel of this file).
+struct ConvF32Plan {
+    ConvF32Split split;
+    int window;
+};
+
+ConvF32Plan conv_f32_plan(const ConvF32Layer &layer, const GemmArgs &g) {
+    struct Key {
+        int geometry[15];
+        int x_misaligned, w_misaligned;        // to 16 bytes: all the planners ask of the addresses
+        PlanSwitch regfed, tile, split;
+    } key;
+    std::memset(&key, 0, sizeof(key));
+    static_assert(offsetof(ConvF32Layer, x_dev) >= sizeof(key.geometry), "fifteen ints in front of the addresses");
+    std::memcpy(key.geometry, &layer, sizeof(key.geometry));
+    key.x_misaligned = int(reinterpret_cast<uintptr_t>(layer.x_dev) % 16);
+    key.w_misaligned = int(reinterpret_cast<uintptr_t>(layer.w_dev) % 16);
+    const auto make = [&] {
+        ConvF32Plan plan{};
+        double cycles = 0;
+        plan.window = window_tile(layer, g, &cycles);
+        plan.split = split_choice(layer, plan.window, cycles);
+        return plan;
+    };
+    if (!key.regfed.read("TSX_GEMM_F32_REGFED") || !key.tile.read("TSX_CONV_F32_TILE") || !key.split.read("TSX_CONV_F32_SPLIT")) return make();
+    return kept_plan<ConvF32Plan>(key, make);
 }
 
 }  // namespace
@@ -782,7 +810,7 @@ size_t tsx_conv2d_f32_workspace_bytes(const tsx_conv2d_geom *geo, const float *w
     tsx::ConvLoader ld;
     if (!geo || conv_f32_problem(geo, nullptr, w_oihw_dev, 0.f, nullptr, TSX_ACT_NONE, 0.f, nullptr, g, ld)) return 0;
     if (tsx::conv3x3_small_takes(g, ld)) return 0;
-    return tsx::split_choice(tsx::window_layer(geo, g, ld), g).workspace_bytes;
+    return tsx::conv_f32_plan(tsx::window_layer(geo, g, ld), g).split.workspace_bytes;
 }
 
 int tsx_conv2d_f32_nchw(const tsx_conv2d_geom *geo, const float *x_dev, const float *w_oihw_dev, float padding_value,
@@ -802,15 +830,14 @@ int tsx_conv2d_f32_nchw_ws(const tsx_conv2d_geom *geo, const float *x_dev, const
         return geo->c <= 32 ? tsx::launch_conv3x3_small<2>(g, ld, tsx::as_stream(stream))
                             : tsx::launch_conv3x3_small<4>(g, ld, tsx::as_stream(stream));
     const tsx::ConvF32Layer layer = tsx::window_layer(geo, g, ld);
+    const tsx::ConvF32Plan plan = tsx::conv_f32_plan(layer, g);
     if (workspace_dev) {
         TSX_REQUIRE(reinterpret_cast<uintptr_t>(workspace_dev) % 16 == 0, "conv2d_f32: workspace not aligned to 16 bytes");
-        const tsx::ConvF32Split split = tsx::split_choice(layer, g);
-        if (split.tile >= 0 && split.workspace_bytes <= workspace_bytes)
-            return tsx::conv_f32_split(layer, split.tile, bias_dev, act, slope, padding_value, out_dev, workspace_dev, tsx::as_stream(stream));
+        if (plan.split.tile >= 0 && plan.split.workspace_bytes <= workspace_bytes)
+            return tsx::conv_f32_split(layer, plan.split.tile, bias_dev, act, slope, padding_value, out_dev, workspace_dev, tsx::as_stream(stream));
     }
-    const int tile = tsx::window_tile(layer, g);
-    if (tile >= 0)
-        return tsx::conv_f32_window(layer, tile, bias_dev, act, slope, padding_value, out_dev, tsx::as_stream(stream));
+    if (plan.window >= 0)
+        return tsx::conv_f32_window(layer, plan.window, bias_dev, act, slope, padding_value, out_dev, tsx::as_stream(stream));
     return tsx::launch(g, ld, 1, tsx::as_stream(stream));
 }
 
@@ -826,14 +853,15 @@ int tsx_conv2d_f32_plan_info(const tsx_conv2d_geom *geo, const float *w_oihw_dev
     }
     const tsx::ConvF32Layer layer = tsx::window_layer(geo, g, ld);
     char with_workspace[128] = "";
-    const tsx::ConvF32Split split = tsx::split_choice(layer, g);
+    const tsx::ConvF32Plan plan = tsx::conv_f32_plan(layer, g);
+    const tsx::ConvF32Split split = plan.split;
     if (split.tile >= 0) {
         int rows, positions, patch;
         tsx::conv_f32_split_tile_size(split.tile, &rows, &positions, &patch);
         std::snprintf(with_workspace, sizeof(with_workspace), " workspace_kernel=bf16_split workspace_tile=%dx%d workspace_patch=%d workspace_window=%s",
                       rows, positions, patch, split.tile % 2 ? "flat" : "segments");
     }
-    const int win = tsx::window_tile(layer, g);
+    const int win = plan.window;
     if (win >= 0) {            // a K-split 32-row tile or a larger one without, by its input patches
         int rows, positions;
         tsx::conv_f32_window_tile_size(win, &rows, &positions);

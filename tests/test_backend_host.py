@@ -139,6 +139,43 @@ def test_every_tile_of_the_bf16_split_kernel_is_reached(monkeypatch):
     assert len(names) == len(set(names)) == len(named) and set(names) == chosen, set(names) ^ chosen
 
 
+def test_kept_fp32_plans_follow_what_they_depend_on(monkeypatch):
+    """A thread keeps its plans: with every switch, weights' alignment and geometry in turn they are what a thread that has
+    planned nothing yet answers."""
+    import threading
+    from tennis_amd import capi
+    L = capi.lib()
+    for name in ("TSX_CONV_F32_SMALL", "TSX_GEMM_F32_REGFED", "TSX_CONV_F32_SPLIT", "TSX_CONV_F32_TILE"):
+        monkeypatch.delenv(name, raising=False)
+
+    def plan(geom, address):
+        buf = ctypes.create_string_buffer(256)
+        assert L.tsx_conv2d_f32_plan_info(ctypes.byref(geom), ctypes.c_void_p(address), buf, len(buf)) == 0
+        return buf.value, L.tsx_conv2d_f32_workspace_bytes(ctypes.byref(geom), ctypes.c_void_p(address))
+
+    def in_a_new_thread(*args):
+        answer = []
+        thread = threading.Thread(target=lambda: answer.append(plan(*args)))
+        thread.start()
+        thread.join()
+        return answer[0]
+
+    layers = [capi.ConvGeom(8, 256, 28, 28, 256, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1), capi.ConvGeom(8, 256, 28, 28, 256, 3, 3, 1, 1, 1, 1, 1, 1, 2, 1),
+              capi.ConvGeom(8, 256, 28, 28, 256, 3, 3, 1, 0, 1, 1, 1, 1, 1, 1), capi.ConvGeom(1, 128, 28, 28, 128, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1),
+              capi.ConvGeom(4, 100, 33, 41, 150, 5, 5, 2, 2, 2, 2, 1, 1, 1, 1)]
+    answers = set()
+    for switch in ({}, {"TSX_CONV_F32_SPLIT": "0"}, {"TSX_CONV_F32_SPLIT": "3"}, {"TSX_CONV_F32_TILE": "1"}, {"TSX_GEMM_F32_REGFED": "0"}, {}):
+        with monkeypatch.context() as m:
+            for name, value in switch.items():
+                m.setenv(name, value)
+            for geom in layers:
+                for address in (4096, 4100):
+                    first = plan(geom, address)
+                    assert plan(geom, address) == first == in_a_new_thread(geom, address), (switch, address)
+                    answers.add(first)
+    assert len(answers) > 10
+
+
 def test_hot_path_operators_are_registered_for_hip():
     from tennis_amd import operators as ops
     for name in ops.SYMBOLS:
