@@ -4,6 +4,9 @@
 // bench(device) -> offline_create(bubble, strict) -> offline_run).
 #include <cstring>
 #include <string>
+#include <vector>
+
+#include <hip/hip_runtime_api.h>
 
 #include "hip/tsx_ts.h"
 
@@ -117,6 +120,41 @@ int tsxop_run_op(const char *device, int device_id, const char *op, int strict, 
         out->bytes = int64_t(y.count()) * ts::type_bytes(y.dtype());
         if (out->bytes > out->capacity) throw ts::Exception("output buffer too small");
         std::memcpy(out->data, y.data(), size_t(out->bytes));
+    });
+}
+
+// Device memory, in bytes, that `copies` operators of one DeviceContext and the context keep when each has run once on the
+// inputs and its output is gone.
+int tsxop_kept_memory(const char *device, int device_id, const char *op, int nparams, const tsxop_tensor *params, int ninputs,
+                      const tsxop_tensor *inputs, int copies, int64_t *bytes) {
+    return guarded([&] {
+        const auto used = [] {
+            size_t free = 0, total = 0;
+            if (hipDeviceSynchronize() != hipSuccess || hipMemGetInfo(&free, &total) != hipSuccess) throw ts::Exception("hipMemGetInfo failed");
+            return int64_t(total - free);
+        };
+        ts::ComputingDevice computing(device, device_id);
+        ts::DeviceContext context(computing);
+        ts::DeviceContext *previous = ts::DeviceContext::Switch(&context);
+        struct Restore {
+            ts::DeviceContext *previous;
+            ~Restore() { ts::DeviceContext::Switch(previous); }
+        } restore{previous};
+
+        const int64_t before = used();
+        std::vector<ts::Operator::shared> operators;
+        for (int c = 0; c < copies; ++c) {
+            auto oper = ts::OperatorCreator::Create(device, op, true);
+            oper->set("#op", ts::tensor::from(std::string(op)));
+            oper->set("#name", ts::tensor::from(std::string(op)));
+            for (int i = 0; i < nparams; ++i) oper->set(params[i].name, host_tensor(params[i]));
+            oper->init();
+            operators.push_back(oper);
+            ts::Stack stack(context.memory_device);
+            for (int i = 0; i < ninputs; ++i) stack.push(host_tensor(inputs[i]));
+            if (oper->run(stack) != 1) throw ts::Exception("operator returned != 1 outputs");
+        }
+        *bytes = used() - before;
     });
 }
 

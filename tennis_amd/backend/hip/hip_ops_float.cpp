@@ -25,9 +25,9 @@ public:
         if (kernel_packed) TS_LOG_ERROR << "[hip] conv2d expects OIHW weights (kernel_packed=false)" << eject;
         const tsx_conv2d_geom g = make_geom(x, w, padding, stride, dilation);
         const size_t ws_bytes = tsx_conv2d_f32_workspace_bytes(&g, w.data<float>());
-        if (ws_bytes && (m_workspace.empty() || size_t(m_workspace.count()) < ws_bytes)) m_workspace = byte_tensor(out.device(), ws_bytes);
+        void *workspace = ws_bytes ? context_scratch(ws_bytes, out.device(), m_workspace) : nullptr;
         check(tsx_conv2d_f32_nchw_ws(&g, x.data<float>(), w.data<float>(), padding_value, nullptr, TSX_ACT_NONE, 0.f,
-                                     out.data<float>(), ws_bytes ? m_workspace.data() : nullptr, ws_bytes, current_stream()),
+                                     out.data<float>(), workspace, ws_bytes, current_stream()),
               "tsx_conv2d_f32_nchw_ws");
     }
 
@@ -37,7 +37,7 @@ protected:
     bool covers(Stack &stack) override { return format_is_nchw(*this) && inputs_are(stack, 2, FLOAT32); }
 
 private:
-    Tensor m_workspace;
+    Tensor m_workspace;   // where no context is bound
 };
 
 // ---------------------------------------------------------------- conv2d_winograd (fp32, F(6,3) and F(2,3))

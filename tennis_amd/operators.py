@@ -108,6 +108,18 @@ def run_op(op, params, inputs, device="hip", device_id=0, strict=True, infer_onl
     return buf[:out.bytes].view(_TS2NP[out.dtype]).reshape(shape).copy()
 
 
+def kept_memory(op, params, inputs, copies, device="hip", device_id=0):
+    """Bytes of device memory that `copies` operators of one DeviceContext keep when each has run once on the inputs."""
+    keep = []
+    p = (_Tensor * max(len(params), 1))(*[_pack(k, v, keep) for k, v in params.items()])
+    i = (_Tensor * max(len(inputs), 1))(*[_pack("", v, keep) for v in inputs])
+    kept = ctypes.c_int64()
+    rc = lib().tsxop_kept_memory(device.encode(), int(device_id), op.encode(), len(params), p, len(inputs), i, int(copies), ctypes.byref(kept))
+    if rc:
+        _raise(rc)
+    return kept.value
+
+
 def conv_params(pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1), padding_value=0.0):
     """The parameter block of conv2d / conv2d_quantized as a graph carries it (NCHW)."""
     return {
