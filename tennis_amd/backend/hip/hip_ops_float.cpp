@@ -89,15 +89,14 @@ public:
         const bool f23 = mode == F2X2_3X3;
         const size_t ws_bytes = f23 ? tsx_winograd_f23_workspace_bytes(&g) : tsx_winograd_f63_workspace_bytes(&g);
         if (ws_bytes == 0) TS_LOG_ERROR << "[hip] conv2d_winograd: " << tsx_last_error() << eject;
-        if (m_workspace.empty() || size_t(m_workspace.count()) < ws_bytes)
-            m_workspace = byte_tensor(out.device(), ws_bytes);
+        void *workspace = context_scratch(ws_bytes, out.device(), m_workspace);
         if (f23)
             check(tsx_conv2d_winograd_f23_nchw(&g, x.data<float>(), static_cast<float *>(m_u.data()), padding_value, nullptr, TSX_ACT_NONE,
-                                               0.f, out.data<float>(), m_workspace.data(), ws_bytes, current_stream()),
+                                               0.f, out.data<float>(), workspace, ws_bytes, current_stream()),
                   "tsx_conv2d_winograd_f23_nchw");
         else
             check(tsx_conv2d_winograd_f63_nchw(&g, x.data<float>(), static_cast<float *>(m_u.data()), padding_value, nullptr, TSX_ACT_NONE,
-                                               0.f, out.data<float>(), m_workspace.data(), ws_bytes, current_stream()),
+                                               0.f, out.data<float>(), workspace, ws_bytes, current_stream()),
                   "tsx_conv2d_winograd_f63_nchw");
     }
 
@@ -106,7 +105,7 @@ protected:
 
 private:
     Tensor m_u;          // transformed kernel, [64 or 16][cout][cin], device memory
-    Tensor m_workspace;
+    Tensor m_workspace;  // where no context is bound
     WinogradConv2DMode m_mode = F6X6_3X3;
     int m_cout = 0, m_cin = 0;
 };

@@ -275,24 +275,30 @@ def test_mish_composition_operators(ops, port):
         ops.run_op("softplus", {}, [x.astype(np.float64)])
 
 
-@pytest.mark.parametrize("op, weights_kept", [("conv2d_quantized", 1), ("conv2d", 0)])
-def test_operators_of_a_context_share_their_workspace(ops, op, weights_kept):
-    """What one more operator keeps is its packed weights; the workspace of a call is the context's."""
+@pytest.mark.parametrize("op", ["conv2d_quantized", "conv2d", "conv2d_winograd"])
+def test_operators_of_a_context_share_their_workspace(ops, op):
+    """What one more operator keeps is its packed or transformed weights; the workspace of a call is the context's."""
+    import ctypes
+    from tennis_amd import capi
     rng = np.random.default_rng(520)
     c, size = 256, 28
     fp32 = op != "conv2d_quantized"
-    x, w = rng.standard_normal((8, c, size, size)), rng.standard_normal((c, c, 3, 3))
+    x, w = rng.standard_normal((16, c, size, size)), rng.standard_normal((c, c, 3, 3))
     x, w = (x.astype(np.float32), w.astype(np.float32)) if fp32 else ((x * 30).astype(np.int8), (w * 30).astype(np.int8))
     params = ops.conv_params((1, 1, 1, 1))
-    if not fp32:
+    geom = ctypes.byref(capi.make_geom(x.shape, w.shape, (1, 1, 1, 1), (1, 1), (1, 1)))
+    L = capi.lib()
+    if op == "conv2d_quantized":
         params["dequantize_scales"] = np.full(c, 0.01, np.float32)
-    from tennis_amd import capi
-    import ctypes
-    geom = capi.make_geom(x.shape, w.shape, (1, 1, 1, 1), (1, 1), (1, 1))
-    workspace = (capi.lib().tsx_conv2d_f32_workspace_bytes(ctypes.byref(geom), ctypes.c_void_p(4096)) if fp32
-                 else capi.lib().tsx_conv2d_i8_workspace_bytes(ctypes.byref(geom)))
-    assert workspace > 1 << 20
+        weights, workspace = 2 * w.nbytes, L.tsx_conv2d_i8_workspace_bytes(geom)        # packed, and those they are packed from
+    elif op == "conv2d":
+        weights, workspace = 0, L.tsx_conv2d_f32_workspace_bytes(geom, ctypes.c_void_p(4096))
+    else:
+        del params["stride"], params["dilation"]
+        weights, workspace = L.tsx_winograd_f63_kernel_bytes(c, c), L.tsx_winograd_f63_workspace_bytes(geom)
+    pages = 2 << 20                                     # an allocation takes whole pages
+    kept = weights + (pages if weights else 0)
+    assert workspace > pages
     ops.kept_memory(op, params, [x, w], 1)              # (code objects are loaded with the first call)
     one, nine = ops.kept_memory(op, params, [x, w], 1), ops.kept_memory(op, params, [x, w], 9)
-    pages = 2 << 20                                     # an allocation takes whole pages
-    assert nine - one <= 8 * weights_kept * (w.nbytes + pages) + pages < 8 * (weights_kept * (w.nbytes + pages) + workspace), (one, nine)
+    assert nine - one <= 8 * kept + pages < 8 * (kept + workspace), (one, nine)
