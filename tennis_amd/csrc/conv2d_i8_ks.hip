@@ -261,10 +261,11 @@ void ks_plan(const WsGeom &g, WsPlan *pl) {
     pl->ks = 0;
     if (!pl->ok || g.gemm) return;
     // TSX_CONV_I8_KS, read at every plan: "0" never; a number: that tile wherever the geometry allows (tests).  A test that
-    // puts layers on another kernel by that kernel's switch gets it.
+    // names the kernel a layer is to take, or those it is not to take, by the other kernels' switches gets what these leave.
+    const auto set = [](const char *name) { const char *value = std::getenv(name); return value && value[0]; };
     const char *e = std::getenv("TSX_CONV_I8_KS");
     const int only = e && e[0] ? std::atoi(e) : -1;
-    if (only == 0 || only > TILE_COUNT || (only < 0 && (std::getenv("TSX_CONV_I8_FLAT") || std::getenv("TSX_CONV_I8_RS")))) return;
+    if (only == 0 || only > TILE_COUNT || (only < 0 && (set("TSX_CONV_I8_FLAT") || set("TSX_CONV_I8_RS")))) return;
     const int64_t image = int64_t(g.hs) * g.ws * g.cp, positions = int64_t(g.n) * g.ho * g.wo;
     // 32-bit offsets from a tile's first image
     if (image * (2 + 32 / (int64_t(g.ho) * g.wo)) >= (int64_t(1) << 31) || positions >= (int64_t(1) << 31) - 64) return;

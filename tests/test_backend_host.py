@@ -139,6 +139,30 @@ def test_every_tile_of_the_bf16_split_kernel_is_reached(monkeypatch):
     assert len(names) == len(set(names)) == len(named) and set(names) == chosen, set(names) ^ chosen
 
 
+def test_other_kernels_switches_keep_layers_off_the_k_split_kernel_where_they_have_a_value(monkeypatch):
+    from tennis_amd import capi
+    L = capi.lib()
+    layer = capi.ConvGeom(1, 256, 14, 14, 256, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1)
+
+    def kernel(**switches):
+        buf = ctypes.create_string_buffer(256)
+        with monkeypatch.context() as m:
+            for name in ("FLAT", "RS", "KS"):
+                m.delenv("TSX_CONV_I8_" + name, raising=False)
+            for name, value in switches.items():
+                m.setenv("TSX_CONV_I8_" + name, value)
+            assert L.tsx_conv2d_i8_plan_info(ctypes.byref(layer), buf, len(buf)) == 0
+        return dict(word.split("=", 1) for word in buf.value.decode().split())["kernel"]
+
+    assert kernel() == "k_split"
+    for name in ("FLAT", "RS"):
+        assert kernel(**{name: ""}) == "k_split", name
+        for value in ("0", "1", "force"):
+            assert kernel(**{name: value}) != "k_split", (name, value)
+        assert kernel(**{name: "force", "KS": "1"}) == "k_split"
+        assert kernel(**{name: "0", "KS": "0"}) == "window_stationary"
+
+
 def test_kept_fp32_plans_follow_what_they_depend_on(monkeypatch):
     """A thread keeps its plans: with every switch, weights' alignment and geometry in turn they are what a thread that has
     planned nothing yet answers."""
