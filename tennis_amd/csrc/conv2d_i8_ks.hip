@@ -3,12 +3,12 @@
 // cpu::Conv2DQuantizedCore, src/kernels/cpu/quantized/conv2d_quantized_core.cpp:18-147).
 //
 // The window-stationary kernel gives each wavefront all of K for its output channels; on a 7x7 map that is 72 K-steps in
-// a row on eight workgroups, each step an L2 latency's share.  Here the W wavefronts of a workgroup own the same 32 MT
-// channels x 32 NT positions and a W-th of the K-steps.  Nothing is shared before the end, so there is no window, no barrier
+// a row on eight workgroups, each step an L2 latency's share.  Here the four wavefronts of a workgroup own the same R MT
+// channels x R positions and a quarter of the K-steps.  Nothing is shared before the end, so there is no window, no barrier
 // and no LDS in front of the MFMAs: weights and activations go from L2 straight into registers (a 1x1 layer's stride, or
 // a tap, is an offset), D K-steps of them requested before the first is used, and the epilogue's scales, biases and
 // residual values right behind them: a layer is one round trip to memory, the MFMAs, and one exchange through LDS in
-// which the W partial sums meet (int32: any order is exact).
+// which the four partial sums meet (int32: any order is exact).
 #include "conv2d_i8_ks.hpp"
 
 #include <cstdlib>
@@ -30,8 +30,10 @@ struct KsParams : EpiParams {
 // (udiv, with the divisor 1 that most of these are taken without a division as well)
 __device__ __forceinline__ int quotient(int n, int d, unsigned magic) { return d == 1 ? n : udiv(n, d, magic); }
 
-template <int R, int MT, int NT, int W, int D, bool MISHX>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MT * NT == 1 ? 4 : 2))) void conv_i8_ks_kernel(KsParams p) {
+constexpr int W = 4;               // wavefronts of a workgroup
+
+template <int R, int MT, int D, bool MISHX>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MT == 1 ? 4 : 2))) void conv_i8_ks_kernel(KsParams p) {
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];   // partial sums [unit][wavefront][lane][4]
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), in = lane % R, part = lane / R;
     // Tiles that read the same weights are consecutive, and each XCD takes a contiguous run of tiles: the weights,
@@ -39,28 +41,20 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MT * NT 
     const int total = p.tiles_m * p.tiles_n, per_xcd = (total + 7) / 8;
     const int t = int(blockIdx.x & 7) * per_xcd + int(blockIdx.x >> 3);
     if (int(blockIdx.x >> 3) >= per_xcd || t >= total) return;
-    const int tm = quotient(t, p.tiles_n, p.tiles_n_magic), m0 = tm * (R * MT), n0 = (t - tm * p.tiles_n) * (R * NT);
+    const int tm = quotient(t, p.tiles_n, p.tiles_n_magic), m0 = tm * (R * MT), n0 = (t - tm * p.tiles_n) * R;
 
-    // ---- this lane's positions, and where their pixels lie from the tile's first image on: 32 bits
+    // ---- this lane's position, and where its pixel lies from the tile's first image on: 32 bits
     const int img0 = quotient(n0, p.howo, p.howo_magic);
     const int8_t *x_base = p.xs + int64_t(img0) * p.hs * p.ws * p.cp;
-    int pos[NT], img[NT], rem[NT], oh[NT];
-    unsigned b_off[NT];
-    static_for<0, NT>([&](auto jc) {
-        constexpr int j = decltype(jc)::value;
-        pos[j] = n0 + j * R + in;
-        const int at = min(pos[j], p.positions - 1);                       // beyond the last: computed, never stored
-        img[j] = quotient(at, p.howo, p.howo_magic);
-        rem[j] = at - img[j] * p.howo;
-        oh[j] = quotient(rem[j], p.wo, p.wo_magic);
-        b_off[j] = unsigned((((img[j] - img0) * p.hs + oh[j] * p.sh) * p.ws + (rem[j] - oh[j] * p.wo) * p.sw) * p.cp + part * 16);
-    });
+    const int pos = n0 + in, at = min(pos, p.positions - 1);               // beyond the last: computed, never stored
+    const int img = quotient(at, p.howo, p.howo_magic), rem = at - img * p.howo, oh = quotient(rem, p.wo, p.wo_magic);
+    const unsigned b_off = unsigned((((img - img0) * p.hs + oh * p.sh) * p.ws + (rem - oh * p.wo) * p.sw) * p.cp + part * 16);
     // ---- operands.  K-steps in the order (tap, channel block), a run of them per wavefront: two channel blocks of a pixel
     // share a cache line.
     // Lane l supplies row / column l % R and 16 bytes of K, group l / R, of v_mfma_i32_32x32x32_i8 or _16x16x64_i8.
     constexpr int HALVES = R / 16;             // MFMAs (and loads of an operand) per K-step: K of 32 or 64
     const unsigned a_off = R == 32 ? unsigned(lane * 16) : unsigned((part / 2) * 1024 + (part % 2) * 512 + in * 16);
-    v4i a[D][MT][HALVES], b[D][NT][HALVES];
+    v4i a[D][MT][HALVES], b[D][HALVES];
     const int k_first = p.ksteps * wave / W, k_end = p.ksteps * (wave + 1) / W;
     auto load = [&](auto slot, int k) __attribute__((always_inline)) {
         constexpr int s = decltype(slot)::value;
@@ -76,28 +70,23 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MT * NT 
             asm volatile("" : "+v"(off));                                  // (scalar base + lane offset: no address arithmetic)
             static_for<0, HALVES>([&](auto hc) { a[s][i][decltype(hc)::value] = *reinterpret_cast<const v4i *>(wi + off + decltype(hc)::value * 1024); });
         });
-        static_for<0, NT>([&](auto jc) {
-            constexpr int j = decltype(jc)::value;
-            unsigned off = b_off[j];
-            asm volatile("" : "+v"(off));
-            static_for<0, HALVES>([&](auto hc) { b[s][j][decltype(hc)::value] = *reinterpret_cast<const v4i *>(xk + off + decltype(hc)::value * 32); });
-        });
+        unsigned off = b_off;
+        asm volatile("" : "+v"(off));
+        static_for<0, HALVES>([&](auto hc) { b[s][decltype(hc)::value] = *reinterpret_cast<const v4i *>(xk + off + decltype(hc)::value * 32); });
     };
     static_for<0, D>([&](auto sc) { load(sc, k_first + decltype(sc)::value); });
 
     // ---- epilogue units: 4 consecutive channels (accumulator registers 4g..4g+3) by 64 / R by a fragment's R positions.  A
     // wavefront takes U of them, all of one fragment; with more wavefronts than units the last ones take none.  What a
     // unit's values meet is requested now.
-    constexpr int PER_FRAG = R == 32 ? 4 : 1, UNITS = PER_FRAG * MT * NT, U = UNITS >= W ? UNITS / W : 1;
+    constexpr int PER_FRAG = R == 32 ? 4 : 1, UNITS = PER_FRAG * MT, U = UNITS >= W ? UNITS / W : 1;
     static_assert((UNITS % W == 0 || W % UNITS == 0) && U <= PER_FRAG, "whole units per wavefront, of one fragment");
     const bool mine = wave * U < UNITS;
     const bool want_q = p.out_i8 || p.st_out, values = p.out_f32 || want_q;
-    const int frag = wave * U / PER_FRAG, frag_m = frag / NT, frag_n = frag - frag_m * NT;
-    int e_img = img[0], e_rem = rem[0], e_oh = oh[0], e_pos = pos[0];
-    if (NT > 1 && frag_n == 1) { e_img = img[NT - 1]; e_rem = rem[NT - 1]; e_oh = oh[NT - 1]; e_pos = pos[NT - 1]; }
-    const int co_first = m0 + frag_m * R + wave * U % PER_FRAG * 8 + part * 4;     // unit u: 8u channels on
-    const bool live = mine && e_pos < p.positions;
-    const int64_t idx_first = (int64_t(e_img) * p.cout + co_first) * p.howo + e_rem;
+    const int frag = wave * U / PER_FRAG;
+    const int co_first = m0 + frag * R + wave * U % PER_FRAG * 8 + part * 4;       // unit u: 8u channels on
+    const bool live = mine && pos < p.positions;
+    const int64_t idx_first = (int64_t(img) * p.cout + co_first) * p.howo + rem;
     float dq[U][4], bias[U][4], res[U][4];
     static_for<0, U>([&](auto uc) {
         static_for<0, 4>([&](auto rc) {
@@ -111,24 +100,20 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MT * NT 
     });
     // one consumer scale per tensor or per image; anything else is looked up by element
     const bool q_simple = p.n_qscales == 1 || p.q_group_len == int64_t(p.cout) * p.howo;
-    const float q_scale = want_q ? p.q_scales[p.n_qscales == 1 || !q_simple ? 0 : e_img] : 0.f;
+    const float q_scale = want_q ? p.q_scales[p.n_qscales == 1 || !q_simple ? 0 : img] : 0.f;
 
     // ---- K: whole rounds of the ring with the next one requested, then the last round
     typedef int Acc __attribute__((ext_vector_type(R * R / 64)));
-    Acc acc[MT][NT];
-    static_for<0, MT>([&](auto ic) {
-        static_for<0, NT>([&](auto jc) { acc[decltype(ic)::value][decltype(jc)::value] = Acc(0); });
-    });
+    Acc acc[MT];
+    static_for<0, MT>([&](auto ic) { acc[decltype(ic)::value] = Acc(0); });
     auto multiply = [&](auto slot) __attribute__((always_inline)) {
         constexpr int s = decltype(slot)::value;
         static_for<0, HALVES>([&](auto hc) {
             constexpr int h = decltype(hc)::value;
             static_for<0, MT>([&](auto ic) {
-                static_for<0, NT>([&](auto jc) {
-                    constexpr int i = decltype(ic)::value, j = decltype(jc)::value;
-                    if constexpr (R == 32) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[s][i][h], b[s][j][h], acc[i][j], 0, 0, 0);
-                    else acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[s][i][h], b[s][j][h], acc[i][j], 0, 0, 0);
-                });
+                constexpr int i = decltype(ic)::value;
+                if constexpr (R == 32) acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[s][i][h], b[s][h], acc[i], 0, 0, 0);
+                else acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[s][i][h], b[s][h], acc[i], 0, 0, 0);
             });
         });
     };
@@ -147,12 +132,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MT * NT 
 
     // ---- the partial sums meet
     static_for<0, MT>([&](auto ic) {
-        static_for<0, NT>([&](auto jc) {
-            static_for<0, PER_FRAG>([&](auto gc) {
-                constexpr int i = decltype(ic)::value, j = decltype(jc)::value, g = decltype(gc)::value;
-                const v4i sums = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-                *reinterpret_cast<v4i *>(lds + ((((i * NT + j) * PER_FRAG + g) * W + wave) * 64 + lane) * 16) = sums;
-            });
+        static_for<0, PER_FRAG>([&](auto gc) {
+            constexpr int i = decltype(ic)::value, g = decltype(gc)::value;
+            const v4i sums = {acc[i][4 * g], acc[i][4 * g + 1], acc[i][4 * g + 2], acc[i][4 * g + 3]};
+            *reinterpret_cast<v4i *>(lds + (((i * PER_FRAG + g) * W + wave) * 64 + lane) * 16) = sums;
         });
     });
     __syncthreads();
@@ -205,7 +188,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MT * NT 
         });
         if (p.st_out) {
             const int up = p.st_up == 2 ? 2 : 1;
-            int8_t *dst = p.st_out + ((int64_t(e_img) * p.st_hs + up * e_oh + p.st_pt) * p.st_ws + up * (e_rem - e_oh * p.wo) + p.st_pl) * p.st_cp + co_first + 8 * u;
+            int8_t *dst = p.st_out + ((int64_t(img) * p.st_hs + up * oh + p.st_pt) * p.st_ws + up * (rem - oh * p.wo) + p.st_pl) * p.st_cp + co_first + 8 * u;
             auto put = [&](int8_t *to) {
                 if (left >= 4) *reinterpret_cast<uint32_t *>(to) = word;
                 else each([&](auto rc) {
@@ -223,36 +206,35 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MT * NT 
     });
 }
 
-template <int R, int MT, int NT, int W, int D>
+template <int R, int MT, int D>
 int launch(const KsParams &p, hipStream_t stream) {
-    const auto kernel = p.act == TSX_ACT_MISH ? conv_i8_ks_kernel<R, MT, NT, W, D, true> : conv_i8_ks_kernel<R, MT, NT, W, D, false>;
-    constexpr size_t lds_bytes = size_t((R == 32 ? 4 : 1) * MT * NT) * W * 1024;
+    const auto kernel = p.act == TSX_ACT_MISH ? conv_i8_ks_kernel<R, MT, D, true> : conv_i8_ks_kernel<R, MT, D, false>;
+    constexpr size_t lds_bytes = size_t((R == 32 ? 4 : 1) * MT) * W * 1024;
     static_assert(lds_bytes <= 65536, "what every kernel may have");
     hipLaunchKernelGGL(kernel, dim3(unsigned((p.tiles_m * p.tiles_n + 7) / 8 * 8)), dim3(64 * W), lds_bytes, stream, p);
     TSX_LAUNCH_CHECK("conv_i8_ks_kernel");
     return 0;
 }
 
-template <int R, int MT, int NT, int W>
+template <int R, int MT>
 int launch_depth(KsParams p, hipStream_t stream) {
     // the ring: the shortest of 1, 2, 3, 5 and 9 K-steps that takes as few rounds as the longest
-    constexpr int MOST = R == 16 && MT * NT == 1 ? 9 : MT * NT <= 2 ? 5 : 3;
+    constexpr int MOST = R == 16 && MT == 1 ? 9 : 5;
     const int steps = (p.ksteps + W - 1) / W;
     p.rounds = (steps + MOST - 1) / MOST;
     const int depth = (steps + p.rounds - 1) / p.rounds;
-    if (depth <= 1) return launch<R, MT, NT, W, 1>(p, stream);
-    if (depth <= 2) return launch<R, MT, NT, W, 2>(p, stream);
-    if (depth <= 3) return launch<R, MT, NT, W, 3>(p, stream);
-    if constexpr (MOST >= 5)
-        if (depth <= 5) return launch<R, MT, NT, W, 5>(p, stream);
-    return launch<R, MT, NT, W, MOST>(p, stream);
+    if (depth <= 1) return launch<R, MT, 1>(p, stream);
+    if (depth <= 2) return launch<R, MT, 2>(p, stream);
+    if (depth <= 3) return launch<R, MT, 3>(p, stream);
+    if (depth <= 5) return launch<R, MT, 5>(p, stream);
+    return launch<R, MT, MOST>(p, stream);
 }
 
 struct KsTile {
     int rows, columns;         // output channels, positions
     int (*launch)(KsParams, hipStream_t);
 };
-const KsTile TILES[] = {{32, 32, launch_depth<32, 1, 1, 4>}, {16, 16, launch_depth<16, 1, 1, 4>}, {32, 16, launch_depth<16, 2, 1, 4>}};
+const KsTile TILES[] = {{32, 32, launch_depth<32, 1>}, {16, 16, launch_depth<16, 1>}, {32, 16, launch_depth<16, 2>}};
 constexpr int TILE_COUNT = int(sizeof(TILES) / sizeof(TILES[0]));
 
 }  // namespace
