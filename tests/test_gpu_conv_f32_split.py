@@ -22,6 +22,12 @@ LAYERS = [
     (2, 68, 10, 14, 70, 1, (0, 0, 0, 0), (1, 1), 1),
     (3, 5, 12, 13, 31, 1, (1, 0, 0, 1), (2, 2), 1),
     (1, 131, 4, 4, 300, 1, (0, 0, 0, 0), (1, 1), 1),
+    # channels in whole eights, which a padding of 0 takes without looking at them one by one, but not in whole chunks
+    (3, 8, 7, 6, 33, 3, (1, 1, 1, 1), (1, 1), 1),
+    (1, 24, 11, 70, 40, 3, (1, 2, 1, 1), (1, 1), 1),
+    (2, 8, 9, 40, 33, 5, (2, 2, 2, 2), (1, 1), 1),
+    (2, 24, 9, 13, 130, 1, (0, 0, 0, 0), (1, 1), 1),
+    (3, 40, 8, 7, 33, 1, (1, 0, 1, 2), (2, 1), 1),
 ]
 TILES = range(20)                # ten tiles, each with column segments and with flat positions
 
@@ -36,10 +42,10 @@ def uses_split(capi, x, w, pads, st, dl):
     return capi.lib().tsx_conv2d_f32_workspace_bytes(ctypes.byref(geom), ctypes.c_void_p(16)) > 0
 
 
-@pytest.mark.parametrize("padding_value", [np.nan, np.inf, 3.0])
-def test_conv_f32_split_tiles(port, monkeypatch, padding_value):
-    """With 3.0 everything is a small integer; otherwise NaN and infinities lie in the padding, in the last channels, all over
-    the last image and in one weight, and have to stay where the windows that hold them are."""
+@pytest.mark.parametrize("padding_value, finite", [(np.nan, False), (np.inf, False), (3.0, True), (0.0, True), (0.0, False)])
+def test_conv_f32_split_tiles(port, monkeypatch, padding_value, finite):
+    """Finite: everything is a small integer; otherwise NaN and infinities lie in the padding where that can hold them, in the
+    last channels, all over the last image and in one weight, and have to stay where the windows that hold them are."""
     from tennis_amd import capi
     for env in ("TSX_CONV_F32_SMALL", "TSX_GEMM_F32_REGFED"):
         monkeypatch.setenv(env, "0")
@@ -51,7 +57,7 @@ def test_conv_f32_split_tiles(port, monkeypatch, padding_value):
         x = rng.integers(-8, 9, (n, c, h, w)).astype(np.float32)
         wt = rng.integers(-4, 5, (cout, c, k, k)).astype(np.float32)
         bias = rng.integers(-9, 10, cout).astype(np.float32)
-        if not np.isfinite(padding_value):
+        if not finite:
             x[0, c - 1, h // 2, w // 3] = np.inf
             x[0, 0, 0, w - 1] = -np.inf
             x[0, c // 2, h - 1, 0] = np.nan
@@ -76,6 +82,33 @@ def test_conv_f32_split_tiles(port, monkeypatch, padding_value):
             runs[tile] += 1
     # a pointwise patch is the tile's positions: flat only
     assert all(r > 0 for t, r in enumerate(runs) if t not in (16, 18)), runs
+
+
+@pytest.mark.parametrize("act", ["relu", "leaky_relu"])
+@pytest.mark.parametrize("case", [(3, 24, 7, 5, 33, 3), (1, 17, 5, 41, 67, 3), (1, 40, 7, 9, 33, 5), (1, 72, 5, 7, 65, 1)])
+def test_conv_f32_split_activations(port, monkeypatch, case, act):
+    """Bias and activation of every tile, on outputs whose number is no multiple of 4: the last ones lie behind the activation's
+    SIMD body, which takes a NaN for another value than they do.  With and without a NaN in the last window of every channel."""
+    from tennis_amd import capi
+    for env in ("TSX_CONV_F32_SMALL", "TSX_GEMM_F32_REGFED"):
+        monkeypatch.setenv(env, "0")
+    n, c, h, w, cout, k = case
+    rng = np.random.default_rng(78)
+    x = rng.integers(-8, 9, (n, c, h, w)).astype(np.float32)
+    wt = rng.integers(-4, 5, (cout, c, k, k)).astype(np.float32)
+    bias = rng.integers(-9, 10, cout).astype(np.float32)
+    pads = (k // 2,) * 4
+    for last in (x[n - 1, 0, h - 1, w - 1], np.nan):
+        x[n - 1, 0, h - 1, w - 1] = last
+        plain = port.add_bias(port.conv2d_f32(x, wt, pads, (1, 1), (1, 1)), bias)
+        assert plain.size % 4 and np.isnan(plain[n - 1, :, h - 1, w - 1]).all() == np.isnan(last)
+        exp = port.relu(plain) if act == "relu" else port.leaky_relu(plain, 0.1)
+        nan, runs = np.isnan(exp), 0
+        for mode in split_modes(monkeypatch, capi, x, wt, pads):
+            got = capi.conv2d_f32(dev(x), dev(wt), pads, bias=dev(bias), act=act, slope=0.1).cpu().numpy()
+            assert np.array_equal(np.isnan(got), nan) and np.array_equal(bits(got[~nan]), bits(exp[~nan])), (mode, last)
+            runs += 1
+        assert runs > 2
 
 
 @pytest.mark.parametrize("case", [(2, 48, 20, 20, 64, 3), (1, 256, 28, 28, 128, 3), (2, 64, 24, 24, 32, 5), (4, 512, 14, 14, 128, 1)])
