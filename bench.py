@@ -29,6 +29,7 @@ sys.path.insert(0, ROOT)
 PEAK_INT8_TOPS = 5000.0   # MI355X dense int8 MFMA, 5.0 POP/s
 PEAK_HBM_GBS = 8000.0     # MI355X HBM3E, 8 TB/s
 PEAK_FP32_TFLOPS = 157.3  # MI355X dense fp32 MFMA
+PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA
 
 CFG = dict(n=32, c=256, h=28, w=28, cout=256, k=3, pad=1)
 
@@ -402,7 +403,8 @@ def kernels_leg(reps=20):
         e1.record()
         torch.cuda.synchronize()
         t = e0.elapsed_time(e1) * 1e-3 / reps
-        peak = {"hbm": PEAK_HBM_GBS * 1e9, "mfma_i8": PEAK_INT8_TOPS * 1e12, "mfma_f32": PEAK_FP32_TFLOPS * 1e12}[bound]
+        peak = {"hbm": PEAK_HBM_GBS * 1e9, "mfma_i8": PEAK_INT8_TOPS * 1e12, "mfma_f32": PEAK_FP32_TFLOPS * 1e12,
+                "mfma_bf16": PEAK_BF16_TFLOPS * 1e12}[bound]
         rows.append({"kernel": name, "bound": bound, "us": t * 1e6, "work": work, "achieved": work / t,
                      "unit": "B/s" if bound == "hbm" else "op/s", "frac": work / t / peak})
 
@@ -417,11 +419,12 @@ def kernels_leg(reps=20):
     # fp32 on a shape the reference's selector routes to Winograd F(6,3): 8x256x28x28 * 256x256x3x3
     x8, w8, b8 = torch.rand((8, 256, 28, 28), device=dev) * 2 - 1, rnd(256, 256, 3, 3) * 0.03, rnd(256) * 0.01
     flops8 = 2.0 * 8 * 256 * 28 * 28 * 256 * 9
-    timed("conv2d_f32 8x256x28x28 (conv_f32_window_kernel)", "mfma_f32", flops8, lambda: capi.conv2d_f32(x8, w8, (1, 1, 1, 1), bias=b8, act="relu"))
+    # (both direct layers: eight bf16 products to one of the convolution)
+    timed("conv2d_f32 8x256x28x28 (conv_f32_split_kernel)", "mfma_bf16", 8 * flops8, lambda: capi.conv2d_f32(x8, w8, (1, 1, 1, 1), bias=b8, act="relu"))
     w63b = capi.WinogradF63(w8, (1, 1, 1, 1))
     timed("winograd F(6,3) 8x256x28x28 (direct-conv flops)", "mfma_f32", flops8, lambda: w63b(x8, bias=b8, act="relu"))
     x11, w11 = rnd(32, 256, 56, 56), rnd(256, 256, 1, 1) * 0.06
-    timed("conv2d_f32 1x1 256->256 @56x56 bs32 (conv_f32_window_kernel)", "mfma_f32", 2.0 * 32 * 256 * 56 * 56 * 256, lambda: capi.conv2d_f32(x11, w11))
+    timed("conv2d_f32 1x1 256->256 @56x56 bs32 (conv_f32_split_kernel)", "mfma_bf16", 8 * 2.0 * 32 * 256 * 56 * 56 * 256, lambda: capi.conv2d_f32(x11, w11))
     del x11
     # int8 GEMM: largest and a mid shape of BASELINE config 3, and the weight-streaming single row
     k = n = 4096
