@@ -201,13 +201,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
     // Two forms of what follows, neither with a branch between the MFMAs.  0: eight channels are there or not, padding is 0.
     // 1: any channels and padding value.
     const bool ragged = p.C % 8 != 0 || p.padding_value != 0.f;
-    // Channels FROM to TO of the chunk for slot i.  A chunk behind the last one reads nothing: its loads are out of bounds.
+    // Channels FROM to TO of the chunk for slot i.  A chunk behind the last one has no channel, and reads nothing:
+    // its offsets are beyond the buffer (whose size stays above every channel's scalar offset, from which the hardware counts).
     auto load_patch = [&](auto form, auto ic, auto from, auto to, int chunk) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
         const bool live = chunk < p.chunks;
         const int c0 = live ? chunk * CC : 0, at = c0 * int(plane) * 4;
-        const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(p.x) + at), 0, live ? x_bytes - at : 0, 0x00020000);
-        const int left = p.C - c0 - 8 * x_octet(i);
+        const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(p.x) + at), 0, x_bytes - at, 0x00020000);
+        const int left = (live ? p.C - c0 : 0) - 8 * x_octet(i);
         unsigned base = x_off[i];
         if constexpr (decltype(form)::value != 0) asm volatile("" : "+v"(base));      // no sums of it kept either
         static_for<decltype(from)::value, decltype(to)::value>([&](auto jc) {
