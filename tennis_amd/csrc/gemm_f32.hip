@@ -720,9 +720,10 @@ int window_tile(const ConvF32Layer &layer, const GemmArgs &g, double *cycles = n
 // on the window kernel by that: 1x256x28x28, 256 3x3 filters (25 us against 49), 8x512x14x14 to 512 1x1 (15 against 22), all
 // layers of some 10 us.  Of 156 layers two take longer this way by more than 2 % (33.2 -> 36.3 us, 74.4 -> 76.2).
 ConvF32Split split_choice(const ConvF32Layer &layer, int window, double cycles) {
-    const ConvF32Split none{-1, 0, 0.}, split = conv_f32_split_choose(layer);
-    if (split.tile < 0 || window < 0) return none;
-    if (split.us == 0) return split;
+    const ConvF32Split none{-1, 0, 0.};
+    if (window < 0) return none;
+    const ConvF32Split split = conv_f32_split_choose(layer);
+    if (split.tile < 0 || split.us == 0) return split;
     const bool vector = layer.c * layer.kh * layer.kw % 4 == 0 && (layer.kh == 1 || layer.kh == 3) && reinterpret_cast<uintptr_t>(layer.w_dev) % 16 == 0;
     return split.us * 1.05 < cycles / 2200 * (vector ? 1.2 : 1.9) + 4 ? split : none;
 }
