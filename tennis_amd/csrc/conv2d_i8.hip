@@ -524,8 +524,10 @@ __global__ __launch_bounds__(WGM *WGN * 64) void igemm_i8_kernel(GemmParams p) {
     static_assert(A_BYTES % (16 * THREADS) == 0 && B_BYTES % (16 * THREADS) == 0, "tile/threads mismatch");
 
     __shared__ __attribute__((aligned(16))) int8_t lds[2][A_BYTES + B_BYTES];
+    __shared__ tsx::MishTables mish_tables;
 
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+    if (!SWAP && p.act == TSX_ACT_MISH) mish_tables.fill(tid);      // (read behind the K loop's barriers)
     const int wm = wave / WGN, wn = wave % WGN;
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
 
@@ -678,7 +680,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void igemm_i8_kernel(GemmParams p) {
                         }
                         const float qs = want_q ? p.q_scales[p.n_qscales == 1 ? 0 : n] : 0.f;
                         tsx::epilogue_rows16(p, acc[i][j], dq, bias, base[j] + int64_t(co0) * p.howo, p.howo, qs,
-                                             p.n_qscales == 1, st_dst);
+                                             p.n_qscales == 1, st_dst, tsx::MishTablesInLds{&mish_tables});
                     }
                 });
             } else {

@@ -13,7 +13,7 @@ constexpr int FL_PIX = 80;        // LDS bytes per window pixel (64 channels + 1
 constexpr int FL_THREADS = 512;   // 8 wavefronts: two per SIMD
 constexpr int FL_MAX_FILL = 4;    // window chunks per thread per channel block
 constexpr int FL_MAX_WP = FL_MAX_FILL * FL_THREADS / 4;   // 512 window pixels
-constexpr int FL_MAX_LDS = 160 * 1024;                    // LDS of one CU, all of it available to one workgroup
+constexpr int FL_MAX_LDS = 160 * 1024 - 2048;             // LDS of one CU, all of it available to one workgroup, less the exact Mish's tables
 
 struct FlParams : EpiParams {
     const int8_t *xs;   // staged activations [n][hs][ws][cp]
@@ -56,7 +56,7 @@ namespace {
 // wavefronts that finish first store their output while the others still multiply.  Otherwise the window
 // is double buffered, one channel block ahead, with one barrier per block.
 template <int NT, bool EXTRA, bool STREAM, bool RESIDENT, bool MISHX>
-__device__ __forceinline__ void fl_wave(const FlParams &p, int8_t *lds, int tile, int wave_m, int frag0) {
+__device__ __forceinline__ void fl_wave(const FlParams &p, int8_t *lds, MishTables *mish_tables, int tile, int wave_m, int frag0) {
     const int tid = threadIdx.x, lane = tid % 64;
     const int P0 = tile * p.frags * 32;   // first flat position (n, oh, ow) of the tile
     const int R0 = udiv(P0, p.wo, p.wo_magic);   // its row in the batch-wide row sequence
@@ -169,6 +169,7 @@ __device__ __forceinline__ void fl_wave(const FlParams &p, int8_t *lds, int tile
             });
         });
     }
+    if (MISHX) mish_tables->fill(tid);
     window_store(0);
     __syncthreads();
     if (!RESIDENT && p.cblocks > 1) window_load(1);   // block cb+1, in flight during block cb's taps
@@ -330,7 +331,20 @@ __device__ __forceinline__ void fl_wave(const FlParams &p, int8_t *lds, int tile
                 constexpr int r = decltype(rc)::value;
                 v[r] = __fadd_rn(v[r], res[j][r]);
             });
-            if (p.act == TSX_ACT_RELU) {
+            const float q_scale = want_q ? p.q_scales[p.n_qscales == 1 ? 0 : pimg[j]] : 0.f;
+            const bool q_only = MISHX && !p.out_f32 && want_q;       // the Mish's fp32 values go nowhere
+            const MishTablesInLds tables{mish_tables};
+            uint32_t word[4];        // requantized values, four consecutive channels to a word
+            if (MISHX) {
+                // (only layers with the exact Mish come here) nothing but the requantized values leaves: the exact form only
+                // where it decides a rounding
+                if (q_only) {
+                    if (EXTRA && p.residual && p.res_after) mish_words_for_rounding<true>(v, res[j], q_scale, q_even, word, tables);
+                    else mish_words_for_rounding<false>(v, res[j], q_scale, q_even, word, tables);
+                } else {
+                    mish_fragment(v, tables);
+                }
+            } else if (p.act == TSX_ACT_RELU) {
                 static_for<0, 16>([&](auto rc) {
                     constexpr int r = decltype(rc)::value;
                     v[r] = v[r] > 0.f ? v[r] : 0.f;
@@ -340,18 +354,13 @@ __device__ __forceinline__ void fl_wave(const FlParams &p, int8_t *lds, int tile
                     constexpr int r = decltype(rc)::value;
                     v[r] = apply_act_conv_i8(v[r], TSX_ACT_LEAKY_RELU, p.slope, true);
                 });
-            } else if (MISHX && p.act == TSX_ACT_MISH) {
-                // nothing but the requantized values leaves: the exact form only where it decides a rounding
-                if (!p.out_f32 && want_q)
-                    mish_fragment_for_rounding(v, res[j], EXTRA && p.residual && p.res_after, p.q_scales[p.n_qscales == 1 ? 0 : pimg[j]]);
-                else mish_fragment(v);
             } else if (p.act == TSX_ACT_MISH_FAST) {
                 static_for<0, 16>([&](auto rc) {
                     constexpr int r = decltype(rc)::value;
                     v[r] = apply_act_conv_i8(v[r], TSX_ACT_MISH_FAST, 0.f, true);
                 });
             }
-            if (EXTRA && p.residual && p.res_after) static_for<0, 16>([&](auto rc) {
+            if (EXTRA && p.residual && p.res_after && !q_only) static_for<0, 16>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
                 v[r] = __fadd_rn(v[r], res[j][r]);
             });
@@ -365,31 +374,26 @@ __device__ __forceinline__ void fl_wave(const FlParams &p, int8_t *lds, int tile
                 else *o = v[r];
             });
             if (want_q) {
-                const float q_scale = p.q_scales[p.n_qscales == 1 ? 0 : pimg[j]];
-                int qv[16];
-                if (q_even) static_for<0, 16>([&](auto rc) {
+                if (!q_only) static_for<0, 4>([&](auto gc) { word[decltype(gc)::value] = 0; });
+                if (q_only) {
+                } else if (q_even) static_for<0, 16>([&](auto rc) {
                     constexpr int r = decltype(rc)::value;
-                    qv[r] = quantize_value(__fmul_rn(v[r], q_scale), true);
+                    word[r / 4] = quantize_pack<r % 4>(__fmul_rn(v[r], q_scale), true, word[r / 4]);
                 });
                 else static_for<0, 16>([&](auto rc) {
                     constexpr int r = decltype(rc)::value;
-                    qv[r] = quantize_value(__fmul_rn(v[r], q_scale), false);
+                    word[r / 4] = quantize_pack<r % 4>(__fmul_rn(v[r], q_scale), false, word[r / 4]);
                 });
+                static_for<0, 4>([&](auto gc) { word[decltype(gc)::value] ^= 0x80808080u; });
                 if (p.out_i8) static_for<0, 16>([&](auto rc) {
                     constexpr int r = decltype(rc)::value;
                     constexpr int dco = 8 * (r / 4) + (r % 4);
-                    (p.out_i8 + base + int64_t(dco) * howo)[lane_off] = int8_t(qv[r]);
+                    (p.out_i8 + base + int64_t(dco) * howo)[lane_off] = int8_t(word[r / 4] >> (8 * (r % 4)));
                 });
                 if (EXTRA && p.st_out) {
                     // consumer's staged layout [pixel][channel]: registers 4g..4g+3 of a lane are 4 consecutive
                     // channels of one pixel, the pixel's other 16 channels of this fragment sit in lane +-32.  Two
                     // half-wave swaps leave every lane with 16 consecutive channels for one 16-byte store.
-                    uint32_t word[4];
-                    static_for<0, 4>([&](auto gc) {
-                        constexpr int g4 = decltype(gc)::value;
-                        word[g4] = uint32_t(qv[4 * g4] & 0xff) | (uint32_t(qv[4 * g4 + 1] & 0xff) << 8) |
-                                   (uint32_t(qv[4 * g4 + 2] & 0xff) << 16) | (uint32_t(qv[4 * g4 + 3] & 0xff) << 24);
-                    });
                     const auto s02 = __builtin_amdgcn_permlane32_swap(word[0], word[2], false, false);
                     const auto s13 = __builtin_amdgcn_permlane32_swap(word[1], word[3], false, false);
                     const int oh = udiv(prem[j], p.wo, p.wo_magic), ow = prem[j] - oh * p.wo;
@@ -411,10 +415,19 @@ __device__ __forceinline__ void fl_wave(const FlParams &p, int8_t *lds, int tile
             constexpr int j = decltype(jc)::value;
             const int co0 = cf + 4 * (lane / 32);
             const int64_t base = (int64_t(pimg[j]) * p.cout + co0) * howo + prem[j];
-            static_for<0, 16>([&](auto rc) {
+            if constexpr (MISHX) {
+                const v16i a = acc[j];        // (a loop: unrolled, the inlined Mish is most of the kernel's code)
+                v16f d, b;
+                static_for<0, 16>([&](auto rc) { d[decltype(rc)::value] = dq[decltype(rc)::value], b[decltype(rc)::value] = bias[decltype(rc)::value]; });
+#pragma clang loop unroll(disable)
+                for (int r = 0; r < 16; ++r) {
+                    const int dco = 8 * (r / 4) + (r % 4);
+                    if (pok[j] && co0 + dco < p.cout) emit<true>(p, a[r], base + int64_t(dco) * howo, d[r], b[r], 0.f);
+                }
+            } else static_for<0, 16>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
                 constexpr int dco = 8 * (r / 4) + (r % 4);
-                if (pok[j] && co0 + dco < p.cout) emit<MISHX>(p, acc[j][r], base + int64_t(dco) * howo, dq[r], bias[r], 0.f);
+                if (pok[j] && co0 + dco < p.cout) emit<false>(p, acc[j][r], base + int64_t(dco) * howo, dq[r], bias[r], 0.f);
             });
         });
     }
@@ -435,6 +448,7 @@ __global__ __launch_bounds__(FL_THREADS) void conv_i8_fl_kernel(FlParams p_in) {
     }
     p.row_scale = nullptr;
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];   // (RESIDENT ? cblocks : 2) x wpix x FL_PIX
+    __shared__ MishTables mish_tables;                             // (exists in the instantiations that read it)
     // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2: give every XCD a contiguous run of
     // tiles, so the halo rows two neighbouring tiles share are fetched from HBM once.  gridDim.x is a multiple
     // of 8, so the workgroups of one tile (blockIdx.y) land on the same XCD too.
@@ -447,9 +461,9 @@ __global__ __launch_bounds__(FL_THREADS) void conv_i8_fl_kernel(FlParams p_in) {
     // the tile's output under the other group's K loop.
     if (wave < 4) {
         __builtin_amdgcn_s_setprio(3);
-        fl_wave<NTA, EXTRA, STREAM, RESIDENT, MISHX>(p, lds, tile, wave, 0);
+        fl_wave<NTA, EXTRA, STREAM, RESIDENT, MISHX>(p, lds, &mish_tables, tile, wave, 0);
     } else {
-        fl_wave<NTB, EXTRA, STREAM, RESIDENT, MISHX>(p, lds, tile, wave - 4, NTA);
+        fl_wave<NTB, EXTRA, STREAM, RESIDENT, MISHX>(p, lds, &mish_tables, tile, wave - 4, NTA);
     }
 }
 

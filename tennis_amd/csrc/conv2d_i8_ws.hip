@@ -129,7 +129,7 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
             const bool straddle = g.ho % t != 0;
             const int wr = (t - 1) * g.sh + (g.kh - 1) * g.dil_h + 1 + (straddle && wrap > 0 ? wrap : 0);
             const int wp = wr * wc;
-            if (wp > MAX_WP || size_t(2) * wp * PIX > 65536) continue;   // two windows must fit 64 KiB of LDS
+            if (wp > MAX_WP || size_t(2) * wp * PIX > WS_MAX_LDS) continue;   // two windows must fit
             const int64_t wgs = tiles * (coutp / bm);
             const int64_t frags = tiles * nt * wn;
             const int64_t per_cu = (wgs + 255) / 256;
@@ -156,8 +156,13 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
             }
             // A 1x1 layer's workgroup is mostly epilogue, its time is the traffic of its tile, and what pays is many small
             // workgroups in flight per CU (us, 32 images: 64 to 256 channels 56x56 with a residual join, 4 fragments per
-            // wavefront 63, 2 55; 256 to 128 56x56 20.9 -> 17.9; 256 to 1024 14x14 with a join 18.1 -> 15.8).
+            // wavefront 63, 2 46; 256 to 128 56x56 20.9 -> 16.9; 256 to 1024 14x14 with a join 18.1 -> 17.4).
             if (!several_taps && (!g.gemm || g.cblocks <= 2) && nt > 2) continue;
+            // Two fragments share a wavefront's set-up; a grid of less than one and a half workgroups per CU takes one (us, one /
+            // two: 32 images 256 to 64 56x56 14.5 / 14.0, 128 to 512 28x28 with a join 26.8 / 25.6, 512 to 2048 7x7 13.2 / 11.4,
+            // but 1024 to 256 14x14 9.5 / 10.0, 2048 to 512 7x7 11.5 / 13.5).
+            if (!several_taps && !g.gemm && g.wo == 1 && g.ho >= 64 * wn &&
+                nt == (ceil_div(int64_t(g.n) * g.ho, 64 * wn) * (coutp / bm) >= 384 ? 1 : 2)) continue;
             if (best_cost < 0 || cost < best_cost || (cost == best_cost && frags < best_frags)) {
                 best_cost = cost;
                 best_frags = frags;
@@ -188,7 +193,7 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
     pl.cbs = 1;
     if (g.kh == 1 && g.kw == 1)
         for (int c = 4; c > 1; c >>= 1)
-            if (g.cblocks % c == 0 && pl.wp * 4 * c <= MAX_FILL * WS_THREADS && size_t(2) * pl.wp * (64 * c + 16) <= 65536) {
+            if (g.cblocks % c == 0 && pl.wp * 4 * c <= MAX_FILL * WS_THREADS && size_t(2) * pl.wp * (64 * c + 16) <= WS_MAX_LDS) {
                 pl.cbs = c;
                 break;
             }
@@ -213,10 +218,12 @@ int ws_pack_weights(const WsGeom &g, const WsPlan &pl, const int8_t *w_oihw, int
 int ws_launch(const WsGeom &g, const WsPlan &plan, const int8_t *xs, const int8_t *packed, const EpiParams &ep,
               hipStream_t stream) {
     WsPlan pl = plan;
-    // The exact Mish's arithmetic is most of a 1x1 layer: tiles of one fragment per wavefront, which hide it behind one another
-    // (us, 8 images: 64 to 64 channels 304x304, fp32 output, 146 -> 138; 128 to 64 152x152 45.8 -> 40.4).  A small grid keeps
-    // its tiles.
-    if (ep.act == TSX_ACT_MISH && g.kh * g.kw == 1 && pl.wo == 1 && pl.nt == 2 && pl.th == pl.wp && pl.th % 2 == 0 && pl.tiles * ceil_div(g.cout, 32 * pl.wm) >= 1024) {
+    // With the exact Mish a 1x1 layer that hands out its fp32 values evaluates the whole chain for each: tiles of one fragment
+    // per wavefront, five wavefronts per SIMD for three (us, 8 images: 64 to 64 channels 304x304 127 -> 118; 128 to 64 152x152
+    // 40.8 -> 37.5; 256 to 256 38x38 19.8 -> 16.7).  Where only int8 leaves, two keep their lead (57.6 against 58.4 on the
+    // first of these) down to two workgroups per CU.
+    if (ep.act == TSX_ACT_MISH && g.kh * g.kw == 1 && pl.wo == 1 && pl.nt == 2 && pl.th == pl.wp && pl.th % 2 == 0 &&
+        (ep.out_f32 || pl.tiles * ceil_div(g.cout, 32 * pl.wm) < 512)) {
         pl.nt = 1;
         pl.th = pl.wr = pl.wp = pl.th / 2;
         pl.tiles = ceil_div(int64_t(g.n) * pl.ho, pl.th);
@@ -276,6 +283,9 @@ int ws_launch(const WsGeom &g, const WsPlan &plan, const int8_t *xs, const int8_
     p.blocks_m = (g.cout + bm - 1) / bm;
     const int64_t total = pl.tiles * p.blocks_m;
     p.per_xcd = total < (1 << 23) ? int((total + 7) / 8) : 0;      // (a launch holds fewer than 2^32 work items along x)
+    p.ho_magic = div_magic(p.ho, int64_t(g.n) * p.ho);
+    p.blocks_magic = div_magic(p.blocks_m, total + 7);
+    p.ctiles_magic = div_magic(p.ctiles, pl.tiles);
     const dim3 grid = p.per_xcd ? dim3(unsigned(p.per_xcd * 8)) : dim3(unsigned(pl.tiles), unsigned(p.blocks_m));
     // two window buffers (one channel block ahead); a layer whose channels fit one window never swaps and takes one:
     // more workgroups per CU where the window is large (stride-2 3x3 layers on 32 or 64 channels)

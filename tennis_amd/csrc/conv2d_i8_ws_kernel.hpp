@@ -13,6 +13,7 @@ constexpr int WS_THREADS = 256;
 constexpr int WS_FM = 1;        // 32-cout fragments per wavefront
 constexpr int MAX_FILL = 7;     // window chunks per thread per channel block
 constexpr int SMALL_FILL = 4;   // ... of the kernels compiled for small windows (fewer registers: one more workgroup per CU)
+constexpr size_t WS_MAX_LDS = 65536 - sizeof(MishTables);   // both windows: 64 KiB less the tables of the exact Mish
 constexpr int MAX_WP = MAX_FILL * WS_THREADS / 4;   // 448 window pixels
 
 struct WsParams : EpiParams {
@@ -33,6 +34,7 @@ struct WsParams : EpiParams {
     int rowmajor;     // GEMM: output index position * cout + channel, row_scale[position] applied behind dq
     // per-lane divisions by uniform divisors as one multiply-high (div_magic / udiv)
     unsigned wc_magic, tw_magic, ow_magic;
+    unsigned ho_magic, blocks_magic, ctiles_magic;      // of a tile's first row and of its own index (scalar)
 };
 
 
@@ -71,8 +73,15 @@ namespace {
 // MFMAs.  A wavefront with one fragment spends 2 MFMAs (64 cycles) on a K-step, half of an LDS read's latency: read
 // one half-step ahead (the other form), the small maps at the end of a network -- under one wavefront per SIMD,
 // nothing else to issue -- ran at one K-step per two LDS latencies.
+//
+// ws_waves: wavefronts per SIMD the registers have to leave room for.  The small tiles wait for memory more than they
+// multiply (64 to 64 channels 304x304 with the exact Mish, 8 images: 135 us at four wavefronts per SIMD, 118 at five); what
+// does not fit is left at what it needs.
+constexpr int ws_waves(int nt, int fill, bool look, bool mishx) {
+    return nt > 4 ? 1 : fill != SMALL_FILL ? 2 : nt == 1 && !look ? 5 : mishx && nt == 2 ? 3 : 4;
+}
 template <int NT, int FM, bool EXTRA, bool STREAM, bool ROWM, int FILL, bool LOOK, bool MISHX = false>
-__global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <= 4 ? 2 : 1))) void conv_i8_ws_kernel(WsParams p_in) {
+__global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_waves(NT, FILL, LOOK, MISHX)))) void conv_i8_ws_kernel(WsParams p_in) {
     WsParams p = p_in;
     if (!EXTRA) {
         p.residual = nullptr;
@@ -80,6 +89,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
     }
     if (!ROWM) p.row_scale = nullptr;
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];   // 2 x wpix x PIX
+    __shared__ MishTables mish_tables;                             // (exists in the instantiations that read it)
     // the wavefront's index as a scalar: what derives from it (first cout, tile bases, the choice of epilogue path)
     // then stays in scalar registers and branches uniformly
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -89,14 +99,14 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
     int tile = blockIdx.x, block_m = blockIdx.y;
     if (p.per_xcd) {
         const int t = int(blockIdx.x & 7) * p.per_xcd + int(blockIdx.x >> 3);
-        tile = p.blocks_m == 1 ? t : t / p.blocks_m;
+        tile = udiv(t, p.blocks_m, p.blocks_magic);
         block_m = t - tile * p.blocks_m;
         if (tile >= p.tiles) return;
     }
-    const int rtile = p.ctiles == 1 ? tile : tile / p.ctiles;
+    const int rtile = udiv(tile, p.ctiles, p.ctiles_magic);
     const int col0 = (tile - rtile * p.ctiles) * p.tw;         // first output column of the tile
     const int row0 = rtile * p.th;           // first output row of the tile, counted over the whole batch
-    const int img = row0 / p.ho;             // image of the tile's first row
+    const int img = udiv(row0, p.ho, p.ho_magic);   // image of the tile's first row
     const int th0 = row0 - img * p.ho;       // ... and that row inside it
     const int rows_total = p.n * p.ho;
     // staged rows from where output row `ho` of an image would start to the next image's first row
@@ -212,6 +222,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
     // a tile may end in the next image: one consumer scale per image, selected per lane
     const float q_scale_a = (fast && want_q) ? p.q_scales[p.n_qscales == 1 ? 0 : img] : 0.f;
     const float q_scale_b = (fast && want_q) ? p.q_scales[p.n_qscales == 1 ? 0 : min(img + 1, p.n - 1)] : 0.f;
+    const bool q_only = MISHX && !ROWM && !p.out_f32 && want_q;      // the Mish's fp32 values go nowhere
     const bool q_even = p.n_qscales == 1;   // single-scale quantize rounds half to even in its bulk
     // the wavefront's dequantize scales and biases are read behind the K-loop; touching their lines now leaves them
     // in the caches by then (one load per array: 32 channels per fragment)
@@ -223,6 +234,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
     });
     asm volatile("; epilogue operands touched" ::"v"(touch));
 
+    if (MISHX) mish_tables.fill(tid);
     window_store(0);
     __syncthreads();
     int cb = 0, tap = 0, kc = 0, buf = 0;
@@ -446,7 +458,18 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
                         constexpr int r = decltype(rc)::value;
                         v[r] = __fadd_rn(v[r], res[j][r]);
                     });
-                    if (p.act == TSX_ACT_RELU) {
+                    const MishTablesInLds tables{&mish_tables};
+                    uint32_t word[4];        // requantized values, four consecutive channels to a word
+                    if (MISHX) {
+                        // (only layers with the exact Mish come here) nothing but the requantized values leaves: the exact
+                        // form only where it decides a rounding
+                        if (q_only) {
+                            if (EXTRA && p.residual && p.res_after) mish_words_for_rounding<true>(v, res[j], q_scale, q_even, word, tables);
+                            else mish_words_for_rounding<false>(v, res[j], q_scale, q_even, word, tables);
+                        } else {
+                            mish_fragment(v, tables);
+                        }
+                    } else if (p.act == TSX_ACT_RELU) {
                         static_for<0, 16>([&](auto rc) {
                             constexpr int r = decltype(rc)::value;
                             v[r] = v[r] > 0.f ? v[r] : 0.f;
@@ -456,18 +479,13 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
                             constexpr int r = decltype(rc)::value;
                             v[r] = apply_act_conv_i8(v[r], TSX_ACT_LEAKY_RELU, p.slope, true);
                         });
-                    } else if (MISHX && p.act == TSX_ACT_MISH) {
-                        // nothing but the requantized values leaves: the exact form only where it decides a rounding (the
-                        // largest tile has no registers left for it)
-                        if (NT < 7 && !ROWM && !p.out_f32 && want_q) mish_fragment_for_rounding(v, res[j], EXTRA && p.residual && p.res_after, q_scale);
-                        else mish_fragment(v);
                     } else if (p.act == TSX_ACT_MISH_FAST) {
                         static_for<0, 16>([&](auto rc) {
                             constexpr int r = decltype(rc)::value;
                             v[r] = apply_act_conv_i8(v[r], TSX_ACT_MISH_FAST, 0.f, true);
                         });
                     }
-                    if (EXTRA && p.residual && p.res_after) static_for<0, 16>([&](auto rc) {
+                    if (EXTRA && p.residual && p.res_after && !q_only) static_for<0, 16>([&](auto rc) {
                         constexpr int r = decltype(rc)::value;
                         v[r] = __fadd_rn(v[r], res[j][r]);
                     });
@@ -493,8 +511,9 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
                     if (!ROWM && want_q) {
                         // the 16 requantized values as 4 dwords of 4 consecutive channels (quantize_pack: the value of
                         // quantize_value, converted, clamped and packed by one instruction)
-                        uint32_t word[4] = {0u, 0u, 0u, 0u};
-                        if (q_even) static_for<0, 16>([&](auto rc) {
+                        if (!q_only) static_for<0, 4>([&](auto gc) { word[decltype(gc)::value] = 0; });
+                        if (q_only) {
+                        } else if (q_even) static_for<0, 16>([&](auto rc) {
                             constexpr int r = decltype(rc)::value;
                             word[r / 4] = quantize_pack<r % 4>(__fmul_rn(v[r], q_scale), true, word[r / 4]);
                         });
@@ -553,11 +572,21 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(NT <
                                           : (int64_t(img + (wrapped ? 1 : 0)) * p.cout + co0) * howo + oh * p.wo + ow;
                 const int64_t co_stride = ROWM ? 1 : howo;
                 const float rs = (ROWM && p.row_scale && pos_ok) ? p.row_scale[row0 + tr] : 0.f;
-                static_for<0, 16>([&](auto rc) {
+                if constexpr (EXTRA) {
+                    // a loop that stays one, like mish_fragment's: unrolled it is nine tenths of the kernel's code
+                    const v16i a = acc[f][j];
+                    v16f d, b;
+                    static_for<0, 16>([&](auto rc) { d[decltype(rc)::value] = dq[decltype(rc)::value], b[decltype(rc)::value] = bias[decltype(rc)::value]; });
+#pragma clang loop unroll(disable)
+                    for (int r = 0; r < 16; ++r) {
+                        const int dco = 8 * (r / 4) + (r % 4);
+                        if (pos_ok && co0 + dco < p.cout) emit<MISHX>(p, a[r], base + int64_t(dco) * co_stride, d[r], b[r], rs);
+                    }
+                } else static_for<0, 16>([&](auto rc) {
                     constexpr int r = decltype(rc)::value;
                     constexpr int dco = 8 * (r / 4) + (r % 4);
                     if (pos_ok && co0 + dco < p.cout)
-                        emit<MISHX>(p, acc[f][j][r], base + int64_t(dco) * co_stride, dq[r], bias[r], rs);
+                        emit<false>(p, acc[f][j][r], base + int64_t(dco) * co_stride, dq[r], bias[r], rs);
                 });
             });
         }

@@ -7,6 +7,7 @@ namespace tsx {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 
 struct EpiParams {
     const float *dq, *row_scale, *bias, *q_scales;
@@ -28,13 +29,16 @@ struct EpiParams {
 
 // Division of a non-negative n by a uniform divisor d as one multiply-high: magic = ceil(2^32 / d) gives
 // floor(n / d) = mulhi(n, magic) whenever n * d <= 2^32.  0 = no magic number (d = 1, or n_max too large): the
-// kernel then divides.
+// kernel then takes n itself, or divides (some thirty instructions: the tiles of 1x1 layers, one pixel wide, spent a third
+// of a wavefront's vector instructions on divisions by 1).
 inline unsigned div_magic(int d, int64_t n_max) {
     if (d <= 1 || n_max * d > (int64_t(1) << 32)) return 0u;
     return unsigned(((uint64_t(1) << 32) + unsigned(d) - 1) / unsigned(d));
 }
 #ifdef __HIPCC__
-__device__ __forceinline__ int udiv(int n, int d, unsigned magic) { return magic ? int(__umulhi(unsigned(n), magic)) : n / d; }
+__device__ __forceinline__ int udiv(int n, int d, unsigned magic) {
+    return magic ? int(__umulhi(unsigned(n), magic)) : d == 1 ? n : n / d;
+}
 #endif
 
 // fp32 value of one accumulator after dequant -> row scale -> bias -> residual -> activation;
@@ -91,10 +95,9 @@ __device__ __forceinline__ void emit(const EpiParams &p, int acc, int64_t idx, f
 // output, every element in the activation's SIMD-body range, one quantize scale for this lane's
 // image (q_scale, rounding half to even iff q_even).  st_dst = the lane's pixel in the consumer's
 // staged layout at its first channel row, or null.
-template <bool MISHX = true>
 __device__ __forceinline__ void epilogue_rows16(const EpiParams &p, const v16i &acc, const float (&dq)[16],
                                                 const float (&bias)[16], int64_t idx0, int64_t row_stride, float q_scale,
-                                                bool q_even, int8_t *st_dst) {
+                                                bool q_even, int8_t *st_dst, const MishTablesInLds &tables) {
     float v[16];
     static_for<0, 16>([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fmul_rn(float(acc[r]), dq[r]); });
     if (p.bias) {
@@ -110,21 +113,24 @@ __device__ __forceinline__ void epilogue_rows16(const EpiParams &p, const v16i &
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = __fadd_rn(v[r], res[r]);
     }
+    const bool q_only = p.act == TSX_ACT_MISH && !p.out_f32 && (p.out_i8 || st_dst);      // the Mish's fp32 values go nowhere
+    uint32_t word[4] = {0u, 0u, 0u, 0u};        // requantized values
     if (p.act == TSX_ACT_RELU) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = v[r] > 0.f ? v[r] : 0.f;
     } else if (p.act == TSX_ACT_LEAKY_RELU) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = apply_act_conv_i8(v[r], TSX_ACT_LEAKY_RELU, p.slope, true);
-    } else if (MISHX && p.act == TSX_ACT_MISH) {
+    } else if (p.act == TSX_ACT_MISH) {
         // nothing but the requantized values leaves: the exact form only where it decides a rounding
-        if (!p.out_f32 && (p.out_i8 || st_dst)) mish_fragment_for_rounding(v, res, p.residual && p.res_after, q_scale);
-        else mish_fragment(v);
+        if (!q_only) mish_fragment(v, tables);
+        else if (p.residual && p.res_after) mish_words_for_rounding<true>(v, res, q_scale, q_even, word, tables);
+        else mish_words_for_rounding<false>(v, res, q_scale, q_even, word, tables);
     } else if (p.act == TSX_ACT_MISH_FAST) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = apply_act_conv_i8(v[r], TSX_ACT_MISH_FAST, 0.f, true);
     }
-    if (p.residual && p.res_after) {
+    if (p.residual && p.res_after && !q_only) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = __fadd_rn(v[r], res[r]);
     }
@@ -133,23 +139,25 @@ __device__ __forceinline__ void epilogue_rows16(const EpiParams &p, const v16i &
         for (int r = 0; r < 16; ++r) p.out_f32[idx0 + int64_t(8 * (r / 4) + (r % 4)) * row_stride] = v[r];
     }
     if (p.out_i8 || st_dst) {
-        int qv[16];
-        if (q_even) {
+        if (q_only) {
+        } else if (q_even) static_for<0, 16>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            word[r / 4] = quantize_pack<r % 4>(__fmul_rn(v[r], q_scale), true, word[r / 4]);
+        });
+        else static_for<0, 16>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            word[r / 4] = quantize_pack<r % 4>(__fmul_rn(v[r], q_scale), false, word[r / 4]);
+        });
 #pragma unroll
-            for (int r = 0; r < 16; ++r) qv[r] = quantize_value(__fmul_rn(v[r], q_scale), true);
-        } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) qv[r] = quantize_value(__fmul_rn(v[r], q_scale), false);
-        }
+        for (int g4 = 0; g4 < 4; ++g4) word[g4] ^= 0x80808080u;
         if (p.out_i8) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) p.out_i8[idx0 + int64_t(8 * (r / 4) + (r % 4)) * row_stride] = int8_t(qv[r]);
+            for (int r = 0; r < 16; ++r) p.out_i8[idx0 + int64_t(8 * (r / 4) + (r % 4)) * row_stride] = int8_t(word[r / 4] >> (8 * (r % 4)));
         }
         if (st_dst) {
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
-                const uint32_t w = uint32_t(qv[4 * g4] & 0xff) | (uint32_t(qv[4 * g4 + 1] & 0xff) << 8) |
-                                   (uint32_t(qv[4 * g4 + 2] & 0xff) << 16) | (uint32_t(qv[4 * g4 + 3] & 0xff) << 24);
+                const uint32_t w = word[g4];
                 *reinterpret_cast<uint32_t *>(st_dst + 8 * g4) = w;
                 if (p.st_up == 2) {   // st_dst is staged pixel (2 oh, 2 ow): the other three of the 2 x 2 block
                     *reinterpret_cast<uint32_t *>(st_dst + p.st_cp + 8 * g4) = w;

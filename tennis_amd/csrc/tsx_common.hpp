@@ -116,17 +116,20 @@ __device__ __forceinline__ float apply_act_basic(float v, int act, float slope, 
 // The fast form for layers bound by the activation's arithmetic (the 608x608 and 304x304 layers of a YOLOv4-shaped
 // backbone spend more issue slots on an exact Mish than the VALUs have in the time the layer's bytes take): one
 // exponential and one reciprocal at the hardware's 1 ulp,
-//     tanh(softplus(x)) = w / (w + 2) = 1 - 2 / (w + 2),  w = e (e + 2),  e = e^x = 2^(x log2 e),
-// 14 issue slots.  1 - 2r with r = 1 / (w + 2) in (0, 0.5] has the shape of the host's tanh: an absolute error of about
-// 1e-7 in the quotient, so about 1e-7 |x| in the result (at most 2e-6 absolute for negative x, where Mish itself is
-// small) -- and, like the host's, exactly 0 (-0 for the product) once x is below about -17, where w + 2 rounds to 2.
+//     tanh(softplus(x)) = 1 - 2 / (w + 2),  w = e (e + 2),  e = e^x = 2^(x log2 e),
+// with -2 / (w + 2) as the reciprocal of -(e (e/2 + 1) + 1): five operations and the two transcendental ones (an issue slot
+// of four cycles and ten cycles each).  1 - 2r with r = 1 / (w + 2) in (0, 0.5] has the shape of the host's tanh: an absolute
+// error of about 1e-7 in the quotient, so about 1e-7 |x| in the result (at most 2e-6 absolute for negative x, where Mish
+// itself is small) -- and, like the host's, exactly 0 (-0 for the product) once x is below about -17, where the divisor
+// rounds to 1; 1 above 17, also where e^x or its square overflow.
 // NaN -> NaN, +-inf as the host's.  A requantized int8 value differs from the exact form's in about one of a million.
 // Opt-in (TSX_ACT_MISH_FAST); TSX_ACT_MISH is the exact form, mish_value.
+__device__ __forceinline__ float mish_minus_quotient(float x) {      // -2 / (w + 2)
+    const float e = __builtin_amdgcn_exp2f(__fmul_rn(x, 1.4426950216293335f));
+    return __builtin_amdgcn_rcpf(__builtin_fmaf(e, __builtin_fmaf(e, -0.5f, -1.f), -1.f));
+}
 __device__ __forceinline__ float mish_short(float x) {
-    const float e = __builtin_amdgcn_exp2f(__fmul_rn(fminf(x, 30.f), 1.4426950216293335f));   // beyond 30 the quotient is 1
-    const float d = __builtin_fmaf(e, __fadd_rn(e, 2.f), 2.f);
-    const float t = __builtin_fmaf(-2.f, __builtin_amdgcn_rcpf(d), 1.f);
-    return __fmul_rn(x, t);
+    return __fmul_rn(x, __fadd_rn(1.f, mish_minus_quotient(x)));
 }
 
 // The activation of every epilogue: none / relu / leaky_relu / Mish (exact) / Mish (fast).  One function for all
@@ -137,26 +140,23 @@ __device__ __forceinline__ float apply_act(float v, int act, float slope, bool i
     if (act == TSX_ACT_MISH_FAST) return mish_short(v);
     return apply_act_basic(v, act, slope, in_body);
 }
-// The tables of the exact Mish held by the wavefront itself: lane l keeps entry l % 32 of the host's expf in two registers and
-// entry l of the logarithm's in three, and a look-up is two or three cross-lane reads (ds_bpermute) instead of a gather from
-// memory -- three times per Mish value, in the middle of its dependent chain.  Every lane must be active where it is used.
-struct Exp2fTableInLanes {
-    int lo, hi, inv, log_lo, log_hi;
-    __device__ __forceinline__ explicit Exp2fTableInLanes(int lane) {
-        const uint64_t mine = exp2f_table[lane & 31], log_mine = bits_of_f64(log_of_interval[lane & 63]);
-        lo = int(uint32_t(mine));
-        hi = int(uint32_t(mine >> 32));
-        inv = __float_as_int(log_inverse[lane & 63]);
-        log_lo = int(uint32_t(log_mine));
-        log_hi = int(uint32_t(log_mine >> 32));
+// The tables of the exact Mish in the workgroup's LDS: the 32 entries of the exponential's take two banks each, so a read of
+// any 64 of them is free of conflicts.  (Held in the wavefront's lanes and read with ds_bpermute, a look-up takes 28 cycles
+// of a SIMD's share of the LDS pipe per 32 bits: seven of them were as long as the arithmetic.)
+struct MishTables {
+    uint64_t exp2[32];
+    double inverse[64], log_of[64];
+    __device__ __forceinline__ void fill(int tid) {       // by at least 160 threads, in front of a barrier
+        if (tid < 32) exp2[tid] = exp2f_table[tid];
+        else if (tid < 96) inverse[tid - 32] = double(log_inverse[tid - 32]);
+        else if (tid < 160) log_of[tid - 96] = log_of_interval[tid - 96];
     }
-    __device__ __forceinline__ static uint64_t read(int addr, int lo, int hi) {
-        return uint64_t(uint32_t(__builtin_amdgcn_ds_bpermute(addr, lo))) |
-               (uint64_t(uint32_t(__builtin_amdgcn_ds_bpermute(addr, hi))) << 32);
-    }
-    __device__ __forceinline__ uint64_t operator()(uint64_t i) const { return read(int(i) * 4, lo, hi); }
-    __device__ __forceinline__ float inverse(int i) const { return __int_as_float(__builtin_amdgcn_ds_bpermute(i * 4, inv)); }
-    __device__ __forceinline__ double log_of(int i) const { return f64_of_bits(read(i * 4, log_lo, log_hi)); }
+};
+struct MishTablesInLds {
+    const MishTables *t;
+    __device__ __forceinline__ uint64_t exp2(uint32_t i) const { return t->exp2[i]; }
+    __device__ __forceinline__ double inverse(int i) const { return t->inverse[i]; }
+    __device__ __forceinline__ double log_of(int i) const { return t->log_of[i]; }
 };
 
 // The exact Mish of the 16 values of an accumulator fragment, two values per turn of a loop that stays a loop: each
@@ -164,55 +164,82 @@ struct Exp2fTableInLanes {
 // side would push a kernel that keeps its accumulators and operands in registers into scratch memory; two give the
 // scheduler something to put into the other's latencies.  The loop counter is uniform: the values are reached by
 // register indexing.
-__device__ __forceinline__ void mish_fragment(float (&v)[16]) {
+template <class Table>
+__device__ __forceinline__ void mish_fragment(float (&v)[16], const Table &table) {
     typedef float v16f __attribute__((ext_vector_type(16)));
     v16f t;
 #pragma unroll
     for (int r = 0; r < 16; ++r) t[r] = v[r];
-    if (__builtin_amdgcn_ballot_w64(true) == ~0ull) {
-        const Exp2fTableInLanes table(int(threadIdx.x));
 #pragma clang loop unroll(disable)
-        for (int r = 0; r < 16; r += 2) {
-            const float a = mish_value(t[r], table), b = mish_value(t[r + 1], table);
-            t[r] = a;
-            t[r + 1] = b;
-        }
-    } else {
-#pragma clang loop unroll(disable)
-        for (int r = 0; r < 16; ++r) t[r] = mish_value(t[r]);
+    for (int r = 0; r < 16; r += 2) {
+        const float a = mish_value(t[r], table), b = mish_value(t[r + 1], table);
+        t[r] = a;
+        t[r + 1] = b;
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) v[r] = t[r];
 }
 
-// The exact Mish where only a requantized int8 value leaves the kernel: round((mish(x) [+ add]) * scale) has to be
-// the exact form's, the float in between does not.  mish_short is within 5.21 * 2^-24 |x| of mish_value for every
-// float x (all 2^32 inputs compared on the device, tests/test_gpu_yolo.py), so wherever the short form's product
-// lies further from a rounding boundary k + 1/2 than that bound (taken as 8 * 2^-24 |x scale|, plus 2^-21 of the
-// product for the two float roundings behind the activation) both forms round to the same integer.  The few values
-// that lie closer -- about one in ten thousand -- are evaluated again by the exact chain, a wavefront at a time and
-// only where a lane asks.  Values in v: pre-activation in, mish out (exact where it matters).
-__device__ __forceinline__ void mish_fragment_for_rounding(float (&v)[16], const float (&add)[16], bool with_add, float scale) {
+// The exact Mish where only requantized int8 values leave the kernel: round((mish(x) [+ add]) * scale) has to be the exact
+// form's, the float in between does not.  A short form, x - 2x / (w + 2) as one fused multiply-add behind mish_short's
+// reciprocal, is within 6 * 2^-24 |x| of mish_value for every float x (mish_short is, by comparing all 2^32 inputs on the
+// device, tests/test_gpu_yolo.py; its own two roundings are 2^-24 |x| of that), so with t = the short form's product with the scale + 128
+// both forms round to the same integer wherever t lies further from a rounding boundary k + 1/2 than
+// 2^-20 |x scale| + 2^-16, or, with an addend, 2^-20 |x scale| + 2^-21 |t| + 2^-14: the bound and the roundings of sum, product
+// and t, each at most 2^-24 of what it rounds.  There the conversion to a byte, which rounds and saturates to [0, 255], gives the value of
+// quantize_value + 128 whatever its rule for ties.  The few values that lie closer -- about one in ten thousand, and every
+// one whose product is large, infinite or NaN -- are evaluated again by the exact chain, a wavefront at a time and only
+// where a lane asks; eleven operations and the two transcendental ones a value otherwise.
+// word: the 16 values as offset binary (^ 0x80808080 makes them int8), four to a word.
+template <bool WITH_ADD, class Table>
+__device__ __forceinline__ void mish_words_for_rounding(const float (&v)[16], const float (&add)[16], float scale, bool half_even,
+                                                        uint32_t (&word)[4], const Table &table) {
     typedef float v16f __attribute__((ext_vector_type(16)));
-    v16f x, m;
-    unsigned near = 0;
+    typedef unsigned v4u __attribute__((ext_vector_type(4)));
+    const float per_x = __builtin_fabsf(__fmul_rn(scale, 0x1p-20f));
+    auto product = [&](float x, float a) __attribute__((always_inline)) {
+        const float m = __builtin_fmaf(x, mish_minus_quotient(x), x);
+        return __builtin_fmaf(WITH_ADD ? __fadd_rn(m, a) : m, scale, 128.f);
+    };
+    auto is_near = [&](float x, float t) __attribute__((always_inline)) {
+        float margin = __builtin_fmaf(__builtin_fabsf(x), per_x, WITH_ADD ? 0x1p-14f : 0x1p-16f);
+        if (WITH_ADD) margin = __builtin_fmaf(__builtin_fabsf(t), 0x1p-21f, margin);
+        return !(__builtin_fabsf(__fsub_rn(__builtin_amdgcn_fractf(t), 0.5f)) > margin);      // NaN and infinity: near
+    };
+    unsigned groups = 0;       // words that hold such a value, by wavefront
+    static_for<0, 4>([&](auto gc) {
+        constexpr int g = decltype(gc)::value;
+        bool any = false;
+        word[g] = 0;
+        static_for<0, 4>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            const float t = product(v[4 * g + j], add[4 * g + j]);
+            any |= is_near(v[4 * g + j], t);
+            word[g] = __builtin_amdgcn_cvt_pk_u8_f32(t, j, word[g]);
+        });
+        groups |= __builtin_amdgcn_ballot_w64(any) != 0 ? 1u << g : 0u;
+    });
+    if (groups != 0) {
+        v16f x, a;
+        v4u w;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        x[r] = v[r];
-        m[r] = mish_short(v[r]);
-        const float sum = with_add ? __fadd_rn(m[r], add[r]) : m[r];
-        const float a = __builtin_fabsf(__fmul_rn(sum, scale));
-        const float dist = __builtin_fabsf(__fsub_rn(__fsub_rn(a, __builtin_floorf(a)), 0.5f));
-        const float margin = __builtin_fmaf(__builtin_fabsf(__fmul_rn(v[r], scale)), 0x1p-21f, __builtin_fmaf(a, 0x1p-21f, 1e-30f));
-        near |= dist > margin ? 0u : 1u << r;      // NaN and infinity: near
-    }
-    if (__builtin_amdgcn_ballot_w64(near != 0) != 0) {
+        for (int r = 0; r < 16; ++r) x[r] = v[r], a[r] = WITH_ADD ? add[r] : 0.f;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) w[g] = word[g];
 #pragma clang loop unroll(disable)
-        for (int r = 0; r < 16; ++r)
-            if ((near >> r) & 1u) m[r] = mish_value(x[r]);
-    }
+        for (int r = 0; r < 16; ++r) {
+            if (!((groups >> (r >> 2)) & 1u)) continue;
+            const float xr = x[r], ar = a[r];
+            if (is_near(xr, product(xr, ar))) {
+                const float m = mish_value(xr, table);
+                const int q = quantize_value(__fmul_rn(WITH_ADD ? __fadd_rn(m, ar) : m, scale), half_even);
+                const int shift = 8 * (r & 3);
+                w[r >> 2] = (w[r >> 2] & ~(255u << shift)) | (unsigned(q + 128) << shift);
+            }
+        }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = m[r];
+        for (int g = 0; g < 4; ++g) word[g] = w[g];
+    }
 }
 
 __device__ __forceinline__ float apply_act_conv_i8(float v, int act, float slope, bool in_body) {

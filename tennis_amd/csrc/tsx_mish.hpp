@@ -73,10 +73,10 @@ TSX_MISH_FN float div_rn(float a, float b) { return __fdiv_rn(a, b); }   // IEEE
 TSX_MISH_FN float div_rn(float a, float b) { return a / b; }
 #endif
 // where expf_host finds 2^(i/32), and log_precise its interval: these tables in memory, or whatever holds a copy of them (on
-// the device, the lanes of the wavefront)
-struct Exp2fTableInMemory {
-    TSX_MISH_MEMBER uint64_t operator()(uint64_t i) const { return exp2f_table[i]; }
-    TSX_MISH_MEMBER float inverse(int i) const { return log_inverse[i]; }
+// the device, the workgroup's LDS)
+struct MishTablesInMemory {
+    TSX_MISH_MEMBER uint64_t exp2(uint32_t i) const { return exp2f_table[i]; }
+    TSX_MISH_MEMBER double inverse(int i) const { return double(log_inverse[i]); }
     TSX_MISH_MEMBER double log_of(int i) const { return log_of_interval[i]; }
 };
 
@@ -88,42 +88,44 @@ TSX_MISH_FN uint64_t bits_of_f64(double d) { uint64_t u; __builtin_memcpy(&u, &d
 // early returns -- inf, 0, the largest and smallest finite results beyond |x| of 88 -- come out of the same
 // arithmetic on the clamped argument: the double result overflows or underflows the float conversion as the host's
 // special cases say.  NaN -> NaN.
-template <class Table = Exp2fTableInMemory>
-TSX_MISH_FN float expf_host(float x, const Table &table = Table()) {
-    const double xd = double(__builtin_fminf(__builtin_fmaxf(x, -150.f), 89.f));
-    const double z = 0x1.71547652b82fep+5 * xd;          // x * 32 / ln2
+// exp2_of_32nds: the body of it, from z = x * 32 / ln2, for arguments whose result neither overflows nor needs the clamp.
+template <class Table = MishTablesInMemory>
+TSX_MISH_FN float exp2_of_32nds(double z, const Table &table = Table()) {
     double kd = z + 0x1.8p+52;                           // the integer nearest to z, in the low mantissa bits
     const uint64_t ki = bits_of_f64(kd);
     kd -= 0x1.8p+52;
     const double r = z - kd;
-    const double s = f64_of_bits(table(ki & 31) + (ki << 47));
+    const double s = f64_of_bits(table.exp2(uint32_t(ki) & 31) + (ki << 47));
     const double c = __builtin_fma(0x1.c6af84b912394p-5 / 32768.0, r, 0x1.ebfce50fac4f3p-3 / 1024.0);
     const double r2 = r * r;
     double y = __builtin_fma(0x1.62e42ff0c52d6p-1 / 32.0, r, 1.0);
     y = __builtin_fma(c, r2, y);
-    const float e = float(y * s);
+    return float(y * s);
+}
+template <class Table = MishTablesInMemory>
+TSX_MISH_FN float expf_host(float x, const Table &table = Table()) {
+    const double xd = double(__builtin_fminf(__builtin_fmaxf(x, -150.f), 89.f));
+    const float e = exp2_of_32nds(0x1.71547652b82fep+5 * xd, table);
     return x != x ? x : e;
 }
 
 // log(s) for a finite double s >= 1, to under 2^-50 relative: s = 2^k m with m in [1, 2), m = (1 + r) / c with the c of m's
-// interval, |r| < 2^-6, log s = k ln2 - log c + log(1 + r), the last as its series up to r^9 / 9.  Rounded to float it is what
-// the host's log gives rounded to float: both are far inside half a float ulp of the exact value.  (Without the table, by
-// atanh((m - 1) / (m + 1)), it is a double division and eleven terms: 45 issue slots instead of 20 of the chain's 127.)
-template <class Table = Exp2fTableInMemory>
+// interval, -0.0077 < r <= 2^-6, log s = k ln2 - log c + log(1 + r), the last as r + r^2 p(r) with p the polynomial through
+// (log(1 + r) - r) / r^2 at that interval's Chebyshev nodes (2^-52.6 of log(1 + r)).  Rounded to float it is what
+// the host's log gives rounded to float: both are far inside half a float ulp of the exact value.
+template <class Table = MishTablesInMemory>
 TSX_MISH_FN double log_precise(double s, const Table &table = Table()) {
     const uint64_t ix = bits_of_f64(s);
     const uint32_t hi = uint32_t(ix >> 32);
     const int i = int(hi >> 14) & 63;
     const double m = f64_of_bits((uint64_t((hi & 0xfffffu) | 0x3ff00000u) << 32) | uint32_t(ix));
-    const double r = __builtin_fma(m, double(table.inverse(i)), -1.0);
-    double p = 1.0 / 9;
-    p = __builtin_fma(p, r, -1.0 / 8);
-    p = __builtin_fma(p, r, 1.0 / 7);
-    p = __builtin_fma(p, r, -1.0 / 6);
-    p = __builtin_fma(p, r, 1.0 / 5);
-    p = __builtin_fma(p, r, -1.0 / 4);
-    p = __builtin_fma(p, r, 1.0 / 3);
-    p = __builtin_fma(p, r, -1.0 / 2);
+    const double r = __builtin_fma(m, table.inverse(i), -1.0);
+    double p = 0x1.1e976e180c123p-3;
+    p = __builtin_fma(p, r, -0x1.55535716b7ee6p-3);
+    p = __builtin_fma(p, r, 0x1.9999ba4316280p-3);
+    p = __builtin_fma(p, r, -0x1.0000000acd4cep-2);
+    p = __builtin_fma(p, r, 0x1.55555555413c3p-2);
+    p = __builtin_fma(p, r, -0x1.fffffffffffabp-2);
     const double lm = __builtin_fma(r * r, p, r);
     const double kd = double(int(hi >> 20) - 1023);
     // k ln2, ln2 in two parts
@@ -131,25 +133,45 @@ TSX_MISH_FN double log_precise(double s, const Table &table = Table()) {
 }
 
 // cpu::Softplus (src/kernels/cpu/softplus.cpp:30-39): float(log(double(expf(x)) + 1.0))
-template <class Table = Exp2fTableInMemory>
+template <class Table = MishTablesInMemory>
 TSX_MISH_FN float softplus_value(float x, const Table &table = Table()) {
     const double s = double(expf_host(x, table)) + 1.0;
-    // outside the condition: a table held by a wavefront's lanes is read by all of them
     const double l = log_precise(s, table);
     return s < __builtin_inf() ? float(l) : float(s);   // +inf and NaN pass through
 }
 
 // cpu::Tanh (src/kernels/cpu/tanh.cpp:14-23): T(2) * (T(1) / (T(1) + exp(-(T(2) * x)))) - T(1) in float
-template <class Table = Exp2fTableInMemory>
+template <class Table = MishTablesInMemory>
 TSX_MISH_FN float tanh_value(float y, const Table &table = Table()) {
     const float u = expf_host(-(2.f * y), table);
     const float q = div_rn(1.f, 1.f + u);
     return __builtin_fmaf(2.f, q, -1.f);   // 2q is exact: one rounding, fused or not
 }
 
-template <class Table = Exp2fTableInMemory>
+// 1 / d rounded to nearest for d in [1, 2]: no scaling is needed there, two Newton steps on the device's reciprocal (every d
+// compared with the division, tests/test_gpu_yolo.py: all of them are in the sweep over Mish's arguments).
+#ifdef __HIP_DEVICE_COMPILE__
+TSX_MISH_FN float reciprocal_rn_1_2(float d) {
+    const float a = __builtin_amdgcn_rcpf(d);
+    const float b = __builtin_fmaf(__builtin_fmaf(-d, a, 1.f), a, a);
+    return __builtin_fmaf(__builtin_fmaf(-d, b, 1.f), b, b);
+}
+#else
+TSX_MISH_FN float reciprocal_rn_1_2(float d) { return 1.f / d; }
+#endif
+
+// x * tanh_value(softplus_value(x)), the same bits without what the composition needs only at the ends of the float range:
+// below -20 the tangent is 0 and above 40 it is 1 whatever the argument, so the argument is clamped to these once (a NaN
+// too: the product with x makes it one again); the exponentials then neither overflow nor vanish, e^x + 1 is finite, and
+// the divisor 1 + e^(-2y) lies in [1, 2].  -2y * 32 / ln2 is the host's product, scaled by a power of two.  56 double- and
+// single-precision operations and four table reads, where the composition has 92 and (with tables in the lanes) seven.
+template <class Table = MishTablesInMemory>
 TSX_MISH_FN float mish_value(float x, const Table &table = Table()) {
-    return x * tanh_value(softplus_value(x, table), table);
+    const double xd = double(__builtin_fminf(__builtin_fmaxf(x, -20.f), 40.f));
+    const float e = exp2_of_32nds(0x1.71547652b82fep+5 * xd, table);
+    const float y = float(log_precise(double(e) + 1.0, table));
+    const float u = exp2_of_32nds(-0x1.71547652b82fep+6 * double(y), table);
+    return x * __builtin_fmaf(2.f, reciprocal_rn_1_2(1.f + u), -1.f);
 }
 
 }  // namespace tsx
