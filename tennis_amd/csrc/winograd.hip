@@ -276,56 +276,210 @@ __global__ __launch_bounds__(256) void wino23_input_transform_kernel(const float
 }
 
 // M_f = U_f V_f for every frequency, in the reference's accumulation order.  A wavefront computes 32 output channels x
-// FN fragments of columns; the four wavefronts of a workgroup take consecutive row fragments of the same columns (their V
+// FN fragments of columns; the wavefronts of a workgroup take consecutive row fragments of the same columns (their V
 // loads meet in L1).  Workgroups b, b + 8, ... run on one XCD: each XCD gets whole frequencies, whose U and V then
 // stay in its L2 (8 x 456 KB at 8 images of 28x28x256).  RING groups of 8 channels are in flight per wavefront.
-// Bound by the fp32 MFMA: 1.68 GFLOP at that shape = 11 us at 157 TFLOP/s.
-// It takes 26 .. 28 us there (the tail's
-// fragments hold 8 real columns of 32, and a wavefront's chain of 128 dependent MFMAs fills its SIMD 3.5 times over; MFMAs
-// are busy 58 % of the CUs' time); chains on the vector ALUs, one lane per 4 x 4 outputs, took 276 + 31 us.
+// Bound by the fp32 MFMA and by what a CU fetches besides: 1.68 GFLOP at that shape = 11 us at 157 TFLOP/s, 128 dependent MFMAs
+// per wavefront.  It takes 20 .. 21 us there with its launch, from 26 .. 28 at one wavefront per SIMD, whose addresses waited
+// for its MFMAs, and with the tail's 8 real columns computed as 32 (the whole convolution 41.5 -> 36.2 us; 16 images 112x112, 64 to 64
+// channels, F(6,3) 156 -> 113, F(2,3) 320 -> 220; 1 image 304x304, 16 to 32, 45 -> 27 and 72 -> 33).  Chains on the vector ALUs,
+// one lane per 4 x 4 outputs, took 276 + 31 us.
 constexpr int WG_RING = 4;
-constexpr int TAIL_RING = 4;
 
-template <int FN>
-__device__ __forceinline__ void wino_gemm_chain(const v4f *__restrict__ u, const v4f *__restrict__ v, float *__restrict__ m, const WinoGeom &g,
-                                                int f, int rf, int cf0, int lane) {
-    const int T = g.kgroups;
-    const v4f *ua = u + (int64_t(f) * g.rfrags + rf) * T * 64 + lane;
-    const v4f *vb[FN];
+// A fragment of U or V (T groups) as a buffer, and a lane's operand element in it.  Base and group are scalar, the lane's offset is
+// constant: an address that the vector ALUs compute per load goes to registers that MFMAs in the pipe still read, and waits for
+// them.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t fragment_buffer(const float *base, int64_t index, int T) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base) + index * T * 256, 0, T * 1024, 0x00020000);
+}
+__device__ __forceinline__ v4f fragment_element(__amdgpu_buffer_rsrc_t fragment, int lane_offset, int group_offset) {
+    return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(fragment, lane_offset, group_offset, 0));
+}
+
+// The four chains of the 32 x 16 outputs in s[row half] combined, and the channels left over chained behind them.
+__device__ __forceinline__ void wino_tail_store(const float *__restrict__ u, const float *__restrict__ v, float *__restrict__ m, const WinoGeom &g,
+                                                int f, int rf, int cf, int lane, const v16f (&s)[2]) {
+    const int T = g.kgroups, q = lane / 16, i = lane % 16, k4 = g.c / 4 * 4;
+    const int m8 = g.cout / 8 * 8;
+    float *dst = m + int64_t(f) * g.cout * g.cols + g.mfrags * 32 + cf * 16 + i;
+    // channels k4 .. c - 1, at most three: all their operands before the first use
+    float ul[3][2][4] = {}, vl[3] = {};
+    if (k4 < g.c)
 #pragma unroll
-    for (int n = 0; n < FN; ++n) vb[n] = v + (int64_t(f) * g.nfrags + min(cf0 + n, g.mfrags - 1)) * T * 64 + lane;
-    v4f a[WG_RING], b[FN][WG_RING];
-    v16f acc[FN];
+    for (int e = 0; e < 3; ++e) {
+        const int k = min(k4 + e, g.c - 1);
+        const int64_t at = int64_t(k / 8) * 256 + 128 * (k % 2) + k % 8 / 2;
+        vl[e] = v[(int64_t(f) * g.nfrags + g.mfrags + cf / 2) * T * 256 + at + 4 * (16 * (cf % 2) + i)];
 #pragma unroll
-    for (int n = 0; n < FN; ++n)
+        for (int r = 0; r < 8; ++r) ul[e][r / 4][r % 4] = u[(int64_t(f) * g.rfrags + rf) * T * 256 + at + 4 * (16 * (r / 4) + 4 * q + r % 4)];
+    }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[n][r] = 0.f;
-    auto load = [&](auto slot, int t) __attribute__((always_inline)) {
-        constexpr int s = decltype(slot)::value;
-        const int tt = min(t, T - 1);                        // beyond the last group: its lines again, never used
-        a[s] = ua[tt * 64];
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int n = 0; n < FN; ++n) b[n][s] = vb[n][tt * 64];
+        for (int r = 0; r < 4; ++r) {
+            const int row = rf * 32 + 16 * h + 4 * q + r;
+            const float s01 = s[h][r] + s[h][4 + r], s23 = s[h][8 + r] + s[h][12 + r];
+            float acc = row < m8 ? (0.f + s01) + s23 : (s01 + s[h][8 + r]) + s[h][12 + r];
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (k4 + e < g.c) acc = fmaf(ul[e][h][r], vl[e], acc);
+            if (row < g.cout) dst[int64_t(row) * g.cols] = acc;
+        }
+}
+
+// The tail columns: chains over k = q, q + 4, q + 8, ... (q = 0..3) up to k4 = k/4*4, their combination, then the up to
+// three channels left as a chain behind it.  v_mfma_f32_16x16x1_f32 is four blocks of 16 x 16 with one multiply-add per step
+// each: block q takes chain q, and a lane then holds all four chains of its outputs (accumulator 4 q + i of lane l: chain q,
+// row 4 (l / 16) + i, column l % 16).  A fragment is 32 rows x 16 columns, an image leaves at
+// most 7 columns here; a wavefront takes one, or two beside one another.
+template <int NC, int RING>
+__device__ __forceinline__ void wino_gemm_tail(const float *__restrict__ u, const float *__restrict__ v, float *__restrict__ m, const WinoGeom &g,
+                                               int f, int rf, int cf, int tails, int lane) {
+    const int T = g.kgroups, q = lane / 16, i = lane % 16;
+    // A lane loads the operand element (four channels of one parity) of its row, of the row sixteen further (+ 64 floats) and of
+    // its columns: the lower half-wave those of group 2 p, the upper of group 2 p + 1.  Chain q's channels 8t + q and 8t + 4 + q
+    // are floats q / 2 and q / 2 + 2 of both groups: a half-wave swap each.
+    // (The group is part of the lane's offset here: loads beyond the last one are then outside of the fragment's buffer.)
+    const auto ua = fragment_buffer(u, int64_t(f) * g.rfrags + rf, T);
+    const int row_at = 16 * (i + 32 * (q % 2)) + 1024 * (q / 2);
+    int column_at[NC];
+#pragma unroll
+    for (int n = 0; n < NC; ++n) column_at[n] = row_at + 256 * ((cf + n) % 2);
+    v16f s[NC][2];
+#pragma unroll
+    for (int n = 0; n < NC; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[n][0][r] = s[n][1][r] = 0.f;
+    const int steps = g.c / 4;                               // of four channels, one to a chain
+    v4f a[RING][2], b[RING][NC];                   // [slot][row half], [slot][columns]
+    auto load = [&](auto slot, int pair) __attribute__((always_inline)) {
+        constexpr int sl = decltype(slot)::value;
+        a[sl][0] = fragment_element(ua, row_at + pair * 2048, 0);
+        a[sl][1] = fragment_element(ua, row_at + 256 + pair * 2048, 0);
+#pragma unroll
+        for (int n = 0; n < NC; ++n)
+            b[sl][n] = fragment_element(fragment_buffer(v, int64_t(f) * g.nfrags + g.mfrags + min(cf + n, tails - 1) / 2, T), column_at[n] + pair * 2048, 0);
     };
-    auto multiply = [&](auto slot) __attribute__((always_inline)) {
-        constexpr int s = decltype(slot)::value;
+    auto split = [](const v4f &e, float (&of_step)[4]) __attribute__((always_inline)) {
+        const auto low = __builtin_amdgcn_permlane32_swap(__float_as_int(e[0]), __float_as_int(e[1]), false, false);
+        const auto high = __builtin_amdgcn_permlane32_swap(__float_as_int(e[2]), __float_as_int(e[3]), false, false);
+        of_step[0] = __int_as_float(low[0]);
+        of_step[1] = __int_as_float(high[0]);
+        of_step[2] = __int_as_float(low[1]);
+        of_step[3] = __int_as_float(high[1]);
+    };
+    auto multiply = [&](auto slot, int live) __attribute__((always_inline)) {      // the first `live` steps of the pair
+        constexpr int sl = decltype(slot)::value;
+        float ea[2][4], eb[NC][4];
+        split(a[sl][0], ea[0]);
+        split(a[sl][1], ea[1]);
+#pragma unroll
+        for (int n = 0; n < NC; ++n) split(b[sl][n], eb[n]);
+        static_for<0, 4>([&](auto ec) {
+            constexpr int e = decltype(ec)::value;
+            if (e < live) {
+#pragma unroll
+                for (int n = 0; n < NC; ++n)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) s[n][h] = __builtin_amdgcn_mfma_f32_16x16x1f32(ea[h][e], eb[n][e], s[n][h], 0, 0, 0);
+            }
+        });
+    };
+    static_for<0, RING - 1>([&](auto sc) {
+        load(sc, decltype(sc)::value);
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    int pair = 0;
+    for (; 4 * (pair + RING) <= steps; pair += RING)
+        static_for<0, RING>([&](auto sc) {
+            constexpr int sl = decltype(sc)::value;
+            load(std::integral_constant<int, (sl + RING - 1) % RING>{}, pair + sl + RING - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(sc, 4);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    // what is left: pairs of groups, the last perhaps of fewer steps
+    static_for<0, RING>([&](auto sc) {
+        constexpr int sl = decltype(sc)::value;
+        if constexpr (sl == RING - 1) load(sc, pair + sl);
+        multiply(sc, steps - 4 * (pair + sl));
+    });
+#pragma unroll
+    for (int n = 0; n < NC; ++n)
+        if (cf + n < tails) wino_tail_store(u, v, m, g, f, rf, cf + n, lane, s[n]);
+}
+
+// TAIL: and one fragment of 16 tail columns (see wino_gemm_tail) with them, whose rows are these.
+template <int FN, bool TAIL>
+__device__ __forceinline__ void wino_gemm_chain(const float *__restrict__ u, const float *__restrict__ v, float *__restrict__ m, const WinoGeom &g,
+                                                int f, int rf, int cf0, int tf, int lane) {
+    const int T = g.kgroups, q = lane / 16;
+    const auto ua = fragment_buffer(u, int64_t(f) * g.rfrags + rf, T), vt = fragment_buffer(v, int64_t(f) * g.nfrags + g.mfrags + tf / 2, T);
+    const int upper = q < 2 ? 0 : -1;                        // (bits selected: a choice between elements becomes an index)
+    const int at = lane * 16, at_tail = (16 * (tf % 2) + lane % 16 + 32 * (q % 2)) * 16;
+    v4f a[WG_RING], b[FN][WG_RING], bt[TAIL ? WG_RING : 1];
+    v16f acc[FN], s[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+#pragma unroll
+        for (int n = 0; n < FN; ++n) acc[n][r] = 0.f;
+        if (TAIL) s[0][r] = s[1][r] = 0.f;
+    }
+    const int full = g.c / 8, steps = g.c / 4;               // groups without padding; the tail's steps, two to a group
+    auto load = [&](auto slot, int t) __attribute__((always_inline)) {
+        constexpr int sl = decltype(slot)::value;
+        const int tt = min(t, T - 1) * 1024;                 // beyond the last group: its lines again, never used
+        a[sl] = fragment_element(ua, at, tt);
+#pragma unroll
+        for (int n = 0; n < FN; ++n) b[n][sl] = fragment_element(fragment_buffer(v, int64_t(f) * g.nfrags + min(cf0 + n, g.mfrags - 1), T), at, tt);
+        if constexpr (TAIL) bt[sl] = fragment_element(vt, at_tail, tt);
+    };
+    auto multiply = [&](auto slot, int live) __attribute__((always_inline)) {      // live: the tail's steps of this group
+        constexpr int sl = decltype(slot)::value;
+        // the tail's operands before the group's MFMAs: channels 8t + 4e + q of rows 0..15 and 16..31 are quarters of the
+        // operand, two swaps away
+        float rows[2][2], column[2];
+        if constexpr (TAIL) {
+            static_for<0, 2>([&](auto ec) {
+                constexpr int e = decltype(ec)::value;
+                const auto w = __builtin_amdgcn_permlane32_swap(__float_as_int(a[sl][2 * e]), __float_as_int(a[sl][2 * e + 1]), false, false);
+                const auto r = __builtin_amdgcn_permlane16_swap(w[0], w[1], false, false);
+                rows[e][0] = __int_as_float(r[0]);
+                rows[e][1] = __int_as_float(r[1]);
+                column[e] = __int_as_float((__float_as_int(bt[sl][2 * e]) & ~upper) | (__float_as_int(bt[sl][2 * e + 1]) & upper));
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        auto tail_step = [&](auto ec) __attribute__((always_inline)) {
+            constexpr int e = decltype(ec)::value;
+            if (TAIL && e < live)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) s[h] = __builtin_amdgcn_mfma_f32_16x16x1f32(rows[e][h], column[e], s[h], 0, 0, 0);
+        };
+        tail_step(std::integral_constant<int, 0>{});
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int n = 0; n < FN; ++n) acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s][j], b[n][s][j], acc[n], 0, 0, 0);
+            for (int n = 0; n < FN; ++n) acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[sl][j], b[n][sl][j], acc[n], 0, 0, 0);
+        tail_step(std::integral_constant<int, 1>{});
     };
-    static_for<0, WG_RING - 1>([&](auto sc) { load(sc, decltype(sc)::value); });
+    static_for<0, WG_RING - 1>([&](auto sc) {
+        load(sc, decltype(sc)::value);
+        __builtin_amdgcn_sched_barrier(0);                   // in the order of the loop's: what the loop waits for is counted
+    });
     int t = 0;
-    for (; t + WG_RING <= T; t += WG_RING)
+    for (; t + WG_RING <= full; t += WG_RING)                // (no condition in here: where paths meet the compiler waits for all of them)
         static_for<0, WG_RING>([&](auto sc) {
-            constexpr int s = decltype(sc)::value;
-            load(std::integral_constant<int, (s + WG_RING - 1) % WG_RING>{}, t + s + WG_RING - 1);
+            constexpr int sl = decltype(sc)::value;
+            load(std::integral_constant<int, (sl + WG_RING - 1) % WG_RING>{}, t + sl + WG_RING - 1);
             __builtin_amdgcn_sched_barrier(0);               // left alone the scheduler sinks the loads to where they are waited for
-            multiply(sc);
+            multiply(sc, 2);
             __builtin_amdgcn_sched_barrier(0);
         });
-    static_for<0, WG_RING - 1>([&](auto sc) {                // the groups left over are in the ring already
-        if (t + decltype(sc)::value < T) multiply(sc);
+    static_for<0, WG_RING>([&](auto sc) {                    // the groups left over, all but the last of four in the ring already
+        constexpr int sl = decltype(sc)::value;
+        if constexpr (sl == WG_RING - 1) load(sc, t + sl);
+        if (t + sl < T) multiply(sc, steps - 2 * (t + sl));
     });
 #pragma unroll
     for (int n = 0; n < FN; ++n) {
@@ -337,89 +491,34 @@ __device__ __forceinline__ void wino_gemm_chain(const v4f *__restrict__ u, const
             if (rf * 32 + row < g.cout) dst[int64_t(row) * g.cols] = acc[n][r];
         }
     }
+    if constexpr (TAIL) wino_tail_store(u, v, m, g, f, rf, tf, lane, s);
 }
 
-// The tail columns: chains over k = q, q + 4, q + 8, ... (q = 0..3) up to k4 = k/4*4, their combination, then the up to
-// three channels left as a chain behind it.  An MFMA step takes channels 8t + q and 8t + 4 + q: lanes of half H need
-// elements 2H, 2H + 1 of both half-lanes' operands, two 8-byte loads.
-__device__ __forceinline__ void wino_gemm_tail(const float *__restrict__ u, const float *__restrict__ v, float *__restrict__ m, const WinoGeom &g,
-                                               int f, int rf, int cf, int lane) {
-    const int T = g.kgroups, H = lane / 32;
-    const float *ua = u + operand_index(0, 1, 0, lane % 32, 2 * H) + (int64_t(f) * g.rfrags + rf) * T * 256;
-    const float *vb = v + operand_index(0, 1, 0, lane % 32, 2 * H) + (int64_t(f) * g.nfrags + cf) * T * 256;
-    v16f s[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[q][r] = 0.f;
-    const int k4 = g.c / 4 * 4, full = k4 / 8;
-    v2f a[TAIL_RING][2], b[TAIL_RING][2];                    // [slot][parity]
-    auto load = [&](auto slot, int t) __attribute__((always_inline)) {
-        constexpr int sl = decltype(slot)::value;
-        const int64_t off = int64_t(min(t, T - 1)) * 256;
-#pragma unroll
-        for (int par = 0; par < 2; ++par) {
-            a[sl][par] = *reinterpret_cast<const v2f *>(ua + off + par * 128);
-            b[sl][par] = *reinterpret_cast<const v2f *>(vb + off + par * 128);
-        }
-    };
-    auto multiply = [&](auto slot, bool live) __attribute__((always_inline)) {
-        constexpr int sl = decltype(slot)::value;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            s[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(live ? a[sl][q % 2][q / 2] : -0.f, live ? b[sl][q % 2][q / 2] : 0.f, s[q], 0, 0, 0);
-    };
-    static_for<0, TAIL_RING - 1>([&](auto sc) { load(sc, decltype(sc)::value); });
-    int t = 0;
-    for (; t + TAIL_RING <= full; t += TAIL_RING)
-        static_for<0, TAIL_RING>([&](auto sc) {
-            constexpr int sl = decltype(sc)::value;
-            load(std::integral_constant<int, (sl + TAIL_RING - 1) % TAIL_RING>{}, t + sl + TAIL_RING - 1);
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(sc, true);
-            __builtin_amdgcn_sched_barrier(0);
-        });
-    // the groups left over, and behind them one whose upper four channels are not chained
-    static_for<0, TAIL_RING>([&](auto sc) {
-        constexpr int sl = decltype(sc)::value;
-        if constexpr (sl == TAIL_RING - 1) load(sc, t + sl);
-        if (t + sl < full) multiply(sc, true);
-        else if (t + sl == full && k4 % 8) multiply(sc, H == 0);
-    });
-    v16f acc;
-    const int m8 = g.cout / 8 * 8;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int row = rf * 32 + 8 * (r / 4) + 4 * H + r % 4;
-        const float s01 = s[0][r] + s[1][r], s23 = s[2][r] + s[3][r];
-        acc[r] = row < m8 ? (0.f + s01) + s23 : (s01 + s[2][r]) + s[3][r];
-    }
-    for (int k = k4; k < g.c; k += 2) {                      // channels k and k + 1, one per half
-        const int kk = k + H, at = kk / 8 * 256 + (kk % 2) * 128 + (kk % 8) / 2 - 2 * H;
-        const bool live = kk < g.c;
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(live ? ua[live ? at : 0] : -0.f, live ? vb[live ? at : 0] : 0.f, acc, 0, 0, 0);
-    }
-    float *dst = m + (int64_t(f) * g.cout + rf * 32) * g.cols + cf * 32 + lane % 32;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int row = 8 * (r / 4) + 4 * H + r % 4;
-        if (rf * 32 + row < g.cout) dst[int64_t(row) * g.cols] = acc[r];
-    }
-}
-
-// A launch takes the column blocks from `first` on, of col_blocks blocks of FN fragments and, behind them, the tail's fragments.
+// A workgroup's wavefronts are wr row fragments x wc column blocks of FN fragments.  Items are, per XCD and counted from `first`:
+// row blocks of col_items of its frequencies, one frequency after the other.  The tail's fragments of 16 go with the first column
+// blocks, one each (`attached`), or follow as items of their own, two fragments each.
+// Registers for two (FN = 4) or four wavefronts per SIMD (the compiler's own choice, 267, left one).
 template <int FN>
-__global__ __launch_bounds__(256) void wino_gemm_kernel(const float *__restrict__ u, const float *__restrict__ v, float *__restrict__ m, WinoGeom g,
-                                                       int row_blocks, int col_blocks, int first) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FN == 1 ? 4 : 2))) void wino_gemm_kernel(
+    const float *__restrict__ u, const float *__restrict__ v, float *__restrict__ m, WinoGeom g, int wr, int wc, int row_blocks, int col_blocks,
+    int tails, int attached, int rounds, int64_t first) {
     const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const int f = (blockIdx.x & 7) + 8 * blockIdx.y;         // frequencies are a multiple of 8, so is a row of the grid
-    const int item = blockIdx.x >> 3, cb = first + item / row_blocks;
-    const int rf = (item % row_blocks) * 4 + wave;
-    if (rf >= g.rfrags) return;
-    if (cb < col_blocks)
-        wino_gemm_chain<FN>(reinterpret_cast<const v4f *>(u), reinterpret_cast<const v4f *>(v), m, g, f, rf, cb * FN, lane);
-    else
-        wino_gemm_tail(u, v, m, g, f, rf, g.mfrags + cb - col_blocks, lane);
+    const int tail_blocks = attached ? 0 : (tails + 1) / 2, col_items = (col_blocks + wc - 1) / wc, tail_items = (tail_blocks + wc - 1) / wc;
+    const int64_t item = first + (blockIdx.x >> 3), chains = int64_t(rounds) * col_items * row_blocks;
+    const bool tail = item >= chains;
+    const int64_t at = tail ? item - chains : item;
+    const int per_f = row_blocks * (tail ? tail_items : col_items), round = int(at / per_f), rest = int(at - int64_t(round) * per_f);
+    const int f = (blockIdx.x & 7) + 8 * round;              // frequencies are a multiple of 8
+    const int ci = rest / row_blocks, cb = ci * wc + wave / wr, rf = (rest - ci * row_blocks) * wr + wave % wr;
+    if (rf >= g.rfrags || wave >= wr * wc || cb >= (tail ? tail_blocks : col_blocks)) return;
+    if (tail) {
+        if (tails == 1) wino_gemm_tail<1, 4>(u, v, m, g, f, rf, 0, tails, lane);
+        else wino_gemm_tail<2, 3>(u, v, m, g, f, rf, cb * 2, tails, lane);
+    } else if (attached && cb < tails) {
+        wino_gemm_chain<FN, true>(u, v, m, g, f, rf, cb * FN, cb, lane);
+    } else {
+        wino_gemm_chain<FN, false>(u, v, m, g, f, rf, cb * FN, 0, lane);
+    }
 }
 
 // Y = A^T M A of F(6,3), cut to the true output, then the optional add_bias / activation that follow the convolution in
@@ -593,17 +692,28 @@ int conv2d(const tsx_conv2d_geom *q, const float *x, const float *u, float paddi
                            g, v);
     TSX_LAUNCH_CHECK("wino_input_transform_kernel");
 
-    // two column fragments per wavefront halve the loads of U; a layer that fills the SIMDs less than twice that way takes one
-    // fragment each (8 images of 28x28x256: 41.9 us against 43.8)
-    const int row_blocks = (g.rfrags + 3) / 4, tails = g.nfrags - g.mfrags;
-    const bool two = int64_t(FREQS) * g.rfrags * ((g.mfrags + 1) / 2) >= 2048;
-    const int col_blocks = two ? (g.mfrags + 1) / 2 : g.mfrags;
+    // Wavefronts of a workgroup: as many as there are row fragments along these, the others along columns where the grid is large
+    // enough to fill the CUs with what is left.
+    const int rounds = FREQS / 8, wr = g.rfrags >= 3 ? 4 : g.rfrags, row_blocks = (g.rfrags + wr - 1) / wr;
+    const int64_t frag_items = int64_t(FREQS) * row_blocks * g.mfrags;
+    const int wc = frag_items > 512 ? 4 / wr : 1, tails = int(ceil_div(int64_t(g.n) * (g.tiles - g.n8), 16));
+    // One column fragment per wavefront: three or four wavefronts per SIMD hide one another's loads.  Where that is more than three
+    // workgroups per CU and four fragments make it one, long sums go faster so: what a CU fetches halves.  (32 images
+    // 14x14, 256 to 256 channels, F(6,3): 55.2 us against 47.4 with four; 4 images 56x56, 128 to 128, F(2,3): 38.3 against 47.4.)
+    const bool four = frag_items > 768 * wc && g.kgroups >= 16 && int64_t(FREQS) * row_blocks * ceil_div(ceil_div(g.mfrags, 4), wc) <= 256;
+    const int fn = four ? 4 : 1;
+    const int col_blocks = (g.mfrags + fn - 1) / fn;
+    // The tail's fragments with the column blocks: by themselves they fetch all of U again, beside these on the same CUs (8 images
+    // 28x28, 256 to 256 channels, by the wavefronts' clocks: 15 us without the tail, 20 with it, 30 with it as workgroups of its own).
+    // A grid that leaves CUs idle computes them there (1 image 14x14, 512 to 512, F(2,3): 25.9 us attached, 21.7).
+    const int attached = tails <= col_blocks && int64_t(FREQS) * row_blocks * ceil_div(col_blocks, wc) >= 256;
+    const int64_t items = int64_t(rounds) * row_blocks * (ceil_div(col_blocks, wc) + (attached ? 0 : ceil_div((tails + 1) / 2, wc)));
+    const auto gemm = four ? wino_gemm_kernel<4> : wino_gemm_kernel<1>;
     // one launch, except where its work items would be 2^32 or more
-    const int all = col_blocks + tails, most = int(((int64_t(1) << 24) - 1) / (8 * row_blocks));
-    for (int first = 0; first < all; first += most) {
-        const dim3 grid(8u * unsigned(row_blocks) * unsigned(std::min(most, all - first)), FREQS / 8);
-        if (two) hipLaunchKernelGGL(wino_gemm_kernel<2>, grid, dim3(256), 0, stream, u, v, m, g, row_blocks, col_blocks, first);
-        else hipLaunchKernelGGL(wino_gemm_kernel<1>, grid, dim3(256), 0, stream, u, v, m, g, row_blocks, col_blocks, first);
+    const int64_t most = ((int64_t(1) << 24) - 1) / 8;
+    for (int64_t first = 0; first < items; first += most) {
+        const dim3 grid(8u * unsigned(std::min(most, items - first)));
+        hipLaunchKernelGGL(gemm, grid, dim3(256), 0, stream, u, v, m, g, wr, wc, row_blocks, col_blocks, tails, attached, rounds, first);
         TSX_LAUNCH_CHECK("wino_gemm_kernel");
     }
 

@@ -17,7 +17,9 @@ CASES = [
     (2, 13, 48, 24, 40),       # 32 tiles of F(6,3), no tail; remainder channel
     (1, 23, 30, 31, 72),       # 30 tiles: 24 chained, 6 in the tail; three remainder channels
     (5, 34, 28, 28, 65),       # columns of several images in one fragment
-    (4, 64, 62, 40, 128),      # enough wavefronts for two fragments each, an odd number of fragments
+    (4, 64, 62, 40, 128),      # tail fragments computed with the column blocks
+    (6, 20, 6, 42, 33),        # seven tiles of F(6,3) an image, all in the tail: three fragments of 16, an odd number of channel groups
+    (8, 131, 18, 110, 128),    # F(6,3): four column fragments per wavefront, the last block of two, and a tail fragment with them
 ]
 
 
