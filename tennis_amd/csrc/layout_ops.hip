@@ -142,22 +142,24 @@ __global__ __launch_bounds__(256) void depthwise_kernel(const float *__restrict_
 
 // 3x3, stride 1, dilation 1, padding 1 on both sides of a row whose length is a multiple of 4: a lane's four centre
 // columns are one aligned 16-byte load (a wavefront reads whole cache lines) and the two columns beside them come from the
-// neighbouring lanes' registers.  A lane walks DW_ROWS output rows down, all its input rows requested up front: an input
+// neighbouring lanes' registers: a wavefront's first and last lane only hand them on (loads of their own for these columns in
+// two lanes were two more loads per row: 38.5 -> 36.8 us).  A lane walks DW_ROWS output rows down, all its input rows requested up front: an input
 // row is loaded DW_ROWS + 2 times in DW_ROWS instead of three times, and four times the bytes are in flight per wavefront
-// (a row per lane: 58 us on 32x256x56x56; here 38.5).  Lanes run over (plane, row group, run) of the whole tensor: no workgroup is
+// (a row per lane: 58 us on 32x256x56x56).  Lanes run over (plane, row group, run) of the whole tensor: no workgroup is
 // left half empty at a plane's end.  BASIC: the activation is none / relu / leaky_relu.
-constexpr int DW_ROWS = 4;
+constexpr int DW_ROWS = 4, DW_LANES = 62;
 
 template <bool BASIC>
 __global__ __launch_bounds__(256) void depthwise3x3_kernel(const float *__restrict__ x, const float *__restrict__ wt, DwGeom g, int64_t items,
                                                           const float *__restrict__ bias, int act, float slope, int64_t act_body,
                                                           float *__restrict__ out) {
-    const int64_t id = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    const bool live = id < items;
-    const unsigned u = unsigned(live ? id : items - 1);           // items below 2^32
+    const int lane = threadIdx.x % 64;
+    const int64_t id = (int64_t(blockIdx.x) * 4 + threadIdx.x / 64) * DW_LANES + lane - 1;
+    const bool live = lane > 0 && lane <= DW_LANES && id < items;
+    const unsigned u = unsigned(id < 0 ? 0 : id < items ? id : items - 1);           // items below 2^32
     const unsigned runs = unsigned(g.w) / 4, groups = unsigned(g.ho + DW_ROWS - 1) / DW_ROWS;
     const unsigned r1 = u / runs, run = u - r1 * runs, plane = r1 / groups, group = r1 - plane * groups;
-    const int ci = int(plane % unsigned(g.c)), oh0 = int(group) * DW_ROWS, lane = threadIdx.x % 64;
+    const int ci = int(plane % unsigned(g.c)), oh0 = int(group) * DW_ROWS;
     const float *in = x + int64_t(plane) * g.h * g.w + 4 * run;
     const bool first = run == 0, last = run == runs - 1;
     v4f row[DW_ROWS + 2];
@@ -166,8 +168,6 @@ __global__ __launch_bounds__(256) void depthwise3x3_kernel(const float *__restri
     for (int i = 0; i < DW_ROWS + 2; ++i) {
         const float *at = in + min(max(oh0 - g.pt + i, 0), g.h - 1) * g.w;
         row[i] = *reinterpret_cast<const v4f *>(at);
-        left[i] = lane == 0 && !first ? at[-1] : g.padding_value;
-        right[i] = lane == 63 && !last ? at[4] : g.padding_value;
     }
     float kk[9];
 #pragma unroll
@@ -176,8 +176,8 @@ __global__ __launch_bounds__(256) void depthwise3x3_kernel(const float *__restri
 #pragma unroll
     for (int i = 0; i < DW_ROWS + 2; ++i) {
         const float l = __shfl_up(row[i][3], 1), r = __shfl_down(row[i][0], 1);
-        if (lane > 0 && !first) left[i] = l;
-        if (lane < 63 && !last) right[i] = r;
+        left[i] = first ? g.padding_value : l;
+        right[i] = last ? g.padding_value : r;
         const int hi = oh0 - g.pt + i;
         if (hi < 0 || hi >= g.h) {
             row[i] = v4f{g.padding_value, g.padding_value, g.padding_value, g.padding_value};
@@ -262,9 +262,9 @@ int tsx_depthwise_conv2d_f32(const tsx_conv2d_geom *g, const float *x_dev, const
     const dim3 grid(unsigned(planes), unsigned(tsx::ceil_div(lanes_per_plane, 256)));
     const bool k3 = g->kh == 3 && g->kw == 3 && g->stride_h == 1 && g->stride_w == 1 && g->dilation_h == 1 && g->dilation_w == 1;
     const int64_t items = planes * tsx::ceil_div(ho, DW_ROWS) * (g->w / 4);
-    if (k3 && g->pad_left == 1 && wo == g->w && g->w % 4 == 0 && items < (int64_t(1) << 32) - 256 &&
+    if (k3 && g->pad_left == 1 && wo == g->w && g->w % 4 == 0 && tsx::ceil_div(items, 4 * DW_LANES) * 256 < (int64_t(1) << 32) &&
         reinterpret_cast<uintptr_t>(x_dev) % 16 == 0 && reinterpret_cast<uintptr_t>(out_dev) % 16 == 0) {
-        const dim3 flat(unsigned(tsx::ceil_div(items, 256)));
+        const dim3 flat(unsigned(tsx::ceil_div(items, 4 * DW_LANES)));
         if (act >= TSX_ACT_MISH)
             hipLaunchKernelGGL(depthwise3x3_kernel<false>, flat, dim3(256), 0, tsx::as_stream(stream), x_dev, w_dev, d, items, bias_dev, act, slope,
                                total / 4 * 4, out_dev);

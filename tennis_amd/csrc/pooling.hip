@@ -97,13 +97,15 @@ __global__ __launch_bounds__(256) void pooling2d_kernel(const float *__restrict_
 // Global pooling (one window over the whole map): every plane is one sequential chain in the reference, 784 dependent steps
 // of a memory round trip for a lane that walks its plane by itself (247 us for 32x256 planes of 29x29; 13 us here).  Here a workgroup
 // takes 16 planes, its wavefronts copy them to LDS in chunks with whole cache lines and all of a chunk's loads in flight,
-// and 16 lanes walk one plane each from there, the next chunk's loads on their way.  LDS pitch odd: the walking lanes
-// meet no bank twice.
+// and 16 lanes walk one plane each from there, the next chunk's loads on their way.  They read 32 elements ahead, 16 bytes at a
+// time (the pitch leaves them each their own four banks): the walk is then the chain of additions (read eight at a time where
+// they are used it waited for LDS: 32x256 planes of 28x28 15.4 -> 9.8 us).
 constexpr int GP_PLANES = 16, GP_CHUNK = 512, GP_PER = GP_CHUNK / 64, GP_ROWS = GP_PLANES / 4;
 
 __global__ __launch_bounds__(256) void global_pooling2d_kernel(const float *__restrict__ x, int64_t planes, int count, int type, float divisor,
                                                                float *__restrict__ out) {
-    __shared__ float buf[GP_PLANES][GP_CHUNK + 1];
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    __shared__ __attribute__((aligned(16))) float buf[GP_PLANES][GP_CHUNK + 4];
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     const int64_t first = int64_t(blockIdx.x) * GP_PLANES;
     float v[GP_ROWS][GP_PER];
@@ -126,15 +128,31 @@ __global__ __launch_bounds__(256) void global_pooling2d_kernel(const float *__re
         if (at + GP_CHUNK < count) load(at + GP_CHUNK);
         if (threadIdx.x < GP_PLANES) {
             const float *row = buf[threadIdx.x];
-            const int n = min(GP_CHUNK, count - at);
-            if (type == 0) {
-                if (at == 0) acc = row[0];
-#pragma unroll 8
-                for (int i = 0; i < n; ++i) acc = row[i] > acc ? row[i] : acc;
-            } else {
-#pragma unroll 8
-                for (int i = 0; i < n; ++i) acc = __fadd_rn(acc, row[i]);
-            }
+            const int n = min(GP_CHUNK, count - at), blocks = n / 32;
+            if (type == 0 && at == 0) acc = row[0];
+            auto walk = [&](auto &&step) {
+                v4f even[8], odd[8];
+                auto read = [&](v4f(&to)[8], int b) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) to[i] = *reinterpret_cast<const v4f *>(row + min(b, GP_CHUNK / 32 - 1) * 32 + 4 * i);
+                };
+                auto take = [&](const v4f(&from)[8]) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) step(from[i][j]);
+                };
+                read(even, 0);
+                for (int b = 0; b < blocks; b += 2) {
+                    read(odd, b + 1);
+                    take(even);
+                    read(even, b + 2);
+                    if (b + 1 < blocks) take(odd);
+                }
+                for (int i = blocks * 32; i < n; ++i) step(row[i]);
+            };
+            if (type == 0) walk([&](float v) { acc = v > acc ? v : acc; });
+            else walk([&](float v) { acc = __fadd_rn(acc, v); });
         }
         __syncthreads();
     }
@@ -144,34 +162,34 @@ __global__ __launch_bounds__(256) void global_pooling2d_kernel(const float *__re
 // 3x3 max pooling at stride 2 with one row and column of padding in front, on rows of a multiple of 4 (28x28 and up of
 // the usual networks): a lane takes two neighbouring outputs of MP_ROWS output rows, so that its input is one aligned
 // 16-byte load per row plus the column to the left from the neighbouring lane, each row loaded once for both output rows
-// that read it.  The windows are walked in the reference's order (the first valid element, then `>`).  One output per
+// that read it; the first lane only hands its last column on (a load of its own for that column in one lane was a second load
+// per row: 24.0 -> 22.8 us).  The windows are walked in the reference's order (the first valid element, then `>`).  One output per
 // lane and nine 4-byte loads each took 37 us on 32x256x56x56 (129 MB).
-constexpr int MP_ROWS = 2;
+constexpr int MP_ROWS = 2, MP_LANES = 63;
 
 __global__ __launch_bounds__(256) void max_pooling2d_3x3s2_kernel(const float *__restrict__ x, int64_t items, int h, int w, int ho, int wo,
                                                                   float *__restrict__ out) {
     typedef float v4f __attribute__((ext_vector_type(4)));
-    const int64_t id = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    const bool live = id < items;
-    const unsigned u = unsigned(live ? id : items - 1);           // items below 2^32
+    const int lane = threadIdx.x % 64;
+    const int64_t id = (int64_t(blockIdx.x) * 4 + threadIdx.x / 64) * MP_LANES + lane - 1;
+    const bool live = lane > 0 && id < items;
+    const unsigned u = unsigned(id < 0 ? 0 : id < items ? id : items - 1);           // items below 2^32
     const unsigned runs = unsigned(wo + 1) / 2, groups = unsigned(ho + MP_ROWS - 1) / MP_ROWS;
     const unsigned r1 = u / runs, run = u - r1 * runs, plane = r1 / groups, group = r1 - plane * groups;
     const float *in = x + int64_t(plane) * h * w;
     const int col = 4 * int(run);                                 // w: only the window at the right border's last column
     const bool inside = col < w;
-    const int oh0 = int(group) * MP_ROWS, lane = threadIdx.x % 64;
+    const int oh0 = int(group) * MP_ROWS;
     v4f row[2 * MP_ROWS + 1];
     float left[2 * MP_ROWS + 1];
 #pragma unroll
     for (int i = 0; i < 2 * MP_ROWS + 1; ++i) {
         const float *at = in + min(max(2 * oh0 - 1 + i, 0), h - 1) * w;
         row[i] = *reinterpret_cast<const v4f *>(at + (inside ? col : 0));
-        left[i] = lane == 0 && run > 0 ? at[col - 1] : 0.f;
     }
 #pragma unroll
     for (int i = 0; i < 2 * MP_ROWS + 1; ++i) {
-        const float next = __shfl_up(row[i][3], 1);
-        if (lane > 0) left[i] = next;
+        left[i] = __shfl_up(row[i][3], 1);
     }
     if (!live) return;
 #pragma unroll
@@ -333,8 +351,8 @@ int tsx_pooling2d_f32(const float *x_dev, int64_t planes, int32_t h, int32_t w, 
     if (type == 0 && kh == 3 && kw == 3 && stride_h == 2 && stride_w == 2 && pad_top == 1 && pad_left == 1 && w % 4 == 0 && out_w <= w / 2 + 1 &&
         reinterpret_cast<uintptr_t>(x_dev) % 16 == 0) {
         const int64_t items = planes * ((out_w + 1) / 2) * tsx::ceil_div(out_h, MP_ROWS);
-        if (items < (int64_t(1) << 32) - 256) {
-            hipLaunchKernelGGL(max_pooling2d_3x3s2_kernel, dim3(unsigned(tsx::ceil_div(items, 256))), dim3(256), 0, tsx::as_stream(stream), x_dev, items,
+        if (tsx::ceil_div(items, 4 * MP_LANES) * 256 < (int64_t(1) << 32)) {
+            hipLaunchKernelGGL(max_pooling2d_3x3s2_kernel, dim3(unsigned(tsx::ceil_div(items, 4 * MP_LANES))), dim3(256), 0, tsx::as_stream(stream), x_dev, items,
                                h, w, out_h, out_w, out_dev);
             TSX_LAUNCH_CHECK("max_pooling2d_3x3s2_kernel");
             return 0;

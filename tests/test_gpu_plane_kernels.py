@@ -14,7 +14,8 @@ def _dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
-@pytest.mark.parametrize("shape", [(1, 1, 4, 4), (1, 17, 3, 7), (3, 11, 16, 32), (2, 9, 19, 27), (1, 33, 37, 41)])
+@pytest.mark.parametrize("shape", [(1, 1, 4, 4), (1, 17, 3, 7), (3, 11, 16, 32), (2, 9, 19, 27), (1, 33, 37, 41), (2, 3, 1, 31), (2, 3, 4, 8), (1, 5, 3, 33),
+                                   (1, 3, 24, 24), (2, 9, 34, 32)])
 @pytest.mark.parametrize("kind", ["avg", "max"])
 def test_global_pooling(port, shape, kind):
     from tennis_amd import capi
@@ -52,7 +53,7 @@ def test_depthwise_3x3(port, shape, pads):
     assert got.shape == exp.shape and np.array_equal(bits(got), bits(exp))
 
 
-@pytest.mark.parametrize("shape", [(4, 256, 16, 16), (1, 1025, 15, 20), (2, 512, 12, 21), (33, 32, 36, 29)])
+@pytest.mark.parametrize("shape", [(4, 256, 16, 16), (1, 1025, 15, 20), (2, 512, 12, 21), (33, 32, 36, 29), (2, 512, 46, 46), (4, 256, 32, 32), (4, 256, 28, 37)])
 def test_plane_batch_norm(port, shape):
     from tennis_amd import capi
     rng = np.random.default_rng(4)
@@ -62,3 +63,15 @@ def test_plane_batch_norm(port, shape):
     for got, exp in ((capi.batch_norm(*d[:3]), port.batch_norm(x, mean, var)), (capi.batch_scale(d[0], d[3], d[4]), port.batch_scale(x, scale, bias)),
                      (capi.fused_batch_norm(*d), port.fused_batch_norm(x, mean, var, scale, bias))):
         assert np.array_equal(bits(got.cpu().numpy()), bits(exp))
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 256, 16), (32, 256, 1000), (17, 257, 33), (5, 300, 100), (64, 511, 20), (3, 512, 40), (2, 513, 17), (33, 1024, 31),
+                                   (4, 1025, 50), (16, 2048, 65)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_inner_product_of_few_rows(m, k, n, transpose):
+    """Sums of small whole numbers, exact in any order: every K block counted once, whatever the ring holds of them."""
+    from tennis_amd import capi
+    rng = np.random.default_rng(k)
+    a, b = rng.integers(-8, 9, (m, k)).astype(np.float32), rng.integers(-8, 9, (k, n)).astype(np.float32)
+    got = capi.inner_prod_f32(_dev(a), _dev(b.T if transpose else b), transpose=transpose).cpu().numpy()
+    assert np.array_equal(got, a @ b)
