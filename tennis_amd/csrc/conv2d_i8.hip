@@ -726,75 +726,6 @@ __global__ __launch_bounds__(WGM *WGN * 64) void igemm_i8_kernel(GemmParams p) {
     }
 }
 
-// ------------------------------------------------------------------ skinny int8 GEMM (m <= 32 rows)
-// With at most 32 activation rows the whole left operand is ONE MFMA B fragment and the GEMM is a
-// stream over the packed weights: HBM-bound (K*N bytes), not MFMA-bound.  The 128x128-tile kernel
-// would launch N/128 workgroups and walk K serially; here one workgroup owns 32 output columns and
-// its 8 wavefronts split K (interleaved K-steps, 4 in flight each), then add their int32 partial
-// sums through LDS -- exact, so results equal the tiled kernel's and the oracle's.
-// acc register r of lane l: column (weight row) 8*(r/4) + 4*(l/32) + r%4 of the fragment, activation row l%32.
-constexpr int SK_WAVES = 8;
-constexpr int SK_BATCH = 4;
-
-__global__ __launch_bounds__(SK_WAVES * 64) void gemm_i8_skinny_kernel(GemmParams p) {
-    __shared__ int red[SK_WAVES][16][64];
-    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-    const int frag = blockIdx.x;
-    const int frags = p.coutp / 32;
-    const int ksteps = p.cblocks;
-    const int row = lane % 32;
-    const bool row_ok = row < p.positions;
-    // B operand: activation row `row`, the 16 K bytes of group lane/32 of each half K-step
-    const int64_t b_off = int64_t(row_ok ? row : 0) * p.pitch + (lane / 32) * 16;
-    const int64_t b_limit = p.x_bytes - 16;     // the last piece of the matrix
-    // A operand: packed[ks][frag][half][lane][16]
-    const int8_t *a_ptr = p.wp + (int64_t(frag) * 128 + lane) * 16;
-    const int64_t a_kstride = int64_t(frags) * 2048;
-    v16i acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0;
-    const v4i zero = {0, 0, 0, 0};
-    for (int ks0 = wave; ks0 < ksteps; ks0 += SK_WAVES * SK_BATCH) {
-        v4i a[SK_BATCH][2], b[SK_BATCH][2];
-        tsx::static_for<0, SK_BATCH>([&](auto uc) {
-            constexpr int u = decltype(uc)::value;
-            const int ks = ks0 + u * SK_WAVES;
-            const bool on = ks < ksteps;
-            const int kk = on ? ks : 0;
-            tsx::static_for<0, 2>([&](auto hc) {
-                constexpr int h = decltype(hc)::value;
-                a[u][h] = on ? *reinterpret_cast<const v4i *>(a_ptr + kk * a_kstride + h * 1024) : zero;
-                b[u][h] = (on && row_ok) ? tsx::load_piece(p.xs + min(b_off + kk * 64 + h * 32, b_limit)) : zero;
-            });
-        });
-        tsx::static_for<0, SK_BATCH>([&](auto uc) {
-            constexpr int u = decltype(uc)::value;
-            if (ks0 + u * SK_WAVES == ksteps - 1 && p.pitch != p.cp) {      // uniform
-                tsx::static_for<0, 2>([&](auto hc) {
-                    constexpr int h = decltype(hc)::value;
-                    b[u][h] = tsx::shift_piece(b[u][h], int(max(b_off + (ksteps - 1) * 64 + h * 32 - b_limit, int64_t(0))));
-                });
-            }
-            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u][0], b[u][0], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u][1], b[u][1], acc, 0, 0, 0);
-        });
-    }
-    tsx::static_for<0, 16>([&](auto rc) { red[wave][decltype(rc)::value][lane] = acc[decltype(rc)::value]; });
-    __syncthreads();
-    // wavefront w finishes accumulator registers 2w and 2w+1
-    tsx::static_for<0, 2>([&](auto tc) {
-        const int r = wave * 2 + decltype(tc)::value;
-        int sum = 0;
-#pragma unroll
-        for (int w = 0; w < SK_WAVES; ++w) sum += red[w][r][lane];
-        const int co = frag * 32 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4);
-        if (row_ok && co < p.cout) {
-            const float rs = p.row_scale ? p.row_scale[row] : 0.f;
-            tsx::emit_row(p, p.cout, sum, row, int64_t(row) * p.cout + co, p.dq ? p.dq[co] : 0.f, p.bias ? p.bias[co] : 0.f, rs);
-        }
-    });
-}
-
 // ------------------------------------------------------------------ K-split int8 GEMM (a few hundred rows)
 // A GEMM with a few hundred activation rows and a large weight matrix has too few output tiles to give every CU a
 // tile of a shape that reuses its operands: the tiled kernels would walk K serially on a fraction of the chip, or
@@ -876,6 +807,90 @@ __device__ __forceinline__ void ksplit_finish(const GemmParams &p, v16i (&acc)[F
                             tsx::emit_row(p, p.cout, sum[j], row[i], idx + j, p.dq ? p.dq[co[i] + j] : 0.f, p.bias ? p.bias[co[i] + j] : 0.f, rs[i]);
                 }
             }
+        }
+    });
+}
+
+// ------------------------------------------------------------------ skinny int8 GEMM (few tiles of 32 x 32)
+// With at most 32 activation rows the whole left operand is ONE MFMA B fragment and the GEMM is a
+// stream over the packed weights: HBM-bound (K*N bytes), not MFMA-bound.  The 128x128-tile kernel
+// would launch N/128 workgroups and walk K serially; here one workgroup owns 32 output columns of 32 rows and
+// its 8 wavefronts split K (interleaved K-steps, 4 in flight each: one round trip to memory up to K = 2048), then add their
+// int32 partial sums through LDS -- exact, so results equal the tiled kernel's and the oracle's.
+// acc register r of lane l: column (weight row) 8*(r/4) + 4*(l/32) + r%4 of the fragment, activation row l%32.
+// MANY: more than 32 rows, as long as their tiles of 32 x 32 are few.  The wavefronts that finish a tile store four consecutive
+// columns per lane (with one row of many columns all eight with a value per lane are faster: K = N = 4096 4.8 us against 5.6).
+constexpr int SK_WAVES = KS_WAVES;
+constexpr int SK_BATCH = 4;
+
+template <bool MANY>
+__global__ __launch_bounds__(SK_WAVES * 64) void gemm_i8_skinny_kernel(GemmParams p, int row_blocks) {
+    __shared__ int red[SK_WAVES][1][16][64];
+    const int tid = threadIdx.x, lane = tid % 64, wave = MANY ? __builtin_amdgcn_readfirstlane(tid / 64) : tid / 64;
+    const int frags = p.coutp / 32;
+    int frag = blockIdx.x, row0 = 0;
+    if (MANY) {
+        // tiles of the same weights are consecutive, and each XCD takes a contiguous run of tiles
+        const int total = (p.cout + 31) / 32 * row_blocks, per_xcd = (total + 7) / 8;
+        const int t = int(blockIdx.x & 7) * per_xcd + int(blockIdx.x >> 3);
+        if (int(blockIdx.x >> 3) >= per_xcd || t >= total) return;
+        frag = t / row_blocks;
+        row0 = (t - frag * row_blocks) * 32;
+    }
+    const int ksteps = p.cblocks;
+    const int row = row0 + lane % 32;
+    const bool row_ok = row < p.positions;
+    // B operand: activation row `row`, the 16 K bytes of group lane/32 of each half K-step
+    const int64_t b_off = int64_t(row_ok ? row : 0) * p.pitch + (lane / 32) * 16;
+    const int64_t b_limit = p.x_bytes - 16;     // the last piece of the matrix
+    // A operand: packed[ks][frag][half][lane][16]
+    const int8_t *a_ptr = p.wp + (int64_t(frag) * 128 + lane) * 16;
+    const int64_t a_kstride = int64_t(frags) * 2048;
+    v16i acc[1][1];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][0][r] = 0;
+    const v4i zero = {0, 0, 0, 0};
+    for (int ks0 = wave; ks0 < ksteps; ks0 += SK_WAVES * SK_BATCH) {
+        v4i a[SK_BATCH][2], b[SK_BATCH][2];
+        tsx::static_for<0, SK_BATCH>([&](auto uc) {
+            constexpr int u = decltype(uc)::value;
+            const int ks = ks0 + u * SK_WAVES;
+            const bool on = ks < ksteps;
+            const int kk = on ? ks : 0;
+            tsx::static_for<0, 2>([&](auto hc) {
+                constexpr int h = decltype(hc)::value;
+                a[u][h] = on ? *reinterpret_cast<const v4i *>(a_ptr + kk * a_kstride + h * 1024) : zero;
+                b[u][h] = (on && row_ok) ? tsx::load_piece(p.xs + min(b_off + kk * 64 + h * 32, b_limit)) : zero;
+            });
+        });
+        tsx::static_for<0, SK_BATCH>([&](auto uc) {
+            constexpr int u = decltype(uc)::value;
+            if (ks0 + u * SK_WAVES == ksteps - 1 && p.pitch != p.cp) {      // uniform
+                tsx::static_for<0, 2>([&](auto hc) {
+                    constexpr int h = decltype(hc)::value;
+                    b[u][h] = tsx::shift_piece(b[u][h], int(max(b_off + (ksteps - 1) * 64 + h * 32 - b_limit, int64_t(0))));
+                });
+            }
+            acc[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u][0], b[u][0], acc[0][0], 0, 0, 0);
+            acc[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u][1], b[u][1], acc[0][0], 0, 0, 0);
+        });
+    }
+    if (MANY) {
+        ksplit_finish<1, 1>(p, acc, red, frag, row0, lane, wave);
+        return;
+    }
+    tsx::static_for<0, 16>([&](auto rc) { red[wave][0][decltype(rc)::value][lane] = acc[0][0][decltype(rc)::value]; });
+    __syncthreads();
+    // wavefront w finishes accumulator registers 2w and 2w+1
+    tsx::static_for<0, 2>([&](auto tc) {
+        const int r = wave * 2 + decltype(tc)::value;
+        int sum = 0;
+#pragma unroll
+        for (int w = 0; w < SK_WAVES; ++w) sum += red[w][0][r][lane];
+        const int co = frag * 32 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4);
+        if (row_ok && co < p.cout) {
+            const float rs = p.row_scale ? p.row_scale[row] : 0.f;
+            tsx::emit_row(p, p.cout, sum, row, int64_t(row) * p.cout + co, p.dq ? p.dq[co] : 0.f, p.bias ? p.bias[co] : 0.f, rs);
         }
     });
 }
@@ -1581,11 +1596,23 @@ int tsx_gemm_i8(int32_t m, int32_t n, int32_t k, const int8_t *a_dev, const void
         p.x_bytes = int64_t(m) * kp;
         return 0;
     };
-    if (m <= 32) {
-        if (p.x_bytes < 16 && (rc = pad_rows())) return rc;      // less than a piece
-        hipLaunchKernelGGL(gemm_i8_skinny_kernel, dim3(unsigned(tsx::ceil_div(n, 32))), dim3(SK_WAVES * 64), 0, stream, p);
-        TSX_LAUNCH_CHECK("gemm_i8_skinny_kernel");
-        return 0;
+    // Few tiles of 32 x 32: the K-split kernel's 64 x 64 would leave most CUs idle, and a tile is one round trip to memory here.  Up
+    // to one workgroup per CU, or two with a K that keeps what a CU fetches below a tile of theirs (us, theirs -> here: 197 x
+    // 777, K = 1500, fp32 10.0 -> 5.4, int8 11.5 -> 6.1; 256 x 1024, K = 1024, 5.7 -> 4.6; 48 x 4096, K = 4096, 10.8 -> 7.9; 131 x 95,
+    // K = 2179, 12.9 -> 10.2; 400 x 500, K = 300, 6.0 -> 3.9; 2048 x 256, K = 512, 5.0 -> 4.9; but 256 x 2048, K = 2048, 7.8 -> 8.1
+    // and 640 x 1024, K = 128, 4.4 -> 5.5).  A switch of another kernel leaves more than 32 rows to these.
+    {
+        const auto set = [](const char *name) { const char *value = std::getenv(name); return value && value[0]; };
+        const int row_blocks = int(tsx::ceil_div(m, 32));
+        const int64_t tiles = tsx::ceil_div(n, 32) * row_blocks;
+        const bool few = (tiles <= 256 || (tiles <= 512 && tiles * kp <= 900000)) && !set("TSX_GEMM_I8_KSPLIT") && !set("TSX_GEMM_I8_TILE");
+        if (m <= 32 || few) {
+            if (p.x_bytes < 16 && (rc = pad_rows())) return rc;      // less than a piece
+            if (m <= 32) hipLaunchKernelGGL(gemm_i8_skinny_kernel<false>, dim3(unsigned(tiles)), dim3(SK_WAVES * 64), 0, stream, p, 1);
+            else hipLaunchKernelGGL(gemm_i8_skinny_kernel<true>, dim3(unsigned((tiles + 7) / 8 * 8)), dim3(SK_WAVES * 64), 0, stream, p, row_blocks);
+            TSX_LAUNCH_CHECK("gemm_i8_skinny_kernel");
+            return 0;
+        }
     }
     // TSX_GEMM_I8_KSPLIT: "0" never, "force" every GEMM of more than 32 rows (tests); otherwise GEMMs whose 64 x 64 tiles
     // run in one round (at most 256: one workgroup per CU) with a K long enough to split.  Measured, fp32 output, against
