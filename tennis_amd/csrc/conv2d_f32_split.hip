@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
+#include <cstring>
 
 namespace tsx {
 namespace {
@@ -61,23 +62,27 @@ __device__ __forceinline__ Parts split8(const float (&number)[8]) {
 // ---- weights [M][C][taps] to MFMA operands [16 channels][tap][32 rows][part][lane][8], zeros behind M and C.
 // A workgroup takes 16 channels of 32 rows, through LDS: read as they lie (a lane reading its own 8 channels x taps touches a
 // cache line per lane and load: 7.2 us for 256 x 256 x 3 x 3), written a KiB per store instruction.
+// No thread splits more than two pieces: few layers have the workgroups to fill the chip, and with 256 threads a 5x5 layer's
+// fifty loads and seven pieces of a thread were a chain of 8 us (183 channels to 77; now 5.6), a 3x3 layer's of 5.4 (now 4.2).
+constexpr int split_weights_threads(int taps) { return taps == 25 ? 800 : taps == 9 ? 576 : 64; }
 template <int TAPS>
-__global__ __launch_bounds__(256) void split_weights_kernel(const float *w, int M, int C, int mfrags, v4u *out) {
-    constexpr int RUN = 16 * TAPS, PITCH = RUN + 1, LOADS = 32 * RUN / 256;
+__global__ __launch_bounds__(split_weights_threads(TAPS)) void split_weights_kernel(const float *w, int M, int C, int mfrags, v4u *out) {
+    constexpr int THREADS = split_weights_threads(TAPS), RUN = 16 * TAPS, PITCH = RUN + 1, LOADS = 32 * RUN / THREADS;
+    static_assert(LOADS * THREADS == 32 * RUN && 64 * TAPS % THREADS == 0, "whole rounds");
     __shared__ float rows[32 * PITCH];
     const int tid = threadIdx.x, c0 = blockIdx.y * 16, live = min(16, C - c0) * TAPS;
     float x[LOADS];
     static_for<0, LOADS>([&](auto ic) {
-        const int e = tid + 256 * decltype(ic)::value, k = e % RUN, row = blockIdx.x * 32 + e / RUN;
+        const int e = tid + THREADS * decltype(ic)::value, k = e % RUN, row = blockIdx.x * 32 + e / RUN;
         x[decltype(ic)::value] = row < M && k < live ? w[(int64_t(row) * C + c0) * TAPS + k] : 0.f;
     });
     static_for<0, LOADS>([&](auto ic) {
-        const int e = tid + 256 * decltype(ic)::value;
+        const int e = tid + THREADS * decltype(ic)::value;
         rows[e / RUN * PITCH + e % RUN] = x[decltype(ic)::value];
     });
     __syncthreads();
     v4u *to = out + (int64_t(blockIdx.y) * TAPS * mfrags + blockIdx.x) * 192;
-    for (int e = tid; e < 64 * TAPS; e += 256) {
+    for (int e = tid; e < 64 * TAPS; e += THREADS) {
         const int lane = e % 64, tap = e / 64;
         float v[8];
         static_for<0, 8>([&](auto jc) { v[decltype(jc)::value] = rows[lane % 32 * PITCH + (8 * (lane / 32) + decltype(jc)::value) * TAPS + tap]; });
@@ -89,6 +94,19 @@ __global__ __launch_bounds__(256) void split_weights_kernel(const float *w, int 
     }
 }
 
+// A divisor of 1 to 2^30 for numbers below 2^31: with l = ceil(log2 d) and m = ceil(2^(31 + l) / d), which fits in 32 bits,
+// n m >> (31 + l) is n / d, since m d < 2^(31 + l) + 2^l.  (The two dozen divisions of a tile's start and end by unknown
+// divisors were 2 of its 9 us beside the steps.)
+struct Divisor {
+    unsigned m, l;
+};
+Divisor divisor(int64_t d) {
+    unsigned l = 0;
+    while ((int64_t(1) << l) < d) ++l;
+    return {unsigned(((uint64_t(1) << (31 + l)) + uint64_t(d) - 1) / uint64_t(d)), l};
+}
+__device__ __forceinline__ int quotient(int n, Divisor d) { return int(__umulhi(unsigned(n) << 1, d.m) >> d.l); }
+
 struct SplitParams {
     const float *x, *w32, *bias;
     const void *w;                 // split weights
@@ -97,8 +115,10 @@ struct SplitParams {
     int n, C, H, W, dil_h, sh, sw, pad_top, pad_left;
     int ho, wo, howo;
     int hv, wv;                    // rows of one image with the padding its windows reach; patch columns
+    Divisor by_tiles, by_tiles_m, by_col_tiles, by_seg_rows, by_wo, by_ho, by_howo, by_hv, by_wv;
     int seg, col_tiles;            // a fragment is 32 columns of one row; column tiles per row
     int chunks, mfrags, tiles_m, tiles_n;
+    int slices, slice_chunks;      // chunks of one slice; the sums of slice i go to out + i M N
     unsigned w_bytes;
     float padding_value;
     int act;
@@ -120,12 +140,16 @@ __device__ __forceinline__ void lds_barrier() {
 // to LDS once per element, here in three parts, [part][8 channels][PITCH cells][8], and every tap is a shifted read; a
 // thread converts eight channels of a cell at a time while the other wavefront of its SIMD multiplies.  TAPS: 9 (3x3), 25
 // (5x5), 1 (the patch is the tile's positions themselves, at any stride).
+// Layers of few tiles leave most CUs idle while each tile walks all channels: their chunks go to `slices` of workgroups, whose
+// sums another kernel adds in order (2 images of 38x12, 233 channels to 98, 3x3 of stride 2: 47 -> 20 us, of which the fp32
+// MFMA kernel's chain of 30 chunks was 1.4 us each; 3 of 30x30, 398 to 31, 5x5: 175 -> 39).  The patches of 768 cells, with one
+// workgroup a CU, are strided layers' (6 images of 33x33, 446 to 213, 5x5 of stride 2: 551 us without a tile here, 84).
 // What bounds it: the MFMAs at the clock the bf16 matrix cores leave, with conversions, operand reads and weights beside them
 // (six products instead of eight, a quarter of the MFMAs less: 55 us instead of 64 on 8 images of 28x28x256 with 256 3x3
 // filters).  Against the fp32 MFMAs (us, weights' split included): that layer 84 -> 64, 128 channels at 56x56 77 -> 55, 256 to
 // 256 channels 1x1 at 56x56, 32 images, 132 -> 105, 100 to 150 channels 5x5 at 33x41, 4 images, 128 -> 67.
 template <int WM, int WN, int TAPS, int PITCH, int CC>
-__global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitParams p) {
+__global__ __launch_bounds__(64 * WM * WN, WM * WN == 4 && PITCH > 384 ? 1 : 2) void conv_f32_split_kernel(SplitParams p) {
     constexpr int THREADS = 64 * WM * WN;
     constexpr int BM = 32 * WM, BN = 64 * WN, KW = TAPS == 9 ? 3 : TAPS == 25 ? 5 : 1;
     constexpr int SUBS = CC / 16, STEPS = SUBS * TAPS;
@@ -140,15 +164,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
     const int hf = lane / 32;
     const int wn = wave % WN, wm = wave / WN;
 
-    // Tiles that share their positions are consecutive, and each XCD takes a contiguous run of tiles: a patch is fetched
-    // into one L2.
-    const int total = p.tiles_m * p.tiles_n, per_xcd = (total + 7) / 8;
-    const int t = int(blockIdx.x & 7) * per_xcd + int(blockIdx.x >> 3);
-    if (int(blockIdx.x >> 3) >= per_xcd || t >= total) return;
-    const int tn = t / p.tiles_m, m0 = (t - tn * p.tiles_m) * BM;
+    // Tiles of a slice that share their positions are consecutive, and each XCD takes a contiguous run of tiles: a patch, and
+    // where there are many slices their weights, are fetched into one L2.
+    const int tiles = p.tiles_m * p.tiles_n, total = tiles * p.slices, per_xcd = (total + 7) / 8;
+    const int index = int(blockIdx.x & 7) * per_xcd + int(blockIdx.x >> 3);
+    if (int(blockIdx.x >> 3) >= per_xcd || index >= total) return;
+    const int slice = quotient(index, p.by_tiles), t = index - slice * tiles;
+    const int tn = quotient(t, p.by_tiles_m), m0 = (t - tn * p.tiles_m) * BM;
+    const int first_chunk = slice * p.slice_chunks, end_chunk = min(p.chunks, first_chunk + p.slice_chunks);
 
     // ---- positions: flat over the batch, or segments (image, first row inside it, first column)
-    const int seg_rows = (p.ho + BN / 32 - 1) / (BN / 32), seg_tile = p.seg ? tn / p.col_tiles : 0, seg_img = seg_tile / seg_rows;
+    const int seg_rows = (p.ho + BN / 32 - 1) / (BN / 32), seg_tile = p.seg ? quotient(tn, p.by_col_tiles) : 0, seg_img = quotient(seg_tile, p.by_seg_rows);
     const int seg_row = (seg_tile - seg_img * seg_rows) * (BN / 32);
     const int col0 = p.seg ? (tn - seg_tile * p.col_tiles) * 32 : 0;
     auto decode = [&](int q, int &row, int &col) -> bool {                 // tile position -> batch-wide output row, column
@@ -158,12 +184,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
             return seg_row + q / 32 < p.ho && col < p.wo;
         }
         const int pos = tn * BN + q;
-        row = pos / p.wo;
+        row = quotient(pos, p.by_wo);
         col = pos - row * p.wo;
         return pos < p.N;
     };
-    auto virtual_row = [&](int row) { const int img = row / p.ho; return img * p.hv + (row - img * p.ho) * p.sh; };
-    const int vr0 = virtual_row(p.seg ? seg_img * p.ho + seg_row : tn * BN / p.wo);
+    auto virtual_row = [&](int row) { const int img = quotient(row, p.by_ho); return img * p.hv + (row - img * p.ho) * p.sh; };
+    const int vr0 = virtual_row(p.seg ? seg_img * p.ho + seg_row : quotient(tn * BN, p.by_wo));
 
     // ---- patch bookkeeping: slot i of a thread is cell (tid + 512 i) % PITCH of the chunk's eight channels (tid + 512 i) / PITCH
     constexpr unsigned NOWHERE = 0x80000000u;                              // beyond any buffer: loads 0, stores nothing
@@ -175,14 +201,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
         int img, h, w;
         bool in = true;
         if (TAPS == 1) {
-            const int pos = tn * BN + cell, r = pos % p.howo, oh = r / p.wo;
-            img = pos / p.howo;
+            const int pos = tn * BN + cell;
+            img = quotient(pos, p.by_howo);
+            const int r = pos - img * p.howo, oh = quotient(r, p.by_wo);
             in = pos < p.N;
             h = oh * p.sh - p.pad_top;
             w = (r - oh * p.wo) * p.sw - p.pad_left;
         } else {
-            const int pr = cell / p.wv, v = vr0 + pr;
-            img = v / p.hv;
+            const int pr = quotient(cell, p.by_wv), v = vr0 + pr;
+            img = quotient(v, p.by_hv);
             in = img < p.n;                                                // cells behind the tile's patch: loaded, never used
             h = v - img * p.hv - p.pad_top;
             w = cell - pr * p.wv + col0 * p.sw - p.pad_left;
@@ -205,7 +232,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
     // its offsets are beyond the buffer (whose size stays above every channel's scalar offset, from which the hardware counts).
     auto load_patch = [&](auto form, auto ic, auto from, auto to, int chunk) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
-        const bool live = chunk < p.chunks;
+        const bool live = chunk < end_chunk;
         const int c0 = live ? chunk * CC : 0, at = c0 * int(plane) * 4;
         const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(p.x) + at), 0, x_bytes - at, 0x00020000);
         const int left = (live ? p.C - c0 : 0) - 8 * x_octet(i);
@@ -241,7 +268,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
     struct B { v4u part[2][3]; } b;
     auto load_weights = [&](auto sc, int chunk) __attribute__((always_inline)) {      // step sc of the chunk, its steps beyond STEPS in the next
         constexpr int s = decltype(sc)::value % STEPS, over = decltype(sc)::value / STEPS, sub = s / TAPS, tap = s % TAPS;
-        const int q = ((min(chunk + over, p.chunks - 1) * (CC / 16) + sub) * TAPS + tap) * w_step;
+        const int q = ((min(chunk + over, end_chunk - 1) * (CC / 16) + sub) * TAPS + tap) * w_step;
         static_for<0, 3>([&](auto pc) {
             constexpr int part = decltype(pc)::value;
             a[s % AHEAD].part[part] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(wr, w_off + part * 1024, q, 0));
@@ -295,14 +322,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
     auto run = [&](auto form) __attribute__((always_inline)) {
         const std::integral_constant<int, 0> none;
         const std::integral_constant<int, 8> all;
-        static_for<0, SLOTS>([&](auto ic) { load_patch(form, ic, none, all, 0); });
-        static_for<0, AHEAD>([&](auto sc) { load_weights(sc, 0); });
-        static_for<0, SLOTS>([&](auto ic) { store_patch(form, ic, 0, 0); });
-        static_for<0, SLOTS>([&](auto ic) { load_patch(form, ic, none, all, 1); });
+        static_for<0, SLOTS>([&](auto ic) { load_patch(form, ic, none, all, first_chunk); });
+        static_for<0, AHEAD>([&](auto sc) { load_weights(sc, first_chunk); });
+        static_for<0, SLOTS>([&](auto ic) { store_patch(form, ic, first_chunk, 0); });
+        static_for<0, SLOTS>([&](auto ic) { load_patch(form, ic, none, all, first_chunk + 1); });
         sum[0] = sum[1] = small[0] = small[1] = v16f{};
         lds_barrier();
         b = read(none, 0);
-        int chunk = 0, now = 0;
+        int chunk = first_chunk, now = 0;
         do {
             const int next = BUFFER - now;
             large[0] = large[1] = v16f{};
@@ -335,7 +362,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
             sum[0] += large[0];
             sum[1] += large[1];
             now = next;
-        } while (++chunk < p.chunks);
+        } while (++chunk < end_chunk);
     };
     if (ragged) run(std::integral_constant<int, 1>{});
     else run(std::integral_constant<int, 0>{});
@@ -351,13 +378,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
         constexpr int BLOCK = 8;               // MFMAs per fragment whose operands are requested together
         const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.x), 0, x_bytes, 0x00020000);
         const auto wr32 = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.w32), 0, p.M * p.C * TAPS * 4, 0x00020000);
-        const int products = p.C * TAPS, w_row = min(m0 + wm * 32 + in_row, p.M - 1) * products;
+        const int w_row = min(m0 + wm * 32 + in_row, p.M - 1) * p.C * TAPS, products = min(p.C, end_chunk * CC) * TAPS;
         unsigned first[2], inside[2];          // element of the first tap in the first channel; a bit per tap
         static_for<0, 2>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
             int row, col;
             const bool ok = decode((wn * 2 + j) * 32 + in_row, row, col);
-            const int img = row / p.ho, h = (row - img * p.ho) * p.sh - p.pad_top, w = col * p.sw - p.pad_left;
+            const int img = quotient(row, p.by_ho), h = (row - img * p.ho) * p.sh - p.pad_top, w = col * p.sw - p.pad_left;
             first[j] = unsigned(img) * unsigned(p.C) * plane + unsigned(h * p.W + w);
             inside[j] = 0;
             for (int tap = 0; tap < TAPS; ++tap) {
@@ -366,7 +393,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
             }
         });
         sum[0] = sum[1] = v16f{};
-        for (int k0 = 0; k0 < products; k0 += 2 * BLOCK) {
+        for (int k0 = first_chunk * CC * TAPS; k0 < products; k0 += 2 * BLOCK) {
             float w[BLOCK], x[2][BLOCK];
             unsigned at[2][BLOCK];
             static_for<0, BLOCK>([&](auto ec) {
@@ -410,13 +437,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
         bias[r] = p.bias ? p.bias[min(m0 + wm * 32 + 8 * (r / 4) + 4 * half + r % 4, p.M - 1)] : 0.f;
     });
     // A lane's element of a row is its own offset plus a uniform one; 32-bit offsets, the output is below 2 GiB.
-    const auto out = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, int(int64_t(p.M) * p.N * 4), 0x00020000);
+    const auto out = __builtin_amdgcn_make_buffer_rsrc(p.out + int64_t(slice) * p.M * p.N, 0, int(int64_t(p.M) * p.N * 4), 0x00020000);
     const bool body = p.act_body == int64_t(p.M) * p.N;      // no element behind the activation's SIMD body
     static_for<0, 2>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
         int row, col;
         const bool ok = decode((wn * 2 + j) * 32 + in_row, row, col);
-        const int img = row / p.ho;
+        const int img = quotient(row, p.by_ho);
         const int base = img * p.M * p.howo + (row - img * p.ho) * p.wo + col + (m0 + wm * 32 + 4 * half) * p.howo;
         static_for<0, 16>([&](auto rc) {
             constexpr int r = decltype(rc)::value, up = 8 * (r / 4) + r % 4;
@@ -427,6 +454,40 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void conv_f32_split_kernel(SplitPa
             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), out, in ? base * 4 : int(NOWHERE), up * p.howo * 4, 0);
         });
     });
+}
+
+// ---- slices' sums [slice][output] to the output, in the order of the slices.  VEC: 4 outputs at a time, which start a channel
+// or lie inside one.
+struct SliceParams {
+    const float *sums, *bias;
+    float *out;
+    unsigned total, howo, M;
+    int slices, act;
+    float slope;
+    int64_t act_body;
+};
+
+template <int VEC>
+__global__ __launch_bounds__(256) void sum_slices_kernel(SliceParams p) {
+    typedef float vec __attribute__((ext_vector_type(VEC)));
+    const unsigned at = (blockIdx.x * 256 + threadIdx.x) * VEC;
+    if (at >= p.total) return;
+    const float bias = p.bias ? p.bias[at / p.howo % p.M] : 0.f;
+    auto slice = [&](int s) __attribute__((always_inline)) { return *reinterpret_cast<const vec *>(p.sums + int64_t(s) * p.total + at); };
+    vec sum = slice(0);
+    int s = 1;
+    for (; s + 4 <= p.slices; s += 4) {        // four requests in flight
+        vec q[4];
+        static_for<0, 4>([&](auto ic) { q[decltype(ic)::value] = slice(s + decltype(ic)::value); });
+        static_for<0, 4>([&](auto ic) { sum += q[decltype(ic)::value]; });
+    }
+    for (; s < p.slices; ++s) sum += slice(s);
+    static_for<0, VEC>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        const float v = p.bias ? __fadd_rn(sum[i], bias) : sum[i];
+        sum[i] = apply_act_basic(v, p.act, p.slope, int64_t(at) + i < p.act_body);
+    });
+    *reinterpret_cast<vec *>(p.out + at) = sum;
 }
 
 // ---- tiles.  Each with the patch pitches it is built for, smallest first.
@@ -451,7 +512,7 @@ int launch_split(const SplitParams &p, hipStream_t stream) {
             if (dev < 64) granted[dev].store(true);
         }
     }
-    const int total = p.tiles_m * p.tiles_n;
+    const int total = p.tiles_m * p.tiles_n * p.slices;
     hipLaunchKernelGGL(kernel, dim3(unsigned((total + 7) / 8 * 8)), dim3(64 * WM * WN), lds_bytes, stream, p);
     TSX_LAUNCH_CHECK("conv_f32_split_kernel");
     return 0;
@@ -464,6 +525,8 @@ const SplitTile SPLIT_TILES[] = {
     split_tile<2, 2, 9, 256, 16>(), split_tile<2, 2, 9, 384, 16>(), split_tile<4, 1, 9, 256, 16>(), split_tile<4, 1, 9, 384, 16>(), split_tile<4, 2, 9, 512, 16>(),
     split_tile<2, 2, 25, 384, 16>(), split_tile<4, 1, 25, 256, 16>(), split_tile<4, 1, 25, 384, 16>(),
     split_tile<4, 1, 1, 64, 64>(), split_tile<2, 2, 1, 128, 32>(),
+    split_tile<4, 2, 9, 768, 16>(), split_tile<2, 2, 9, 768, 16>(), split_tile<4, 1, 9, 768, 16>(),
+    split_tile<4, 2, 25, 768, 16>(), split_tile<2, 2, 25, 768, 16>(), split_tile<4, 1, 25, 768, 16>(),
 };
 constexpr int SPLIT_TILE_COUNT = int(sizeof(SPLIT_TILES) / sizeof(SPLIT_TILES[0]));
 
@@ -488,6 +551,15 @@ bool plan_tile(const ConvF32Layer &l, int tile, bool flat, SplitParams *p) {
     const int64_t tiles_n = flat ? ceil_div(p->N, bn) : int64_t(l.n) * ceil_div(l.ho, bn / 32) * p->col_tiles;
     if (tiles_n * p->tiles_m >= (int64_t(1) << 22)) return false;
     p->tiles_n = int(tiles_n);
+    p->by_tiles = divisor(tiles_n * p->tiles_m);
+    p->by_tiles_m = divisor(p->tiles_m);
+    p->by_col_tiles = divisor(p->col_tiles);
+    p->by_seg_rows = divisor(ceil_div(l.ho, bn / 32));
+    p->by_wo = divisor(p->wo);
+    p->by_ho = divisor(p->ho);
+    p->by_howo = divisor(p->howo);
+    p->by_hv = divisor(p->hv);
+    p->by_wv = divisor(p->wv);
     if (k > 1) {
         // rows of the largest patch: output rows a tile touches, and per image border it crosses the padding rows between
         const int64_t rows = flat ? ceil_div(bn + l.wo - 1, l.wo) : bn / 32;
@@ -503,10 +575,13 @@ bool plan_tile(const ConvF32Layer &l, int tile, bool flat, SplitParams *p) {
 }  // namespace
 
 ConvF32Split conv_f32_split_choose(const ConvF32Layer &l) {
-    ConvF32Split best{-1, 0, 0.};
-    const char *e = std::getenv("TSX_CONV_F32_SPLIT");         // "0": never; a number: that tile wherever it suits (tests)
+    ConvF32Split best{-1, 0, 0., 1};
+    // "0": never; a number: that tile wherever it suits, in one slice or, "number/slices", in so many where there are the chunks (tests)
+    const char *e = std::getenv("TSX_CONV_F32_SPLIT");
     if (e && e[0] == '0' && !e[1]) return best;
     const int only = e && e[0] ? std::atoi(e) - 1 : -1;
+    const char *slash = only >= 0 ? std::strchr(e, '/') : nullptr;
+    const int only_slices = slash ? std::max(1, std::atoi(slash + 1)) : 1;
     const int64_t most = (int64_t(1) << 31) - 64;              // 32-bit byte offsets into every tensor
     const int64_t positions = int64_t(l.n) * l.ho * l.wo;
     if (int64_t(l.n) * l.c * l.h * l.w * 4 > most || positions * l.cout * 4 > most || positions >= (int64_t(1) << 30) || l.pad_top < 0 || l.pad_left < 0)
@@ -516,12 +591,25 @@ ConvF32Split conv_f32_split_choose(const ConvF32Layer &l) {
             SplitParams p{};
             if ((only >= 0 && i * 2 + flat != only) || !plan_tile(l, i, flat != 0, &p)) continue;
             const SplitTile &t = SPLIT_TILES[i];
-            // Time of the busiest CU in us: a step's 16 MFMAs at the 1.7 GHz that the bf16 matrix cores come to beside everything
-            // else, 2 for a tile's start and end, 8 for the launches and the weights.  Chosen together with the line in
-            // split_choice by the tiles of 156 layers of 0.05 to 13 GFLOP.
-            const double tiles = double(ceil_div(int64_t(p.tiles_m) * p.tiles_n, 256)), waves = t.wm * t.wn / 4;
-            const double us = tiles * (waves * p.chunks * (t.cc / 16) * t.taps * 512 / 1700. + 2) + 8;
-            if (best.tile < 0 || us < best.us) best = {i * 2 + flat, p.w_bytes, us};
+            // Time in us: the launches; by the tiles of a CU their steps (16 MFMAs are 512 cycles, at 1.7 GHz beside everything
+            // else; whole eights of channels take the form without a look at each, a SIMD's two wavefronts of one workgroup
+            // share what is beside the MFMAs), their start and end, of which little is seen where a CU holds two workgroups, and
+            // its last, half empty round; the weights and the output.  Slices cost their sums' way through memory and one more
+            // launch.  Fitted to all combinations of tile and slices on 400 layers of 0.01 to 13 GFLOP, which it meets by 8 %
+            // (rms); the combinations it picks take 1 % longer than the fastest.
+            const bool eight = t.wm * t.wn == 8, alone = t.pitch > 384, whole = l.c % 8 == 0;
+            const double sums = double(positions) * l.cout * 4e-6, weights = double(l.cout) * l.c * t.taps * 1e-6;
+            for (int slices = 1; slices <= p.chunks; ++slices) {
+                const int each = int(ceil_div(p.chunks, slices));
+                if (only >= 0 ? slices != int(ceil_div(p.chunks, ceil_div(p.chunks, only_slices))) : ceil_div(p.chunks, each) != slices) continue;
+                const double tiles = double(p.tiles_m) * p.tiles_n * slices / 256, up = double(ceil_div(int64_t(p.tiles_m) * p.tiles_n * slices, 256));
+                const double rounds = tiles <= 1 ? 0.81 + 0.19 * tiles : tiles + (alone ? 1 : 0.5) * (up - tiles);
+                const double step = (eight ? whole ? 1.66 : 1.78 : (tiles <= 1 ? 1.26 : 1.17) * (whole ? 0.85 : 1)) * 512 / 1700.;
+                const double us = 8.6 + rounds * (each * (t.cc / 16) * t.taps * step + (alone ? 7.2 : 2)) + 5.7 * weights + 0.11 * sums +
+                                  (slices > 1 ? 1.6 + 0.27 * slices * sums : 0) + t.pitch * 1e-4 + t.wn * 0.1;      // of equal ones the smaller patch, the taller tile
+                if (best.tile < 0 || us < best.us)
+                    best = {i * 2 + flat, p.w_bytes + (slices > 1 ? size_t(slices) * size_t(positions) * l.cout * 4 : 0), us, slices};
+            }
         }
     if (only >= 0) best.us = 0;
     return best;
@@ -533,26 +621,42 @@ void conv_f32_split_tile_size(int tile, int *rows, int *positions, int *patch) {
     *patch = SPLIT_TILES[tile / 2].pitch;
 }
 
-int conv_f32_split(const ConvF32Layer &l, int tile, const float *bias, int act, float slope, float padding_value, float *out, void *workspace,
-                   hipStream_t stream) {
+int conv_f32_split(const ConvF32Layer &l, const ConvF32Split &choice, const float *bias, int act, float slope, float padding_value, float *out,
+                   void *workspace, hipStream_t stream) {
     SplitParams p{};
+    const int tile = choice.tile, slices = choice.slices;
     if (tile < 0 || tile / 2 >= SPLIT_TILE_COUNT || !plan_tile(l, tile / 2, tile % 2 != 0, &p))
         return fail(TSX_E_INVALID, "conv_f32_split: tile %d does not suit this layer", tile);
     const SplitTile &t = SPLIT_TILES[tile / 2];
     const dim3 grid(unsigned(p.mfrags), unsigned(p.chunks * (t.cc / 16)));
     const auto pack = t.taps == 9 ? split_weights_kernel<9> : t.taps == 25 ? split_weights_kernel<25> : split_weights_kernel<1>;
-    hipLaunchKernelGGL(pack, grid, dim3(256), 0, stream, l.w_dev, l.cout, l.c, p.mfrags, static_cast<v4u *>(workspace));
+    hipLaunchKernelGGL(pack, grid, dim3(unsigned(split_weights_threads(t.taps))), 0, stream, l.w_dev, l.cout, l.c, p.mfrags, static_cast<v4u *>(workspace));
     TSX_LAUNCH_CHECK("split_weights_kernel");
     p.x = l.x_dev;
     p.w32 = l.w_dev;
     p.w = workspace;
-    p.bias = bias;
-    p.out = out;
     p.padding_value = padding_value;
-    p.act = act;
-    p.slope = slope;
-    p.act_body = int64_t(p.N) * p.M / 4 * 4;
-    return t.launch(p, stream);
+    p.slices = slices;
+    p.slice_chunks = int(ceil_div(p.chunks, slices));
+    const int64_t total = int64_t(p.N) * p.M, act_body = total / 4 * 4;
+    if (slices == 1) {
+        p.bias = bias;
+        p.out = out;
+        p.act = act;
+        p.slope = slope;
+        p.act_body = act_body;
+        return t.launch(p, stream);
+    }
+    p.out = reinterpret_cast<float *>(static_cast<char *>(workspace) + p.w_bytes);
+    p.act = TSX_ACT_NONE;
+    p.act_body = total;
+    const int rc = t.launch(p, stream);
+    if (rc) return rc;
+    const SliceParams q{p.out, bias, out, unsigned(total), unsigned(p.howo), unsigned(p.M), slices, act, slope, act_body};
+    const bool vec = p.howo % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+    hipLaunchKernelGGL(vec ? sum_slices_kernel<4> : sum_slices_kernel<1>, dim3(unsigned(ceil_div(total, vec ? 1024 : 256))), dim3(256), 0, stream, q);
+    TSX_LAUNCH_CHECK("sum_slices_kernel");
+    return 0;
 }
 
 }  // namespace tsx

@@ -716,18 +716,24 @@ int window_tile(const ConvF32Layer &layer, const GemmArgs &g, double *cycles = n
     return conv_f32_window_tile(layer, cycles);
 }
 
-// The tile on the bf16 matrix cores for the layer, where that is expected to be at least a twentieth faster than the window
-// kernel; what the register-fed kernel takes stays there.  The window kernel's time is its cost model's at 2.2 GHz times
-// what 45 layers of 0.01 to 17 GFLOP took over it at least: 1.2 with its vector forms, 1.9 without (1.6 to 4.6 measured).  Kept
-// on the window kernel by that: 1x256x28x28, 256 3x3 filters (25 us against 49), 8x512x14x14 to 512 1x1 (15 against 22), all
-// layers of some 10 us.  Of 156 layers two take longer this way by more than 2 % (33.2 -> 36.3 us, 74.4 -> 76.2).
+// The tile on the bf16 matrix cores for the layer, where that is expected to be at least a twentieth faster than the kernel
+// without a workspace (a quarter, than the register-fed one, whose line rests on ten layers), of whose time `cycles` is the window kernel's model (0: a forced tile, which stays).  At 2.2 GHz the
+// window kernel takes those cycles with its vector forms, 1.35 times as long in its K-split tile; 1.75 times without, or 1.05
+// where it has one tap; the register-fed kernel twice, on 5x5 windows 1.1 times; and all of them their launch and output.
+// Fitted, rather too short than too long, to 250 layers of 0.01 to 13 GFLOP, of which one takes longer this way by more than
+// 2 % (22.5 -> 24.9 us); kept where they were: 1x256x28x28, 256 3x3 filters (25 us), and nearly all layers below 15 us.
 ConvF32Split split_choice(const ConvF32Layer &layer, int window, double cycles) {
-    const ConvF32Split none{-1, 0, 0.};
-    if (window < 0) return none;
+    const ConvF32Split none{-1, 0, 0., 1};
     const ConvF32Split split = conv_f32_split_choose(layer);
     if (split.tile < 0 || split.us == 0) return split;
-    const bool vector = layer.c * layer.kh * layer.kw % 4 == 0 && (layer.kh == 1 || layer.kh == 3) && reinterpret_cast<uintptr_t>(layer.w_dev) % 16 == 0;
-    return split.us * 1.05 < cycles / 2200 * (vector ? 1.2 : 1.9) + 4 ? split : none;
+    if (cycles == 0) return none;
+    const int taps = layer.kh * layer.kw;
+    const bool vector = layer.c * taps % 4 == 0 && (layer.kh == 1 || layer.kh == 3) && reinterpret_cast<uintptr_t>(layer.w_dev) % 16 == 0;
+    int rows = 0, positions = 0;
+    if (window >= 0) conv_f32_window_tile_size(window, &rows, &positions);
+    const double factor = window < 0 ? (taps == 25 ? 1.1 : 2.) : vector ? (rows * positions == 1024 ? 1.35 : 1.) : taps == 1 ? 1.05 : 1.75;
+    const double other = 6 + factor * cycles / 2200 + 0.44 * layer.n * layer.ho * layer.wo * layer.cout * 4e-6;
+    return split.us * (window < 0 ? 1.25 : 1.05) < other ? split : none;
 }
 
 // What a layer beyond the small-layer kernel runs on: with its workspace, and without (-1: a kernel of this file).
@@ -751,7 +757,11 @@ ConvF32Plan conv_f32_plan(const ConvF32Layer &layer, const GemmArgs &g) {
         ConvF32Plan plan{};
         double cycles = 0;
         plan.window = window_tile(layer, g, &cycles);
-        plan.split = split_choice(layer, plan.window, cycles);
+        plan.split = {-1, 0, 0., 1};
+        const char *e = std::getenv("TSX_GEMM_F32_REGFED");
+        const bool small = plan.window < 0 && choose_gemm(g, 1) == GEMM_REGISTER_FED && !(e && e[0] == 'f');
+        if (small) conv_f32_window_tile(layer, &cycles);
+        if (small || plan.window >= 0) plan.split = split_choice(layer, plan.window, cycles);
         return plan;
     };
     if (!key.regfed.read("TSX_GEMM_F32_REGFED") || !key.tile.read("TSX_CONV_F32_TILE") || !key.split.read("TSX_CONV_F32_SPLIT")) return make();
@@ -837,7 +847,7 @@ int tsx_conv2d_f32_nchw_ws(const tsx_conv2d_geom *geo, const float *x_dev, const
     if (workspace_dev) {
         TSX_REQUIRE(reinterpret_cast<uintptr_t>(workspace_dev) % 16 == 0, "conv2d_f32: workspace not aligned to 16 bytes");
         if (plan.split.tile >= 0 && plan.split.workspace_bytes <= workspace_bytes)
-            return tsx::conv_f32_split(layer, plan.split.tile, bias_dev, act, slope, padding_value, out_dev, workspace_dev, tsx::as_stream(stream));
+            return tsx::conv_f32_split(layer, plan.split, bias_dev, act, slope, padding_value, out_dev, workspace_dev, tsx::as_stream(stream));
     }
     if (plan.window >= 0)
         return tsx::conv_f32_window(layer, plan.window, bias_dev, act, slope, padding_value, out_dev, tsx::as_stream(stream));
@@ -855,14 +865,14 @@ int tsx_conv2d_f32_plan_info(const tsx_conv2d_geom *geo, const float *w_oihw_dev
         return 0;
     }
     const tsx::ConvF32Layer layer = tsx::window_layer(geo, g, ld);
-    char with_workspace[128] = "";
+    char with_workspace[160] = "";
     const tsx::ConvF32Plan plan = tsx::conv_f32_plan(layer, g);
     const tsx::ConvF32Split split = plan.split;
     if (split.tile >= 0) {
         int rows, positions, patch;
         tsx::conv_f32_split_tile_size(split.tile, &rows, &positions, &patch);
-        std::snprintf(with_workspace, sizeof(with_workspace), " workspace_kernel=bf16_split workspace_tile=%dx%d workspace_patch=%d workspace_window=%s",
-                      rows, positions, patch, split.tile % 2 ? "flat" : "segments");
+        std::snprintf(with_workspace, sizeof(with_workspace), " workspace_kernel=bf16_split workspace_tile=%dx%d workspace_patch=%d workspace_window=%s workspace_slices=%d",
+                      rows, positions, patch, split.tile % 2 ? "flat" : "segments", split.slices);
     }
     const int win = plan.window;
     if (win >= 0) {            // a K-split 32-row tile or a larger one without, by its input patches
