@@ -99,7 +99,9 @@ __global__ __launch_bounds__(256) void pooling2d_kernel(const float *__restrict_
 // takes 16 planes, its wavefronts copy them to LDS in chunks with whole cache lines and all of a chunk's loads in flight,
 // and 16 lanes walk one plane each from there, the next chunk's loads on their way.  They read 32 elements ahead, 16 bytes at a
 // time (the pitch leaves them each their own four banks): the walk is then the chain of additions (read eight at a time where
-// they are used it waited for LDS: 32x256 planes of 28x28 15.4 -> 9.8 us).
+// they are used it waited for LDS: 32x256 planes of 28x28 10.7 -> 7.5 us, of 56x56 35.0 -> 22.5).  What is behind the last 32, and
+// planes of less than 64, go eight at a time (one at a time 32x2048 planes of 7x7 took 11.7 us, now 9.2; the last
+// 32 held in registers as well cost half the wavefronts in flight, 15).
 constexpr int GP_PLANES = 16, GP_CHUNK = 512, GP_PER = GP_CHUNK / 64, GP_ROWS = GP_PLANES / 4;
 
 __global__ __launch_bounds__(256) void global_pooling2d_kernel(const float *__restrict__ x, int64_t planes, int count, int type, float divisor,
@@ -128,7 +130,7 @@ __global__ __launch_bounds__(256) void global_pooling2d_kernel(const float *__re
         if (at + GP_CHUNK < count) load(at + GP_CHUNK);
         if (threadIdx.x < GP_PLANES) {
             const float *row = buf[threadIdx.x];
-            const int n = min(GP_CHUNK, count - at), blocks = n / 32;
+            const int n = min(GP_CHUNK, count - at), blocks = n < 64 ? 0 : n / 32;
             if (type == 0 && at == 0) acc = row[0];
             auto walk = [&](auto &&step) {
                 v4f even[8], odd[8];
@@ -142,13 +144,14 @@ __global__ __launch_bounds__(256) void global_pooling2d_kernel(const float *__re
 #pragma unroll
                         for (int j = 0; j < 4; ++j) step(from[i][j]);
                 };
-                read(even, 0);
+                if (blocks > 0) read(even, 0);
                 for (int b = 0; b < blocks; b += 2) {
                     read(odd, b + 1);
                     take(even);
                     read(even, b + 2);
                     if (b + 1 < blocks) take(odd);
                 }
+#pragma unroll 8
                 for (int i = blocks * 32; i < n; ++i) step(row[i]);
             };
             if (type == 0) walk([&](float v) { acc = v > acc ? v : acc; });

@@ -15,7 +15,8 @@ def _dev(a):
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 4, 4), (1, 17, 3, 7), (3, 11, 16, 32), (2, 9, 19, 27), (1, 33, 37, 41), (2, 3, 1, 31), (2, 3, 4, 8), (1, 5, 3, 33),
-                                   (1, 3, 24, 24), (2, 9, 34, 32)])
+                                   (1, 3, 24, 24), (2, 9, 34, 32),
+                                   (3, 19, 7, 7), (1, 5, 7, 9), (1, 3, 5, 19), (1, 3, 8, 12), (2, 3, 17, 33)])
 @pytest.mark.parametrize("kind", ["avg", "max"])
 def test_global_pooling(port, shape, kind):
     from tennis_amd import capi
