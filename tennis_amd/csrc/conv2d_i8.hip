@@ -1605,7 +1605,7 @@ int tsx_gemm_i8(int32_t m, int32_t n, int32_t k, const int8_t *a_dev, const void
         const auto set = [](const char *name) { const char *value = std::getenv(name); return value && value[0]; };
         const int row_blocks = int(tsx::ceil_div(m, 32));
         const int64_t tiles = tsx::ceil_div(n, 32) * row_blocks;
-        const bool few = (tiles <= 256 || (tiles <= 512 && tiles * kp <= 900000)) && !set("TSX_GEMM_I8_KSPLIT") && !set("TSX_GEMM_I8_TILE");
+        const bool few = m > 32 && (tiles <= 256 || (tiles <= 512 && tiles * kp <= 900000)) && !set("TSX_GEMM_I8_KSPLIT") && !set("TSX_GEMM_I8_TILE");
         if (m <= 32 || few) {
             if (p.x_bytes < 16 && (rc = pad_rows())) return rc;      // less than a piece
             if (m <= 32) hipLaunchKernelGGL(gemm_i8_skinny_kernel<false>, dim3(unsigned(tiles)), dim3(SK_WAVES * 64), 0, stream, p, 1);
