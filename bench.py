@@ -441,7 +441,7 @@ def kernels_leg(reps=20):
                   lambda a=a, rs=rs: gemm(a, dq=dq, row_scale=rs, bias=bias))
     ragged = capi.GemmI8(ri8(1500, 777))
     a, rdq, rqs = ri8(197, 1500), torch.rand(777, device=dev) * 1e-2, torch.full((197,), 32.0, device=dev)
-    timed("gemm_i8 197x777 K=1500, int8 out (gemm_i8_ksplit_lds_kernel)", "mfma_i8", 2.0 * 197 * 777 * 1500,
+    timed("gemm_i8 197x777 K=1500, int8 out (gemm_i8_skinny_kernel)", "mfma_i8", 2.0 * 197 * 777 * 1500,
           lambda: ragged(a, dq=rdq, q_scales=rqs, act="relu", want_f32=False))
     # memory-bound 1x1 int8 layer (ResNet stage 1 expansion, 64 -> 256 channels at 56x56, batch 32), staged int8 in, fp32 out
     xq = ri8(32, 64, 56, 56)
