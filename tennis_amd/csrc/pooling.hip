@@ -100,14 +100,15 @@ __global__ __launch_bounds__(256) void pooling2d_kernel(const float *__restrict_
 // and 16 lanes walk one plane each from there, the next chunk's loads on their way.  They read 32 elements ahead, 16 bytes at a
 // time (the pitch leaves them each their own four banks): the walk is then the chain of additions (read eight at a time where
 // they are used it waited for LDS: 32x256 planes of 28x28 10.7 -> 7.5 us, of 56x56 35.0 -> 22.5).  What is behind the last 32, and
-// planes of less than 64, go eight at a time (one at a time 32x2048 planes of 7x7 took 11.7 us, now 9.2; the last
+// planes of less than 64, go eight at a time (one at a time 32x2048 planes of 7x7 took 11.7 us, with the registers of the read-ahead 9.2, now 8.9; the last
 // 32 held in registers as well cost half the wavefronts in flight, 15).
 constexpr int GP_PLANES = 16, GP_CHUNK = 512, GP_PER = GP_CHUNK / 64, GP_ROWS = GP_PLANES / 4;
 
+template <bool AHEAD>      // planes of 64 elements and more
 __global__ __launch_bounds__(256) void global_pooling2d_kernel(const float *__restrict__ x, int64_t planes, int count, int type, float divisor,
                                                                float *__restrict__ out) {
     typedef float v4f __attribute__((ext_vector_type(4)));
-    __shared__ __attribute__((aligned(16))) float buf[GP_PLANES][GP_CHUNK + 4];
+    __shared__ __attribute__((aligned(16))) float buf[GP_PLANES][GP_CHUNK + (AHEAD ? 4 : 1)];
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     const int64_t first = int64_t(blockIdx.x) * GP_PLANES;
     float v[GP_ROWS][GP_PER];
@@ -130,7 +131,7 @@ __global__ __launch_bounds__(256) void global_pooling2d_kernel(const float *__re
         if (at + GP_CHUNK < count) load(at + GP_CHUNK);
         if (threadIdx.x < GP_PLANES) {
             const float *row = buf[threadIdx.x];
-            const int n = min(GP_CHUNK, count - at), blocks = n < 64 ? 0 : n / 32;
+            const int n = min(GP_CHUNK, count - at), blocks = AHEAD ? n / 32 : 0;
             if (type == 0 && at == 0) acc = row[0];
             auto walk = [&](auto &&step) {
                 v4f even[8], odd[8];
@@ -144,8 +145,8 @@ __global__ __launch_bounds__(256) void global_pooling2d_kernel(const float *__re
 #pragma unroll
                         for (int j = 0; j < 4; ++j) step(from[i][j]);
                 };
-                if (blocks > 0) read(even, 0);
-                for (int b = 0; b < blocks; b += 2) {
+                if (AHEAD) read(even, 0);
+                for (int b = 0; AHEAD && b < blocks; b += 2) {
                     read(odd, b + 1);
                     take(even);
                     read(even, b + 2);
@@ -346,7 +347,8 @@ int tsx_pooling2d_f32(const float *x_dev, int64_t planes, int32_t h, int32_t w, 
     if (out_h == 1 && out_w == 1 && pad_top == 0 && pad_left == 0 && kh >= h && kw >= w && h * int64_t(w) >= 16 && int64_t(h) * w < (1 << 30) &&
         plane_blocks * 256 < (int64_t(1) << 32)) {
         const float divisor = white_padding ? float(kh * kw) : float(h * w);
-        hipLaunchKernelGGL(global_pooling2d_kernel, dim3(unsigned(plane_blocks)), dim3(256), 0, tsx::as_stream(stream), x_dev,
+        const auto kernel = int64_t(h) * w < 64 ? global_pooling2d_kernel<false> : global_pooling2d_kernel<true>;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(plane_blocks)), dim3(256), 0, tsx::as_stream(stream), x_dev,
                            planes, h * w, type, divisor, out_dev);
         TSX_LAUNCH_CHECK("global_pooling2d_kernel");
         return 0;
