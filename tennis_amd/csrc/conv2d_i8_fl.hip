@@ -93,6 +93,15 @@ void fl_plan(const WsGeom &g, WsPlan *pl) {
     if (best <= ws_cost || force) pl->flat = true;
 }
 
+// The exact Mish's tables lie beside the windows: a layer whose windows leave no room for them keeps two at a time, or, where not
+// even those fit, its window-stationary tiles.
+static int fl_windows(const WsGeom &g, const WsPlan &pl, const EpiParams &ep) {
+    const int budget = ep.act == TSX_ACT_MISH ? FL_MAX_LDS_MISH : FL_MAX_LDS, window = pl.fl_wr * pl.fl_rowp;
+    return pl.fl_resident && g.cblocks * window <= budget ? g.cblocks : 2 * window <= budget ? 2 : 0;
+}
+
+bool fl_takes(const WsGeom &g, const WsPlan &pl, const EpiParams &ep) { return pl.flat && fl_windows(g, pl, ep) > 0; }
+
 int fl_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t *packed, const EpiParams &ep,
               hipStream_t stream) {
     FlParams p{};
@@ -124,7 +133,8 @@ int fl_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t 
     p.tiles = int(pl.fl_tiles);
     p.tiles_per_xcd = int((pl.fl_tiles + 7) / 8);
     p.positions = int(int64_t(g.n) * g.ho * g.wo);
-    p.resident = pl.fl_resident ? 1 : 0;
+    const int windows = fl_windows(g, pl, ep);
+    p.resident = pl.fl_resident && windows == g.cblocks ? 1 : 0;
     p.wc_magic = div_magic(p.wc, FL_MAX_WP);
     p.wo_magic = div_magic(p.wo, p.positions);
     p.ho_magic = div_magic(p.ho, int64_t(g.n) * g.ho);
@@ -132,7 +142,7 @@ int fl_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t 
     // an output of L2 size or more that no fused consumer reads: stream it
     p.stream_out = (!ep.residual && !ep.st_out && ep.out_f32 && int64_t(g.n) * g.cout * g.ho * g.wo * 4 >= (int64_t(16) << 20)) ? 1 : 0;
     const dim3 grid(unsigned(p.tiles_per_xcd * 8), unsigned((g.cout + 127) / 128));
-    const size_t lds_bytes = size_t(pl.fl_resident ? g.cblocks : 2) * pl.fl_wr * pl.fl_rowp;
+    const size_t lds_bytes = size_t(windows) * pl.fl_wr * pl.fl_rowp;
     const int key = pl.fl_nta * 10 + pl.fl_ntb;
     switch (key) {
         case 11: return fl_launch_nt<1, 1>(p, grid, lds_bytes, stream);

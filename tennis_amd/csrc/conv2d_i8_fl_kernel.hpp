@@ -13,7 +13,8 @@ constexpr int FL_PIX = 80;        // LDS bytes per window pixel (64 channels + 1
 constexpr int FL_THREADS = 512;   // 8 wavefronts: two per SIMD
 constexpr int FL_MAX_FILL = 4;    // window chunks per thread per channel block
 constexpr int FL_MAX_WP = FL_MAX_FILL * FL_THREADS / 4;   // 512 window pixels
-constexpr int FL_MAX_LDS = 160 * 1024 - 2048;             // LDS of one CU, all of it available to one workgroup, less the exact Mish's tables
+constexpr int FL_MAX_LDS = 160 * 1024;                    // LDS of one CU, all of it available to one workgroup
+constexpr int FL_MAX_LDS_MISH = FL_MAX_LDS - int(sizeof(MishTables));   // ... of the instantiations with the exact Mish's tables
 
 struct FlParams : EpiParams {
     const int8_t *xs;   // staged activations [n][hs][ws][cp]
@@ -481,7 +482,7 @@ int fl_launch_nt<TSX_FL_NTA, TSX_FL_NTB>(const FlParams &p, dim3 grid, size_t ld
         auto kernel = conv_i8_fl_kernel<NTA, NTB, EXTRA, STREAM, RESIDENT, SLOT == 3>;                        \
         if (lds_bytes > 65536 && dev < 64 && !granted[RESIDENT][SLOT][dev].load()) {                          \
             TSX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),                               \
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, FL_MAX_LDS));             \
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, SLOT == 3 ? FL_MAX_LDS_MISH : FL_MAX_LDS)); \
             granted[RESIDENT][SLOT][dev].store(true);                                                         \
         }                                                                                                     \
         hipLaunchKernelGGL(kernel, grid, dim3(FL_THREADS), lds_bytes, stream, p);                             \

@@ -230,7 +230,7 @@ int ws_launch(const WsGeom &g, const WsPlan &plan, const int8_t *xs, const int8_
     }
     if (pl.ks) return ks_launch(g, pl, xs, packed, ep, stream);
     if (rs_takes(pl, ep, int64_t(g.n) * g.cout * g.ho * g.wo)) return rs_launch(g, pl, xs, packed, ep, stream);
-    if (pl.flat) return fl_launch(g, pl, xs, packed, ep, stream);
+    if (fl_takes(g, pl, ep)) return fl_launch(g, pl, xs, packed, ep, stream);
     WsParams p{};
     static_cast<EpiParams &>(p) = ep;
     p.xs = xs;

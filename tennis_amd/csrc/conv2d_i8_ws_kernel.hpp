@@ -5,6 +5,8 @@
 #pragma once
 #include "igemm_i8.hpp"
 
+#include <atomic>
+
 namespace tsx {
 
 constexpr int RING = 4;         // A register ring depth (K-steps)
@@ -13,7 +15,7 @@ constexpr int WS_THREADS = 256;
 constexpr int WS_FM = 1;        // 32-cout fragments per wavefront
 constexpr int MAX_FILL = 7;     // window chunks per thread per channel block
 constexpr int SMALL_FILL = 4;   // ... of the kernels compiled for small windows (fewer registers: one more workgroup per CU)
-constexpr size_t WS_MAX_LDS = 65536 - sizeof(MishTables);   // both windows: 64 KiB less the tables of the exact Mish
+constexpr size_t WS_MAX_LDS = 65536;   // both windows; the exact Mish's tables come on top, in its layers only
 constexpr int MAX_WP = MAX_FILL * WS_THREADS / 4;   // 448 window pixels
 
 struct WsParams : EpiParams {
@@ -608,15 +610,21 @@ int ws_launch_nt<TSX_WS_NT>(const WsParams &p, dim3 grid, size_t lds_bytes, hipS
 #define TSX_WS_LAUNCH(EXTRA, STREAM, ROWM, MISHX)                                                                      \
     do {                                                                                                               \
         constexpr int F = NT <= 2 ? SMALL_FILL : MAX_FILL;                                                             \
-        if (NT == 1 && look)                                                                                           \
-            hipLaunchKernelGGL((conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, NT == 1, MISHX>), grid,           \
-                               dim3(WS_THREADS), lds_bytes, stream, p);                                                \
-        else if (NT <= 2 && small_fill)                                                                                \
-            hipLaunchKernelGGL((conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, false, MISHX>), grid,             \
-                               dim3(WS_THREADS), lds_bytes, stream, p);                                                \
-        else                                                                                                           \
-            hipLaunchKernelGGL((conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, MAX_FILL, false, MISHX>), grid,      \
-                               dim3(WS_THREADS), lds_bytes, stream, p);                                                \
+        const int fill = NT == 1 && look ? 0 : NT <= 2 && small_fill ? 1 : 2;                                          \
+        const auto kernel = fill == 0 ? conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, NT == 1, MISHX>           \
+                            : fill == 1 ? conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, false, MISHX>           \
+                                        : conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, MAX_FILL, false, MISHX>;   \
+        if (MISHX && lds_bytes + sizeof(MishTables) > 65536) {      /* granted per kernel and device */                \
+            static std::atomic<bool> granted[3][64];                                                                   \
+            int dev = 0;                                                                                               \
+            TSX_HIP(hipGetDevice(&dev));                                                                               \
+            if (dev >= 64 || !granted[fill][dev].load()) {                                                             \
+                TSX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),                                    \
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, int(WS_MAX_LDS)));             \
+                if (dev < 64) granted[fill][dev].store(true);                                                          \
+            }                                                                                                          \
+        }                                                                                                              \
+        hipLaunchKernelGGL(kernel, grid, dim3(WS_THREADS), lds_bytes, stream, p);                                      \
     } while (0)
     // the exact Mish: one instantiation (with every other epilogue term) that only its layers run
     if (p.act == TSX_ACT_MISH) {

@@ -207,8 +207,10 @@ WsPlan ws_plan(const WsGeom &g);
 int ws_pack_weights(const WsGeom &g, const WsPlan &pl, const int8_t *w_oihw, int c, int8_t *packed, hipStream_t stream);
 int ws_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t *packed, const EpiParams &ep,
               hipStream_t stream);
-// flat-tile kernel: fills the fl_* fields of a valid plan when the layer suits it; launch
+// flat-tile kernel: fills the fl_* fields of a valid plan when the layer suits it; whether it has the LDS for a given
+// epilogue; launch
 void fl_plan(const WsGeom &g, WsPlan *pl);
+bool fl_takes(const WsGeom &g, const WsPlan &pl, const EpiParams &ep);
 int fl_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t *packed, const EpiParams &ep,
               hipStream_t stream);
 // weight-stationary kernel: fills the rs_* fields of a valid plan when the layer suits it; whether it writes a

@@ -163,6 +163,22 @@ def test_other_kernels_switches_keep_layers_off_the_k_split_kernel_where_they_ha
         assert kernel(**{name: "0", "KS": "0"}) == "window_stationary"
 
 
+@pytest.mark.parametrize("layer, fragments, tiles", [
+    ((10, 287, 139, 59, 162, 3, 2, 1), 3, 512), ((28, 330, 130, 134, 23, 5, 2, 2), 1, 1820), ((31, 54, 50, 50, 28, 5, 1, 2), 2, 310),
+])
+def test_int8_windows_may_fill_64_kib(monkeypatch, layer, fragments, tiles):
+    """The largest tile whose two windows fit: what only some activations need in LDS beside them is no other layer's loss."""
+    from tennis_amd import capi
+    for name in ("FLAT", "RS", "KS"):
+        monkeypatch.delenv("TSX_CONV_I8_" + name, raising=False)
+    n, c, h, w, cout, k, stride, pad = layer
+    geom = capi.ConvGeom(n, c, h, w, cout, k, k, pad, pad, pad, pad, stride, stride, 1, 1)
+    buf = ctypes.create_string_buffer(256)
+    assert capi.lib().tsx_conv2d_i8_plan_info(ctypes.byref(geom), buf, len(buf)) == 0
+    info = dict(word.split("=", 1) for word in buf.value.decode().split())
+    assert info["kernel"] == "window_stationary" and (int(info["fragments_per_wavefront"]), int(info["tiles"])) == (fragments, tiles)
+
+
 def test_kept_fp32_plans_follow_what_they_depend_on(monkeypatch):
     """A thread keeps its plans: with every switch, weights' alignment and geometry in turn they are what a thread that has
     planned nothing yet answers."""

@@ -58,3 +58,35 @@ def test_every_kind_of_argument(port, monkeypatch, images, side, join):
     q = conv.run_staged(staged, dev(np.ones(cout, np.float32)), dev(bias), "mish", 0.0, q_scales=dev(scales), want_f32=False,
                         residual=None if res is None else dev(res), residual_after_act=join == "after")[1]
     assert np.array_equal(q.cpu().numpy(), expected)
+
+
+@pytest.mark.parametrize("act", ["leaky_relu", "mish"])
+@pytest.mark.parametrize("case", [
+    # n, c, h, w, cout, (kh, kw), stride, pads, forced flat tile: windows that leave no room for the exact Mish's tables in 64 KiB ...
+    (15, 70, 47, 47, 17, (5, 5), 2, 2, None), (2, 70, 189, 189, 17, (3, 3), 2, 1, None), (7, 130, 91, 26, 57, (5, 5), 2, 2, None),
+    # ... or, all the layer's windows at once, in 160 (two of them do), or not even two
+    (7, 300, 5, 10, 70, (3, 3), 1, 1, "33"), (6, 300, 11, 7, 130, (3, 3), 1, 1, "43"), (1, 70, 300, 2, 70, (42, 2), 1, 0, "32"),
+], ids=lambda c: "-".join(map(str, c)))
+def test_windows_of_the_whole_lds(port, monkeypatch, case, act):
+    from tennis_amd import capi
+    n, c, h, w, cout, kernel, stride, pad, flat = case
+    monkeypatch.setenv("TSX_CONV_I8_KS", "0")
+    monkeypatch.setenv("TSX_CONV_I8_RS", "0")
+    monkeypatch.setenv("TSX_CONV_I8_FLAT", "force" + flat if flat else "0")
+    rng = np.random.default_rng(17)
+    x = rng.integers(-128, 128, (n, c, h, w)).astype(np.int8)
+    wt = rng.integers(-127, 128, (cout, c) + kernel).astype(np.int8)
+    dq = rng.uniform(1e-5, 3e-5, cout).astype(np.float32)
+    bias = rng.standard_normal(cout).astype(np.float32)
+    qs = rng.uniform(20, 30, n).astype(np.float32)
+    conv = capi.Conv2dI8(dev(wt), (pad,) * 4, (stride, stride))
+    info = capi.conv2d_i8_plan_info(conv._plan(x.shape)[0])
+    assert info["kernel"] == ("flat_tile" if flat else "window_stationary"), info
+    plain = port.add_bias(port.conv2d_quantized(x, wt, dq, (pad,) * 4, (stride, stride)), bias)
+    res = rng.standard_normal(plain.shape).astype(np.float32)
+    value = port.mish(plain) if act == "mish" else port.leaky_relu(plain, 0.1)
+    for join, expected in ((None, value), (res, port.add(value, res))):
+        out, q, _ = conv(dev(x), dq=dev(dq), bias=dev(bias), act=act, slope=0.1, q_scales=dev(qs), residual=None if join is None else dev(join),
+                         residual_after_act=join is not None)
+        assert np.array_equal(out.cpu().numpy().view(np.int32), expected.view(np.int32))
+        assert np.array_equal(q.cpu().numpy(), port.quantize(expected, qs))
