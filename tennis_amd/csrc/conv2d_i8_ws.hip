@@ -158,10 +158,14 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
             // workgroups in flight per CU (us, 32 images: 64 to 256 channels 56x56 with a residual join, 4 fragments per
             // wavefront 63, 2 46; 256 to 128 56x56 20.9 -> 16.9; 256 to 1024 14x14 with a join 18.1 -> 17.4).
             if (!several_taps && (!g.gemm || g.cblocks <= 2) && nt > 2) continue;
-            // Two fragments share a wavefront's set-up; a grid of less than one and a half workgroups per CU takes one (us, one /
-            // two: 32 images 256 to 64 56x56 14.5 / 14.0, 128 to 512 28x28 with a join 26.8 / 25.6, 512 to 2048 7x7 13.2 / 11.4,
-            // but 1024 to 256 14x14 9.5 / 10.0, 2048 to 512 7x7 11.5 / 13.5).
-            if (!several_taps && !g.gemm && g.wo == 1 && g.ho >= 64 * wn &&
+            // Two fragments share a wavefront's set-up, which pays where every fragment's channels exist and its stores are whole
+            // cache lines, that is, where a plane is a multiple of 64 bytes of fp32 (us, one / two: 32 images 256 to 64 56x56 14.5 / 14.0,
+            // 128 to 512 28x28 with a join 26.8 / 25.6, 13x48x48, 36 to 256, 15.9 / 14.9; 30 such layers 3 % on average, between
+            // -14 % and 7 %).  Elsewhere the model above decides, mostly for one (plane lengths not a multiple of 16: 13x29x226x74 to 52
+            // 31.3 / 40.0, 12x8x29x29, 3x3, to 776 23.6 / 27.8; channels not of 32: 24x6x91x91 to 47 24.9 / 33.0, 3x96x122x27 to 801
+            // 28.0 / 34.2; 32 channels, a join: 28.7 / 32.0), as for a grid of less than one and a half workgroups per CU (1024 to
+            // 256 14x14 9.5 / 10.0).  Only pixels in a row (hs == ho): any tile of them fits.
+            if (!several_taps && !g.gemm && g.wo == 1 && g.hs == g.ho && g.ho % 16 == 0 && g.cout % 32 == 0 && wm >= 2 && g.ho >= 64 * wn &&
                 nt == (ceil_div(int64_t(g.n) * g.ho, 64 * wn) * (coutp / bm) >= 384 ? 1 : 2)) continue;
             if (best_cost < 0 || cost < best_cost || (cost == best_cost && frags < best_frags)) {
                 best_cost = cost;

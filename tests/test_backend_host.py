@@ -179,6 +179,26 @@ def test_int8_windows_may_fill_64_kib(monkeypatch, layer, fragments, tiles):
     assert info["kernel"] == "window_stationary" and (int(info["fragments_per_wavefront"]), int(info["tiles"])) == (fragments, tiles)
 
 
+@pytest.mark.parametrize("layer, fragments", [
+    # two where fragments are whole and planes are whole cache lines ...
+    ((32, 256, 56, 56, 64, 1, 1, 0), "2"), ((32, 128, 28, 28, 512, 1, 1, 0), "2"),
+    # ... the model's one where they are not
+    ((13, 29, 226, 74, 52, 1, 1, 0), "1"), ((24, 6, 91, 91, 47, 1, 1, 0), "1"), ((13, 8, 29, 29, 776, 3, 1, 0), "1"),
+    ((3, 96, 122, 27, 801, 1, 1, 0), "1"), ((7, 168, 166, 176, 32, 1, 1, 0), "1"),
+])
+def test_int8_layers_of_one_tap_take_two_fragments_where_that_pays(monkeypatch, layer, fragments):
+    from tennis_amd import capi
+    for name in ("FLAT", "RS"):
+        monkeypatch.delenv("TSX_CONV_I8_" + name, raising=False)
+    monkeypatch.setenv("TSX_CONV_I8_KS", "0")
+    n, c, h, w, cout, k, stride, pad = layer
+    geom = capi.ConvGeom(n, c, h, w, cout, k, k, pad, pad, pad, pad, stride, stride, 1, 1)
+    buf = ctypes.create_string_buffer(256)
+    assert capi.lib().tsx_conv2d_i8_plan_info(ctypes.byref(geom), buf, len(buf)) == 0
+    info = dict(word.split("=", 1) for word in buf.value.decode().split())
+    assert (info["kernel"], info["fragments_per_wavefront"]) == ("window_stationary", fragments)
+
+
 def test_kept_fp32_plans_follow_what_they_depend_on(monkeypatch):
     """A thread keeps its plans: with every switch, weights' alignment and geometry in turn they are what a thread that has
     planned nothing yet answers."""
