@@ -421,10 +421,9 @@ __device__ __forceinline__ void fl_wave(const FlParams &p, int8_t *lds, MishTabl
                 v16f d, b;
                 static_for<0, 16>([&](auto rc) { d[decltype(rc)::value] = dq[decltype(rc)::value], b[decltype(rc)::value] = bias[decltype(rc)::value]; });
 #pragma clang loop unroll(disable)
-                for (int r = 0; r < 16; ++r) {
-                    const int dco = 8 * (r / 4) + (r % 4);
-                    if (pok[j] && co0 + dco < p.cout) emit<true>(p, a[r], base + int64_t(dco) * howo, d[r], b[r], 0.f);
-                }
+                for (int r = 0; r < 16; r += 4)
+                    emit_rows4<true>(p, {a[r], a[r + 1], a[r + 2], a[r + 3]}, base + int64_t(2 * r) * howo, howo, pok[j] ? p.cout - co0 - 2 * r : 0,
+                                     {d[r], d[r + 1], d[r + 2], d[r + 3]}, {b[r], b[r + 1], b[r + 2], b[r + 3]}, MishTablesInLds{mish_tables});
             } else static_for<0, 16>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
                 constexpr int dco = 8 * (r / 4) + (r % 4);

@@ -88,6 +88,60 @@ __device__ __forceinline__ void emit(const EpiParams &p, int acc, int64_t idx, f
     }
 }
 
+// The same for four consecutive output channels of one position of a convolution, `left` of which exist (idx0: the first one's
+// element, row_stride: a plane).  What emit does for one channel waits for its loads and divides 64-bit indices; here the four
+// channels' loads are requested together (those of channels that do not exist read the last one again) and the indices are taken
+// apart once.  One channel per turn of a loop, layers with ragged channels and a join, or with the exact Mish, took up to a fifth
+// longer than with all sixteen of a fragment unrolled, and these are most of a kernel's code.
+template <bool MISHX, class Table>
+__device__ __forceinline__ void emit_rows4(const EpiParams &p, const int (&acc)[4], int64_t idx0, int row_stride, int left, const float (&dq)[4],
+                                           const float (&bias)[4], const Table &table) {
+    if (left <= 0) return;
+    int64_t at[4];
+    auto each = [&](auto &&f) __attribute__((always_inline)) { static_for<0, 4>(f); };
+    each([&](auto rc) { constexpr int r = decltype(rc)::value; at[r] = idx0 + int64_t(min(r, left - 1)) * row_stride; });
+    if (p.out_acc) each([&](auto rc) { constexpr int r = decltype(rc)::value; if (r < left) p.out_acc[at[r]] = acc[r]; });
+    if (!p.out_f32 && !p.out_i8 && !p.st_out) return;
+    float v[4], res[4] = {};
+    if (p.residual) each([&](auto rc) { constexpr int r = decltype(rc)::value; res[r] = p.residual[at[r]]; });
+    each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fmul_rn(float(acc[r]), dq[r]); });
+    if (p.bias) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], bias[r]); });
+    if (p.residual && !p.res_after) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], res[r]); });
+    if (MISHX) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_value(v[r], table); });
+    else if (p.act == TSX_ACT_MISH_FAST) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_short(v[r]); });
+    else if (p.act != TSX_ACT_NONE) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = apply_act_basic(v[r], p.act, p.slope, at[r] < p.act_body); });
+    if (p.residual && p.res_after) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], res[r]); });
+    if (p.out_f32) each([&](auto rc) { constexpr int r = decltype(rc)::value; if (r < left) p.out_f32[at[r]] = v[r]; });
+    if (!p.out_i8 && !p.st_out) return;
+    uint32_t word = 0;
+    if (p.n_qscales == 1) {
+        const float scale = p.q_scales[0];
+        each([&](auto rc) { constexpr int r = decltype(rc)::value; word = quantize_pack<r>(__fmul_rn(v[r], scale), at[r] < p.q_bulk8, word); });
+    } else {
+        const int64_t group = idx0 / p.q_group_len, next = (group + 1) * p.q_group_len;
+        const float scale = p.q_scales[group];
+        each([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            word = quantize_pack<r>(__fmul_rn(v[r], r == 0 || at[r] < next ? scale : p.q_scales[at[r] / p.q_group_len]), false, word);
+        });
+    }
+    word ^= 0x80808080u;
+    if (p.out_i8) each([&](auto rc) { constexpr int r = decltype(rc)::value; if (r < left) p.out_i8[at[r]] = int8_t(word >> (8 * r)); });
+    if (p.st_out) {
+        const int64_t row = idx0 / p.o_w, plane = row / p.o_h, image = plane / p.o_c;
+        const int ow = int(idx0 - row * p.o_w), oh = int(row - plane * p.o_h), co = int(plane - image * p.o_c), up = p.st_up == 2 ? 2 : 1;
+        int8_t *dst = p.st_out + ((image * p.st_hs + up * oh + p.st_pt) * p.st_ws + up * ow + p.st_pl) * p.st_cp + co;
+        each([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            if (r < left) {
+                const int8_t q = int8_t(word >> (8 * r));
+                dst[r] = q;
+                if (up == 2) dst[p.st_cp + r] = dst[int64_t(p.st_ws) * p.st_cp + r] = dst[int64_t(p.st_ws + 1) * p.st_cp + r] = q;
+            }
+        });
+    }
+}
+
 // Epilogue of one 32x32 accumulator fragment for one lane, rows = output channels: accumulator r is
 // channel row 8*(r/4) + (r%4) relative to the lane's first row, at linear index idx0 + row * row_stride.
 // One pass per epilogue term behind a single uniform branch each (testing the uniform options per

@@ -49,3 +49,42 @@ def test_conv_i8_tiles(port, monkeypatch, case, act):
     assert np.array_equal(bits(out.cpu().numpy()), bits(joined))
     got = second.run_staged(to, dev(dq2))[0].cpu().numpy()
     assert np.array_equal(bits(got), bits(port.conv2d_quantized(port.quantize(joined, qs), second.w.cpu().numpy(), dq2, (1, 1, 1, 1))))
+
+
+@pytest.mark.parametrize("n", [1, 2])
+@pytest.mark.parametrize("act", ["mish", "mish_fast", "relu"])
+@pytest.mark.parametrize("cout", [9, 18, 33, 47, 63, 65])
+def test_channels_of_partial_fragments(port, monkeypatch, cout, act, n):
+    """Fragments whose 32 channels do not all exist, with a join: raw sums, fp32, NCHW int8 (one image: half to even up to the last
+    whole eight; two: a scale each) and staged int8, by itself and upsampled."""
+    from tennis_amd import capi
+    monkeypatch.setenv("TSX_CONV_I8_KS", "0")
+    c, h, w = 70, 11, 9
+    rng = np.random.default_rng(cout)
+    x = rng.integers(-128, 128, (n, c, h, w)).astype(np.int8)
+    wt = rng.integers(-127, 128, (cout, c, 1, 1)).astype(np.int8)
+    dq = rng.uniform(1e-4, 3e-4, cout).astype(np.float32)
+    bias = rng.standard_normal(cout).astype(np.float32)
+    qs = rng.uniform(20, 30, n).astype(np.float32)
+    conv = capi.Conv2dI8(dev(wt))
+    plain = port.add_bias(port.conv2d_quantized(x, wt, dq), bias)
+    res = rng.standard_normal(plain.shape).astype(np.float32)
+    activated = port.relu(plain) if act == "relu" else port.mish(plain)
+    if act == "mish_fast":       # the short form's values, by a layer whose epilogue has no join
+        short = conv(dev(x), dq=dev(dq), bias=dev(bias), act=act)[0].cpu().numpy()
+        assert np.all(np.abs(short - activated) <= 6 * 2.0 ** -24 * np.abs(plain))
+        activated = short
+    joined = port.add(activated, res)
+    expected = port.quantize(joined, qs)
+    out, q, acc = conv(dev(x), dq=dev(dq), bias=dev(bias), act=act, q_scales=dev(qs), residual=dev(res), residual_after_act=True, want_acc=True)
+    assert np.array_equal(acc.cpu().numpy(), np.einsum("nchw,oc->nohw", x.astype(np.int32), wt[:, :, 0, 0].astype(np.int32)))
+    assert np.array_equal(bits(out.cpu().numpy()), bits(joined)) and np.array_equal(q.cpu().numpy(), expected)
+    q = conv(dev(x), dq=dev(dq), bias=dev(bias), act=act, q_scales=dev(qs), residual=dev(res), residual_after_act=True, want_f32=False)[1]
+    assert np.array_equal(q.cpu().numpy(), expected)
+    staged = capi.StagedInput(conv, x.shape)
+    conv.stage(dev(x), staged)
+    for up in (1, 2):
+        to = capi.StagedInput(capi.Conv2dI8(dev(np.zeros((8, cout, 3, 3), np.int8)), (1, 1, 1, 1)), (n, cout, up * h, up * w))
+        to = to if up == 1 else capi.StagedSlice(to, 0, cout, upsample=2)
+        conv.run_staged(staged, dev(dq), dev(bias), act, 0.0, q_scales=dev(qs), want_f32=False, residual=dev(res), residual_after_act=True, staged_out=to)
+        assert np.array_equal(capi.staged_interior(to, range(n)).cpu().numpy(), port.quantize(joined, qs))
