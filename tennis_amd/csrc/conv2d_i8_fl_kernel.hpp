@@ -418,12 +418,18 @@ __device__ __forceinline__ void fl_wave(const FlParams &p, int8_t *lds, MishTabl
             const int64_t base = (int64_t(pimg[j]) * p.cout + co0) * howo + prem[j];
             if constexpr (MISHX) {
                 const v16i a = acc[j];        // (a loop: unrolled, the inlined Mish is most of the kernel's code)
+                const auto pixel = [&](int &row, int &col) {
+                    row = udiv(prem[j], p.wo, p.wo_magic);
+                    col = prem[j] - row * p.wo;
+                };
                 v16f d, b;
                 static_for<0, 16>([&](auto rc) { d[decltype(rc)::value] = dq[decltype(rc)::value], b[decltype(rc)::value] = bias[decltype(rc)::value]; });
 #pragma clang loop unroll(disable)
-                for (int r = 0; r < 16; r += 4)
-                    emit_rows4<true>(p, {a[r], a[r + 1], a[r + 2], a[r + 3]}, base + int64_t(2 * r) * howo, howo, pok[j] ? p.cout - co0 - 2 * r : 0,
-                                     {d[r], d[r + 1], d[r + 2], d[r + 3]}, {b[r], b[r + 1], b[r + 2], b[r + 3]}, MishTablesInLds{mish_tables});
+                for (int r = 0; r < 16; r += 2) {
+                    const int dco = 8 * (r / 4) + r % 4;
+                    emit_rows<2, true>(p, {a[r], a[r + 1]}, base + int64_t(dco) * howo, howo, pok[j] ? p.cout - co0 - dco : 0, pimg[j], co0 + dco,
+                                       pixel, {d[r], d[r + 1]}, {b[r], b[r + 1]}, MishTablesInLds{mish_tables});
+                }
             } else static_for<0, 16>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
                 constexpr int dco = 8 * (r / 4) + (r % 4);

@@ -577,12 +577,19 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
                 if constexpr (EXTRA) {
                     // a loop that stays one, like mish_fragment's: unrolled it is most of the kernel's code
                     const v16i a = acc[f][j];
+                    const auto pixel = [&](int &row, int &col) {      // (this kernel's rows may be virtual)
+                        const int pix = oh * p.wo + ow;
+                        row = p.wo == p.o_w ? oh : udiv(pix, p.o_w, p.ow_magic);
+                        col = pix - row * p.o_w;
+                    };
                     v16f d, b;
                     static_for<0, 16>([&](auto rc) { d[decltype(rc)::value] = dq[decltype(rc)::value], b[decltype(rc)::value] = bias[decltype(rc)::value]; });
 #pragma clang loop unroll(disable)
-                    for (int r = 0; r < 16; r += 4)
-                        emit_rows4<MISHX>(p, {a[r], a[r + 1], a[r + 2], a[r + 3]}, base + int64_t(2 * r) * howo, howo, pos_ok ? p.cout - co0 - 2 * r : 0,
-                                          {d[r], d[r + 1], d[r + 2], d[r + 3]}, {b[r], b[r + 1], b[r + 2], b[r + 3]}, MishTablesInLds{&mish_tables});
+                    for (int r = 0; r < 16; r += 2) {
+                        const int dco = 8 * (r / 4) + r % 4;
+                        emit_rows<2, MISHX>(p, {a[r], a[r + 1]}, base + int64_t(dco) * howo, howo, pos_ok ? p.cout - co0 - dco : 0, img + (wrapped ? 1 : 0),
+                                            co0 + dco, pixel, {d[r], d[r + 1]}, {b[r], b[r + 1]}, MishTablesInLds{&mish_tables});
+                    }
                 } else static_for<0, 16>([&](auto rc) {
                     constexpr int r = decltype(rc)::value;
                     constexpr int dco = 8 * (r / 4) + (r % 4);

@@ -8,6 +8,7 @@ namespace tsx {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 struct EpiParams {
     const float *dq, *row_scale, *bias, *q_scales;
@@ -88,49 +89,48 @@ __device__ __forceinline__ void emit(const EpiParams &p, int acc, int64_t idx, f
     }
 }
 
-// The same for four consecutive output channels of one position of a convolution, `left` of which exist (idx0: the first one's
-// element, row_stride: a plane).  What emit does for one channel waits for its loads and divides 64-bit indices; here the four
-// channels' loads are requested together (those of channels that do not exist read the last one again) and the indices are taken
-// apart once.  One channel per turn of a loop, layers with ragged channels and a join, or with the exact Mish, took up to a fifth
-// longer than with all sixteen of a fragment unrolled, and these are most of a kernel's code.
-template <bool MISHX, class Table>
-__device__ __forceinline__ void emit_rows4(const EpiParams &p, const int (&acc)[4], int64_t idx0, int row_stride, int left, const float (&dq)[4],
-                                           const float (&bias)[4], const Table &table) {
+// The same for N consecutive output channels of one position of a convolution, from channel `co` on, `left` of which exist (idx0: the
+// first one's element, row_stride: a plane).  What emit does for one channel waits for its loads and takes a linear index apart by
+// 64-bit divisions; here the channels' loads are requested together (those of channels that do not exist read the last one again), and
+// the caller knows where it is (pixel: its output row and column).  The kernels call it in a loop that stays one, since unrolled it is
+// most of their code.  N = 2: 400 layers of ragged channels with a join or the exact Mish take 0.93 of what they took with emit
+// unrolled sixteen times, none more than 3 % longer; in a loop of one channel they took up to 1.2 times as long.  Four channels
+// are 0.91, but their scalar registers cost the layers of whole fragments 1 % (the YOLOv4 shape).
+template <int N, bool MISHX, class Table, class Pixel>
+__device__ __forceinline__ void emit_rows(const EpiParams &p, const int (&acc)[N], int64_t idx0, int row_stride, int left, int image, int co,
+                                          const Pixel &pixel, const float (&dq)[N], const float (&bias)[N], const Table &table) {
     if (left <= 0) return;
-    int64_t at[4];
-    auto each = [&](auto &&f) __attribute__((always_inline)) { static_for<0, 4>(f); };
-    each([&](auto rc) { constexpr int r = decltype(rc)::value; at[r] = idx0 + int64_t(min(r, left - 1)) * row_stride; });
-    if (p.out_acc) each([&](auto rc) { constexpr int r = decltype(rc)::value; if (r < left) p.out_acc[at[r]] = acc[r]; });
+    auto each = [&](auto &&f) __attribute__((always_inline)) { static_for<0, N>(f); };
+    int at[N];       // from idx0
+    each([&](auto rc) { constexpr int r = decltype(rc)::value; at[r] = min(r, left - 1) * row_stride; });
+    if (p.out_acc) each([&](auto rc) { constexpr int r = decltype(rc)::value; if (r < left) (p.out_acc + idx0)[at[r]] = acc[r]; });
     if (!p.out_f32 && !p.out_i8 && !p.st_out) return;
-    float v[4], res[4] = {};
-    if (p.residual) each([&](auto rc) { constexpr int r = decltype(rc)::value; res[r] = p.residual[at[r]]; });
+    float v[N], res[N] = {};
+    if (p.residual) each([&](auto rc) { constexpr int r = decltype(rc)::value; res[r] = (p.residual + idx0)[at[r]]; });
     each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fmul_rn(float(acc[r]), dq[r]); });
     if (p.bias) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], bias[r]); });
     if (p.residual && !p.res_after) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], res[r]); });
     if (MISHX) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_value(v[r], table); });
     else if (p.act == TSX_ACT_MISH_FAST) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_short(v[r]); });
-    else if (p.act != TSX_ACT_NONE) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = apply_act_basic(v[r], p.act, p.slope, at[r] < p.act_body); });
+    else if (p.act != TSX_ACT_NONE) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = apply_act_basic(v[r], p.act, p.slope, idx0 + at[r] < p.act_body); });
     if (p.residual && p.res_after) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], res[r]); });
-    if (p.out_f32) each([&](auto rc) { constexpr int r = decltype(rc)::value; if (r < left) p.out_f32[at[r]] = v[r]; });
+    if (p.out_f32) each([&](auto rc) { constexpr int r = decltype(rc)::value; if (r < left) (p.out_f32 + idx0)[at[r]] = v[r]; });
     if (!p.out_i8 && !p.st_out) return;
+    const float s = p.q_scales[p.n_qscales == 1 ? 0 : image];
+    float scale[N];
+    each([&](auto rc) { scale[decltype(rc)::value] = s; });
+    // a group's length is rounded in float: in large tensors it is not an image's
+    if (p.n_qscales != 1 && p.q_group_len != int64_t(p.o_c) * row_stride)
+        each([&](auto rc) { constexpr int r = decltype(rc)::value; scale[r] = p.q_scales[(idx0 + at[r]) / p.q_group_len]; });
     uint32_t word = 0;
-    if (p.n_qscales == 1) {
-        const float scale = p.q_scales[0];
-        each([&](auto rc) { constexpr int r = decltype(rc)::value; word = quantize_pack<r>(__fmul_rn(v[r], scale), at[r] < p.q_bulk8, word); });
-    } else {
-        const int64_t group = idx0 / p.q_group_len, next = (group + 1) * p.q_group_len;
-        const float scale = p.q_scales[group];
-        each([&](auto rc) {
-            constexpr int r = decltype(rc)::value;
-            word = quantize_pack<r>(__fmul_rn(v[r], r == 0 || at[r] < next ? scale : p.q_scales[at[r] / p.q_group_len]), false, word);
-        });
-    }
+    each([&](auto rc) { constexpr int r = decltype(rc)::value; word = quantize_pack<r>(__fmul_rn(v[r], scale[r]), p.n_qscales == 1 && idx0 + at[r] < p.q_bulk8, word); });
     word ^= 0x80808080u;
-    if (p.out_i8) each([&](auto rc) { constexpr int r = decltype(rc)::value; if (r < left) p.out_i8[at[r]] = int8_t(word >> (8 * r)); });
+    if (p.out_i8) each([&](auto rc) { constexpr int r = decltype(rc)::value; if (r < left) (p.out_i8 + idx0)[at[r]] = int8_t(word >> (8 * r)); });
     if (p.st_out) {
-        const int64_t row = idx0 / p.o_w, plane = row / p.o_h, image = plane / p.o_c;
-        const int ow = int(idx0 - row * p.o_w), oh = int(row - plane * p.o_h), co = int(plane - image * p.o_c), up = p.st_up == 2 ? 2 : 1;
-        int8_t *dst = p.st_out + ((image * p.st_hs + up * oh + p.st_pt) * p.st_ws + up * ow + p.st_pl) * p.st_cp + co;
+        int oh, ow;
+        pixel(oh, ow);
+        const int up = p.st_up == 2 ? 2 : 1;
+        int8_t *dst = p.st_out + ((int64_t(image) * p.st_hs + up * oh + p.st_pt) * p.st_ws + up * ow + p.st_pl) * p.st_cp + co;
         each([&](auto rc) {
             constexpr int r = decltype(rc)::value;
             if (r < left) {
