@@ -551,15 +551,6 @@ bool plan_tile(const ConvF32Layer &l, int tile, bool flat, SplitParams *p) {
     const int64_t tiles_n = flat ? ceil_div(p->N, bn) : int64_t(l.n) * ceil_div(l.ho, bn / 32) * p->col_tiles;
     if (tiles_n * p->tiles_m >= (int64_t(1) << 22)) return false;
     p->tiles_n = int(tiles_n);
-    p->by_tiles = divisor(tiles_n * p->tiles_m);
-    p->by_tiles_m = divisor(p->tiles_m);
-    p->by_col_tiles = divisor(p->col_tiles);
-    p->by_seg_rows = divisor(ceil_div(l.ho, bn / 32));
-    p->by_wo = divisor(p->wo);
-    p->by_ho = divisor(p->ho);
-    p->by_howo = divisor(p->howo);
-    p->by_hv = divisor(p->hv);
-    p->by_wv = divisor(p->wv);
     if (k > 1) {
         // rows of the largest patch: output rows a tile touches, and per image border it crosses the padding rows between
         const int64_t rows = flat ? ceil_div(bn + l.wo - 1, l.wo) : bn / 32;
@@ -570,6 +561,19 @@ bool plan_tile(const ConvF32Layer &l, int tile, bool flat, SplitParams *p) {
     if (w_bytes > (int64_t(1) << 31) - 64) return false;
     p->w_bytes = unsigned(w_bytes);
     return true;
+}
+
+// What a launch needs beyond the plan (not a part of it: nine divisions of 64 bits for each of some fifteen tiles were half of its time).
+void set_divisors(SplitParams *p, int bn) {
+    p->by_tiles = divisor(int64_t(p->tiles_n) * p->tiles_m);
+    p->by_tiles_m = divisor(p->tiles_m);
+    p->by_col_tiles = divisor(p->col_tiles);
+    p->by_seg_rows = divisor(ceil_div(p->ho, bn / 32));
+    p->by_wo = divisor(p->wo);
+    p->by_ho = divisor(p->ho);
+    p->by_howo = divisor(p->howo);
+    p->by_hv = divisor(p->hv);
+    p->by_wv = divisor(p->wv);
 }
 
 }  // namespace
@@ -599,14 +603,23 @@ ConvF32Split conv_f32_split_choose(const ConvF32Layer &l) {
             // (rms); the combinations it picks take 1 % longer than the fastest.
             const bool eight = t.wm * t.wn == 8, alone = t.pitch > 384, whole = l.c % 8 == 0;
             const double sums = double(positions) * l.cout * 4e-6, weights = double(l.cout) * l.c * t.taps * 1e-6;
-            for (int slices = 1; slices <= p.chunks; ++slices) {
-                const int each = int(ceil_div(p.chunks, slices));
-                if (only >= 0 ? slices != int(ceil_div(p.chunks, ceil_div(p.chunks, only_slices))) : ceil_div(p.chunks, each) != slices) continue;
-                const double tiles = double(p.tiles_m) * p.tiles_n * slices / 256, up = double(ceil_div(int64_t(p.tiles_m) * p.tiles_n * slices, 256));
-                const double rounds = tiles <= 1 ? 0.81 + 0.19 * tiles : tiles + (alone ? 1 : 0.5) * (up - tiles);
+            const int steps = t.cc / 16 * t.taps, all = p.tiles_m * p.tiles_n;
+            const double start = alone ? 7.2 : 2, tile_cost = t.pitch * 1e-4 + t.wn * 0.1;      // of equal ones the smaller patch, the taller tile
+            // every number of slices that leaves none empty, by the chunks of each, as long as what only grows with it stays
+            // below the best: twenty tiles of 128 chunks are planned in 3 us
+            for (int each = p.chunks; each > 0; --each) {
+                const int slices = (p.chunks + each - 1) / each;
+                each = (p.chunks + slices - 1) / slices;
+                const double tiles = double(all) * slices / 256;
                 const double step = (eight ? whole ? 1.66 : 1.78 : (tiles <= 1 ? 1.26 : 1.17) * (whole ? 0.85 : 1)) * 512 / 1700.;
-                const double us = 8.6 + rounds * (each * (t.cc / 16) * t.taps * step + (alone ? 7.2 : 2)) + 5.7 * weights + 0.11 * sums +
-                                  (slices > 1 ? 1.6 + 0.27 * slices * sums : 0) + t.pitch * 1e-4 + t.wn * 0.1;      // of equal ones the smaller patch, the taller tile
+                const double rest = 8.6 + 5.7 * weights + 0.11 * sums + (slices > 1 ? 1.6 + 0.27 * slices * sums : 0) + tile_cost;
+                if (only >= 0) {
+                    if (slices != int(ceil_div(p.chunks, ceil_div(p.chunks, only_slices)))) continue;
+                } else if (best.tile >= 0 && rest + tiles * start + double(all) / 256 * p.chunks * steps * (eight || tiles > 1 ? step : step / 1.26 * 1.17) >= best.us) {
+                    break;
+                }
+                const double rounds = tiles <= 1 ? 0.81 + 0.19 * tiles : tiles + (alone ? 1 : 0.5) * (int((int64_t(all) * slices + 255) / 256) - tiles);
+                const double us = rest + rounds * (each * steps * step + start);
                 if (best.tile < 0 || us < best.us)
                     best = {i * 2 + flat, p.w_bytes + (slices > 1 ? size_t(slices) * size_t(positions) * l.cout * 4 : 0), us, slices};
             }
@@ -628,6 +641,7 @@ int conv_f32_split(const ConvF32Layer &l, const ConvF32Split &choice, const floa
     if (tile < 0 || tile / 2 >= SPLIT_TILE_COUNT || !plan_tile(l, tile / 2, tile % 2 != 0, &p))
         return fail(TSX_E_INVALID, "conv_f32_split: tile %d does not suit this layer", tile);
     const SplitTile &t = SPLIT_TILES[tile / 2];
+    set_divisors(&p, t.bn());
     const dim3 grid(unsigned(p.mfrags), unsigned(p.chunks * (t.cc / 16)));
     const auto pack = t.taps == 9 ? split_weights_kernel<9> : t.taps == 25 ? split_weights_kernel<25> : split_weights_kernel<1>;
     hipLaunchKernelGGL(pack, grid, dim3(unsigned(split_weights_threads(t.taps))), 0, stream, l.w_dev, l.cout, l.c, p.mfrags, static_cast<v4u *>(workspace));

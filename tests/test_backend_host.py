@@ -301,3 +301,44 @@ def test_parameter_checking_follows_the_reference():
         ops.check_params("global_pooling2d", {"format": "NCHW"})
     ops.check_params("add", {})
     ops.check_params("depthwise_conv2d", {k: v for k, v in good.items() if k != "dequantize_scales"})
+
+
+def seconds_per_call(calls):
+    import time
+    best = 1e9
+    for _ in range(7):
+        start = time.perf_counter()
+        for call in calls:
+            call()
+        best = min(best, (time.perf_counter() - start) / len(calls))
+    return best
+
+
+def test_plans_of_many_channels_cost_no_more(monkeypatch):
+    """Planning a layer of 2048 channels weighs as many tiles as one of 64, and only those numbers of slices that can win."""
+    from tennis_amd import capi
+    L = capi.lib()
+    for name in ("TSX_CONV_F32_SMALL", "TSX_GEMM_F32_REGFED", "TSX_CONV_F32_SPLIT", "TSX_CONV_F32_TILE"):
+        monkeypatch.delenv(name, raising=False)
+
+    def plans(channels):      # more layers than a thread keeps: each call plans
+        geoms = [capi.ConvGeom(8, channels, 28 + i, 28, 256, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1) for i in range(1500)]
+        return seconds_per_call([lambda g=g: L.tsx_conv2d_f32_workspace_bytes(ctypes.byref(g), ctypes.c_void_p(4096)) for g in geoms])
+
+    assert any(plans(2048) < 1.6 * plans(64) for _ in range(3))      # (another process may take the CPU meanwhile)
+
+
+def test_the_layers_of_a_network_are_planned_once(monkeypatch):
+    """Sixty layers in turn take the time of one again and again: none displaces another's plan."""
+    import random
+    from tennis_amd import capi
+    L = capi.lib()
+    for name in ("TSX_CONV_F32_SMALL", "TSX_GEMM_F32_REGFED", "TSX_CONV_F32_SPLIT", "TSX_CONV_F32_TILE"):
+        monkeypatch.delenv(name, raising=False)
+    rng = random.Random(2)
+    geoms = [capi.ConvGeom(rng.choice([1, 8, 32]), 64 * rng.randint(1, 32), size, size, 64 * rng.randint(1, 32), k, k, k // 2, k // 2, k // 2, k // 2, 1, 1, 1, 1)
+             for k, size in zip([1, 3] * 30, [7, 14, 28, 56] * 15)]
+    call = lambda g: L.tsx_conv2d_f32_workspace_bytes(ctypes.byref(g), ctypes.c_void_p(4096))
+    in_turn = lambda: seconds_per_call([lambda g=g: call(g) for g in geoms * 20])
+    alone = lambda: max(seconds_per_call([lambda g=g: call(g)] * 200) for g in geoms[::6])
+    assert any(in_turn() < 1.5 * alone() for _ in range(3))
