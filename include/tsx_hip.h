@@ -215,7 +215,9 @@ int tsx_conv2d_f32_nchw(const tsx_conv2d_geom *g, const float *x_dev, const floa
  * on the bf16 matrix cores, every float as the exact sum of three bf16 numbers.  Any floats: denormals count
  * in full, and what meets numbers of 2^89 and more, infinities, NaN or sums above 2^50 is computed by the fp32 MFMA after all.
  * A sum is off by less than the fp32 MFMA's chain of roundings leaves, a single product by at most 2^-24 + 2^-29 of it.
- * The workspace is 16-byte aligned device memory; its contents are written and read by each call. */
+ * The workspace is 16-byte aligned device memory; its contents are written and read by each call.  It holds the weights as
+ * bf16 numbers and, of layers with few output tiles, sums over slices of the input channels: in a smaller one the call takes
+ * fewer slices, or another tile, as far as its bytes go, and without room for the weights it runs as without a workspace. */
 size_t tsx_conv2d_f32_workspace_bytes(const tsx_conv2d_geom *g, const float *w_oihw_dev);
 int tsx_conv2d_f32_nchw_ws(const tsx_conv2d_geom *g, const float *x_dev, const float *w_oihw_dev, float padding_value,
                            const float *bias_dev, int32_t act, float slope, float *out_dev, void *workspace_dev,
@@ -223,11 +225,11 @@ int tsx_conv2d_f32_nchw_ws(const tsx_conv2d_geom *g, const float *x_dev, const f
 /* Which kernel tsx_conv2d_f32_nchw launches for this layer and these weights (their alignment counts), as text:
  * "kernel=small_3x3 | register_fed | staged_64x64 | staged_32x32_ksplit tiles=<output tiles>", and where
  * tsx_conv2d_f32_nchw_ws with its workspace launches another one, that: "workspace_kernel=bf16_split
- * workspace_tile=<output channels>x<positions> workspace_patch=<cells> workspace_window=flat | segments".  No counterpart
- * in the reference; for tests that must know a given kernel ran, and for logs.  The environment variables
+ * workspace_tile=<output channels>x<positions> workspace_patch=<cells> workspace_window=flat | segments
+ * workspace_slices=<slices of the input channels>".  No counterpart in the reference; for tests that must know a given kernel ran, and for logs.  The environment variables
  * TSX_CONV_F32_SMALL and TSX_GEMM_F32_REGFED ("0" = never, "force" = wherever the operands allow) and TSX_CONV_F32_SPLIT
  * ("0" = the workspace is not used, a number = that tile and patch form of the kernel on the bf16 matrix cores wherever it
- * suits the layer) are read at every call. */
+ * suits the layer, "number/slices" = the same in so many slices where there are the channels) are read at every call. */
 int tsx_conv2d_f32_plan_info(const tsx_conv2d_geom *g, const float *w_oihw_dev, char *text, size_t text_bytes);
 
 /* cpu::InnerProd::inner_prod (src/kernels/cpu/inner_prod.cpp:54-69, interface

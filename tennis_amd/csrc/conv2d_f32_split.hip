@@ -578,9 +578,10 @@ void set_divisors(SplitParams *p, int bn) {
 
 }  // namespace
 
-ConvF32Split conv_f32_split_choose(const ConvF32Layer &l) {
+ConvF32Split conv_f32_split_choose(const ConvF32Layer &l, size_t workspace_bytes) {
     ConvF32Split best{-1, 0, 0., 1};
-    // "0": never; a number: that tile wherever it suits, in one slice or, "number/slices", in so many where there are the chunks (tests)
+    // "0": never; a number: that tile wherever it suits, in one slice or, "number/slices", in so many where there are the chunks
+    // and the workspace (tests)
     const char *e = std::getenv("TSX_CONV_F32_SPLIT");
     if (e && e[0] == '0' && !e[1]) return best;
     const int only = e && e[0] ? std::atoi(e) - 1 : -1;
@@ -594,6 +595,7 @@ ConvF32Split conv_f32_split_choose(const ConvF32Layer &l) {
         for (int flat = 1; flat >= 0; --flat) {
             SplitParams p{};
             if ((only >= 0 && i * 2 + flat != only) || !plan_tile(l, i, flat != 0, &p)) continue;
+            if (p.w_bytes > workspace_bytes) continue;
             const SplitTile &t = SPLIT_TILES[i];
             // Time in us: the launches; by the tiles of a CU their steps (16 MFMAs are 512 cycles, at 1.7 GHz beside everything
             // else; whole eights of channels take the form without a look at each, a SIMD's two wavefronts of one workgroup
@@ -613,18 +615,18 @@ ConvF32Split conv_f32_split_choose(const ConvF32Layer &l) {
                 const double tiles = double(all) * slices / 256;
                 const double step = (eight ? whole ? 1.66 : 1.78 : (tiles <= 1 ? 1.26 : 1.17) * (whole ? 0.85 : 1)) * 512 / 1700.;
                 const double rest = 8.6 + 5.7 * weights + 0.11 * sums + (slices > 1 ? 1.6 + 0.27 * slices * sums : 0) + tile_cost;
+                const size_t bytes = p.w_bytes + (slices > 1 ? size_t(slices) * size_t(positions) * l.cout * 4 : 0);
+                if (bytes > workspace_bytes) break;
                 if (only >= 0) {
-                    if (slices != int(ceil_div(p.chunks, ceil_div(p.chunks, only_slices)))) continue;
-                } else if (best.tile >= 0 && rest + tiles * start + double(all) / 256 * p.chunks * steps * (eight || tiles > 1 ? step : step / 1.26 * 1.17) >= best.us) {
-                    break;
+                    if (slices <= int(ceil_div(p.chunks, ceil_div(p.chunks, only_slices)))) best = {i * 2 + flat, bytes, 0., slices};
+                    continue;
                 }
+                if (best.tile >= 0 && rest + tiles * start + double(all) / 256 * p.chunks * steps * (eight || tiles > 1 ? step : step / 1.26 * 1.17) >= best.us) break;
                 const double rounds = tiles <= 1 ? 0.81 + 0.19 * tiles : tiles + (alone ? 1 : 0.5) * (int((int64_t(all) * slices + 255) / 256) - tiles);
                 const double us = rest + rounds * (each * steps * step + start);
-                if (best.tile < 0 || us < best.us)
-                    best = {i * 2 + flat, p.w_bytes + (slices > 1 ? size_t(slices) * size_t(positions) * l.cout * 4 : 0), us, slices};
+                if (best.tile < 0 || us < best.us) best = {i * 2 + flat, bytes, us, slices};
             }
         }
-    if (only >= 0) best.us = 0;
     return best;
 }
 

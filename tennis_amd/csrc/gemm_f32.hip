@@ -722,9 +722,9 @@ int window_tile(const ConvF32Layer &layer, const GemmArgs &g, double *cycles = n
 // where it has one tap; the register-fed kernel twice, on 5x5 windows 1.1 times; and all of them their launch and output.
 // Fitted, rather too short than too long, to 250 layers of 0.01 to 13 GFLOP, of which one takes longer this way by more than
 // 2 % (22.5 -> 24.9 us); kept where they were: 1x256x28x28, 256 3x3 filters (25 us), and nearly all layers below 15 us.
-ConvF32Split split_choice(const ConvF32Layer &layer, int window, double cycles) {
+ConvF32Split split_choice(const ConvF32Layer &layer, int window, double cycles, size_t workspace_bytes) {
     const ConvF32Split none{-1, 0, 0., 1};
-    const ConvF32Split split = conv_f32_split_choose(layer);
+    const ConvF32Split split = conv_f32_split_choose(layer, workspace_bytes);
     if (split.tile < 0 || split.us == 0) return split;
     if (cycles == 0) return none;
     const int taps = layer.kh * layer.kw;
@@ -742,8 +742,10 @@ struct ConvF32Plan {
     int window;
 };
 
-ConvF32Plan conv_f32_plan(const ConvF32Layer &layer, const GemmArgs &g) {
+// The split kernel's part is for a workspace of up to workspace_bytes: the one it asks for, or what a caller has.
+ConvF32Plan conv_f32_plan(const ConvF32Layer &layer, const GemmArgs &g, size_t workspace_bytes = SIZE_MAX) {
     struct Key {
+        size_t workspace_bytes;
         int geometry[15];
         int x_misaligned, w_misaligned;        // to 16 bytes: all the planners ask of the addresses
         PlanSwitch regfed, tile, split;
@@ -751,6 +753,7 @@ ConvF32Plan conv_f32_plan(const ConvF32Layer &layer, const GemmArgs &g) {
     std::memset(&key, 0, sizeof(key));
     static_assert(offsetof(ConvF32Layer, x_dev) >= sizeof(key.geometry), "fifteen ints in front of the addresses");
     std::memcpy(key.geometry, &layer, sizeof(key.geometry));
+    key.workspace_bytes = workspace_bytes;
     key.x_misaligned = int(reinterpret_cast<uintptr_t>(layer.x_dev) % 16);
     key.w_misaligned = int(reinterpret_cast<uintptr_t>(layer.w_dev) % 16);
     const auto make = [&] {
@@ -761,7 +764,7 @@ ConvF32Plan conv_f32_plan(const ConvF32Layer &layer, const GemmArgs &g) {
         const char *e = std::getenv("TSX_GEMM_F32_REGFED");
         const bool small = plan.window < 0 && choose_gemm(g, 1) == GEMM_REGISTER_FED && !(e && e[0] == 'f');
         if (small) conv_f32_window_tile(layer, &cycles);
-        if (small || plan.window >= 0) plan.split = split_choice(layer, plan.window, cycles);
+        if (small || plan.window >= 0) plan.split = split_choice(layer, plan.window, cycles, workspace_bytes);
         return plan;
     };
     if (!key.regfed.read("TSX_GEMM_F32_REGFED") || !key.tile.read("TSX_CONV_F32_TILE") || !key.split.read("TSX_CONV_F32_SPLIT")) return make();
@@ -843,10 +846,11 @@ int tsx_conv2d_f32_nchw_ws(const tsx_conv2d_geom *geo, const float *x_dev, const
         return geo->c <= 32 ? tsx::launch_conv3x3_small<2>(g, ld, tsx::as_stream(stream))
                             : tsx::launch_conv3x3_small<4>(g, ld, tsx::as_stream(stream));
     const tsx::ConvF32Layer layer = tsx::window_layer(geo, g, ld);
-    const tsx::ConvF32Plan plan = tsx::conv_f32_plan(layer, g);
+    tsx::ConvF32Plan plan = tsx::conv_f32_plan(layer, g);
     if (workspace_dev) {
         TSX_REQUIRE(reinterpret_cast<uintptr_t>(workspace_dev) % 16 == 0, "conv2d_f32: workspace not aligned to 16 bytes");
-        if (plan.split.tile >= 0 && plan.split.workspace_bytes <= workspace_bytes)
+        if (plan.split.tile >= 0 && plan.split.workspace_bytes > workspace_bytes) plan = tsx::conv_f32_plan(layer, g, workspace_bytes);
+        if (plan.split.tile >= 0)
             return tsx::conv_f32_split(layer, plan.split, bias_dev, act, slope, padding_value, out_dev, workspace_dev, tsx::as_stream(stream));
     }
     if (plan.window >= 0)

@@ -95,7 +95,9 @@ def test_conv_f32_slices_bias_and_activation(port, monkeypatch, case, act):
 @pytest.mark.parametrize("case", [(2, 233, 19, 6, 98, 3), (1, 256, 14, 14, 64, 3), (2, 64, 12, 12, 32, 5), (2, 512, 7, 7, 128, 1)])
 @pytest.mark.parametrize("positive", [False, True])
 def test_conv_f32_slices_are_no_less_exact(monkeypatch, case, positive):
-    """Than the fp32 MFMA kernel; and a captured call gives the same bits on every replay."""
+    """Than the fp32 MFMA kernel, nor than one slice but for the roundings of the slices' sums: each of them is off by at most 2^-24 of
+    a partial sum, which is no larger than the result here, independently of the others.  And a captured call gives the same bits on every
+    replay."""
     import torch
     from tennis_amd import capi
     n, c, h, w, cout, k = case
@@ -110,10 +112,13 @@ def test_conv_f32_slices_are_no_less_exact(monkeypatch, case, positive):
     monkeypatch.setenv("TSX_CONV_F32_SPLIT", "0")
     most = error(run())
     for number in NUMBERS:
+        monkeypatch.setenv("TSX_CONV_F32_SPLIT", f"{number}")
+        one = error(run())
         for slices in (2, 4, 64):
             monkeypatch.setenv("TSX_CONV_F32_SPLIT", f"{number}/{slices}")
-            if slices_of(capi, x, wt, pads, (1, 1), (1, 1)) > 1:
-                assert error(run()) <= most, (number, slices)
+            used = slices_of(capi, x, wt, pads, (1, 1), (1, 1))
+            if used > 1:
+                assert error(run()) <= min(most, one + used ** 0.5 * 2.0 ** -24), (number, slices)
     monkeypatch.delenv("TSX_CONV_F32_SPLIT")
     eager = run()
     stream = torch.cuda.Stream()
@@ -145,3 +150,49 @@ def test_conv_f32_slices_choice(monkeypatch):
         size = capi.lib().tsx_conv2d_f32_workspace_bytes(ctypes.byref(geom), ctypes.c_void_p(16))
         sums = slices * x[0] * w[0] * ho * wo * 4 if sliced else 0
         assert size - sums >= np.prod(w) * 6 and (size - sums) % 3072 == 0
+
+
+@pytest.mark.parametrize("case", [(2, 233, 19, 6, 98, 3), (1, 100, 14, 14, 64, 5), (2, 512, 7, 7, 128, 1)])
+def test_conv_f32_in_the_workspace_that_there_is(monkeypatch, case):
+    """A workspace below what the layer asks for is used as far as it goes: fewer slices down to one in the split weights' bytes, and the
+    kernel without a workspace below these."""
+    import torch
+    from tennis_amd import capi
+    n, c, h, w, cout, k = case
+    g = torch.Generator().manual_seed(6)
+    x, wt = torch.randn(n, c, h, w, generator=g).cuda(), torch.randn(cout, c, k, k, generator=g).cuda()
+    pads, lib = (k // 2,) * 4, capi.lib()
+    geom = capi.make_geom(tuple(x.shape), tuple(wt.shape), pads)
+    pointer = lambda t: ctypes.c_void_p(t.data_ptr())
+    asked = lambda: lib.tsx_conv2d_f32_workspace_bytes(ctypes.byref(geom), pointer(wt))
+
+    def run(size):
+        out, space = torch.full((n, cout, h, w), np.nan, device="cuda"), torch.full((size + 64,), 77, dtype=torch.uint8, device="cuda")
+        capi.check(lib.tsx_conv2d_f32_nchw_ws(ctypes.byref(geom), pointer(x), pointer(wt), 0.0, None, 0, 0.0, pointer(out), pointer(space), size,
+                                              ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        assert bool((space[size:] == 77).all())
+        return out
+
+    sums = n * cout * h * w * 4
+    for number in NUMBERS:
+        monkeypatch.setenv("TSX_CONV_F32_SPLIT", f"{number}")
+        if not asked():
+            continue
+        weights, results = asked(), {}
+        for slices in (1, 2, 3):
+            monkeypatch.setenv("TSX_CONV_F32_SPLIT", f"{number}/{slices}")
+            assert asked() == weights + (slices * sums if slices > 1 else 0)
+            results[slices] = run(asked())
+        plain = run(weights - 16)
+        for size, slices in ((weights + 3 * sums - 16, 2), (weights + 2 * sums, 2), (weights + 2 * sums - 16, 1), (weights, 1)):
+            assert torch.equal(run(size), results[slices]), (number, size)
+        assert not torch.equal(results[1], results[2]) and not torch.equal(plain, results[1])
+    # by itself: where the layer's own choice does not fit it is another choice of the same kernel, not the kernel without a workspace
+    monkeypatch.delenv("TSX_CONV_F32_SPLIT")
+    if k == 1:      # (stays on that one)
+        return
+    assert asked() > sums
+    best = run(asked())
+    less = run(asked() - 16)
+    assert not torch.equal(less, plain) and float((less - best).norm() / best.norm()) < 2e-6
