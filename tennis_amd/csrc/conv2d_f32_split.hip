@@ -597,33 +597,35 @@ ConvF32Split conv_f32_split_choose(const ConvF32Layer &l, size_t workspace_bytes
             if ((only >= 0 && i * 2 + flat != only) || !plan_tile(l, i, flat != 0, &p)) continue;
             if (p.w_bytes > workspace_bytes) continue;
             const SplitTile &t = SPLIT_TILES[i];
-            // Time in us: the launches; by the tiles of a CU their steps (16 MFMAs are 512 cycles, at 1.7 GHz beside everything
-            // else; whole eights of channels take the form without a look at each, a SIMD's two wavefronts of one workgroup
-            // share what is beside the MFMAs), their start and end, of which little is seen where a CU holds two workgroups, and
-            // its last, half empty round; the weights and the output.  Slices cost their sums' way through memory and one more
-            // launch.  Fitted to all combinations of tile and slices on 400 layers of 0.01 to 13 GFLOP, which it meets by 8 %
-            // (rms); the combinations it picks take 1 % longer than the fastest.
+            // Time in us: the launches; by the tiles of a CU and their chunks the steps of MFMAs (of eight wavefronts two to a SIMD)
+            // and the conversion of the patch, twice as much where channels are no whole eights and each is looked at; the tiles'
+            // start and end, of which little is seen where a CU holds two workgroups; the last, partly empty round; the weights
+            // and the output.  Slices cost their sums' way through memory and one more launch.  Fitted to 23 000 combinations of tile
+            // and slices on 800 layers of 0.01 to 15 GFLOP, which it meets by 5 % (rms); the combinations it picks take 0.5 %
+            // longer than the fastest on average, one in a hundred more than 7 %.
             const bool eight = t.wm * t.wn == 8, alone = t.pitch > 384, whole = l.c % 8 == 0;
             const double sums = double(positions) * l.cout * 4e-6, weights = double(l.cout) * l.c * t.taps * 1e-6;
             const int steps = t.cc / 16 * t.taps, all = p.tiles_m * p.tiles_n;
-            const double start = alone ? 7.2 : 2, tile_cost = t.pitch * 1e-4 + t.wn * 0.1;      // of equal ones the smaller patch, the taller tile
+            const double start = alone ? eight ? 3.2 : 4.6 : 1.35, patch = (t.taps == 1 ? t.bn() : t.pitch) * (t.cc / 16) * (whole ? 0.0010 : 0.00215);
+            const double tile_cost = t.pitch * 1e-4 + t.wn * 0.1;      // of equal ones the smaller patch, the taller tile
             // every number of slices that leaves none empty, by the chunks of each, as long as what only grows with it stays
             // below the best: twenty tiles of 128 chunks are planned in 3 us
             for (int each = p.chunks; each > 0; --each) {
                 const int slices = (p.chunks + each - 1) / each;
                 each = (p.chunks + slices - 1) / slices;
                 const double tiles = double(all) * slices / 256;
-                const double step = (eight ? whole ? 1.66 : 1.78 : (tiles <= 1 ? 1.26 : 1.17) * (whole ? 0.85 : 1)) * 512 / 1700.;
-                const double rest = 8.6 + 5.7 * weights + 0.11 * sums + (slices > 1 ? 1.6 + 0.27 * slices * sums : 0) + tile_cost;
+                const double step = (eight ? 0.488 : tiles <= 1 ? 0.29 : 0.27) * (t.taps == 1 ? 0.9 : 1);
+                const double rest = 9.2 + 2.6 * weights + 0.18 * sums + (slices > 1 ? 1.8 + 0.4 * slices * sums : 0) + tile_cost;
                 const size_t bytes = p.w_bytes + (slices > 1 ? size_t(slices) * size_t(positions) * l.cout * 4 : 0);
                 if (bytes > workspace_bytes) break;
                 if (only >= 0) {
                     if (slices <= int(ceil_div(p.chunks, ceil_div(p.chunks, only_slices)))) best = {i * 2 + flat, bytes, 0., slices};
                     continue;
                 }
-                if (best.tile >= 0 && rest + tiles * start + double(all) / 256 * p.chunks * steps * (eight || tiles > 1 ? step : step / 1.26 * 1.17) >= best.us) break;
-                const double rounds = tiles <= 1 ? 0.81 + 0.19 * tiles : tiles + (alone ? 1 : 0.5) * (int((int64_t(all) * slices + 255) / 256) - tiles);
-                const double us = rest + rounds * (each * steps * step + start);
+                if (best.tile >= 0 && rest + tiles * start + double(all) / 256 * p.chunks * (steps * (eight || tiles > 1 ? step : step / 0.29 * 0.27) + patch) >= best.us) break;
+                const double rounds = tiles <= 1 ? 0.8 + 0.2 * tiles : tiles + (alone ? 1 : 0.69) * (int((int64_t(all) * slices + 255) / 256) - tiles);
+                const double lone = eight || alone ? 1 + 0.12 * std::clamp((tiles - 1) / 3, 0., 1.) : 1;      // a CU's only workgroup, one after the other
+                const double us = rest + rounds * lone * (each * (steps * step + patch) + start);
                 if (best.tile < 0 || us < best.us) best = {i * 2 + flat, bytes, us, slices};
             }
         }

@@ -506,7 +506,7 @@ int conv_f32_window_tile(const ConvF32Layer &l, double *cycles) {
         return -1;
     if (positions >= (int64_t(1) << 30) || l.pad_top < 0 || l.pad_left < 0) return -1;
     int best = -1;
-    double best_cost = 0;
+    double best_cost = 0, best_slow = 1;
     for (int i = 0; i < WIN_TILE_COUNT; ++i)
         for (int flat = 1; flat >= (l.kh * l.kw == 1 ? 1 : 0); --flat) {
             WinParams p{};
@@ -527,10 +527,11 @@ int conv_f32_window_tile(const ConvF32Layer &l, double *cycles) {
             if (best < 0 || cost < best_cost) {
                 best = i * 2 + flat;
                 best_cost = cost;
+                best_slow = kind == 0 && p.cc == 2 && l.kh * l.kw <= 9 ? 1.3 : 1;      // chunks of a few steps
             }
         }
     // the best tile's fragments on four SIMDs: K / 2 MFMAs of 64 cycles each
-    if (cycles) *cycles = best_cost * l.c * l.kh * l.kw * 8;
+    if (cycles) *cycles = best_cost * best_slow * l.c * l.kh * l.kw * 8;
     const char *e = std::getenv("TSX_CONV_F32_TILE");
     if (e && e[0]) {
         best = std::atoi(e);

@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdlib>
 
 namespace tsx {
@@ -716,24 +717,36 @@ int window_tile(const ConvF32Layer &layer, const GemmArgs &g, double *cycles = n
     return conv_f32_window_tile(layer, cycles);
 }
 
-// The tile on the bf16 matrix cores for the layer, where that is expected to be at least a twentieth faster than the kernel
-// without a workspace (a quarter, than the register-fed one, whose line rests on ten layers), of whose time `cycles` is the window kernel's model (0: a forced tile, which stays).  At 2.2 GHz the
-// window kernel takes those cycles with its vector forms, 1.35 times as long in its K-split tile; 1.75 times without, or 1.05
-// where it has one tap; the register-fed kernel twice, on 5x5 windows 1.1 times; and all of them their launch and output.
-// Fitted, rather too short than too long, to 250 layers of 0.01 to 13 GFLOP, of which one takes longer this way by more than
-// 2 % (22.5 -> 24.9 us); kept where they were: 1x256x28x28, 256 3x3 filters (25 us), and nearly all layers below 15 us.
+// The tile on the bf16 matrix cores for the layer, where that is expected to be faster than the kernel without a workspace (by a quarter,
+// than the register-fed one on 3x3 layers), of whose time `cycles` is the window kernel's model (0: a forced tile, which stays).  That
+// kernel's us: its launch, start and end; the cycles at 2.2 GHz, apart for the part of its tiles' last round that is work and the
+// part that idles; MB of output; and of one tap MB of input.  By kernel, taps and, of 3x3 layers, the vector form, fitted to 700 layers of
+// 0.01 to 15 GFLOP.  1300 layers, 500 of them not of the fit, take 2.4 % less by it than by a fit to 250 layers; against the choice of
+// before there were slices nine of them take 5 % and more longer (3x624x179x127 to 32, 3x3 of stride 2, 90 -> 107 us) where twenty-nine
+// did (10x78x20x20 to 971, 3x3 of stride 2, 32 -> 59, now 31).
 ConvF32Split split_choice(const ConvF32Layer &layer, int window, double cycles, size_t workspace_bytes) {
     const ConvF32Split none{-1, 0, 0., 1};
     const ConvF32Split split = conv_f32_split_choose(layer, workspace_bytes);
     if (split.tile < 0 || split.us == 0) return split;
     if (cycles == 0) return none;
-    const int taps = layer.kh * layer.kw;
-    const bool vector = layer.c * taps % 4 == 0 && (layer.kh == 1 || layer.kh == 3) && reinterpret_cast<uintptr_t>(layer.w_dev) % 16 == 0;
-    int rows = 0, positions = 0;
+    const int taps = layer.kh * layer.kw;      // 1, 9 or 25
+    const bool vector = layer.c * taps % 4 == 0 && reinterpret_cast<uintptr_t>(layer.w_dev) % 16 == 0;
+    int rows = 32, positions = 32;
     if (window >= 0) conv_f32_window_tile_size(window, &rows, &positions);
-    const double factor = window < 0 ? (taps == 25 ? 1.1 : 2.) : vector ? (rows * positions == 1024 ? 1.35 : 1.) : taps == 1 ? 1.05 : 1.75;
-    const double other = 6 + factor * cycles / 2200 + 0.44 * layer.n * layer.ho * layer.wo * layer.cout * 4e-6;
-    return split.us * (window < 0 ? 1.25 : 1.05) < other ? split : none;
+    const bool k_split = rows * positions == 1024;
+    struct Coefficients {
+        double launch, work, idle, output;
+    };
+    const Coefficients c = window < 0 ? (taps == 25 ? Coefficients{6, 0.9, 1.1, 6} : taps == 9 ? Coefficients{6, 2, 2, 0.44} : Coefficients{5.5, 1.2, 2.9, 6.6})
+                         : taps == 1  ? (k_split ? Coefficients{5.4, 0.7, 1.5, 1.5} : Coefficients{7.35, 1.2, 1.2, 0.3})
+                         : taps == 25 ? (k_split ? Coefficients{8, 1.75, 1.75, 0.5} : Coefficients{10, 1.3, 2.1, 0.4})
+                         : !vector    ? Coefficients{9.7, 1.67, 2.9, 0.4}
+                                      : (k_split ? Coefficients{6.3, 1.03, 1.32, 0.8} : Coefficients{8.3, 1, 1, 0.33});
+    const int64_t outputs = int64_t(layer.n) * layer.ho * layer.wo;
+    const double tiles = double(ceil_div(layer.cout, rows) * ceil_div(outputs, positions)) / 256, part = tiles / std::ceil(tiles);
+    const double other = c.launch + cycles / 2200 * (c.work * part + c.idle * (1 - part)) + c.output * double(outputs) * layer.cout * 4e-6 +
+                         (taps == 1 && window >= 0 ? 0.1 / layer.stride_h * layer.n * layer.c * double(layer.h) * layer.w * 4e-6 : 0);
+    return split.us * (window < 0 && taps == 9 ? 1.25 : 1.02) < other ? split : none;
 }
 
 // What a layer beyond the small-layer kernel runs on: with its workspace, and without (-1: a kernel of this file).

@@ -104,6 +104,22 @@ def test_fp32_plan_info_names_the_kernel_of_a_call_with_workspace(monkeypatch):
     assert "workspace_kernel" not in plan(capi.ConvGeom(1, 128, 28, 28, 128, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1))
 
 
+@pytest.mark.parametrize("layer, takes", [
+    # us without a workspace / with one: 59 / 31, 27 / 18, 35 / 32, 88 / 36 ...
+    ((10, 78, 20, 20, 971, 3, 2, 1), True), ((1, 85, 42, 42, 84, 3, 2, 1), True), ((2, 179, 81, 81, 292, 1, 1, 0), True), ((4, 90, 121, 138, 32, 3, 2, 1), True),
+    # ... and 62 / 88, 40 / 46, 44 / 49, 20 / 25, 89 / 98
+    ((3, 124, 261, 261, 32, 3, 2, 1), False), ((25, 32, 11, 179, 432, 1, 1, 0), False), ((2, 31, 103, 201, 541, 1, 1, 0), False),
+    ((1, 32, 68, 173, 747, 1, 1, 0), False), ((8, 32, 216, 216, 31, 5, 2, 2), False),
+])
+def test_fp32_layers_use_a_workspace_where_that_is_faster(monkeypatch, layer, takes):
+    from tennis_amd import capi
+    for name in ("TSX_CONV_F32_SMALL", "TSX_GEMM_F32_REGFED", "TSX_CONV_F32_SPLIT", "TSX_CONV_F32_TILE"):
+        monkeypatch.delenv(name, raising=False)
+    n, c, h, w, cout, k, stride, pad = layer
+    geom = capi.ConvGeom(n, c, h, w, cout, k, k, pad, pad, pad, pad, stride, stride, 1, 1)
+    assert (capi.lib().tsx_conv2d_f32_workspace_bytes(ctypes.byref(geom), ctypes.c_void_p(4096)) > 0) == takes
+
+
 def test_every_tile_of_the_bf16_split_kernel_is_reached(monkeypatch):
     """Each tile that TSX_CONV_F32_SPLIT can name takes some layer, is no twin of another one, and is what the planner
     chooses for some layer by itself."""
