@@ -331,34 +331,29 @@ __device__ __forceinline__ void wino_tail_store(const float *__restrict__ u, con
 // three channels left as a chain behind it.  v_mfma_f32_16x16x1_f32 is four blocks of 16 x 16 with one multiply-add per step
 // each: block q takes chain q, and a lane then holds all four chains of its outputs (accumulator 4 q + i of lane l: chain q,
 // row 4 (l / 16) + i, column l % 16).  A fragment is 32 rows x 16 columns, an image leaves at
-// most 7 columns here; a wavefront takes one, or two beside one another.
-template <int NC, int RING>
+// most 7 columns here; a wavefront takes one.  (Two beside one another, which share U's operands, leave half the wavefronts to hide
+// one another's loads: 78 layers took 8 % longer so, 8 images 11x11, 465 to 21 channels, F(6,3), 24.4 us for 19.6.)
 __device__ __forceinline__ void wino_gemm_tail(const float *__restrict__ u, const float *__restrict__ v, float *__restrict__ m, const WinoGeom &g,
-                                               int f, int rf, int cf, int tails, int lane) {
+                                               int f, int rf, int cf, int lane) {
+    constexpr int RING = 4;
     const int T = g.kgroups, q = lane / 16, i = lane % 16;
     // A lane loads the operand element (four channels of one parity) of its row, of the row sixteen further (+ 64 floats) and of
-    // its columns: the lower half-wave those of group 2 p, the upper of group 2 p + 1.  Chain q's channels 8t + q and 8t + 4 + q
+    // its column: the lower half-wave those of group 2 p, the upper of group 2 p + 1.  Chain q's channels 8t + q and 8t + 4 + q
     // are floats q / 2 and q / 2 + 2 of both groups: a half-wave swap each.
     // (The group is part of the lane's offset here: loads beyond the last one are then outside of the fragment's buffer.)
     const auto ua = fragment_buffer(u, int64_t(f) * g.rfrags + rf, T);
-    const int row_at = 16 * (i + 32 * (q % 2)) + 1024 * (q / 2);
-    int column_at[NC];
+    const auto vb = fragment_buffer(v, int64_t(f) * g.nfrags + g.mfrags + cf / 2, T);
+    const int row_at = 16 * (i + 32 * (q % 2)) + 1024 * (q / 2), column_at = row_at + 256 * (cf % 2);
+    v16f s[2];
 #pragma unroll
-    for (int n = 0; n < NC; ++n) column_at[n] = row_at + 256 * ((cf + n) % 2);
-    v16f s[NC][2];
-#pragma unroll
-    for (int n = 0; n < NC; ++n)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[n][0][r] = s[n][1][r] = 0.f;
+    for (int r = 0; r < 16; ++r) s[0][r] = s[1][r] = 0.f;
     const int steps = g.c / 4;                               // of four channels, one to a chain
-    v4f a[RING][2], b[RING][NC];                   // [slot][row half], [slot][columns]
+    v4f a[RING][2], b[RING];                       // [slot][row half], [slot]
     auto load = [&](auto slot, int pair) __attribute__((always_inline)) {
         constexpr int sl = decltype(slot)::value;
         a[sl][0] = fragment_element(ua, row_at + pair * 2048, 0);
         a[sl][1] = fragment_element(ua, row_at + 256 + pair * 2048, 0);
-#pragma unroll
-        for (int n = 0; n < NC; ++n)
-            b[sl][n] = fragment_element(fragment_buffer(v, int64_t(f) * g.nfrags + g.mfrags + min(cf + n, tails - 1) / 2, T), column_at[n] + pair * 2048, 0);
+        b[sl] = fragment_element(vb, column_at + pair * 2048, 0);
     };
     auto split = [](const v4f &e, float (&of_step)[4]) __attribute__((always_inline)) {
         const auto low = __builtin_amdgcn_permlane32_swap(__float_as_int(e[0]), __float_as_int(e[1]), false, false);
@@ -370,18 +365,15 @@ __device__ __forceinline__ void wino_gemm_tail(const float *__restrict__ u, cons
     };
     auto multiply = [&](auto slot, int live) __attribute__((always_inline)) {      // the first `live` steps of the pair
         constexpr int sl = decltype(slot)::value;
-        float ea[2][4], eb[NC][4];
+        float ea[2][4], eb[4];
         split(a[sl][0], ea[0]);
         split(a[sl][1], ea[1]);
-#pragma unroll
-        for (int n = 0; n < NC; ++n) split(b[sl][n], eb[n]);
+        split(b[sl], eb);
         static_for<0, 4>([&](auto ec) {
             constexpr int e = decltype(ec)::value;
             if (e < live) {
 #pragma unroll
-                for (int n = 0; n < NC; ++n)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) s[n][h] = __builtin_amdgcn_mfma_f32_16x16x1f32(ea[h][e], eb[n][e], s[n][h], 0, 0, 0);
+                for (int h = 0; h < 2; ++h) s[h] = __builtin_amdgcn_mfma_f32_16x16x1f32(ea[h][e], eb[e], s[h], 0, 0, 0);
             }
         });
     };
@@ -404,9 +396,7 @@ __device__ __forceinline__ void wino_gemm_tail(const float *__restrict__ u, cons
         if constexpr (sl == RING - 1) load(sc, pair + sl);
         multiply(sc, steps - 4 * (pair + sl));
     });
-#pragma unroll
-    for (int n = 0; n < NC; ++n)
-        if (cf + n < tails) wino_tail_store(u, v, m, g, f, rf, cf + n, lane, s[n]);
+    wino_tail_store(u, v, m, g, f, rf, cf, lane, s);
 }
 
 // TAIL: and one fragment of 16 tail columns (see wino_gemm_tail) with them, whose rows are these.
@@ -496,14 +486,14 @@ __device__ __forceinline__ void wino_gemm_chain(const float *__restrict__ u, con
 
 // A workgroup's wavefronts are wr row fragments x wc column blocks of FN fragments.  Items are, per XCD and counted from `first`:
 // row blocks of col_items of its frequencies, one frequency after the other.  The tail's fragments of 16 go with the first column
-// blocks, one each (`attached`), or follow as items of their own, two fragments each.
+// blocks, one each (`attached`), or follow as items of their own.
 // Registers for two (FN = 4) or four wavefronts per SIMD (the compiler's own choice, 267, left one).
 template <int FN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FN == 1 ? 4 : 2))) void wino_gemm_kernel(
     const float *__restrict__ u, const float *__restrict__ v, float *__restrict__ m, WinoGeom g, int wr, int wc, int row_blocks, int col_blocks,
     int tails, int attached, int rounds, int64_t first) {
     const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const int tail_blocks = attached ? 0 : (tails + 1) / 2, col_items = (col_blocks + wc - 1) / wc, tail_items = (tail_blocks + wc - 1) / wc;
+    const int tail_blocks = attached ? 0 : tails, col_items = (col_blocks + wc - 1) / wc, tail_items = (tail_blocks + wc - 1) / wc;
     const int64_t item = first + (blockIdx.x >> 3), chains = int64_t(rounds) * col_items * row_blocks;
     const bool tail = item >= chains;
     const int64_t at = tail ? item - chains : item;
@@ -512,8 +502,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FN == 1 ? 4
     const int ci = rest / row_blocks, cb = ci * wc + wave / wr, rf = (rest - ci * row_blocks) * wr + wave % wr;
     if (rf >= g.rfrags || wave >= wr * wc || cb >= (tail ? tail_blocks : col_blocks)) return;
     if (tail) {
-        if (tails == 1) wino_gemm_tail<1, 4>(u, v, m, g, f, rf, 0, tails, lane);
-        else wino_gemm_tail<2, 3>(u, v, m, g, f, rf, cb * 2, tails, lane);
+        wino_gemm_tail(u, v, m, g, f, rf, cb, lane);
     } else if (attached && cb < tails) {
         wino_gemm_chain<FN, true>(u, v, m, g, f, rf, cb * FN, cb, lane);
     } else {
@@ -707,7 +696,7 @@ int conv2d(const tsx_conv2d_geom *q, const float *x, const float *u, float paddi
     // 28x28, 256 to 256 channels, by the wavefronts' clocks: 15 us without the tail, 20 with it, 30 with it as workgroups of its own).
     // A grid that leaves CUs idle computes them there (1 image 14x14, 512 to 512, F(2,3): 25.9 us attached, 21.7).
     const int attached = tails <= col_blocks && int64_t(FREQS) * row_blocks * ceil_div(col_blocks, wc) >= 256;
-    const int64_t items = int64_t(rounds) * row_blocks * (ceil_div(col_blocks, wc) + (attached ? 0 : ceil_div((tails + 1) / 2, wc)));
+    const int64_t items = int64_t(rounds) * row_blocks * (ceil_div(col_blocks, wc) + (attached ? 0 : ceil_div(tails, wc)));
     const auto gemm = four ? wino_gemm_kernel<4> : wino_gemm_kernel<1>;
     // one launch, except where its work items would be 2^32 or more
     const int64_t most = ((int64_t(1) << 24) - 1) / 8;

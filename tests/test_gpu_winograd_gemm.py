@@ -1,7 +1,7 @@
 """The Winograd GEMMs on the matrix cores at the sizes where their tiling can go wrong, bit for bit against the oracle:
 channel counts that leave a part of a group of 8 (and a remainder behind the four interleaved chains), output channels
-beside a fragment of 32 and a block of 8, tile counts with and without tail columns, one and two column fragments per
-wavefront."""
+beside a fragment of 32 and a block of 8, tile counts with and without tail columns, one and four column fragments per
+wavefront, and a workgroup's wavefronts along rows, along columns and along both."""
 import numpy as np
 import pytest
 
@@ -20,6 +20,10 @@ CASES = [
     (4, 64, 62, 40, 128),      # tail fragments computed with the column blocks
     (6, 20, 6, 42, 33),        # seven tiles of F(6,3) an image, all in the tail: three fragments of 16, an odd number of channel groups
     (8, 131, 18, 110, 128),    # F(6,3): four column fragments per wavefront, the last block of two, and a tail fragment with them
+    # wavefronts of a workgroup along the columns, the last of whose groups has one block: two rows of them by two, or four in a row
+    (2, 20, 78, 66, 40), (2, 20, 78, 66, 31),      # F(6,3): nine column fragments, a tail fragment with them
+    (3, 20, 41, 37, 40), (3, 20, 41, 37, 31),      # F(2,3): 37, two tail fragments with them, or by themselves
+    (3, 21, 65, 67, 29),                           # F(2,3): 105 in fours, one with them; remainder channel
 ]
 
 
