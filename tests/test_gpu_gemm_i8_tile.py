@@ -46,11 +46,16 @@ def test_gemm_i8_tile_kernel(port, monkeypatch, m, k, n, tile):
 
 @pytest.mark.parametrize("m,k,n", [(1, 7, 5), (1, 17, 64), (2, 8, 33), (32, 100, 33), (31, 1500, 96), (33, 1, 40), (129, 3, 33), (192, 5, 144), (130, 77, 64),
                                    (197, 1500, 77), (65, 2049, 66), (64, 2500, 72), (130, 1985, 48), (70, 2048, 64)])
-def test_gemm_i8_rows_of_any_length(port, m, k, n):
+@pytest.mark.parametrize("kernel", ["chosen", "window_stationary", "tile_1", "tile_2", "tile_3", "k_split"])
+def test_gemm_i8_rows_of_any_length(port, monkeypatch, m, k, n, kernel):
     """Rows that are no multiple of a K-step, from a pointer that is no multiple of anything, read where they are: the
-    last row's last pieces, rows shorter than a piece, a matrix shorter than one, on the skinny, the tile and the K-split kernel."""
+    last row's last pieces, rows shorter than a piece, a matrix shorter than one; above 32 rows on the kernel of few tiles, which the sizes
+    give them, and on each of the others."""
     import torch
     from tennis_amd import capi
+    if kernel != "chosen":
+        monkeypatch.setenv("TSX_GEMM_I8_KSPLIT", "force" if kernel == "k_split" else "0")
+        monkeypatch.setenv("TSX_GEMM_I8_TILE", kernel[-1] if kernel.startswith("tile") else "0")
     rng = np.random.default_rng(350 + m + n)
     a = rng.integers(-128, 128, (m, k)).astype(np.int8)
     b = rng.integers(-128, 128, (k, n)).astype(np.int8)

@@ -590,12 +590,24 @@ def test_gemm_i8(tsx, port, m, k, n, transpose):
     assert np.array_equal(bits(out.cpu().numpy()), bits(exp))
 
 
+# GEMMs of more than 32 rows by the kernel that the sizes give them (few tiles of 32 x 32, for those of these tests), and by each of the others
+GEMM_KERNELS = ["chosen", "window_stationary", "tile_1", "tile_2", "tile_3", "k_split"]
+
+
+def gemm_kernel(monkeypatch, kernel):
+    if kernel != "chosen":
+        monkeypatch.setenv("TSX_GEMM_I8_KSPLIT", "force" if kernel == "k_split" else "0")
+        monkeypatch.setenv("TSX_GEMM_I8_TILE", kernel[-1] if kernel.startswith("tile") else "0")
+
+
 @pytest.mark.parametrize("m,k,n", [(33, 64, 128), (256, 1024, 1024), (130, 200, 260), (257, 320, 96), (100, 512, 30),
                                    (64, 128, 64), (500, 192, 1000)])
 @pytest.mark.parametrize("act", [None, "relu"])
-def test_gemm_i8_f32_output_only(tsx, port, m, k, n, act):
-    """More than 32 rows and only the fp32 output wanted: the window-stationary kernel's row-major epilogue
-    (16-byte stores; scalar stores when n is not a multiple of 4), with and without the per-row scale."""
+@pytest.mark.parametrize("kernel", GEMM_KERNELS)
+def test_gemm_i8_f32_output_only(tsx, port, monkeypatch, m, k, n, act, kernel):
+    """More than 32 rows and only the fp32 output wanted: the row-major epilogues (of the window-stationary kernel: 16-byte
+    stores; scalar stores when n is not a multiple of 4), with and without the per-row scale."""
+    gemm_kernel(monkeypatch, kernel)
     rng = np.random.default_rng(310 + m)
     a = rng.integers(-128, 128, (m, k)).astype(np.int8)
     b = rng.integers(-128, 128, (k, n)).astype(np.int8)
@@ -644,8 +656,10 @@ def test_gemm_i8_k_split_kernel(tsx, port, monkeypatch, m, k, n):
     assert np.array_equal(q.cpu().numpy(), port.quantize(exp, qs))
 
 
-def test_gemm_i8_requantized_rows(tsx, port):
+@pytest.mark.parametrize("kernel", GEMM_KERNELS)
+def test_gemm_i8_requantized_rows(tsx, port, monkeypatch, kernel):
     """int8 output with one consumer scale per row (base_quantize.cpp:26 groups by the first extent)."""
+    gemm_kernel(monkeypatch, kernel)
     rng = np.random.default_rng(320)
     m, k, n = 70, 256, 136
     a = rng.integers(-128, 128, (m, k)).astype(np.int8)
