@@ -182,10 +182,11 @@ __device__ __forceinline__ void mish_fragment(float (&v)[16], const Table &table
 
 // The exact Mish where only requantized int8 values leave the kernel: round((mish(x) [+ add]) * scale) has to be the exact
 // form's, the float in between does not.  A short form, x - 2x / (w + 2) as one fused multiply-add behind mish_short's
-// reciprocal, is within 6 * 2^-24 |x| of mish_value for every float x (mish_short is, by comparing all 2^32 inputs on the
-// device, tests/test_gpu_yolo.py; its own two roundings are 2^-24 |x| of that), so with t = the short form's product with the scale + 128
+// reciprocal, is within 8 * 2^-24 |x| of mish_value for every float x: mish_short is within 6 (all 2^32 inputs compared on the
+// device, tests/test_gpu_yolo.py), and its last two roundings, of 1 + quotient and of the product, are 1.5 of that.  With t = the
+// short form's product with the scale + 128
 // both forms round to the same integer wherever t lies further from a rounding boundary k + 1/2 than
-// 2^-20 |x scale| + 2^-16, or, with an addend, 2^-20 |x scale| + 2^-21 |t| + 2^-14: the bound and the roundings of sum, product
+// 2^-20 |x scale| + 2^-16, or, with an addend, 2^-20 |x scale| + 2^-21 |t| + 2^-14: twice the bound and the roundings of sum, product
 // and t, each at most 2^-24 of what it rounds.  There the conversion to a byte, which rounds and saturates to [0, 255], gives the value of
 // quantize_value + 128 whatever its rule for ties.  The few values that lie closer -- about one in ten thousand, and every
 // one whose product is large, infinite or NaN -- are evaluated again by the exact chain, a wavefront at a time and only

@@ -148,8 +148,9 @@ TSX_MISH_FN float tanh_value(float y, const Table &table = Table()) {
     return __builtin_fmaf(2.f, q, -1.f);   // 2q is exact: one rounding, fused or not
 }
 
-// 1 / d rounded to nearest for d in [1, 2]: no scaling is needed there, two Newton steps on the device's reciprocal (every d
-// compared with the division, tests/test_gpu_yolo.py: all of them are in the sweep over Mish's arguments).
+// 1 / d rounded to nearest for d in [1, 2]: no scaling is needed there, two Newton steps on the device's reciprocal.  (Every d that
+// occurs gives the division's bits in Mish: tests/test_gpu_yolo.py, which holds mish_value against x tanh(softplus(x)) by
+// the functions above for all floats on the device.)
 #ifdef __HIP_DEVICE_COMPILE__
 TSX_MISH_FN float reciprocal_rn_1_2(float d) {
     const float a = __builtin_amdgcn_rcpf(d);
