@@ -82,8 +82,24 @@ namespace {
 constexpr int ws_waves(int nt, int fill, bool look, bool mishx) {
     return nt > 4 ? 1 : fill != SMALL_FILL ? 2 : nt == 1 && !look ? 5 : mishx && nt == 2 ? 3 : 4;
 }
-template <int NT, int FM, bool EXTRA, bool STREAM, bool ROWM, int FILL, bool LOOK, bool MISHX = false>
-__global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_waves(NT, FILL, LOOK, MISHX)))) void conv_i8_ws_kernel(WsParams p_in) {
+
+// The hot case of the epilogue: no raw accumulators wanted, every element inside the activation's SIMD-body range,
+// a tensor small enough for 32-bit lane offsets, and -- for the requantized output -- one
+// quantize group per image (or a single scale whose round-half-even bulk covers everything),
+// so the consumer's scale is uniform for a tile and needs no per-element division.
+__host__ __device__ inline bool ws_uniform(const WsParams &p) {
+    const int64_t image = int64_t(p.cout) * (p.ho * p.wo), count = p.n * image;
+    const bool want_q = p.out_i8 || p.st_out;
+    const bool q_uniform = !want_q || (p.n_qscales == 1 ? p.q_bulk8 == count : p.q_group_len == image);
+    return (p.out_f32 || want_q) && !p.out_acc && p.act_body == count && count < (int64_t(1) << 30) && q_uniform;
+}
+
+// MISHX: 0 without the exact Mish; 1 with it; 2 with it where every fragment is whole and takes the epilogue of the hot case
+// below, so that the other one, whose scalars are most of what the kernel holds, is not in it (spilled scalars 50 - 66 in the
+// general kernels of one and two fragments, none in these; YOLOv4's pass on 8 images, every
+// layer of whole fragments: 2645 us without them, 2533 with).
+template <int NT, int FM, bool EXTRA, bool STREAM, bool ROWM, int FILL, bool LOOK, int MISHX>
+__global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_waves(NT, FILL, LOOK, MISHX != 0)))) void conv_i8_ws_kernel(WsParams p_in) {
     WsParams p = p_in;
     if (!EXTRA) {
         p.residual = nullptr;
@@ -211,16 +227,10 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
     // its K-loop waits a full memory latency there, with nothing else on its SIMD to hide it
     const int tile_pos = p.th * p.tw;
     const int howo = p.ho * p.wo;
-    const int64_t count = int64_t(p.n) * p.cout * howo;
-    // hot case: no raw accumulators wanted, every element inside the activation's SIMD-body range,
-    // a tensor small enough for 32-bit lane offsets, and -- for the requantized output -- one
-    // quantize group per image (or a single scale whose round-half-even bulk covers everything),
-    // so the consumer's scale is uniform for this tile and needs no per-element division
     const bool want_q = p.out_i8 || p.st_out;
-    const bool q_uniform = !want_q || (p.n_qscales == 1 ? p.q_bulk8 == count : p.q_group_len == int64_t(p.cout) * howo);
     // the GEMM form stores 4 consecutive channels at once, and its quantize groups are rows, not images
     const bool rowm_ok = !ROWM || (!want_q && p.cout % 4 == 0 && reinterpret_cast<uintptr_t>(p.out_f32) % 16 == 0);
-    const bool fast = (p.out_f32 || want_q) && !p.out_acc && p.act_body == count && count < (int64_t(1) << 30) && q_uniform && rowm_ok;
+    const bool fast = MISHX == 2 || (ws_uniform(p) && rowm_ok);
     // a tile may end in the next image: one consumer scale per image, selected per lane
     const float q_scale_a = (fast && want_q) ? p.q_scales[p.n_qscales == 1 ? 0 : img] : 0.f;
     const float q_scale_b = (fast && want_q) ? p.q_scales[p.n_qscales == 1 ? 0 : min(img + 1, p.n - 1)] : 0.f;
@@ -371,7 +381,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
         constexpr int f = decltype(fc)::value;
         const int cf = m0 + f * 32;   // first cout of this fragment (uniform)
         // fast: all 32 channels exist, the loads need no bounds and combine into 16-byte ones
-        const bool fast_f = fast && cf + 32 <= p.cout;
+        const bool fast_f = fast && cf + 32 <= p.cout;   // (a wavefront of the last block may have no channel at all)
         // Loads without per-element branches: the fast case needs no bounds (consecutive channels combine into
         // 16-byte loads); otherwise the index is clamped, and what a channel beyond cout loads is never stored.
         float dq[16], bias[16];
@@ -561,7 +571,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
             fragments(std::true_type{});
         } else if (fast && !EXTRA && !MISHX) {
             if constexpr (!EXTRA && !MISHX) fragments(std::false_type{});
-        } else {
+        } else if constexpr (MISHX != 2) {
             static_for<0, NT>([&](auto jc) {
                 constexpr int j = decltype(jc)::value;
                 const int pos = pos0 + j * 32 + lane % 32;
@@ -587,7 +597,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
 #pragma clang loop unroll(disable)
                     for (int r = 0; r < 16; r += 2) {
                         const int dco = 8 * (r / 4) + r % 4;
-                        emit_rows<2, MISHX>(p, {a[r], a[r + 1]}, base + int64_t(dco) * howo, howo, pos_ok ? p.cout - co0 - dco : 0, img + (wrapped ? 1 : 0),
+                        emit_rows<2, MISHX != 0>(p, {a[r], a[r + 1]}, base + int64_t(dco) * howo, howo, pos_ok ? p.cout - co0 - dco : 0, img + (wrapped ? 1 : 0),
                                             co0 + dco, pixel, {d[r], d[r + 1]}, {b[r], b[r + 1]}, MishTablesInLds{&mish_tables});
                     }
                 } else static_for<0, 16>([&](auto rc) {
@@ -632,15 +642,16 @@ int ws_launch_nt<TSX_WS_NT>(const WsParams &p, dim3 grid, size_t lds_bytes, hipS
         }                                                                                                              \
         hipLaunchKernelGGL(kernel, grid, dim3(WS_THREADS), lds_bytes, stream, p);                                      \
     } while (0)
-    // the exact Mish: one instantiation (with every other epilogue term) that only its layers run
+    // the exact Mish: instantiations (with every other epilogue term) that only its layers run
     if (p.act == TSX_ACT_MISH) {
         if (p.rowmajor) return fail(TSX_E_INVALID, "conv_i8_ws: the exact Mish is not compiled into the row-major form");
-        TSX_WS_LAUNCH(true, false, false, true);
+        if (NT <= 2 && p.cout % 32 == 0 && ws_uniform(p)) TSX_WS_LAUNCH(true, false, false, NT <= 2 ? 2 : 1);
+        else TSX_WS_LAUNCH(true, false, false, 1);
     }
-    else if (p.rowmajor) TSX_WS_LAUNCH(false, false, true, false);
-    else if (p.residual || p.st_out) TSX_WS_LAUNCH(true, false, false, false);
-    else if (p.stream_out) TSX_WS_LAUNCH(false, true, false, false);
-    else TSX_WS_LAUNCH(false, false, false, false);
+    else if (p.rowmajor) TSX_WS_LAUNCH(false, false, true, 0);
+    else if (p.residual || p.st_out) TSX_WS_LAUNCH(true, false, false, 0);
+    else if (p.stream_out) TSX_WS_LAUNCH(false, true, false, 0);
+    else TSX_WS_LAUNCH(false, false, false, 0);
 #undef TSX_WS_LAUNCH
     TSX_LAUNCH_CHECK("conv_i8_ws_kernel");
     return 0;

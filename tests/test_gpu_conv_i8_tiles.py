@@ -53,9 +53,10 @@ def test_conv_i8_tiles(port, monkeypatch, case, act):
 
 @pytest.mark.parametrize("n", [1, 2])
 @pytest.mark.parametrize("act", ["mish", "mish_fast", "relu"])
-@pytest.mark.parametrize("cout", [9, 18, 33, 47, 63, 65])
+@pytest.mark.parametrize("cout", [9, 18, 33, 47, 63, 65, 32, 96])
 def test_channels_of_partial_fragments(port, monkeypatch, cout, act, n):
-    """Fragments whose 32 channels do not all exist, with a join: raw sums, fp32, NCHW int8 (one image: half to even up to the last
+    """Fragments whose 32 channels do not all exist, and those that do where a kernel has nothing else (a wavefront of the last block
+    may have no channel at all there; with raw sums they take the other epilogue), with a join: raw sums, fp32, NCHW int8 (one image: half to even up to the last
     whole eight; two: a scale each) and staged int8, by itself and upsampled."""
     from tennis_amd import capi
     monkeypatch.setenv("TSX_CONV_I8_KS", "0")
@@ -78,6 +79,8 @@ def test_channels_of_partial_fragments(port, monkeypatch, cout, act, n):
     expected = port.quantize(joined, qs)
     out, q, acc = conv(dev(x), dq=dev(dq), bias=dev(bias), act=act, q_scales=dev(qs), residual=dev(res), residual_after_act=True, want_acc=True)
     assert np.array_equal(acc.cpu().numpy(), np.einsum("nchw,oc->nohw", x.astype(np.int32), wt[:, :, 0, 0].astype(np.int32)))
+    assert np.array_equal(bits(out.cpu().numpy()), bits(joined)) and np.array_equal(q.cpu().numpy(), expected)
+    out, q, _ = conv(dev(x), dq=dev(dq), bias=dev(bias), act=act, q_scales=dev(qs), residual=dev(res), residual_after_act=True)
     assert np.array_equal(bits(out.cpu().numpy()), bits(joined)) and np.array_equal(q.cpu().numpy(), expected)
     q = conv(dev(x), dq=dev(dq), bias=dev(bias), act=act, q_scales=dev(qs), residual=dev(res), residual_after_act=True, want_f32=False)[1]
     assert np.array_equal(q.cpu().numpy(), expected)
