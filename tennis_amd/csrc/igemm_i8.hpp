@@ -148,7 +148,8 @@ __device__ __forceinline__ void emit_rows(const EpiParams &p, const int (&acc)[N
 // element costs more instructions than the arithmetic).  Caller guarantees: no raw-accumulator
 // output, every element in the activation's SIMD-body range, one quantize scale for this lane's
 // image (q_scale, rounding half to even iff q_even).  st_dst = the lane's pixel in the consumer's
-// staged layout at its first channel row, or null.
+// staged layout at its first channel row, or null.  MISHX: the activation is the exact Mish.
+template <bool MISHX>
 __device__ __forceinline__ void epilogue_rows16(const EpiParams &p, const v16i &acc, const float (&dq)[16],
                                                 const float (&bias)[16], int64_t idx0, int64_t row_stride, float q_scale,
                                                 bool q_even, int8_t *st_dst, const MishTablesInLds &tables) {
@@ -167,19 +168,19 @@ __device__ __forceinline__ void epilogue_rows16(const EpiParams &p, const v16i &
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = __fadd_rn(v[r], res[r]);
     }
-    const bool q_only = p.act == TSX_ACT_MISH && !p.out_f32 && (p.out_i8 || st_dst);      // the Mish's fp32 values go nowhere
+    const bool q_only = MISHX && !p.out_f32 && (p.out_i8 || st_dst);      // the Mish's fp32 values go nowhere
     uint32_t word[4] = {0u, 0u, 0u, 0u};        // requantized values
-    if (p.act == TSX_ACT_RELU) {
+    if (MISHX) {
+        // nothing but the requantized values leaves: the exact form only where it decides a rounding
+        if (!q_only) mish_fragment(v, tables);
+        else if (p.residual && p.res_after) mish_words_for_rounding<true>(v, res, q_scale, q_even, word, tables);
+        else mish_words_for_rounding<false>(v, res, q_scale, q_even, word, tables);
+    } else if (p.act == TSX_ACT_RELU) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = v[r] > 0.f ? v[r] : 0.f;
     } else if (p.act == TSX_ACT_LEAKY_RELU) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = apply_act_conv_i8(v[r], TSX_ACT_LEAKY_RELU, p.slope, true);
-    } else if (p.act == TSX_ACT_MISH) {
-        // nothing but the requantized values leaves: the exact form only where it decides a rounding
-        if (!q_only) mish_fragment(v, tables);
-        else if (p.residual && p.res_after) mish_words_for_rounding<true>(v, res, q_scale, q_even, word, tables);
-        else mish_words_for_rounding<false>(v, res, q_scale, q_even, word, tables);
     } else if (p.act == TSX_ACT_MISH_FAST) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = apply_act_conv_i8(v[r], TSX_ACT_MISH_FAST, 0.f, true);
