@@ -1603,12 +1603,17 @@ int tsx_gemm_i8(int32_t m, int32_t n, int32_t k, const int8_t *a_dev, const void
     // to one workgroup per CU, or two with a K that keeps what a CU fetches below a tile of theirs (us, theirs -> here: 197 x
     // 777, K = 1500, fp32 10.0 -> 5.4, int8 11.5 -> 6.1; 256 x 1024, K = 1024, 5.7 -> 4.6; 48 x 4096, K = 4096, 10.8 -> 7.9; 131 x 95,
     // K = 2179, 12.9 -> 10.2; 400 x 500, K = 300, 6.0 -> 3.9; 2048 x 256, K = 512, 5.0 -> 4.9; but 256 x 2048, K = 2048, 7.8 -> 8.1
-    // and 640 x 1024, K = 128, 4.4 -> 5.5).  A switch of another kernel leaves more than 32 rows to these.
+    // and 640 x 1024, K = 128, 4.4 -> 5.5).  Pieces at odd addresses take a CU longer to fetch, once for each of its tiles: two tiles
+    // a CU then pay up to a third of that (1215 x 211, K = 2809, 15.4 -> 18.8; 474 x 608, K = 1565, 9.8 -> 11.2; 330 tiles with K =
+    // 1900 12.9 -> 18.9; below the line 0.7 - 0.95 of theirs), one up to K = 7000 (60 x 3468, K = 7239, 21.9 -> 23.2).
+    // A switch of another kernel leaves more than 32 rows to these.
     {
         const auto set = [](const char *name) { const char *value = std::getenv(name); return value && value[0]; };
         const int row_blocks = int(tsx::ceil_div(m, 32));
         const int64_t tiles = tsx::ceil_div(n, 32) * row_blocks;
-        const bool few = m > 32 && (tiles <= 256 || (tiles <= 512 && tiles * kp <= 900000)) && !set("TSX_GEMM_I8_KSPLIT") && !set("TSX_GEMM_I8_TILE");
+        const bool odd = k % 4 != 0 || reinterpret_cast<uintptr_t>(a_dev) % 4 != 0;
+        const bool pays = tiles <= 256 ? !odd || kp <= 7000 : tiles <= 512 && tiles * kp <= (odd ? 330000 : 900000);
+        const bool few = m > 32 && pays && !set("TSX_GEMM_I8_KSPLIT") && !set("TSX_GEMM_I8_TILE");
         if (m <= 32 || few) {
             if (p.x_bytes < 16 && (rc = pad_rows())) return rc;      // less than a piece
             if (m <= 32) hipLaunchKernelGGL(gemm_i8_skinny_kernel<false>, dim3(unsigned(tiles)), dim3(SK_WAVES * 64), 0, stream, p, 1);

@@ -18,7 +18,9 @@ def bits(a):
 
 @pytest.mark.parametrize("kernel", ["few", "ksplit"])
 @pytest.mark.parametrize("m,k,n", [(33, 64, 32), (64, 65, 31), (65, 2049, 33), (40, 2048, 95), (200, 15, 100), (34, 16, 4), (1000, 63, 40), (160, 2112, 132),
-                                   (35, 4100, 5), (256, 512, 1024), (500, 300, 1024)])
+                                   (35, 4100, 5), (256, 512, 1024), (500, 300, 1024),
+                                   # rows at odd addresses, which this kernel takes up to a K of 7000, or two tiles a CU up to a shorter one
+                                   (33, 6931, 96), (33, 7001, 96), (300, 1061, 928), (300, 1301, 928)])
 def test_few_tiles(port, monkeypatch, m, k, n, kernel):
     import torch
     from tennis_amd import capi
