@@ -151,8 +151,8 @@ __global__ __launch_bounds__(256) void channel_affine_kernel(const float *__rest
 
 // The same with one wavefront per plane, for planes of a multiple of 4 elements: the channel's parameters, and with them
 // the reciprocal root in double (as many issue slots as fifteen elements), are worked out once per plane instead of once
-// per 4 elements (32x256x56x56: 38.8 us, with whole
-// rounds of 256 runs, the last of four nearly empty, 38.5, now 33).
+// per 4 elements (32x256x56x56: 38.8 us; 38.5 with whole rounds of 256 runs, the last of four nearly empty; 33 so, 30 of them
+// the kernel's by rocprofv3).
 template <int NORM>
 __global__ __launch_bounds__(256) void plane_affine_kernel(const float *__restrict__ x, int64_t planes, int channels, int inner4,
                                                           const float *__restrict__ mean, const float *__restrict__ variance,
