@@ -345,21 +345,8 @@ __device__ __forceinline__ void fl_wave(const FlParams &p, int8_t *lds, MishTabl
                 } else {
                     mish_fragment(v, tables);
                 }
-            } else if (p.act == TSX_ACT_RELU) {
-                static_for<0, 16>([&](auto rc) {
-                    constexpr int r = decltype(rc)::value;
-                    v[r] = v[r] > 0.f ? v[r] : 0.f;
-                });
-            } else if (p.act == TSX_ACT_LEAKY_RELU) {
-                static_for<0, 16>([&](auto rc) {
-                    constexpr int r = decltype(rc)::value;
-                    v[r] = apply_act_conv_i8(v[r], TSX_ACT_LEAKY_RELU, p.slope, true);
-                });
-            } else if (p.act == TSX_ACT_MISH_FAST) {
-                static_for<0, 16>([&](auto rc) {
-                    constexpr int r = decltype(rc)::value;
-                    v[r] = apply_act_conv_i8(v[r], TSX_ACT_MISH_FAST, 0.f, true);
-                });
+            } else {
+                activate_results(v, p.act, p.slope);
             }
             if (EXTRA && p.residual && p.res_after && !q_only) static_for<0, 16>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
@@ -375,17 +362,7 @@ __device__ __forceinline__ void fl_wave(const FlParams &p, int8_t *lds, MishTabl
                 else *o = v[r];
             });
             if (want_q) {
-                if (!q_only) static_for<0, 4>([&](auto gc) { word[decltype(gc)::value] = 0; });
-                if (q_only) {
-                } else if (q_even) static_for<0, 16>([&](auto rc) {
-                    constexpr int r = decltype(rc)::value;
-                    word[r / 4] = quantize_pack<r % 4>(__fmul_rn(v[r], q_scale), true, word[r / 4]);
-                });
-                else static_for<0, 16>([&](auto rc) {
-                    constexpr int r = decltype(rc)::value;
-                    word[r / 4] = quantize_pack<r % 4>(__fmul_rn(v[r], q_scale), false, word[r / 4]);
-                });
-                static_for<0, 4>([&](auto gc) { word[decltype(gc)::value] ^= 0x80808080u; });
+                if (!q_only) quantize_words(v, q_scale, q_even, word);
                 if (p.out_i8) static_for<0, 16>([&](auto rc) {
                     constexpr int r = decltype(rc)::value;
                     constexpr int dco = 8 * (r / 4) + (r % 4);

@@ -159,7 +159,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MT == 1 
         if (p.bias) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], bias[u][r]); });
         if (p.residual && !p.res_after) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], res[u][r]); });
         if (MISHX) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_value(v[r]); });
-        else if (p.act == TSX_ACT_MISH_FAST) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_short(v[r]); });
+        else if (p.act == TSX_ACT_MISH_FAST) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_short_behind_a_branch(v[r]); });
         else if (p.act != TSX_ACT_NONE) each([&](auto rc) {
             constexpr int r = decltype(rc)::value;
             v[r] = apply_act_basic(v[r], p.act, p.slope, idx0 + int64_t(r) * p.howo < p.act_body);

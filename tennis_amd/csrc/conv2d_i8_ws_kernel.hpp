@@ -481,21 +481,8 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
                         } else {
                             mish_fragment(v, tables);
                         }
-                    } else if (p.act == TSX_ACT_RELU) {
-                        static_for<0, 16>([&](auto rc) {
-                            constexpr int r = decltype(rc)::value;
-                            v[r] = v[r] > 0.f ? v[r] : 0.f;
-                        });
-                    } else if (p.act == TSX_ACT_LEAKY_RELU) {
-                        static_for<0, 16>([&](auto rc) {
-                            constexpr int r = decltype(rc)::value;
-                            v[r] = apply_act_conv_i8(v[r], TSX_ACT_LEAKY_RELU, p.slope, true);
-                        });
-                    } else if (p.act == TSX_ACT_MISH_FAST) {
-                        static_for<0, 16>([&](auto rc) {
-                            constexpr int r = decltype(rc)::value;
-                            v[r] = apply_act_conv_i8(v[r], TSX_ACT_MISH_FAST, 0.f, true);
-                        });
+                    } else {
+                        activate_results(v, p.act, p.slope);
                     }
                     if (EXTRA && p.residual && p.res_after && !q_only) static_for<0, 16>([&](auto rc) {
                         constexpr int r = decltype(rc)::value;
@@ -521,19 +508,8 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
                         else *o = v[r];
                     });
                     if (!ROWM && want_q) {
-                        // the 16 requantized values as 4 dwords of 4 consecutive channels (quantize_pack: the value of
-                        // quantize_value, converted, clamped and packed by one instruction)
-                        if (!q_only) static_for<0, 4>([&](auto gc) { word[decltype(gc)::value] = 0; });
-                        if (q_only) {
-                        } else if (q_even) static_for<0, 16>([&](auto rc) {
-                            constexpr int r = decltype(rc)::value;
-                            word[r / 4] = quantize_pack<r % 4>(__fmul_rn(v[r], q_scale), true, word[r / 4]);
-                        });
-                        else static_for<0, 16>([&](auto rc) {
-                            constexpr int r = decltype(rc)::value;
-                            word[r / 4] = quantize_pack<r % 4>(__fmul_rn(v[r], q_scale), false, word[r / 4]);
-                        });
-                        static_for<0, 4>([&](auto gc) { word[decltype(gc)::value] ^= 0x80808080u; });
+                        // the 16 requantized values as 4 dwords of 4 consecutive channels
+                        if (!q_only) quantize_words(v, q_scale, q_even, word);
                         if (p.out_i8) static_for<0, 16>([&](auto rc) {
                             constexpr int r = decltype(rc)::value;
                             constexpr int dco = 8 * (r / 4) + (r % 4);

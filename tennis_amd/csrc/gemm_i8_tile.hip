@@ -37,7 +37,7 @@ __device__ __forceinline__ void activate(float (&v)[N], const EpiParams &p, Body
     } else if (p.act == TSX_ACT_LEAKY_RELU) {
         static_for<0, N>([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = apply_act_basic(v[r], TSX_ACT_LEAKY_RELU, p.slope, in_body(rc)); });
     } else if (p.act == TSX_ACT_MISH_FAST) {
-        static_for<0, N>([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_short(v[r]); });
+        static_for<0, N>([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_short_behind_a_branch(v[r]); });
     }
 }
 
@@ -256,15 +256,7 @@ __global__ __launch_bounds__(THREADS) void gemm_i8_tile_kernel(GemmTileParams p)
                     if (p.row_scale) static_for<0, 16>([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fmul_rn(v[r], rs); });
                     if (p.bias) static_for<0, 16>([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], bias[r / 4][r % 4]); });
                     activate(v, p, [](auto) { return true; });
-                    static_for<0, 4>([&](auto gc) {
-                        constexpr int g = decltype(gc)::value;
-                        uint32_t bytes = 0;
-                        static_for<0, 4>([&](auto jc) {
-                            constexpr int j = decltype(jc)::value;
-                            bytes = quantize_pack<j>(__fmul_rn(v[4 * g + j], qs), false, bytes);
-                        });
-                        word[g] = bytes ^ 0x80808080u;
-                    });
+                    quantize_words(v, qs, false, word);
                     const auto s02 = __builtin_amdgcn_permlane32_swap(word[0], word[2], false, false);
                     const auto s13 = __builtin_amdgcn_permlane32_swap(word[1], word[3], false, false);
                     const int co = cf + 16 * (lane / 32);

@@ -111,7 +111,7 @@ __device__ __forceinline__ void emit_rows(const EpiParams &p, const int (&acc)[N
     if (p.bias) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], bias[r]); });
     if (p.residual && !p.res_after) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], res[r]); });
     if (MISHX) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_value(v[r], table); });
-    else if (p.act == TSX_ACT_MISH_FAST) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_short(v[r]); });
+    else if (p.act == TSX_ACT_MISH_FAST) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = mish_short_behind_a_branch(v[r]); });
     else if (p.act != TSX_ACT_NONE) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = apply_act_basic(v[r], p.act, p.slope, idx0 + at[r] < p.act_body); });
     if (p.residual && p.res_after) each([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], res[r]); });
     if (p.out_f32) each([&](auto rc) { constexpr int r = decltype(rc)::value; if (r < left) (p.out_f32 + idx0)[at[r]] = v[r]; });
@@ -169,21 +169,14 @@ __device__ __forceinline__ void epilogue_rows16(const EpiParams &p, const v16i &
         for (int r = 0; r < 16; ++r) v[r] = __fadd_rn(v[r], res[r]);
     }
     const bool q_only = MISHX && !p.out_f32 && (p.out_i8 || st_dst);      // the Mish's fp32 values go nowhere
-    uint32_t word[4] = {0u, 0u, 0u, 0u};        // requantized values
+    uint32_t word[4];        // requantized values
     if (MISHX) {
         // nothing but the requantized values leaves: the exact form only where it decides a rounding
         if (!q_only) mish_fragment(v, tables);
         else if (p.residual && p.res_after) mish_words_for_rounding<true>(v, res, q_scale, q_even, word, tables);
         else mish_words_for_rounding<false>(v, res, q_scale, q_even, word, tables);
-    } else if (p.act == TSX_ACT_RELU) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = v[r] > 0.f ? v[r] : 0.f;
-    } else if (p.act == TSX_ACT_LEAKY_RELU) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = apply_act_conv_i8(v[r], TSX_ACT_LEAKY_RELU, p.slope, true);
-    } else if (p.act == TSX_ACT_MISH_FAST) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = apply_act_conv_i8(v[r], TSX_ACT_MISH_FAST, 0.f, true);
+    } else {
+        activate_results(v, p.act, p.slope);
     }
     if (p.residual && p.res_after && !q_only) {
 #pragma unroll
@@ -194,17 +187,7 @@ __device__ __forceinline__ void epilogue_rows16(const EpiParams &p, const v16i &
         for (int r = 0; r < 16; ++r) p.out_f32[idx0 + int64_t(8 * (r / 4) + (r % 4)) * row_stride] = v[r];
     }
     if (p.out_i8 || st_dst) {
-        if (q_only) {
-        } else if (q_even) static_for<0, 16>([&](auto rc) {
-            constexpr int r = decltype(rc)::value;
-            word[r / 4] = quantize_pack<r % 4>(__fmul_rn(v[r], q_scale), true, word[r / 4]);
-        });
-        else static_for<0, 16>([&](auto rc) {
-            constexpr int r = decltype(rc)::value;
-            word[r / 4] = quantize_pack<r % 4>(__fmul_rn(v[r], q_scale), false, word[r / 4]);
-        });
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) word[g4] ^= 0x80808080u;
+        if (!q_only) quantize_words(v, q_scale, q_even, word);
         if (p.out_i8) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) p.out_i8[idx0 + int64_t(8 * (r / 4) + (r % 4)) * row_stride] = int8_t(word[r / 4] >> (8 * (r % 4)));
