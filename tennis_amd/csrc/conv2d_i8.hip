@@ -21,6 +21,7 @@
 // so any consistent K permutation gives the same exact integer result.  Accumulator register
 // r of lane l holds row 8*(r/4) + 4*(l/32) + (r%4), column l % 32.
 #include "gemm_i8_tile.hpp"
+#include "conv2d_i8_px.hpp"
 #include "igemm_i8.hpp"
 #include "stage_i8.hpp"
 
@@ -28,6 +29,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <mutex>
 
 namespace {
@@ -1086,7 +1088,7 @@ int make_plan(const tsx_conv2d_geom *g, Plan *pl) {
             pl->use_ws = true;
             pl->packed_bytes = pl->wsp.packed_bytes;
         } else if (strided_1x1) {
-            pl->wsp.coutp = pl->coutp;     // the K-split kernel, which small ones take, reads the generic kernel's weights
+            pl->wsp.coutp = pl->coutp;     // the K-split and the pixel-stream kernel read the generic kernel's weights
         }
     }
     return 0;
@@ -1269,7 +1271,7 @@ int run_staged(const tsx_conv2d_geom *g, const Plan &pl, const void *staged, con
     p.o_c = g->cout;
     p.o_h = pl.ho;
     p.o_w = pl.wo;
-    if (pl.use_ws || pl.wsp.ks)
+    if (pl.use_ws || pl.wsp.ks || tsx::px_takes(pl.wsg, pl.wsp, p))
         return tsx::ws_launch(pl.wsg, pl.wsp, p.xs, p.wp, static_cast<const tsx::EpiParams &>(p), stream);
     return launch_igemm<false>(p, stream);
 }
@@ -1323,6 +1325,10 @@ int tsx_conv2d_i8_plan_info(const tsx_conv2d_geom *g, char *text, size_t text_by
     else
         std::snprintf(text, text_bytes, "kernel=%s fp32_kernel=%s", base, base);
     if (pl.wsp.ks) std::snprintf(text, text_bytes, "kernel=k_split fp32_kernel=k_split tile=%d", pl.wsp.ks);
+    else if (pl.wsp.px) {      // for fp32 and staged outputs; the kernel named before writes the others
+        const size_t used = std::strlen(text);
+        std::snprintf(text + used, text_bytes - used, " pixel_stream=1");
+    }
     return 0;
 }
 
@@ -1512,7 +1518,7 @@ int tsx_conv2d_i8_staged_at(const tsx_conv2d_geom *g, const void *staged_dev, in
             return tsx::fail(TSX_E_INVALID, "staged_at: a %dx%d staged buffer does not fit this layer's kernel", staged_hs,
                              staged_ws);
         }
-    } else if (pl.wsp.ks) {
+    } else if (pl.wsp.ks || pl.wsp.px) {
         pl.wsg.hs = staged_hs;
         pl.wsg.ws = staged_ws;
         const tsx::WsPlan wide = tsx::ws_plan(pl.wsg);

@@ -33,6 +33,7 @@
 // of lane l is row 8*(r/4) + 4*(l/32) + r%4, column l%32.  Rows = cout, columns = positions.
 #include "conv2d_i8_ws_kernel.hpp"
 #include "conv2d_i8_ks.hpp"
+#include "conv2d_i8_px.hpp"
 #include "tsx_plans.hpp"
 
 #include <algorithm>
@@ -78,11 +79,13 @@ static WsPlan make_ws_plan(const WsGeom &g_in);
 WsPlan ws_plan(const WsGeom &g) {
     struct Key {
         WsGeom g;
-        PlanSwitch flat, rs, ks;
+        PlanSwitch flat, rs, ks, px;
     } key;
     std::memset(&key, 0, sizeof(key));
     key.g = g;
-    if (!key.flat.read("TSX_CONV_I8_FLAT") || !key.rs.read("TSX_CONV_I8_RS") || !key.ks.read("TSX_CONV_I8_KS")) return make_ws_plan(g);
+    if (!key.flat.read("TSX_CONV_I8_FLAT") || !key.rs.read("TSX_CONV_I8_RS") || !key.ks.read("TSX_CONV_I8_KS") ||
+        !key.px.read("TSX_CONV_I8_PX"))
+        return make_ws_plan(g);
     return kept_plan<WsPlan>(key, [&] { return make_ws_plan(g); });
 }
 
@@ -208,6 +211,7 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
     fl_plan(g_in, &pl);   // layers the flat-tile kernel suits better (same packed weights)
     rs_plan(g_in, &pl);   // ... and the weight-stationary one
     ks_plan(g_in, &pl);   // ... and the one that splits K
+    px_plan(g_in, &pl);   // ... and the one for streams of pixels
     return pl;
 }
 
@@ -233,6 +237,7 @@ int ws_launch(const WsGeom &g, const WsPlan &plan, const int8_t *xs, const int8_
         pl.tiles = ceil_div(int64_t(g.n) * pl.ho, pl.th);
     }
     if (pl.ks) return ks_launch(g, pl, xs, packed, ep, stream);
+    if (px_takes(g, pl, ep)) return px_launch(g, pl, xs, packed, ep, stream);
     if (rs_takes(pl, ep, int64_t(g.n) * g.cout * g.ho * g.wo)) return rs_launch(g, pl, xs, packed, ep, stream);
     if (fl_takes(g, pl, ep)) return fl_launch(g, pl, xs, packed, ep, stream);
     WsParams p{};

@@ -230,6 +230,8 @@ struct WsPlan {
     // fragments x 64 output channels; same packed weights
     bool rs;
     int rs_frags, rs_ptiles, rs_nr, rs_rowp, rs_wc, rs_lds;
+    // pixel-stream kernel (conv2d_i8_px.hip) for the epilogues it writes; same packed weights
+    bool px;
     // K-split kernel (conv2d_i8_ks.hip): its tile, counted from 1, or 0; same packed weights
     int ks;
 };

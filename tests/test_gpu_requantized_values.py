@@ -19,19 +19,21 @@ SPECIAL = np.array([0.0, -0.0, 0.5, -0.5, 1.5, 2.5, -2.5, 0.49999997, -0.4999999
 
 @pytest.mark.parametrize("images", [1, 3])
 @pytest.mark.parametrize("act", ["none", "relu", "leaky_relu"])
-@pytest.mark.parametrize("kernel", ["window_stationary", "flat_tile", "igemm"])
+@pytest.mark.parametrize("kernel", ["pixel_stream", "window_stationary", "flat_tile", "igemm"])
 def test_requantized_special_values(port, monkeypatch, kernel, act, images):
     """Products on ties, beyond int8 and int32, infinite and NaN: the bias alone (the input is zero)."""
     from tennis_amd import capi
     monkeypatch.setenv("TSX_CONV_I8_KS", "0")
+    if kernel != "pixel_stream":
+        monkeypatch.setenv("TSX_CONV_I8_PX", "0")
     if kernel == "flat_tile":
         monkeypatch.setenv("TSX_CONV_I8_FLAT", "force")
-    k, st = (1, 2) if kernel == "igemm" else (3, 1)
+    k, st = (1, 2) if kernel == "igemm" else (1, 1) if kernel == "pixel_stream" else (3, 1)
     n, c, h, cout = images, 64, 16, 128
     bias = np.concatenate([SPECIAL, SPECIAL[::-1]] * 2)
     conv = capi.Conv2dI8(dev(np.ones((cout, c, k, k), np.int8)), (k // 2,) * 4, (st, st))
     info = capi.conv2d_i8_plan_info(conv._plan((n, c, h, h))[0])
-    assert info["kernel"] == kernel, info
+    assert info["kernel"] == ("window_stationary" if kernel == "pixel_stream" else kernel) and ("pixel_stream" in info) == (kernel == "pixel_stream"), info
     ho = (h - 1) // st + 1
     second = capi.Conv2dI8(dev(np.zeros((32, cout, 1, 1), np.int8)))
     out, staged = capi.StagedInput(second, (n, cout, ho, ho)), capi.StagedInput(conv, (n, c, h, h))
