@@ -16,7 +16,7 @@
 // 64 15.2 -> 11.6; 64 to 256 with a join (fp32 and int8 out) 50.2 -> 44.2, 5.4 TB/s; 128 to 512 28x28 34.5 -> 28.3; 256 to 1024 14x14 22.4 ->
 // 19.6 (these read and write fp32 planes in pieces of 128 bytes, for which 205 MB take 37 us at 56x56 and 51 MB 12.4 at 14x14
 // with nothing else done); 1024 to 256 14x14 9.0 -> 7.4; 256 to 512 56x56 at stride 2 19.8 -> 13.1, 1024 to 2048 14x14 17.9 -> 12.7.  8
-// images with the exact Mish: 64 to 64 304x304, int8 out, 57.5 -> 38.6 (vector instructions), fp32 and int8 126 -> 114; 512 to 512 19x19 8.3 -> 6.8.
+// images with the exact Mish: 64 to 64 304x304, int8 out, 57.5 -> 38.6 (vector instructions), fp32 and int8 126 -> 97; 512 to 512 19x19 8.3 -> 6.8.
 #include "conv2d_i8_px.hpp"
 
 #include <algorithm>
@@ -44,7 +44,7 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // wavefronts per SIMD that the registers leave room for
-constexpr int px_waves(int ks, int wn, bool res, bool mishx) { return ks == 16 ? 2 : ks == 8 || (res && (ks == 4 || (mishx && ks * wn == 8))) ? 3 : 4; }
+constexpr int px_waves(int ks, int wn, bool res, bool mishx) { return ks == 16 ? 2 : ks == 8 || (res && ks == 4) || (mishx && ks * wn == 8) ? 3 : 4; }
 
 // KS: K-steps of 64 channels.  WN: fragments of a group (4 / WN wavefronts along cout).  RES: a residual joins.  F32, Q: fp32
 // values, requantized ones leave.  MISHX: the activation is the exact Mish.  The loads and stores of a turn are the same in every

@@ -196,21 +196,24 @@ __device__ __forceinline__ float apply_act(float v, int act, float slope, bool i
     return apply_act_basic(v, act, slope, in_body);
 }
 // The tables of the exact Mish in the workgroup's LDS: the 32 entries of the exponential's take two banks each, so a read of
-// any 64 of them is free of conflicts.  (Held in the wavefront's lanes and read with ds_bpermute, a look-up takes 28 cycles
-// of a SIMD's share of the LDS pipe per 32 bits: seven of them were as long as the arithmetic.)
-struct MishTables {
+// any 64 of them is free of conflicts; the logarithm's two are read by one instruction, at multiples of 512 bytes from each other.
+// (Held in the wavefront's lanes and read with ds_bpermute, a look-up takes 28 cycles of a SIMD's share of the LDS pipe per 32
+// bits: seven of them were as long as the arithmetic.)
+struct __attribute__((aligned(512))) MishTables {
+    double twice_inverse[256], log_of[256];
     uint64_t exp2[32];
-    double inverse[64], log_of[64];
-    __device__ __forceinline__ void fill(int tid) {       // by at least 160 threads, in front of a barrier
-        if (tid < 32) exp2[tid] = exp2f_table[tid];
-        else if (tid < 96) inverse[tid - 32] = double(log_inverse[tid - 32]);
-        else if (tid < 160) log_of[tid - 96] = log_of_interval[tid - 96];
+    __device__ __forceinline__ void fill(int tid) {       // by at least 256 threads, in front of a barrier
+        if (tid >= 256) return;
+        const MishTablesInMemory from;
+        twice_inverse[tid] = from.twice_inverse(tid);
+        log_of[tid] = from.log_of(tid);
+        if (tid < 32) exp2[tid] = from.exp2(tid);
     }
 };
 struct MishTablesInLds {
     const MishTables *t;
     __device__ __forceinline__ uint64_t exp2(uint32_t i) const { return t->exp2[i]; }
-    __device__ __forceinline__ double inverse(int i) const { return t->inverse[i]; }
+    __device__ __forceinline__ double twice_inverse(int i) const { return t->twice_inverse[i]; }
     __device__ __forceinline__ double log_of(int i) const { return t->log_of[i]; }
 };
 
@@ -225,9 +228,11 @@ __device__ __forceinline__ void mish_fragment(float (&v)[16], const Table &table
     v16f t;
 #pragma unroll
     for (int r = 0; r < 16; ++r) t[r] = v[r];
+    MishAddends add;
+    asm volatile("" : "+v"(add.exp2), "+v"(add.log));
 #pragma clang loop unroll(disable)
     for (int r = 0; r < 16; r += 2) {
-        const float a = mish_value(t[r], table), b = mish_value(t[r + 1], table);
+        const float a = mish_value(t[r], table, add), b = mish_value(t[r + 1], table, add);
         t[r] = a;
         t[r + 1] = b;
     }
