@@ -1328,6 +1328,9 @@ int tsx_conv2d_i8_plan_info(const tsx_conv2d_geom *g, char *text, size_t text_by
     else if (pl.wsp.px) {      // for fp32 and staged outputs; the kernel named before writes the others
         const size_t used = std::strlen(text);
         std::snprintf(text + used, text_bytes - used, " pixel_stream=1");
+    } else if (pl.use_ws && pl.wsp.pt) {      // the same
+        const size_t used = std::strlen(text);
+        std::snprintf(text + used, text_bytes - used, " tile_stream=%dx%d", pl.wsp.pt_th, pl.wsp.pt_tw);
     }
     return 0;
 }

@@ -18,6 +18,7 @@
 // with nothing else done); 1024 to 256 14x14 9.0 -> 7.4; 256 to 512 56x56 at stride 2 19.8 -> 13.1, 1024 to 2048 14x14 17.9 -> 12.7.  8
 // images with the exact Mish: 64 to 64 304x304, int8 out, 57.5 -> 38.6 (vector instructions), fp32 and int8 126 -> 97; 512 to 512 19x19 8.3 -> 6.8.
 #include "conv2d_i8_px.hpp"
+#include "conv2d_i8_px_fragment.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -34,21 +35,11 @@ struct PxParams : EpiParams {
     int groups, per_xcd, blocks, slots;      // groups of WN fragments, those of an XCD; workgroups along cout; groups an XCD works on at a time
 };
 
-constexpr unsigned NOWHERE = 0xfffffff0u;      // beyond any buffer: loads 0, stores nothing
-
-// all of LDS written and read, no wait for global loads and stores
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // wavefronts per SIMD that the registers leave room for
 constexpr int px_waves(int ks, int wn, bool res, bool mishx) { return ks == 16 ? 2 : ks == 8 || (res && ks == 4) || (mishx && ks * wn == 8) ? 3 : 4; }
 
 // KS: K-steps of 64 channels.  WN: fragments of a group (4 / WN wavefronts along cout).  RES: a residual joins.  F32, Q: fp32
-// values, requantized ones leave.  MISHX: the activation is the exact Mish.  The loads and stores of a turn are the same in every
-// one, without branches: the compiler counts how many are in flight and waits for those it needs only.
+// values, requantized ones leave.  MISHX: the activation is the exact Mish.
 template <int KS, int WN, bool RES, bool F32, bool Q, bool MISHX>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(px_waves(KS, WN, RES, MISHX)))) void conv_i8_px_kernel(PxParams p) {
     constexpr int PITCH = KS * 64 + 16, CHUNKS = WN * 32 * KS * 4, FILL = (CHUNKS + 255) / 256, WM = 4 / WN;
@@ -93,9 +84,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(px_waves(KS
         });
     };
     // ---- position l % 32 of this wavefront's fragment: where its values go
-    struct Where { unsigned out, st; float scale; };
     auto where = [&](int group) __attribute__((always_inline)) {
-        Where w;
+        PxWhere w;
         const int pos = (group * WN + wave / WM) * 32 + lane % 32, at = min(pos, p.positions - 1);
         const int img = udiv(at, p.howo, p.howo_magic), rem = at - img * p.howo;
         w.out = pos < p.positions ? unsigned((img * p.cout + 4 * half) * p.howo + rem) * 4u : NOWHERE;
@@ -111,14 +101,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(px_waves(KS
     };
     const unsigned row0 = unsigned(m0) * unsigned(p.howo) * 4u, row = unsigned(p.howo) * 4u;
     float res[16];
-    auto load_res = [&](const Where &w) __attribute__((always_inline)) {
+    auto load_res = [&](const PxWhere &w) __attribute__((always_inline)) {
         if (RES) static_for<0, 16>([&](auto rc) {
             constexpr int r = decltype(rc)::value;
             res[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(resr, int(w.out), int(row0 + (8 * (r / 4) + r % 4) * row), 0));
         });
     };
     load_group(g);
-    Where now = where(g);
+    PxWhere now = where(g);
     load_res(now);
     v4i a[KS][2];
     static_for<0, KS>([&](auto kc) {
@@ -133,14 +123,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(px_waves(KS
         else if (p.bias) term = p.bias[m0 + lane - 32];
         terms[wave][lane] = term;
     }
-    const bool q_even = p.n_qscales == 1;
     store_group(0);
     lds_barrier();
     int buf = 0;
 
     auto turn = [&](auto more) __attribute__((always_inline)) {
         constexpr bool MORE = decltype(more)::value;
-        Where next = now;
+        PxWhere next = now;
         if (MORE) {
             load_group(g + p.slots);
             next = where(g + p.slots);
@@ -152,48 +141,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(px_waves(KS
             acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[k][0], *reinterpret_cast<const v4i *>(b + k * 64), acc, 0, 0, 0);
             acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[k][1], *reinterpret_cast<const v4i *>(b + k * 64 + 32), acc, 0, 0, 0);
         });
-        float v[16];
-        int at = 4 * half;
-        asm volatile("" : "+v"(at));     // (read in every turn, not kept in 32 registers)
-        const float *term = terms[wave] + at;
-        static_for<0, 4>([&](auto gc) {
-            constexpr int g4 = decltype(gc)::value;
-            const v4f dq = *reinterpret_cast<const v4f *>(term + 8 * g4), bias = *reinterpret_cast<const v4f *>(term + 32 + 8 * g4);
-            static_for<0, 4>([&](auto ic) { constexpr int i = decltype(ic)::value; v[4 * g4 + i] = __fadd_rn(__fmul_rn(float(acc[4 * g4 + i]), dq[i]), bias[i]); });
-        });
-        if (RES && !p.res_after) static_for<0, 16>([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], res[r]); });
-        uint32_t word[4];
-        if (MISHX) {
-            if constexpr (Q && !F32) {
-                if (RES && p.res_after) mish_words_for_rounding<true>(v, res, now.scale, q_even, word, tables);
-                else mish_words_for_rounding<false>(v, res, now.scale, q_even, word, tables);
-            } else {
-                mish_fragment(v, tables);
-            }
-        } else {
-            activate_results(v, p.act, p.slope);
-        }
-        if (RES && p.res_after && !(MISHX && Q && !F32)) static_for<0, 16>([&](auto rc) { constexpr int r = decltype(rc)::value; v[r] = __fadd_rn(v[r], res[r]); });
-        if (MORE) load_res(next);
-        if (F32) static_for<0, 16>([&](auto rc) {
-            constexpr int r = decltype(rc)::value;
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v[r]), outr, int(now.out), int(row0 + (8 * (r / 4) + r % 4) * row), 0);
-        });
-        if (Q) {
-            if (!(MISHX && !F32)) quantize_words(v, now.scale, q_even, word);
-            const auto s02 = __builtin_amdgcn_permlane32_swap(word[0], word[2], false, false);
-            const auto s13 = __builtin_amdgcn_permlane32_swap(word[1], word[3], false, false);
-            typedef unsigned v4u __attribute__((ext_vector_type(4)));
-            const v4u packed = {s02[0], s02[1], s13[0], s13[1]};
-            __builtin_amdgcn_raw_buffer_store_b128(packed, str, int(now.st), 0, 0);
-            if (p.st_up == 2) {
-                const unsigned right = unsigned(p.st_cp), down = unsigned(p.st_ws) * unsigned(p.st_cp);
-                const bool in = now.st != NOWHERE;
-                __builtin_amdgcn_raw_buffer_store_b128(packed, str, int(in ? now.st + right : NOWHERE), 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b128(packed, str, int(in ? now.st + down : NOWHERE), 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b128(packed, str, int(in ? now.st + down + right : NOWHERE), 0, 0);
-            }
-        }
+        px_finish<RES, F32, Q, MISHX>(p, acc, terms[wave], res, now, row0, row, outr, str, tables, [&] { if (MORE) load_res(next); });
         now = next;
         if (MORE) {
             store_group(buf ^ 1);

@@ -34,6 +34,7 @@
 #include "conv2d_i8_ws_kernel.hpp"
 #include "conv2d_i8_ks.hpp"
 #include "conv2d_i8_px.hpp"
+#include "conv2d_i8_pt.hpp"
 #include "tsx_plans.hpp"
 
 #include <algorithm>
@@ -79,12 +80,12 @@ static WsPlan make_ws_plan(const WsGeom &g_in);
 WsPlan ws_plan(const WsGeom &g) {
     struct Key {
         WsGeom g;
-        PlanSwitch flat, rs, ks, px;
+        PlanSwitch flat, rs, ks, px, pt;
     } key;
     std::memset(&key, 0, sizeof(key));
     key.g = g;
     if (!key.flat.read("TSX_CONV_I8_FLAT") || !key.rs.read("TSX_CONV_I8_RS") || !key.ks.read("TSX_CONV_I8_KS") ||
-        !key.px.read("TSX_CONV_I8_PX"))
+        !key.px.read("TSX_CONV_I8_PX") || !key.pt.read("TSX_CONV_I8_PT"))
         return make_ws_plan(g);
     return kept_plan<WsPlan>(key, [&] { return make_ws_plan(g); });
 }
@@ -212,6 +213,7 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
     rs_plan(g_in, &pl);   // ... and the weight-stationary one
     ks_plan(g_in, &pl);   // ... and the one that splits K
     px_plan(g_in, &pl);   // ... and the one for streams of pixels
+    pt_plan(g_in, &pl);   // ... and the one for streams of small tiles
     return pl;
 }
 
@@ -238,6 +240,7 @@ int ws_launch(const WsGeom &g, const WsPlan &plan, const int8_t *xs, const int8_
     }
     if (pl.ks) return ks_launch(g, pl, xs, packed, ep, stream);
     if (px_takes(g, pl, ep)) return px_launch(g, pl, xs, packed, ep, stream);
+    if (pt_takes(g, pl, ep)) return pt_launch(g, pl, xs, packed, ep, stream);
     if (rs_takes(pl, ep, int64_t(g.n) * g.cout * g.ho * g.wo)) return rs_launch(g, pl, xs, packed, ep, stream);
     if (fl_takes(g, pl, ep)) return fl_launch(g, pl, xs, packed, ep, stream);
     WsParams p{};

@@ -232,6 +232,11 @@ struct WsPlan {
     int rs_frags, rs_ptiles, rs_nr, rs_rowp, rs_wc, rs_lds;
     // pixel-stream kernel (conv2d_i8_px.hip) for the epilogues it writes; same packed weights
     bool px;
+    // small-tile kernel (conv2d_i8_pt.hip) for the epilogues it writes: output rows and columns of a tile, tiles along a row and
+    // in all, columns and pixels of a tile's window; same packed weights
+    bool pt;
+    int pt_th, pt_tw, pt_ctiles, pt_wc, pt_wpix;
+    int64_t pt_tiles;
     // K-split kernel (conv2d_i8_ks.hip): its tile, counted from 1, or 0; same packed weights
     int ks;
 };
