@@ -5,6 +5,7 @@
 #pragma once
 #include "igemm_i8.hpp"
 
+#include <algorithm>
 #include <atomic>
 
 namespace tsx {
@@ -76,6 +77,15 @@ namespace {
 // one half-step ahead (the other form), the small maps at the end of a network -- under one wavefront per SIMD,
 // nothing else to issue -- ran at one K-step per two LDS latencies.
 //
+// LOOK = 2: the workgroup has eight wavefronts, the second four for the second half of the channel blocks with windows of
+// their own; their sums (whole numbers: the same in any order) join through LDS.  What bounds a layer of at most one workgroup per CU is
+// each wavefront's way through K, 210 cycles a K-step for 64 of MFMAs, and a second wavefront per SIMD shortens
+// it by what the weights' way into registers leaves (65 of 130 B/ns per CU before).  us: 512 to 512 channels 3x3 7x7, 32 images, 13.9 ->
+// 13.0, at stride 2 from 14x14 14.4 -> 13.6, 2048 to 512 1x1 10.4 -> 9.5, 2048 to 256 3x3 14x14, 8 images, 36.4 -> 31.0.  Of 270 layers with
+// 256 channels and more 1.08 in the geometric mean, none slower by more than 0.7 %; with 128 channels 3x3, one block each, 0.93 to
+// 1.03, and with more workgroups than CUs slower (256 to 256 14x14, 448 of them, 11.3 -> 12.3).  Quarters: no more than halves below
+// 2048 channels (256 to 512 7x7 8.1 -> 9.4), 1.05 there.
+//
 // ws_waves: wavefronts per SIMD the registers have to leave room for.  The small tiles wait for memory more than they
 // multiply (64 to 64 channels 304x304 with the exact Mish, 8 images: 135 us at four wavefronts per SIMD, 118 at five); what
 // does not fit is left at what it needs.
@@ -98,19 +108,21 @@ __host__ __device__ inline bool ws_uniform(const WsParams &p) {
 // below, so that the other one, whose scalars are most of what the kernel holds, is not in it (spilled scalars 50 - 66 in the
 // general kernels of one and two fragments, none in these; YOLOv4's pass on 8 images, every
 // layer of whole fragments: 2645 us without them, 2533 with).
-template <int NT, int FM, bool EXTRA, bool STREAM, bool ROWM, int FILL, bool LOOK, int MISHX>
-__global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_waves(NT, FILL, LOOK, MISHX != 0)))) void conv_i8_ws_kernel(WsParams p_in) {
+template <int NT, int FM, bool EXTRA, bool STREAM, bool ROWM, int FILL, int LOOK, int MISHX>
+__global__ __launch_bounds__((LOOK > 1 ? LOOK : 1) * WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_waves(NT, FILL, LOOK != 0, MISHX != 0)))) void conv_i8_ws_kernel(WsParams p_in) {
     WsParams p = p_in;
     if (!EXTRA) {
         p.residual = nullptr;
         p.st_out = nullptr;
     }
     if (!ROWM) p.row_scale = nullptr;
-    extern __shared__ __attribute__((aligned(16))) int8_t lds[];   // 2 x wpix x PIX
+    extern __shared__ __attribute__((aligned(16))) int8_t lds_all[];   // 2 x wpix x PIX, for each half of K
     __shared__ MishTables mish_tables;                             // (exists in the instantiations that read it)
     // the wavefront's index as a scalar: what derives from it (first cout, tile bases, the choice of epilogue path)
     // then stays in scalar registers and branches uniformly
-    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int tid = threadIdx.x % WS_THREADS, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int part_k = LOOK > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / WS_THREADS) : 0;
+    if (LOOK > 1) p.ksteps /= LOOK, p.cblocks /= LOOK;
     // Each XCD takes a contiguous run of position tiles with all their channel blocks: what neighbouring tiles share -- the
     // cache line that a run of output positions ends in, halo rows, the window that all channel blocks read -- meets in one
     // L2, and so does what the layer before left there for these positions.
@@ -134,6 +146,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
     const int m0 = (block_m * p.wm + wave_m) * (32 * FM);         // first cout of this wavefront
     const int taps = p.kh * p.kw;
     const int win_bytes = p.wpix * p.pix;
+    int8_t *const lds = lds_all + part_k * (p.cblocks > 1 ? 2 : 1) * win_bytes;
 
     // ---- window fill bookkeeping: chunk q = tid + i*256 -> pixel q / chunks-per-pixel, 16-byte chunk q % ...
     // A uniform 64-bit base (the window's first staged row and column) plus one 32-bit byte offset per chunk: the
@@ -144,7 +157,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
     const int col_base = col0 * p.sw;
     const int row_last = int(min(int64_t(p.n) * p.hs - 1 - row_base, int64_t(1) << 20));   // last tile: rows no stored output uses
     const int col_last = p.ws - 1 - col_base;                                               // last column tile: likewise
-    const int8_t *xs_base = p.xs + (row_base * p.ws + col_base) * p.cp;
+    const int8_t *xs_base = p.xs + (row_base * p.ws + col_base) * p.cp + part_k * p.cblocks * p.stage_bytes;
     unsigned fill_off[FILL];
     int fill_dst[FILL];
     static_for<0, FILL>([&](auto ic) {
@@ -202,6 +215,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
     // ---- A ring: the wavefront's FM fragments (32 cout each) x 2 halves of K-step ks, 1 KiB each
     const int8_t *a_ptr = p.wp + (int64_t(m0 / 32) * 128 + lane) * 16;
     const int64_t a_kstride = int64_t(p.coutp / 32) * 128 * 16;
+    if (LOOK > 1) a_ptr += part_k * p.ksteps * a_kstride;
     v4i areg[RING][2 * FM];
     auto a_load = [&](auto slot, int ks) __attribute__((always_inline)) {
         constexpr int s = decltype(slot)::value;
@@ -246,7 +260,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
     });
     asm volatile("; epilogue operands touched" ::"v"(touch));
 
-    if (MISHX) mish_tables.fill(tid);
+    if (MISHX) mish_tables.fill(tid);      // (both halves of K the same)
     window_store(0);
     __syncthreads();
     int cb = 0, tap = 0, kc = 0, buf = 0;
@@ -264,7 +278,7 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
         });
     };
     int ks = 0;
-    if constexpr (LOOK) {
+    if constexpr (LOOK != 0) {
         // ---- K-loop with the B ring: slot u holds both halves of K-step (round start + u).  The read pointer runs
         // RING - 1 K-steps ahead of the MFMAs and is the one that swaps the windows when it enters a channel block.
         v4i bq[RING][2][NT];
@@ -316,6 +330,15 @@ __global__ __launch_bounds__(WS_THREADS) __attribute__((amdgpu_waves_per_eu(ws_w
         static_for<0, RING - 1>([&](auto uc) {
             if (decltype(uc)::value < left) k_step(uc, std::false_type{});
         });
+        if constexpr (LOOK > 1) {      // the other half's sums, through the windows
+            v16i *const theirs = reinterpret_cast<v16i *>(lds_all) + wave * 64 + lane;
+            __syncthreads();
+            if (part_k > 0) *theirs = acc[0][0];
+            __syncthreads();
+            if (part_k > 0) return;
+            const v16i other = *theirs;
+            static_for<0, 16>([&](auto rc) { acc[0][0][decltype(rc)::value] += other[decltype(rc)::value]; });
+        }
     } else {
         // B fragments are read one half-step ahead of the MFMAs that use them (one wavefront per
         // SIMD: nothing else hides the LDS latency).
@@ -599,15 +622,19 @@ int ws_launch_nt<TSX_WS_NT>(const WsParams &p, dim3 grid, size_t lds_bytes, hipS
     // one fragment per wavefront, a K of two rounds or more, and few enough workgroups that a SIMD holds one or
     // two wavefronts: the B ring (more registers: three workgroups per CU)
     const bool look = NT == 1 && small_fill && p.ksteps >= 2 * RING && int64_t(p.tiles) * p.blocks_m <= 1024;
+    // no more workgroups than CUs, and two channel blocks or more for each: K in halves
+    const int parts = look && int64_t(p.tiles) * p.blocks_m <= 256 && p.cblocks >= 4 && p.cblocks % 2 == 0 && 2 * lds_bytes <= 57344 ? 2 : 1;
 #define TSX_WS_LAUNCH(EXTRA, STREAM, ROWM, MISHX)                                                                      \
     do {                                                                                                               \
         constexpr int F = NT <= 2 ? SMALL_FILL : MAX_FILL;                                                             \
-        const int fill = NT == 1 && look ? 0 : NT <= 2 && small_fill ? 1 : 2;                                          \
-        const auto kernel = fill == 0 ? conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, NT == 1, MISHX>           \
-                            : fill == 1 ? conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, false, MISHX>           \
-                                        : conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, MAX_FILL, false, MISHX>;   \
-        if (MISHX && lds_bytes + sizeof(MishTables) > 65536) {      /* granted per kernel and device */                \
-            static std::atomic<bool> granted[3][64];                                                                   \
+        const int fill = NT == 1 && parts > 1 ? 3 : NT == 1 && look ? 0 : NT <= 2 && small_fill ? 1 : 2;                  \
+        const auto kernel = fill == 3 ? conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, NT == 1 ? 2 : 0, MISHX>   \
+                            : fill == 0 ? conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, NT == 1 ? 1 : 0, MISHX> \
+                            : fill == 1 ? conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, 0, MISHX>               \
+                                        : conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, MAX_FILL, 0, MISHX>;       \
+        const size_t dynamic = parts > 1 ? std::max<size_t>(2 * lds_bytes, 16384) : lds_bytes;                         \
+        if (MISHX && dynamic + sizeof(MishTables) > 65536) {      /* granted per kernel and device */                \
+            static std::atomic<bool> granted[4][64];                                                                   \
             int dev = 0;                                                                                               \
             TSX_HIP(hipGetDevice(&dev));                                                                               \
             if (dev >= 64 || !granted[fill][dev].load()) {                                                             \
@@ -616,7 +643,7 @@ int ws_launch_nt<TSX_WS_NT>(const WsParams &p, dim3 grid, size_t lds_bytes, hipS
                 if (dev < 64) granted[fill][dev].store(true);                                                          \
             }                                                                                                          \
         }                                                                                                              \
-        hipLaunchKernelGGL(kernel, grid, dim3(WS_THREADS), lds_bytes, stream, p);                                      \
+        hipLaunchKernelGGL(kernel, grid, dim3(parts * WS_THREADS), dynamic, stream, p);                                 \
     } while (0)
     // the exact Mish: instantiations (with every other epilogue term) that only its layers run
     if (p.act == TSX_ACT_MISH) {
