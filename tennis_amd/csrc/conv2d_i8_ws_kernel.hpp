@@ -622,8 +622,10 @@ int ws_launch_nt<TSX_WS_NT>(const WsParams &p, dim3 grid, size_t lds_bytes, hipS
     // one fragment per wavefront, a K of two rounds or more, and few enough workgroups that a SIMD holds one or
     // two wavefronts: the B ring (more registers: three workgroups per CU)
     const bool look = NT == 1 && small_fill && p.ksteps >= 2 * RING && int64_t(p.tiles) * p.blocks_m <= 1024;
-    // no more workgroups than CUs, and two channel blocks or more for each: K in halves
-    const int parts = look && int64_t(p.tiles) * p.blocks_m <= 256 && p.cblocks >= 4 && p.cblocks % 2 == 0 && 2 * lds_bytes <= 57344 ? 2 : 1;
+    // no more workgroups than CUs, and two channel blocks or more for each: K in halves.  Below 24 K-steps joining the sums takes what
+    // halves save: 1x1 layers on 512 to 1024 channels, times without halves : with them 0.97 to 1.025 (1.00 in the mean, 80 layers), on
+    // 1536 0.995 to 1.07 (1.02), on 2048 0.99 to 1.10 (1.05).
+    const int parts = look && int64_t(p.tiles) * p.blocks_m <= 256 && p.ksteps >= 24 && p.cblocks >= 4 && p.cblocks % 2 == 0 && 2 * lds_bytes <= 57344 ? 2 : 1;
 #define TSX_WS_LAUNCH(EXTRA, STREAM, ROWM, MISHX)                                                                      \
     do {                                                                                                               \
         constexpr int F = NT <= 2 ? SMALL_FILL : MAX_FILL;                                                             \

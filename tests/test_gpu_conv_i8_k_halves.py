@@ -1,5 +1,5 @@
-"""Window-stationary layers of one fragment per wavefront with K in halves (at most 256 workgroups, four channel blocks and more, an
-even number) and beside the rule's edges, against the oracle: taps, strides, windows of one and of several blocks, every epilogue."""
+"""Window-stationary layers of one fragment per wavefront with K in halves (at most 256 workgroups, 24 K-steps, four channel
+blocks and more, an even number) and beside the rule's edges, against the oracle: taps, strides, windows of one and of several blocks, every epilogue."""
 import numpy as np
 import pytest
 
@@ -15,7 +15,8 @@ LAYERS = [
     (8, 512, 14, 13, 64, 3, 2),
     (6, 640, 5, 5, 128, 5, 1),
     (30, 2048, 7, 7, 100, 1, 1),     # a window of four blocks
-    (9, 1100, 6, 7, 255, 1, 1),
+    (9, 1100, 6, 7, 255, 1, 1),      # 18 K-steps: not in halves
+    (9, 1536, 6, 7, 255, 1, 1),      # 24
 ]
 
 
