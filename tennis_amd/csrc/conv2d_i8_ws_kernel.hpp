@@ -116,11 +116,11 @@ __global__ __launch_bounds__((LOOK > 1 ? LOOK : 1) * WS_THREADS) __attribute__((
         p.st_out = nullptr;
     }
     if (!ROWM) p.row_scale = nullptr;
-    extern __shared__ __attribute__((aligned(16))) int8_t lds_all[];   // 2 x wpix x PIX, for each half of K
+    extern __shared__ __attribute__((aligned(16))) int8_t lds[];       // 2 x wpix x PIX, for each half of K
     __shared__ MishTables mish_tables;                             // (exists in the instantiations that read it)
     // the wavefront's index as a scalar: what derives from it (first cout, tile bases, the choice of epilogue path)
     // then stays in scalar registers and branches uniformly
-    const int tid = threadIdx.x % WS_THREADS, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int tid = LOOK > 1 ? threadIdx.x % WS_THREADS : threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int part_k = LOOK > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / WS_THREADS) : 0;
     if (LOOK > 1) p.ksteps /= LOOK, p.cblocks /= LOOK;
     // Each XCD takes a contiguous run of position tiles with all their channel blocks: what neighbouring tiles share -- the
@@ -146,7 +146,9 @@ __global__ __launch_bounds__((LOOK > 1 ? LOOK : 1) * WS_THREADS) __attribute__((
     const int m0 = (block_m * p.wm + wave_m) * (32 * FM);         // first cout of this wavefront
     const int taps = p.kh * p.kw;
     const int win_bytes = p.wpix * p.pix;
-    int8_t *const lds = lds_all + part_k * (p.cblocks > 1 ? 2 : 1) * win_bytes;
+    // this half's windows.  (As an offset, 0 in the other kernels: a pointer to them costs these a register per chunk of the window, 136
+    // for 127 with two fragments and three wavefronts per SIMD for four; 21 images 25 to 32 channels 233x42, int8 out, 23.7 us for 22.1.)
+    const int part_lds = LOOK > 1 ? part_k * (p.cblocks > 1 ? 2 : 1) * win_bytes : 0;
 
     // ---- window fill bookkeeping: chunk q = tid + i*256 -> pixel q / chunks-per-pixel, 16-byte chunk q % ...
     // A uniform 64-bit base (the window's first staged row and column) plus one 32-bit byte offset per chunk: the
@@ -157,7 +159,8 @@ __global__ __launch_bounds__((LOOK > 1 ? LOOK : 1) * WS_THREADS) __attribute__((
     const int col_base = col0 * p.sw;
     const int row_last = int(min(int64_t(p.n) * p.hs - 1 - row_base, int64_t(1) << 20));   // last tile: rows no stored output uses
     const int col_last = p.ws - 1 - col_base;                                               // last column tile: likewise
-    const int8_t *xs_base = p.xs + (row_base * p.ws + col_base) * p.cp + part_k * p.cblocks * p.stage_bytes;
+    const int8_t *xs_base = p.xs + (row_base * p.ws + col_base) * p.cp;
+    if (LOOK > 1) xs_base += part_k * p.cblocks * p.stage_bytes;
     unsigned fill_off[FILL];
     int fill_dst[FILL];
     static_for<0, FILL>([&](auto ic) {
@@ -194,7 +197,7 @@ __global__ __launch_bounds__((LOOK > 1 ? LOOK : 1) * WS_THREADS) __attribute__((
     auto window_store = [&](int buf) __attribute__((always_inline)) {
         static_for<0, FILL>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
-            if (i < n_fill) *reinterpret_cast<v4i *>(&lds[buf * win_bytes + fill_dst[i]]) = wreg[i];
+            if (i < n_fill) *reinterpret_cast<v4i *>(&lds[part_lds + buf * win_bytes + fill_dst[i]]) = wreg[i];
         });
     };
 
@@ -274,7 +277,7 @@ __global__ __launch_bounds__((LOOK > 1 ? LOOK : 1) * WS_THREADS) __attribute__((
     auto b_read = [&](v4i(&dst)[NT], int off) __attribute__((always_inline)) {
         static_for<0, NT>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
-            dst[j] = *reinterpret_cast<const v4i *>(&lds[b_base[j] + off]);
+            dst[j] = *reinterpret_cast<const v4i *>(&lds[b_base[j] + part_lds + off]);
         });
     };
     int ks = 0;
@@ -331,7 +334,7 @@ __global__ __launch_bounds__((LOOK > 1 ? LOOK : 1) * WS_THREADS) __attribute__((
             if (decltype(uc)::value < left) k_step(uc, std::false_type{});
         });
         if constexpr (LOOK > 1) {      // the other half's sums, through the windows
-            v16i *const theirs = reinterpret_cast<v16i *>(lds_all) + wave * 64 + lane;
+            v16i *const theirs = reinterpret_cast<v16i *>(lds) + wave * 64 + lane;
             __syncthreads();
             if (part_k > 0) *theirs = acc[0][0];
             __syncthreads();
