@@ -30,7 +30,7 @@ namespace {
 struct PxParams : EpiParams {
     const int8_t *xs;      // staged activations [n][hs][ws][cp]
     const int8_t *wp;      // packed weights [ks][coutp/32][2 halves][64 lanes][16]
-    int cout, wfrags, positions, wo, howo, hs, ws, cp, sh, sw, flat;
+    int cout, wfrags, positions, wo, howo, hs, ws, cp, sh, sw, flat, stream;
     unsigned howo_magic, wo_magic, blocks_magic, out_bytes, st_bytes;
     int groups, per_xcd, blocks, slots;      // groups of WN fragments, those of an XCD; workgroups along cout; groups an XCD works on at a time
 };
@@ -39,8 +39,8 @@ struct PxParams : EpiParams {
 constexpr int px_waves(int ks, int wn, bool res, bool mishx) { return ks == 16 ? 2 : ks == 8 || (res && ks == 4) || (mishx && ks * wn == 8) ? 3 : 4; }
 
 // KS: K-steps of 64 channels.  WN: fragments of a group (4 / WN wavefronts along cout).  RES: a residual joins.  F32, Q: fp32
-// values, requantized ones leave.  MISHX: the activation is the exact Mish.
-template <int KS, int WN, bool RES, bool F32, bool Q, bool MISHX>
+// values, requantized ones leave.  MISHX: the activation is the exact Mish.  STREAM: the fp32 values in streaming stores.
+template <int KS, int WN, bool RES, bool F32, bool Q, bool MISHX, bool STREAM = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(px_waves(KS, WN, RES, MISHX)))) void conv_i8_px_kernel(PxParams p) {
     constexpr int PITCH = KS * 64 + 16, CHUNKS = WN * 32 * KS * 4, FILL = (CHUNKS + 255) / 256, WM = 4 / WN;
     __shared__ MishTables mish_tables;
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(px_waves(KS
             acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[k][0], *reinterpret_cast<const v4i *>(b + k * 64), acc, 0, 0, 0);
             acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[k][1], *reinterpret_cast<const v4i *>(b + k * 64 + 32), acc, 0, 0, 0);
         });
-        px_finish<RES, F32, Q, MISHX>(p, acc, terms[wave], res, now, row0, row, outr, str, tables, [&] { if (MORE) load_res(next); });
+        px_finish<RES, F32, Q, MISHX, STREAM>(p, acc, terms[wave], res, now, row0, row, outr, str, tables, [&] { if (MORE) load_res(next); });
         now = next;
         if (MORE) {
             store_group(buf ^ 1);
@@ -158,6 +158,7 @@ int launch(const PxParams &p, unsigned grid, hipStream_t stream) {
     const bool f32 = p.out_f32, q = p.st_out;
     auto kernel = f32 ? (q ? conv_i8_px_kernel<KS, WN, false, true, true, MISHX> : conv_i8_px_kernel<KS, WN, false, true, false, MISHX>)
                       : conv_i8_px_kernel<KS, WN, false, false, true, MISHX>;
+    if (p.stream) kernel = conv_i8_px_kernel<KS, WN, false, true, false, MISHX, true>;
     if constexpr (KS <= 4)
         if (p.residual) kernel = f32 ? (q ? conv_i8_px_kernel<KS, WN, true, true, true, MISHX> : conv_i8_px_kernel<KS, WN, true, true, false, MISHX>)
                                      : conv_i8_px_kernel<KS, WN, true, false, true, MISHX>;
@@ -230,6 +231,11 @@ int px_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t 
     p.wo_magic = div_magic(p.wo, p.howo);
     p.out_bytes = unsigned(int64_t(p.positions) * g.cout * 4);
     p.st_bytes = unsigned(int64_t(g.n) * ep.st_hs * ep.st_ws * ep.st_cp);
+    // A large plain fp32 output leaves in streaming stores where planes are whole half cache lines: 137 layers with 64 to 1024 channels
+    // 0.93 of the time of stores that L2 keeps (us, window-stationary, L2, streaming: 7 images of 32x32 1024 to 2048 30.8, 35.0, 28.6;
+    // 26 of 200x200 128 to 64 71.6, 85.7, 65.2), and what the kernels behind it read stays in L2 (the ResNet-50 shape on 32 images: its
+    // first projection 22.3 -> 23.0, the join behind it 55.0 -> 44.8).  Planes of another length write parts of lines, which L2 joins.
+    p.stream = streams_fp32(ep, int64_t(p.positions) * g.cout) && p.howo % 16 == 0;
     switch (g.cblocks) {
         case 1: return launch_ks<1>(p, stream);
         case 2: return launch_ks<2>(p, stream);

@@ -6,6 +6,7 @@
 namespace tsx {
 
 constexpr unsigned NOWHERE = 0xfffffff0u;      // beyond any buffer: loads 0, stores nothing
+constexpr int STREAMING = 2;                   // a buffer instruction's non-temporal bit
 
 // all of LDS written and read, no wait for global loads and stores
 __device__ __forceinline__ void lds_barrier() {
@@ -18,11 +19,12 @@ __device__ __forceinline__ void lds_barrier() {
 // in the consumer's staged one (or NOWHERE), and the consumer's scale
 struct PxWhere { unsigned out, st; float scale; };
 
-// RES: a residual joins.  F32, Q: fp32 values, requantized ones leave.  MISHX: the activation is the exact Mish.  terms: the 32 channels'
+// RES: a residual joins.  F32, Q: fp32 values, requantized ones leave.  MISHX: the activation is the exact Mish.  STREAM: fp32 values in
+// streaming stores.  terms: the 32 channels'
 // scales and biases in LDS; row0, row: byte offset of the first channel in an fp32 image, and of one to the next.  next_residual() is called
 // when res is free.  The loads and stores are the same in every call, without branches: the compiler counts how many are in flight
 // and waits for those it needs only.
-template <bool RES, bool F32, bool Q, bool MISHX, class Next>
+template <bool RES, bool F32, bool Q, bool MISHX, bool STREAM = false, class Next>
 __device__ __forceinline__ void px_finish(const EpiParams &p, const v16i &acc, const float *terms, const float (&res)[16], const PxWhere &to, unsigned row0, unsigned row,
                                           __amdgpu_buffer_rsrc_t outr, __amdgpu_buffer_rsrc_t str, const MishTablesInLds &tables, Next &&next_residual) {
     float v[16];
@@ -50,7 +52,7 @@ __device__ __forceinline__ void px_finish(const EpiParams &p, const v16i &acc, c
     next_residual();
     if (F32) static_for<0, 16>([&](auto rc) {
         constexpr int r = decltype(rc)::value;
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v[r]), outr, int(to.out), int(row0 + (8 * (r / 4) + r % 4) * row), 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v[r]), outr, int(to.out), int(row0 + (8 * (r / 4) + r % 4) * row), STREAM ? STREAMING : 0);
     });
     if (Q) {
         if (!(MISHX && !F32)) quantize_words(v, to.scale, p.n_qscales == 1, word);

@@ -283,8 +283,7 @@ int ws_launch(const WsGeom &g, const WsPlan &plan, const int8_t *xs, const int8_
         p.tap_row = 0;
         p.tap_col = 64;
     }
-    // an output of L2 size or more that no fused consumer reads: stream it
-    p.stream_out = (!ep.residual && !ep.st_out && ep.out_f32 && int64_t(g.n) * g.cout * g.ho * g.wo * 4 >= (int64_t(16) << 20)) ? 1 : 0;
+    p.stream_out = streams_fp32(ep, int64_t(g.n) * g.cout * g.ho * g.wo) ? 1 : 0;
     p.rowmajor = g.gemm ? 1 : 0;
     if (g.gemm) p.stream_out = 0;
     p.wc_magic = div_magic(p.wc, MAX_WP);

@@ -28,6 +28,11 @@ struct EpiParams {
     int res_after;       // residual joins behind the activation instead of in front of it
 };
 
+// a plain fp32 output of L2 size or more, of `count` values, that no fused consumer reads: not to be kept there
+inline bool streams_fp32(const EpiParams &ep, int64_t count) {
+    return ep.out_f32 && !ep.residual && !ep.st_out && count * 4 >= (int64_t(16) << 20);
+}
+
 // Division of a non-negative n by a uniform divisor d as one multiply-high: magic = ceil(2^32 / d) gives
 // floor(n / d) = mulhi(n, magic) whenever n * d <= 2^32.  0 = no magic number (d = 1, or n_max too large): the
 // kernel then takes n itself, or divides (some thirty instructions: the tiles of 1x1 layers, one pixel wide, spent a third

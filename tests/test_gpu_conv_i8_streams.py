@@ -1,0 +1,47 @@
+"""What the streaming int8 kernels choose for large outputs, at the sizes where they choose it, bit for bit against the kernels they take
+layers from and against the oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def device(shape, seed, values=None):
+    """Values on the device, without a host copy of large tensors: int8 of the whole range, or standard normal floats."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randint(-128, 128, shape, device="cuda", dtype=torch.int8, generator=g) if values is None else torch.randn(shape, device="cuda", generator=g) * values
+
+
+def layer(n, c, h, w, cout, k=1, stride=1, seed=3):
+    """The layer, its scales and biases, and its staged input."""
+    from tennis_amd import capi
+    conv = capi.Conv2dI8(device((cout, c, k, k), seed), (k // 2,) * 4, (stride, stride))
+    staged = capi.StagedInput(conv, (n, c, h, w))
+    conv.stage(device((n, c, h, w), seed + 1), staged)
+    return conv, device((cout,), seed + 2, 1e-5).abs() * (30 / k) / c ** 0.5 + 1e-6, device((cout,), seed + 3, 1.0), staged
+
+
+def streams(monkeypatch, conv, shape, name, on):
+    from tennis_amd import capi
+    monkeypatch.setenv("TSX_CONV_I8_" + {"pixel_stream": "PX", "tile_stream": "PT"}[name], "1" if on else "0")
+    info = capi.conv2d_i8_plan_info(conv._plan(shape)[0])
+    assert (name in info) == on and info["kernel"] != "k_split", info
+
+
+@pytest.mark.parametrize("c", [64, 100, 256, 512, 1000])
+@pytest.mark.parametrize("cout, h, w", [(32, 256, 132), (64, 256, 68), (128, 128, 64), (256, 56, 76), (384, 49, 64)])
+def test_streaming_stores(monkeypatch, c, cout, h, w):
+    """16 MiB and more of fp32 values, planes of whole half cache lines, the last group of pixels full or not."""
+    if cout % (32 if c <= 128 else 64 if c <= 256 else 128):
+        pytest.skip("no pixel stream for these channels")
+    import torch
+    n = 4
+    conv, dq, bias, staged = layer(n, c, h, w, cout)
+    assert n * cout * h * w * 4 >= 16 << 20 and h * w % 16 == 0
+    for act in ("none", "leaky_relu", "mish"):
+        got = []
+        for on in (False, True):
+            streams(monkeypatch, conv, (n, c, h, w), "pixel_stream", on)
+            got.append(conv.run_staged(staged, dq, bias, act, 0.1)[0])
+        assert torch.equal(got[0].view(torch.int32), got[1].view(torch.int32)), act

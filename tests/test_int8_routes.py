@@ -1,0 +1,111 @@
+"""The kernels that int8 calls launch, by name and grid: a plan names the kernels a layer may take, a call's epilogue decides among them.
+The library is loaded in a process where the runtime's launch calls are recorded and not carried out: no device and no
+memory are needed."""
+import json
+import os
+import re
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+RECORDER = r"""
+#include <stdint.h>
+#include <stdio.h>
+#include <string.h>
+typedef struct { uint32_t x, y, z; } dims;
+static dims grid, block;
+static size_t dynamic;
+static struct { const void *host; char name[240]; } kernels[8192];
+static int count;
+char launched[4096];
+void **__hipRegisterFatBinary(const void *data) { static void *handle; return &handle; }
+void __hipUnregisterFatBinary(void **modules) {}
+void __hipRegisterVar() {}
+void __hipRegisterManagedVar() {}
+void __hipRegisterFunction(void **modules, const void *host, char *device_name, const char *name, unsigned limit, void *a, void *b, void *c, void *d, int *e) {
+    if (count < 8192) {
+        kernels[count].host = host;
+        strncpy(kernels[count++].name, name, 239);
+    }
+}
+unsigned __hipPushCallConfiguration(dims g, dims b, size_t shared, void *stream) { grid = g; block = b; dynamic = shared; return 0; }
+unsigned __hipPopCallConfiguration(dims *g, dims *b, size_t *shared, void **stream) { *g = grid; *b = block; *shared = dynamic; *stream = 0; return 0; }
+int hipLaunchKernel(const void *f, dims g, dims b, void **args, size_t shared, void *stream) {
+    for (int i = 0; i < count; ++i)
+        if (kernels[i].host == f) sprintf(launched + strlen(launched), "%s %u %u;", kernels[i].name, g.x * g.y, b.x);
+    return 0;
+}
+int hipGetLastError(void) { return 0; }
+int hipGetDevice(int *device) { *device = 0; return 0; }
+int hipFuncSetAttribute(const void *f, int what, int value) { return 0; }
+"""
+
+CALLS = r"""
+import ctypes, json, sys
+recorder = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+L = ctypes.CDLL(sys.argv[2])
+sys.path.insert(0, sys.argv[4])
+from tennis_amd.capi import ConvGeom, Epilogue, SIGNATURES, _ACT
+L.tsx_conv2d_i8_staged.argtypes = SIGNATURES["tsx_conv2d_i8_staged"][1]
+L.tsx_conv2d_i8_plan_info.argtypes = SIGNATURES["tsx_conv2d_i8_plan_info"][1]
+L.tsx_last_error.restype = ctypes.c_char_p
+launched = (ctypes.c_char * 4096).in_dll(recorder, "launched")
+at = 1 << 20                      # an address that nothing reads
+out = []
+for n, c, h, w, cout, k, s, act, outputs in json.loads(sys.argv[3]):
+    kh, kw = k if isinstance(k, list) else (k, k)
+    geom = ConvGeom(n, c, h, w, cout, kh, kw, kh // 2, kh // 2, kw // 2, kw // 2, s, s, 1, 1)
+    ho, wo = (h + 2 * (kh // 2) - kh) // s + 1, (w + 2 * (kw // 2) - kw) // s + 1
+    ep = Epilogue(dq_dev=at, bias_dev=at, act=_ACT[act], slope=0.1)
+    if "i8" in outputs or "staged" in outputs:
+        ep.q_scales_dev, ep.n_qscales = at, n
+    if "staged" in outputs:
+        ep.staged_out_dev, ep.staged_hs, ep.staged_ws, ep.staged_cp = at, ho, wo, (cout + 63) // 64 * 64
+    if "join" in outputs:
+        ep.residual_dev = at
+    launched.value = b""
+    rc = L.tsx_conv2d_i8_staged(ctypes.byref(geom), at, at, ctypes.byref(ep), at if "f32" in outputs else None, at if "i8" in outputs else None, None, None)
+    info = ctypes.create_string_buffer(512)
+    assert L.tsx_conv2d_i8_plan_info(ctypes.byref(geom), info, 512) == 0
+    out.append([rc, launched.value.decode(), info.value.decode()] if rc == 0 else [rc, L.tsx_last_error().decode(), ""])
+print(json.dumps(out))
+"""
+
+
+@pytest.fixture(scope="module")
+def route(tmp_path_factory):
+    """Calls (n, c, h, w, cout, k, stride, activation, outputs) -> for each the kernel's name with its template arguments, its
+    workgroups, the plan's text."""
+    from tennis_amd.build import LIB_PATH
+    where = tmp_path_factory.mktemp("recorder")
+    source, so = where / "recorder.c", where / "librecorder.so"
+    source.write_text(RECORDER)
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(so), str(source)])
+    env = {k: v for k, v in os.environ.items() if not k.startswith("TSX_")}
+
+    def routes(calls):
+        run = subprocess.run([sys.executable, "-c", CALLS, str(so), LIB_PATH, json.dumps(calls), ROOT], capture_output=True, text=True, cwd=ROOT, env=env)
+        assert run.returncode == 0, run.stderr
+        out = []
+        for call, (rc, launched, info) in zip(calls, json.loads(run.stdout)):
+            assert rc == 0 and launched.count(";") == 1, (call, rc, launched)
+            name, workgroups, threads = launched.rstrip(";").split(" ")
+            name = subprocess.run(["c++filt", name], capture_output=True, text=True, check=True).stdout
+            name = re.search(r"(\w+)<([^<>]*)>", name)
+            out.append((name.group(1) + "<" + name.group(2) + ">", int(workgroups), dict(word.split("=", 1) for word in info.split())))
+        return out
+    return routes
+
+
+def test_large_plain_fp32_outputs_of_whole_half_lines_are_streamed(route):
+    calls = [([32, 256, 56, 56, 512, 1, 2, "none", "f32"], True), ([7, 1024, 32, 32, 2048, 1, 1, "relu", "f32"], True), ([8, 64, 304, 304, 64, 1, 1, "mish", "f32"], True),
+             ([4, 64, 128, 128, 64, 1, 1, "none", "f32"], True),                                    # 16 MiB
+             ([4, 64, 124, 128, 64, 1, 1, "none", "f32"], False),                                   # less
+             ([4, 64, 130, 130, 64, 1, 1, "none", "f32"], False),                                   # planes of 16900 values
+             ([32, 64, 56, 56, 256, 1, 1, "relu", "f32 join"], False), ([32, 64, 56, 56, 256, 1, 1, "relu", "f32 staged"], False)]
+    for (call, streams), (kernel, _, _) in zip(calls, route([call for call, _ in calls])):
+        arguments = kernel[:-1].split("<")[1].split(", ")
+        assert kernel.startswith("conv_i8_px_kernel<") and arguments[-1] == ("true" if streams else "false"), (call, kernel)
