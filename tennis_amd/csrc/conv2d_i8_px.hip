@@ -167,6 +167,31 @@ int launch(const PxParams &p, unsigned grid, hipStream_t stream) {
     return 0;
 }
 
+// One turn where an XCD's CUs hold all of its groups, else two or three: more leave the last ones fewer wavefronts to hide their
+// memory behind (us for 1, 2, 3, 4, 6 turns: 64 to 256 channels 56x56 with a join 45.6, 46.2, 44.3, 45.9, 46.9; 64 to 64 56x56 7.1, 7.3, 7.0,
+// 7.8, 8.8; 64 to 64 304x304 with the exact Mish 46.6, 39.7, 38.7, 39.3, 39.7).  waves: those per SIMD.
+int turns_of(int per_xcd, int blocks, int waves) {
+    return int(std::min<int64_t>(3, ceil_div(int64_t(per_xcd) * blocks, 32 * waves)));
+}
+// Weights of 1024 channels leave room for two workgroups per CU: a third on some CUs is a whole turn of nothing beside it, and three
+// turns of it were up to a third longer than the best number (us for 1 to 6 turns, 8 images of 40x58, to 384 channels, both outputs, exact Mish, with three by the rule
+// above: 35.9, 38.5, 42.4, 35.6, 40.1, 40.6, window-stationary 37.4; 4 of 74x74, to 1024, fp32: 62.8, 58.7, 56.4, 53.4, 53.8, 51.0).  The
+// rounds of the busiest CU decide: two that share it take 1.3 of the time of one alone, and before its first turn a workgroup takes
+// as long as 1.3 turns, 0.3 of the longer ones with the exact Mish.  131 layers: 0.944 of the time of the rule above and none
+// longer than on the window-stationary kernel, where with that rule some took up to 1.13 of its time.
+int turns_of_two_per_cu(int per_xcd, int blocks, bool mishx) {
+    int best = 1;
+    double shortest = 0;
+    for (int turns = 1; turns <= 6; ++turns) {
+        const int64_t per_cu = ceil_div(ceil_div(per_xcd, turns) * blocks, 32);
+        const double time = (turns + (mishx ? 0.3 : 1.3)) * (1.3 * double(per_cu / 2) + double(per_cu % 2));
+        if (turns > 1 && time >= shortest) continue;
+        shortest = time;
+        best = turns;
+    }
+    return best;
+}
+
 template <int KS>
 int launch_ks(PxParams &p, hipStream_t stream) {
     const int mfrags = p.cout / 32, wm = mfrags % 4 == 0 ? 4 : mfrags % 2 == 0 ? 2 : 1, wn = 4 / wm;
@@ -174,14 +199,10 @@ int launch_ks(PxParams &p, hipStream_t stream) {
     p.blocks_magic = div_magic(p.blocks, int64_t(1) << 24);
     p.groups = int(ceil_div(p.positions, 32 * wn));
     p.per_xcd = int(ceil_div(p.groups, 8));
-    // One turn where an XCD's CUs hold all of its groups, else two or three: more leave the last ones fewer wavefronts to hide their
-    // memory behind (us for 1, 2, 3, 4, 6 turns: 64 to 256 channels 56x56 with a join 45.6, 46.2, 44.3, 45.9, 46.9; 64 to 64 56x56 7.1, 7.3, 7.0,
-    // 7.8, 8.8; 64 to 64 304x304 with the exact Mish 46.6, 39.7, 38.7, 39.3, 39.7).
-    const int64_t resident = 32 * px_waves(KS, wn, p.residual, p.act == TSX_ACT_MISH);
-    const int turns = int(std::min<int64_t>(3, ceil_div(int64_t(p.per_xcd) * p.blocks, resident)));
+    const bool mish = p.act == TSX_ACT_MISH;
+    const int turns = KS == 16 ? turns_of_two_per_cu(p.per_xcd, p.blocks, mish) : turns_of(p.per_xcd, p.blocks, px_waves(KS, wn, p.residual, mish));
     p.slots = int(ceil_div(p.per_xcd, turns));
     const unsigned grid = unsigned(8 * p.blocks * p.slots);
-    const bool mish = p.act == TSX_ACT_MISH;
     if (wn == 1) return mish ? launch<KS, 1, true>(p, grid, stream) : launch<KS, 1, false>(p, grid, stream);
     if constexpr (KS <= 4) if (wn == 2) return mish ? launch<KS, 2, true>(p, grid, stream) : launch<KS, 2, false>(p, grid, stream);
     if constexpr (KS <= 2) return mish ? launch<KS, 4, true>(p, grid, stream) : launch<KS, 4, false>(p, grid, stream);

@@ -45,3 +45,28 @@ def test_streaming_stores(monkeypatch, c, cout, h, w):
             streams(monkeypatch, conv, (n, c, h, w), "pixel_stream", on)
             got.append(conv.run_staged(staged, dq, bias, act, 0.1)[0])
         assert torch.equal(got[0].view(torch.int32), got[1].view(torch.int32)), act
+
+
+def same_outputs(monkeypatch, conv, dq, bias, staged, shape, out_shape, act, f32, requantized, residual=None):
+    """Whole output buffers of the layer with and without the pixel stream."""
+    import torch
+    from tennis_amd import capi
+    second = capi.Conv2dI8(torch.zeros((32, out_shape[1], 1, 1), dtype=torch.int8, device="cuda"))
+    scales = device((shape[0],), 17, 1.0).abs() * 10 + 20
+    got = []
+    for on in (False, True):
+        streams(monkeypatch, conv, shape, "pixel_stream", on)
+        out = capi.StagedInput(second, out_shape) if requantized else None
+        y = conv.run_staged(staged, dq, bias, act, 0.1, want_f32=f32, q_scales=scales if requantized else None, staged_out=out, residual=residual)[0]
+        got.append((y.view(torch.int32) if f32 else None, out.buf if requantized else None))
+    for a, b in zip(*got):
+        assert a is None or torch.equal(a, b), act
+
+
+@pytest.mark.parametrize("n, h, w, cout", [(20, 8, 8, 512), (8, 40, 58, 384), (4, 74, 74, 1024), (3, 67, 59, 128)])     # one turn; four and six, the last ones not full
+def test_turns_of_1024_channels(monkeypatch, n, h, w, cout):
+    monkeypatch.setenv("TSX_CONV_I8_KS", "0")
+    c = 1000
+    conv, dq, bias, staged = layer(n, c, h, w, cout)
+    for act, f32, requantized in (("relu", True, False), ("none", False, True), ("mish", True, True)):
+        same_outputs(monkeypatch, conv, dq, bias, staged, (n, c, h, w), (n, cout, h, w), act, f32, requantized)

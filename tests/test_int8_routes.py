@@ -109,3 +109,11 @@ def test_large_plain_fp32_outputs_of_whole_half_lines_are_streamed(route):
     for (call, streams), (kernel, _, _) in zip(calls, route([call for call, _ in calls])):
         arguments = kernel[:-1].split("<")[1].split(", ")
         assert kernel.startswith("conv_i8_px_kernel<") and arguments[-1] == ("true" if streams else "false"), (call, kernel)
+
+
+def test_pixel_streams_of_1024_channels_fill_rounds_of_two_workgroups_per_cu(route):
+    """Turns by what the busiest CU of an XCD takes: its groups of 32 pixels over 32 CUs, two at a time."""
+    calls = [([8, 1024, 40, 58, 384, 1, 1, "mish", "f32 staged"], 73, 3, 4), ([2, 1024, 182, 21, 1024, 1, 1, "mish", "f32 staged"], 30, 8, 4),
+             ([20, 1024, 14, 14, 256, 1, 1, "relu", "staged"], 16, 2, 1), ([4, 1024, 74, 74, 1024, 1, 1, "relu", "f32"], 86, 8, 6)]
+    for (call, per_xcd, blocks, turns), (kernel, workgroups, _) in zip(calls, route([c[0] for c in calls])):
+        assert kernel.startswith("conv_i8_px_kernel<16, 1, ") and workgroups == 8 * blocks * -(-per_xcd // turns), (call, kernel, workgroups)
