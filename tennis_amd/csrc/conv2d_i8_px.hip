@@ -31,8 +31,10 @@ struct PxParams : EpiParams {
     const int8_t *xs;      // staged activations [n][hs][ws][cp]
     const int8_t *wp;      // packed weights [ks][coutp/32][2 halves][64 lanes][16]
     int cout, wfrags, positions, wo, howo, hs, ws, cp, sh, sw, flat, stream;
-    unsigned howo_magic, wo_magic, blocks_magic, out_bytes, st_bytes;
+    unsigned howo_magic, wo_magic, out_bytes, st_bytes;
     int groups, per_xcd, blocks, slots;      // groups of WN fragments, those of an XCD; workgroups along cout; groups an XCD works on at a time
+    int panel, span;                         // channel blocks that are taken for all of an XCD's slots before the next ones; their workgroups
+    unsigned panel_magic, span_magic;
 };
 
 // wavefronts per SIMD that the registers leave room for
@@ -50,8 +52,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(px_waves(KS
     if (MISHX) mish_tables.fill(tid);                                 // (in front of the first barrier)
     const MishTablesInLds tables{&mish_tables};
     // Each XCD takes a contiguous run of groups with all their channels: cache lines that two groups share meet in one L2.
-    const int xcd = int(blockIdx.x & 7), j = int(blockIdx.x >> 3), slot = udiv(j, p.blocks, p.blocks_magic);
-    const int m0 = ((j - slot * p.blocks) * WM + wave % WM) * 32;
+    const int xcd = int(blockIdx.x & 7), j = int(blockIdx.x >> 3), past = udiv(j, p.span, p.span_magic), at_span = j - past * p.span;
+    const int slot = udiv(at_span, p.panel, p.panel_magic), m0 = ((past * p.panel + at_span - slot * p.panel) * WM + wave % WM) * 32;
     int g = xcd * p.per_xcd + slot;
     const int g_end = min((xcd + 1) * p.per_xcd, p.groups);
     if (g >= g_end) return;
@@ -196,12 +198,22 @@ template <int KS>
 int launch_ks(PxParams &p, hipStream_t stream) {
     const int mfrags = p.cout / 32, wm = mfrags % 4 == 0 ? 4 : mfrags % 2 == 0 ? 2 : 1, wn = 4 / wm;
     p.blocks = mfrags / wm;
-    p.blocks_magic = div_magic(p.blocks, int64_t(1) << 24);
     p.groups = int(ceil_div(p.positions, 32 * wn));
     p.per_xcd = int(ceil_div(p.groups, 8));
     const bool mish = p.act == TSX_ACT_MISH;
     const int turns = KS == 16 ? turns_of_two_per_cu(p.per_xcd, p.blocks, mish) : turns_of(p.per_xcd, p.blocks, px_waves(KS, wn, p.residual, mish));
     p.slots = int(ceil_div(p.per_xcd, turns));
+    // The workgroups of a group of pixels come one behind the other: they read the same pixels.  Where planes end inside a cache line, the two
+    // groups that write a line (and read the residual's) have to meet in L2, and with 16 blocks of channels and more in between the second came
+    // when the line had left.  Large outputs of such planes take two blocks at a time (us, window-stationary, all blocks, two: joins of 64 to 2048
+    // channels 10 images of 54x54 131.2, 154.5, 118.3, 256 to 4096 32 of 19x19 155, 168, 117; 80 such layers 1.00, 1.18 at most, of the
+    // window-stationary kernel's time with all and 0.83 with two).  Smaller outputs stay in L2 (16 blocks, 16 to 32 MiB, 1.00 of the time, up to 1.15),
+    // and the exact Mish leaves the second group less behind (32 to 64 MiB 1.01).
+    const bool lines_leave = p.out_f32 && p.howo % 32 != 0 && p.blocks >= 16 && p.out_bytes >= (mish ? 64u << 20 : 32u << 20);
+    p.panel = !lines_leave ? p.blocks : p.blocks % 2 == 0 ? 2 : 1;
+    p.span = p.panel * p.slots;
+    p.panel_magic = div_magic(p.panel, p.span);
+    p.span_magic = div_magic(p.span, int64_t(p.blocks) * p.slots);
     const unsigned grid = unsigned(8 * p.blocks * p.slots);
     if (wn == 1) return mish ? launch<KS, 1, true>(p, grid, stream) : launch<KS, 1, false>(p, grid, stream);
     if constexpr (KS <= 4) if (wn == 2) return mish ? launch<KS, 2, true>(p, grid, stream) : launch<KS, 2, false>(p, grid, stream);

@@ -70,3 +70,12 @@ def test_turns_of_1024_channels(monkeypatch, n, h, w, cout):
     conv, dq, bias, staged = layer(n, c, h, w, cout)
     for act, f32, requantized in (("relu", True, False), ("none", False, True), ("mish", True, True)):
         same_outputs(monkeypatch, conv, dq, bias, staged, (n, c, h, w), (n, cout, h, w), act, f32, requantized)
+
+
+@pytest.mark.parametrize("n, c, h, w, cout", [(12, 64, 41, 43, 2048), (9, 256, 33, 35, 2176), (6, 100, 57, 57, 4096)])
+def test_large_outputs_whose_planes_share_lines(monkeypatch, n, c, h, w, cout):
+    """Two blocks of channels at a time, or one where their number is odd."""
+    conv, dq, bias, staged = layer(n, c, h, w, cout)
+    res = device((n, cout, h, w), 23, 1.0)
+    for act, f32, requantized, residual in (("relu", True, False, res), ("leaky_relu", True, True, res), ("none", True, False, None), ("mish", True, True, None)):
+        same_outputs(monkeypatch, conv, dq, bias, staged, (n, c, h, w), (n, cout, h, w), act, f32, requantized, residual)
