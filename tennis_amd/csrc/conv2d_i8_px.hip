@@ -31,10 +31,8 @@ struct PxParams : EpiParams {
     const int8_t *xs;      // staged activations [n][hs][ws][cp]
     const int8_t *wp;      // packed weights [ks][coutp/32][2 halves][64 lanes][16]
     int cout, wfrags, positions, wo, howo, hs, ws, cp, sh, sw, flat, stream;
-    unsigned howo_magic, wo_magic, out_bytes, st_bytes;
+    unsigned howo_magic, wo_magic, blocks_magic, out_bytes, st_bytes;
     int groups, per_xcd, blocks, slots;      // groups of WN fragments, those of an XCD; workgroups along cout; groups an XCD works on at a time
-    int panel, span;                         // channel blocks that are taken for all of an XCD's slots before the next ones; their workgroups
-    unsigned panel_magic, span_magic;
 };
 
 // wavefronts per SIMD that the registers leave room for
@@ -42,7 +40,8 @@ constexpr int px_waves(int ks, int wn, bool res, bool mishx) { return ks == 16 ?
 
 // KS: K-steps of 64 channels.  WN: fragments of a group (4 / WN wavefronts along cout).  RES: a residual joins.  F32, Q: fp32
 // values, requantized ones leave.  MISHX: the activation is the exact Mish.  STREAM: the fp32 values in streaming stores.
-template <int KS, int WN, bool RES, bool F32, bool Q, bool MISHX, bool STREAM = false>
+// PANELS: workgroups by grid.y first (p.blocks of them along cout).
+template <int KS, int WN, bool RES, bool F32, bool Q, bool MISHX, bool STREAM = false, bool PANELS = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(px_waves(KS, WN, RES, MISHX)))) void conv_i8_px_kernel(PxParams p) {
     constexpr int PITCH = KS * 64 + 16, CHUNKS = WN * 32 * KS * 4, FILL = (CHUNKS + 255) / 256, WM = 4 / WN;
     __shared__ MishTables mish_tables;
@@ -52,8 +51,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(px_waves(KS
     if (MISHX) mish_tables.fill(tid);                                 // (in front of the first barrier)
     const MishTablesInLds tables{&mish_tables};
     // Each XCD takes a contiguous run of groups with all their channels: cache lines that two groups share meet in one L2.
-    const int xcd = int(blockIdx.x & 7), j = int(blockIdx.x >> 3), past = udiv(j, p.span, p.span_magic), at_span = j - past * p.span;
-    const int slot = udiv(at_span, p.panel, p.panel_magic), m0 = ((past * p.panel + at_span - slot * p.panel) * WM + wave % WM) * 32;
+    const int xcd = int(blockIdx.x & 7), j = int(blockIdx.x >> 3), slot = udiv(j, p.blocks, p.blocks_magic);
+    const int m0 = (((PANELS ? int(blockIdx.y) * p.blocks : 0) + j - slot * p.blocks) * WM + wave % WM) * 32;
     int g = xcd * p.per_xcd + slot;
     const int g_end = min((xcd + 1) * p.per_xcd, p.groups);
     if (g >= g_end) return;
@@ -156,7 +155,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(px_waves(KS
 }
 
 template <int KS, int WN, bool MISHX>
-int launch(const PxParams &p, unsigned grid, hipStream_t stream) {
+int launch(const PxParams &p, dim3 grid, hipStream_t stream) {
     const bool f32 = p.out_f32, q = p.st_out;
     auto kernel = f32 ? (q ? conv_i8_px_kernel<KS, WN, false, true, true, MISHX> : conv_i8_px_kernel<KS, WN, false, true, false, MISHX>)
                       : conv_i8_px_kernel<KS, WN, false, false, true, MISHX>;
@@ -164,7 +163,12 @@ int launch(const PxParams &p, unsigned grid, hipStream_t stream) {
     if constexpr (KS <= 4)
         if (p.residual) kernel = f32 ? (q ? conv_i8_px_kernel<KS, WN, true, true, true, MISHX> : conv_i8_px_kernel<KS, WN, true, true, false, MISHX>)
                                      : conv_i8_px_kernel<KS, WN, true, false, true, MISHX>;
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, p);
+    if constexpr (WN == 1) if (grid.y > 1) {
+        kernel = q ? conv_i8_px_kernel<KS, 1, false, true, true, MISHX, false, true> : conv_i8_px_kernel<KS, 1, false, true, false, MISHX, false, true>;
+        if constexpr (KS <= 4)
+            if (p.residual) kernel = q ? conv_i8_px_kernel<KS, 1, true, true, true, MISHX, false, true> : conv_i8_px_kernel<KS, 1, true, true, false, MISHX, false, true>;
+    }
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, p);
     TSX_LAUNCH_CHECK("conv_i8_px_kernel");
     return 0;
 }
@@ -208,13 +212,12 @@ int launch_ks(PxParams &p, hipStream_t stream) {
     // when the line had left.  Large outputs of such planes take two blocks at a time (us, window-stationary, all blocks, two: joins of 64 to 2048
     // channels 10 images of 54x54 131.2, 154.5, 118.3, 256 to 4096 32 of 19x19 155, 168, 117; 80 such layers 1.00, 1.18 at most, of the
     // window-stationary kernel's time with all and 0.83 with two).  Smaller outputs stay in L2 (16 blocks, 16 to 32 MiB, 1.00 of the time, up to 1.15),
-    // and the exact Mish leaves the second group less behind (32 to 64 MiB 1.01).
-    const bool lines_leave = p.out_f32 && p.howo % 32 != 0 && p.blocks >= 16 && p.out_bytes >= (mish ? 64u << 20 : 32u << 20);
-    p.panel = !lines_leave ? p.blocks : p.blocks % 2 == 0 ? 2 : 1;
-    p.span = p.panel * p.slots;
-    p.panel_magic = div_magic(p.panel, p.span);
-    p.span_magic = div_magic(p.span, int64_t(p.blocks) * p.slots);
-    const unsigned grid = unsigned(8 * p.blocks * p.slots);
+    // and the exact Mish leaves the second group less behind (32 to 64 MiB 1.01).  In instantiations of their own: the longer way to a workgroup's place, at the head
+    // of its chain of loads, cost the other layers 0.5 %.
+    const int blocks = p.blocks;
+    if (p.out_f32 && !p.stream && p.howo % 32 != 0 && blocks >= 16 && p.out_bytes >= (mish ? 64u << 20 : 32u << 20)) p.blocks = blocks % 2 == 0 ? 2 : 1;
+    p.blocks_magic = div_magic(p.blocks, int64_t(p.blocks) * p.slots);
+    const dim3 grid(unsigned(8 * p.blocks * p.slots), unsigned(blocks / p.blocks));
     if (wn == 1) return mish ? launch<KS, 1, true>(p, grid, stream) : launch<KS, 1, false>(p, grid, stream);
     if constexpr (KS <= 4) if (wn == 2) return mish ? launch<KS, 2, true>(p, grid, stream) : launch<KS, 2, false>(p, grid, stream);
     if constexpr (KS <= 2) return mish ? launch<KS, 4, true>(p, grid, stream) : launch<KS, 4, false>(p, grid, stream);

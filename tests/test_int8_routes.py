@@ -57,8 +57,9 @@ at = 1 << 20                      # an address that nothing reads
 out = []
 for n, c, h, w, cout, k, s, act, outputs in json.loads(sys.argv[3]):
     kh, kw = k if isinstance(k, list) else (k, k)
-    geom = ConvGeom(n, c, h, w, cout, kh, kw, kh // 2, kh // 2, kw // 2, kw // 2, s, s, 1, 1)
-    ho, wo = (h + 2 * (kh // 2) - kh) // s + 1, (w + 2 * (kw // 2) - kw) // s + 1
+    sh, sw = s if isinstance(s, list) else (s, s)
+    geom = ConvGeom(n, c, h, w, cout, kh, kw, kh // 2, kh // 2, kw // 2, kw // 2, sh, sw, 1, 1)
+    ho, wo = (h + 2 * (kh // 2) - kh) // sh + 1, (w + 2 * (kw // 2) - kw) // sw + 1
     ep = Epilogue(dq_dev=at, bias_dev=at, act=_ACT[act], slope=0.1)
     if "i8" in outputs or "staged" in outputs:
         ep.q_scales_dev, ep.n_qscales = at, n
@@ -108,7 +109,7 @@ def test_large_plain_fp32_outputs_of_whole_half_lines_are_streamed(route):
              ([32, 64, 56, 56, 256, 1, 1, "relu", "f32 join"], False), ([32, 64, 56, 56, 256, 1, 1, "relu", "f32 staged"], False)]
     for (call, streams), (kernel, _, _) in zip(calls, route([call for call, _ in calls])):
         arguments = kernel[:-1].split("<")[1].split(", ")
-        assert kernel.startswith("conv_i8_px_kernel<") and arguments[-1] == ("true" if streams else "false"), (call, kernel)
+        assert kernel.startswith("conv_i8_px_kernel<") and arguments[6] == ("true" if streams else "false"), (call, kernel)
 
 
 def test_pixel_streams_of_1024_channels_fill_rounds_of_two_workgroups_per_cu(route):
@@ -117,3 +118,14 @@ def test_pixel_streams_of_1024_channels_fill_rounds_of_two_workgroups_per_cu(rou
              ([20, 1024, 14, 14, 256, 1, 1, "relu", "staged"], 16, 2, 1), ([4, 1024, 74, 74, 1024, 1, 1, "relu", "f32"], 86, 8, 6)]
     for (call, per_xcd, blocks, turns), (kernel, workgroups, _) in zip(calls, route([c[0] for c in calls])):
         assert kernel.startswith("conv_i8_px_kernel<16, 1, ") and workgroups == 8 * blocks * -(-per_xcd // turns), (call, kernel, workgroups)
+
+
+def test_pixel_streams_whose_planes_share_lines_take_two_blocks_of_channels_at_a_time(route):
+    calls = [([10, 64, 54, 54, 2048, 1, 1, "relu", "f32 join"], True), ([32, 256, 19, 19, 4096, 1, 1, "mish", "f32 staged join"], True), ([16, 1024, 37, 37, 2048, 1, 1, "relu", "f32"], True),
+             ([9, 256, 33, 35, 2176, 1, 1, "relu", "f32 join"], True),                             # 17 blocks: one at a time
+             ([10, 64, 56, 56, 2048, 1, 1, "relu", "f32 join"], False), ([10, 64, 54, 54, 1024, 1, 1, "relu", "f32 join"], False),        # whole lines; 8 blocks
+             ([2, 64, 41, 43, 2048, 1, 1, "relu", "f32 join"], False), ([3, 64, 41, 43, 2048, 1, 1, "mish", "f32 join"], False),          # below 32 MiB; 64
+             ([10, 64, 54, 54, 2048, 1, 1, "relu", "staged"], False), ([10, 64, 52, 52, 2048, 1, 1, "relu", "f32"], False)]               # no fp32 output; a streamed one
+    for (call, panels), (kernel, workgroups, _) in zip(calls, route([c for c, _ in calls])):
+        assert kernel.startswith("conv_i8_px_kernel<") and (kernel[:-1].split(", ")[-1] == "true") == panels, (call, kernel)
+        assert workgroups % (8 * call[4] // 128) == 0
