@@ -87,10 +87,20 @@ void pt_plan(const WsGeom &g, WsPlan *pl) {
         if (tw >= 4 && tw <= px) consider(tw);
     }
     for (int tw = 4; tw <= px; tw *= 2) consider(tw);
+    // Tiles that are mostly empty, where windows of strided layers leave little of a map's height and width to choose from: below 0.45 of
+    // their positions 1.19 times the other kernels' time (30 layers, 1.64 at most), to 0.6 1.08 (22), above 0.7 0.89 (1240).
+    if (pl->pt && int64_t(g.n) * g.ho * g.wo * 5 < pl->pt_tiles * px * 3) pl->pt = false;
     // Too few workgroups leave the tiles that the others could share: 100 to 128 of them 0.91 to 0.97 times as fast as the other
     // kernels (32 images of 14x14, 64 or 128 channels; 7x7 to 512), from 196 on (4 of 28x28 64 to 512; 112x112 64 to 64) 1.06 and more.
     const int wm = 4 / fragments_side_by_side(g.cout);
     if (pl->pt && pl->pt_tiles * (g.cout / 32 / wm) < 160) pl->pt = false;
+}
+
+// The workgroups that a CU holds of the kernel that runs the layer, as it is compiled.
+static int pt_resident(const WsGeom &g, const WsPlan &pl, bool mishx) {
+    const int taps = g.kh * g.kw, fill = pl.pt_wpix * 4 * g.cblocks <= 3 * 256 ? 3 : 5;
+    if (!mishx && g.cblocks == 1) return taps == 6 ? 4 : 3;      // (157 registers and fewer, where pt_waves promises two and three)
+    return pt_waves(g.cblocks, taps, fill);
 }
 
 bool pt_takes(const WsGeom &g, const WsPlan &pl, const EpiParams &ep) {
@@ -99,6 +109,18 @@ bool pt_takes(const WsGeom &g, const WsPlan &pl, const EpiParams &ep) {
     // offsets reach
     const int64_t image = int64_t(g.cout) * g.ho * g.wo, count = g.n * image, reach = 0xffff0000;
     if (ep.act_body != count || !(ep.n_qscales == 1 ? ep.q_bulk8 == count : ep.q_group_len == image)) return false;
+    // What is left to the window-stationary kernel, by the tiles of an XCD times their channel blocks (us, that kernel -> this one).  A little
+    // more than its CUs hold two at a time is two turns on a part of them, where that kernel's small tiles fill all: between one round and one
+    // and a half, with two channel blocks in and 128 channels out at a time 1.07 in the mean of 47 layers (one image of 151x151 128 to 256 14.1 -> 16.1; 0.92
+    // below, 0.91 above), with the exact Mish 1.10 in that of 79 (9 of 70x70 128 to 128 17.5 -> 19.9; 0.92 on both sides); where the flat-tile kernel
+    // is the other one 0.96 (84).  The exact Mish makes a turn long: 1.02 in the mean of 136 layers up to 48 (16 of 29x29 64 to 128 8.0 -> 8.4),
+    // 0.93 to 64.  It computes empty positions too.
+    const bool mishx = ep.act == TSX_ACT_MISH;
+    const int wn = fragments_side_by_side(g.cout);
+    const int64_t wgs = ceil_div(pl.pt_tiles, 8) * (g.cout / 32 / (4 / wn)), positions = int64_t(g.n) * g.ho * g.wo;
+    if (mishx && wn == 1 && wgs <= 48) return false;
+    if (mishx && positions * 25 < pl.pt_tiles * 32 * pt_frags(wn) * 18) return false;
+    if (!pl.flat && pt_resident(g, pl, mishx) == 2 && (mishx || wn == 1) && wgs > 64 && wgs <= 96) return false;
     return int64_t(g.n) * ep.st_hs * ep.st_ws * ep.st_cp <= reach && int64_t(g.n) * g.hs * g.ws * g.cp <= reach && count < (int64_t(1) << 31);
 }
 

@@ -79,3 +79,38 @@ def test_large_outputs_whose_planes_share_lines(monkeypatch, n, c, h, w, cout):
     res = device((n, cout, h, w), 23, 1.0)
     for act, f32, requantized, residual in (("relu", True, False, res), ("leaky_relu", True, True, res), ("none", True, False, None), ("mish", True, True, None)):
         same_outputs(monkeypatch, conv, dq, bias, staged, (n, c, h, w), (n, cout, h, w), act, f32, requantized, residual)
+
+
+TILE_STREAMS_WITH_MISH = [
+    # n, c, h, w, cout, taps, strides: a layer for each instantiation of the small-tile kernel that the exact Mish is left on
+    (11, 64, 53, 51, 128, (3, 3), (1, 1)), (8, 64, 53, 51, 64, (3, 3), (1, 1)), (9, 50, 120, 110, 32, (3, 3), (1, 1)), (9, 64, 141, 150, 256, (3, 3), (2, 2)),
+    (3, 64, 141, 150, 64, (3, 3), (2, 2)), (9, 64, 140, 71, 128, (3, 2), (2, 1)), (3, 64, 70, 81, 64, (2, 3), (1, 1)), (12, 100, 50, 50, 128, (3, 3), (1, 1)),
+    (3, 128, 64, 63, 64, (3, 3), (1, 1)),
+]
+
+
+@pytest.mark.parametrize("case", TILE_STREAMS_WITH_MISH, ids=lambda c: "-".join(map(str, c[:5])) + "-k%d%d-s%d%d" % (c[5] + c[6]))
+def test_tile_streams_with_the_exact_mish(port, monkeypatch, case):
+    """... whole output buffers against the other kernels, and two images of them against the oracle."""
+    import torch
+    from tennis_amd import capi
+    n, c, h, w, cout, (kh, kw), strides = case
+    conv = capi.Conv2dI8(device((cout, c, kh, kw), 3), (kh // 2, kh // 2, kw // 2, kw // 2), strides)
+    x = device((n, c, h, w), 4)
+    staged = capi.StagedInput(conv, x.shape)
+    conv.stage(x, staged)
+    dq, bias = device((cout,), 5, 1e-5).abs() * 10 / c ** 0.5 + 1e-6, device((cout,), 6, 1.0)
+    scales = device((n,), 7, 1.0).abs() * 10 + 20
+    ho, wo = (h + 2 * (kh // 2) - kh) // strides[0] + 1, (w + 2 * (kw // 2) - kw) // strides[1] + 1
+    second = capi.Conv2dI8(torch.zeros((32, cout, 3, 3), dtype=torch.int8, device="cuda"), (1, 1, 1, 1))
+    got = []
+    for on in (False, True):
+        streams(monkeypatch, conv, x.shape, "tile_stream", on)
+        out = capi.StagedInput(second, (n, cout, ho, wo))
+        conv.run_staged(staged, dq, bias, "mish", want_f32=False, q_scales=scales, staged_out=out)
+        got.append(out)
+    assert torch.equal(got[0].buf, got[1].buf)
+    two = x[n - 2:].cpu().numpy()       # (one scale each: a single one is rounded half to even)
+    weights = device((cout, c, kh, kw), 3).cpu().numpy()
+    plain = port.add_bias(port.conv2d_quantized(two, weights, dq.cpu().numpy(), (kh // 2, kh // 2, kw // 2, kw // 2), strides), bias.cpu().numpy())
+    assert np.array_equal(capi.staged_interior(got[1], [n - 2, n - 1]).cpu().numpy(), port.quantize(port.mish(plain), scales[n - 2:].cpu().numpy()))

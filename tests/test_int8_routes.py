@@ -129,3 +129,26 @@ def test_pixel_streams_whose_planes_share_lines_take_two_blocks_of_channels_at_a
     for (call, panels), (kernel, workgroups, _) in zip(calls, route([c for c, _ in calls])):
         assert kernel.startswith("conv_i8_px_kernel<") and (kernel[:-1].split(", ")[-1] == "true") == panels, (call, kernel)
         assert workgroups % (8 * call[4] // 128) == 0
+
+
+def test_small_tiles_keep_the_layers_that_gain(route):
+    """Little more than a round of two workgroups per CU, few tiles with the exact Mish and tiles that are mostly empty stay on the other kernels."""
+    tiles = [([32, 64, 56, 56, 64, 3, 1, "relu", "staged"], "1, 9, 2, 3, false"), ([32, 128, 28, 28, 128, 3, 1, "relu", "staged"], "2, 9, 1, 4, false"),
+             ([8, 128, 76, 76, 256, 3, 1, "leaky_relu", "staged"], "2, 9, 1, 4, false"), ([8, 128, 76, 76, 256, 3, 1, "mish", "staged"], "2, 9, 1, 4, true"),
+             ([8, 64, 304, 304, 128, 3, 2, "mish", "staged"], "1, 9, 1, 5, true"), ([8, 64, 608, 304, 64, [3, 2], [2, 1], "mish", "staged"], "1, 6, 2, 3, true"),
+             ([3, 128, 64, 63, 64, 3, 1, "relu", "staged"], "2, 9, 2, 4, false"),
+             ([26, 100, 36, 36, 128, 3, 1, "mish", "staged"], "2, 9, 1, 4, true")]               # (the other kernel: flat tiles)
+    for (call, arguments), (kernel, _, _) in zip(tiles, route([c for c, _ in tiles])):
+        assert kernel == "conv_i8_pt_kernel<" + arguments + ">", (call, kernel)
+    others = [[1, 128, 151, 151, 256, 3, 1, "none", "staged"], [9, 128, 70, 70, 128, 3, 1, "mish", "staged"], [16, 64, 29, 29, 128, 3, 1, "mish", "staged"],
+              [20, 128, 12, 251, 256, 3, 2, "mish", "staged"], [8, 128, 7, 167, 512, 3, 2, "none", "staged"]]
+    for call, (kernel, _, _) in zip(others, route(others)):
+        assert not kernel.startswith("conv_i8_pt_kernel<"), (call, kernel)
+
+
+def test_the_exact_mish_on_small_tiles_is_compared(route):
+    from test_gpu_conv_i8_streams import TILE_STREAMS_WITH_MISH
+    calls = [[n, c, h, w, cout, list(taps), list(strides), "mish", "staged"] for n, c, h, w, cout, taps, strides in TILE_STREAMS_WITH_MISH]
+    kernels = [kernel for kernel, _, _ in route(calls)]
+    assert sorted(kernels) == sorted("conv_i8_pt_kernel<%s, true>" % a for a in
+                                     ("1, 9, 1, 3", "1, 9, 2, 3", "1, 9, 4, 3", "1, 9, 1, 5", "1, 9, 2, 5", "1, 6, 1, 3", "1, 6, 2, 3", "2, 9, 1, 4", "2, 9, 2, 4")), kernels
