@@ -169,6 +169,9 @@ int pt_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t 
         shortest = time;
         p.slots = int(slots);
     }
+    // ... or one, where CUs hold all workgroups as the kernels are compiled.  (Between what the model takes for that and what it is, us, two turns -> one:
+    // 14 images of 73x73 at stride 2 64 to 256 11.4 -> 9.9, 0.89 of the time in the mean of 7 layers; six taps 0.94 in that of 40.)
+    if (int64_t(p.per_xcd) * p.blocks <= 32 * pt_resident(g, pl, ep.act == TSX_ACT_MISH)) p.slots = p.per_xcd;
     p.blocks_magic = div_magic(p.blocks, int64_t(p.blocks) * p.slots);
     const unsigned grid = unsigned(8 * p.blocks * p.slots);
     const size_t lds_bytes = size_t(2) * pl.pt_wpix * pitch;

@@ -152,3 +152,18 @@ def test_the_exact_mish_on_small_tiles_is_compared(route):
     kernels = [kernel for kernel, _, _ in route(calls)]
     assert sorted(kernels) == sorted("conv_i8_pt_kernel<%s, true>" % a for a in
                                      ("1, 9, 1, 3", "1, 9, 2, 3", "1, 9, 4, 3", "1, 9, 1, 5", "1, 9, 2, 5", "1, 6, 1, 3", "1, 6, 2, 3", "2, 9, 1, 4", "2, 9, 2, 4")), kernels
+
+
+def test_small_tiles_take_one_turn_where_the_compiled_kernels_hold_all_workgroups(route):
+    """Three workgroups with five window chunks a thread to a CU, four with six taps: 96 and 128 to an XCD."""
+    calls = [([14, 64, 73, 73, 256, 3, 2, "none", "staged"], "1, 9, 1, 5, false", 2, True), ([18, 64, 73, 73, 256, 3, 2, "none", "staged"], "1, 9, 1, 5, false", 2, False),
+             ([8, 64, 100, 71, 64, [3, 2], 1, "relu", "staged"], "1, 6, 2, 3, false", 1, True), ([10, 64, 100, 71, 64, [3, 2], 1, "relu", "staged"], "1, 6, 2, 3, false", 1, False),
+             ([9, 64, 73, 73, 256, 3, 2, "mish", "staged"], "1, 9, 1, 5, true", 2, True)]
+    for (call, arguments, blocks, one), (kernel, workgroups, info) in zip(calls, route([c[0] for c in calls])):
+        assert kernel == "conv_i8_pt_kernel<" + arguments + ">", (call, kernel)
+        n, _, h, w, _, k, s = call[:7]
+        kh, kw = k if isinstance(k, list) else (k, k)
+        th, tw = (int(v) for v in info["tile_stream"].split("x"))
+        rows, columns = n * ((h + 2 * (kh // 2) - kh) // s + 1), (w + 2 * (kw // 2) - kw) // s + 1
+        per_xcd = -(-(-(-rows // th) * -(-columns // tw)) // 8)
+        assert (workgroups == 8 * blocks * per_xcd) == one, (call, workgroups, per_xcd)
