@@ -128,8 +128,10 @@ size_t tsx_conv2d_i8_workspace_bytes(const tsx_conv2d_geom *g);
  * TSX_CONV_I8_RS ("0" = never, "force" = wherever the geometry allows) are read at every call that plans, and so is
  * TSX_CONV_I8_KS ("0" = never, a number = that tile of the K-split kernel wherever the geometry allows).  Where that is
  * not set and one of the other two has a value, any value, no layer takes the K-split kernel.
- * " pixel_stream=1" and " tile_stream=<rows>x<columns>" behind it say that calls whose outputs are fp32 or staged (of
- * tile streams: staged only, without a residual) run on the streaming kernel for 1x1 layers or the one for small tiles instead;
+ * "k_parts=2" (window_stationary) says that the workgroups multiply K in halves.  " pixel_stream=1" behind the kernel says that
+ * calls with fp32 and staged outputs only run on the streaming kernel for 1x1 layers instead, " pixel_stream_joins=0" that those with a
+ * residual do not; " tile_stream=<rows>x<columns>" that calls whose output is staged only, without a residual, run on the one for
+ * small tiles (with the exact Mish, and where little more than one round of workgroups is left, not all of them);
  * TSX_CONV_I8_PX and TSX_CONV_I8_PT = "0" keep layers off these. */
 int tsx_conv2d_i8_plan_info(const tsx_conv2d_geom *g, char *text, size_t text_bytes);
 /* padding_value is the reference's float parameter; it is cast to int8 as the reference

@@ -1320,15 +1320,15 @@ int tsx_conv2d_i8_plan_info(const tsx_conv2d_geom *g, char *text, size_t text_by
         std::snprintf(text, text_bytes, "kernel=%s fp32_kernel=%s fragments_per_tile=%d tiles=%lld resident=%d", base, base,
                       pl.wsp.fl_nta + pl.wsp.fl_ntb, (long long)(pl.wsp.fl_tiles * (pl.wsp.coutp / 128)), int(pl.wsp.fl_resident));
     else if (pl.use_ws)
-        std::snprintf(text, text_bytes, "kernel=%s fp32_kernel=%s fragments_per_wavefront=%d wavefronts_along_cout=%d tiles=%lld blocks_per_window=%d",
-                      base, base, pl.wsp.nt, pl.wsp.wm, (long long)(pl.wsp.tiles * ((g->cout + 32 * pl.wsp.wm - 1) / (32 * pl.wsp.wm))), pl.wsp.cbs);
+        std::snprintf(text, text_bytes, "kernel=%s fp32_kernel=%s fragments_per_wavefront=%d wavefronts_along_cout=%d tiles=%lld blocks_per_window=%d k_parts=%d",
+                      base, base, pl.wsp.nt, pl.wsp.wm, (long long)(pl.wsp.tiles * ((g->cout + 32 * pl.wsp.wm - 1) / (32 * pl.wsp.wm))), pl.wsp.cbs, tsx::ws_k_parts(pl.wsg, pl.wsp));
     else
         std::snprintf(text, text_bytes, "kernel=%s fp32_kernel=%s", base, base);
     if (pl.wsp.ks) std::snprintf(text, text_bytes, "kernel=k_split fp32_kernel=k_split tile=%d", pl.wsp.ks);
-    else if (pl.wsp.px) {      // for fp32 and staged outputs; the kernel named before writes the others
+    else if (pl.wsp.px) {      // for fp32 and staged outputs; the kernel named before writes the others, and some joins
         const size_t used = std::strlen(text);
-        std::snprintf(text + used, text_bytes - used, " pixel_stream=1");
-    } else if (pl.use_ws && pl.wsp.pt) {      // the same
+        std::snprintf(text + used, text_bytes - used, " pixel_stream=1 pixel_stream_joins=%d", int(tsx::px_joins(pl.wsg)));
+    } else if (pl.use_ws && pl.wsp.pt) {      // for some activations' staged outputs
         const size_t used = std::strlen(text);
         std::snprintf(text + used, text_bytes - used, " tile_stream=%dx%d", pl.wsp.pt_th, pl.wsp.pt_tw);
     }

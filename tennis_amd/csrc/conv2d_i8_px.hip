@@ -235,9 +235,11 @@ void px_plan(const WsGeom &g, WsPlan *pl) {
              g.cout % (ks <= 2 ? 32 : ks <= 4 ? 64 : 128) == 0;
 }
 
+// with a residual, weights of 512 channels leave too few registers (512 to 2048 7x7, 32 images: 14.0 us window-stationary, 15.5 here)
+bool px_joins(const WsGeom &g) { return g.cblocks <= 4; }
+
 bool px_takes(const WsGeom &g, const WsPlan &pl, const EpiParams &ep) {
-    // with a residual, weights of 512 channels leave too few registers (512 to 2048 7x7, 32 images: 14.0 us window-stationary, 15.5 here)
-    if (!pl.px || (g.cblocks > 4 && ep.residual)) return false;
+    if (!pl.px || (ep.residual && !px_joins(g))) return false;
     // fp32 values and staged ones only; all of them in the activation's SIMD body, with one scale per image (or one for all, rounded
     // the same way); tensors that 32-bit offsets reach
     const int64_t image = int64_t(g.cout) * g.ho * g.wo, count = g.n * image, positions = int64_t(g.n) * g.ho * g.wo, reach = 0xffff0000;

@@ -7,6 +7,7 @@ namespace tsx {
 // Whether the kernel serves the layer (WsPlan::px); whether it also writes the epilogue and reaches the tensors of a call;
 // launch.  g holds the extents of the buffer that is read; the weights are packed as for the layer's other kernels.
 void px_plan(const WsGeom &g, WsPlan *pl);
+bool px_joins(const WsGeom &g);      // whether a residual may join
 bool px_takes(const WsGeom &g, const WsPlan &pl, const EpiParams &ep);
 int px_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t *packed, const EpiParams &ep, hipStream_t stream);
 

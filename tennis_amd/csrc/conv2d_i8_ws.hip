@@ -225,6 +225,17 @@ int ws_pack_weights(const WsGeom &g, const WsPlan &pl, const int8_t *w_oihw, int
     return 0;
 }
 
+int ws_k_parts(const WsGeom &g, const WsPlan &pl) {
+    // One fragment per wavefront, no more workgroups than CUs, and two channel blocks or more for each half of K.  Below 24 K-steps joining the
+    // sums takes what halves save: 1x1 layers on 512 to 1024 channels, times without halves : with them 0.97 to 1.025 (1.00 in the mean, 80 layers),
+    // on 1536 0.995 to 1.07 (1.02), on 2048 0.99 to 1.10 (1.05).  (Such a launch writes 4 MiB of fp32 at most: never streamed.)
+    const int windows = g.cblocks / pl.cbs;
+    const size_t lds_bytes = size_t(windows > 1 ? 2 : 1) * pl.wp * (64 * pl.cbs + 16);
+    const bool small_fill = ceil_div(pl.wp * 4 * pl.cbs, WS_THREADS) <= SMALL_FILL;
+    return pl.nt == 1 && small_fill && pl.tiles * ceil_div(g.cout, 32 * WS_FM * pl.wm) <= 256 && g.cblocks * g.kh * g.kw >= 24 && windows >= 4 &&
+           windows % 2 == 0 && 2 * lds_bytes <= 57344 ? 2 : 1;
+}
+
 int ws_launch(const WsGeom &g, const WsPlan &plan, const int8_t *xs, const int8_t *packed, const EpiParams &ep,
               hipStream_t stream) {
     WsPlan pl = plan;
@@ -284,6 +295,7 @@ int ws_launch(const WsGeom &g, const WsPlan &plan, const int8_t *xs, const int8_
         p.tap_col = 64;
     }
     p.stream_out = streams_fp32(ep, int64_t(g.n) * g.cout * g.ho * g.wo) ? 1 : 0;
+    p.k_parts = ws_k_parts(g, pl);
     p.rowmajor = g.gemm ? 1 : 0;
     if (g.gemm) p.stream_out = 0;
     p.wc_magic = div_magic(p.wc, MAX_WP);

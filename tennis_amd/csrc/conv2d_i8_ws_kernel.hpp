@@ -34,6 +34,7 @@ struct WsParams : EpiParams {
     int pix, chunk_shift, stage_bytes, tap_row, tap_col;
     int per_xcd, tiles, blocks_m;   // workgroups of each XCD's run (0: grid of tiles x channel blocks), position tiles, channel blocks
     int stream_out;   // fp32 output written with streaming stores
+    int k_parts;      // 2: K in halves (LOOK = 2)
     int rowmajor;     // GEMM: output index position * cout + channel, row_scale[position] applied behind dq
     // per-lane divisions by uniform divisors as one multiply-high (div_magic / udiv)
     unsigned wc_magic, tw_magic, ow_magic;
@@ -625,19 +626,15 @@ int ws_launch_nt<TSX_WS_NT>(const WsParams &p, dim3 grid, size_t lds_bytes, hipS
     // one fragment per wavefront, a K of two rounds or more, and few enough workgroups that a SIMD holds one or
     // two wavefronts: the B ring (more registers: three workgroups per CU)
     const bool look = NT == 1 && small_fill && p.ksteps >= 2 * RING && int64_t(p.tiles) * p.blocks_m <= 1024;
-    // no more workgroups than CUs, and two channel blocks or more for each: K in halves.  Below 24 K-steps joining the sums takes what
-    // halves save: 1x1 layers on 512 to 1024 channels, times without halves : with them 0.97 to 1.025 (1.00 in the mean, 80 layers), on
-    // 1536 0.995 to 1.07 (1.02), on 2048 0.99 to 1.10 (1.05).
-    const int parts = look && int64_t(p.tiles) * p.blocks_m <= 256 && p.ksteps >= 24 && p.cblocks >= 4 && p.cblocks % 2 == 0 && 2 * lds_bytes <= 57344 ? 2 : 1;
 #define TSX_WS_LAUNCH(EXTRA, STREAM, ROWM, MISHX)                                                                      \
     do {                                                                                                               \
         constexpr int F = NT <= 2 ? SMALL_FILL : MAX_FILL;                                                             \
-        const int fill = NT == 1 && parts > 1 ? 3 : NT == 1 && look ? 0 : NT <= 2 && small_fill ? 1 : 2;                  \
-        const auto kernel = fill == 3 ? conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, NT == 1 ? 2 : 0, MISHX>   \
+        const int fill = NT == 1 && p.k_parts > 1 ? 3 : NT == 1 && look ? 0 : NT <= 2 && small_fill ? 1 : 2;                  \
+        const auto kernel = fill == 3 ? conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, NT == 1 && !(STREAM) ? 2 : 0, MISHX> \
                             : fill == 0 ? conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, NT == 1 ? 1 : 0, MISHX> \
                             : fill == 1 ? conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, F, 0, MISHX>               \
                                         : conv_i8_ws_kernel<NT, WS_FM, EXTRA, STREAM, ROWM, MAX_FILL, 0, MISHX>;       \
-        const size_t dynamic = parts > 1 ? std::max<size_t>(2 * lds_bytes, 16384) : lds_bytes;                         \
+        const size_t dynamic = p.k_parts > 1 ? std::max<size_t>(2 * lds_bytes, 16384) : lds_bytes;                         \
         if (MISHX && dynamic + sizeof(MishTables) > 65536) {      /* granted per kernel and device */                \
             static std::atomic<bool> granted[4][64];                                                                   \
             int dev = 0;                                                                                               \
@@ -648,7 +645,7 @@ int ws_launch_nt<TSX_WS_NT>(const WsParams &p, dim3 grid, size_t lds_bytes, hipS
                 if (dev < 64) granted[fill][dev].store(true);                                                          \
             }                                                                                                          \
         }                                                                                                              \
-        hipLaunchKernelGGL(kernel, grid, dim3(parts * WS_THREADS), dynamic, stream, p);                                 \
+        hipLaunchKernelGGL(kernel, grid, dim3(p.k_parts * WS_THREADS), dynamic, stream, p);                                 \
     } while (0)
     // the exact Mish: instantiations (with every other epilogue term) that only its layers run
     if (p.act == TSX_ACT_MISH) {

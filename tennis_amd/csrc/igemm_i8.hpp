@@ -254,6 +254,8 @@ struct WsGeom {
 };
 
 WsPlan ws_plan(const WsGeom &g);
+// parts of K that a workgroup of the window-stationary kernel multiplies side by side: 1, 2
+int ws_k_parts(const WsGeom &g, const WsPlan &pl);
 int ws_pack_weights(const WsGeom &g, const WsPlan &pl, const int8_t *w_oihw, int c, int8_t *packed, hipStream_t stream);
 int ws_launch(const WsGeom &g, const WsPlan &pl, const int8_t *xs, const int8_t *packed, const EpiParams &ep,
               hipStream_t stream);

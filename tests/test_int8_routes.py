@@ -87,17 +87,16 @@ def route(tmp_path_factory):
     subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(so), str(source)])
     env = {k: v for k, v in os.environ.items() if not k.startswith("TSX_")}
 
-    def routes(calls):
-        run = subprocess.run([sys.executable, "-c", CALLS, str(so), LIB_PATH, json.dumps(calls), ROOT], capture_output=True, text=True, cwd=ROOT, env=env)
+    def routes(calls, **switches):
+        run = subprocess.run([sys.executable, "-c", CALLS, str(so), LIB_PATH, json.dumps(calls), ROOT], capture_output=True, text=True, cwd=ROOT,
+                             env=dict(env, **{"TSX_CONV_I8_" + k: v for k, v in switches.items()}))
         assert run.returncode == 0, run.stderr
         out = []
         for call, (rc, launched, info) in zip(calls, json.loads(run.stdout)):
             assert rc == 0 and launched.count(";") == 1, (call, rc, launched)
-            name, workgroups, threads = launched.rstrip(";").split(" ")
-            name = subprocess.run(["c++filt", name], capture_output=True, text=True, check=True).stdout
-            name = re.search(r"(\w+)<([^<>]*)>", name)
-            out.append((name.group(1) + "<" + name.group(2) + ">", int(workgroups), dict(word.split("=", 1) for word in info.split())))
-        return out
+            out.append(launched.rstrip(";").split(" ")[:2] + [dict(word.split("=", 1) for word in info.split())])
+        names = subprocess.run(["c++filt"], input="\n".join(name for name, _, _ in out), capture_output=True, text=True, check=True).stdout.splitlines()
+        return [("%s<%s>" % re.search(r"(\w+)<([^<>]*)>", name).groups(), int(workgroups), info) for name, (_, workgroups, info) in zip(names, out)]
     return routes
 
 
@@ -167,3 +166,20 @@ def test_small_tiles_take_one_turn_where_the_compiled_kernels_hold_all_workgroup
         rows, columns = n * ((h + 2 * (kh // 2) - kh) // s + 1), (w + 2 * (kw // 2) - kw) // s + 1
         per_xcd = -(-(-(-rows // th) * -(-columns // tw)) // 8)
         assert (workgroups == 8 * blocks * per_xcd) == one, (call, workgroups, per_xcd)
+
+
+def test_plans_say_which_pixel_streams_take_joins(route):
+    calls = [[40, c, 14, 14, 256, 1, 1, "relu", outputs] for c in (64, 250, 512, 1000) for outputs in ("f32", "f32 join", "staged", "staged join")]
+    for call, (kernel, _, info) in zip(calls, route(calls, KS="0")):
+        joins = call[1] <= 256
+        assert info["pixel_stream"] == "1" and info["pixel_stream_joins"] == str(int(joins)), info
+        assert kernel.startswith("conv_i8_px_kernel<") == (joins or "join" not in call[-1]), (call, kernel)
+
+
+def test_plans_say_which_layers_have_k_in_halves(route):
+    layers = [((4, 256, 7, 7, 128, 3, 1), 2), ((32, 512, 7, 7, 96, 3, 1), 2), ((2, 448, 9, 8, 130, 3, 1), 1), ((8, 512, 14, 13, 64, 3, 2), 1), ((8, 512, 14, 14, 128, 3, 2), 2),
+              ((6, 640, 5, 5, 128, 5, 1), 2), ((30, 2048, 7, 7, 100, 1, 1), 2), ((9, 1100, 6, 7, 255, 1, 1), 1), ((9, 1536, 6, 7, 255, 1, 1), 2)]
+    calls = [(list(layer) + [act, outputs], parts) for layer, parts in layers for outputs in ("f32", "f32 staged", "staged join") for act in ("relu", "mish")]
+    for (call, parts), (kernel, _, info) in zip(calls, route([c for c, _ in calls], KS="0", PX="0", FLAT="0", RS="0")):
+        assert kernel.startswith("conv_i8_ws_kernel<1, ") and info["k_parts"] == str(parts), (call, kernel, info)
+        assert (kernel.split(", ")[6] == "2") == (parts == 2), (call, kernel)
