@@ -183,3 +183,10 @@ def test_plans_say_which_layers_have_k_in_halves(route):
     for (call, parts), (kernel, _, info) in zip(calls, route([c for c, _ in calls], KS="0", PX="0", FLAT="0", RS="0")):
         assert kernel.startswith("conv_i8_ws_kernel<1, ") and info["k_parts"] == str(parts), (call, kernel, info)
         assert (kernel.split(", ")[6] == "2") == (parts == 2), (call, kernel)
+
+
+def test_layers_with_special_values_run_on_the_small_tiles(route):
+    calls = [[n, c, 104, 104, 256, 3, 1, act, "staged"] for n in (1, 3) for c in (64, 128) for act in ("none", "relu", "leaky_relu")]
+    calls += [[n, 64, 16, 16, 8192, 3, 1, "mish", "staged"] for n in (1, 2)]
+    for call, (kernel, _, _) in zip(calls, route(calls, KS="0")):
+        assert kernel.startswith("conv_i8_pt_kernel<"), (call, kernel)
