@@ -9,11 +9,11 @@
 // one is multiplied, and waits in the other half of LDS, one barrier a tile.  Windows have a pitch of 80 or 144 bytes a pixel:
 // the operands' 16-byte reads are free of bank conflicts.
 //
-// Measured, us, window-stationary or flat-tile kernel -> here, each layer on buffers of its own.  32 images: 64 to 64 56x56 14.3 -> 11.4,
-// 64 to 128 112x112 59.6 -> 50.7, 64 to 512 28x28 22.4 -> 16.2, 128 to 128 28x28 10.6 -> 10.2, 128 to 128 57x57 32.8 -> 25.4.  8 images: 128 to
-// 256 76x76 25.4 -> 22.1 (1.23 of the 2.3 Pop/s that products with both operands' supply alone reach), 64 to 128 304x304 at stride 2
-// with the exact Mish 43.7 -> 41.1, 3x2 taps 64 to 64 608x304 at stride 2, 1 with it 70.5 -> 57.8.  143 layers of 1 to 32 images,
-// 16 to 128 channels, maps of 28x28 to 224x224: 1.06 to 2.0 times as fast, 1.22 in the geometric mean.
+// Measured, us, window-stationary or flat-tile kernel -> here, each layer on buffers of its own.  32 images: 64 to 64 56x56 15.4 -> 11.3, 128 to
+// 128 28x28 10.9 -> 10.1 (inside the network 10.7 on both).  8 images: 128 to 256 76x76 25.4 -> 22.1 (1.23 of the 2.3 Pop/s that products
+// with both operands' supply alone reach), 64 to 128 304x304 at stride 2 with the exact Mish 45.7 -> 42.0, with the fast one 43.8 -> 32.7; 3x2 taps
+// 64 to 64 608x304 at stride 2, 1 with the exact one 70.5 -> 57.8.  300 random layers of 1 to 32 images, 32 to 128 channels: 0.84 of the time in the
+// geometric mean, none above 1.05 (with the rules of pt_takes).
 //
 // Not taken: fp32 values too (a small tile writes pieces of 32 bytes of a plane's rows; 128 to 128 224x224 13.8 -> 17.4); joins (the
 // same, and a residual's 16 registers: 128 to 128 76x76 with the exact Mish 30 -> 39).

@@ -12,11 +12,12 @@
 // straight from memory, 32 pixels per instruction, they come at 38 bytes per ns and CU from a pitch of 128 bytes on (67 at 64), 16 pixels of
 // 64 consecutive bytes at 108.  Scales and biases wait in LDS too, read in every turn: 32 registers less.
 //
-// us, window-stationary (strided: generic) kernel -> this one, 32 images, cold caches: 64 to 64 channels 56x56 10.4 -> 7.2; 256 to
-// 64 15.2 -> 11.6; 64 to 256 with a join (fp32 and int8 out) 50.2 -> 44.2, 5.4 TB/s; 128 to 512 28x28 34.5 -> 28.3; 256 to 1024 14x14 22.4 ->
-// 19.6 (these read and write fp32 planes in pieces of 128 bytes, for which 205 MB take 37 us at 56x56 and 51 MB 12.4 at 14x14
-// with nothing else done); 1024 to 256 14x14 9.0 -> 7.4; 256 to 512 56x56 at stride 2 19.8 -> 13.1, 1024 to 2048 14x14 17.9 -> 12.7.  8
-// images with the exact Mish: 64 to 64 304x304, int8 out, 57.5 -> 38.6 (vector instructions), fp32 and int8 126 -> 97; 512 to 512 19x19 8.3 -> 6.8.
+// us, window-stationary (strided: generic) kernel -> this one, 32 images, each layer on buffers of its own: 64 to 64 channels 56x56 11.0 -> 7.4; 256
+// to 64 15.3 -> 11.4; 64 to 256 with a join (fp32 and int8 out) 56.4 -> 52.7, 4.5 TB/s; 128 to 512 28x28 38.5 -> 32.4; 256 to 1024 14x14 24.5 ->
+// 21.3 (these read and write fp32 planes in pieces of 128 bytes, for which 205 MB take 37 us at 56x56 and 51 MB 12.4 at 14x14
+// with nothing else done; inside the network the first of them stay where they were, 54.2 -> 54.6, 54.3 -> 53.1); 1024 to 256 14x14
+// 8.7 -> 7.1; 256 to 512 56x56 at stride 2 22.5 -> 17.7, 1024 to 2048 14x14 20.5 -> 13.2.  8 images with the exact Mish: 64 to 64 304x304, int8 out,
+// 57.7 -> 37.2 (vector instructions), fp32 and int8 128 -> 99; 256 to 256 38x38 8.7 -> 6.9.  900 random layers: 0.76 of the time.
 #include "conv2d_i8_px.hpp"
 #include "conv2d_i8_px_fragment.hpp"
 
@@ -35,7 +36,8 @@ struct PxParams : EpiParams {
     int groups, per_xcd, blocks, slots;      // groups of WN fragments, those of an XCD; workgroups along cout; groups an XCD works on at a time
 };
 
-// wavefronts per SIMD that the registers leave room for
+// Wavefronts per SIMD that the registers have to leave room for, and that the turns are reckoned with.  (Many instantiations fit more
+// often as compiled, up to eight times; two K-steps, four fragments side by side and the tables of the exact Mish three times, by their LDS.)
 constexpr int px_waves(int ks, int wn, bool res, bool mishx) { return ks == 16 ? 2 : ks == 8 || (res && ks == 4) || (mishx && ks * wn == 8) ? 3 : 4; }
 
 // KS: K-steps of 64 channels.  WN: fragments of a group (4 / WN wavefronts along cout).  RES: a residual joins.  F32, Q: fp32

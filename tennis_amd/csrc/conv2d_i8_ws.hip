@@ -159,8 +159,10 @@ static WsPlan make_ws_plan(const WsGeom &g_in) {
                 cost = double(rounds) * (1.0 + 0.5 * double(std::min<int64_t>(per_cu, resident) - 1)) * (0.5 + nt * (nt > 4 ? 1.45 : 1.0));
             }
             // A 1x1 layer's workgroup is mostly epilogue, its time is the traffic of its tile, and what pays is many small
-            // workgroups in flight per CU (us, 32 images: 64 to 256 channels 56x56 with a residual join, 4 fragments per
-            // wavefront 63, 2 46; 256 to 128 56x56 20.9 -> 16.9; 256 to 1024 14x14 with a join 18.1 -> 17.4).
+            // workgroups in flight per CU (us, 32 images, larger tiles -> these: 64 to 256 channels 56x56 with a residual join 63 -> 46,
+            // 256 to 128 56x56 20.9 -> 16.9).  The pixel streams write fp32 and staged values of such channels now; of 140
+            // layers that they leave, on 192, 320 and more channels or with int8 in planes, this rule and the next change 25: from 0.86 (12 images of 144x144,
+            // 256 to 64 with a join, 41.3 -> 35.6) to 1.17 of the model's time (21 of 57x43, 768 to 96, both outputs, 24.1 -> 28.2), 1.03 in the mean.
             if (!several_taps && (!g.gemm || g.cblocks <= 2) && nt > 2) continue;
             // Two fragments share a wavefront's set-up, which pays where every fragment's channels exist and its stores are whole
             // cache lines, that is, where a plane is a multiple of 64 bytes of fp32 (us, one / two: 32 images 256 to 64 56x56 14.5 / 14.0,
@@ -240,9 +242,9 @@ int ws_launch(const WsGeom &g, const WsPlan &plan, const int8_t *xs, const int8_
               hipStream_t stream) {
     WsPlan pl = plan;
     // With the exact Mish a 1x1 layer that hands out its fp32 values evaluates the whole chain for each: tiles of one fragment
-    // per wavefront, five wavefronts per SIMD for three (us, 8 images: 64 to 64 channels 304x304 127 -> 118; 128 to 64 152x152
-    // 40.8 -> 37.5; 256 to 256 38x38 19.8 -> 16.7).  Where only int8 leaves, two keep their lead (57.6 against 58.4 on the
-    // first of these) down to two workgroups per CU.
+    // per wavefront, five wavefronts per SIMD for three: 0.93 of the time in the mean of 70 layers that the pixel streams leave, 0.82 to 1.10
+    // (us, 30 images of 59x21, 192 to 128 channels with a join, 28.0 -> 22.8; 9 of 28x44, 640 to 512, 25.3 -> 27.8).  Where only int8
+    // leaves, two keep their lead (8 images of 304x304, 64 to 64, 57.6 against 58.4) down to two workgroups per CU.
     if (ep.act == TSX_ACT_MISH && g.kh * g.kw == 1 && pl.wo == 1 && pl.nt == 2 && pl.th == pl.wp && pl.th % 2 == 0 &&
         (ep.out_f32 || pl.tiles * ceil_div(g.cout, 32 * pl.wm) < 512)) {
         pl.nt = 1;

@@ -82,8 +82,8 @@ namespace {
 // their own; their sums (whole numbers: the same in any order) join through LDS.  What bounds a layer of at most one workgroup per CU is
 // each wavefront's way through K, 210 cycles a K-step for 64 of MFMAs, and a second wavefront per SIMD shortens
 // it by what the weights' way into registers leaves (65 of 130 B/ns per CU before).  us: 512 to 512 channels 3x3 7x7, 32 images, 13.9 ->
-// 13.0, at stride 2 from 14x14 14.4 -> 13.6, 2048 to 512 1x1 10.4 -> 9.5, 2048 to 256 3x3 14x14, 8 images, 36.4 -> 31.0.  Of 270 layers with
-// 256 channels and more 1.08 in the geometric mean, none slower by more than 0.7 %; with 128 channels 3x3, one block each, 0.93 to
+// 13.0, at stride 2 from 14x14 14.4 -> 13.6, 2048 to 512 1x1 10.4 -> 9.5, 2048 to 256 3x3 14x14, 8 images, 36.4 -> 31.0.  Of 160 layers with
+// 256 channels and more 0.91 of the time in the geometric mean, none above 1.005; with 128 channels 3x3, one block each, 0.93 to
 // 1.03, and with more workgroups than CUs slower (256 to 256 14x14, 448 of them, 11.3 -> 12.3).  Quarters: no more than halves below
 // 2048 channels (256 to 512 7x7 8.1 -> 9.4), 1.05 there.
 //

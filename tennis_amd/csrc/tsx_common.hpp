@@ -132,7 +132,7 @@ __device__ __forceinline__ float mish_short(float x) {
     return __fmul_rn(x, __fadd_rn(1.f, mish_minus_quotient(x)));
 }
 
-// The same for N values, N / 4 words of four int8 each (not offset binary), in 5.25 instructions an element for 7: the
+// quantize_pack for N values, N / 4 words of four int8 each (not offset binary), in 5.25 instructions an element for 7: the
 // clamp by the median of three (a NaN gives its lower end), the rounding offset, a conversion that truncates, and three byte
 // operations a word; one look at the largest of the N finds what converts to INT_MIN, products of 2^31 and more.  With
 // activate_results, of a fragment's 29 instructions a value 11 went; the kernels wait for memory more than they issue, so
@@ -187,9 +187,9 @@ __device__ __forceinline__ float mish_short_behind_a_branch(float v) {
     return mish_short(v);
 }
 
-// The activation of every epilogue: none / relu / leaky_relu / Mish (exact) / Mish (fast).  One function for all
-// kernels and all their paths, so an element's value never depends on the kernel or tile it falls into, and a fused
-// node gives what the separate operators give.
+// The activation of every epilogue: none / relu / leaky_relu / Mish (exact) / Mish (fast), an element at a time; activate_results is
+// the same for a whole fragment of the SIMD body.  Both give the same bits for every value, so an element's value never depends on the
+// kernel or tile it falls into, and a fused node gives what the separate operators give.
 __device__ __forceinline__ float apply_act(float v, int act, float slope, bool in_body) {
     if (act == TSX_ACT_MISH) return mish_value(v);
     if (act == TSX_ACT_MISH_FAST) return mish_short_behind_a_branch(v);

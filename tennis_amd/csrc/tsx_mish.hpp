@@ -209,8 +209,8 @@ struct MishAddends {
 };
 
 #ifdef __HIP_DEVICE_COMPILE__
-// 1 / d rounded to nearest for d in [1, 2]: no scaling is needed there, one Newton step on the device's reciprocal (all 2^23 + 1
-// such d compared with the division)
+// 1 / d rounded to nearest for d in [1, 2]: no scaling is needed there, one Newton step on the device's reciprocal.  (Every d that
+// occurs gives the division's bits in Mish: the comparison of mish_value with the operators, which divide, for all 2^32 floats.)
 TSX_MISH_FN float reciprocal_rn_1_2(float d) {
     const float a = __builtin_amdgcn_rcpf(d);
     return __builtin_fmaf(__builtin_fmaf(-d, a, 1.f), a, a);
